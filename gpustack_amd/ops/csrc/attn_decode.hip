@@ -1,19 +1,30 @@
 // Paged-attention decode for MI355X (gfx950) — the TPOT-dominant kernel.
 //
 // Single new token per sequence attends over the paged KV cache.
-// Replaces what the reference delegates to vLLM's paged_attention kernels
-// (SURVEY.md §2.9 #1); designed for CDNA4 rather than ported:
+// Replaces what the reference delegates to vLLM's paged_attention kernels;
+// designed for CDNA4 rather than ported:
 //
-//  - one workgroup per (sequence, kv_head); GQA q-heads (GQ = Hq/Hkv) share
-//    the K/V stream so each KV byte is read exactly once per step.
-//  - 4 waves * 4 lane-groups of 16 = 16 independent online-softmax streams;
-//    a 16-lane group owns one token per iteration, lane = 8 head dims
-//    (16 B = u16x8 loads -> 1 KiB per wave per iteration, fully coalesced
-//    against the [block, kv_head, block_size, D] pool layout).
-//  - streams merge via 64-wide shuffles (cross-group) then LDS (cross-wave);
-//    accumulation entirely in f32.
+//  - a workgroup owns (sequence, kv head, part of the keys); the GQ = Hq/Hkv
+//    query heads of a kv head share its K/V stream, so each KV byte is read
+//    exactly once per step. The keys of a sequence are cut into parts when
+//    (sequences x kv heads) alone leaves CUs without work (decode_splits);
+//    a second kernel joins the parts.
+//  - 4 waves per workgroup, 32 keys (two pages) per wave and step. Scores are
+//    a matrix product, S^T = K Q^T on mfma_f32_16x16x32_bf16: K rows are the
+//    16-byte loads of the A operand as they lie in the page, the GQ query
+//    rows (zero rows up to 16) the B operand. One lane then holds one head's
+//    scores of 8 keys, so maximum and sum take two cross-lane steps per 32
+//    keys instead of four per key.
+//  - probabilities stay fp32: they go through LDS to a layout of 16 lanes a
+//    value row (D/16 channels each) x 4 keys, where the weighted sum is fp32
+//    FMA on values loaded 16 bytes (bf16) or 8 bytes (fp8) a lane.
+//  - fp8 keys become bf16 exactly (e4m3 has 3 mantissa bits) in registers.
 //
-// KV pool layout: [num_blocks, Hkv, BS, D] bf16, BS = 16 tokens.
+// Bound by the K/V stream: 32 keys cost a SIMD about 1300 cycles (GQ = 4),
+// 31 TB/s over the chip in bf16 and 15 TB/s in fp8, so memory sets the time
+// once enough of it is in flight (16 KB a wave, 16 waves a CU).
+//
+// KV pool layout: [num_blocks, Hkv, BS, D] bf16 | fp8, BS = 16 tokens.
 #include "common.h"
 
 #include <type_traits>
@@ -23,12 +34,54 @@ namespace {
 constexpr int BS = 16;       // tokens per KV block (page)
 constexpr int NWAVES = 4;    // waves per workgroup
 constexpr int THREADS = NWAVES * WAVE_SIZE;
+constexpr int STEP = 32;     // keys per wave and step (two pages)
+constexpr float LOG2E = 1.4426950408889634f;
 
-// EXT=false compiles the exact validated fast path (no sinks / window /
-// softcap code at all — bit-identical to the r1/r2-measured kernel);
-// EXT=true carries the GPT-OSS/Gemma feature variants and only ever
-// launches when one of those features is requested.
-template <int D, int GQ, bool FP8, bool EXT = false>
+typedef __attribute__((ext_vector_type(8))) short s16x8;
+typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
+
+// `n` bytes as 32-bit words, loaded in the widest pieces
+template <int WORDS>
+DEVICE_INLINE void load_words(unsigned int* dst, const void* src) {
+  if constexpr (WORDS >= 4) {
+#pragma unroll
+    for (int i = 0; i < WORDS / 4; ++i) {
+      const u32x4 v = reinterpret_cast<const u32x4*>(src)[i];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) dst[i * 4 + j] = v[j];
+    }
+  } else if constexpr (WORDS == 2) {
+    const u32x2 v = *reinterpret_cast<const u32x2*>(src);
+    dst[0] = v[0];
+    dst[1] = v[1];
+  } else {
+    dst[0] = *reinterpret_cast<const unsigned int*>(src);
+  }
+}
+
+// four fp8 -> four f32
+DEVICE_INLINE void fp8x4_f32(unsigned int w, float* o) {
+  const f32x2 a = __builtin_amdgcn_cvt_pk_f32_fp8((int)w, false);
+  const f32x2 b = __builtin_amdgcn_cvt_pk_f32_fp8((int)w, true);
+  o[0] = a[0]; o[1] = a[1]; o[2] = b[0]; o[3] = b[1];
+}
+
+// the high halves of two f32 as one word of bf16 (exact when the low halves
+// are zero)
+DEVICE_INLINE unsigned int pack_hi(float lo, float hi) {
+  return __builtin_amdgcn_perm(__builtin_bit_cast(unsigned int, hi),
+                               __builtin_bit_cast(unsigned int, lo),
+                               0x07060302u);
+}
+
+// keys per part of a sequence of `len` tokens: whole steps, at least 128
+DEVICE_INLINE int part_tokens(int len, int nsplit) {
+  const int per = (len + nsplit - 1) / nsplit;
+  return max((per + STEP - 1) / STEP * STEP, 4 * STEP);
+}
+
+// EXT: sinks / sliding window / softcap (GPT-OSS and Gemma variants).
+template <int D, int GQ, bool FP8, bool EXT>
 __global__ __launch_bounds__(THREADS) void paged_attn_decode_kernel(
     unsigned short* __restrict__ out,        // [N, Hq, D]
     const unsigned short* __restrict__ q,    // [N, Hq, D]
@@ -36,253 +89,295 @@ __global__ __launch_bounds__(THREADS) void paged_attn_decode_kernel(
     const void* __restrict__ vc,             // [B, Hkv, BS, D]
     const int* __restrict__ block_tables,    // [N, max_blocks]
     const int* __restrict__ seq_lens,        // [N]
+    float* __restrict__ part,                // [N, Hkv, nsplit, GQ, D + 2]
     int Hkv, int max_blocks, float scale, long q_stride,
     const float* __restrict__ sinks,         // [Hq] or null (GPT-OSS)
     int window,                              // 0 = full attention
     float softcap) {                         // 0 = off (Gemma-2 tanh cap)
-  constexpr int LPG = 16;           // lanes per token-group
-  constexpr int DV = D / LPG;       // dims per lane (4/8/16 for D 64/128/256)
-  static_assert(DV == 4 || DV == 8 || DV == 16,
-                "decode kernel assumes D in {64, 128, 256}");
-  constexpr int NV = (DV >= 8) ? DV / 8 : 1;  // u16x8 vectors per lane slice
-  // tokens batched per softmax update: trade VALU savings against VGPR
-  // pressure (GQ>=4 would spill at TB=4)
-  constexpr int TB = (GQ <= 2) ? (BS / 4) : ((GQ <= 5) ? 2 : 1);
+  constexpr int DV = D / 16;        // value channels per lane
+  constexpr int ES = FP8 ? 1 : 2;   // bytes per cached number
+  constexpr int QK = D / 32;        // products per 16 keys
+  constexpr int KW = 8 * ES / 4;    // words of a K fragment
+  constexpr int VW = DV * ES / 4;   // words of a lane's value channels
+  constexpr int GP = GQ <= 2 ? GQ : (GQ + 3) / 4 * 4;  // padded P row
+  static_assert(D == 64 || D == 128 || D == 256, "D in {64, 128, 256}");
 
   const int seq = blockIdx.x;
-  const int h = blockIdx.y;        // kv head
+  const int h = blockIdx.y;         // kv head
+  const int nsplit = gridDim.z;
   const int Hq = Hkv * GQ;
   const int len = seq_lens[seq];
-  const int npages = (len + BS - 1) / BS;
+  const int span = part_tokens(len, nsplit);
+  // sliding window (EXT): the query sits at position len - 1 and attends
+  // [max(0, len - window), len)
+  const int wstart = (EXT && window > 0 && len > window) ? len - window : 0;
+  const int t0 = (int)blockIdx.z * span;
+  const int t1 = min(len, t0 + span);
+  if (nsplit > 1 && t0 >= len) return;     // the join skips it as well
 
   const int lane = threadIdx.x & (WAVE_SIZE - 1);
   const int wave = threadIdx.x / WAVE_SIZE;
-  const int g = lane >> 4;         // token-group within wave [0,4)
-  const int sub = lane & 15;       // dim-slice within group [0,16)
+  const int g = lane >> 4;          // key group / k-slot group
+  const int sub = lane & 15;        // head (scores), channel slice (values)
 
-  // Load q rows for this kv head's GQ query heads. bf16 path: keep q PACKED
-  // (u16x8 = 4 VGPRs/head vs 8 for f32) and dot with the native
-  // v_dot2c_f32_bf16 instruction — halves both q/k register pressure and
-  // dot-product instruction count (occupancy was the bottleneck: 2-3
-  // waves/SIMD at 168-200 VGPRs, profiles/r02_optimization_log.md).
-  // fp8 path: f32 q pre-scaled as before (k dequants through f32 anyway).
-  // lane slice = DV dims: one u16x4 (DV=4) or NV u16x8 vectors
-  using U16V = std::conditional_t<DV == 4, u16x4, u16x8>;
-  using U8V = std::conditional_t<DV == 4, u8x4, u8x8>;
-  constexpr int VW = (DV == 4) ? 4 : 8;     // elements per vector
-  float qr[FP8 ? GQ : 1][DV];
-  U16V qb[FP8 ? 1 : GQ][NV];
+  __shared__ float lds_p[NWAVES][STEP][GP];
+  __shared__ float lds_c[NWAVES][GP];
+  __shared__ float lds_acc[NWAVES][GQ][D];
+  __shared__ float lds_ms[NWAVES][GQ][2];
+
+  // Q as the B operand: column `sub` = head, rows g*8 .. g*8+7 of each chunk
+  u16x8 qf[QK];
 #pragma unroll
-  for (int gq = 0; gq < GQ; ++gq) {
-    const unsigned short* qp =
-        q + (long)seq * q_stride + ((long)h * GQ + gq) * D + sub * DV;
-#pragma unroll
-    for (int vv = 0; vv < NV; ++vv) {
-      U16V u = *reinterpret_cast<const U16V*>(qp + vv * VW);
-      if constexpr (FP8) {
-#pragma unroll
-        for (int j = 0; j < VW; ++j)
-          qr[gq][vv * VW + j] = bf2f(u[j]) * scale;
-      } else {
-        qb[gq][vv] = u;
-      }
-    }
+  for (int kk = 0; kk < QK; ++kk) {
+    u16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (sub < GQ)
+      z = *reinterpret_cast<const u16x8*>(
+          q + (long)seq * q_stride + ((long)h * GQ + sub) * D + kk * 32 + g * 8);
+    qf[kk] = z;
   }
 
-  float m[GQ], s[GQ], acc[GQ][DV];
+  float m = -INFINITY, s = 0.f;     // of head `sub`; s: this lane's keys
+  float acc[GQ][DV];
 #pragma unroll
-  for (int gq = 0; gq < GQ; ++gq) {
-    m[gq] = -INFINITY;
-    s[gq] = 0.f;
+  for (int gq = 0; gq < GQ; ++gq)
 #pragma unroll
     for (int j = 0; j < DV; ++j) acc[gq][j] = 0.f;
-  }
 
-  using KVT = std::conditional_t<FP8, unsigned char, unsigned short>;
-  // sliding window (EXT): the single decode query sits at position len-1
-  // and attends [max(0, len-window), len)
-  const int wstart =
-      (EXT && window > 0 && len > window) ? len - window : 0;
-  const int page0 = EXT ? wstart / BS : 0;
+  const char* kbase = reinterpret_cast<const char*>(kc) + (long)h * BS * D * ES;
+  const char* vbase = reinterpret_cast<const char*>(vc) + (long)h * BS * D * ES;
+  const long page_bytes = (long)Hkv * BS * D * ES;
   const int* bt = block_tables + (long)seq * max_blocks;
-  for (int page = page0 + wave; page < npages; page += NWAVES) {
-    const long blk = bt[page];
-    const KVT* kbase = (const KVT*)kc + ((blk * Hkv + h) * BS) * D;
-    const KVT* vbase = (const KVT*)vc + ((blk * Hkv + h) * BS) * D;
-    // Whole page per wave-iteration: the group's 4 tokens are processed
-    // together — 4 independent dots (ILP across the shuffle-reduce
-    // chains), then ONE softmax update per gq for all 4 (cuts the
-    // exp/rescale VALU work ~2.5x vs per-token online updates).
+  const int last_page = (len - 1) / BS;
+  const float sc = scale * LOG2E;
+  const int first = EXT ? max(t0, wstart / STEP * STEP) : t0;
+
+  for (int c0 = first + wave * STEP; c0 < t1; c0 += NWAVES * STEP) {
+    const int page = c0 / BS;
+    long at[2];
 #pragma unroll
-    for (int tb = 0; tb < BS / 4; tb += TB) {
-      const int base_tok = page * BS + tb * 4 + g;
-      using VecT = std::conditional_t<FP8, U8V, U16V>;
-      VecT vu[TB][NV];
-      VecT ku[TB][NV];          // bf16: K stays packed (dot2 consumes it)
-      float kf[FP8 ? TB : 1][DV];  // fp8: K dequanted once, reused per gq
+    for (int p = 0; p < 2; ++p)
+      at[p] = (long)bt[min(page + p, last_page)] * page_bytes;
+    unsigned int kw[2][QK][KW], vw[8][VW];
 #pragma unroll
-      for (int it = 0; it < TB; ++it) {
-        const int tok = (tb + it) * 4 + g;
+    for (int p = 0; p < 2; ++p)
 #pragma unroll
-        for (int vv = 0; vv < NV; ++vv) {
-          ku[it][vv] = *reinterpret_cast<const VecT*>(
-              kbase + tok * D + sub * DV + vv * VW);
-          vu[it][vv] = *reinterpret_cast<const VecT*>(
-              vbase + tok * D + sub * DV + vv * VW);
-          if constexpr (FP8) {
+      for (int kk = 0; kk < QK; ++kk)
+        load_words<KW>(kw[p][kk],
+                       kbase + at[p] + (sub * D + kk * 32 + g * 8) * ES);
 #pragma unroll
-            for (int j = 0; j < VW; ++j)
-              kf[it][vv * VW + j] = fp8_to_f32(ku[it][vv][j]);
+    for (int i = 0; i < 8; ++i)
+      load_words<VW>(vw[i], vbase + at[i / 4] +
+                                (((i & 3) * 4 + g) * D + sub * DV) * ES);
+
+    // scores: lane = head `sub`, keys c0 + p*16 + g*4 + r
+    float x[8];
+    float mx = -INFINITY;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      f32x4 st{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kk = 0; kk < QK; ++kk) {
+        u32x4 a;
+        if constexpr (FP8) {
+#pragma unroll
+          for (int w = 0; w < 2; ++w) {
+            float f[4];
+            fp8x4_f32(kw[p][kk][w], f);
+            a[w * 2] = pack_hi(f[0], f[1]);
+            a[w * 2 + 1] = pack_hi(f[2], f[3]);
           }
+        } else {
+          a = u32x4{kw[p][kk][0], kw[p][kk][1], kw[p][kk][2], kw[p][kk][3]};
         }
+        st = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            __builtin_bit_cast(s16x8, a), __builtin_bit_cast(s16x8, qf[kk]),
+            st, 0, 0, 0);
       }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int tok = c0 + p * 16 + g * 4 + r;
+        float v = st[r] * sc;
+        bool ok = tok < t1;
+        if constexpr (EXT) {
+          if (softcap > 0.f)
+            v = tanhf(st[r] * scale / softcap) * (softcap * LOG2E);
+          ok = ok && tok >= wstart;
+        }
+        v = ok ? v : -INFINITY;
+        x[p * 4 + r] = v;
+        mx = fmaxf(mx, v);
+      }
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE_SIZE));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE_SIZE));
+    const float nm = fmaxf(m, mx);
+    const float base = nm == -INFINITY ? 0.f : nm;
+    const float corr = __builtin_amdgcn_exp2f(m - base);
+    m = nm;
+    s *= corr;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      x[i] = __builtin_amdgcn_exp2f(x[i] - base);
+      s += x[i];
+    }
+    if (sub < GQ) {
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          lds_p[wave][p * 16 + g * 4 + r][sub] = x[p * 4 + r];
+      if (g == 0) lds_c[wave][sub] = corr;
+    }
+    // one wave's LDS operations stay in order; the compiler must keep them so
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (__any(sub < GQ && corr != 1.f)) {
 #pragma unroll
       for (int gq = 0; gq < GQ; ++gq) {
-        float dot[TB];
+        const float c = lds_c[wave][gq];
 #pragma unroll
-        for (int it = 0; it < TB; ++it) {
-          float d = 0.f;
-          if constexpr (FP8) {
-#pragma unroll
-            for (int j = 0; j < DV; ++j) d += qr[gq][j] * kf[it][j];
-          } else {
-            const bf16x2* qa = reinterpret_cast<const bf16x2*>(&qb[gq][0]);
-            const bf16x2* ka = reinterpret_cast<const bf16x2*>(&ku[it][0]);
-#pragma unroll
-            for (int j = 0; j < DV / 2; ++j)
-              d = __builtin_amdgcn_fdot2_f32_bf16(qa[j], ka[j], d, false);
-            d *= scale;  // q not pre-scaled on this path (kept packed)
-          }
-          dot[it] = d;
-        }
-#pragma unroll
-        for (int it = 0; it < TB; ++it)
-          dot[it] = group16_reduce_sum(dot[it]);  // all 16 lanes get the dot
-        float pmax = -INFINITY;
-#pragma unroll
-        for (int it = 0; it < TB; ++it) {
-          if constexpr (EXT) {
-            const int tpos = base_tok + it * 4;
-            const bool valid = tpos < len && tpos >= wstart;
-            float dv = dot[it];
-            if (softcap > 0.f) dv = tanhf(dv / softcap) * softcap;
-            dot[it] = valid ? dv : -INFINITY;
-          } else {
-            const bool valid = base_tok + it * 4 < len;
-            dot[it] = valid ? dot[it] : -INFINITY;
-          }
-          pmax = fmaxf(pmax, dot[it]);
-        }
-        if (pmax == -INFINITY) continue;
-        const float nm = fmaxf(m[gq], pmax);
-        const float corr = __expf(m[gq] - nm);  // exp(-inf - finite) = 0
-        float p[TB];
-        float psum = 0.f;
-#pragma unroll
-        for (int it = 0; it < TB; ++it) {
-          p[it] = (dot[it] == -INFINITY) ? 0.f : __expf(dot[it] - nm);
-          psum += p[it];
-        }
-        s[gq] = s[gq] * corr + psum;
-#pragma unroll
-        for (int j = 0; j < DV; ++j) {
-          float a = acc[gq][j] * corr;
-#pragma unroll
-          for (int it = 0; it < TB; ++it)
-            a += p[it] * (FP8 ? fp8_to_f32(vu[it][j / VW][j % VW])
-                              : bf2f(vu[it][j / VW][j % VW]));
-          acc[gq][j] = a;
-        }
-        m[gq] = nm;
+        for (int j = 0; j < DV; ++j) acc[gq][j] *= c;
       }
     }
+    // values: lane = channels sub*DV .., keys (i/4)*16 + (i%4)*4 + g
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      float pr[GQ], vf[DV];
+#pragma unroll
+      for (int gq = 0; gq < GQ; ++gq)
+        pr[gq] = lds_p[wave][i * 4 + g][gq];
+#pragma unroll
+      for (int w = 0; w < VW; ++w) {
+        if constexpr (FP8) {
+          fp8x4_f32(vw[i][w], vf + w * 4);
+        } else {
+          vf[w * 2] = __builtin_bit_cast(float, vw[i][w] << 16);
+          vf[w * 2 + 1] = __builtin_bit_cast(float, vw[i][w] & 0xffff0000u);
+        }
+      }
+#pragma unroll
+      for (int gq = 0; gq < GQ; ++gq)
+#pragma unroll
+        for (int j = 0; j < DV; ++j) acc[gq][j] += pr[gq] * vf[j];
+    }
+    asm volatile("" ::: "memory");  // P is read before the next step's writes
   }
 
-  // Merge the 4 token-group streams within each wave (butterfly over
-  // lane masks 16 and 32). Lanes with equal `sub` end up identical.
+  // the four key groups of a wave, then the waves
+  s += __shfl_xor(s, 16, WAVE_SIZE);
+  s += __shfl_xor(s, 32, WAVE_SIZE);
 #pragma unroll
-  for (int mask = 16; mask <= 32; mask <<= 1) {
+  for (int gq = 0; gq < GQ; ++gq) {
 #pragma unroll
-    for (int gq = 0; gq < GQ; ++gq) {
-      const float om = __shfl_xor(m[gq], mask, WAVE_SIZE);
-      const float os = __shfl_xor(s[gq], mask, WAVE_SIZE);
-      float oacc[DV];
-#pragma unroll
-      for (int j = 0; j < DV; ++j)
-        oacc[j] = __shfl_xor(acc[gq][j], mask, WAVE_SIZE);
-      const float nm = fmaxf(m[gq], om);
-      if (os > 0.f || s[gq] > 0.f) {
-        const float w1 = (s[gq] > 0.f) ? __expf(m[gq] - nm) : 0.f;
-        const float w2 = (os > 0.f) ? __expf(om - nm) : 0.f;
-        s[gq] = s[gq] * w1 + os * w2;
-#pragma unroll
-        for (int j = 0; j < DV; ++j)
-          acc[gq][j] = acc[gq][j] * w1 + oacc[j] * w2;
-        m[gq] = nm;
-      }
+    for (int j = 0; j < DV; ++j) {
+      float a = acc[gq][j];
+      a += __shfl_xor(a, 16, WAVE_SIZE);
+      a += __shfl_xor(a, 32, WAVE_SIZE);
+      if (g == 0) lds_acc[wave][gq][sub * DV + j] = a;
     }
   }
-
-  // Cross-wave merge through LDS.
-  __shared__ float lds_acc[NWAVES][GQ][D];
-  __shared__ float lds_m[NWAVES][GQ];
-  __shared__ float lds_s[NWAVES][GQ];
-  if (g == 0) {  // one representative lane-group per wave
-#pragma unroll
-    for (int gq = 0; gq < GQ; ++gq) {
-#pragma unroll
-      for (int j = 0; j < DV; ++j) lds_acc[wave][gq][sub * DV + j] = acc[gq][j];
-      if (sub == 0) {
-        lds_m[wave][gq] = m[gq];
-        lds_s[wave][gq] = s[gq];
-      }
-    }
+  if (g == 0 && sub < GQ) {
+    lds_ms[wave][sub][0] = m;
+    lds_ms[wave][sub][1] = s;
   }
   __syncthreads();
 
-  // 256 threads cover (gq, d) output elements.
   for (int u = threadIdx.x; u < GQ * D; u += THREADS) {
     const int gq = u / D;
     const int d = u % D;
     float M = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < NWAVES; ++w)
-      if (lds_s[w][gq] > 0.f) M = fmaxf(M, lds_m[w][gq]);
-    // GPT-OSS attention sink (EXT): a per-head learned logit joins the
-    // softmax DENOMINATOR only (no value contribution)
-    float sden = 0.f;
+    for (int w = 0; w < NWAVES; ++w) M = fmaxf(M, lds_ms[w][gq][0]);
+    float extra = 0.f;
     if constexpr (EXT) {
-      if (sinks != nullptr) {
-        const float sk = sinks[h * GQ + gq];
+      // an attention sink joins the softmax denominator only; with several
+      // parts the join adds it
+      if (sinks != nullptr && nsplit == 1) {
+        const float sk = sinks[h * GQ + gq] * LOG2E;
         M = fmaxf(M, sk);
-        sden = __expf(sk - M);
+        extra = __builtin_amdgcn_exp2f(sk - M);
       }
     }
-    float num = 0.f, den = sden;
+    const float base = M == -INFINITY ? 0.f : M;
+    float num = 0.f, den = extra;
 #pragma unroll
     for (int w = 0; w < NWAVES; ++w) {
-      if (lds_s[w][gq] > 0.f) {
-        const float wt = __expf(lds_m[w][gq] - M);
-        num += wt * lds_acc[w][gq][d];
-        den += wt * lds_s[w][gq];
+      const float wt = __builtin_amdgcn_exp2f(lds_ms[w][gq][0] - base);
+      num += wt * lds_acc[w][gq][d];
+      den += wt * lds_ms[w][gq][1];
+    }
+    if (nsplit == 1) {
+      out[((long)seq * Hq + (long)h * GQ + gq) * D + d] =
+          f2bf(den > 0.f ? num / den : 0.f);
+    } else {
+      float* pp = part + ((((long)seq * Hkv + h) * nsplit + blockIdx.z) * GQ +
+                          gq) * (D + 2);
+      pp[d] = num;
+      if (d == 0) {
+        pp[D] = M;
+        pp[D + 1] = den;
       }
     }
-    out[((long)seq * Hq + (long)h * GQ + gq) * D + d] =
-        f2bf(den > 0.f ? num / den : 0.f);
   }
+}
+
+// Joins the parts of one (sequence, query head): a few KB that the decode
+// kernel left in the L2, bound by the launch.
+template <int D>
+__global__ __launch_bounds__(D) void paged_attn_join_kernel(
+    unsigned short* __restrict__ out,       // [N, Hq, D]
+    const float* __restrict__ part,         // [N, Hkv, nsplit, GQ, D + 2]
+    const int* __restrict__ seq_lens, int GQ, int nsplit,
+    const float* __restrict__ sinks) {
+  const int seq = blockIdx.x, hq = blockIdx.y, Hq = gridDim.y;
+  const int h = hq / GQ, gq = hq % GQ, d = threadIdx.x;
+  const int len = seq_lens[seq];
+  const int span = part_tokens(len, nsplit);
+  const int n = min(nsplit, (len + span - 1) / span);
+  const float* pp = part +
+      (((long)seq * (Hq / GQ) + h) * nsplit * GQ + gq) * (D + 2);
+  const long step = (long)GQ * (D + 2);
+  float M = -INFINITY;
+  for (int i = 0; i < n; ++i) M = fmaxf(M, pp[i * step + D]);
+  float num = 0.f, den = 0.f;
+  if (sinks != nullptr) {
+    const float sk = sinks[hq] * LOG2E;
+    M = fmaxf(M, sk);
+    den = __builtin_amdgcn_exp2f(sk - M);
+  }
+  const float base = M == -INFINITY ? 0.f : M;
+  for (int i = 0; i < n; ++i) {
+    const float wt = __builtin_amdgcn_exp2f(pp[i * step + D] - base);
+    num += wt * pp[i * step + d];
+    den += wt * pp[i * step + D + 1];
+  }
+  out[((long)seq * Hq + hq) * D + d] = f2bf(den > 0.f ? num / den : 0.f);
 }
 
 }  // namespace
 
+// Parts per sequence. 256 CUs hold about 1024 of these workgroups at once:
+// below that the keys are cut until there are about 2048 (two rounds even out
+// unequal lengths), of at least 128 keys each — shorter parts save less than
+// their join costs. max_blocks is the width of the block table, so a captured
+// graph keeps its grid; parts behind a sequence's end return at once.
+int decode_splits(int N, int Hkv, int max_blocks) {
+  const long base = (long)N * Hkv;
+  if (base >= 1024) return 1;
+  long n = (2048 + base - 1) / base;
+  const long most = ((long)max_blocks * BS + 4 * STEP - 1) / (4 * STEP);
+  if (n > most) n = most;
+  return (int)(n < 1 ? 1 : n > 64 ? 64 : n);
+}
+
 void paged_attn_decode_launch(void* out, const void* q, const void* kc,
                               const void* vc, const int* block_tables,
-                              const int* seq_lens, int N, int Hq, int Hkv,
-                              int D, int max_blocks, float scale, long q_stride,
-                              int fp8, const float* sinks, int window,
-                              float softcap, int* err_unsupported,
-                              hipStream_t s) {
+                              const int* seq_lens, float* part, int nsplit,
+                              int N, int Hq, int Hkv, int D, int max_blocks,
+                              float scale, long q_stride, int fp8,
+                              const float* sinks, int window, float softcap,
+                              int* err_unsupported, hipStream_t s) {
   const int GQ = Hq / Hkv;
-  dim3 grid(N, Hkv);
+  dim3 grid(N, Hkv, nsplit);
   dim3 block(THREADS);
   *err_unsupported = 0;
   if (D != 128 && D != 64 && D != 256) { *err_unsupported = 1; return; }
@@ -291,7 +386,7 @@ void paged_attn_decode_launch(void* out, const void* q, const void* kc,
 #define LAUNCH_D(DD, G, F, E)                                                  \
   hipLaunchKernelGGL((paged_attn_decode_kernel<DD, G, F, E>), grid, block, 0,  \
                      s, (unsigned short*)out, (const unsigned short*)q, kc,    \
-                     vc, block_tables, seq_lens, Hkv, max_blocks, scale,       \
+                     vc, block_tables, seq_lens, part, Hkv, max_blocks, scale, \
                      q_stride, sinks, window, softcap)
 #define LAUNCH_GQ2(G, F)                                                       \
   do {                                                                         \
@@ -322,4 +417,13 @@ void paged_attn_decode_launch(void* out, const void* q, const void* kc,
 #undef LAUNCH_GQ
 #undef LAUNCH_GQ2
 #undef LAUNCH_D
+  if (nsplit <= 1) return;
+#define JOIN(DD)                                                              \
+  hipLaunchKernelGGL((paged_attn_join_kernel<DD>), dim3(N, Hq), dim3(DD), 0,  \
+                     s, (unsigned short*)out, part, seq_lens, GQ, nsplit,     \
+                     sinks)
+  if (D == 128) JOIN(128);
+  else if (D == 64) JOIN(64);
+  else JOIN(256);
+#undef JOIN
 }

@@ -12,7 +12,8 @@ void silu_and_mul_launch(void*, const void*, long, int, hipStream_t);
 void reshape_and_cache_launch(const void*, const void*, void*, void*, const long*, int, int, int, int, long, long, int, hipStream_t);
 void greedy_sample_launch(long*, const void*, int, int, hipStream_t);
 void mla_decode_launch(float*, const void*, const void*, const int*, const int*, int, int, int, int, int, int, float, int*, hipStream_t);
-void paged_attn_decode_launch(void*, const void*, const void*, const void*, const int*, const int*, int, int, int, int, int, float, long, int, const float*, int, float, int*, hipStream_t);
+int decode_splits(int, int, int);
+void paged_attn_decode_launch(void*, const void*, const void*, const void*, const int*, const int*, float*, int, int, int, int, int, int, float, long, int, const float*, int, float, int*, hipStream_t);
 void flash_prefill_launch(void*, const void*, const void*, const void*, const int*, const int*, const int*, int, int, int, int, int, float, long, long, long, const float*, int, float, int*, hipStream_t);
 void flash_prefill_paged_launch(void*, const void*, const void*, const void*, const int*, const int*, const int*, const int*, const int*, const int*, int, int, int, int, int, float, long, const float*, int, float, int*, hipStream_t);
 void mfma_probe_launch(float*, const void*, const void*, hipStream_t);
@@ -188,9 +189,17 @@ void paged_attn_decode(at::Tensor out, at::Tensor q, at::Tensor k_cache,
   const int max_blocks = block_tables.size(1);
   const float* sink_ptr = sink_ptr_checked(sinks, Hq);
   int err = 0;
+  const int nsplit = decode_splits(N, Hkv, max_blocks);
+  // this call's own workspace, from the stream's allocator
+  at::Tensor part;
+  if (nsplit > 1)
+    part = at::empty({(long)N * Hq * nsplit * (D + 2)},
+                     out.options().dtype(at::kFloat));
   paged_attn_decode_launch(out.data_ptr(), q.data_ptr(), k_cache.data_ptr(),
                            v_cache.data_ptr(), block_tables.data_ptr<int>(),
-                           seq_lens.data_ptr<int>(), N, Hq, Hkv, D, max_blocks,
+                           seq_lens.data_ptr<int>(),
+                           nsplit > 1 ? part.data_ptr<float>() : nullptr,
+                           nsplit, N, Hq, Hkv, D, max_blocks,
                            (float)scale, qstride,
                            is_fp8_cache(k_cache) ? 1 : 0, sink_ptr,
                            (int)window, (float)softcap, &err, cur_stream(q));

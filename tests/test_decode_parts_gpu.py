@@ -1,0 +1,66 @@
+"""Decode attention whose keys are cut into parts: lengths at the edges of a
+step (32 keys) and of a part (128), every group size, both cache types, and
+batches large enough to stay whole."""
+import math
+
+import pytest
+import torch
+
+pytestmark = [pytest.mark.gpu,
+              pytest.mark.skipif(not torch.cuda.is_available(),
+                                 reason="needs a GPU")]
+
+
+def _reference(q, kc, vc, bt, lens, scale):
+    N, Hq, D = q.shape
+    G = kc.shape[1]
+    out = torch.empty(N, Hq, D, dtype=torch.float64, device=q.device)
+    for i, n in enumerate(lens):
+        j = torch.arange(n, device=q.device)
+        blk = bt[i, j // 16].long()
+        k = kc[blk, :, j % 16].double().repeat_interleave(Hq // G, 1)
+        v = vc[blk, :, j % 16].double().repeat_interleave(Hq // G, 1)
+        p = ((q[i].double() * k).sum(-1) * scale).softmax(0)
+        out[i] = (p[:, :, None] * v).sum(0)
+    return out
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("Hq,Hkv", [(4, 4), (8, 4), (32, 8), (10, 2), (12, 2),
+                                    (28, 4), (32, 4)])
+@pytest.mark.parametrize("lens", [
+    [1], [31, 32, 33], [127, 128, 129], [4095, 1, 300], [2049],
+    [1 + 7 * i for i in range(300)]])
+def test_parts_against_double(fp8, Hq, Hkv, lens):
+    from gpustack_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(len(lens) + Hq + lens[0])
+    maxb = (max(lens) + 15) // 16 + 3
+    need = [(n + 15) // 16 for n in lens]
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    kc = rnd(sum(need) + 1, Hkv, 16, 128).bfloat16()
+    vc = rnd(sum(need) + 1, Hkv, 16, 128).bfloat16()
+    if fp8:
+        kc, vc = kc.to(torch.float8_e4m3fn), vc.to(torch.float8_e4m3fn)
+    pages = torch.randperm(sum(need), generator=g, device="cuda").int()
+    bt = torch.full((len(lens), maxb), sum(need), dtype=torch.int32,
+                    device="cuda")
+    at = 0
+    for i, n in enumerate(need):
+        bt[i, :n] = pages[at:at + n]
+        at += n
+    q = rnd(len(lens), Hq, 128).bfloat16()
+    out = torch.empty_like(q)
+    scale = 1 / math.sqrt(128)
+    ops.paged_attn_decode(out, q, kc, vc, bt,
+                          torch.tensor(lens, dtype=torch.int32,
+                                       device="cuda"), scale)
+    f = lambda t: t.float() if fp8 else t
+    ref = _reference(q, f(kc), f(vc), bt, lens, scale)
+    # the result is rounded to bf16 once (8 significant bits: half a step is at
+    # most 2^-8 of the value);
+    # everything before it is fp32, whose sums over n keys of size <= 5 and
+    # exponentials stay within 1e-5 * 5 of the exact ones
+    err = (out.double() - ref).abs()
+    assert bool((err <= ref.abs() * 2.0 ** -8 + 1e-4).all()), \
+        float((err - ref.abs() * 2.0 ** -8).max())
