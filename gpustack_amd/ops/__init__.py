@@ -186,11 +186,11 @@ def mla_decode(ctx_out, q_cat, lat_cache, block_tables, seq_lens,
     hip.mla_decode(ctx_out, q_cat, lat_cache, block_tables, seq_lens, scale)
 
 
-_PREFILL_BQ = 64
+_PREFILL_BQ = 128
 
 
 def build_prefill_tiles(seq_lens: list[int], device) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-    """Map varlen sequences to fixed 64-row q tiles for the MFMA kernel."""
+    """Map varlen sequences to fixed 128-row q tiles for the MFMA kernel."""
     starts, q0s, lens = [], [], []
     tok = 0
     for L in seq_lens:
@@ -230,7 +230,7 @@ def varlen_prefill_attn(out, q, k, v, seq_lens: list[int], scale: float,
 
 def build_paged_prefill_tiles(seq_starts: list[int], seq_hists: list[int],
                               seq_news: list[int], device):
-    """Map per-seq suffix rows to fixed 64-row q tiles for the paged
+    """Map per-seq suffix rows to fixed 128-row q tiles for the paged
     prefill-with-history kernel (one entry set per (seq, q-tile))."""
     qstart, q0s, hists, news, seqi = [], [], [], [], []
     for i, (st, h, n) in enumerate(zip(seq_starts, seq_hists, seq_news)):

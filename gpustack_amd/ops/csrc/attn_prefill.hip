@@ -1,549 +1,375 @@
-// Varlen causal flash-attention prefill for MI355X (gfx950) on MFMA — v2.
+// Causal flash attention of prompt rows for MI355X (gfx950) on MFMA: whole
+// prompts (keys and values in the step's own rows) and rows behind a cached
+// history (keys and values in the paged pool), one kernel template.
 //
-// Replaces the prefill attention the reference gets from vLLM/SGLang
-// (SURVEY.md §2.9 #1). CDNA4-first structure (not a CUDA port):
+// Replaces the prefill attention the reference gets from vLLM/SGLang.
 //
-//  - mfma_f32_16x16x32_bf16 tiles; wavefront-64 fragment layouts:
-//      A-frag: lane holds A[row = l&15][k = (l>>4)*8 + j]   (u16x8)
-//      B-frag: lane holds B[k = (l>>4)*8 + j][col = l&15]   (u16x8)
-//      C/D  : lane holds D[row = (l>>4)*4 + r][col = l&15]  (f32x4)
-//  - swapped QK^T (S^T = K · Q^T) so BOTH operands are row-contiguous
-//    u16x8 reads (K from LDS, Q from registers).
-//  - K tile LDS-staged with the ((row&7)<<4) byte-XOR swizzle (guide §6 G4).
-//  - V staged TRANSPOSED (VT[D][BK+pad]) so PV B-fragments are b128 reads.
-//  - v2: BK = 64 kv per tile (twice the MFMA work per barrier pair) and
-//    async-stage split (guide T14): each iteration ISSUES the next tile's
-//    global loads into registers BEFORE the MFMA work, then writes them to
-//    LDS after the barrier — HBM latency hides under compute.
-//  - online softmax in f32 registers; per-q-row stats shared via shuffles.
-//  - templated head_dim D in {64, 128} (GPT-OSS is D=64); optional
-//    per-head attention-SINK logits (join the softmax denominator only)
-//    and sliding WINDOW (kvpos in (qpos-window, qpos]), matching
-//    torch_ref._sink_softmax / _window_mask exactly.
+//  - a workgroup owns 128 query rows of one head, 4 waves x 32 rows, and
+//    walks the keys 64 at a time; mfma_f32_32x32x16_bf16, lane layouts
+//      A: lane holds A[row = l&31][k = (l>>5)*8 + j]
+//      B: lane holds B[k = (l>>5)*8 + j][col = l&31]
+//      D: lane holds D[row = 8*(r>>2) + 4*(l>>5) + (r&3)][col = l&31]
+//    (twice the work per LDS byte of the 16x16x32 form).
+//  - S^T = K Q^T, so a lane holds 32 scores of ONE query row: maximum and sum
+//    are in-lane but for one exchange with lane^32, and the rescaling factor
+//    of a row sits in the lanes that hold the row's output.
+//  - O^T = V^T P^T takes P as it lies in the registers: the k slots of a
+//    product are the keys {4h..4h+3, 8+4h..8+4h+3} of 16 (h = l>>5), and V^T
+//    is read in the same order (two 8-byte LDS reads).
+//  - V is transposed on its way into the LDS: a thread loads 4 rows x 8
+//    channels with 16-byte loads, pairs the rows with v_perm and writes eight
+//    4-key units. VT rows have 68 elements and units are XORed with
+//    2 * (d/32): conflict-free writes (32 lanes, 4 x 8-aligned windows) and
+//    reads (17 d mod 32). K rows keep their order, 16-byte chunks XORed with
+//    the row.
+//  - two LDS buffers: the next tile's global loads fly under this tile's
+//    products, one barrier per tile; 66 KB, two workgroups a CU, so one's
+//    exponentials run beside the other's products.
+//  - the running maximum moves only when a row's scores pass it by 2^8: P is
+//    then at most 2^8, which neither bf16 P nor the fp32 sums notice, and the
+//    output is rescaled in few tiles.
+//  - workgroups of one kv head go to one XCD (head order below), whose L2
+//    then holds that head's keys and values; the tiles with the most keys
+//    start first.
 //
-// Tiling: BQ = 64 q rows per workgroup (4 waves x 16 rows), BK = 64 kv.
+// Bound by the products and exponentials together (16 + 16 MFMAs of 32 cycles
+// and 32 exponentials of 16 cycles a wave and tile).
 #include "common.h"
 
 namespace {
 
-constexpr int BQ = 64;
+constexpr int BQ = 128;
 constexpr int BK = 64;
 constexpr int PF_WAVES = 4;
 constexpr int PF_THREADS = PF_WAVES * WAVE_SIZE;
-constexpr int VT_PAD = 4;  // elements; breaks the bank cycle on VT/P rows
-constexpr int NST = BK / 16;       // S^T stiles per tile (4)
-constexpr int KC2 = BK / 32;       // PV k-chunks per tile (2)
+constexpr int VT_ROW = BK + 4;     // elements of a V^T row in the LDS
+constexpr int PP_BS = 16;          // pool block size (tokens per KV block)
+constexpr float LOG2E = 1.4426950408889634f;
+constexpr float SLACK = 8.f;       // see "running maximum" above
 
 typedef __attribute__((ext_vector_type(8))) short s16x8;
+typedef __attribute__((ext_vector_type(16))) float f32x16;
+typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
 
 DEVICE_INLINE f32x4 mfma16x16x32_bf16(u16x8 a, u16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(
       __builtin_bit_cast(s16x8, a), __builtin_bit_cast(s16x8, b), c, 0, 0, 0);
 }
 
-// byte offset of (kv, dbyte) in the swizzled K tile
-template <int D>
-DEVICE_INLINE int kswz(int kv, int dbyte) {
-  return kv * (D * 2) + (dbyte ^ ((kv & 7) << 4));
+DEVICE_INLINE f32x16 mfma32x32x16_bf16(u32x4 a, u32x4 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+      __builtin_bit_cast(s16x8, a), __builtin_bit_cast(s16x8, b), c, 0, 0, 0);
 }
 
-// EXT=false is the exact validated fast path (no sinks/window/softcap
-// code); EXT=true carries the GPT-OSS/Gemma variants. DVK is the VALUE
-// head dim (defaults to D; MLA expand-prefill runs D=192 qk over DVK=128
-// values).
-template <int D, bool EXT = false, int DVK = D>
-__global__ __launch_bounds__(PF_THREADS) void flash_prefill_kernel(
+DEVICE_INLINE unsigned int pack_bf16(float lo, float hi) {
+  const f32x2 v{lo, hi};
+  return __builtin_bit_cast(unsigned int,
+                            __builtin_convertvector(v, bf16x2));
+}
+
+// EXT: sinks / sliding window / softcap. PAGED: k / v are pools
+// [nblocks, Hkv, 16, D]; otherwise rows of the batch.
+// A tile: the sequence's first row in q and out, the tile's first row within
+// the sequence's rows, the cached tokens in front of them, their number, and
+// the sequence's row of the block tables.
+template <int D, int DVK, bool EXT, bool PAGED>
+__global__ __launch_bounds__(PF_THREADS, D > 128 ? 1 : 2)
+void flash_prefill_kernel(
     unsigned short* __restrict__ out,      // [T, Hq, DVK]
     const unsigned short* __restrict__ q,  // [T, Hq, D]
-    const unsigned short* __restrict__ k,  // [T, Hkv, D]
-    const unsigned short* __restrict__ v,  // [T, Hkv, DVK]
-    const int* __restrict__ tile_start,    // [ntiles] seq start (global row)
-    const int* __restrict__ tile_q0,       // [ntiles] q-tile offset in seq
-    const int* __restrict__ tile_len,      // [ntiles] seq length
-    int Hq, int Hkv, float scale,
+    const unsigned short* __restrict__ k,
+    const unsigned short* __restrict__ v,
+    const int* __restrict__ block_tables,  // [nseq, maxb]
+    const int* __restrict__ tile_start, const int* __restrict__ tile_q0,
+    const int* __restrict__ tile_hist, const int* __restrict__ tile_new,
+    const int* __restrict__ tile_seq,
+    int Hq, int Hkv, int maxb, float scale,
     long qs, long ks, long vs,             // row strides (elements)
     const float* __restrict__ sinks,       // [Hq] or null
     int window,                            // 0 = full causal
     float softcap) {                       // 0 = off (Gemma-2 tanh cap)
-  constexpr int KU = BK * (D / 8) / PF_THREADS;    // K u16x8 units/thread
-  constexpr int VU = DVK * (BK / 8) / PF_THREADS;  // VT units/thread
-  constexpr int QK = D / 32;                       // q k-chunks
-  const int tile = blockIdx.x;
-  const int qh = blockIdx.y;
+  constexpr int CH = D / 8;                // 16-byte chunks of a key row
+  constexpr int KU = CH / 4;               // K chunks a lane stages
+  constexpr int VB = (DVK / 8 * 4 + 63) / 64;  // V blocks a lane stages
+  constexpr int KMASK = D % 128 == 0 ? 15 : 7;
+  constexpr int QK = D / 16;
+  constexpr int NT = DVK / 32;
+  constexpr int K_ELEMS = BK * D;
+  constexpr int BUF = K_ELEMS + DVK * VT_ROW;
+
+  static_assert(2 * BUF >= BQ * DVK, "the output goes through the buffers");
+  __shared__ __attribute__((aligned(16))) unsigned short lds[2 * BUF];
+
+  // heads of one kv head on one XCD (workgroups go round the 8 XCDs)
+  int qh = blockIdx.x % Hq;
+  if (Hq % 8 == 0) qh = (qh % 8) * (Hq / 8) + qh / 8;
+  const int tile = (gridDim.x - 1 - blockIdx.x) / Hq;
   const int kvh = qh / (Hq / Hkv);
-  const int seq0 = tile_start[tile];
+  const int row0 = tile_start[tile];
   const int q0 = tile_q0[tile];
-  const int len = tile_len[tile];
+  const int hist = PAGED ? tile_hist[tile] : 0;
+  const int nnew = tile_new[tile];
+  const int len = hist + nnew;
+  const int* bt = PAGED ? block_tables + (long)tile_seq[tile] * maxb : nullptr;
 
   const int lane = threadIdx.x & (WAVE_SIZE - 1);
-  const int wave = threadIdx.x / WAVE_SIZE;
-  const int lc = lane & 15;        // column / row-id within 16
-  const int lg = lane >> 4;        // 4-lane group id
-  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
+  const int lc = lane & 31;
+  const int hf = lane >> 5;
 
-  __shared__ unsigned short Kl[BK * D];            // swizzled
-  __shared__ unsigned short VTl[DVK][BK + VT_PAD]; // transposed V
-  __shared__ unsigned short Pl[PF_WAVES][16][BK + VT_PAD];
-
-  // Hoist this wave's 16 q rows into B-fragments (QK k-chunks of 32).
-  const int qrow_local = q0 + wave * 16 + lc;
-  const int qrow_clamped = (qrow_local < len) ? qrow_local : (len - 1);
-  u16x8 qfrag[QK];
+  // this wave's 32 query rows as the B operand
+  const int qrow = q0 + wave * 32 + lc;            // within the new rows
+  const int qpos = hist + qrow;
+  u32x4 qf[QK];
+  {
+    const unsigned short* qp =
+        q + (long)(row0 + min(qrow, nnew - 1)) * qs + (long)qh * D + hf * 8;
 #pragma unroll
-  for (int kk = 0; kk < QK; ++kk) {
-    const unsigned short* qp = q + (long)(seq0 + qrow_clamped) * qs +
-                               (long)qh * D + kk * 32 + lg * 8;
-    qfrag[kk] = *reinterpret_cast<const u16x8*>(qp);
+    for (int kk = 0; kk < QK; ++kk)
+      qf[kk] = *reinterpret_cast<const u32x4*>(qp + kk * 16);
   }
 
-  float mcol = -INFINITY;  // running max for q row `lc` (this wave)
-  float lcol = 0.f;        // running denom for q row `lc`
-  f32x4 o[DVK / 16];       // O[q=(lg*4+r)][d=lc+nt*16]
+  float m = -INFINITY, l = 0.f;
+  f32x16 o[NT];
 #pragma unroll
-  for (int nt = 0; nt < DVK / 16; ++nt) o[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[t][r] = 0.f;
 
-  const int q_hi = q0 + BQ - 1;
-  const int kv_end = min(len, q_hi + 1);           // causal bound
-  const int ntiles_kv = (kv_end + BK - 1) / BK;
-  const int wave_q_hi = q0 + wave * 16 + 15;       // this wave's causal bound
-  const int wave_q_lo = q0 + wave * 16;            // lowest window start
+  const int lo_wave = hist + q0 + wave * 32;       // this wave's first row
+  const int kv_end = min(len, hist + q0 + BQ);     // causal bound
+  const int kt_end = (kv_end + BK - 1) / BK;
+  // the first tile any row of the workgroup can see
+  int kt0 = 0;
+  if constexpr (EXT)
+    if (window > 0) kt0 = max(0, hist + q0 - window + 1) / BK;
 
-  // staging assignment (fixed per thread):
-  //   K: unit u = tid + r*256 -> (kv = u/(D/8), d0 = (u%(D/8))*8)
-  //   VT: unit u -> (d = u%D, kvc = (u/D)*8)
-  int kst_kv[KU];
-#pragma unroll
-  for (int r = 0; r < KU; ++r) kst_kv[r] = (tid + r * PF_THREADS) / (D / 8);
-  const int kst_d0 = (tid % (D / 8)) * 8;
-  const int vst_d = tid % DVK;
-  const int vst_kvc0 = (tid / DVK) * 8;  // + r*(8*PF_THREADS/DVK) per round
-  constexpr int VST_STEP = 8 * PF_THREADS / DVK;
+  u32x4 kst[KU], vst[VB][4];
 
-  u16x8 kstage[KU];
-  unsigned short vstage[VU][8];
-
-  auto issue_loads = [&](int kv0) {
-#pragma unroll
-    for (int r = 0; r < KU; ++r) {
-      const int kv = kv0 + kst_kv[r];
-      kstage[r] = (kv < len)
-          ? *reinterpret_cast<const u16x8*>(
-                k + (long)(seq0 + kv) * ks + (long)kvh * D + kst_d0)
-          : u16x8{0, 0, 0, 0, 0, 0, 0, 0};
-    }
-#pragma unroll
-    for (int r = 0; r < VU; ++r) {
-      const int kvc = vst_kvc0 + r * VST_STEP;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int kv = kv0 + kvc + j;
-        vstage[r][j] = (kv < len)
-            ? v[(long)(seq0 + kv) * vs + (long)kvh * DVK + vst_d]
-            : (unsigned short)0;
-      }
-    }
-  };
-
-  auto write_lds = [&]() {
-#pragma unroll
-    for (int r = 0; r < KU; ++r) {
-      *reinterpret_cast<u16x8*>(reinterpret_cast<char*>(Kl) +
-                                kswz<D>(kst_kv[r], kst_d0 * 2)) = kstage[r];
-    }
-#pragma unroll
-    for (int r = 0; r < VU; ++r) {
-      *reinterpret_cast<u16x8*>(&VTl[vst_d][vst_kvc0 + r * VST_STEP]) =
-          *reinterpret_cast<u16x8*>(vstage[r]);
-    }
-  };
-
-  issue_loads(0);
-  for (int kt = 0; kt < ntiles_kv; ++kt) {
-    const int kv0 = kt * BK;
-    __syncthreads();   // previous tile's LDS reads are done
-    write_lds();
-    __syncthreads();   // tile ready
-    if (kt + 1 < ntiles_kv) issue_loads(kv0 + BK);  // hide HBM under MFMA
-
-    if (kv0 > wave_q_hi) continue;  // fully masked for this wave
-    // sliding window (EXT): tile entirely below every row's window
-    if (EXT && window > 0 && kv0 + BK <= wave_q_lo - window + 1) continue;
-
-    // ---- S^T = K · Q^T  (NST stiles x QK k-chunks) ----
-    f32x4 st[NST];
-#pragma unroll
-    for (int i = 0; i < NST; ++i) st[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int stile = 0; stile < NST; ++stile) {
-#pragma unroll
-      for (int kk = 0; kk < QK; ++kk) {
-        const u16x8 a = *reinterpret_cast<const u16x8*>(
-            reinterpret_cast<char*>(Kl) +
-            kswz<D>(stile * 16 + lc, (kk * 32 + lg * 8) * 2));
-        st[stile] = mfma16x16x32_bf16(a, qfrag[kk], st[stile]);
-      }
-    }
-
-    // ---- mask + online softmax (stats per q row lc) ----
-    const int qpos = q0 + wave * 16 + lc;
-    float sv[NST * 4];
-    float tmax = -INFINITY;
-#pragma unroll
-    for (int stile = 0; stile < NST; ++stile) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int kvpos = kv0 + stile * 16 + lg * 4 + r;
-        float x = st[stile][r] * scale;
-        bool ok = (kvpos <= qpos) && (kvpos < len) && (qpos < len);
-        if constexpr (EXT) {
-          if (softcap > 0.f) x = tanhf(x / softcap) * softcap;
-          if (window > 0) ok = ok && (kvpos > qpos - window);
-        }
-        x = ok ? x : -INFINITY;
-        sv[stile * 4 + r] = x;
-        tmax = fmaxf(tmax, x);
-      }
-    }
-#pragma unroll
-    for (int msk = 16; msk <= 32; msk <<= 1)
-      tmax = fmaxf(tmax, __shfl_xor(tmax, msk, WAVE_SIZE));
-
-    const float nm = fmaxf(mcol, tmax);
-    float corr = 1.f, tsum = 0.f;
-    float pv[NST * 4];
-    if (nm != -INFINITY) {
-      corr = __expf(mcol - nm);
-#pragma unroll
-      for (int i = 0; i < NST * 4; ++i) {
-        pv[i] = (sv[i] == -INFINITY) ? 0.f : __expf(sv[i] - nm);
-        tsum += pv[i];
-      }
-      mcol = nm;
+  // wave w stages rows 16 w .. 16 w + 15 of a tile (one page of a pool)
+  auto issue = [&](int kt) {
+    const int kv0 = kt * BK + wave * 16;
+    const unsigned short *kp, *vp;
+    long kstep, vstep;
+    int last;                                      // rows behind it repeat it
+    if constexpr (PAGED) {
+      const int page = min(kv0, len - 1) / PP_BS;
+      const long at = ((long)bt[page] * Hkv + kvh) * PP_BS;
+      kp = k + at * D;
+      vp = v + at * DVK;
+      kstep = D;
+      vstep = DVK;
+      last = PP_BS - 1;
     } else {
-#pragma unroll
-      for (int i = 0; i < NST * 4; ++i) pv[i] = 0.f;
+      const int r = min(kv0, len - 1);
+      kp = k + (long)(row0 + r) * ks + (long)kvh * D;
+      vp = v + (long)(row0 + r) * vs + (long)kvh * DVK;
+      kstep = ks;
+      vstep = vs;
+      last = min(15, len - 1 - r);
     }
 #pragma unroll
-    for (int msk = 16; msk <= 32; msk <<= 1)
-      tsum += __shfl_xor(tsum, msk, WAVE_SIZE);
-    lcol = lcol * corr + tsum;
-
-    // ---- stage P (bf16) into this wave's LDS buffer: P[q=lc][kv] ----
+    for (int i = 0; i < KU; ++i) {
+      const int u = lane + i * WAVE_SIZE;
+      kst[i] = *reinterpret_cast<const u32x4*>(
+          kp + min(u / CH, last) * kstep + (u % CH) * 8);
+    }
 #pragma unroll
-    for (int stile = 0; stile < NST; ++stile) {
+    for (int b = 0; b < VB; ++b) {
+      const int u = lane + b * WAVE_SIZE;
+      if (DVK >= 128 || u < DVK / 2) {
+        const int r0 = u / (DVK / 8) * 4, d0 = u % (DVK / 8) * 8;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        Pl[wave][lc][stile * 16 + lg * 4 + r] = f2bf(pv[stile * 4 + r]);
+        for (int j = 0; j < 4; ++j) {
+          vst[b][j] = *reinterpret_cast<const u32x4*>(
+              vp + min(r0 + j, last) * vstep + d0);
+          // a page's rows behind the sequence's end are not the sequence's
+          if (PAGED && kv0 + r0 + j >= len) vst[b][j] = u32x4{0, 0, 0, 0};
+        }
       }
     }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  };
 
-    // ---- rescale O by this tile's correction (row-matched via shuffle) ----
+  auto stash = [&](unsigned short* buf) {
+    unsigned short* vt = buf + K_ELEMS;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int orow = lg * 4 + r;
-      const float c = __shfl(corr, orow, WAVE_SIZE);
-#pragma unroll
-      for (int nt = 0; nt < DVK / 16; ++nt) o[nt][r] *= c;
+    for (int i = 0; i < KU; ++i) {
+      const int u = lane + i * WAVE_SIZE;
+      const int row = wave * 16 + u / CH;
+      *reinterpret_cast<u32x4*>(
+          buf + row * D + (((u % CH) ^ (row & KMASK)) * 8)) = kst[i];
     }
-
-    // ---- O += P · V  (A = P from LDS, B = V^T rows from LDS) ----
 #pragma unroll
-    for (int kk2 = 0; kk2 < KC2; ++kk2) {
-      const u16x8 pa = *reinterpret_cast<const u16x8*>(
-          &Pl[wave][lc][kk2 * 32 + lg * 8]);
+    for (int b = 0; b < VB; ++b) {
+      const int u = lane + b * WAVE_SIZE;
+      if (DVK >= 128 || u < DVK / 2) {
+        const int unit = wave * 4 + u / (DVK / 8), d0 = u % (DVK / 8) * 8;
+        unsigned short* at =
+            vt + d0 * VT_ROW + (unit ^ (2 * ((d0 >> 5) & 3))) * 4;
 #pragma unroll
-      for (int nt = 0; nt < DVK / 16; ++nt) {
-        const u16x8 b = *reinterpret_cast<const u16x8*>(
-            &VTl[nt * 16 + lc][kk2 * 32 + lg * 8]);
-        o[nt] = mfma16x16x32_bf16(pa, b, o[nt]);
+        for (int w = 0; w < 4; ++w) {
+          // channels 2w and 2w + 1 of four rows
+          u32x2 e, f;
+          e[0] = __builtin_amdgcn_perm(vst[b][1][w], vst[b][0][w], 0x05040100u);
+          e[1] = __builtin_amdgcn_perm(vst[b][3][w], vst[b][2][w], 0x05040100u);
+          f[0] = __builtin_amdgcn_perm(vst[b][1][w], vst[b][0][w], 0x07060302u);
+          f[1] = __builtin_amdgcn_perm(vst[b][3][w], vst[b][2][w], 0x07060302u);
+          *reinterpret_cast<u32x2*>(at + (2 * w) * VT_ROW) = e;
+          *reinterpret_cast<u32x2*>(at + (2 * w + 1) * VT_ROW) = f;
+        }
       }
     }
+  };
+
+  const float sc = scale * LOG2E;
+  issue(kt0);
+  stash(lds);
+  __syncthreads();
+  for (int kt = kt0; kt < kt_end; ++kt) {
+    const int kv0 = kt * BK;
+    const unsigned short* kl = lds + ((kt - kt0) & 1) * BUF;
+    const unsigned short* vt = kl + K_ELEMS;
+    const bool more = kt + 1 < kt_end;
+    if (more) issue(kt + 1);
+
+    bool live = kv0 <= lo_wave + 31;               // not above the diagonal
+    if constexpr (EXT)
+      live = live && !(window > 0 && kv0 + BK <= lo_wave - window + 1);
+    if (live) {
+      f32x16 st[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) st[t][r] = 0.f;
+        const int row = t * 32 + lc;
+#pragma unroll
+        for (int kk = 0; kk < QK; ++kk) {
+          const u32x4 a = *reinterpret_cast<const u32x4*>(
+              kl + row * D + (((kk * 2 + hf) ^ (row & KMASK)) * 8));
+          st[t] = mfma32x32x16_bf16(a, qf[kk], st[t]);
+        }
+      }
+      // scores in powers of two
+      bool edge = kv0 + BK - 1 > lo_wave || kv0 + BK > len;
+      if constexpr (EXT) edge = edge || window > 0;
+      float mx = -INFINITY;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          float x = st[t][r] * sc;
+          if constexpr (EXT)
+            if (softcap > 0.f)
+              x = tanhf(st[t][r] * scale / softcap) * (softcap * LOG2E);
+          if (edge) {
+            const int kv = kv0 + t * 32 + 8 * (r >> 2) + 4 * hf + (r & 3);
+            bool ok = kv <= qpos && kv < len;
+            if constexpr (EXT) ok = ok && (window <= 0 || kv > qpos - window);
+            x = ok ? x : -INFINITY;
+          }
+          st[t][r] = x;
+          mx = fmaxf(mx, x);
+        }
+      mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE_SIZE));
+      if (__any(mx > m + SLACK)) {
+        const float nm = fmaxf(m, mx);
+        const float corr =
+            nm == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - nm);
+        m = nm;
+        l *= corr;
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[t][r] *= corr;
+      }
+      const float base = m == -INFINITY ? 0.f : m;
+      u32x4 pf[4];
+      float sum = 0.f;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const float a = __builtin_amdgcn_exp2f(
+              st[t >> 1][(t & 1) * 8 + w * 2] - base);
+          const float b = __builtin_amdgcn_exp2f(
+              st[t >> 1][(t & 1) * 8 + w * 2 + 1] - base);
+          sum += a + b;
+          pf[t][w] = pack_bf16(a, b);
+        }
+      l += sum;
+      // O^T += V^T P^T
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+          const unsigned short* at = vt + (n * 32 + lc) * VT_ROW;
+          const u32x2 a = *reinterpret_cast<const u32x2*>(
+              at + ((t * 4 + hf) ^ (2 * (n & 3))) * 4);
+          const u32x2 b = *reinterpret_cast<const u32x2*>(
+              at + ((t * 4 + 2 + hf) ^ (2 * (n & 3))) * 4);
+          o[n] = mfma32x32x16_bf16(u32x4{a[0], a[1], b[0], b[1]}, pf[t], o[n]);
+        }
+    }
+    if (more) stash(lds + ((kt - kt0 + 1) & 1) * BUF);
+    __syncthreads();
   }
 
-  // ---- epilogue: normalize rows and write; the SINK logit joins the
-  // denominator only (GPT-OSS: its probability mass drops, no value) ----
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int orow = lg * 4 + r;
-    float denom = __shfl(lcol, orow, WAVE_SIZE);
-    float onum = 1.f;
-    if constexpr (EXT) {
-      if (sinks != nullptr) {
-        const float m_row = __shfl(mcol, orow, WAVE_SIZE);
-        const float sk = sinks[qh];
-        const float M2 = fmaxf(m_row, sk);
-        onum = (m_row == -INFINITY) ? 0.f : __expf(m_row - M2);
-        denom = denom * onum + __expf(sk - M2);
-      }
+  // normalise; a SINK logit joins the denominator only
+  l += __shfl_xor(l, 32, WAVE_SIZE);
+  float num = 1.f;
+  if constexpr (EXT) {
+    if (sinks != nullptr) {
+      const float sk = sinks[qh] * LOG2E;
+      const float M = fmaxf(m, sk);
+      num = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - M);
+      l = l * num + __builtin_amdgcn_exp2f(sk - M);
     }
-    const int qrow = q0 + wave * 16 + orow;
-    if (qrow >= len || denom <= 0.f) continue;
-    const float inv = onum / denom;
+  }
+  const float inv = l > 0.f ? num / l : 0.f;
+  // through the LDS to whole rows: unit u (4 channels) of row r at
+  // u ^ (r & 15), each wave its own 32 rows
+  unsigned short* ol = lds + wave * 32 * DVK;
 #pragma unroll
-    for (int nt = 0; nt < DVK / 16; ++nt) {
-      out[((long)(seq0 + qrow) * Hq + qh) * DVK + nt * 16 + lc] =
-          f2bf(o[nt][r] * inv);
+  for (int n = 0; n < NT; ++n)
+#pragma unroll
+    for (int rr = 0; rr < 4; ++rr) {
+      u32x2 w;
+      w[0] = pack_bf16(o[n][rr * 4] * inv, o[n][rr * 4 + 1] * inv);
+      w[1] = pack_bf16(o[n][rr * 4 + 2] * inv, o[n][rr * 4 + 3] * inv);
+      const int unit = n * 8 + rr * 2 + hf;
+      *reinterpret_cast<u32x2*>(ol + lc * DVK + (unit ^ (lc & 15)) * 4) = w;
     }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  constexpr int OC = DVK / 8;              // 16-byte chunks of an output row
+#pragma unroll
+  for (int i = 0; i < OC / 2; ++i) {
+    const int u = lane + i * WAVE_SIZE;
+    const int r = u / OC, c = u % OC;
+    const u32x2 a = *reinterpret_cast<const u32x2*>(
+        ol + r * DVK + ((2 * c) ^ (r & 15)) * 4);
+    const u32x2 b = *reinterpret_cast<const u32x2*>(
+        ol + r * DVK + ((2 * c + 1) ^ (r & 15)) * 4);
+    const int row = q0 + wave * 32 + r;
+    if (row < nnew)
+      *reinterpret_cast<u32x4*>(
+          out + ((long)(row0 + row) * Hq + qh) * DVK + c * 8) =
+          u32x4{a[0], a[1], b[0], b[1]};
   }
 }
 
-}  // namespace
-
-// ---------------------------------------------------------------------------
-// Prefill-with-history: same MFMA flash structure, but the K/V stream is
-// gathered block-wise from the PAGED pool ([nblocks, Hkv, 16, D] bf16)
-// through the sequence's block table. Used for prefix-cache suffixes and
-// chunked-prefill continuations, whose rows previously ran as paged-decode
-// rows at ~3.5x the attention cost (profiles/r03 chunked A/B) — the
-// measured round-1 penalty this kernel removes. The new tokens' K/V are
-// already scattered into the pool (reshape_and_cache runs before
-// attention), so ALL positions stream from the pool uniformly.
-// ---------------------------------------------------------------------------
-namespace {
-
-constexpr int PP_BS = 16;  // pool block size (tokens per KV block)
-
-template <int D, bool EXT = false>
-__global__ __launch_bounds__(PF_THREADS) void flash_prefill_paged_kernel(
-    unsigned short* __restrict__ out,      // [T, Hq, D] (suffix rows)
-    const unsigned short* __restrict__ q,  // [T, Hq, D] (suffix rows)
-    const unsigned short* __restrict__ kc, // [nblocks, Hkv, BS, D]
-    const unsigned short* __restrict__ vc, // [nblocks, Hkv, BS, D]
-    const int* __restrict__ block_tables,  // [nseq, maxb]
-    const int* __restrict__ tile_qstart,   // [ntiles] seq's first row in q/out
-    const int* __restrict__ tile_q0,       // [ntiles] q-tile offset in suffix
-    const int* __restrict__ tile_hist,     // [ntiles] cached tokens (history)
-    const int* __restrict__ tile_new,      // [ntiles] suffix length
-    const int* __restrict__ tile_seq,      // [ntiles] row into block_tables
-    int Hq, int Hkv, int maxb, float scale, long qs,
-    const float* __restrict__ sinks,       // [Hq] or null
-    int window,                            // 0 = full causal
-    float softcap) {                       // 0 = off (Gemma-2 tanh cap)
-  constexpr int KU = BK * (D / 8) / PF_THREADS;
-  constexpr int VU = D * (BK / 8) / PF_THREADS;
-  constexpr int QK = D / 32;
-  const int tile = blockIdx.x;
-  const int qh = blockIdx.y;
-  const int kvh = qh / (Hq / Hkv);
-  const int qstart = tile_qstart[tile];
-  const int q0 = tile_q0[tile];
-  const int hist = tile_hist[tile];
-  const int nnew = tile_new[tile];
-  const int len = hist + nnew;  // total context length
-  const int* bt = block_tables + (long)tile_seq[tile] * maxb;
-
-  const int lane = threadIdx.x & (WAVE_SIZE - 1);
-  const int wave = threadIdx.x / WAVE_SIZE;
-  const int lc = lane & 15;
-  const int lg = lane >> 4;
-  const int tid = threadIdx.x;
-
-  __shared__ unsigned short Kl[BK * D];
-  __shared__ unsigned short VTl[D][BK + VT_PAD];
-  __shared__ unsigned short Pl[PF_WAVES][16][BK + VT_PAD];
-
-  const int qrow_local = q0 + wave * 16 + lc;           // row within suffix
-  const int qrow_clamped = (qrow_local < nnew) ? qrow_local : (nnew - 1);
-  u16x8 qfrag[QK];
-#pragma unroll
-  for (int kk = 0; kk < QK; ++kk) {
-    const unsigned short* qp = q + (long)(qstart + qrow_clamped) * qs +
-                               (long)qh * D + kk * 32 + lg * 8;
-    qfrag[kk] = *reinterpret_cast<const u16x8*>(qp);
-  }
-
-  float mcol = -INFINITY;
-  float lcol = 0.f;
-  f32x4 o[D / 16];
-#pragma unroll
-  for (int nt = 0; nt < D / 16; ++nt) o[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const int q_hi_abs = hist + q0 + BQ - 1;              // absolute position
-  const int kv_end = min(len, q_hi_abs + 1);
-  const int ntiles_kv = (kv_end + BK - 1) / BK;
-  const int wave_q_hi_abs = hist + q0 + wave * 16 + 15;
-  const int wave_q_lo_abs = hist + q0 + wave * 16;
-
-  int kst_kv[KU];
-#pragma unroll
-  for (int r = 0; r < KU; ++r) kst_kv[r] = (tid + r * PF_THREADS) / (D / 8);
-  const int kst_d0 = (tid % (D / 8)) * 8;
-  const int vst_d = tid % D;
-  const int vst_kvc0 = (tid / D) * 8;
-  constexpr int VST_STEP = 8 * PF_THREADS / D;
-
-  u16x8 kstage[KU];
-  unsigned short vstage[VU][8];
-
-  // pool row base (elements) for token position `kv`
-  auto pool_row = [&](int kv) {
-    const int blk = bt[kv / PP_BS];
-    return (((long)blk * Hkv + kvh) * PP_BS + kv % PP_BS) * D;
-  };
-
-  auto issue_loads = [&](int kv0) {
-    // clamp BEFORE the block-table lookup: a speculated address compute
-    // for masked-out lanes must not index past the table row
-#pragma unroll
-    for (int r = 0; r < KU; ++r) {
-      const int kv = kv0 + kst_kv[r];
-      const bool ok = kv < len;
-      const u16x8 val = *reinterpret_cast<const u16x8*>(
-          kc + pool_row(ok ? kv : len - 1) + kst_d0);
-      kstage[r] = ok ? val : u16x8{0, 0, 0, 0, 0, 0, 0, 0};
-    }
-#pragma unroll
-    for (int r = 0; r < VU; ++r) {
-      const int kvc = vst_kvc0 + r * VST_STEP;
-      // 8 consecutive positions span at most 2 pool blocks; resolving the
-      // row base per element keeps the gather exact at block boundaries
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int kv = kv0 + kvc + j;
-        const bool ok = kv < len;
-        const unsigned short val = vc[pool_row(ok ? kv : len - 1) + vst_d];
-        vstage[r][j] = ok ? val : (unsigned short)0;
-      }
-    }
-  };
-
-  auto write_lds = [&]() {
-#pragma unroll
-    for (int r = 0; r < KU; ++r) {
-      *reinterpret_cast<u16x8*>(reinterpret_cast<char*>(Kl) +
-                                kswz<D>(kst_kv[r], kst_d0 * 2)) = kstage[r];
-    }
-#pragma unroll
-    for (int r = 0; r < VU; ++r) {
-      *reinterpret_cast<u16x8*>(&VTl[vst_d][vst_kvc0 + r * VST_STEP]) =
-          *reinterpret_cast<u16x8*>(vstage[r]);
-    }
-  };
-
-  issue_loads(0);
-  for (int kt = 0; kt < ntiles_kv; ++kt) {
-    const int kv0 = kt * BK;
-    __syncthreads();
-    write_lds();
-    __syncthreads();
-    if (kt + 1 < ntiles_kv) issue_loads(kv0 + BK);
-
-    if (kv0 > wave_q_hi_abs) continue;
-    if (EXT && window > 0 && kv0 + BK <= wave_q_lo_abs - window + 1)
-      continue;
-
-    f32x4 st[NST];
-#pragma unroll
-    for (int i = 0; i < NST; ++i) st[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int stile = 0; stile < NST; ++stile) {
-#pragma unroll
-      for (int kk = 0; kk < QK; ++kk) {
-        const u16x8 a = *reinterpret_cast<const u16x8*>(
-            reinterpret_cast<char*>(Kl) +
-            kswz<D>(stile * 16 + lc, (kk * 32 + lg * 8) * 2));
-        st[stile] = mfma16x16x32_bf16(a, qfrag[kk], st[stile]);
-      }
-    }
-
-    const int qpos = hist + q0 + wave * 16 + lc;  // absolute position
-    const bool qvalid = (q0 + wave * 16 + lc) < nnew;
-    float sv[NST * 4];
-    float tmax = -INFINITY;
-#pragma unroll
-    for (int stile = 0; stile < NST; ++stile) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int kvpos = kv0 + stile * 16 + lg * 4 + r;
-        float x = st[stile][r] * scale;
-        bool ok = (kvpos <= qpos) && (kvpos < len) && qvalid;
-        if constexpr (EXT) {
-          if (softcap > 0.f) x = tanhf(x / softcap) * softcap;
-          if (window > 0) ok = ok && (kvpos > qpos - window);
-        }
-        x = ok ? x : -INFINITY;
-        sv[stile * 4 + r] = x;
-        tmax = fmaxf(tmax, x);
-      }
-    }
-#pragma unroll
-    for (int msk = 16; msk <= 32; msk <<= 1)
-      tmax = fmaxf(tmax, __shfl_xor(tmax, msk, WAVE_SIZE));
-
-    const float nm = fmaxf(mcol, tmax);
-    float corr = 1.f, tsum = 0.f;
-    float pv[NST * 4];
-    if (nm != -INFINITY) {
-      corr = __expf(mcol - nm);
-#pragma unroll
-      for (int i = 0; i < NST * 4; ++i) {
-        pv[i] = (sv[i] == -INFINITY) ? 0.f : __expf(sv[i] - nm);
-        tsum += pv[i];
-      }
-      mcol = nm;
-    } else {
-#pragma unroll
-      for (int i = 0; i < NST * 4; ++i) pv[i] = 0.f;
-    }
-#pragma unroll
-    for (int msk = 16; msk <= 32; msk <<= 1)
-      tsum += __shfl_xor(tsum, msk, WAVE_SIZE);
-    lcol = lcol * corr + tsum;
-
-#pragma unroll
-    for (int stile = 0; stile < NST; ++stile) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        Pl[wave][lc][stile * 16 + lg * 4 + r] = f2bf(pv[stile * 4 + r]);
-      }
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int orow = lg * 4 + r;
-      const float c = __shfl(corr, orow, WAVE_SIZE);
-#pragma unroll
-      for (int nt = 0; nt < D / 16; ++nt) o[nt][r] *= c;
-    }
-
-#pragma unroll
-    for (int kk2 = 0; kk2 < KC2; ++kk2) {
-      const u16x8 pa = *reinterpret_cast<const u16x8*>(
-          &Pl[wave][lc][kk2 * 32 + lg * 8]);
-#pragma unroll
-      for (int nt = 0; nt < D / 16; ++nt) {
-        const u16x8 b = *reinterpret_cast<const u16x8*>(
-            &VTl[nt * 16 + lc][kk2 * 32 + lg * 8]);
-        o[nt] = mfma16x16x32_bf16(pa, b, o[nt]);
-      }
-    }
-  }
-
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int orow = lg * 4 + r;
-    float denom = __shfl(lcol, orow, WAVE_SIZE);
-    float onum = 1.f;
-    if constexpr (EXT) {
-      if (sinks != nullptr) {
-        const float m_row = __shfl(mcol, orow, WAVE_SIZE);
-        const float sk = sinks[qh];
-        const float M2 = fmaxf(m_row, sk);
-        onum = (m_row == -INFINITY) ? 0.f : __expf(m_row - M2);
-        denom = denom * onum + __expf(sk - M2);
-      }
-    }
-    const int qrow = q0 + wave * 16 + orow;
-    if (qrow >= nnew || denom <= 0.f) continue;
-    const float inv = onum / denom;
-#pragma unroll
-    for (int nt = 0; nt < D / 16; ++nt) {
-      out[((long)(qstart + qrow) * Hq + qh) * D + nt * 16 + lc] =
-          f2bf(o[nt][r] * inv);
-    }
-  }
+template <int D, int DVK, bool EXT, bool PAGED>
+void launch(void* out, const void* q, const void* k, const void* v,
+            const int* bt, const int* start, const int* q0, const int* hist,
+            const int* nnew, const int* seq, int ntiles, int Hq, int Hkv,
+            int maxb, float scale, long qs, long ks, long vs,
+            const float* sinks, int window, float softcap, hipStream_t s) {
+  if (ntiles == 0) return;
+  hipLaunchKernelGGL((flash_prefill_kernel<D, DVK, EXT, PAGED>),
+                     dim3((unsigned)ntiles * Hq), dim3(PF_THREADS), 0, s,
+                     (unsigned short*)out, (const unsigned short*)q,
+                     (const unsigned short*)k, (const unsigned short*)v, bt,
+                     start, q0, hist, nnew, seq, Hq, Hkv, maxb, scale, qs, ks,
+                     vs, sinks, window, softcap);
 }
 
 }  // namespace
@@ -560,15 +386,11 @@ void flash_prefill_paged_launch(
     *err_unsupported = 1;
     return;
   }
-  dim3 grid(ntiles, Hq);
   const bool ext = (sinks != nullptr) || window > 0 || softcap > 0.f;
 #define PPG_LAUNCH(DD, E)                                                     \
-  hipLaunchKernelGGL((flash_prefill_paged_kernel<DD, E>), grid,               \
-                     dim3(PF_THREADS), 0, s, (unsigned short*)out,            \
-                     (const unsigned short*)q, (const unsigned short*)kc,     \
-                     (const unsigned short*)vc, block_tables, tile_qstart,    \
-                     tile_q0, tile_hist, tile_new, tile_seq, Hq, Hkv, maxb,   \
-                     scale, qs, sinks, window, softcap)
+  launch<DD, DD, E, true>(out, q, kc, vc, block_tables, tile_qstart, tile_q0, \
+                          tile_hist, tile_new, tile_seq, ntiles, Hq, Hkv,     \
+                          maxb, scale, qs, 0, 0, sinks, window, softcap, s)
   if (D == 128) {
     if (ext) PPG_LAUNCH(128, true);
     else PPG_LAUNCH(128, false);
@@ -594,15 +416,11 @@ void flash_prefill_launch(void* out, const void* q, const void* k,
     *err_unsupported = 1;
     return;
   }
-  dim3 grid(ntiles, Hq);
   const bool ext = (sinks != nullptr) || window > 0 || softcap > 0.f;
-#define PF_LAUNCH(DD, E, DVV)                                                \
-  hipLaunchKernelGGL((flash_prefill_kernel<DD, E, DVV>), grid,               \
-                     dim3(PF_THREADS), 0, s, (unsigned short*)out,           \
-                     (const unsigned short*)q, (const unsigned short*)k,     \
-                     (const unsigned short*)v, tile_start, tile_q0,          \
-                     tile_len, Hq, Hkv, scale, qs, ks, vs, sinks, window,    \
-                     softcap)
+#define PF_LAUNCH(DD, E, DVV)                                                 \
+  launch<DD, DVV, E, false>(out, q, k, v, nullptr, tile_start, tile_q0,       \
+                            nullptr, tile_len, nullptr, ntiles, Hq, Hkv, 0,   \
+                            scale, qs, ks, vs, sinks, window, softcap, s)
   if (mla_dims) {
     // MLA expand-prefill (DeepSeek): 192-dim qk over 128-dim values
     PF_LAUNCH(192, false, 128);

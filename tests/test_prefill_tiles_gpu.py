@@ -1,0 +1,92 @@
+"""Prompt attention at the edges of its tiles (128 query rows, 64 keys, 32
+rows a wave, 16 a page), whole prompts as views of a fused projection and rows
+behind a cached history in shuffled pages."""
+import math
+
+import pytest
+import torch
+
+pytestmark = [pytest.mark.gpu,
+              pytest.mark.skipif(not torch.cuda.is_available(),
+                                 reason="needs a GPU")]
+
+
+def _check(out, q, k, v, hist, scale):
+    """out / q [n, Hq, D] of one sequence, k / v [hist + n, G, D]."""
+    n, Hq, _ = q.shape
+    rep = Hq // k.shape[1]
+    k = k.double().repeat_interleave(rep, 1).transpose(0, 1)
+    v = v.double().repeat_interleave(rep, 1).transpose(0, 1)
+    s = torch.matmul(q.double().transpose(0, 1),
+                     k.transpose(1, 2).contiguous()) * scale
+    hide = torch.arange(k.shape[1], device=q.device)[None, :] > \
+        torch.arange(hist, hist + n, device=q.device)[:, None]
+    p = s.masked_fill(hide, float("-inf")).softmax(-1)
+    ref = torch.matmul(p, v).transpose(0, 1)
+    # weights are rounded to bf16 (2^-8 of each at most), the result once more;
+    # the rest is fp32
+    bound = torch.matmul(p, v.abs()).transpose(0, 1) * 2.0 ** -8 \
+        + ref.abs() * 2.0 ** -8 + 1e-4
+    err = (out.double() - ref).abs()
+    assert bool((err <= bound).all()), float((err - bound).max())
+
+
+@pytest.mark.parametrize("Hq,Hkv", [(4, 4), (32, 8), (16, 2), (6, 2)])
+@pytest.mark.parametrize("lens", [
+    [1], [31, 32, 33], [63, 64, 65, 2], [127, 128, 129], [200, 1, 257, 16],
+    [1000]])
+def test_whole_prompts(Hq, Hkv, lens):
+    from gpustack_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(sum(lens) + Hq)
+    qkv = torch.randn(sum(lens), (Hq + 2 * Hkv) * 128, generator=g,
+                      device="cuda").bfloat16()
+    q, k, v = (qkv[:, a * 128:b * 128].unflatten(1, (b - a, 128))
+               for a, b in ((0, Hq), (Hq, Hq + Hkv), (Hq + Hkv, Hq + 2 * Hkv)))
+    q = q * 3          # scores whose maximum moves by more than the slack
+    out = torch.full((sum(lens), Hq, 128), 9.0, device="cuda").bfloat16()
+    scale = 1 / math.sqrt(128)
+    ops.varlen_prefill_attn(out, q, k, v, lens, scale)
+    at = 0
+    for n in lens:
+        _check(out[at:at + n], q[at:at + n], k[at:at + n], v[at:at + n], 0,
+               scale)
+        at += n
+
+
+@pytest.mark.parametrize("Hq,Hkv", [(32, 8), (8, 8)])
+@pytest.mark.parametrize("seqs", [
+    [(0, 1)], [(1, 127), (15, 129)], [(16, 64), (17, 33), (63, 1)],
+    [(64, 200)], [(1000, 130), (0, 300)]])
+def test_rows_behind_history(Hq, Hkv, seqs):
+    from gpustack_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(seqs[0][0] + Hq)
+    need = [(h + n + 15) // 16 for h, n in seqs]
+    pools = [torch.randn(sum(need) + 1, Hkv, 16, 128, generator=g,
+                         device="cuda").bfloat16() for _ in range(2)]
+    pages = torch.randperm(sum(need), generator=g, device="cuda")
+    bt = torch.full((len(seqs), max(need)), sum(need), dtype=torch.int32,
+                    device="cuda")
+    at, starts, rows = 0, [], 0
+    for i, (n, (_, new)) in enumerate(zip(need, seqs)):
+        bt[i, :n] = pages[at:at + n].int()
+        at += n
+        starts.append(rows)
+        rows += new
+    # what lies behind a sequence's end in its last page is not its own
+    for i, (h, n) in enumerate(seqs):
+        if (h + n) % 16:
+            pools[0][bt[i, need[i] - 1].long(), :, (h + n) % 16:] = float("nan")
+            pools[1][bt[i, need[i] - 1].long(), :, (h + n) % 16:] = float("nan")
+    q = (torch.randn(rows, Hq, 128, generator=g, device="cuda") * 3).bfloat16()
+    out = torch.full_like(q, 9.0)
+    scale = 1 / math.sqrt(128)
+    ops.paged_prefill_attn(out, q, *pools, bt, starts, [h for h, _ in seqs],
+                           [n for _, n in seqs], scale)
+    for i, (h, n) in enumerate(seqs):
+        j = torch.arange(h + n, device="cuda")
+        blk = bt[i, j // 16].long()
+        st = starts[i]
+        _check(out[st:st + n], q[st:st + n], pools[0][blk, :, j % 16],
+               pools[1][blk, :, j % 16], h, scale)
