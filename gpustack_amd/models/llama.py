@@ -709,39 +709,8 @@ class MoEMLP(nn.Module):
         else:
             self.shared_gate_up_w = None
 
-    def _routing_consts(self, T: int, device):
-        """Per-T cached routing constants — rebuilt tensors per layer per
-        step showed up as ~27% glue kernels in the r2 profile.
-
-        Entries are kept for the module's lifetime in a dict: a hipGraph
-        captured after an eager warmup references the cached tensor by
-        ADDRESS, so evicting/overwriting an entry would leave captured
-        graphs reading freed (re-used) memory — garbage token indices and
-        out-of-bounds gathers at replay. Only decode-bucket-sized T values
-        are cached (<=1024 seqs); large prefill shapes compute fresh."""
-        cache = getattr(self, "_rc", None)
-        if cache is None:
-            cache = self._rc = {}
-        c = cache.get(T)
-        if c is None:
-            flat_tok = torch.arange(T, device=device).repeat_interleave(self.top_k)
-            ones = torch.ones(T * self.top_k, dtype=torch.int32, device=device)
-            if T > 1024:
-                return flat_tok, ones
-            c = cache[T] = (flat_tok, ones)
-        return c
-
-    def forward(self, x, meta: ForwardMeta | None = None):
-        # MoE expert MLPs do not take LoRA (rejected at adapter load);
-        # attention adapters still apply upstream
-        T = x.shape[0]
-        rw = getattr(self, "_router_w_f32", None)
-        if rw is None or rw.device != x.device:
-            self._router_w_f32 = self.router_w.float()
-            rw = self._router_w_f32
-        logits = F.linear(x.float(), rw)                          # [T, E]
-        if self.spec.router_logit_bias and self.router_bias is not None:
-            logits = logits + self.router_bias  # GPT-OSS: bias on logits
+    def _route(self, logits):
+        """Router logits [T, E] (fp32) -> weights, experts [T, k]."""
         if self.spec.router_mode == "sigmoid_bias":
             # GLM-4.5/DeepSeek routing (HF Glm4MoeTopkRouter): sigmoid
             # scores; the learned bias only influences the CHOICE, the
@@ -750,11 +719,11 @@ class MoEMLP(nn.Module):
             choice = scores + self.router_bias
             ng, tg = self.spec.n_group, self.spec.topk_group
             if ng > 1:
-                gs = (choice.view(T, ng, self.e // ng)
+                gs = (choice.view(-1, ng, self.e // ng)
                       .topk(2, dim=-1)[0].sum(dim=-1))
                 gi = torch.topk(gs, k=tg, dim=-1, sorted=False)[1]
                 gmask = torch.zeros_like(gs).scatter_(1, gi, 1)
-                smask = gmask.unsqueeze(-1).expand(T, ng, self.e // ng)                     .reshape(T, self.e)
+                smask = gmask.unsqueeze(-1).expand(-1, ng, self.e // ng)                     .reshape(-1, self.e)
                 choice = choice.masked_fill(~smask.bool(), float("-inf"))
             experts = torch.topk(choice, k=self.top_k, dim=-1,
                                  sorted=False)[1]
@@ -771,34 +740,47 @@ class MoEMLP(nn.Module):
             # un-renormalized: keep the full-softmax probabilities
             probs = torch.softmax(logits, dim=-1)
             weights, experts = torch.topk(probs, self.top_k, dim=-1)
+        return weights, experts
+
+    def forward(self, x, meta: ForwardMeta | None = None):
+        # MoE expert MLPs do not take LoRA (rejected at adapter load);
+        # attention adapters still apply upstream
+        T = x.shape[0]
+        rw = getattr(self, "_router_w_f32", None)
+        if rw is None or rw.device != x.device:
+            self._router_w_f32 = self.router_w.float()
+            rw = self._router_w_f32
+        logits = F.linear(x.float(), rw)                          # [T, E]
+        if self.spec.router_logit_bias and self.router_bias is not None:
+            logits = logits + self.router_bias  # GPT-OSS: bias on logits
+        fused = self._fused_ok(x)
+        if fused and self.spec.router_mode != "sigmoid_bias" \
+                and self.e <= 1024:
+            # softmax routing in one launch (a top-k, a sort and a softmax
+            # otherwise)
+            experts = torch.empty(T, self.top_k, dtype=torch.int32,
+                                  device=x.device)
+            weights = torch.empty(T, self.top_k, dtype=torch.float32,
+                                  device=x.device)
+            ops._load_hip().moe_topk(experts, weights, logits,
+                                     bool(self.spec.norm_topk_prob))
+        else:
+            weights, experts = self._route(logits)
+        if fused:
+            out = self._fused_dispatch(x, experts, weights)
+            return self.comm.all_reduce(self._add_shared(x, out))
         flat_exp = experts.reshape(-1)                            # [T*k]
-        flat_tok, ones_i32 = self._routing_consts(T, x.device)
+        flat_tok = torch.arange(T, device=x.device) \
+            .repeat_interleave(self.top_k)
         flat_w32 = weights.reshape(-1)                            # f32
         # Per-assignment contributions land at UNIQUE rows of a [T*k, h]
         # buffer, then reduce over the fixed k axis — index_add_ over
         # duplicated token rows would use atomics, whose order (and thus
         # the bf16 rounding) varies run to run and flips the next layer's
         # router on near-ties (observed on HW).
-        # Three dispatch paths:
-        #  - fused grouped-GEMM HIP kernels (ops/csrc/moe_gemm.hip): no host
-        #    sync anywhere, fixed launch grids — hipGraph-capturable; the
-        #    default on GPU for MFMA-aligned dims
-        #  - decode-shaped torch fallback: ONE padded strided-batched GEMM
-        #    pair (pays a per-layer counts.max() host sync)
-        #  - prefill-shaped: per-expert loop GEMMs (large per-expert work)
-        # decode-shaped batches take the fused kernels (which re-stream
-        # each expert's weight panel per 16-row m-tile — free when experts
-        # hold <=32 rows, ruinous at prefill occupancy, where the
-        # per-expert hipBLASLt loop wins). Under hipGraph CAPTURE the
-        # fused path is forced for ANY size: the torch fallbacks sync with
-        # the host per layer, which capture cannot record (large decode
-        # buckets on many-expert models would otherwise crash at init).
-        capturing = x.is_cuda and torch.cuda.is_current_stream_capturing()
-        if self._fused_ok(x) and (flat_exp.numel() <= 32 * self.e
-                                  or capturing):
-            out = self._fused_dispatch(x, flat_exp, flat_tok, flat_w32,
-                                       ones_i32)
-            return self.comm.all_reduce(self._add_shared(x, out))
+        # Aligned sizes on the GPU run the grouped expert kernels above
+        # (ops/csrc/moe_gemm.hip; no host sync, capturable); what is left
+        # here is the per-expert loop, and the padded batched product.
         flat_w = flat_w32.to(x.dtype)
         contrib = x.new_zeros(T * self.top_k, x.shape[1])
         # prefill-shaped on GPU with many experts: padded-bmm. The r2
@@ -902,33 +884,44 @@ class MoEMLP(nn.Module):
                 and os.environ.get("GPUSTACK_AMD_FUSED_MOE", "1") == "1"
                 and act_ok
                 and self.i % 128 == 0 and x.shape[1] % 128 == 0
-                and ops.hip_available())
+                and self.e <= 4096 and ops.hip_available())
 
-    def _fused_dispatch(self, x, flat_exp, flat_tok, flat_w32, ones_i32):
-        """Sync-free grouped expert GEMMs: sort assignments by expert on
-        device, run the two fused kernels, reduce over the k axis. Every
+    # Rows per expert from which the 128-row tiles are faster than the
+    # 16-row form, which streams an expert's weights once per 16 rows
+    _TILE_ROWS = 24
+
+    def _fused_dispatch(self, x, experts, weights):
+        """Sync-free grouped expert products: sort the assignments by expert
+        on the device, run the two expert kernels, sum over the k axis. Every
         tensor shape here depends only on (T, k, E) — safe under hipGraph
-        capture (reference capability: vLLM fused_moe; re-designed for
-        CDNA4 per SURVEY.md §2.9 #1)."""
-        T = x.shape[0]
-        TK = flat_exp.numel()
-        order = torch.argsort(flat_exp, stable=True)
-        s_tok = flat_tok[order].to(torch.int32)
-        # scatter_add instead of bincount: bincount computes max() on host
-        counts = torch.zeros(self.e, dtype=torch.int32, device=x.device)
-        counts.scatter_add_(0, flat_exp, ones_i32)
-        offs = (counts.cumsum(0, dtype=torch.int32) - counts).to(torch.int32)
+        capture (reference capability: vLLM fused_moe)."""
+        T, k = experts.shape
+        TK = T * k
         hip = ops._load_hip()
-        act = x.new_empty(TK, self.i)
+        flat = experts.reshape(-1).to(torch.int32)
+        flat_w = weights.reshape(-1).float()
+        order, s_tok, counts, offs, tiles, ntiles = hip.moe_sort(
+            flat, self.e, k)
         act_mode = 1 if self.spec.moe_act == "clamped_swiglu" else 0
-        hip.moe_gate_up_silu(act, x, self._bank("gate_up"), s_tok, offs,
-                             counts, bias=self.gate_up_b, act_mode=act_mode)
-        contrib = x.new_empty(TK, x.shape[1])
         # down bias on tp rank 0 only: the TP all-reduce must sum it once
         db = self.down_b if self.comm.tp_rank == 0 else None
-        hip.moe_down_scale(contrib, act, self._bank("down"), offs, counts,
-                           order.to(torch.int32), flat_w32, bias=db)
-        return contrib.view(T, self.top_k, -1).sum(dim=1).to(x.dtype)
+        act = x.new_empty(TK, self.i)
+        contrib = x.new_empty(TK, x.shape[1])
+        if TK >= self._TILE_ROWS * self.e:
+            hip.moe_tile(False, act, x, self._bank("gate_up"), s_tok, tiles,
+                         ntiles, offs, counts, bias=self.gate_up_b,
+                         act_mode=act_mode)
+            hip.moe_tile(True, contrib, act, self._bank("down"), order, tiles,
+                         ntiles, offs, counts, flat_w, bias=db)
+        else:
+            hip.moe_gate_up_silu(act, x, self._bank("gate_up"), s_tok, offs,
+                                 counts, bias=self.gate_up_b,
+                                 act_mode=act_mode)
+            hip.moe_down_scale(contrib, act, self._bank("down"), offs, counts,
+                               order, flat_w, bias=db)
+        out = torch.empty_like(x)
+        hip.moe_sum(out, contrib, k)
+        return out
 
     def _act_mul(self, gu):
         """[T', 2i] -> [T', i]: SiLU-mul (fused kernel/ref) or GPT-OSS

@@ -23,6 +23,10 @@ void skinny_gemm_v2_launch(void*, const void*, const void*, void*, int, int, int
 void gemm_lab_launch(void*, const void*, const void*, int, int, int, int, int*, hipStream_t);
 void moe_gate_up_silu_launch(void*, const void*, const void*, const int*, const int*, const int*, const void*, int, int, int, int, int*, hipStream_t);
 void moe_down_scale_launch(void*, const void*, const void*, const int*, const int*, const int*, const float*, const void*, int, int, int, int*, hipStream_t);
+void moe_topk_launch(int*, float*, const float*, int, int, int, int, int*, hipStream_t);
+void moe_sort_launch(int*, int*, int*, int*, int*, int*, const int*, int, int, int, int*, hipStream_t);
+void moe_sum_launch(void*, const void*, long, int, int, hipStream_t);
+void moe_tile_launch(int, void*, const void*, const void*, const int*, const int*, const int*, const int*, const int*, const float*, const void*, int, int, int, int, int*, hipStream_t);
 void w4_gemm_launch(void*, const void*, const void*, const void*, const void*, int, int, int, int*, hipStream_t);
 void w4_dequant_launch(void*, const void*, const void*, const void*, long, int, int*, hipStream_t);
 
@@ -354,6 +358,101 @@ void moe_down_scale(at::Tensor contrib, at::Tensor act, at::Tensor w,
   HIP_CHECK_LAST();
 }
 
+void check_i32(const at::Tensor& t, long n, const char* name) {
+  TORCH_CHECK(t.is_cuda() && t.scalar_type() == at::kInt && t.is_contiguous()
+              && t.numel() >= n, name, " must be a GPU int32 list of ", n);
+}
+
+void moe_topk(at::Tensor experts, at::Tensor weights, at::Tensor logits,
+              bool renorm) {
+  const int T = logits.size(0), E = logits.size(1), k = experts.size(1);
+  check_i32(experts, (long)T * k, "experts");
+  TORCH_CHECK(logits.is_cuda() && logits.scalar_type() == at::kFloat
+              && logits.is_contiguous(), "logits must be fp32");
+  TORCH_CHECK(weights.is_cuda() && weights.scalar_type() == at::kFloat
+              && weights.is_contiguous()
+              && weights.numel() == (long)T * k
+              && experts.numel() == (long)T * k, "experts / weights [T, k]");
+  int err = 0;
+  moe_topk_launch(experts.data_ptr<int>(), weights.data_ptr<float>(),
+                  logits.data_ptr<float>(), T, E, k, renorm ? 1 : 0, &err,
+                  cur_stream(logits));
+  TORCH_CHECK(!err, "moe_topk: unsupported E=", E, " k=", k);
+  HIP_CHECK_LAST();
+}
+
+// -> (order, s_tok, counts, offs, tiles, ntiles)
+std::vector<at::Tensor> moe_sort(at::Tensor experts, long E, long k) {
+  const long TK = experts.numel();
+  check_i32(experts, TK, "experts");
+  TORCH_CHECK(TK < (1L << 30) && k >= 1 && E >= 1, "moe_sort sizes");
+  auto o = experts.options();
+  at::Tensor order = at::empty({TK}, o), s_tok = at::empty({TK}, o);
+  at::Tensor counts = at::empty({E}, o), offs = at::empty({E}, o);
+  at::Tensor tiles = at::empty({TK / 128 + E, 2}, o), n = at::empty({1}, o);
+  int err = 0;
+  moe_sort_launch(order.data_ptr<int>(), s_tok.data_ptr<int>(),
+                  counts.data_ptr<int>(), offs.data_ptr<int>(),
+                  tiles.data_ptr<int>(), n.data_ptr<int>(),
+                  experts.data_ptr<int>(), (int)TK, (int)E, (int)k, &err,
+                  cur_stream(experts));
+  TORCH_CHECK(!err, "moe_sort: unsupported E=", E);
+  HIP_CHECK_LAST();
+  return {order, s_tok, counts, offs, tiles, n};
+}
+
+void moe_sum(at::Tensor out, at::Tensor contrib, long k) {
+  check_bf16(out, "out"); check_bf16(contrib, "contrib");
+  const long T = out.size(0);
+  const int H = out.size(1);
+  TORCH_CHECK(H % 8 == 0 && contrib.numel() == T * k * H, "moe_sum shapes");
+  moe_sum_launch(out.data_ptr(), contrib.data_ptr(), T, (int)k, H,
+                 cur_stream(out));
+  HIP_CHECK_LAST();
+}
+
+// down: contrib[rows[j]] = (src[j] @ w[e]^T + bias) * flat_w[rows[j]];
+// else act[j] = act(src[rows[j]] @ gate^T, ... @ up^T), over the tile list
+void moe_tile(bool down, at::Tensor out, at::Tensor src, at::Tensor w,
+              at::Tensor rows, at::Tensor tiles, at::Tensor ntiles,
+              at::Tensor offs, at::Tensor counts,
+              c10::optional<at::Tensor> flat_w,
+              c10::optional<at::Tensor> bias, long act_mode) {
+  check_bf16(out, "out"); check_bf16(src, "src"); check_bf16(w, "w");
+  const int E = w.size(0), K = w.size(2);
+  const long N = down ? w.size(1) : w.size(1) / 2;
+  check_i32(rows, out.size(0), "rows");
+  check_i32(ntiles, 1, "ntiles");
+  check_i32(offs, E, "offs");
+  check_i32(counts, E, "counts");
+  check_i32(tiles, 2 * (out.size(0) / 128 + E), "tiles");
+  TORCH_CHECK(src.size(1) == K && out.size(1) == N, "moe_tile shapes");
+  TORCH_CHECK(!down || src.size(0) == out.size(0), "moe_tile rows");
+  const float* fw = nullptr;
+  if (down) {
+    TORCH_CHECK(flat_w.has_value() && flat_w->is_cuda()
+                && flat_w->scalar_type() == at::kFloat
+                && flat_w->is_contiguous()
+                && flat_w->numel() == out.size(0), "flat_w [TK] fp32");
+    fw = flat_w->data_ptr<float>();
+  }
+  const void* bias_ptr = nullptr;
+  if (bias.has_value()) {
+    check_bf16(*bias, "bias");
+    TORCH_CHECK(bias->numel() == (long)E * w.size(1), "bias shape");
+    bias_ptr = bias->data_ptr();
+  }
+  int err = 0;
+  moe_tile_launch(down ? 1 : 0, out.data_ptr(), src.data_ptr(), w.data_ptr(),
+                  rows.data_ptr<int>(), tiles.data_ptr<int>(),
+                  ntiles.data_ptr<int>(), offs.data_ptr<int>(),
+                  counts.data_ptr<int>(), fw, bias_ptr, (int)act_mode,
+                  (int)(out.size(0) / 128 + E), (int)N, K, &err,
+                  cur_stream(src));
+  TORCH_CHECK(!err, "moe_tile: unsupported dims N=", N, " K=", K);
+  HIP_CHECK_LAST();
+}
+
 void w4_gemm(at::Tensor out, at::Tensor x, at::Tensor qw, at::Tensor sc,
              at::Tensor zs) {
   check_bf16(out, "out"); check_bf16(x, "x");
@@ -437,6 +536,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_gemm", &skinny_gemm, "split-K skinny GEMM (bf16, f32 accum)");
   m.def("gemm8", &gemm8, "8-phase pipelined 256x256 GEMM (bf16, f32 accum)");
   m.def("gemm_lab", &gemm_lab, "GEMM schedule lab variants (A/B vs hipBLASLt)");
+  m.def("moe_topk", &moe_topk, "softmax routing, top k");
+  m.def("moe_sort", &moe_sort, "assignments by expert, and the tile list");
+  m.def("moe_sum", &moe_sum, "sum of a row's expert contributions");
+  m.def("moe_tile", &moe_tile, "expert products in 128x128 tiles",
+        py::arg("down"), py::arg("out"), py::arg("src"), py::arg("w"),
+        py::arg("rows"), py::arg("tiles"), py::arg("ntiles"), py::arg("offs"),
+        py::arg("counts"), py::arg("flat_w") = py::none(),
+        py::arg("bias") = py::none(), py::arg("act_mode") = 0);
   m.def("moe_gate_up_silu", &moe_gate_up_silu,
         py::arg("act"), py::arg("x"), py::arg("w"), py::arg("s_tok"),
         py::arg("offs"), py::arg("counts"), py::arg("bias") = py::none(),

@@ -1,10 +1,7 @@
-// Grouped MoE expert GEMMs for MI355X (gfx950) — the sync-free dispatch
-// path (round-2 item: remove the per-layer bincount/max host syncs and the
-// padded-bmm overcompute so MoE decode can run under hipGraphs).
+// Grouped MoE expert GEMMs for MI355X (gfx950): routing, expert sort, both
+// expert products and the sum over a row's experts without a host readback.
 //
-// Two kernels over the expert-sorted assignment list (sorting/count/offset
-// tensors are computed on-device by torch ops in models/llama.py MoEMLP —
-// no host readback anywhere):
+// Two products over the expert-sorted assignment list:
 //
 //   moe_gate_up_silu: act[j, :] = silu(x[tok_j] @ Wg[e_j]^T) * (x[tok_j] @ Wu[e_j]^T)
 //   moe_down_scale:   contrib[order[j], :] = (act[j] @ Wd[e_j]^T) * w_j
@@ -15,11 +12,14 @@
 //   contrib[order[j], :] = ((act[j] @ Wd[e_j]^T) + bd[e_j]) * w_j
 // (matches models/llama.py MoEMLP._act_mul / the HF GptOss experts)
 //
-// Fixed launch grids (E x N-tiles) independent of the routing outcome:
-// workgroups for empty experts exit immediately. MFMA 16x16x32 tiles,
-// A = 16 gathered token rows staged through LDS in 512-element K chunks,
-// B = expert weight panels streamed from HBM (read once per 16-row m-tile;
-// typical decode occupancy is <= 2 m-tiles per expert).
+// in two forms with fixed launch grids, independent of the routing outcome:
+//
+// * few rows per expert (decode): workgroups of (expert, 64 columns), those
+//   of empty experts exit. MFMA 16x16x32 tiles, A = 16 gathered token rows
+//   staged through LDS in 512-element K chunks, B = expert weight panels
+//   streamed from HBM, once per 16-row m-tile. Bound by that stream: 128
+//   experts x (1536 + 768) x 2048 at 64 rows run at 4.7 and 5.0 TB/s.
+// * many rows per expert (prompts): 128 x 128 tiles, below.
 #include "common.h"
 
 namespace {
@@ -227,7 +227,419 @@ __global__ __launch_bounds__(MOE_THREADS) void moe_down_scale_kernel(
   }
 }
 
+// ---------------------------------------------------------------------------
+// Prompt form. A tile is 128 rows of one expert x 128 weight rows (of gate and
+// up: 64 each, 32 + 32 beside each other per wave, so that a lane holds a
+// column's gate and up), four waves of 64 x 64 on mfma_f32_32x32x16_bf16, K in
+// steps of 64 through two LDS buffers that global_load_lds fills 16 bytes a
+// lane (the next step's loads fly under this step's products, one barrier a
+// step; 64 KB, two workgroups a CU). 16-byte chunks are XORed with (row >> 1):
+// eight chunks a row, conflict-free over 16 rows of one chunk. Weights are the
+// A operand: a lane ends with 4 neighbouring columns of a row, which go
+// through the LDS to whole 16-byte stores.
+// The tile list (moe_sort) holds only tiles that exist, and workgroups are
+// dealt to the XCDs in runs, so the tiles of one expert meet its weights and
+// rows in one L2.
+// Bound by the products and the weight stream alike: 254 rows per expert of
+// 128 x (1536 + 768) x 2048 are 0.31 TFLOP and 1.2 GB a layer.
+// ---------------------------------------------------------------------------
+constexpr int MT_M = 128, MT_N = 128, MT_K = 64;
+
+typedef __attribute__((ext_vector_type(16))) float f32x16;
+typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
+
+DEVICE_INLINE unsigned int moe_pack(float lo, float hi) {
+  const f32x2 v{lo, hi};
+  return __builtin_bit_cast(unsigned int, __builtin_convertvector(v, bf16x2));
+}
+
+template <bool DOWN, bool EXTM>
+__global__ __launch_bounds__(MOE_THREADS, 2) void moe_tile_kernel(
+    unsigned short* __restrict__ out,        // act [TK, I] | contrib [TK, H]
+    const unsigned short* __restrict__ src,  // x [T, H] | act [TK, I]
+    const unsigned short* __restrict__ w,    // [E, 2I, H] | [E, H, I]
+    const int* __restrict__ rows,            // s_tok | order, [TK]
+    const int* __restrict__ tiles,           // [max, 2] expert, first row
+    const int* __restrict__ ntiles,          // [1]
+    const int* __restrict__ offs, const int* __restrict__ counts,
+    const float* __restrict__ flat_w,        // DOWN: [TK] routing weights
+    const unsigned short* __restrict__ bias, // [E, 2I] | [E, H] or null
+    int act_mode, int N, int K) {            // N = I | H
+  constexpr int BUF = (MT_M + MT_N) * MT_K;  // elements of a buffer
+  __shared__ __attribute__((aligned(16))) unsigned short lds[2 * BUF];
+
+  const int nnt = N / (DOWN ? MT_N : MT_N / 2);
+  const int nwg = ntiles[0] * nnt;
+  int wg = blockIdx.x;
+  if (wg >= nwg) return;
+  {
+    const int q = nwg / 8, r = nwg % 8, xcd = wg % 8, idx = wg / 8;
+    wg = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + idx;
+  }
+  const int tile = wg / nnt, nt = wg % nnt;
+  const int e = tiles[2 * tile], m0 = tiles[2 * tile + 1];
+  const int first = offs[e] + m0;            // sorted row of the tile's first
+  const int nrows = min(MT_M, counts[e] - m0);
+
+  const int tid = threadIdx.x;
+  const int lane = tid & (WAVE_SIZE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE_SIZE);
+  const int wm = wave >> 1, wn = wave & 1;
+  const int lc = lane & 31, hf = lane >> 5;
+
+  // staging: a wave instruction fills 8 rows of 128 bytes; instruction i of
+  // wave w takes rows (i * 4 + w) * 8 ..
+  const unsigned short* ap[4];
+  const unsigned short* bp[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = (i * 4 + wave) * 8 + lane / 8;
+    const int chunk = (lane & 7) ^ ((row >> 1) & 7);
+    const int at = first + min(row, nrows - 1);
+    const long arow = DOWN ? (long)at : (long)rows[at];
+    ap[i] = src + arow * K + chunk * 8;
+    long brow;
+    if constexpr (DOWN) {
+      brow = (long)e * N + nt * MT_N + row;
+    } else {
+      const int col = nt * 64 + (row >> 6) * 32 + (row & 31);
+      brow = (long)e * 2 * N + ((row & 32) ? N : 0) + col;
+    }
+    bp[i] = w + brow * K + chunk * 8;
+  }
+  auto stage = [&](int buf, int k0) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      unsigned short* d = lds + buf * BUF + (i * 4 + wave) * 8 * MT_K;
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) unsigned int*)(ap[i] + k0),
+          (__attribute__((address_space(3))) unsigned int*)d, 16, 0, 0);
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) unsigned int*)(bp[i] + k0),
+          (__attribute__((address_space(3))) unsigned int*)(d + MT_M * MT_K),
+          16, 0, 0);
+    }
+  };
+
+  f32x16 acc[2][2];                          // [weight tile][row tile]
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
+
+  const int nk = K / MT_K;
+  stage(0, 0);
+  for (int kt = 0; kt < nk; ++kt) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (kt + 1 < nk) stage((kt + 1) & 1, (kt + 1) * MT_K);
+    const unsigned short* al = lds + (kt & 1) * BUF;
+    const unsigned short* bl = al + MT_M * MT_K;
+#pragma unroll
+    for (int kk = 0; kk < MT_K / 16; ++kk) {
+      u32x4 fa[2], fb[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const int rb = wn * 64 + t * 32 + lc, ra = wm * 64 + t * 32 + lc;
+        fb[t] = *reinterpret_cast<const u32x4*>(
+            bl + rb * MT_K + ((kk * 2 + hf) ^ ((rb >> 1) & 7)) * 8);
+        fa[t] = *reinterpret_cast<const u32x4*>(
+            al + ra * MT_K + ((kk * 2 + hf) ^ ((ra >> 1) & 7)) * 8);
+      }
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+          acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              __builtin_bit_cast(m_s16x8, fb[a]),
+              __builtin_bit_cast(m_s16x8, fa[b]), acc[a][b], 0, 0, 0);
+    }
+  }
+  __syncthreads();
+
+  // acc[a][b][r]: weight row 8 (r>>2) + 4 hf + (r&3) of tile a, row lc of
+  // tile b. Rows of the result through the LDS, 8-byte units XORed with row.
+  constexpr int OW = DOWN ? MT_N : MT_N / 2; // columns of the result
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    const int row = wm * 64 + b * 32 + lc;
+    float rw = 1.f;
+    if constexpr (DOWN) rw = flat_w[rows[first + min(row, nrows - 1)]];
+#pragma unroll
+    for (int a = 0; a < (DOWN ? 2 : 1); ++a)
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) {
+        const int c = wn * (OW / 2) + a * 32 + rr * 8 + hf * 4;
+        float v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int r = rr * 4 + j;
+          if constexpr (DOWN) {
+            float bd = 0.f;
+            if constexpr (EXTM)
+              if (bias != nullptr)
+                bd = bf2f(bias[(long)e * N + nt * OW + c + j]);
+            v[j] = (acc[a][b][r] + bd) * rw;
+          } else {
+            float g = acc[0][b][r], u = acc[1][b][r];
+            if constexpr (EXTM) {
+              if (bias != nullptr) {
+                g += bf2f(bias[(long)e * 2 * N + nt * OW + c + j]);
+                u += bf2f(bias[(long)e * 2 * N + N + nt * OW + c + j]);
+              }
+            }
+            if (EXTM && act_mode == 1) {       // GPT-OSS clamped swiglu
+              g = fminf(g, 7.f);
+              u = fminf(fmaxf(u, -7.f), 7.f);
+              v[j] = (u + 1.f) * g / (1.f + __expf(-1.702f * g));
+            } else {
+              v[j] = g / (1.f + __expf(-g)) * u;
+            }
+          }
+        }
+        *reinterpret_cast<u32x2*>(lds + row * OW + ((c / 4) ^ (row & 15)) * 4) =
+            u32x2{moe_pack(v[0], v[1]), moe_pack(v[2], v[3])};
+      }
+  }
+  __syncthreads();
+  constexpr int OC = OW / 8;
+#pragma unroll
+  for (int i = 0; i < MT_M * OC / MOE_THREADS; ++i) {
+    const int u = tid + i * MOE_THREADS;
+    const int row = u / OC, c = u % OC;
+    if (row >= nrows) continue;
+    const u32x2 a = *reinterpret_cast<const u32x2*>(
+        lds + row * OW + ((2 * c) ^ (row & 15)) * 4);
+    const u32x2 b = *reinterpret_cast<const u32x2*>(
+        lds + row * OW + ((2 * c + 1) ^ (row & 15)) * 4);
+    const long orow = DOWN ? (long)rows[first + row] : (long)(first + row);
+    *reinterpret_cast<u32x4*>(out + orow * N + nt * OW + c * 8) =
+        u32x4{a[0], a[1], b[0], b[1]};
+  }
+}
+
+// Softmax routing: the k largest logits of a row in descending order (lowest
+// index first among equals) and their weights: softmax over the chosen ones
+// (renorm) or their share of the softmax over all. One wave per row, NV
+// logits a lane. Bound by the launch.
+template <int NV>
+__global__ __launch_bounds__(256) void moe_topk_kernel(
+    int* __restrict__ experts,         // [T, k]
+    float* __restrict__ weights,       // [T, k]
+    const float* __restrict__ logits,  // [T, E]
+    int T, int E, int k, int renorm) {
+  const int lane = threadIdx.x & 63;
+  const int t = blockIdx.x * 4 + threadIdx.x / 64;
+  if (t >= T) return;
+  float v[NV];
+  unsigned taken = 0;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int e = i * 64 + lane;
+    v[i] = e < E ? logits[(long)t * E + e] : -INFINITY;
+    if (e >= E) taken |= 1u << i;
+  }
+  float top = 0.f, mine = 0.f, sum = 0.f;
+  for (int j = 0; j < k; ++j) {
+    float best = -INFINITY;
+    int at = 1 << 30;
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+      if (!(taken >> i & 1) && (v[i] > best || (v[i] == best && at == 1 << 30))) {
+        best = v[i];
+        at = i * 64 + lane;
+      }
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) {
+      const float ob = __shfl_xor(best, m, 64);
+      const int oa = __shfl_xor(at, m, 64);
+      if (ob > best || (ob == best && oa < at)) {
+        best = ob;
+        at = oa;
+      }
+    }
+    at = min(at, E - 1);               // rows of NaN: any expert, in range
+    if ((at & 63) == lane) taken |= 1u << (at >> 6);
+    if (j == 0) top = best;
+    const float p = __expf(best - top);
+    sum += p;
+    if (lane == j) mine = p;
+    if (lane == 0) experts[(long)t * k + j] = at;
+  }
+  if (!renorm) {
+    float all = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) all += __expf(v[i] - top);
+    sum = wave_reduce_sum(all);
+  }
+  if (lane < k) weights[(long)t * k + lane] = mine / sum;
+}
+
+constexpr int MOE_MAX_E = 4096;
+
+// Counting sort of the assignments by expert in one workgroup: counts,
+// offsets, the sorted rows and the prompt form's tile list. The order within
+// an expert is free: a row's result does not depend on its place. Takes about
+// 5 us at 512 assignments (a radix sort, a scatter and the casts around them
+// took 100) and is one pass over the list beyond that.
+__global__ __launch_bounds__(1024) void moe_sort_kernel(
+    int* __restrict__ order, int* __restrict__ s_tok,  // [TK]
+    int* __restrict__ counts, int* __restrict__ offs,  // [E]
+    int* __restrict__ tiles, int* __restrict__ ntiles,
+    const int* __restrict__ experts, int TK, int E, int k) {
+  __shared__ int cnt[MOE_MAX_E];       // counts, then the next free places
+  __shared__ int wsum[2][16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int e = tid; e < MOE_MAX_E; e += 1024) cnt[e] = 0;
+  __syncthreads();
+  for (int i = tid; i < TK; i += 1024)
+    atomicAdd(&cnt[min(max(experts[i], 0), E - 1)], 1);
+  __syncthreads();
+  // thread tid owns experts EPT * tid ..
+  constexpr int EPT = MOE_MAX_E / 1024;
+  int c[EPT], a = 0, b = 0;
+#pragma unroll
+  for (int j = 0; j < EPT; ++j) {
+    c[j] = cnt[tid * EPT + j];
+    a += c[j];
+    b += (c[j] + MT_M - 1) / MT_M;
+  }
+  const int own_a = a, own_b = b;
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) {   // inclusive sums over the wave
+    const int x = __shfl_up(a, m, 64), y = __shfl_up(b, m, 64);
+    if (lane >= m) {
+      a += x;
+      b += y;
+    }
+  }
+  if (lane == 63) {
+    wsum[0][wave] = a;
+    wsum[1][wave] = b;
+  }
+  __syncthreads();
+  for (int i = 0; i < wave; ++i) {
+    a += wsum[0][i];
+    b += wsum[1][i];
+  }
+  if (tid == 1023) ntiles[0] = b;
+  a -= own_a;
+  b -= own_b;
+#pragma unroll
+  for (int j = 0; j < EPT; ++j) {
+    const int e = tid * EPT + j;
+    cnt[e] = a;
+    if (e < E) {
+      counts[e] = c[j];
+      offs[e] = a;
+      for (int r = 0; r < c[j]; r += MT_M, ++b) {
+        tiles[2 * b] = e;
+        tiles[2 * b + 1] = r;
+      }
+    }
+    a += c[j];
+  }
+  __syncthreads();
+  for (int i = tid; i < TK; i += 1024) {
+    const int at = atomicAdd(&cnt[min(max(experts[i], 0), E - 1)], 1);
+    order[at] = i;
+    s_tok[at] = i / k;
+  }
+}
+
+// out[t] = sum over the k contributions of row t, in fp32 in their order.
+// Bound by reading them once.
+__global__ __launch_bounds__(256) void moe_sum_kernel(
+    unsigned short* __restrict__ out,            // [T, H]
+    const unsigned short* __restrict__ contrib,  // [T, k, H]
+    long units, int k, int H) {
+  const int hu = H / 8;
+  for (long u = (long)blockIdx.x * 256 + threadIdx.x; u < units;
+       u += (long)gridDim.x * 256) {
+    const unsigned short* p = contrib + (u / hu) * k * H + (u % hu) * 8;
+    float s[8];
+    bf8_to_f32(*reinterpret_cast<const u16x8*>(p), s);
+    for (int j = 1; j < k; ++j) {
+      float f[8];
+      bf8_to_f32(*reinterpret_cast<const u16x8*>(p + (long)j * H), f);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) s[i] += f[i];
+    }
+    *reinterpret_cast<u32x4*>(out + u * 8) =
+        u32x4{moe_pack(s[0], s[1]), moe_pack(s[2], s[3]),
+              moe_pack(s[4], s[5]), moe_pack(s[6], s[7])};
+  }
+}
+
 }  // namespace
+
+void moe_topk_launch(int* experts, float* weights, const float* logits, int T,
+                     int E, int k, int renorm, int* err_unsupported,
+                     hipStream_t s) {
+  *err_unsupported = 0;
+  if (E < 1 || E > 1024 || k < 1 || k > 64 || k > E) {
+    *err_unsupported = 1;
+    return;
+  }
+  if (T == 0) return;
+#define TOPK(NV)                                                             \
+  hipLaunchKernelGGL((moe_topk_kernel<NV>), dim3((T + 3) / 4), dim3(256), 0, \
+                     s, experts, weights, logits, T, E, k, renorm)
+  if (E <= 64) TOPK(1);
+  else if (E <= 128) TOPK(2);
+  else if (E <= 256) TOPK(4);
+  else if (E <= 512) TOPK(8);
+  else TOPK(16);
+#undef TOPK
+}
+
+void moe_sort_launch(int* order, int* s_tok, int* counts, int* offs,
+                     int* tiles, int* ntiles, const int* experts, int TK,
+                     int E, int k, int* err_unsupported, hipStream_t s) {
+  *err_unsupported = E < 1 || E > MOE_MAX_E;
+  if (*err_unsupported) return;
+  hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(1024), 0, s, order, s_tok,
+                     counts, offs, tiles, ntiles, experts, TK, E, k);
+}
+
+void moe_sum_launch(void* out, const void* contrib, long T, int k, int H,
+                    hipStream_t s) {
+  const long units = T * (H / 8);
+  if (units == 0) return;
+  const long grid = (units + 255) / 256;
+  hipLaunchKernelGGL(moe_sum_kernel, dim3(grid > 8192 ? 8192 : (int)grid),
+                     dim3(256), 0, s, (unsigned short*)out,
+                     (const unsigned short*)contrib, units, k, H);
+}
+
+// max_tiles bounds the tile list: no more than TK / 128 + E tiles exist.
+void moe_tile_launch(int down, void* out, const void* src, const void* w,
+                     const int* rows, const int* tiles, const int* ntiles,
+                     const int* offs, const int* counts, const float* flat_w,
+                     const void* bias, int act_mode, int max_tiles, int N,
+                     int K, int* err_unsupported, hipStream_t s) {
+  const int ow = down ? MT_N : MT_N / 2;
+  *err_unsupported = N % ow != 0 || K % MT_K != 0;
+  if (*err_unsupported || max_tiles == 0) return;
+  const bool extm = bias != nullptr || act_mode != 0;
+#define TILE(D, X)                                                            \
+  hipLaunchKernelGGL((moe_tile_kernel<D, X>),                                 \
+                     dim3((unsigned)max_tiles * (N / ow)), dim3(MOE_THREADS), \
+                     0, s, (unsigned short*)out, (const unsigned short*)src,  \
+                     (const unsigned short*)w, rows, tiles, ntiles, offs,     \
+                     counts, flat_w, (const unsigned short*)bias, act_mode,   \
+                     N, K)
+  if (down) {
+    if (extm) TILE(true, true);
+    else TILE(true, false);
+  } else {
+    if (extm) TILE(false, true);
+    else TILE(false, false);
+  }
+#undef TILE
+}
 
 void moe_gate_up_silu_launch(void* act, const void* x, const void* w,
                              const int* s_tok, const int* offs,

@@ -1,0 +1,116 @@
+"""Expert products of prompts: tile edges (128 rows, 64 / 128 columns), empty
+and overfull experts, both activations; softmax routing, the expert sort and
+the sum over a row's experts."""
+import pytest
+import torch
+
+pytestmark = [pytest.mark.gpu,
+              pytest.mark.skipif(not torch.cuda.is_available(),
+                                 reason="needs a GPU")]
+
+
+def _hip():
+    from gpustack_amd import ops
+
+    return ops._load_hip()
+
+
+def _experts(counts, k, g):
+    """Assignments [T, k] whose expert e has counts[e] rows."""
+    flat = torch.repeat_interleave(
+        torch.arange(len(counts)), torch.tensor(counts)).cuda()
+    assert flat.numel() % k == 0
+    return flat[torch.randperm(flat.numel(), generator=g, device="cuda")] \
+        .int().view(-1, k)
+
+
+@pytest.mark.parametrize("ext", [False, True])
+@pytest.mark.parametrize("counts,k,H,I", [
+    ([1, 0, 0, 1], 2, 128, 128),
+    ([127, 0, 128, 129], 4, 256, 128),
+    ([0, 0, 600, 0, 8], 8, 384, 256),
+    ([33] * 16, 2, 2048, 768)])
+def test_tiles(ext, counts, k, H, I):
+    hip = _hip()
+    E, TK = len(counts), sum(counts)
+    g = torch.Generator(device="cuda").manual_seed(TK)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    experts = _experts(counts, k, g)
+    T = experts.shape[0]
+    x = rnd(T, H).bfloat16()
+    gu = (rnd(E, 2 * I, H) * H ** -0.5).bfloat16()
+    dn = (rnd(E, H, I) * I ** -0.5).bfloat16()
+    gub, dnb = (rnd(E, 2 * I).bfloat16(), rnd(E, H).bfloat16()) if ext \
+        else (None, None)
+    fw = torch.rand(TK, generator=g, device="cuda")
+    order, s_tok, cnt, offs, tiles, n = hip.moe_sort(experts.view(-1), E, k)
+    act = torch.full((TK, I), 9.0, device="cuda").bfloat16()
+    con = torch.full((TK, H), 9.0, device="cuda").bfloat16()
+    hip.moe_tile(False, act, x, gu, s_tok, tiles, n, offs, cnt, bias=gub,
+                 act_mode=int(ext))
+    hip.moe_tile(True, con, act, dn, order, tiles, n, offs, cnt, fw, bias=dnb)
+    out = torch.empty_like(x)
+    hip.moe_sum(out, con, k)
+
+    assert cnt.tolist() == counts
+    assert n.item() == sum((c + 127) // 128 for c in counts)
+    flat = experts.view(-1).long()
+    o = order.long()
+    assert torch.equal(o.sort().values, torch.arange(TK, device="cuda"))
+    assert torch.equal(flat[o].sort().values, flat[o])
+    assert torch.equal(s_tok.long(), o // k)
+    e = flat[o]
+    # 8 significant bits: a rounding moves a value by at most 2^-8 of itself;
+    # fp32 sums of K unit-variance products of size K^-1/2 add under 1e-4
+    close = lambda a, r: bool(((a.double() - r).abs()
+                               <= r.abs() * 2.0 ** -8 + 2e-4).all())
+    h = torch.empty(TK, 2 * I, dtype=torch.float64, device="cuda")
+    y = torch.empty(TK, H, dtype=torch.float64, device="cuda")
+    for i in range(E):
+        r = (e == i).nonzero().flatten()
+        h[r] = x[s_tok[r].long()].double() @ gu[i].double().T
+        y[r] = act[r].double() @ dn[i].double().T
+        if ext:
+            h[r] += gub[i].double()
+            y[r] += dnb[i].double()
+    a, b = h[:, :I], h[:, I:]
+    if ext:
+        a, b = a.clamp(max=7), b.clamp(-7, 7)
+        ref = (b + 1) * a * torch.sigmoid(1.702 * a)
+    else:
+        ref = torch.nn.functional.silu(a) * b
+    # the activation multiplies fp32 errors of both halves by at most ~10
+    assert bool(((act.double() - ref).abs()
+                 <= ref.abs() * 2.0 ** -8 + 2e-3).all())
+    assert close(con[o], y * fw[o].double()[:, None])
+    assert close(out, con.double().view(T, k, H).sum(1))
+
+
+@pytest.mark.parametrize("renorm", [False, True])
+@pytest.mark.parametrize("T,E,k", [(1, 8, 2), (5, 64, 6), (130, 128, 8),
+                                   (7, 100, 1), (3, 384, 8), (4, 1000, 32)])
+def test_softmax_routing(renorm, T, E, k):
+    g = torch.Generator(device="cuda").manual_seed(T * E)
+    logits = torch.randn(T, E, generator=g, device="cuda") * 3
+    logits[0, : k + 1] = 20.0          # equals: the lowest indices win
+    ex = torch.empty(T, k, dtype=torch.int32, device="cuda")
+    w = torch.empty(T, k, device="cuda")
+    _hip().moe_topk(ex, w, logits, renorm)
+    assert ex[0].tolist() == list(range(k))
+    top, at = torch.topk(logits.double(), k, -1)
+    assert torch.equal(ex[1:].long(), at[1:])
+    ref = top.softmax(-1) if renorm else \
+        logits.double().softmax(-1).gather(1, ex.long())
+    torch.testing.assert_close(w.double(), ref, rtol=1e-5, atol=1e-7)
+
+
+def test_sort_of_a_long_list():
+    g = torch.Generator(device="cuda").manual_seed(3)
+    ex = torch.randint(0, 4000, (65536,), generator=g, device="cuda").int()
+    order, s_tok, cnt, offs, tiles, n = _hip().moe_sort(ex, 4096, 8)
+    ref = torch.bincount(ex.long(), minlength=4096)
+    assert torch.equal(cnt.long(), ref)
+    assert torch.equal(offs.long(), ref.cumsum(0) - ref)
+    assert torch.equal(order.long().sort().values,
+                       torch.arange(65536, device="cuda"))
+    assert n.item() == int(((ref + 127) // 128).sum())
