@@ -252,49 +252,71 @@ __global__ void reshape_and_cache_kernel(const unsigned short* __restrict__ k,
 
 // ---------------------------------------------------------------------------
 // Greedy sampling: argmax over vocab per row (ties -> lowest index).
-// One block per row; strided scan with (val, idx) carried per thread.
+// One block per row: 16 waves with four 16-byte loads in flight each, the
+// maximum of eight values first and its place only where it counts. Bound by
+// how fast one CU takes a row in (256 KB of a 128256-word vocabulary): with 4
+// waves and one load at a time 46 us, measured inside a decode step.
 // ---------------------------------------------------------------------------
-__global__ void greedy_sample_kernel(long* __restrict__ out,
-                                     const unsigned short* __restrict__ logits,
-                                     int N, int V) {
+constexpr int GS_THREADS = 1024;
+
+__global__ __launch_bounds__(GS_THREADS) void greedy_sample_kernel(
+    long* __restrict__ out, const unsigned short* __restrict__ logits,
+    int N, int V) {
   const int row = blockIdx.x;
   if (row >= N) return;
   const unsigned short* rp = logits + (long)row * V;
   float best = -INFINITY;
-  int besti = 0x7fffffff;
+  int besti = 0x7fffffff;              // first index of `best` seen so far
   const int nvec = V / 8;
-  for (int v = threadIdx.x; v < nvec; v += blockDim.x) {
-    u16x8 u = *reinterpret_cast<const u16x8*>(rp + v * 8);
+  auto take = [&](const u16x8 u, int v) {
+    float f[8], mx;
+    bf8_to_f32(u, f);
+    mx = fmaxf(fmaxf(fmaxf(f[0], f[1]), fmaxf(f[2], f[3])),
+               fmaxf(fmaxf(f[4], f[5]), fmaxf(f[6], f[7])));
+    if (mx > best) {                   // a thread's indices only grow
+      best = mx;
+      int i = 7;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float f = bf2f(u[i]);
-      const int gi = v * 8 + i;
-      if (f > best || (f == best && gi < besti)) { best = f; besti = gi; }
+      for (int j = 6; j >= 0; --j) i = f[j] == mx ? j : i;
+      besti = v * 8 + i;
     }
+  };
+  int v = threadIdx.x;
+  for (; v + 3 * GS_THREADS < nvec; v += 4 * GS_THREADS) {
+    u16x8 u[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      u[j] = *reinterpret_cast<const u16x8*>(rp + (v + j * GS_THREADS) * 8);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) take(u[j], v + j * GS_THREADS);
   }
-  for (int gi = nvec * 8 + threadIdx.x; gi < V; gi += blockDim.x) {
+  for (; v < nvec; v += GS_THREADS)
+    take(*reinterpret_cast<const u16x8*>(rp + v * 8), v);
+  for (int gi = nvec * 8 + threadIdx.x; gi < V; gi += GS_THREADS) {
     const float f = bf2f(rp[gi]);
-    if (f > best || (f == best && gi < besti)) { best = f; besti = gi; }
+    if (f > best) { best = f; besti = gi; }
   }
   // wave reduce, then LDS reduce
+  auto join = [&](int from) {
 #pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) {
-    const float ov = __shfl_xor(best, m, WAVE_SIZE);
-    const int oi = __shfl_xor(besti, m, WAVE_SIZE);
-    if (ov > best || (ov == best && oi < besti)) { best = ov; besti = oi; }
-  }
-  __shared__ float sv[8];
-  __shared__ int si[8];
+    for (int m = from; m >= 1; m >>= 1) {
+      const float ov = __shfl_xor(best, m, WAVE_SIZE);
+      const int oi = __shfl_xor(besti, m, WAVE_SIZE);
+      if (ov > best || (ov == best && oi < besti)) { best = ov; besti = oi; }
+    }
+  };
+  join(32);
+  __shared__ float sv[GS_THREADS / WAVE_SIZE];
+  __shared__ int si[GS_THREADS / WAVE_SIZE];
   const int wid = threadIdx.x / WAVE_SIZE;
   if ((threadIdx.x & (WAVE_SIZE - 1)) == 0) { sv[wid] = best; si[wid] = besti; }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int i = 1; i < (int)(blockDim.x / WAVE_SIZE); ++i) {
-      if (sv[i] > best || (sv[i] == best && si[i] < besti)) {
-        best = sv[i]; besti = si[i];
-      }
-    }
-    out[row] = besti;
+  if (threadIdx.x < GS_THREADS / WAVE_SIZE) {
+    best = sv[threadIdx.x];
+    besti = si[threadIdx.x];
+    join(GS_THREADS / WAVE_SIZE / 2);
+    // a row without any number (all NaN) still names a word
+    if (threadIdx.x == 0) out[row] = besti == 0x7fffffff ? 0 : besti;
   }
 }
 
@@ -361,6 +383,7 @@ void reshape_and_cache_launch(const void* k, const void* v, void* kc, void* vc,
 
 void greedy_sample_launch(long* out, const void* logits, int N, int V,
                           hipStream_t s) {
-  hipLaunchKernelGGL(greedy_sample_kernel, dim3(N), dim3(256), 0, s, out,
+  if (N == 0) return;
+  hipLaunchKernelGGL(greedy_sample_kernel, dim3(N), dim3(GS_THREADS), 0, s, out,
                      (const unsigned short*)logits, N, V);
 }

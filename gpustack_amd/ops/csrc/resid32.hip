@@ -464,21 +464,34 @@ __global__ __launch_bounds__(ROW_THREADS) void moe_combine_vec_kernel(
   }
 }
 
-__global__ __launch_bounds__(ROW_THREADS) void argmax_f32_kernel(
+// 16 waves a row with four loads in flight each: bound by how fast one CU
+// takes a row in (128 KB at a 32000-word vocabulary)
+constexpr int AM_THREADS = 1024;
+
+__global__ __launch_bounds__(AM_THREADS) void argmax_f32_kernel(
     long* __restrict__ out, const float* __restrict__ logits, int V) {
-  __shared__ float bv[4];
-  __shared__ int bi[4];
+  __shared__ float bv[AM_THREADS / 64];
+  __shared__ int bi[AM_THREADS / 64];
   const long t = blockIdx.x;
   const float* z = logits + t * V;
   float v = -INFINITY;
   int idx = 0x7fffffff;
-  for (int i = threadIdx.x; i < V; i += ROW_THREADS)
+  int i = threadIdx.x;
+  for (; i + 3 * AM_THREADS < V; i += 4 * AM_THREADS) {
+    float f[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) f[j] = z[i + j * AM_THREADS];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (f[j] > v) { v = f[j]; idx = i + j * AM_THREADS; }
+  }
+  for (; i < V; i += AM_THREADS)
     if (z[i] > v) { v = z[i]; idx = i; }
   wave_argmax(v, idx);
   if ((threadIdx.x & 63) == 0) { bv[threadIdx.x >> 6] = v; bi[threadIdx.x >> 6] = idx; }
   __syncthreads();
   if (threadIdx.x == 0) {
-    for (int w = 1; w < 4; ++w)
+    for (int w = 1; w < AM_THREADS / 64; ++w)
       if (bv[w] > v || (bv[w] == v && bi[w] < idx)) { v = bv[w]; idx = bi[w]; }
     out[t] = idx == 0x7fffffff ? 0 : idx;
   }
@@ -636,5 +649,5 @@ void moe_combine_launch(void* out, const void* y, const int* inv,
 void argmax_f32_launch(long* out, const float* logits, int N, int V,
                        hipStream_t s) {
   if (N == 0) return;
-  argmax_f32_kernel<<<N, ROW_THREADS, 0, s>>>(out, logits, V);
+  argmax_f32_kernel<<<N, AM_THREADS, 0, s>>>(out, logits, V);
 }
