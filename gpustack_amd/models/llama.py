@@ -162,21 +162,22 @@ class W4Pack:
 def qlinear(x, w, pack: "W4Pack | None", bias=None):
     """F.linear with an optional W4 runtime pack.
 
-    Default GPU path: the w4_dequant HIP kernel expands the packed weight
-    into a transient bf16 tensor (allocator-cached) and hipBLASLt runs the
-    GEMM at full MFMA rate — weights stay RESIDENT packed (the capacity
-    goal) at a measured ~2.25x packed-read traffic per use. The in-register
-    dequant MFMA kernel (w4_gemm) is kept behind GPUSTACK_AMD_W4_KERNEL=1:
-    both its LDS-staged and direct-L2 variants measured slower than
-    dequant+hipBLASLt at serving shapes so far (profiles/r04)."""
+    Packed weights stay RESIDENT packed (the capacity goal). Up to 64 rows
+    the packed product (ops/csrc/w4_gemm.hip) reads them as they are; more
+    rows expand the weight into a transient bf16 tensor (allocator-cached)
+    and run the library GEMM at full MFMA rate. Measured on 28672x4096, us:
+    16 rows 21 against 98, 64 rows 77 against 102, 128 rows 134 against 107
+    (4096x14336: 20 / 50, 60 / 59, 110 / 70). GPUSTACK_AMD_W4_KERNEL=1 keeps
+    the packed product up to 1024 rows."""
     if pack is None:
-        return F.linear(x, w, bias)
+        return ops.linear_auto(x, w) if bias is None else F.linear(x, w, bias)
     if x.is_cuda:
         import os as _os
 
         hip = ops._load_hip()
-        if (x.shape[0] <= 1024
-                and _os.environ.get("GPUSTACK_AMD_W4_KERNEL", "0") == "1"):
+        most = 1024 if _os.environ.get("GPUSTACK_AMD_W4_KERNEL", "0") == "1" \
+            else 64
+        if 0 < x.shape[0] <= most and x.dim() == 2 and pack.shape[1] <= 131072:
             out = torch.empty(x.shape[0], pack.shape[0], dtype=x.dtype,
                               device=x.device)
             hip.w4_gemm(out, x.contiguous(), pack.qw, pack.sc, pack.zs)
@@ -636,9 +637,7 @@ class MLP(nn.Module):
             act = torch.empty(x.shape[0], self.i, dtype=x.dtype,
                               device=x.device)
             ops.silu_and_mul(act, gu)
-        down = (qlinear(act, self.down_w, self.down_pack)
-                if self.down_pack is not None
-                else ops.linear_auto(act, self.down_w))
+        down = qlinear(act, self.down_w, self.down_pack)
         if meta is not None and meta.lora is not None:
             meta.lora.apply(self.layer_idx, act, down, self._down_projs)
         return self.comm.all_reduce(down)

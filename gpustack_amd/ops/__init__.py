@@ -326,11 +326,29 @@ def skinny_gemm(x, w, out=None, splitk: int | None = None, version: int = 1):
     return out
 
 
+def _rows_gemm_wins(M: int, N: int, K: int) -> bool:
+    """Where the decode product (ops/csrc/rows_gemm.hip) measured faster than
+    the library, us at 1 / 16 rows, weights out of HBM:
+    small weights, whose time is latency: 4096x4096 9.4 / 11.2 against 15.6 /
+    15.5, 2048x4096 8.5 / 10.8 against 14.7 / 14.9, 5120x2048 9.6 / 12.2
+    against 12.1 / 12.2 (24 rows of 4096x4096: 14.0 against 13.3; 6144x4096
+    14.4 / 19.0 against 14.7 / 14.6);
+    wide heads of narrow models: 102400x1536 71 / 80 against 115 / 114,
+    151936x2048 127 / 144 against 205 / 203, 200064x3072 254 / 294 against 382
+    / 374 (102400x1024 50 / 53 against 41 / 42, 102400x4096 175 / 192 against
+    176 / 181, 65536x2048 59 / 65 against 67 / 66)."""
+    if M > 16 or K % 128 != 0:
+        return False
+    return (N * K <= 17 << 20 and 1024 <= K <= 4096) \
+        or (N >= 100000 and 1536 <= K < 4096)
+
+
 def linear_auto(x, w):
-    """Shape-gated GEMM dispatch: the split-K skinny kernel where it
-    measured faster than hipBLASLt (scripts/bench_skinny_gemm.py on
-    MI355X: down_proj-like N=4096 K>=8192 M>=384 at splitk=4, 824 TF vs
-    hipBLASLt 680), F.linear everywhere else."""
+    """Shape-gated GEMM dispatch: the decode product for few rows
+    (_rows_gemm_wins), the split-K skinny kernel where it measured faster than
+    hipBLASLt (scripts/bench_skinny_gemm.py on MI355X: down_proj-like N=4096
+    K>=8192 M>=384 at splitk=4, 824 TF vs hipBLASLt 680), F.linear everywhere
+    else."""
     import os
 
     import torch.nn.functional as F
@@ -339,6 +357,15 @@ def linear_auto(x, w):
             and os.environ.get("GPUSTACK_AMD_SKINNY_GEMM", "1") == "1"):
         M, K = x.shape
         N = w.shape[0]
+        if (_rows_gemm_wins(M, N, K) and M > 0
+                and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+                and w.is_contiguous() and w.data_ptr() % 16 == 0
+                and x.stride(1) == 1 and x.stride(0) % 8 == 0
+                and x.data_ptr() % 16 == 0
+                and not (x.requires_grad or w.requires_grad)):
+            out = torch.empty(M, N, dtype=x.dtype, device=x.device)
+            _load_hip().rows_gemm(out, x, w)
+            return out
         if (N == 4096 and K >= 8192 and 384 <= M <= 1024
                 and K % 256 == 0 and x.stride(1) == 1):
             return skinny_gemm(x, w, splitk=4)

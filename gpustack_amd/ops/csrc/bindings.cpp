@@ -27,6 +27,7 @@ void moe_topk_launch(int*, float*, const float*, int, int, int, int, int*, hipSt
 void moe_sort_launch(int*, int*, int*, int*, int*, int*, const int*, int, int, int, int*, hipStream_t);
 void moe_sum_launch(void*, const void*, long, int, int, hipStream_t);
 void moe_tile_launch(int, void*, const void*, const void*, const int*, const int*, const int*, const int*, const int*, const float*, const void*, int, int, int, int, int*, hipStream_t);
+void rows_gemm_launch(void*, const void*, const void*, int, int, int, long, int*, hipStream_t);
 void w4_gemm_launch(void*, const void*, const void*, const void*, const void*, int, int, int, int*, hipStream_t);
 void w4_dequant_launch(void*, const void*, const void*, const void*, long, int, int*, hipStream_t);
 
@@ -453,6 +454,21 @@ void moe_tile(bool down, at::Tensor out, at::Tensor src, at::Tensor w,
   HIP_CHECK_LAST();
 }
 
+void rows_gemm(at::Tensor out, at::Tensor x, at::Tensor w) {
+  check_bf16(out, "out"); check_bf16(w, "w");
+  TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 && x.dim() == 2
+              && x.stride(1) == 1 && x.stride(0) % 8 == 0
+              && (uintptr_t)x.data_ptr() % 16 == 0, "x rows of bf16");
+  const int M = x.size(0), K = x.size(1), N = w.size(0);
+  TORCH_CHECK(w.size(1) == K && out.size(0) == M && out.size(1) == N,
+              "rows_gemm shapes");
+  int err = 0;
+  rows_gemm_launch(out.data_ptr(), x.data_ptr(), w.data_ptr(), M, N, K,
+                   x.stride(0), &err, cur_stream(x));
+  TORCH_CHECK(!err, "rows_gemm: unsupported M=", M, " K=", K);
+  HIP_CHECK_LAST();
+}
+
 void w4_gemm(at::Tensor out, at::Tensor x, at::Tensor qw, at::Tensor sc,
              at::Tensor zs) {
   check_bf16(out, "out"); check_bf16(x, "x");
@@ -536,6 +552,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_gemm", &skinny_gemm, "split-K skinny GEMM (bf16, f32 accum)");
   m.def("gemm8", &gemm8, "8-phase pipelined 256x256 GEMM (bf16, f32 accum)");
   m.def("gemm_lab", &gemm_lab, "GEMM schedule lab variants (A/B vs hipBLASLt)");
+  m.def("rows_gemm", &rows_gemm, "bf16 product of up to 64 rows");
   m.def("moe_topk", &moe_topk, "softmax routing, top k");
   m.def("moe_sort", &moe_sort, "assignments by expert, and the tile list");
   m.def("moe_sum", &moe_sum, "sum of a row's expert contributions");

@@ -1,121 +1,182 @@
-// W4A16 GEMM for MI355X (gfx950): out[M,N] = x[M,K] @ W^T with W kept
-// PACKED int4 in HBM and dequantized in-register ahead of the MFMAs.
-//
-// Round-2 item: GPTQ/AWQ/Q4 checkpoints previously
-// dequantized to bf16 at load (4x HBM inflation); this kernel halves the
-// weight traffic of decode-shaped GEMMs (M<=1k is weight-stream bound:
-// AI = M flop/byte) and keeps 70B-class models resident packed.
+// Products with packed int4 weights for MI355X (gfx950): out[M, N] =
+// x[M, K] W^T with W kept packed in HBM, and the transient expansion to bf16
+// that prompt-sized products use in front of the library GEMM.
 //
 // Packed layout (models/quantized.py pack_w4_runtime): qw u8 [N, K/2] in
-// FRAGMENT ORDER — within each 128-k block, the 16 bytes lane lg loads
-// contain exactly the 32 nibbles (4 MFMA k-chunks x 8 values) that form
-// its B-fragments, so no cross-lane shuffles are needed:
-//   nibble i (0..31) of lane lg's 16B = q[col][blk*128 + (i/8)*32 + lg*8 + i%8]
-// Scales/zero-scales: bf16 [N, K/128], one group per 128-k block
-// (checkpoint group sizes that divide into 128-blocks are expanded at
-// load). Dequant: w = q * s - zs   (zs = zero * s, precomputed).
+// FRAGMENT ORDER — within each 128-k block, the 16 bytes lane group lg loads
+// hold exactly the 32 nibbles (4 MFMA k-chunks x 8 values) of its operand
+// fragments:
+//   nibble i (0..31) of lg's 16 bytes = q[row][blk*128 + (i/8)*32 + lg*8 + i%8]
+// Scales / zero-scales: bf16 [N, K/128], one group per 128-k block.
+// w = q * s - zs   (zs = zero * s, precomputed).
 //
-// Tiling: BM=256 rows (16 m-frags) x BN=64 cols (4 waves x 16), K step
-// 128. Weights stream ONCE per 256-row M pass; X tiles stage through LDS
-// and re-reads across N-workgroups hit L2 (XCD-aware remap).
+// Few rows (decode). A workgroup of 8 waves owns 16 NTW columns of up to 64
+// rows; its waves take the k blocks in turn (8 neighbouring blocks of a row
+// are read together) and meet in the LDS at the end, so no second kernel and
+// no partial results in memory.
+//  - A nibble becomes bf16 without arithmetic: 0x4300 | q is 128 + q, two at
+//    a time (q_j beside q_{j+4}; x fragments are put in the same order with
+//    four v_perm). The products of a block are exact in q; its scale and
+//    offset are applied to the fp32 sums:
+//      out += s * (x . (128 + q)) - (128 s + zs) * sum(x),
+//    sum(x) coming from one more product with a fragment of ones, shared by
+//    the NTW column tiles. The weights are never rounded to bf16 here, as the
+//    expansion does.
+//  - 16-byte weight loads run one block ahead; scales are staged in the LDS.
+// Bound by the weight stream (0.5 bytes a weight).
 #include "common.h"
 
 namespace {
 
-constexpr int W4_BM = 256;
-constexpr int W4_BN = 64;
 constexpr int W4_KC = 128;
-constexpr int W4_THREADS = 256;  // 4 waves
-constexpr int W4_PAD = 8;        // elements; breaks the LDS bank cycle
+constexpr int W4_WAVES = 8;
+constexpr int W4_THREADS = W4_WAVES * WAVE_SIZE;
 
 typedef __attribute__((ext_vector_type(8))) short w4_s16x8;
 
-DEVICE_INLINE f32x4 w4_mfma(u16x8 a, u16x8 b, f32x4 c) {
+DEVICE_INLINE f32x4 w4_mfma(u32x4 a, u32x4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(
       __builtin_bit_cast(w4_s16x8, a), __builtin_bit_cast(w4_s16x8, b), c, 0, 0, 0);
 }
 
-__global__ __launch_bounds__(W4_THREADS) void w4_gemm_kernel(
-    unsigned short* __restrict__ out,     // [M, N] bf16
-    const unsigned short* __restrict__ x, // [M, K] bf16
-    const unsigned char* __restrict__ qw, // [N, K/2] frag-ordered nibbles
+// eight nibbles as bf16 128 + q in the order 0 4 1 5 2 6 3 7
+DEVICE_INLINE u32x4 w4_bf16(unsigned int d) {
+  u32x4 o;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    o[j] = ((d >> (4 * j)) & 0x000f000fu) | 0x43004300u;
+  return o;
+}
+
+// eight bf16 in that order
+DEVICE_INLINE u32x4 w4_order(u32x4 v) {
+  u32x4 o;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    o[2 * j] = __builtin_amdgcn_perm(v[2 + j], v[j], 0x05040100u);
+    o[2 * j + 1] = __builtin_amdgcn_perm(v[2 + j], v[j], 0x07060302u);
+  }
+  return o;
+}
+
+template <int MT, int NTW>
+__global__ __launch_bounds__(W4_THREADS) void w4_rows_kernel(
+    unsigned short* __restrict__ out,       // [M, N] bf16
+    const unsigned short* __restrict__ x,   // [M, K] bf16
+    const unsigned char* __restrict__ qw,   // [N, K/2] frag-ordered nibbles
     const unsigned short* __restrict__ sc,  // [N, K/128] bf16 scale
     const unsigned short* __restrict__ zs,  // [N, K/128] bf16 zero*scale
     int M, int N, int K) {
-  const int mtiles = (M + W4_BM - 1) / W4_BM;
-  const int nwg = mtiles * (N / W4_BN);
-  int wg = blockIdx.x;
-  {  // bijective XCD remap (8 XCDs share the X panel via their L2s)
-    const int q = nwg / 8, r = nwg % 8;
-    const int xcd = wg % 8, idx = wg / 8;
-    wg = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + idx;
-  }
-  const int m0 = (wg % mtiles) * W4_BM;
-  const int n0 = (wg / mtiles) * W4_BN;
+  constexpr int COLS = 16 * NTW, ROWS = 16 * MT;
+  extern __shared__ __attribute__((aligned(16))) float w4_lds[];
+  const int nb = K / W4_KC;
+  // scales of the workgroup's columns, [nb][COLS] (s low half, zs high), then
+  // the waves' partial sums [8][ROWS][COLS]
+  unsigned int* sz = reinterpret_cast<unsigned int*>(w4_lds);
 
+  const int m0 = blockIdx.y * ROWS;
+  const int n0 = blockIdx.x * COLS;
   const int tid = threadIdx.x;
   const int lane = tid & (WAVE_SIZE - 1);
-  const int wave = tid / WAVE_SIZE;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE_SIZE);
   const int lc = lane & 15;
   const int lg = lane >> 4;
-  const int col = n0 + wave * 16 + lc;  // this lane's output column
 
-  f32x4 acc[W4_BM / 16];
+  const unsigned char* wp[NTW];
 #pragma unroll
-  for (int mf = 0; mf < W4_BM / 16; ++mf) acc[mf] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const int nblk = K / W4_KC;
-  const long qrow = (long)col * (K / 2);
-  const long srow = (long)col * nblk;
-
-  // A-fragments read straight from L2 (decode-shaped X is a few MB and
-  // every N-workgroup re-reads the same panel): no LDS staging, no
-  // barriers, occupancy limited only by registers. Row base offsets are
-  // per-mf invariant; rows past M clamp to M-1 (stores are guarded).
-  long row_off[W4_BM / 16];
+  for (int t = 0; t < NTW; ++t)
+    wp[t] = qw + (long)(n0 + t * 16 + lc) * (K / 2) + lg * 16;
+  const unsigned short* xp[MT];
 #pragma unroll
-  for (int mf = 0; mf < W4_BM / 16; ++mf) {
-    int row = m0 + mf * 16 + lc;
-    if (row >= M) row = M - 1;
-    row_off[mf] = (long)row * K;
+  for (int t = 0; t < MT; ++t)
+    xp[t] = x + (long)min(m0 + t * 16 + lc, M - 1) * K + lg * 8;
+
+  // block numbers start at the workgroup's own place in the row: rows lie a
+  // power of two apart, and workgroups that all read the same columns of
+  // their rows would meet on a few memory channels
+  const int rot = blockIdx.x % nb;
+  auto block = [&](int b) { return b + rot < nb ? b + rot : b + rot - nb; };
+  u32x4 wc[NTW], wn[NTW];
+  const int b0 = block(min(wave, nb - 1));
+#pragma unroll
+  for (int t = 0; t < NTW; ++t)
+    wc[t] = *reinterpret_cast<const u32x4*>(wp[t] + (long)b0 * 64);
+
+  for (int u = tid; u < COLS * nb; u += W4_THREADS) {
+    const int c = u / nb, b = u % nb;
+    const long at = (long)(n0 + c) * nb + b;
+    sz[b * COLS + c] = (unsigned int)sc[at] | ((unsigned int)zs[at] << 16);
   }
+  __syncthreads();
 
-  for (int kb = 0; kb < nblk; ++kb) {
-    // lane's packed weights for this block: 16B = 4 dwords = 32 nibbles
-    const uint4 w = *reinterpret_cast<const uint4*>(
-        qw + qrow + (long)kb * 64 + lg * 16);
-    const float s = bf2f(sc[srow + kb]);
-    const float z = bf2f(zs[srow + kb]);
-    u16x8 bfr[4];
+  f32x4 acc[MT][NTW];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const unsigned int lo = (&w.x)[c];  // dword c = nibbles c*8..c*8+7
+  for (int i = 0; i < MT; ++i)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float q4 = (float)((lo >> (4 * j)) & 0xF);
-        bfr[c][j] = f2bf(q4 * s - z);
-      }
+    for (int t = 0; t < NTW; ++t) acc[i][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const u32x4 ones = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
+
+  for (int j = wave; j < nb; j += W4_WAVES) {
+    const int b = block(j), bn = block(min(j + W4_WAVES, nb - 1));
+#pragma unroll
+    for (int t = 0; t < NTW; ++t)
+      wn[t] = *reinterpret_cast<const u32x4*>(wp[t] + (long)bn * 64);
+    u32x4 xa[MT][4];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        xa[i][c] = w4_order(*reinterpret_cast<const u32x4*>(
+            xp[i] + b * W4_KC + c * 32));
+    f32x4 xs[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      xs[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < 4; ++c) xs[i] = w4_mfma(xa[i][c], ones, xs[i]);
     }
-    const int k0 = kb * W4_KC;
 #pragma unroll
-    for (int mf = 0; mf < W4_BM / 16; ++mf) {
+    for (int t = 0; t < NTW; ++t) {
+      f32x4 p[MT];
+#pragma unroll
+      for (int i = 0; i < MT; ++i) p[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        const u16x8 a = *reinterpret_cast<const u16x8*>(
-            x + row_off[mf] + k0 + c * 32 + lg * 8);
-        acc[mf] = w4_mfma(a, bfr[c], acc[mf]);
+        const u32x4 wf = w4_bf16(wc[t][c]);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) p[i] = w4_mfma(xa[i][c], wf, p[i]);
       }
+      const unsigned int v = sz[b * COLS + t * 16 + lc];
+      const float s = __builtin_bit_cast(float, v << 16);
+      const float z = 128.f * s + __builtin_bit_cast(float, v & 0xffff0000u);
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          acc[i][t][r] += s * p[i][r] - z * xs[i][r];
+      wc[t] = wn[t];
     }
   }
 
+  __syncthreads();                       // the scales are done with
   // D[row = lg*4 + r][col = lc] per 16x16 tile
+  float* red = w4_lds;
 #pragma unroll
-  for (int mf = 0; mf < W4_BM / 16; ++mf) {
+  for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = m0 + mf * 16 + lg * 4 + r;
-      if (row < M) out[(long)row * N + col] = f2bf(acc[mf][r]);
-    }
+    for (int t = 0; t < NTW; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        red[(wave * ROWS + i * 16 + lg * 4 + r) * COLS + t * 16 + lc] =
+            acc[i][t][r];
+  __syncthreads();
+  for (int u = tid; u < ROWS * COLS; u += W4_THREADS) {
+    const int row = m0 + u / COLS;
+    if (row >= M) break;
+    float v = 0.f;
+#pragma unroll
+    for (int w = 0; w < W4_WAVES; ++w) v += red[w * ROWS * COLS + u];
+    out[(long)row * N + n0 + u % COLS] = f2bf(v);
   }
 }
 
@@ -170,15 +231,45 @@ void w4_dequant_launch(void* out, const void* qw, const void* sc,
                      K);
 }
 
+namespace {
+template <int MT, int NTW>
+void w4_rows(void* out, const void* x, const void* qw, const void* sc,
+             const void* zs, int M, int N, int K, hipStream_t s) {
+  const size_t scales = (size_t)(K / W4_KC) * 16 * NTW * 4;
+  const size_t sums = (size_t)W4_WAVES * 16 * MT * 16 * NTW * 4;
+  hipLaunchKernelGGL((w4_rows_kernel<MT, NTW>),
+                     dim3(N / (16 * NTW), (M + 16 * MT - 1) / (16 * MT)),
+                     dim3(W4_THREADS), scales > sums ? scales : sums, s,
+                     (unsigned short*)out, (const unsigned short*)x,
+                     (const unsigned char*)qw, (const unsigned short*)sc,
+                     (const unsigned short*)zs, M, N, K);
+}
+}  // namespace
+
+// Column tiles per wave: one while that leaves fewer than 448 workgroups of
+// two (a short weight needs every wave of the chip), else as many as share
+// the x fragments best; the scales of K / 128 blocks stay under 64 KB.
 void w4_gemm_launch(void* out, const void* x, const void* qw, const void* sc,
                     const void* zs, int M, int N, int K,
                     int* err_unsupported, hipStream_t s) {
   *err_unsupported = 0;
-  if (N % W4_BN != 0 || K % W4_KC != 0) { *err_unsupported = 1; return; }
-  const int mtiles = (M + W4_BM - 1) / W4_BM;
-  dim3 grid(mtiles * (N / W4_BN));
-  hipLaunchKernelGGL(w4_gemm_kernel, grid, dim3(W4_THREADS), 0, s,
-                     (unsigned short*)out, (const unsigned short*)x,
-                     (const unsigned char*)qw, (const unsigned short*)sc,
-                     (const unsigned short*)zs, M, N, K);
+  if (N % 64 != 0 || K % W4_KC != 0 || K / W4_KC > 1024) {
+    *err_unsupported = 1;
+    return;
+  }
+  if (M == 0) return;
+  const int nb = K / W4_KC;
+  const int ntw = N / 64 >= 448 && nb <= 256 ? 4
+                  : N / 32 >= 448 && nb <= 512 ? 2 : 1;
+#define W4_ROWS(MT)                                                          \
+  do {                                                                       \
+    if (ntw == 4) w4_rows<MT, (MT) == 4 ? 2 : 4>(out, x, qw, sc, zs, M, N,   \
+                                                 K, s);                      \
+    else if (ntw == 2) w4_rows<MT, 2>(out, x, qw, sc, zs, M, N, K, s);       \
+    else w4_rows<MT, 1>(out, x, qw, sc, zs, M, N, K, s);                     \
+  } while (0)
+  if (M <= 16) W4_ROWS(1);
+  else if (M <= 32) W4_ROWS(2);
+  else W4_ROWS(4);
+#undef W4_ROWS
 }

@@ -1,0 +1,73 @@
+"""Decode products of few rows, bf16 and packed int4: rows and columns at the
+edges of their 16-wide tiles, block counts that the 8 waves do not divide, and
+every column width that the launch chooses between; the argmax over a row."""
+import pytest
+import torch
+
+pytestmark = [pytest.mark.gpu,
+              pytest.mark.skipif(not torch.cuda.is_available(),
+                                 reason="needs a GPU")]
+
+
+def _hip():
+    from gpustack_amd import ops
+
+    return ops._load_hip()
+
+
+def _close(out, ref, size):
+    # rounded to bf16 once (at most 2^-8 of the value); fp32 sums of terms
+    # that add up to `size` in absolute value are off by less than 2^-18 of it
+    err = (out.double() - ref).abs()
+    bound = ref.abs() * 2.0 ** -8 + size * 2.0 ** -18
+    assert bool((err <= bound).all()), float((err - bound).max())
+
+
+@pytest.mark.parametrize("M", [1, 15, 16, 17, 33, 64])
+@pytest.mark.parametrize("N,K", [(16, 128), (100, 1152), (4096, 1024),
+                                 (16400, 256)])
+def test_rows_gemm(M, N, K):
+    g = torch.Generator(device="cuda").manual_seed(M * N)
+    x = torch.randn(M, K + 8, generator=g, device="cuda").bfloat16()[:, :K]
+    w = torch.randn(N, K, generator=g, device="cuda").bfloat16()
+    out = torch.full((M, N), 9.0, device="cuda").bfloat16()
+    _hip().rows_gemm(out, x, w)
+    _close(out, x.double() @ w.double().T, x.double().abs() @ w.double().abs().T)
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 64, 65])
+@pytest.mark.parametrize("N,K", [(64, 128), (128, 1152), (14400, 256),
+                                 (28736, 384)])
+def test_w4_rows(M, N, K):
+    import gpustack_amd.engine  # noqa: F401  (package import order)
+    from gpustack_amd.models.quantized import pack_w4_runtime
+
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    q = torch.randint(0, 16, (N, K), generator=g, device="cuda")
+    sc = torch.rand(N, K // 128, generator=g, device="cuda") * 0.05 + 0.01
+    zr = torch.randint(0, 16, (N, K // 128), generator=g, device="cuda").float()
+    qw, s, z = pack_w4_runtime(q, sc, zr, 128)
+    x = (torch.randn(M, K, generator=g, device="cuda") + 0.5).bfloat16()
+    out = torch.full((M, N), 9.0, device="cuda").bfloat16()
+    _hip().w4_gemm(out, x, qw, s, z)
+    wide = lambda t: t.double().repeat_interleave(128, 1)
+    w = q.double() * wide(s) - wide(z)
+    # sums run over 128 + q and are corrected by 128 times the sum of x
+    size = x.double().abs() @ (wide(s) * 144 + wide(z).abs()).T
+    _close(out, x.double() @ w.T, size)
+
+
+@pytest.mark.parametrize("V", [7, 1000, 32776, 128256])
+def test_argmax_of_a_row(V):
+    from gpustack_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(V)
+    x = torch.randn(9, V, generator=g, device="cuda")
+    x[0] = -1.0                           # all alike: the first
+    x[1, -1] = 50.0
+    x[2, V // 2:] = 60.0                  # the first of many
+    x[3] = float("-inf")
+    x[3, V // 3] = -1e30
+    for t in (x.bfloat16(), x):
+        ref = torch.stack([(r == r.max()).nonzero()[0, 0] for r in t.float()])
+        assert torch.equal(ops.greedy_sample(t), ref)
