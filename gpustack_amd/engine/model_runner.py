@@ -538,7 +538,8 @@ class ModelRunner:
             starts, hists, news = [0], [0], [1]
             bt[nseq] = bt[0]
         tokens = torch.as_tensor(tok_l, dtype=torch.long).to(dev)
-        tiles = ops.build_paged_prefill_tiles(starts, hists, news, dev)
+        tiles = ops.build_paged_prefill_tiles(starts, hists, news, dev,
+                                                  ops.PREFILL_ROWS)
         meta = ForwardMeta(
             is_prefill=False,
             positions=torch.as_tensor(pos_l, dtype=torch.long).to(dev),
@@ -642,7 +643,7 @@ class ModelRunner:
             n_dec = len(batch.seqs) - n_pre
             # decode rows (mixed batch) produce logits directly
             idx.extend(range(tp, tp + n_dec))
-            tiles = ops.build_prefill_tiles(pre_lens, dev)
+            tiles = ops.build_prefill_tiles(pre_lens, dev, ops.PREFILL_ROWS)
             bt = None
             dec_lens = None
             if self.cfg.spec.kv_lora_rank and dev.type == "cuda":
@@ -701,7 +702,8 @@ class ModelRunner:
                 for i, s in enumerate(batch.seqs):
                     bt[i, : len(s.block_table)] = torch.tensor(
                         s.block_table, dtype=torch.int32)
-                tiles = ops.build_paged_prefill_tiles(starts, hists, news, dev)
+                tiles = ops.build_paged_prefill_tiles(starts, hists, news, dev,
+                                                  ops.PREFILL_ROWS)
                 meta = ForwardMeta(
                     is_prefill=False,
                     positions=positions,
@@ -772,7 +774,7 @@ class ModelRunner:
         tokens = torch.tensor(flat, dtype=torch.long, device=dev)
         pos = torch.tensor(positions, dtype=torch.long, device=dev)
         slots = torch.full((len(flat),), -1, dtype=torch.long, device=dev)
-        tiles = ops.build_prefill_tiles(lens, dev)
+        tiles = ops.build_prefill_tiles(lens, dev, ops.PREFILL_ROWS)
         idx, off = [], 0
         for L in lens:
             idx.append(off + L - 1)
@@ -809,7 +811,7 @@ class ModelRunner:
         tokens = torch.tensor(flat, dtype=torch.long, device=dev)
         pos = torch.tensor(positions, dtype=torch.long, device=dev)
         slots = torch.full((len(flat),), -1, dtype=torch.long, device=dev)
-        tiles = ops.build_prefill_tiles(lens, dev)
+        tiles = ops.build_prefill_tiles(lens, dev, ops.PREFILL_ROWS)
         meta = ForwardMeta(
             is_prefill=True, positions=pos, slot_mapping=slots,
             logits_indices=torch.zeros(1, dtype=torch.long, device=dev),

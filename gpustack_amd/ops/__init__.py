@@ -186,15 +186,20 @@ def mla_decode(ctx_out, q_cat, lat_cache, block_tables, seq_lens,
     hip.mla_decode(ctx_out, q_cat, lat_cache, block_tables, seq_lens, scale)
 
 
-_PREFILL_BQ = 128
+_PREFILL_BQ = 64
+# rows of a workgroup of the prompt kernels: a list of such tiles has no entry
+# that they pass over (in a list of 64-row tiles every second one is)
+PREFILL_ROWS = 128
 
 
-def build_prefill_tiles(seq_lens: list[int], device) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-    """Map varlen sequences to fixed 128-row q tiles for the MFMA kernel."""
+def build_prefill_tiles(seq_lens: list[int], device,
+                        rows: int = _PREFILL_BQ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """Map varlen sequences to q tiles of `rows` (64 or PREFILL_ROWS) for the
+    MFMA kernel."""
     starts, q0s, lens = [], [], []
     tok = 0
     for L in seq_lens:
-        for q0 in range(0, L, _PREFILL_BQ):
+        for q0 in range(0, L, rows):
             starts.append(tok)
             q0s.append(q0)
             lens.append(L)
@@ -218,7 +223,7 @@ def varlen_prefill_attn(out, q, k, v, seq_lens: list[int], scale: float,
                 "GPUSTACK_AMD_MLA_KERNEL=1 for the 192/128 MLA expand "
                 "shape) to opt in")
         if tiles is None or tiles[0] is None:
-            tiles = build_prefill_tiles(seq_lens, q.device)
+            tiles = build_prefill_tiles(seq_lens, q.device, PREFILL_ROWS)
         hip.flash_prefill(out, q, k, v, tiles[0], tiles[1], tiles[2], scale,
                           sinks=_sinks_f32(sinks), window=window,
                           softcap=softcap)
@@ -229,12 +234,13 @@ def varlen_prefill_attn(out, q, k, v, seq_lens: list[int], scale: float,
 
 
 def build_paged_prefill_tiles(seq_starts: list[int], seq_hists: list[int],
-                              seq_news: list[int], device):
-    """Map per-seq suffix rows to fixed 128-row q tiles for the paged
-    prefill-with-history kernel (one entry set per (seq, q-tile))."""
+                              seq_news: list[int], device,
+                              rows: int = _PREFILL_BQ):
+    """Map per-seq suffix rows to q tiles of `rows` (64 or PREFILL_ROWS) for
+    the paged prefill-with-history kernel (one entry set per (seq, q-tile))."""
     qstart, q0s, hists, news, seqi = [], [], [], [], []
     for i, (st, h, n) in enumerate(zip(seq_starts, seq_hists, seq_news)):
-        for q0 in range(0, n, _PREFILL_BQ):
+        for q0 in range(0, n, rows):
             qstart.append(st)
             q0s.append(q0)
             hists.append(h)
@@ -262,7 +268,8 @@ def paged_prefill_attn(out, q, k_cache, v_cache, block_tables,
                 "to opt in")
         if tiles is None:
             tiles = build_paged_prefill_tiles(seq_starts, seq_hists,
-                                              seq_news, q.device)
+                                              seq_news, q.device,
+                                              PREFILL_ROWS)
         hip.flash_prefill_paged(out, q, k_cache, v_cache, block_tables,
                                 tiles[0], tiles[1], tiles[2], tiles[3],
                                 tiles[4], scale, sinks=_sinks_f32(sinks),

@@ -107,6 +107,7 @@ void flash_prefill_kernel(
   const int kvh = qh / (Hq / Hkv);
   const int row0 = tile_start[tile];
   const int q0 = tile_q0[tile];
+  if (q0 % BQ != 0) return;          // the second half of a list of 64-row tiles
   const int hist = PAGED ? tile_hist[tile] : 0;
   const int nnew = tile_new[tile];
   const int len = hist + nnew;

@@ -90,3 +90,22 @@ def test_rows_behind_history(Hq, Hkv, seqs):
         st = starts[i]
         _check(out[st:st + n], q[st:st + n], pools[0][blk, :, j % 16],
                pools[1][blk, :, j % 16], h, scale)
+
+
+@pytest.mark.parametrize("rows", [64, 128])
+def test_tile_lists_of_either_size(rows):
+    from gpustack_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    lens = [1, 64, 65, 193]
+    q = torch.randn(sum(lens), 8, 128, generator=g, device="cuda").bfloat16()
+    k, v = (torch.randn(sum(lens), 2, 128, generator=g,
+                        device="cuda").bfloat16() for _ in range(2))
+    out = torch.full_like(q, 9.0)
+    ops.varlen_prefill_attn(out, q, k, v, lens, 0.1, tiles=ops.
+                            build_prefill_tiles(lens, "cuda", rows))
+    at = 0
+    for n in lens:
+        _check(out[at:at + n], q[at:at + n], k[at:at + n], v[at:at + n], 0,
+               0.1)
+        at += n
