@@ -277,7 +277,7 @@ class EagleProposer:
         dev = self.device
         e = F.embedding(tokens, self.model.embed)
         x = F.linear(torch.cat([e, h_prev], dim=-1), self.fc_ws[0])
-        tiles = ops.build_prefill_tiles(lens, dev)
+        tiles = ops.build_prefill_tiles(lens, dev, ops.PREFILL_ROWS)
         meta = ForwardMeta(
             is_prefill=True,
             positions=positions,

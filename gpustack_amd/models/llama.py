@@ -270,35 +270,20 @@ class Attention(nn.Module):
         q = qkv[:, :nq].unflatten(1, (self.hq, self.d))
         k = qkv[:, nq:nq + nk].unflatten(1, (self.hkv, self.d))
         v = qkv[:, nq + nk:].unflatten(1, (self.hkv, self.d))
-        if self.spec.qk_norm and not self.spec.qk_norm_after_rope:
-            q = q.contiguous()
-            k = k.contiguous()
-            v = v.contiguous()
-            if self.spec.qk_norm_full:
-                self._full_qk_norm(q, k)
-            else:
-                ops.rms_norm(q.view(-1, self.d), q.view(-1, self.d), self.q_norm, self.spec.rms_norm_eps)
-                ops.rms_norm(k.view(-1, self.d), k.view(-1, self.d), self.k_norm, self.spec.rms_norm_eps)
-        if self.use_rope:
-            ops.rotary_embedding(meta.positions, q, k, cos_sin, self.d,
-                                 self.rot_dim, mode=self.spec.rope_mode)
-        if self.spec.qk_norm and self.spec.qk_norm_after_rope:
-            # Hunyuan-dense: per-head norm on the ROTATED q/k
-            q = q.contiguous()
-            k = k.contiguous()
-            v = v.contiguous()
-            ops.rms_norm(q.view(-1, self.d), q.view(-1, self.d),
-                         self.q_norm, self.spec.rms_norm_eps)
-            ops.rms_norm(k.view(-1, self.d), k.view(-1, self.d),
-                         self.k_norm, self.spec.rms_norm_eps)
-        if meta.cp is not None:
-            # CP prefill: assemble the full-batch K/V (global position
-            # order) so the cache write below covers every chunk, not just
-            # this rank's rows; q/attention stay local-row
-            kw, vw = meta.cp.gather_kv(k.contiguous(), v.contiguous())
+        head_norm = self.spec.qk_norm and not (
+            self.spec.qk_norm_full or self.spec.qk_norm_after_rope)
+        if (meta.cp is None and self.use_rope
+                and (head_norm or not self.spec.qk_norm)
+                and ops.qkv_store_ok(qkv, self.d, self.rot_dim,
+                                     self.spec.rope_mode)):
+            ops.qkv_store(qkv, self.hq, self.hkv,
+                          self.q_norm if head_norm else None,
+                          self.k_norm if head_norm else None, cos_sin,
+                          meta.positions, meta.slot_mapping, k_cache, v_cache,
+                          self.spec.rms_norm_eps)
         else:
-            kw, vw = k, v
-        ops.reshape_and_cache(kw, vw, k_cache, v_cache, meta.slot_mapping)
+            q, k, v = self._norm_rope_store(q, k, v, meta, cos_sin, k_cache,
+                                            v_cache)
         out = torch.empty(T, self.hq, self.d, dtype=q.dtype, device=q.device)
         sw = {}
         if self.sinks is not None or self.window:
@@ -330,6 +315,41 @@ class Attention(nn.Module):
         if meta.lora is not None:
             meta.lora.apply(self.layer_idx, out.view(T, -1), o, self._o_projs)
         return self.comm.all_reduce(o)
+
+    def _norm_rope_store(self, q, k, v, meta, cos_sin, k_cache, v_cache):
+        """Norms, rotation and cache write as steps of their own: the CPU,
+        context parallelism, partial or pairwise rotation, whole-projection
+        norms and norms behind the rotation."""
+        if self.spec.qk_norm and not self.spec.qk_norm_after_rope:
+            q = q.contiguous()
+            k = k.contiguous()
+            v = v.contiguous()
+            if self.spec.qk_norm_full:
+                self._full_qk_norm(q, k)
+            else:
+                ops.rms_norm(q.view(-1, self.d), q.view(-1, self.d), self.q_norm, self.spec.rms_norm_eps)
+                ops.rms_norm(k.view(-1, self.d), k.view(-1, self.d), self.k_norm, self.spec.rms_norm_eps)
+        if self.use_rope:
+            ops.rotary_embedding(meta.positions, q, k, cos_sin, self.d,
+                                 self.rot_dim, mode=self.spec.rope_mode)
+        if self.spec.qk_norm and self.spec.qk_norm_after_rope:
+            # Hunyuan-dense: per-head norm on the ROTATED q/k
+            q = q.contiguous()
+            k = k.contiguous()
+            v = v.contiguous()
+            ops.rms_norm(q.view(-1, self.d), q.view(-1, self.d),
+                         self.q_norm, self.spec.rms_norm_eps)
+            ops.rms_norm(k.view(-1, self.d), k.view(-1, self.d),
+                         self.k_norm, self.spec.rms_norm_eps)
+        if meta.cp is not None:
+            # CP prefill: assemble the full-batch K/V (global position
+            # order) so the cache write below covers every chunk, not just
+            # this rank's rows; q/attention stay local-row
+            kw, vw = meta.cp.gather_kv(k.contiguous(), v.contiguous())
+        else:
+            kw, vw = k, v
+        ops.reshape_and_cache(kw, vw, k_cache, v_cache, meta.slot_mapping)
+        return q, k, v
 
     def _full_qk_norm(self, q, k):
         """OLMo-2 full-projection RMSNorm: the mean square runs over ALL

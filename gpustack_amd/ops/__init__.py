@@ -125,6 +125,23 @@ def reshape_and_cache(k, v, k_cache, v_cache, slots) -> None:
         torch_ref.reshape_and_cache(k, v, k_cache, v_cache, slots)
 
 
+def qkv_store_ok(qkv, head_dim: int, rot_dim: int, mode: str) -> bool:
+    """True where ops.qkv_store takes a fused projection: bf16 rows on the
+    GPU, whole heads of 64, 128 or 256 channels rotated in halves."""
+    return (qkv.is_cuda and qkv.dtype == torch.bfloat16 and qkv.dim() == 2
+            and qkv.is_contiguous() and mode == "neox"
+            and rot_dim == head_dim and head_dim in (64, 128, 256))
+
+
+def qkv_store(qkv, q_heads: int, kv_heads: int, q_norm, k_norm, cos_sin,
+              positions, slots, k_cache, v_cache, eps: float) -> None:
+    """qkv [T, (q_heads + 2 kv_heads) * D]: weighted RMS norm of every q and k
+    head (where weights are given), rotation of q and k in place, keys and
+    values to their slots (-1: none). GPU only (qkv_store_ok)."""
+    _load_hip().qkv_store(qkv, q_heads, kv_heads, q_norm, k_norm, cos_sin,
+                          positions, slots, k_cache, v_cache, eps)
+
+
 def greedy_sample_into(out, logits) -> None:
     if logits.is_cuda and logits.dtype == torch.float32:
         # fp32-logit models: whichever fp32-stream library is loaded

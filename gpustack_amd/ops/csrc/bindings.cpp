@@ -12,6 +12,7 @@ void silu_and_mul_launch(void*, const void*, long, int, hipStream_t);
 void reshape_and_cache_launch(const void*, const void*, void*, void*, const long*, int, int, int, int, long, long, int, hipStream_t);
 void greedy_sample_launch(long*, const void*, int, int, hipStream_t);
 void mla_decode_launch(float*, const void*, const void*, const int*, const int*, int, int, int, int, int, int, float, int*, hipStream_t);
+void qkv_store_launch(void*, const void*, const void*, const float*, const long*, const long*, void*, void*, long, int, int, int, int, float, int, int*, hipStream_t);
 int decode_splits(int, int, int);
 void paged_attn_decode_launch(void*, const void*, const void*, const void*, const int*, const int*, float*, int, int, int, int, int, int, float, long, int, const float*, int, float, int*, hipStream_t);
 void flash_prefill_launch(void*, const void*, const void*, const void*, const int*, const int*, const int*, int, int, int, int, int, float, long, long, long, const float*, int, float, int*, hipStream_t);
@@ -133,6 +134,43 @@ void reshape_and_cache(at::Tensor k, at::Tensor v, at::Tensor k_cache,
                            v_cache.data_ptr(), slots.data_ptr<long>(), T, Hkv,
                            D, BS, ks, vs, is_fp8_cache(k_cache) ? 1 : 0,
                            cur_stream(k));
+  HIP_CHECK_LAST();
+}
+
+void qkv_store(at::Tensor qkv, long Hq, long Hk,
+               c10::optional<at::Tensor> q_norm,
+               c10::optional<at::Tensor> k_norm, at::Tensor cos_sin,
+               at::Tensor positions, at::Tensor slots, at::Tensor k_cache,
+               at::Tensor v_cache, double eps) {
+  check_bf16(qkv, "qkv");
+  check_cache(k_cache, "k_cache"); check_cache(v_cache, "v_cache");
+  const long T = qkv.size(0);
+  const int D = k_cache.size(3), BS = k_cache.size(2);
+  TORCH_CHECK(qkv.dim() == 2 && qkv.size(1) == (Hq + 2 * Hk) * D
+              && k_cache.size(1) == Hk && k_cache.sizes() == v_cache.sizes()
+              && k_cache.scalar_type() == v_cache.scalar_type(),
+              "qkv_store shapes");
+  TORCH_CHECK(positions.is_cuda() && positions.scalar_type() == at::kLong
+              && positions.is_contiguous() && positions.numel() == T);
+  TORCH_CHECK(slots.is_cuda() && slots.scalar_type() == at::kLong
+              && slots.is_contiguous() && slots.numel() == T);
+  TORCH_CHECK(cos_sin.is_cuda() && cos_sin.scalar_type() == at::kFloat
+              && cos_sin.is_contiguous() && cos_sin.size(1) == D);
+  const void* nw[2] = {nullptr, nullptr};
+  const c10::optional<at::Tensor>* given[2] = {&q_norm, &k_norm};
+  for (int i = 0; i < 2; ++i)
+    if (given[i]->has_value()) {
+      check_bf16(**given[i], "head norm");
+      TORCH_CHECK((*given[i])->numel() == D, "head norm [D]");
+      nw[i] = (*given[i])->data_ptr();
+    }
+  int err = 0;
+  qkv_store_launch(qkv.data_ptr(), nw[0], nw[1], cos_sin.data_ptr<float>(),
+                   positions.data_ptr<long>(), slots.data_ptr<long>(),
+                   k_cache.data_ptr(), v_cache.data_ptr(), T, (int)Hq,
+                   (int)Hk, D, BS, (float)eps, is_fp8_cache(k_cache) ? 1 : 0,
+                   &err, cur_stream(qkv));
+  TORCH_CHECK(!err, "qkv_store: unsupported head_dim ", D);
   HIP_CHECK_LAST();
 }
 
@@ -528,6 +566,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rotary_embedding", &rotary_embedding, "in-place neox RoPE on q,k");
   m.def("silu_and_mul", &silu_and_mul, "silu(x[:d])*x[d:]");
   m.def("reshape_and_cache", &reshape_and_cache, "scatter K/V into paged pool");
+  m.def("qkv_store", &qkv_store,
+        "head norms, rotation in place and cache write of a q|k|v row");
   m.def("greedy_sample", &greedy_sample, "argmax over vocab");
   m.def("mla_decode", &mla_decode,
         "MLA absorbed decode over the paged latent cache (DeepSeek)");

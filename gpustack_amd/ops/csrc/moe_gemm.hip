@@ -494,8 +494,18 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   for (int e = tid; e < MOE_MAX_E; e += 1024) cnt[e] = 0;
   __syncthreads();
-  for (int i = tid; i < TK; i += 1024)
-    atomicAdd(&cnt[min(max(experts[i], 0), E - 1)], 1);
+  auto walk = [&](auto f) {            // eight loads in flight a thread
+    int i = tid;
+    for (; i + 7 * 1024 < TK; i += 8 * 1024) {
+      int e[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) e[j] = experts[i + j * 1024];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f(i + j * 1024, min(max(e[j], 0), E - 1));
+    }
+    for (; i < TK; i += 1024) f(i, min(max(experts[i], 0), E - 1));
+  };
+  walk([&](int, int e) { atomicAdd(&cnt[e], 1); });
   __syncthreads();
   // thread tid owns experts EPT * tid ..
   constexpr int EPT = MOE_MAX_E / 1024;
@@ -542,11 +552,11 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(
     a += c[j];
   }
   __syncthreads();
-  for (int i = tid; i < TK; i += 1024) {
-    const int at = atomicAdd(&cnt[min(max(experts[i], 0), E - 1)], 1);
+  walk([&](int i, int e) {
+    const int at = atomicAdd(&cnt[e], 1);
     order[at] = i;
     s_tok[at] = i / k;
-  }
+  });
 }
 
 // out[t] = sum over the k contributions of row t, in fp32 in their order.

@@ -251,6 +251,90 @@ __global__ void reshape_and_cache_kernel(const unsigned short* __restrict__ k,
 }
 
 // ---------------------------------------------------------------------------
+// The way from a fused q|k|v projection row to attention in one launch:
+// optional RMS norm of every q and k head (one weight vector each), rotation
+// of q and k in place (halves), keys and values to their cache slots (-1 =
+// skip). LPH = D / 16 lanes share a head: a lane holds 8 channels of the first
+// half and the 8 that they rotate with, so the pair is in its registers and
+// the norm takes log2(LPH) cross-lane steps. Bound by the row's bytes; two
+// norms, three copies, rotation and cache write as launches of their own took
+// 170 us a layer at 4068 rows of 32 + 2 x 4 heads (a workgroup per head).
+// ---------------------------------------------------------------------------
+template <int LPH, bool FP8>
+__global__ __launch_bounds__(256) void qkv_store_kernel(
+    unsigned short* __restrict__ qkv,          // [T, (Hq + 2 Hk) * D]
+    const unsigned short* __restrict__ qw,     // [D] or null
+    const unsigned short* __restrict__ kw,     // [D] or null
+    const float* __restrict__ cos_sin,         // [positions, D]
+    const long* __restrict__ positions, const long* __restrict__ slots,
+    void* __restrict__ kc, void* __restrict__ vc,  // [nb, Hk, BS, D]
+    long heads, int Hq, int Hk, int BS, float eps) {
+  constexpr int D = LPH * 16, HALF = D / 2;
+  const int H = Hq + 2 * Hk;
+  const int c = threadIdx.x % LPH * 8;
+  const long step = (long)gridDim.x * (256 / LPH);
+  for (long u = (long)blockIdx.x * (256 / LPH) + threadIdx.x / LPH; u < heads;
+       u += step) {
+    const long t = u / H;
+    const int h = (int)(u % H);
+    unsigned short* p = qkv + u * D + c;
+    u16x8 a = *reinterpret_cast<const u16x8*>(p);
+    u16x8 b = *reinterpret_cast<const u16x8*>(p + HALF);
+    if (h < Hq + Hk) {
+      float x[8], y[8], o[8];
+      bf8_to_f32(a, x);
+      bf8_to_f32(b, y);
+      const unsigned short* w = h < Hq ? qw : kw;
+      if (w != nullptr) {
+        float ss = 0.f, wx[8], wy[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) ss += x[i] * x[i] + y[i] * y[i];
+#pragma unroll
+        for (int m = LPH / 2; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, 64);
+        const float inv = rsqrtf(ss / D + eps);
+        bf8_to_f32(*reinterpret_cast<const u16x8*>(w + c), wx);
+        bf8_to_f32(*reinterpret_cast<const u16x8*>(w + c + HALF), wy);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          x[i] *= inv * wx[i];
+          y[i] *= inv * wy[i];
+        }
+      }
+      const float* cs = cos_sin + positions[t] * D + c;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float co = cs[i], si = cs[HALF + i];
+        o[i] = x[i] * co - y[i] * si;
+        y[i] = y[i] * co + x[i] * si;
+      }
+      a = f32_to_bf8(o);
+      b = f32_to_bf8(y);
+      *reinterpret_cast<u16x8*>(p) = a;
+      *reinterpret_cast<u16x8*>(p + HALF) = b;
+    }
+    if (h < Hq) continue;
+    const long slot = slots[t];
+    if (slot < 0) continue;
+    const int g = (h - Hq) % Hk;
+    const long dst = ((slot / BS * Hk + g) * BS + slot % BS) * D + c;
+    void* pool = h < Hq + Hk ? kc : vc;
+    if constexpr (FP8) {
+      u8x8 qa, qb;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        qa[i] = f32_to_fp8(bf2f(a[i]));
+        qb[i] = f32_to_fp8(bf2f(b[i]));
+      }
+      *reinterpret_cast<u8x8*>((unsigned char*)pool + dst) = qa;
+      *reinterpret_cast<u8x8*>((unsigned char*)pool + dst + HALF) = qb;
+    } else {
+      *reinterpret_cast<u16x8*>((unsigned short*)pool + dst) = a;
+      *reinterpret_cast<u16x8*>((unsigned short*)pool + dst + HALF) = b;
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Greedy sampling: argmax over vocab per row (ties -> lowest index).
 // One block per row: 16 waves with four 16-byte loads in flight each, the
 // maximum of eight values first and its place only where it counts. Bound by
@@ -386,4 +470,33 @@ void greedy_sample_launch(long* out, const void* logits, int N, int V,
   if (N == 0) return;
   hipLaunchKernelGGL(greedy_sample_kernel, dim3(N), dim3(GS_THREADS), 0, s, out,
                      (const unsigned short*)logits, N, V);
+}
+
+void qkv_store_launch(void* qkv, const void* qw, const void* kw,
+                      const float* cos_sin, const long* positions,
+                      const long* slots, void* kc, void* vc, long T, int Hq,
+                      int Hk, int D, int BS, float eps, int fp8,
+                      int* err_unsupported, hipStream_t s) {
+  *err_unsupported = D != 64 && D != 128 && D != 256;
+  const long heads = T * (Hq + 2 * Hk);
+  if (*err_unsupported || heads == 0) return;
+  const long per = 256 / (D / 16);
+  const long blocks = (heads + per - 1) / per;
+  const unsigned grid = (unsigned)(blocks > 16384 ? 16384 : blocks);
+#define QKV(L, F)                                                             \
+  hipLaunchKernelGGL((qkv_store_kernel<L, F>), dim3(grid), dim3(256), 0, s,   \
+                     (unsigned short*)qkv, (const unsigned short*)qw,         \
+                     (const unsigned short*)kw, cos_sin, positions, slots,    \
+                     kc, vc, heads, Hq, Hk, BS, eps)
+  if (D == 64) {
+    if (fp8) QKV(4, true);
+    else QKV(4, false);
+  } else if (D == 128) {
+    if (fp8) QKV(8, true);
+    else QKV(8, false);
+  } else {
+    if (fp8) QKV(16, true);
+    else QKV(16, false);
+  }
+#undef QKV
 }
