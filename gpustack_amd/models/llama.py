@@ -905,10 +905,6 @@ class MoEMLP(nn.Module):
                 and self.i % 128 == 0 and x.shape[1] % 128 == 0
                 and self.e <= 4096 and ops.hip_available())
 
-    # Rows per expert from which the 128-row tiles are faster than the
-    # 16-row form, which streams an expert's weights once per 16 rows
-    _TILE_ROWS = 24
-
     def _fused_dispatch(self, x, experts, weights):
         """Sync-free grouped expert products: sort the assignments by expert
         on the device, run the two expert kernels, sum over the k axis. Every
@@ -926,18 +922,19 @@ class MoEMLP(nn.Module):
         db = self.down_b if self.comm.tp_rank == 0 else None
         act = x.new_empty(TK, self.i)
         contrib = x.new_empty(TK, x.shape[1])
-        if TK >= self._TILE_ROWS * self.e:
-            hip.moe_tile(False, act, x, self._bank("gate_up"), s_tok, tiles,
-                         ntiles, offs, counts, bias=self.gate_up_b,
-                         act_mode=act_mode)
-            hip.moe_tile(True, contrib, act, self._bank("down"), order, tiles,
-                         ntiles, offs, counts, flat_w, bias=db)
-        else:
-            hip.moe_gate_up_silu(act, x, self._bank("gate_up"), s_tok, offs,
-                                 counts, bias=self.gate_up_b,
-                                 act_mode=act_mode)
+        hip.moe_tile(False, act, x, self._bank("gate_up"), s_tok, tiles,
+                     ntiles, offs, counts, bias=self.gate_up_b,
+                     act_mode=act_mode)
+        # few workgroups of long rows: twice as many of 64 columns (8 experts
+        # of 4096 x 14336, us: 1 row 90 against 191, 8 rows 170 against 215,
+        # 64 rows 350 against 231; 128 of 2048 x 768: 64 rows 83 against 76)
+        if TK <= 16 * self.e and self.i > 2048 \
+                and min(TK, self.e) * (x.shape[1] // 128) < 512:
             hip.moe_down_scale(contrib, act, self._bank("down"), offs, counts,
                                order, flat_w, bias=db)
+        else:
+            hip.moe_tile(True, contrib, act, self._bank("down"), order, tiles,
+                         ntiles, offs, counts, flat_w, bias=db)
         out = torch.empty_like(x)
         hip.moe_sum(out, contrib, k)
         return out

@@ -22,7 +22,7 @@ void skinny_gemm_launch(void*, const void*, const void*, void*, int, int, int, i
 void gemm8_launch(void*, const void*, const void*, int, int, int, int, int*, hipStream_t);
 void skinny_gemm_v2_launch(void*, const void*, const void*, void*, int, int, int, int, hipStream_t);
 void gemm_lab_launch(void*, const void*, const void*, int, int, int, int, int*, hipStream_t);
-void moe_gate_up_silu_launch(void*, const void*, const void*, const int*, const int*, const int*, const void*, int, int, int, int, int*, hipStream_t);
+void moe_tiles_launch(int*, int*, const int*, int, int, hipStream_t);
 void moe_down_scale_launch(void*, const void*, const void*, const int*, const int*, const int*, const float*, const void*, int, int, int, int*, hipStream_t);
 void moe_topk_launch(int*, float*, const float*, int, int, int, int, int*, hipStream_t);
 void moe_sort_launch(int*, int*, int*, int*, int*, int*, const int*, int, int, int, int*, hipStream_t);
@@ -344,33 +344,6 @@ void skinny_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
   HIP_CHECK_LAST();
 }
 
-void moe_gate_up_silu(at::Tensor act, at::Tensor x, at::Tensor w,
-                      at::Tensor s_tok, at::Tensor offs, at::Tensor counts,
-                      c10::optional<at::Tensor> bias, long act_mode) {
-  check_bf16(act, "act"); check_bf16(x, "x"); check_bf16(w, "w");
-  for (auto* t : {&s_tok, &offs, &counts}) {
-    TORCH_CHECK(t->scalar_type() == at::kInt && t->is_contiguous());
-  }
-  const int E = w.size(0), H = x.size(1);
-  const long I2 = w.size(1);
-  const int I = (int)(I2 / 2);
-  TORCH_CHECK(w.size(2) == H && act.size(1) == I);
-  TORCH_CHECK(act.size(0) == s_tok.size(0));
-  const void* bias_ptr = nullptr;
-  if (bias.has_value()) {
-    check_bf16(*bias, "bias");
-    TORCH_CHECK(bias->numel() == (long)E * 2 * I, "gate_up bias must be [E, 2I]");
-    bias_ptr = bias->data_ptr();
-  }
-  int err = 0;
-  moe_gate_up_silu_launch(act.data_ptr(), x.data_ptr(), w.data_ptr(),
-                          s_tok.data_ptr<int>(), offs.data_ptr<int>(),
-                          counts.data_ptr<int>(), bias_ptr, (int)act_mode,
-                          E, H, I, &err, cur_stream(x));
-  TORCH_CHECK(!err, "moe_gate_up_silu: unsupported dims H=", H, " I=", I);
-  HIP_CHECK_LAST();
-}
-
 void moe_down_scale(at::Tensor contrib, at::Tensor act, at::Tensor w,
                     at::Tensor offs, at::Tensor counts, at::Tensor order,
                     at::Tensor flat_w, c10::optional<at::Tensor> bias) {
@@ -505,6 +478,22 @@ void rows_gemm(at::Tensor out, at::Tensor x, at::Tensor w) {
                    x.stride(0), &err, cur_stream(x));
   TORCH_CHECK(!err, "rows_gemm: unsupported M=", M, " K=", K);
   HIP_CHECK_LAST();
+}
+
+// the up product from counts and offsets that the caller sorted by
+void moe_gate_up_silu(at::Tensor act, at::Tensor x, at::Tensor w,
+                      at::Tensor s_tok, at::Tensor offs, at::Tensor counts,
+                      c10::optional<at::Tensor> bias, long act_mode) {
+  const int E = w.size(0);
+  const long most = act.size(0) / 128 + E;
+  check_i32(counts, E, "counts");
+  TORCH_CHECK(act.size(0) == s_tok.size(0));
+  at::Tensor tiles = at::empty({most, 2}, counts.options());
+  at::Tensor n = at::empty({1}, counts.options());
+  moe_tiles_launch(tiles.data_ptr<int>(), n.data_ptr<int>(),
+                   counts.data_ptr<int>(), E, (int)most, cur_stream(x));
+  moe_tile(false, act, x, w, s_tok, tiles, n, offs, counts, c10::nullopt,
+           bias, act_mode);
 }
 
 void w4_gemm(at::Tensor out, at::Tensor x, at::Tensor qw, at::Tensor sc,

@@ -12,19 +12,18 @@
 //   contrib[order[j], :] = ((act[j] @ Wd[e_j]^T) + bd[e_j]) * w_j
 // (matches models/llama.py MoEMLP._act_mul / the HF GptOss experts)
 //
-// in two forms with fixed launch grids, independent of the routing outcome:
-//
-// * few rows per expert (decode): workgroups of (expert, 64 columns), those
-//   of empty experts exit. MFMA 16x16x32 tiles, A = 16 gathered token rows
-//   staged through LDS in 512-element K chunks, B = expert weight panels
-//   streamed from HBM, once per 16-row m-tile. Bound by that stream: 128
-//   experts x (1536 + 768) x 2048 at 64 rows run at 4.7 and 5.0 TB/s.
-// * many rows per expert (prompts): 128 x 128 tiles, below.
+// Launch grids do not depend on the routing outcome: workgroups without a tile
+// exit. Both products run in 128 x 128 tiles (below), from a few rows per
+// expert, where they are bound by the weight stream (128 experts x 1536 x 2048
+// at 64 rows: 146 us, 5.5 TB/s), to whole prompts. The down product has a
+// second form for few workgroups of long rows (moe_down_scale, 64 columns):
+// 16-row MFMA 16x16x32 tiles, A staged through LDS in 512-element K chunks, B
+// streamed from HBM, once per 16 rows.
 #include "common.h"
 
 namespace {
 
-constexpr int MOE_BN = 64;        // N columns per workgroup (16 per wave)
+constexpr int MOE_BN = 64;        // columns of a moe_down_scale workgroup
 constexpr int MOE_KC = 512;       // K chunk staged in LDS
 constexpr int MOE_THREADS = 256;  // 4 waves
 
@@ -35,121 +34,21 @@ DEVICE_INLINE f32x4 moe_mfma(u16x8 a, u16x8 b, f32x4 c) {
       __builtin_bit_cast(m_s16x8, a), __builtin_bit_cast(m_s16x8, b), c, 0, 0, 0);
 }
 
-// stage rows [16][kc] of gathered x into LDS (row padded to KC+8 elements
-// to break the bank cycle on the A-frag reads)
-template <bool GATHER>
+// stage rows [16][kc] into LDS (row padded to KC+8 elements to break the bank
+// cycle on the A-frag reads)
 DEVICE_INLINE void stage_rows(unsigned short* lds, const unsigned short* src,
-                              long src_stride, const int* tok, int base_row,
-                              int nrows, int k0, int kc, int tid) {
+                              long src_stride, int base_row, int nrows, int k0,
+                              int kc, int tid) {
   const int units = 16 * (kc / 8);         // u16x8 units
   for (int u = tid; u < units; u += MOE_THREADS) {
     const int row = u / (kc / 8);
     const int kk = (u % (kc / 8)) * 8;
     u16x8 val = {0, 0, 0, 0, 0, 0, 0, 0};
     if (row < nrows) {
-      const long r = GATHER ? (long)tok[row] : (long)(base_row + row);
-      val = *reinterpret_cast<const u16x8*>(src + r * src_stride + k0 + kk);
+      val = *reinterpret_cast<const u16x8*>(
+          src + (long)(base_row + row) * src_stride + k0 + kk);
     }
     *reinterpret_cast<u16x8*>(lds + row * (MOE_KC + 8) + kk) = val;
-  }
-}
-
-// EXTM=false is the exact validated silu/no-bias fast path (identical to
-// the r2-measured kernel); EXTM=true carries the GPT-OSS clamped-swiglu
-// + expert-bias variant and only launches when those are requested.
-template <bool EXTM = false>
-__global__ __launch_bounds__(MOE_THREADS) void moe_gate_up_silu_kernel(
-    unsigned short* __restrict__ act,       // [TK, I] bf16 (sorted rows)
-    const unsigned short* __restrict__ x,   // [T, H] bf16
-    const unsigned short* __restrict__ w,   // [E, 2I, H] bf16 (gate then up)
-    const int* __restrict__ s_tok,          // [TK] token index per sorted row
-    const int* __restrict__ offs,           // [E]
-    const int* __restrict__ counts,         // [E]
-    const unsigned short* __restrict__ bias,  // [E, 2I] bf16 or null
-    int act_mode,                           // 0 = silu, 1 = clamped swiglu
-    int H, int I) {
-  const int nnt = I / MOE_BN;
-  const int e = blockIdx.x / nnt;
-  const int nt = blockIdx.x % nnt;
-  const int cnt = counts[e];
-  if (cnt == 0) return;
-  const int base = offs[e];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & (WAVE_SIZE - 1);
-  const int wave = tid / WAVE_SIZE;
-  const int lc = lane & 15;
-  const int lg = lane >> 4;
-
-  __shared__ unsigned short Xl[16 * (MOE_KC + 8)];
-
-  const unsigned short* wg_panel =
-      w + ((long)e * 2 * I + nt * MOE_BN + wave * 16) * H;
-  const unsigned short* wu_panel =
-      w + ((long)e * 2 * I + I + nt * MOE_BN + wave * 16) * H;
-
-  // The kernel is weight-stream bound; a wave must keep enough loads in
-  // flight to cover HBM latency (~600 ns). Weights are consumed in
-  // K-blocks of 128 (4 MFMA k-steps), software-pipelined one block ahead:
-  // 8 b128 loads (gate+up) issue while the previous block's 8 MFMAs run.
-  const long wrow = (long)lc * H;  // this lane's weight row offset
-  for (int m0 = 0; m0 < cnt; m0 += 16) {
-    const int nrows = min(16, cnt - m0);
-    f32x4 ag{0.f, 0.f, 0.f, 0.f}, au{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < H; k0 += MOE_KC) {
-      const int kc = min(MOE_KC, H - k0);
-      __syncthreads();
-      stage_rows<true>(Xl, x, H, s_tok + base + m0, 0, nrows, k0, kc, tid);
-      __syncthreads();
-      // constexpr trip count on full chunks: the compiler fully unrolls
-      // the 16 iterations and issues the 32 weight loads deep ahead of
-      // the MFMAs (manual double-buffering with runtime-indexed register
-      // arrays measured 10x SLOWER — selects, no unroll)
-      auto body = [&](int kk) {
-        const u16x8 a = *reinterpret_cast<const u16x8*>(
-            Xl + lc * (MOE_KC + 8) + kk + lg * 8);
-        const u16x8 g = *reinterpret_cast<const u16x8*>(
-            wg_panel + wrow + k0 + kk + lg * 8);
-        const u16x8 u = *reinterpret_cast<const u16x8*>(
-            wu_panel + wrow + k0 + kk + lg * 8);
-        ag = moe_mfma(a, g, ag);
-        au = moe_mfma(a, u, au);
-      };
-      if (kc == MOE_KC) {
-#pragma unroll
-        for (int kk = 0; kk < MOE_KC; kk += 32) body(kk);
-      } else {
-        for (int kk = 0; kk < kc; kk += 32) body(kk);
-      }
-    }
-    // D[row = lg*4 + r][col = lc]; fuse the activation and write.
-    // EXTM: bias depends on the column only — one pair of loads per lane.
-    float bg = 0.f, bu = 0.f;
-    if constexpr (EXTM) {
-      if (bias != nullptr) {
-        const int col = nt * MOE_BN + wave * 16 + lc;
-        bg = bf2f(bias[(long)e * 2 * I + col]);
-        bu = bf2f(bias[(long)e * 2 * I + I + col]);
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = lg * 4 + r;
-      if (row >= nrows) continue;
-      float v;
-      if (EXTM && act_mode == 1) {  // GPT-OSS clamped swiglu
-        const float g = fminf(ag[r] + bg, 7.f);
-        const float u = fminf(fmaxf(au[r] + bu, -7.f), 7.f);
-        v = (u + 1.f) * g / (1.f + __expf(-1.702f * g));
-      } else if constexpr (EXTM) {
-        const float g = ag[r] + bg;
-        v = g / (1.f + __expf(-g)) * (au[r] + bu);
-      } else {
-        const float g = ag[r];
-        v = g / (1.f + __expf(-g)) * au[r];
-      }
-      act[(long)(base + m0 + row) * I + nt * MOE_BN + wave * 16 + lc] = f2bf(v);
-    }
   }
 }
 
@@ -190,7 +89,7 @@ __global__ __launch_bounds__(MOE_THREADS) void moe_down_scale_kernel(
     for (int k0 = 0; k0 < I; k0 += MOE_KC) {
       const int kc = min(MOE_KC, I - k0);
       __syncthreads();
-      stage_rows<false>(Al, act, I, nullptr, first + m0, nrows, k0, kc, tid);
+      stage_rows(Al, act, I, first + m0, nrows, k0, kc, tid);
       __syncthreads();
       auto body = [&](int kk) {
         const u16x8 a = *reinterpret_cast<const u16x8*>(
@@ -228,7 +127,7 @@ __global__ __launch_bounds__(MOE_THREADS) void moe_down_scale_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Prompt form. A tile is 128 rows of one expert x 128 weight rows (of gate and
+// Tile form. A tile is 128 rows of one expert x 128 weight rows (of gate and
 // up: 64 each, 32 + 32 beside each other per wave, so that a lane holds a
 // column's gate and up), four waves of 64 x 64 on mfma_f32_32x32x16_bf16, K in
 // steps of 64 through two LDS buffers that global_load_lds fills 16 bytes a
@@ -240,8 +139,11 @@ __global__ __launch_bounds__(MOE_THREADS) void moe_down_scale_kernel(
 // The tile list (moe_sort) holds only tiles that exist, and workgroups are
 // dealt to the XCDs in runs, so the tiles of one expert meet its weights and
 // rows in one L2.
-// Bound by the products and the weight stream alike: 254 rows per expert of
-// 128 x (1536 + 768) x 2048 are 0.31 TFLOP and 1.2 GB a layer.
+// Bound by the products and the weight stream alike: 256 rows per expert of
+// 128 x (1536 + 768) x 2048 are 0.31 TFLOP and 1.2 GB a layer, 336 + 210 us
+// (613 and 492 TFLOP/s). Steps of 32 through a ring of five buffers, four of
+// them in flight, took 368 + 225: the LDS reads of 64 x 64 wave tiles and the
+// barriers set the pace, not the loads.
 // ---------------------------------------------------------------------------
 constexpr int MT_M = 128, MT_N = 128, MT_K = 64;
 
@@ -559,6 +461,20 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(
   });
 }
 
+// The tile list alone, from counts that the caller brings.
+__global__ __launch_bounds__(64) void moe_tiles_kernel(
+    int* __restrict__ tiles, int* __restrict__ ntiles,
+    const int* __restrict__ counts, int E, int max_tiles) {
+  if (threadIdx.x != 0) return;
+  int n = 0;
+  for (int e = 0; e < E; ++e)
+    for (int r = 0; r < counts[e] && n < max_tiles; r += MT_M, ++n) {
+      tiles[2 * n] = e;
+      tiles[2 * n + 1] = r;
+    }
+  ntiles[0] = n;
+}
+
 // out[t] = sum over the k contributions of row t, in fp32 in their order.
 // Bound by reading them once.
 __global__ __launch_bounds__(256) void moe_sum_kernel(
@@ -614,6 +530,12 @@ void moe_sort_launch(int* order, int* s_tok, int* counts, int* offs,
                      counts, offs, tiles, ntiles, experts, TK, E, k);
 }
 
+void moe_tiles_launch(int* tiles, int* ntiles, const int* counts, int E,
+                      int max_tiles, hipStream_t s) {
+  hipLaunchKernelGGL(moe_tiles_kernel, dim3(1), dim3(64), 0, s, tiles, ntiles,
+                     counts, E, max_tiles);
+}
+
 void moe_sum_launch(void* out, const void* contrib, long T, int k, int H,
                     hipStream_t s) {
   const long units = T * (H / 8);
@@ -649,29 +571,6 @@ void moe_tile_launch(int down, void* out, const void* src, const void* w,
     else TILE(false, false);
   }
 #undef TILE
-}
-
-void moe_gate_up_silu_launch(void* act, const void* x, const void* w,
-                             const int* s_tok, const int* offs,
-                             const int* counts, const void* bias,
-                             int act_mode, int E, int H, int I,
-                             int* err_unsupported, hipStream_t s) {
-  *err_unsupported = 0;
-  if (I % MOE_BN != 0 || H % 128 != 0) { *err_unsupported = 1; return; }
-  dim3 grid(E * (I / MOE_BN));
-  const bool extm = bias != nullptr || act_mode != 0;
-  if (extm)
-    hipLaunchKernelGGL((moe_gate_up_silu_kernel<true>), grid,
-                       dim3(MOE_THREADS), 0, s, (unsigned short*)act,
-                       (const unsigned short*)x, (const unsigned short*)w,
-                       s_tok, offs, counts, (const unsigned short*)bias,
-                       act_mode, H, I);
-  else
-    hipLaunchKernelGGL((moe_gate_up_silu_kernel<false>), grid,
-                       dim3(MOE_THREADS), 0, s, (unsigned short*)act,
-                       (const unsigned short*)x, (const unsigned short*)w,
-                       s_tok, offs, counts, (const unsigned short*)bias,
-                       act_mode, H, I);
 }
 
 void moe_down_scale_launch(void* contrib, const void* act, const void* w,
