@@ -45,25 +45,44 @@ class DecodeGraphRunner:
         pad_slot = self.pad_block * cfg.block_size
 
         mb = self.max_bs
-        self.tokens = torch.zeros(mb, dtype=torch.long, device=dev)
-        self.positions = torch.zeros(mb, dtype=torch.long, device=dev)
-        self.slots = torch.full((mb,), pad_slot, dtype=torch.long, device=dev)
+        # models that read the pool through the ragged batch view also get
+        # static buffers for it: a decode row is its own one-row sequence
+        # (row i uses block table row i), plus each row's previous token
+        self.ragged = bool(getattr(runner, "ragged", False))
+        # recurrent-state models: each row's state slot; padded rows use the
+        # pool's spare slot
+        self.stateful = self.ragged and kv.state_allocator is not None
+        # Everything a step brings per row sits in ONE device buffer with one
+        # pinned mirror and crosses in one copy (each copy of a few hundred
+        # bytes costs a decode step about 5 us on the stream): tokens first,
+        # which stay out of the copy when the sampler feeds them on the device
+        fields = [("tokens", torch.long, 0), ("positions", torch.long, 0),
+                  ("slots", torch.long, pad_slot),
+                  ("seq_lens", torch.int32, 1)]
+        if self.ragged:
+            fields += [("prev", torch.long, -1), ("pos32", torch.int32, 0)]
+        if self.stateful:
+            fields += [("state_slots", torch.int32, kv.pad_state_slot)]
+        fields.sort(key=lambda f: f[1] != torch.long)   # 8-byte fields first
+        pin = dev.type == "cuda"
+        words = sum(mb if t == torch.long else (mb + 1) // 2
+                    for _, t, _ in fields)
+        self._rows_dev = torch.zeros(words, dtype=torch.long, device=dev)
+        self._rows_pin = torch.zeros(words, dtype=torch.long, pin_memory=pin)
+        at = 0
+        for name, t, pad in fields:
+            n = mb if t == torch.long else (mb + 1) // 2
+            for buf, prefix in ((self._rows_dev, ""), (self._rows_pin, "h_")):
+                view = buf[at:at + n].view(t)[:mb]
+                view.fill_(pad)
+                setattr(self, prefix + name, view)
+            # numpy view of the pinned staging (shared memory)
+            setattr(self, "n_" + name, getattr(self, "h_" + name).numpy())
+            at += n
         self.block_tables = torch.full(
             (mb, self.max_blocks), self.pad_block, dtype=torch.int32, device=dev
         )
-        self.seq_lens = torch.ones(mb, dtype=torch.int32, device=dev)
-        # pinned host staging
-        pin = dev.type == "cuda"
-        self.h_tokens = torch.zeros(mb, dtype=torch.long, pin_memory=pin)
-        self.h_positions = torch.zeros(mb, dtype=torch.long, pin_memory=pin)
-        self.h_slots = torch.zeros(mb, dtype=torch.long, pin_memory=pin)
         self.h_bt = torch.zeros(mb, self.max_blocks, dtype=torch.int32, pin_memory=pin)
-        self.h_seq_lens = torch.ones(mb, dtype=torch.int32, pin_memory=pin)
-        # cached numpy views of the pinned staging (shared memory)
-        self.n_tokens = self.h_tokens.numpy()
-        self.n_positions = self.h_positions.numpy()
-        self.n_slots = self.h_slots.numpy()
-        self.n_seq_lens = self.h_seq_lens.numpy()
         self._pad_slot = pad_slot
         self._prev_bs = 0
         # per-row cache for incremental block-table staging: (request_id,
@@ -73,27 +92,9 @@ class DecodeGraphRunner:
         # persistent — every tensor a captured graph references must outlive
         # the graph (an ephemeral arange here caused replay-time faults)
         self.logits_idx = torch.arange(mb, dtype=torch.long, device=dev)
-        # models that read the pool through the ragged batch view also get
-        # static buffers for it: a decode row is its own one-row sequence
-        # (row i uses block table row i), plus each row's previous token
-        self.ragged = bool(getattr(runner, "ragged", False))
         if self.ragged:
-            self.prev = torch.full((mb,), -1, dtype=torch.long, device=dev)
-            self.pos32 = torch.zeros(mb, dtype=torch.int32, device=dev)
             self.row_seq = torch.arange(mb, dtype=torch.int32, device=dev)
-            self.h_prev = torch.full((mb,), -1, dtype=torch.long, pin_memory=pin)
-            self.h_pos32 = torch.zeros(mb, dtype=torch.int32, pin_memory=pin)
-            self.n_prev = self.h_prev.numpy()
-            self.n_pos32 = self.h_pos32.numpy()
-        # recurrent-state models: each row's state slot; padded rows use the
-        # pool's spare slot
-        self.stateful = self.ragged and kv.state_allocator is not None
         if self.stateful:
-            self.state_slots = torch.full((mb,), kv.pad_state_slot,
-                                          dtype=torch.int32, device=dev)
-            self.h_state_slots = torch.full((mb,), kv.pad_state_slot,
-                                            dtype=torch.int32, pin_memory=pin)
-            self.n_state_slots = self.h_state_slots.numpy()
             self.seq_rows_one = torch.ones(mb, dtype=torch.int32, device=dev)
         self.graphs: dict[int, torch.cuda.CUDAGraph] = {}
         self.outs: dict[int, torch.Tensor] = {}
@@ -199,23 +200,16 @@ class DecodeGraphRunner:
             dirty_hi = max(dirty_hi, hi - 1)
         self._prev_bs = bucket
         n = hi
+        first = 0
         if token_src is not None:
             # async pipeline: previous step's sampled ids feed this step
             # device-to-device (same stream => ordered after the sampler)
+            first = self.max_bs
             self.tokens[:bs].copy_(token_src[:bs])
             if n > bs:
                 self.tokens[bs:n].copy_(self.h_tokens[bs:n], non_blocking=True)
-        else:
-            self.tokens[:n].copy_(self.h_tokens[:n], non_blocking=True)
-        self.positions[:n].copy_(self.h_positions[:n], non_blocking=True)
-        self.slots[:n].copy_(self.h_slots[:n], non_blocking=True)
-        self.seq_lens[:n].copy_(self.h_seq_lens[:n], non_blocking=True)
-        if self.ragged:
-            self.pos32[:n].copy_(self.h_pos32[:n], non_blocking=True)
-            self.prev[:n].copy_(self.h_prev[:n], non_blocking=True)
-        if self.stateful:
-            self.state_slots[:n].copy_(self.h_state_slots[:n],
-                                       non_blocking=True)
+        # rows behind n are padding from earlier steps
+        self._rows_dev[first:].copy_(self._rows_pin[first:], non_blocking=True)
         if dirty_hi >= 0:
             self.block_tables[dirty_lo:dirty_hi + 1, :max(maxb, 1)].copy_(
                 self.h_bt[dirty_lo:dirty_hi + 1, :max(maxb, 1)], non_blocking=True
