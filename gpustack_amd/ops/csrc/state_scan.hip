@@ -318,6 +318,244 @@ __global__ __launch_bounds__(256) void state_scan_vec_kernel(
   }
 }
 
+// The same recurrence in chunks of 32 rows on the fp32 matrix instructions,
+// for prompts. Inside a chunk, with c_t the sum of the logarithms of the decays
+// up to row t,
+//   y_t   = sum_{s <= t} e^(c_t - c_s) b_s (q_t . k_s) v_s + e^(c_t) S^T q_t
+//   S_new = e^(c_31) S + sum_s e^(c_31 - c_s) b_s k_s v_s^T
+// so that one chunk is four small products (Q K^T, the weighted scores times V,
+// Q S, K^T V) instead of 32 dependent passes over the state. Everything stays
+// fp32 (v_mfma_f32_16x16x4_f32); the c are summed in double, since their
+// differences, not they, are what the weights are made of.
+//   - a workgroup owns 64 value channels of one (sequence, head), a wave 16 of
+//     them. Waves share q, k, v and the scores through the LDS.
+//   - operands that reduce over their rows' contiguous axis are read 16 bytes
+//     at a time: lane group g takes k = 4 g .. 4 g + 3 of 16, one value per
+//     matrix instruction, in both operands. Rows are 4 floats longer than
+//     their content, which keeps those reads off each other's banks.
+//   - with that order the state, as the accumulators hold it (rows 4 g + r,
+//     column l & 15), is the operand of Q S: it never leaves the registers.
+//   - the next chunk's rows are fetched while this one is worked on; 48 KB.
+// Bound by the chain of chunks of the longest sequence (about 170 matrix
+// instructions of 32 cycles a wave and chunk).
+typedef __attribute__((ext_vector_type(4))) float sc_f32x4;
+
+template <int NT>   // state rows / 16, padded
+__global__ __launch_bounds__(256, 2) void state_chunk_kernel(
+    float* __restrict__ y, const unsigned short* __restrict__ src,
+    const unsigned short* __restrict__ dt_src, ScanArgs p) {
+  constexpr int C = 32, NP = NT * 16, KS = NP + 4, PB = 64, VS = PB + 4;
+  constexpr int KU = C * NP / 8 / 256;       // 16-byte loads of k (and q)
+  static_assert(KU >= 1 && C * NP / 8 % 256 == 0, "NT is 4 or 8");
+  __shared__ __attribute__((aligned(16))) float qs[C][KS];
+  __shared__ __attribute__((aligned(16))) float ks[C][KS];
+  __shared__ __attribute__((aligned(16))) float vs[C][VS];
+  __shared__ __attribute__((aligned(16))) float as[C][C + 4];
+  __shared__ double cs[C];
+  __shared__ float bl[C], el[C], wl[C];
+  const int s = blockIdx.x, h = blockIdx.y, pb0 = blockIdx.z * PB;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lc = lane & 15, g = lane >> 4;
+  const int first = p.seq_first[s], n = p.seq_rows[s];
+  if (first < 0 || n < 1 || first + n > p.T) return;
+  const int slot = min(max(p.state_slots[s], 0), p.nslots - 1);
+  const int hist = p.pos32[first];
+  const int N = p.N, P = p.P;
+  const int grp = h / (p.H / p.G);
+  const int pc = pb0 + wave * 16 + lc;       // this lane's value channel
+  const bool live = pc < P;
+  float* sp = p.state + ((long)slot * p.H + h) * N * P;
+  sc_f32x4 S[NT];                            // rows 16 t + 4 g + r, column pc
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int nn = t * 16 + g * 4 + r;
+      S[t][r] = (hist > 0 && live && nn < N) ? sp[(long)nn * P + pc] : 0.f;
+    }
+  const float skip = p.skip != nullptr ? p.skip[h] : 0.f;
+  const float a_rate = dt_src != nullptr ? expf(p.a_log[h]) : 0.f;
+  const float dtb = dt_src != nullptr ? p.dt_bias[h] : 0.f;
+  const float a_const = dt_src == nullptr ? p.decay[h] : 0.f;
+  const bool neg = a_const < 0.f;            // (-1)^(t - s) beside |a|^(t - s)
+  // far enough down that e^it is 0 in fp32, and still exact in the sums
+  const float log_const = fmaxf(logf(fabsf(a_const)), -1e4f);
+  const u16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+
+  u16x8 kreg[KU], qreg[KU], vreg;
+  float dreg = 0.f;
+  auto fetch = [&](int c0) {
+    const int rows = min(C, n - c0);
+#pragma unroll
+    for (int u = 0; u < KU; ++u) {
+      const int i = tid + u * 256, r = i / (NP / 8), e = i % (NP / 8) * 8;
+      kreg[u] = zero8;
+      qreg[u] = zero8;
+      if (r < rows && e < N) {
+        const unsigned short* rp = src + (long)(first + c0 + r) * p.ld_src;
+        kreg[u] = *reinterpret_cast<const u16x8*>(rp + p.col_b + grp * N + e);
+        qreg[u] = *reinterpret_cast<const u16x8*>(rp + p.col_c + grp * N + e);
+      }
+    }
+    const int r = tid / (PB / 8), e = tid % (PB / 8) * 8;
+    vreg = zero8;
+    if (r < rows && pb0 + e < P)
+      vreg = *reinterpret_cast<const u16x8*>(
+          src + (long)(first + c0 + r) * p.ld_src + p.col_x + h * P + pb0 + e);
+    if (dt_src != nullptr && tid < rows)
+      dreg = bf2f(dt_src[(long)(first + c0 + tid) * p.ld_dt + p.col_dt + h]);
+  };
+  auto put8 = [&](float* to, const u16x8 from) {
+    float f[8];
+    bf8_to_f32(from, f);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (p.act) f[i] = silu_f(f[i]);
+    *reinterpret_cast<sc_f32x4*>(to) = sc_f32x4{f[0], f[1], f[2], f[3]};
+    *reinterpret_cast<sc_f32x4*>(to + 4) = sc_f32x4{f[4], f[5], f[6], f[7]};
+  };
+  auto mm = [](float a, float b, sc_f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  };
+
+  fetch(0);
+  for (int c0 = 0; c0 < n; c0 += C) {
+    const int rows = min(C, n - c0);
+#pragma unroll
+    for (int u = 0; u < KU; ++u) {
+      const int i = tid + u * 256, r = i / (NP / 8), e = i % (NP / 8) * 8;
+      put8(&ks[r][e], kreg[u]);
+      put8(&qs[r][e], qreg[u]);
+    }
+    put8(&vs[tid / (PB / 8)][tid % (PB / 8) * 8], vreg);
+    if (tid < C) {
+      // rows behind the last one: decay 1, weight 0
+      float la = 0.f, b = 0.f;
+      if (tid < rows) {
+        if (dt_src != nullptr) {
+          b = softplus_f(dreg + dtb);
+          la = fmaxf(-a_rate * b, -1e4f);
+        } else {
+          b = 1.f;
+          la = log_const;
+        }
+      }
+      double c = la;
+#pragma unroll
+      for (int m = 1; m < C; m <<= 1) {
+        const double o = __shfl_up(c, m, 32);
+        if (tid >= m) c += o;
+      }
+      const double all = __shfl(c, C - 1, 32);
+      const int last = rows - 1;
+      cs[tid] = c;
+      bl[tid] = b;
+      el[tid] = expf((float)c) * (neg && !(tid & 1) ? -1.f : 1.f);
+      wl[tid] = b * expf((float)(all - c)) *
+                (neg && ((last - tid) & 1) ? -1.f : 1.f);
+    }
+    __syncthreads();
+    if (c0 + C < n) fetch(c0 + C);
+
+    // scores of 16 x 16 rows a wave, weighted
+    const int ti = wave >> 1, si = wave & 1;
+    if (si <= ti) {
+      sc_f32x4 a{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kb = 0; kb < NT; ++kb) {
+        const sc_f32x4 q4 = *reinterpret_cast<const sc_f32x4*>(
+            &qs[ti * 16 + lc][kb * 16 + g * 4]);
+        const sc_f32x4 k4 = *reinterpret_cast<const sc_f32x4*>(
+            &ks[si * 16 + lc][kb * 16 + g * 4]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) a = mm(q4[j], k4[j], a);
+      }
+      const int sr = si * 16 + lc;
+      const double c_s = cs[sr];
+      const float b_s = bl[sr];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int tr = ti * 16 + g * 4 + r;
+        float w = 0.f;
+        if (sr <= tr) {
+          w = a[r] * expf((float)(cs[tr] - c_s)) * b_s;
+          if (neg && ((tr - sr) & 1)) w = -w;
+        }
+        as[tr][sr] = w;
+      }
+    }
+    // what the state brings
+    sc_f32x4 o[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) o[t] = sc_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kb = 0; kb < NT; ++kb) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const sc_f32x4 q4 = *reinterpret_cast<const sc_f32x4*>(
+            &qs[t * 16 + lc][kb * 16 + g * 4]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[t] = mm(q4[j], S[kb][j], o[t]);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[t][r] *= el[t * 16 + g * 4 + r];
+    __syncthreads();
+    // what the chunk's own rows bring
+    float vv[2][4];
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) vv[b][j] = vs[b * 16 + g * 4 + j][wave * 16 + lc];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int b = 0; b <= t; ++b) {
+        const sc_f32x4 a4 = *reinterpret_cast<const sc_f32x4*>(
+            &as[t * 16 + lc][b * 16 + g * 4]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[t] = mm(a4[j], vv[b][j], o[t]);
+      }
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int tr = t * 16 + g * 4 + r;
+        if (tr < rows && live)
+          y[(long)(first + c0 + tr) * p.H * P + h * P + pc] =
+              o[t][r] + skip * vs[tr][wave * 16 + lc];
+      }
+    // the state behind the chunk
+    const float down = expf((float)cs[C - 1]) *
+                       (neg && (rows & 1) ? -1.f : 1.f);
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) S[t][r] *= down;
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int sr = b * 16 + g * 4 + j;
+        const float bv = vv[b][j] * wl[sr];
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+          S[t] = mm(ks[sr][t * 16 + lc], bv, S[t]);
+      }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int nn = t * 16 + g * 4 + r;
+      if (live && nn < N) sp[(long)nn * P + pc] = S[t][r];
+    }
+}
+
 // Single rows (decode): the state itself is the traffic, so one workgroup
 // per (sequence, head) streams it once with 16-byte accesses — a lane
 // owns 4 neighbouring value channels of every RP-th state row — updates it
@@ -549,6 +787,8 @@ void scan_launch(float* y, const void* src, const void* dt, const ScanArgs& p,
 // Rows of the state per lane (NR) and lanes per value channel (TPP): the
 // fewest lanes per channel that keep NR <= 32, but no more channels per wave
 // than the head has.
+constexpr int CHUNK_ROWS = 24;
+
 template <typename TS, typename TD>
 bool scan_pick(float* y, const void* src, const void* dt, const ScanArgs& p,
                int nseq, hipStream_t s) {
@@ -559,6 +799,20 @@ bool scan_pick(float* y, const void* src, const void* dt, const ScanArgs& p,
   const bool vec = p.N % 8 == 0 && p.P % 8 == 0 &&
                    p.ld_src % 8 == 0 && p.col_x % 8 == 0 && p.col_b % 8 == 0 &&
                    p.col_c % 8 == 0;
+  // Chunks on the matrix instructions from CHUNK_ROWS rows a sequence on (on
+  // average: the sizes themselves are on the device), where a wave's 16 value
+  // channels and 16-row state tiles are not mostly padding
+  if (sizeof(TS) == 2 && vec && p.N >= 32 && p.N <= 128 && p.P >= 32 &&
+      (long)p.T >= (long)CHUNK_ROWS * nseq) {
+    const dim3 grid(nseq, p.H, (p.P + 63) / 64);
+    if (p.N <= 64)
+      state_chunk_kernel<4><<<grid, 256, 0, s>>>(
+          y, (const unsigned short*)src, (const unsigned short*)dt, p);
+    else
+      state_chunk_kernel<8><<<grid, 256, 0, s>>>(
+          y, (const unsigned short*)src, (const unsigned short*)dt, p);
+    return true;
+  }
   // few workgroups (long portions of few sequences): more lanes per channel
   // make more, smaller ones, so that every SIMD holds two waves
   while (vec && sizeof(TS) == 2 && tpp < 8 && (p.N + tpp - 1) / tpp >= 16 &&
