@@ -352,19 +352,25 @@ def skinny_gemm(x, w, out=None, splitk: int | None = None, version: int = 1):
 
 def _rows_gemm_wins(M: int, N: int, K: int) -> bool:
     """Where the decode product (ops/csrc/rows_gemm.hip) measured faster than
-    the library, us at 1 / 16 rows, weights out of HBM:
-    small weights, whose time is latency: 4096x4096 9.4 / 11.2 against 15.6 /
-    15.5, 2048x4096 8.5 / 10.8 against 14.7 / 14.9, 5120x2048 9.6 / 12.2
-    against 12.1 / 12.2 (24 rows of 4096x4096: 14.0 against 13.3; 6144x4096
-    14.4 / 19.0 against 14.7 / 14.6);
-    wide heads of narrow models: 102400x1536 71 / 80 against 115 / 114,
-    151936x2048 127 / 144 against 205 / 203, 200064x3072 254 / 294 against 382
-    / 374 (102400x1024 50 / 53 against 41 / 42, 102400x4096 175 / 192 against
-    176 / 181, 65536x2048 59 / 65 against 67 / 66)."""
-    if M > 16 or K % 128 != 0:
+    the library, us at 1 / 8 / 16 rows, weights out of HBM:
+    small weights, whose time is latency: 4096x4096 9.5 / 10.1 / 10.7 against
+    15.6, 2048x4096 8.5 / 9.6 / 10.8 against 14.8, 5120x2048 8.0 / 9.0 / 10.6
+    against 12.3 (24 rows of 4096x4096: 12.9 against 13.4; 6144x4096 13.0 /
+    15.6 / 18.3 against 14.6);
+    many columns: 16384x2048 14 / 15 / 16 against 18, 22016x4096 36 / 39 / 41
+    against 52, 28672x4096 43 / 47 / 53 against 54, 49152x2048 34 / 37 / 42
+    against 47, 65536x4096 88 / 93 against 120 (49152x3072 at 16 rows 65
+    against 60, 16384x5120 34 / 37 / 42 against 34);
+    wide heads of narrow models: 102400x1536 71 / 77 / 80 against 115,
+    151936x2048 127 / 135 / 144 against 205, 200064x2560 220 / 236 / 260
+    against 325 (128256x3072 135 / 150 / 173 against 146, 102400x1024 50 / 52 /
+    53 against 42)."""
+    if M > 16 or K % 128 != 0 or not 1024 <= K <= 4096:
         return False
-    return (N * K <= 17 << 20 and 1024 <= K <= 4096) \
-        or (N >= 100000 and 1536 <= K < 4096)
+    if N >= 100000:
+        return 1536 <= K <= 2560
+    return N * K <= 17 << 20 or (
+        N >= 12288 and N * K <= (280_000_000 if M <= 8 else 130_000_000))
 
 
 def linear_auto(x, w):

@@ -63,13 +63,7 @@ __global__ __launch_bounds__(RG_THREADS) void rows_gemm_kernel(
 #pragma unroll
     for (int t = 0; t < NTW; ++t) acc[i][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  for (int i = wave; i < nb; i += RG_WAVES) {
-    const int b = block(i), bn = block(min(i + RG_WAVES, nb - 1));
-#pragma unroll
-    for (int t = 0; t < NTW; ++t)
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-        wn[t][c] = *reinterpret_cast<const u32x4*>(wp[t] + bn * RG_KC + c * 32);
+  auto multiply = [&](int b) {
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       u32x4 xa[MT];
@@ -84,21 +78,32 @@ __global__ __launch_bounds__(RG_THREADS) void rows_gemm_kernel(
               __builtin_bit_cast(rg_s16x8, xa[m]),
               __builtin_bit_cast(rg_s16x8, wc[t][c]), acc[m][t], 0, 0, 0);
     }
+  };
+  int i = wave;
+  for (; i + RG_WAVES < nb; i += RG_WAVES) {
+    const int bn = block(i + RG_WAVES);
+#pragma unroll
+    for (int t = 0; t < NTW; ++t)
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        wn[t][c] = *reinterpret_cast<const u32x4*>(wp[t] + bn * RG_KC + c * 32);
+    multiply(block(i));
 #pragma unroll
     for (int t = 0; t < NTW; ++t)
 #pragma unroll
       for (int c = 0; c < 4; ++c) wc[t][c] = wn[t][c];
   }
+  if (i < nb) multiply(block(i));
 
   // D[row = lg*4 + r][col = lc] per 16x16 tile
 #pragma unroll
-  for (int i = 0; i < MT; ++i)
+  for (int m = 0; m < MT; ++m)
 #pragma unroll
     for (int t = 0; t < NTW; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        red[(wave * ROWS + i * 16 + lg * 4 + r) * COLS + t * 16 + lc] =
-            acc[i][t][r];
+        red[(wave * ROWS + m * 16 + lg * 4 + r) * COLS + t * 16 + lc] =
+            acc[m][t][r];
   __syncthreads();
   for (int u = tid; u < ROWS * COLS; u += RG_THREADS) {
     const int row = u / COLS, col = n0 + u % COLS;

@@ -10,8 +10,8 @@
 // Scales / zero-scales: bf16 [N, K/128], one group per 128-k block.
 // w = q * s - zs   (zs = zero * s, precomputed).
 //
-// Few rows (decode). A workgroup of 8 waves owns 16 NTW columns of up to 64
-// rows; its waves take the k blocks in turn (8 neighbouring blocks of a row
+// Few rows (decode). A workgroup of 8 or 16 waves owns 16 NTW columns of up to
+// 64 rows; its waves take the k blocks in turn (neighbouring blocks of a row
 // are read together) and meet in the LDS at the end, so no second kernel and
 // no partial results in memory.
 //  - A nibble becomes bf16 without arithmetic: 0x4300 | q is 128 + q, two at
@@ -29,8 +29,6 @@
 namespace {
 
 constexpr int W4_KC = 128;
-constexpr int W4_WAVES = 8;
-constexpr int W4_THREADS = W4_WAVES * WAVE_SIZE;
 
 typedef __attribute__((ext_vector_type(8))) short w4_s16x8;
 
@@ -59,8 +57,8 @@ DEVICE_INLINE u32x4 w4_order(u32x4 v) {
   return o;
 }
 
-template <int MT, int NTW>
-__global__ __launch_bounds__(W4_THREADS) void w4_rows_kernel(
+template <int MT, int NTW, int WAVES>
+__global__ __launch_bounds__(WAVES * WAVE_SIZE) void w4_rows_kernel(
     unsigned short* __restrict__ out,       // [M, N] bf16
     const unsigned short* __restrict__ x,   // [M, K] bf16
     const unsigned char* __restrict__ qw,   // [N, K/2] frag-ordered nibbles
@@ -102,7 +100,7 @@ __global__ __launch_bounds__(W4_THREADS) void w4_rows_kernel(
   for (int t = 0; t < NTW; ++t)
     wc[t] = *reinterpret_cast<const u32x4*>(wp[t] + (long)b0 * 64);
 
-  for (int u = tid; u < COLS * nb; u += W4_THREADS) {
+  for (int u = tid; u < COLS * nb; u += WAVES * WAVE_SIZE) {
     const int c = u / nb, b = u % nb;
     const long at = (long)(n0 + c) * nb + b;
     sz[b * COLS + c] = (unsigned int)sc[at] | ((unsigned int)zs[at] << 16);
@@ -116,11 +114,7 @@ __global__ __launch_bounds__(W4_THREADS) void w4_rows_kernel(
     for (int t = 0; t < NTW; ++t) acc[i][t] = f32x4{0.f, 0.f, 0.f, 0.f};
   const u32x4 ones = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
 
-  for (int j = wave; j < nb; j += W4_WAVES) {
-    const int b = block(j), bn = block(min(j + W4_WAVES, nb - 1));
-#pragma unroll
-    for (int t = 0; t < NTW; ++t)
-      wn[t] = *reinterpret_cast<const u32x4*>(wp[t] + (long)bn * 64);
+  auto multiply = [&](int b) {
     u32x4 xa[MT][4];
 #pragma unroll
     for (int i = 0; i < MT; ++i)
@@ -154,9 +148,19 @@ __global__ __launch_bounds__(W4_THREADS) void w4_rows_kernel(
 #pragma unroll
         for (int r = 0; r < 4; ++r)
           acc[i][t][r] += s * p[i][r] - z * xs[i][r];
-      wc[t] = wn[t];
     }
+  };
+  int j = wave;
+  for (; j + WAVES < nb; j += WAVES) {
+    const long bn = (long)block(j + WAVES) * 64;
+#pragma unroll
+    for (int t = 0; t < NTW; ++t)
+      wn[t] = *reinterpret_cast<const u32x4*>(wp[t] + bn);
+    multiply(block(j));
+#pragma unroll
+    for (int t = 0; t < NTW; ++t) wc[t] = wn[t];
   }
+  if (j < nb) multiply(block(j));
 
   __syncthreads();                       // the scales are done with
   // D[row = lg*4 + r][col = lc] per 16x16 tile
@@ -170,12 +174,12 @@ __global__ __launch_bounds__(W4_THREADS) void w4_rows_kernel(
         red[(wave * ROWS + i * 16 + lg * 4 + r) * COLS + t * 16 + lc] =
             acc[i][t][r];
   __syncthreads();
-  for (int u = tid; u < ROWS * COLS; u += W4_THREADS) {
+  for (int u = tid; u < ROWS * COLS; u += WAVES * WAVE_SIZE) {
     const int row = m0 + u / COLS;
     if (row >= M) break;
     float v = 0.f;
 #pragma unroll
-    for (int w = 0; w < W4_WAVES; ++w) v += red[w * ROWS * COLS + u];
+    for (int w = 0; w < WAVES; ++w) v += red[w * ROWS * COLS + u];
     out[(long)row * N + n0 + u % COLS] = f2bf(v);
   }
 }
@@ -232,23 +236,27 @@ void w4_dequant_launch(void* out, const void* qw, const void* sc,
 }
 
 namespace {
-template <int MT, int NTW>
+template <int MT, int NTW, int WAVES>
 void w4_rows(void* out, const void* x, const void* qw, const void* sc,
              const void* zs, int M, int N, int K, hipStream_t s) {
   const size_t scales = (size_t)(K / W4_KC) * 16 * NTW * 4;
-  const size_t sums = (size_t)W4_WAVES * 16 * MT * 16 * NTW * 4;
-  hipLaunchKernelGGL((w4_rows_kernel<MT, NTW>),
+  const size_t sums = (size_t)WAVES * 16 * MT * 16 * NTW * 4;
+  hipLaunchKernelGGL((w4_rows_kernel<MT, NTW, WAVES>),
                      dim3(N / (16 * NTW), (M + 16 * MT - 1) / (16 * MT)),
-                     dim3(W4_THREADS), scales > sums ? scales : sums, s,
+                     dim3(WAVES * WAVE_SIZE), scales > sums ? scales : sums, s,
                      (unsigned short*)out, (const unsigned short*)x,
                      (const unsigned char*)qw, (const unsigned short*)sc,
                      (const unsigned short*)zs, M, N, K);
 }
 }  // namespace
 
-// Column tiles per wave: one while that leaves fewer than 448 workgroups of
-// two (a short weight needs every wave of the chip), else as many as share
-// the x fragments best; the scales of K / 128 blocks stay under 64 KB.
+// The form by columns: workgroups of four column tiles per wave (two at 64
+// rows) from 448 of them on; of two from 160 on, with 16 waves while x is one
+// row tile (6144 x 4096, us at 16 rows: 9.1 against 12.3 with one tile, at 64
+// rows 21.5 against 33.7); else of one, which keeps every CU on the stream
+// (4096 x 4096 at 16 rows: 7.6 against 8.7 with two), with 16 waves for long
+// rows (4096 x 14336 at one row: 11.9 against 14.5). The scales of K / 128
+// blocks stay under 64 KB.
 void w4_gemm_launch(void* out, const void* x, const void* qw, const void* sc,
                     const void* zs, int M, int N, int K,
                     int* err_unsupported, hipStream_t s) {
@@ -260,16 +268,18 @@ void w4_gemm_launch(void* out, const void* x, const void* qw, const void* sc,
   if (M == 0) return;
   const int nb = K / W4_KC;
   const int ntw = N / 64 >= 448 && nb <= 256 ? 4
-                  : N / 32 >= 448 && nb <= 512 ? 2 : 1;
+                  : N / 32 >= 160 && nb <= 512 ? 2 : 1;
+#define W4_ARGS out, x, qw, sc, zs, M, N, K, s
 #define W4_ROWS(MT)                                                          \
   do {                                                                       \
-    if (ntw == 4) w4_rows<MT, (MT) == 4 ? 2 : 4>(out, x, qw, sc, zs, M, N,   \
-                                                 K, s);                      \
-    else if (ntw == 2) w4_rows<MT, 2>(out, x, qw, sc, zs, M, N, K, s);       \
-    else w4_rows<MT, 1>(out, x, qw, sc, zs, M, N, K, s);                     \
+    if (ntw == 4) w4_rows<MT, (MT) == 4 ? 2 : 4, 8>(W4_ARGS);                \
+    else if (ntw == 2) w4_rows<MT, 2, (MT) == 1 ? 16 : 8>(W4_ARGS);          \
+    else if (nb >= 64 && (MT) <= 2) w4_rows<MT, 1, (MT) <= 2 ? 16 : 8>(W4_ARGS); \
+    else w4_rows<MT, 1, 8>(W4_ARGS);                                         \
   } while (0)
   if (M <= 16) W4_ROWS(1);
   else if (M <= 32) W4_ROWS(2);
   else W4_ROWS(4);
+#undef W4_ARGS
 #undef W4_ROWS
 }
