@@ -136,12 +136,15 @@ __global__ __launch_bounds__(MOE_THREADS) void moe_down_scale_kernel(
 // eight chunks a row, conflict-free over 16 rows of one chunk. Weights are the
 // A operand: a lane ends with 4 neighbouring columns of a row, which go
 // through the LDS to whole 16-byte stores.
-// The tile list (moe_sort) holds only tiles that exist, and workgroups are
-// dealt to the XCDs in runs, so the tiles of one expert meet its weights and
-// rows in one L2.
+// The tile list (moe_sort) holds only tiles that exist; workgroups are dealt to
+// the XCDs in runs, and the tiles of an expert that share weight rows follow
+// each other, so that these are read once into one L2 (tile by tile instead,
+// 8 experts of 4096 x 14336 at 1024 rows each read 17 GB past the L2 and ran
+// at 597 TFLOP/s). Halves of a wave's rows that an expert does not fill are
+// not multiplied (64 rows over 128 experts: 146 us, as the weights take).
 // Bound by the products and the weight stream alike: 256 rows per expert of
-// 128 x (1536 + 768) x 2048 are 0.31 TFLOP and 1.2 GB a layer, 336 + 210 us
-// (613 and 492 TFLOP/s). Steps of 32 through a ring of five buffers, four of
+// 128 x (1536 + 768) x 2048 are 0.31 TFLOP and 1.2 GB a layer, 313 + 200 us
+// (658 and 516 TFLOP/s; 8 experts at 1024 rows: 840 and 762). Steps of 32 through a ring of five buffers, four of
 // them in flight, took 368 + 225: the LDS reads of 64 x 64 wave tiles and the
 // barriers set the pace, not the loads.
 // ---------------------------------------------------------------------------
@@ -178,16 +181,21 @@ __global__ __launch_bounds__(MOE_THREADS, 2) void moe_tile_kernel(
     const int q = nwg / 8, r = nwg % 8, xcd = wg % 8, idx = wg / 8;
     wg = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + idx;
   }
-  const int tile = wg / nnt, nt = wg % nnt;
-  const int e = tiles[2 * tile], m0 = tiles[2 * tile + 1];
+  // an expert's tiles take the same weight rows one after the other
+  const int some = wg / nnt;                 // a tile of the same expert
+  const int e = tiles[2 * some], cnt = counts[e];
+  const int mt_n = (cnt + MT_M - 1) / MT_M;
+  const int local = wg - (some - tiles[2 * some + 1] / MT_M) * nnt;
+  const int nt = local / mt_n, m0 = local % mt_n * MT_M;
   const int first = offs[e] + m0;            // sorted row of the tile's first
-  const int nrows = min(MT_M, counts[e] - m0);
+  const int nrows = min(MT_M, cnt - m0);
 
   const int tid = threadIdx.x;
   const int lane = tid & (WAVE_SIZE - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE_SIZE);
   const int wm = wave >> 1, wn = wave & 1;
   const int lc = lane & 31, hf = lane >> 5;
+  const int mine = nrows - wm * 64;          // rows of this wave's half
 
   // staging: a wave instruction fills 8 rows of 128 bytes; instruction i of
   // wave w takes rows (i * 4 + w) * 8 ..
@@ -239,24 +247,31 @@ __global__ __launch_bounds__(MOE_THREADS, 2) void moe_tile_kernel(
     if (kt + 1 < nk) stage((kt + 1) & 1, (kt + 1) * MT_K);
     const unsigned short* al = lds + (kt & 1) * BUF;
     const unsigned short* bl = al + MT_M * MT_K;
+    if (mine > 0) {
+      // the step's operands first, then its products as they arrive
+      u32x4 fa[MT_K / 16][2], fb[MT_K / 16][2];
 #pragma unroll
-    for (int kk = 0; kk < MT_K / 16; ++kk) {
-      u32x4 fa[2], fb[2];
+      for (int kk = 0; kk < MT_K / 16; ++kk)
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const int rb = wn * 64 + t * 32 + lc, ra = wm * 64 + t * 32 + lc;
-        fb[t] = *reinterpret_cast<const u32x4*>(
-            bl + rb * MT_K + ((kk * 2 + hf) ^ ((rb >> 1) & 7)) * 8);
-        fa[t] = *reinterpret_cast<const u32x4*>(
-            al + ra * MT_K + ((kk * 2 + hf) ^ ((ra >> 1) & 7)) * 8);
-      }
+        for (int t = 0; t < 2; ++t) {
+          const int rb = wn * 64 + t * 32 + lc, ra = wm * 64 + t * 32 + lc;
+          fb[kk][t] = *reinterpret_cast<const u32x4*>(
+              bl + rb * MT_K + ((kk * 2 + hf) ^ ((rb >> 1) & 7)) * 8);
+          if (t == 0 || mine > 32)
+            fa[kk][t] = *reinterpret_cast<const u32x4*>(
+                al + ra * MT_K + ((kk * 2 + hf) ^ ((ra >> 1) & 7)) * 8);
+        }
 #pragma unroll
-      for (int a = 0; a < 2; ++a)
+      for (int kk = 0; kk < MT_K / 16; ++kk)
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
-          acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              __builtin_bit_cast(m_s16x8, fb[a]),
-              __builtin_bit_cast(m_s16x8, fa[b]), acc[a][b], 0, 0, 0);
+        for (int b = 0; b < 2; ++b) {
+          if (b == 1 && mine <= 32) continue;
+#pragma unroll
+          for (int a = 0; a < 2; ++a)
+            acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                __builtin_bit_cast(m_s16x8, fb[kk][a]),
+                __builtin_bit_cast(m_s16x8, fa[kk][b]), acc[a][b], 0, 0, 0);
+        }
     }
   }
   __syncthreads();
