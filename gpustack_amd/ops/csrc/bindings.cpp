@@ -25,7 +25,8 @@ void gemm_lab_launch(void*, const void*, const void*, int, int, int, int, int*, 
 void moe_tiles_launch(int*, int*, const int*, int, int, hipStream_t);
 void moe_down_scale_launch(void*, const void*, const void*, const int*, const int*, const int*, const float*, const void*, int, int, int, int*, hipStream_t);
 void moe_topk_launch(int*, float*, const float*, int, int, int, int, int*, hipStream_t);
-void moe_sort_launch(int*, int*, int*, int*, int*, int*, const int*, int, int, int, int*, hipStream_t);
+int moe_sort_slices(int);
+void moe_sort_launch(int*, int*, int*, int*, int*, int*, int*, const int*, int, int, int, int*, hipStream_t);
 void moe_sum_launch(void*, const void*, long, int, int, hipStream_t);
 void moe_tile_launch(int, void*, const void*, const void*, const int*, const int*, const int*, const int*, const int*, const float*, const void*, int, int, int, int, int*, hipStream_t);
 void rows_gemm_launch(void*, const void*, const void*, int, int, int, long, int*, hipStream_t);
@@ -402,11 +403,13 @@ std::vector<at::Tensor> moe_sort(at::Tensor experts, long E, long k) {
   at::Tensor order = at::empty({TK}, o), s_tok = at::empty({TK}, o);
   at::Tensor counts = at::empty({E}, o), offs = at::empty({E}, o);
   at::Tensor tiles = at::empty({TK / 128 + E, 2}, o), n = at::empty({1}, o);
+  const long slices = moe_sort_slices((int)TK);
+  at::Tensor hist = at::empty({slices * E}, o);
   int err = 0;
   moe_sort_launch(order.data_ptr<int>(), s_tok.data_ptr<int>(),
                   counts.data_ptr<int>(), offs.data_ptr<int>(),
                   tiles.data_ptr<int>(), n.data_ptr<int>(),
-                  experts.data_ptr<int>(), (int)TK, (int)E, (int)k, &err,
+                  hist.data_ptr<int>(), experts.data_ptr<int>(), (int)TK, (int)E, (int)k, &err,
                   cur_stream(experts));
   TORCH_CHECK(!err, "moe_sort: unsupported E=", E);
   HIP_CHECK_LAST();

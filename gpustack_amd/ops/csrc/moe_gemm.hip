@@ -396,40 +396,83 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(
 
 constexpr int MOE_MAX_E = 4096;
 
-// Counting sort of the assignments by expert in one workgroup: counts,
-// offsets, the sorted rows and the prompt form's tile list. The order within
-// an expert is free: a row's result does not depend on its place. Takes about
-// 5 us at 512 assignments (a radix sort, a scatter and the casts around them
-// took 100) and is one pass over the list beyond that.
+// Counting sort of the assignments by expert: counts, offsets, the sorted rows
+// and the tile list. The order within an expert is free: a row's result does
+// not depend on its place. A short list is one workgroup's (about 5 us at 512
+// assignments; a radix sort, a scatter and the casts around them took 100).
+// Longer ones (32544 took it 37 us) are cut into slices of MOE_SLICE: a first
+// kernel counts each slice's experts, and every workgroup of the second adds
+// up for itself where its slice begins in each expert.
+constexpr int MOE_SLICE = 2048;
+
+template <typename F>
+DEVICE_INLINE void moe_walk(const int* experts, int from, int to, int E, F f) {
+  int i = from + (int)threadIdx.x;
+  for (; i + 7 * 1024 < to; i += 8 * 1024) {  // eight loads in flight a thread
+    int e[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) e[j] = experts[i + j * 1024];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) f(i + j * 1024, min(max(e[j], 0), E - 1));
+  }
+  for (; i < to; i += 1024) f(i, min(max(experts[i], 0), E - 1));
+}
+
+__global__ __launch_bounds__(1024) void moe_count_kernel(
+    int* __restrict__ hist,            // [slices, E]
+    const int* __restrict__ experts, int TK, int E) {
+  __shared__ int cnt[MOE_MAX_E];
+  for (int e = threadIdx.x; e < E; e += 1024) cnt[e] = 0;
+  __syncthreads();
+  const int from = blockIdx.x * MOE_SLICE;
+  moe_walk(experts, from, min(TK, from + MOE_SLICE), E,
+           [&](int, int e) { atomicAdd(&cnt[e], 1); });
+  __syncthreads();
+  for (int e = threadIdx.x; e < E; e += 1024)
+    hist[(long)blockIdx.x * E + e] = cnt[e];
+}
+
+// gridDim.x slices with their counts in `hist`, or one workgroup without.
 __global__ __launch_bounds__(1024) void moe_sort_kernel(
     int* __restrict__ order, int* __restrict__ s_tok,  // [TK]
     int* __restrict__ counts, int* __restrict__ offs,  // [E]
     int* __restrict__ tiles, int* __restrict__ ntiles,
-    const int* __restrict__ experts, int TK, int E, int k) {
+    const int* __restrict__ experts, const int* __restrict__ hist, int TK,
+    int E, int k) {
   __shared__ int cnt[MOE_MAX_E];       // counts, then the next free places
   __shared__ int wsum[2][16];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  for (int e = tid; e < MOE_MAX_E; e += 1024) cnt[e] = 0;
-  __syncthreads();
-  auto walk = [&](auto f) {            // eight loads in flight a thread
-    int i = tid;
-    for (; i + 7 * 1024 < TK; i += 8 * 1024) {
-      int e[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) e[j] = experts[i + j * 1024];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) f(i + j * 1024, min(max(e[j], 0), E - 1));
-    }
-    for (; i < TK; i += 1024) f(i, min(max(experts[i], 0), E - 1));
-  };
-  walk([&](int, int e) { atomicAdd(&cnt[e], 1); });
-  __syncthreads();
-  // thread tid owns experts EPT * tid ..
   constexpr int EPT = MOE_MAX_E / 1024;
-  int c[EPT], a = 0, b = 0;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int from = hist != nullptr ? blockIdx.x * MOE_SLICE : 0;
+  const int to = hist != nullptr ? min(TK, from + MOE_SLICE) : TK;
+  // thread tid owns experts EPT * tid .. (one each up to 1024 of them)
+  const int ept = E <= 1024 ? 1 : EPT;
+  int c[EPT], before[EPT];
+#pragma unroll
+  for (int j = 0; j < EPT; ++j) c[j] = before[j] = 0;
+  if (hist == nullptr) {
+    for (int e = tid; e < E; e += 1024) cnt[e] = 0;
+    __syncthreads();
+    moe_walk(experts, from, to, E, [&](int, int e) { atomicAdd(&cnt[e], 1); });
+    __syncthreads();
+  }
 #pragma unroll
   for (int j = 0; j < EPT; ++j) {
-    c[j] = cnt[tid * EPT + j];
+    const int e = tid * ept + j;
+    if (j >= ept || e >= E) continue;
+    if (hist == nullptr) {
+      c[j] = cnt[e];
+    } else {
+      for (int b = 0; b < (int)gridDim.x; ++b) {
+        const int v = hist[(long)b * E + e];
+        c[j] += v;
+        if (b < (int)blockIdx.x) before[j] += v;
+      }
+    }
+  }
+  int a = 0, b = 0;
+#pragma unroll
+  for (int j = 0; j < EPT; ++j) {
     a += c[j];
     b += (c[j] + MT_M - 1) / MT_M;
   }
@@ -451,14 +494,16 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(
     a += wsum[0][i];
     b += wsum[1][i];
   }
-  if (tid == 1023) ntiles[0] = b;
+  const bool lead = blockIdx.x == 0;
+  if (lead && tid == 1023) ntiles[0] = b;
   a -= own_a;
   b -= own_b;
 #pragma unroll
   for (int j = 0; j < EPT; ++j) {
-    const int e = tid * EPT + j;
-    cnt[e] = a;
-    if (e < E) {
+    const int e = tid * ept + j;
+    if (j >= ept || e >= E) continue;
+    cnt[e] = a + before[j];
+    if (lead) {
       counts[e] = c[j];
       offs[e] = a;
       for (int r = 0; r < c[j]; r += MT_M, ++b) {
@@ -469,7 +514,7 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(
     a += c[j];
   }
   __syncthreads();
-  walk([&](int i, int e) {
+  moe_walk(experts, from, to, E, [&](int i, int e) {
     const int at = atomicAdd(&cnt[e], 1);
     order[at] = i;
     s_tok[at] = i / k;
@@ -536,13 +581,24 @@ void moe_topk_launch(int* experts, float* weights, const float* logits, int T,
 #undef TOPK
 }
 
+// hist: [slices, E] for moe_sort_slices(TK) > 0 of them, else unused
+int moe_sort_slices(int TK) {
+  return TK > 2 * MOE_SLICE ? (TK + MOE_SLICE - 1) / MOE_SLICE : 0;
+}
+
 void moe_sort_launch(int* order, int* s_tok, int* counts, int* offs,
-                     int* tiles, int* ntiles, const int* experts, int TK,
-                     int E, int k, int* err_unsupported, hipStream_t s) {
+                     int* tiles, int* ntiles, int* hist, const int* experts,
+                     int TK, int E, int k, int* err_unsupported,
+                     hipStream_t s) {
   *err_unsupported = E < 1 || E > MOE_MAX_E;
   if (*err_unsupported) return;
-  hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(1024), 0, s, order, s_tok,
-                     counts, offs, tiles, ntiles, experts, TK, E, k);
+  const int slices = moe_sort_slices(TK);
+  if (slices > 0)
+    hipLaunchKernelGGL(moe_count_kernel, dim3(slices), dim3(1024), 0, s, hist,
+                       experts, TK, E);
+  hipLaunchKernelGGL(moe_sort_kernel, dim3(slices > 0 ? slices : 1),
+                     dim3(1024), 0, s, order, s_tok, counts, offs, tiles,
+                     ntiles, experts, slices > 0 ? hist : nullptr, TK, E, k);
 }
 
 void moe_tiles_launch(int* tiles, int* ntiles, const int* counts, int E,

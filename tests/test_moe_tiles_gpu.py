@@ -104,13 +104,21 @@ def test_softmax_routing(renorm, T, E, k):
     torch.testing.assert_close(w.double(), ref, rtol=1e-5, atol=1e-7)
 
 
-def test_sort_of_a_long_list():
-    g = torch.Generator(device="cuda").manual_seed(3)
-    ex = torch.randint(0, 4000, (65536,), generator=g, device="cuda").int()
-    order, s_tok, cnt, offs, tiles, n = _hip().moe_sort(ex, 4096, 8)
-    ref = torch.bincount(ex.long(), minlength=4096)
+@pytest.mark.parametrize("TK,E", [(65536, 4096), (4096, 128), (4097, 128),
+                                  (32544, 128), (8192, 1025), (5000, 1)])
+def test_sort_of_a_long_list(TK, E):
+    g = torch.Generator(device="cuda").manual_seed(TK)
+    ex = torch.randint(0, max(1, E - 60), (TK,), generator=g,
+                       device="cuda").int()
+    order, s_tok, cnt, offs, tiles, n = _hip().moe_sort(ex, E, 8)
+    ref = torch.bincount(ex.long(), minlength=E)
     assert torch.equal(cnt.long(), ref)
     assert torch.equal(offs.long(), ref.cumsum(0) - ref)
-    assert torch.equal(order.long().sort().values,
-                       torch.arange(65536, device="cuda"))
-    assert n.item() == int(((ref + 127) // 128).sum())
+    o = order.long()
+    assert torch.equal(o.sort().values, torch.arange(TK, device="cuda"))
+    assert torch.equal(ex[o].sort().values, ex[o])
+    assert torch.equal(s_tok.long(), o // 8)
+    want = [(e, r) for e, c in enumerate(ref.tolist())
+            for r in range(0, c, 128)]
+    assert n.item() == len(want)
+    assert [tuple(t) for t in tiles[:len(want)].tolist()] == want
