@@ -53,17 +53,17 @@ class DenseFF(nn.Module):
                                    requires_grad=False)
 
     def forward(self, h, x32=None):
-        u = F.linear(h, self.up_w)
+        u = ops.linear_auto(h, self.up_w)
         if self.gated:
             g = torch.empty(h.shape[0], self.ff, dtype=h.dtype,
                             device=h.device)
             ops.act_and_mul(g, u[:, :self.cols], self.act)
             if self.extra:
-                return F.linear(g, self.down_w), u[:, self.cols:]
+                return ops.linear_auto(g, self.down_w), u[:, self.cols:]
             u = g
         else:
             ops.act_inplace(u, self.act)
-        return F.linear(u, self.down_w)
+        return ops.linear_auto(u, self.down_w)
 
 
 class RoutedFF(nn.Module):
@@ -203,8 +203,8 @@ class RoutedFF(nn.Module):
         inv[order] = ar
         shared = None
         if self.shared_up_w is not None:
-            su = self._act(F.linear(h, self.shared_up_w))
-            shared = F.linear(su, self.shared_down_w)
+            su = self._act(ops.linear_auto(h, self.shared_up_w))
+            shared = ops.linear_auto(su, self.shared_down_w)
         out = torch.empty(T, W, dtype=self.out_dtype, device=dev)
         ops.moe_combine(out, y, inv.view(T, self.top), weights, shared,
                         logits if self.gated else None, self.e)

@@ -21,7 +21,6 @@ signature, paged pools from KVCache, the ragged batch view).
 from __future__ import annotations
 
 import torch
-import torch.nn.functional as F
 from torch import nn
 
 from .. import ops
@@ -127,7 +126,7 @@ class FusipelForCausalLM(nn.Module):
         ops.rms_norm_rows(y, rows.contiguous(), self.final_norm, eps)
         if return_hidden:
             return y
-        logits = F.linear(y, self.lm_head).float()
+        logits = ops.linear_auto(y, self.lm_head).float()
         if return_both:
             return logits, y
         return logits

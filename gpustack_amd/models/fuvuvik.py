@@ -113,7 +113,7 @@ class FuvuvikForCausalLM(nn.Module):
                       self.ones, self.final_norm)
         if return_hidden:
             return y
-        logits = F.linear(y, self.lm_head).float()
+        logits = ops.linear_auto(y, self.lm_head).float()
         if return_both:
             return logits, y
         return logits

@@ -95,7 +95,7 @@ class LatentAttention(nn.Module):
             ctx_hts = ctx.transpose(0, 1).to(self.uv_t.dtype)
         o = torch.bmm(ctx_hts, self.uv_t)                  # [H, T, Dv]
         o = o.transpose(0, 1).reshape(T, self.h * self.dv)  # [T, H*Dv]
-        out = F.linear(o, self.o_w)
+        out = ops.linear_auto(o, self.o_w)
         return self.comm.all_reduce(out) if self.comm is not None else out
 
 
@@ -153,7 +153,7 @@ class RotaryLatentAttention(nn.Module):
         H, dqr = self.h, self.dq + self.rd
         half = m.rot.layout == "half"
         amp = m.rot.amplitude
-        u = F.linear(h, self.in_w)
+        u = ops.linear_auto(h, self.in_w)
         cq = torch.empty(T, self.qr, dtype=h.dtype, device=h.device)
         groups = (rg.page_groups(k_cache.shape[2])
                   if self.own_kv and h.is_cuda and k_cache.shape[2] == 16
@@ -187,5 +187,5 @@ class RotaryLatentAttention(nn.Module):
             ops.head_gate(o, o_hts, u, self.col_g)
         else:
             o = o_hts.transpose(0, 1).reshape(T, H * self.dv)
-        out = F.linear(o, self.o_w)
+        out = ops.linear_auto(o, self.o_w)
         return self.comm.all_reduce(out) if self.comm is not None else out

@@ -21,7 +21,6 @@ residual add on the fp32 stream and the next layer norm in the GEMM dtype.
 from __future__ import annotations
 
 import torch
-import torch.nn.functional as F
 from torch import nn
 
 from .. import ops
@@ -136,7 +135,7 @@ class LivasunForCausalLM(nn.Module):
                            eps, y)
         if return_hidden:
             return y
-        logits = F.linear(y, self.lm_head).float()
+        logits = ops.linear_auto(y, self.lm_head).float()
         if return_both:
             return logits, y
         return logits

@@ -21,7 +21,6 @@ norm before in the GEMM dtype.
 from __future__ import annotations
 
 import torch
-import torch.nn.functional as F
 from torch import nn
 
 from .. import ops
@@ -139,7 +138,7 @@ class MakezenForCausalLM(nn.Module):
                               self.final_norm, y, center=True)
         if return_hidden:
             return y
-        logits = F.linear(y, self.lm_head).float()
+        logits = ops.linear_auto(y, self.lm_head).float()
         if return_both:
             return logits, y
         return logits

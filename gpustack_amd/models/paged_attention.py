@@ -143,7 +143,8 @@ class PagedRotaryAttention(nn.Module):
         m = self.m
         T = h.shape[0]
         rg = meta.ragged
-        qkv = F.linear(h, self.qkv_w, self.qkv_b)
+        qkv = ops.linear_auto(h, self.qkv_w) if self.qkv_b is None \
+            else F.linear(h, self.qkv_w, self.qkv_b)
         gate = qkv[:, self.col_gate:self.col_gate + m.heads] \
             if m.out_gate else None
         if m.conv:
@@ -202,5 +203,5 @@ class PagedRotaryAttention(nn.Module):
                              m.diff, self.eps)
         else:
             o = a.view(T, A * self.vw)
-        out = F.linear(o, self.o_w)
+        out = ops.linear_auto(o, self.o_w)
         return self.comm.all_reduce(out) if self.comm is not None else out

@@ -21,7 +21,6 @@ decode rows and mixed batches take the same path.
 from __future__ import annotations
 
 import torch
-import torch.nn.functional as F
 from torch import nn
 
 from ..engine.config import EngineConfig
@@ -113,7 +112,7 @@ class SapatarForCausalLM(nn.Module):
                       self.ones, self.final_norm)
         if return_hidden:
             return y
-        logits = F.linear(y, self.lm_head).float()
+        logits = ops.linear_auto(y, self.lm_head).float()
         if return_both:
             return logits, y
         return logits

@@ -82,7 +82,7 @@ class Mamba2Mixer(nn.Module):
         m = self.m
         rg = meta.ragged
         T = h.shape[0]
-        u = F.linear(h, self.in_w)
+        u = ops.linear_auto(h, self.in_w)
         xbc = torch.empty(T, m.conv_channels, dtype=h.dtype, device=h.device)
         ops.causal_conv_silu(xbc, u, self.col_x, self.conv_w, self.conv_b,
                              conv_state, rg.seq_first, rg.seq_rows,
@@ -97,7 +97,7 @@ class Mamba2Mixer(nn.Module):
         g = torch.empty(T, m.inner, dtype=h.dtype, device=h.device)
         ops.gated_group_norm(g, y, u[:, :m.inner], self.norm, m.norm_groups,
                              self.eps, True)
-        out = F.linear(g, self.o_w)
+        out = ops.linear_auto(g, self.o_w)
         return self.comm.all_reduce(out) if self.comm is not None else out
 
 
@@ -123,7 +123,7 @@ class LightningMixer(nn.Module):
         m = self.m
         rg = meta.ragged
         T = h.shape[0]
-        u = F.linear(h, self.qkvg_w)
+        u = ops.linear_auto(h, self.qkvg_w)
         y = torch.empty(T, m.inner, dtype=torch.float32, device=h.device)
         ops.state_scan(y, u, 2 * self.nqk, self.nqk, 0, None, 0, m.heads,
                        m.heads, m.state, m.vdim, True, None, None, None,
@@ -133,7 +133,7 @@ class LightningMixer(nn.Module):
         g = torch.empty(T, m.inner, dtype=h.dtype, device=h.device)
         ops.gated_group_norm(g, y, u[:, 2 * self.nqk + m.inner:], self.norm,
                              1, self.eps, False)
-        out = F.linear(g, self.o_w)
+        out = ops.linear_auto(g, self.o_w)
         return self.comm.all_reduce(out) if self.comm is not None else out
 
 
@@ -169,7 +169,7 @@ class GatedDeltaMixer(nn.Module):
         m = self.m
         rg = meta.ragged
         T = h.shape[0]
-        u = F.linear(h, self.in_w)
+        u = ops.linear_auto(h, self.in_w)
         qkv = torch.empty(T, m.conv_channels, dtype=h.dtype, device=h.device)
         ops.causal_conv_silu(qkv, u, 0, self.conv_w, self.conv_b, conv_state,
                              rg.seq_first, rg.seq_rows, rg.state_slots,
@@ -183,7 +183,7 @@ class GatedDeltaMixer(nn.Module):
         g = torch.empty(T, m.inner, dtype=h.dtype, device=h.device)
         ops.gated_group_norm(g, y, u[:, self.col_gate:self.col_a],
                              self.norm_rows, m.heads, self.eps, 2)
-        out = F.linear(g, self.o_w)
+        out = ops.linear_auto(g, self.o_w)
         return self.comm.all_reduce(out) if self.comm is not None else out
 
 
@@ -204,13 +204,13 @@ class MinGruMixer(nn.Module):
     def forward(self, h, meta, state):
         n = self.m.width
         rg = meta.ragged
-        u = F.linear(h, self.in_w)
+        u = ops.linear_auto(h, self.in_w)
         y = torch.empty(h.shape[0], n, dtype=h.dtype, device=h.device)
         ops.gru_scan(y, u, 0, n, 2 * n, self.z_b, self.u_b, state,
                      rg.seq_first, rg.seq_rows, rg.state_slots, rg.pos32,
                      chunks=rg.scan_chunks(ops.SCAN_CHUNK) if h.is_cuda
                      else None)
-        out = F.linear(y, self.o_w)
+        out = ops.linear_auto(y, self.o_w)
         return self.comm.all_reduce(out) if self.comm is not None else out
 
 
@@ -275,7 +275,7 @@ class RetentionMixer(_MemoryMixer):
                 tables[m.rot] = ops.rope_table(meta.ragged.pos32,
                                                self.inv_freq)
             rot = tables[m.rot]
-        u = F.linear(h, self.in_w)
+        u = ops.linear_auto(h, self.in_w)
         y = self._scan(u[:, :n], u[:, n:2 * n], u[:, 2 * n:2 * n + m.inner],
                        meta, state, k_scale=m.state ** -0.5, decay=self.decay,
                        inv_freq=self.inv_freq, rot=rot)
@@ -321,7 +321,7 @@ class MlstmMixer(_MemoryMixer):
 
     def rows(self, h, meta, state, extra):
         m, n, g, i = self.m, self.nqk, self.col_g, self.col_i
-        u = F.linear(h, self.in_w)
+        u = ops.linear_auto(h, self.in_w)
         rden = torch.empty(h.shape[0], m.heads, dtype=torch.float32,
                            device=h.device)
         y = self._scan(u[:, :n], u[:, n:2 * n], u[:, 2 * n:g], meta, state,

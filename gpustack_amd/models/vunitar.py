@@ -15,7 +15,6 @@ from the scheduler) and asks the runner for the ragged batch view
 from __future__ import annotations
 
 import torch
-import torch.nn.functional as F
 from torch import nn
 
 from .. import ops
@@ -119,7 +118,7 @@ class VunitarForCausalLM(nn.Module):
         ops.rms_norm_f32(y, rows, self.final_norm, spec.rms_norm_eps)
         if return_hidden:
             return y
-        logits = F.linear(y, self.lm_head).float()
+        logits = ops.linear_auto(y, self.lm_head).float()
         if spec.final_logit_softcap:
             ops.softcap_(logits, spec.final_logit_softcap)
         if return_both:

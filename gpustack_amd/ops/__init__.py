@@ -298,9 +298,6 @@ def paged_prefill_attn(out, q, k_cache, v_cache, block_tables,
                                      softcap=softcap)
 
 
-_SG_WORKSPACES: dict = {}
-
-
 def gemm8(x, w, out=None, safe: bool = False):
     """8-phase pipelined 256x256 MFMA GEMM: out[M,N] = x[M,K] @ w[N,K]^T
     (bf16, f32 accumulate). GPU-only; requires N%256==0, K%128==0 —
@@ -341,11 +338,7 @@ def skinny_gemm(x, w, out=None, splitk: int | None = None, version: int = 1):
         out = torch.empty(M, N, dtype=x.dtype, device=x.device)
     ws = None
     if splitk > 1:
-        key = (splitk, M, N, x.device.index)
-        ws = _SG_WORKSPACES.get(key)
-        if ws is None:
-            ws = torch.empty(splitk * M * N, dtype=torch.float32, device=x.device)
-            _SG_WORKSPACES[key] = ws
+        ws = torch.empty(splitk * M * N, dtype=torch.float32, device=x.device)
     _load_hip().skinny_gemm(out, x, w, ws, splitk, version)
     return out
 
@@ -373,9 +366,63 @@ def _rows_gemm_wins(M: int, N: int, K: int) -> bool:
         N >= 12288 and N * K <= (280_000_000 if M <= 8 else 130_000_000))
 
 
+def _rows_tile_plan(M: int, N: int, K: int):
+    """(columns of a tile, parts of K) where the tiled product of up to 128
+    rows (rows_tile_kernel in ops/csrc/rows_gemm.hip) measured fastest, else
+    None. The split aims at one workgroup a CU (256); us against the library,
+    or up to 16 rows against the better of it and the decode product, weights
+    out of HBM:
+    up to 10240 columns, 48 rows: 4096x14336 26.0 / 36.3, 4096x4096 11.8 / 13.8,
+    5120x2048 10.7 / 12.9, 3072x8192 15.3 / 21.7; 96 rows: 4096x14336 30.1 / 50.1,
+    4096x4096 14.9 / 17.1; but 8192x4096 18.5 / 18.1 and 2048x4096 at 96 rows
+    13.5 / 12.8;
+    more columns, where the library loses on rows a multiple of 4 KB apart:
+    28672x4096 41.2 / 50.7 at 48 rows and 45.7 / 57.5 at 96, 128256x4096
+    182 / 254, 16384x2048 15.7 / 18.0, but 51200x3072 72 / 62 and at 96 rows
+    16384x2048 18.9 / 19.0 (18944 columns make 296 tiles, two for some CUs and
+    one for most: 31 / 27 at 2560);
+    up to 16 rows: 28672x4096 40 / 43 at one and 41 / 53 at 16, 4096x11008
+    17 / 31, 102400x4096 153 / 177, but 16384x4096 at one row 27 / 26."""
+    if not 0 < M <= 128 or K % 64 != 0 or N % 8 != 0 or min(N, K) < 1024:
+        return None
+    t64, t128 = -(-N // 64), -(-N // 128)
+    if N > 10240:
+        if 256 < t64 < 400:
+            return None
+        if M <= 16:
+            wins = (N <= 32768 and K >= 2560 and (
+                M > 4 or N >= 22016 or K >= 11008)
+                or N >= 100000 and K >= 3072)
+        elif M <= 64:
+            wins = K % 2048 == 0 and (K <= 8192 or N <= 32768)
+        else:
+            wins = K == 4096 and N >= 22016 or K == 2048 and N >= 51200
+        wide = 160 <= t128 <= 256 or t128 >= 500 or M > 64 and t128 > 256
+        plan = (128 if wide else 64), 1
+    elif K <= 2048:
+        wins = 16 < M <= 64 and (K == 1024 and N >= 2560
+                                 or 5120 <= N <= 8192)
+        plan = 32, 1
+    else:
+        if M <= 16:
+            wins = K >= 11008 or N > 8448
+        elif M <= 64:
+            wins = K >= 11008 or K >= 4096 and not 6144 < N <= 8448
+        else:
+            wins = N >= 3072 <= K or N >= 2048 and K >= 7168
+        parts = min(8, 256 // t64)
+        if t64 <= 24:
+            plan = 32, 8
+        elif parts * t64 >= 216 or parts == 8:
+            plan = 64, parts
+        else:
+            plan = 128, 256 // t128
+    return plan if wins else None
+
+
 def linear_auto(x, w):
-    """Shape-gated GEMM dispatch: the decode product for few rows
-    (_rows_gemm_wins), the split-K skinny kernel where it measured faster than
+    """Shape-gated GEMM dispatch: the products for few rows
+    (_rows_tile_plan, _rows_gemm_wins), the split-K skinny kernel where it measured faster than
     hipBLASLt (scripts/bench_skinny_gemm.py on MI355X: down_proj-like N=4096
     K>=8192 M>=384 at splitk=4, 824 TF vs hipBLASLt 680), F.linear everywhere
     else."""
@@ -387,17 +434,23 @@ def linear_auto(x, w):
             and os.environ.get("GPUSTACK_AMD_SKINNY_GEMM", "1") == "1"):
         M, K = x.shape
         N = w.shape[0]
-        if (_rows_gemm_wins(M, N, K) and M > 0
+        plan = _rows_tile_plan(M, N, K)
+        if ((plan or _rows_gemm_wins(M, N, K)) and M > 0
                 and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
                 and w.is_contiguous() and w.data_ptr() % 16 == 0
                 and x.stride(1) == 1 and x.stride(0) % 8 == 0
                 and x.data_ptr() % 16 == 0
                 and not (x.requires_grad or w.requires_grad)):
             out = torch.empty(M, N, dtype=x.dtype, device=x.device)
-            _load_hip().rows_gemm(out, x, w)
+            if plan:
+                _load_hip().rows_tile(out, x, w, *plan)
+            else:
+                _load_hip().rows_gemm(out, x, w)
             return out
         if (N == 4096 and K >= 8192 and 384 <= M <= 1024
-                and K % 256 == 0 and x.stride(1) == 1):
+                and K % 256 == 0
+                and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+                and x.is_contiguous() and w.is_contiguous()):
             return skinny_gemm(x, w, splitk=4)
     return F.linear(x, w)
 

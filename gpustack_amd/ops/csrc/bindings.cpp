@@ -29,6 +29,7 @@ int moe_sort_slices(int);
 void moe_sort_launch(int*, int*, int*, int*, int*, int*, int*, const int*, int, int, int, int*, hipStream_t);
 void moe_sum_launch(void*, const void*, long, int, int, hipStream_t);
 void moe_tile_launch(int, void*, const void*, const void*, const int*, const int*, const int*, const int*, const int*, const float*, const void*, int, int, int, int, int*, hipStream_t);
+void rows_tile_launch(void*, void*, const void*, const void*, int, int, int, long, int, int, int*, hipStream_t);
 void rows_gemm_launch(void*, const void*, const void*, int, int, int, long, int*, hipStream_t);
 void w4_gemm_launch(void*, const void*, const void*, const void*, const void*, int, int, int, int*, hipStream_t);
 void w4_dequant_launch(void*, const void*, const void*, const void*, long, int, int*, hipStream_t);
@@ -468,6 +469,26 @@ void moe_tile(bool down, at::Tensor out, at::Tensor src, at::Tensor w,
   HIP_CHECK_LAST();
 }
 
+void rows_tile(at::Tensor out, at::Tensor x, at::Tensor w, long cols,
+               long splits) {
+  check_bf16(out, "out"); check_bf16(w, "w");
+  TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 && x.dim() == 2
+              && x.stride(1) == 1 && x.stride(0) % 8 == 0
+              && (uintptr_t)x.data_ptr() % 16 == 0, "x rows of bf16");
+  const int M = x.size(0), K = x.size(1), N = w.size(0);
+  TORCH_CHECK(w.size(1) == K && out.size(0) == M && out.size(1) == N &&
+              (uintptr_t)w.data_ptr() % 16 == 0, "rows_tile shapes");
+  at::Tensor parts;
+  if (splits > 1)
+    parts = at::empty({splits, M, N}, out.options().dtype(at::kFloat));
+  int err = 0;
+  rows_tile_launch(out.data_ptr(), splits > 1 ? parts.data_ptr() : nullptr,
+                   x.data_ptr(), w.data_ptr(), M, N, K, x.stride(0),
+                   (int)cols, (int)splits, &err, cur_stream(x));
+  TORCH_CHECK(!err, "rows_tile: unsupported M=", M, " N=", N, " K=", K);
+  HIP_CHECK_LAST();
+}
+
 void rows_gemm(at::Tensor out, at::Tensor x, at::Tensor w) {
   check_bf16(out, "out"); check_bf16(w, "w");
   TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 && x.dim() == 2
@@ -584,6 +605,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_gemm", &skinny_gemm, "split-K skinny GEMM (bf16, f32 accum)");
   m.def("gemm8", &gemm8, "8-phase pipelined 256x256 GEMM (bf16, f32 accum)");
   m.def("gemm_lab", &gemm_lab, "GEMM schedule lab variants (A/B vs hipBLASLt)");
+  m.def("rows_tile", &rows_tile, "bf16 product of up to 128 rows in tiles");
   m.def("rows_gemm", &rows_gemm, "bf16 product of up to 64 rows");
   m.def("moe_topk", &moe_topk, "softmax routing, top k");
   m.def("moe_sort", &moe_sort, "assignments by expert, and the tile list");

@@ -35,6 +35,33 @@ def test_rows_gemm(M, N, K):
     _close(out, x.double() @ w.double().T, x.double().abs() @ w.double().abs().T)
 
 
+@pytest.mark.parametrize("M", [1, 32, 33, 64, 65, 97, 128])
+@pytest.mark.parametrize("N,K,cols,parts", [
+    (8, 64, 32, 1), (136, 128, 64, 2), (260, 640, 128, 3), (4096, 1088, 32, 5),
+    (33000, 448, 128, 1), (20000, 576, 32, 1)])
+def test_rows_tile(M, N, K, cols, parts):
+    g = torch.Generator(device="cuda").manual_seed(M * N)
+    x = torch.randn(M, K + 8, generator=g, device="cuda").bfloat16()[:, :K]
+    w = torch.randn(N, K, generator=g, device="cuda").bfloat16()
+    out = torch.full((M, N), 9.0, device="cuda").bfloat16()
+    _hip().rows_tile(out, x, w, cols, parts)
+    _close(out, x.double() @ w.double().T, x.double().abs() @ w.double().abs().T)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 28672, 4096), (48, 4096, 14336),
+                                   (17, 1024, 4096), (96, 10240, 3072),
+                                   (64, 5128, 1024), (128, 3072, 3072)])
+def test_linear_auto_takes_the_tiles(M, N, K):
+    from gpustack_amd import ops
+
+    assert ops._rows_tile_plan(M, N, K) is not None
+    g = torch.Generator(device="cuda").manual_seed(N)
+    x = torch.randn(M, K, generator=g, device="cuda").bfloat16()
+    w = torch.randn(N, K, generator=g, device="cuda").bfloat16()
+    _close(ops.linear_auto(x, w), x.double() @ w.double().T,
+           x.double().abs() @ w.double().abs().T)
+
+
 @pytest.mark.parametrize("M", [1, 16, 17, 33, 64, 65])
 @pytest.mark.parametrize("N,K", [(64, 128), (128, 1152), (14400, 256),
                                  (28736, 384)])
