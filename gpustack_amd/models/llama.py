@@ -765,26 +765,50 @@ class MoEMLP(nn.Module):
         # MoE expert MLPs do not take LoRA (rejected at adapter load);
         # attention adapters still apply upstream
         T = x.shape[0]
-        rw = getattr(self, "_router_w_f32", None)
-        if rw is None or rw.device != x.device:
-            self._router_w_f32 = self.router_w.float()
-            rw = self._router_w_f32
-        logits = F.linear(x.float(), rw)                          # [T, E]
-        if self.spec.router_logit_bias and self.router_bias is not None:
-            logits = logits + self.router_bias  # GPT-OSS: bias on logits
         fused = self._fused_ok(x)
-        if fused and self.spec.router_mode != "sigmoid_bias" \
-                and self.e <= 1024:
-            # softmax routing in one launch (a top-k, a sort and a softmax
-            # otherwise)
+        # softmax routing in one launch (a top-k, a sort and a softmax
+        # otherwise)
+        soft = fused and self.spec.router_mode != "sigmoid_bias" \
+            and self.e <= 1024
+        bias = self.router_bias if self.spec.router_logit_bias else None
+        if soft:
+            hip = ops._load_hip()
             experts = torch.empty(T, self.top_k, dtype=torch.int32,
                                   device=x.device)
             weights = torch.empty(T, self.top_k, dtype=torch.float32,
                                   device=x.device)
-            ops._load_hip().moe_topk(experts, weights, logits,
-                                     bool(self.spec.norm_topk_prob))
+        # Products of bf16 are exact in fp32, so the router's product runs on
+        # its bf16 operands: in the launch that chooses (us against cast,
+        # product and choice apart: 8 experts of 4096 at 64 / 4096 rows 9 / 15
+        # and 10 / 35, 128 of 2048 at 4068 rows 26 / 55, but at 512 25 / 19),
+        # for fewer rows in four parts over k (128 of 2048 at 1 / 64 / 128 rows
+        # 11 / 13 / 14 against 16 / 18 / 18; 512 experts 23 / 22).
+        exact = (soft and bias is None
+                 and x.dtype == self.router_w.dtype == torch.bfloat16
+                 and x.is_contiguous() and self.router_w.is_contiguous()
+                 and (x.data_ptr() | self.router_w.data_ptr()) % 16 == 0
+                 and self.router_w.device == x.device)
+        if exact and T <= 128 and 16 < self.e <= 256 and self.e % 4 == 0 \
+                and x.shape[1] >= 1024:
+            hip.moe_topk(experts, weights,
+                         hip.rows_tile_parts(x, self.router_w, 32, 4),
+                         bool(self.spec.norm_topk_prob))
+        elif exact and (self.e <= 64 or self.e <= 128 and T >= 2048):
+            hip.moe_route(experts, weights, x, self.router_w,
+                          bool(self.spec.norm_topk_prob))
         else:
-            weights, experts = self._route(logits)
+            rw = getattr(self, "_router_w_f32", None)
+            if rw is None or rw.device != x.device:
+                self._router_w_f32 = self.router_w.float()
+                rw = self._router_w_f32
+            logits = F.linear(x.float(), rw)                      # [T, E]
+            if bias is not None:
+                logits = logits + bias  # GPT-OSS: bias on logits
+            if soft:
+                hip.moe_topk(experts, weights, logits,
+                             bool(self.spec.norm_topk_prob))
+            else:
+                weights, experts = self._route(logits)
         if fused:
             out = self._fused_dispatch(x, experts, weights)
             return self.comm.all_reduce(self._add_shared(x, out))

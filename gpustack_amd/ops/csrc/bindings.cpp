@@ -24,7 +24,8 @@ void skinny_gemm_v2_launch(void*, const void*, const void*, void*, int, int, int
 void gemm_lab_launch(void*, const void*, const void*, int, int, int, int, int*, hipStream_t);
 void moe_tiles_launch(int*, int*, const int*, int, int, hipStream_t);
 void moe_down_scale_launch(void*, const void*, const void*, const int*, const int*, const int*, const float*, const void*, int, int, int, int*, hipStream_t);
-void moe_topk_launch(int*, float*, const float*, int, int, int, int, int*, hipStream_t);
+void moe_topk_launch(int*, float*, const float*, int, int, int, int, int, int*, hipStream_t);
+void moe_route_launch(int*, float*, const void*, const void*, int, int, int, int, int, int*, hipStream_t);
 int moe_sort_slices(int);
 void moe_sort_launch(int*, int*, int*, int*, int*, int*, int*, const int*, int, int, int, int*, hipStream_t);
 void moe_sum_launch(void*, const void*, long, int, int, hipStream_t);
@@ -379,7 +380,8 @@ void check_i32(const at::Tensor& t, long n, const char* name) {
 
 void moe_topk(at::Tensor experts, at::Tensor weights, at::Tensor logits,
               bool renorm) {
-  const int T = logits.size(0), E = logits.size(1), k = experts.size(1);
+  const int parts = logits.dim() == 3 ? logits.size(0) : 1;
+  const int T = logits.size(-2), E = logits.size(-1), k = experts.size(1);
   check_i32(experts, (long)T * k, "experts");
   TORCH_CHECK(logits.is_cuda() && logits.scalar_type() == at::kFloat
               && logits.is_contiguous(), "logits must be fp32");
@@ -389,9 +391,28 @@ void moe_topk(at::Tensor experts, at::Tensor weights, at::Tensor logits,
               && experts.numel() == (long)T * k, "experts / weights [T, k]");
   int err = 0;
   moe_topk_launch(experts.data_ptr<int>(), weights.data_ptr<float>(),
-                  logits.data_ptr<float>(), T, E, k, renorm ? 1 : 0, &err,
-                  cur_stream(logits));
+                  logits.data_ptr<float>(), T, E, k, renorm ? 1 : 0, parts,
+                  &err, cur_stream(logits));
   TORCH_CHECK(!err, "moe_topk: unsupported E=", E, " k=", k);
+  HIP_CHECK_LAST();
+}
+
+void moe_route(at::Tensor experts, at::Tensor weights, at::Tensor x,
+               at::Tensor w, bool renorm) {
+  check_bf16(x, "x"); check_bf16(w, "w");
+  const int T = x.size(0), H = x.size(1), E = w.size(0), k = experts.size(1);
+  check_i32(experts, (long)T * k, "experts");
+  TORCH_CHECK(w.size(1) == H && (uintptr_t)x.data_ptr() % 16 == 0
+              && (uintptr_t)w.data_ptr() % 16 == 0, "moe_route operands");
+  TORCH_CHECK(weights.is_cuda() && weights.scalar_type() == at::kFloat
+              && weights.is_contiguous()
+              && weights.numel() == (long)T * k
+              && experts.numel() == (long)T * k, "experts / weights [T, k]");
+  int err = 0;
+  moe_route_launch(experts.data_ptr<int>(), weights.data_ptr<float>(),
+                   x.data_ptr(), w.data_ptr(), T, E, H, k, renorm ? 1 : 0,
+                   &err, cur_stream(x));
+  TORCH_CHECK(!err, "moe_route: unsupported E=", E, " H=", H, " k=", k);
   HIP_CHECK_LAST();
 }
 
@@ -467,6 +488,21 @@ void moe_tile(bool down, at::Tensor out, at::Tensor src, at::Tensor w,
                   cur_stream(src));
   TORCH_CHECK(!err, "moe_tile: unsupported dims N=", N, " K=", K);
   HIP_CHECK_LAST();
+}
+
+// fp32 parts [splits, M, N] of the product, not added up
+at::Tensor rows_tile_parts(at::Tensor x, at::Tensor w, long cols, long splits) {
+  check_bf16(x, "x"); check_bf16(w, "w");
+  const int M = x.size(0), K = x.size(1), N = w.size(0);
+  TORCH_CHECK(w.size(1) == K && (uintptr_t)x.data_ptr() % 16 == 0 &&
+              (uintptr_t)w.data_ptr() % 16 == 0, "rows_tile_parts shapes");
+  at::Tensor parts = at::empty({splits, M, N}, x.options().dtype(at::kFloat));
+  int err = 0;
+  rows_tile_launch(nullptr, parts.data_ptr(), x.data_ptr(), w.data_ptr(), M, N,
+                   K, K, (int)cols, (int)splits, &err, cur_stream(x));
+  TORCH_CHECK(!err, "rows_tile_parts: unsupported M=", M, " N=", N, " K=", K);
+  HIP_CHECK_LAST();
+  return parts;
 }
 
 void rows_tile(at::Tensor out, at::Tensor x, at::Tensor w, long cols,
@@ -605,8 +641,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_gemm", &skinny_gemm, "split-K skinny GEMM (bf16, f32 accum)");
   m.def("gemm8", &gemm8, "8-phase pipelined 256x256 GEMM (bf16, f32 accum)");
   m.def("gemm_lab", &gemm_lab, "GEMM schedule lab variants (A/B vs hipBLASLt)");
+  m.def("rows_tile_parts", &rows_tile_parts,
+        "fp32 parts over k of a product of up to 128 rows");
   m.def("rows_tile", &rows_tile, "bf16 product of up to 128 rows in tiles");
   m.def("rows_gemm", &rows_gemm, "bf16 product of up to 64 rows");
+  m.def("moe_route", &moe_route, "router product and choice");
   m.def("moe_topk", &moe_topk, "softmax routing, top k");
   m.def("moe_sort", &moe_sort, "assignments by expert, and the tile list");
   m.def("moe_sum", &moe_sum, "sum of a row's expert contributions");

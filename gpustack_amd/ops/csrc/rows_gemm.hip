@@ -274,10 +274,11 @@ template <int MT, int NT, int S>
 void rows_tile(void* out, void* parts, const void* x, const void* w, int M,
                int N, int K, long xs, int splits, hipStream_t s) {
   const int nt = (N + 16 * NT - 1) / (16 * NT);
-  if (splits > 1) {
+  if (splits > 1 || out == nullptr) {
     hipLaunchKernelGGL((rows_tile_kernel<MT, NT, S, true>), dim3(nt * splits),
                        dim3(256), 0, s, parts, (const unsigned short*)x,
                        (const unsigned short*)w, M, N, K, xs, splits);
+    if (out == nullptr) return;
     const long MN = (long)M * N;
     hipLaunchKernelGGL(rows_join_kernel, dim3((MN / 4 + 255) / 256), dim3(256),
                        0, s, (unsigned short*)out, (const float*)parts, MN,
@@ -317,7 +318,7 @@ void rows_gemm_launch(void* out, const void* x, const void* w, int M, int N,
   }
 }
 
-// parts: fp32 [splits, M, N] where splits > 1
+// parts: fp32 [splits, M, N] where splits > 1, or the result where out is null
 void rows_tile_launch(void* out, void* parts, const void* x, const void* w,
                       int M, int N, int K, long xs, int cols, int splits,
                       int* err_unsupported, hipStream_t s) {

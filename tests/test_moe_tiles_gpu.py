@@ -122,3 +122,35 @@ def test_sort_of_a_long_list(TK, E):
             for r in range(0, c, 128)]
     assert n.item() == len(want)
     assert [tuple(t) for t in tiles[:len(want)].tolist()] == want
+
+
+@pytest.mark.parametrize("T,E,H,k", [(1, 1, 128, 1), (15, 16, 256, 2),
+                                     (17, 33, 2048, 4), (64, 64, 2176, 64),
+                                     (100, 128, 2048, 8), (4068, 127, 4096, 8)])
+@pytest.mark.parametrize("renorm", [True, False])
+@pytest.mark.parametrize("parts", [0, 4])
+def test_route(T, E, H, k, renorm, parts):
+    if parts and (T > 128 or E % 4):
+        pytest.skip("the parts take up to 128 rows, columns in fours")
+    g = torch.Generator(device="cuda").manual_seed(T + E)
+    x = torch.randn(T, H, generator=g, device="cuda").bfloat16()
+    w = (torch.randn(E, H, generator=g, device="cuda") / H ** 0.5).bfloat16()
+    experts = torch.full((T, k), -1, dtype=torch.int32, device="cuda")
+    weights = torch.empty(T, k, device="cuda")
+    if parts:
+        _hip().moe_topk(experts, weights, _hip().rows_tile_parts(
+            x, w, 32, min(parts, H // 64)), renorm)
+    else:
+        _hip().moe_route(experts, weights, x, w, renorm)
+    logits = x.double() @ w.double().T
+    # fp32 sums of exact products: at most 2^-18 of the terms' absolute sum
+    eps = float((x.double().abs() @ w.double().abs().T).max()) * 2.0 ** -18
+    got = logits.gather(1, experts.long())
+    best = logits.sort(1, descending=True).values[:, :k]
+    assert bool(((got - best).abs() <= 2 * eps).all())
+    assert bool((experts.long().sort(1).values.diff(dim=1) > 0).all())
+    p = torch.softmax(got if renorm else logits, 1)
+    want = p if renorm else p.gather(1, experts.long())
+    # a logit off by eps moves a weight by 2 eps of itself; fp32 exp and sum
+    assert bool(((weights.double() - want).abs()
+                 <= want * (4 * eps + 2.0 ** -18) + 2.0 ** -30).all())
