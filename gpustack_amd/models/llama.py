@@ -778,24 +778,20 @@ class MoEMLP(nn.Module):
             weights = torch.empty(T, self.top_k, dtype=torch.float32,
                                   device=x.device)
         # Products of bf16 are exact in fp32, so the router's product runs on
-        # its bf16 operands: in the launch that chooses (us against cast,
-        # product and choice apart: 8 experts of 4096 at 64 / 4096 rows 9 / 15
-        # and 10 / 35, 128 of 2048 at 4068 rows 26 / 55, but at 512 25 / 19),
-        # for fewer rows in four parts over k (128 of 2048 at 1 / 64 / 128 rows
-        # 11 / 13 / 14 against 16 / 18 / 18; 512 experts 23 / 22).
+        # its bf16 operands, up to 16 experts in the launch that chooses.
         exact = (soft and bias is None
                  and x.dtype == self.router_w.dtype == torch.bfloat16
                  and x.is_contiguous() and self.router_w.is_contiguous()
                  and (x.data_ptr() | self.router_w.data_ptr()) % 16 == 0
                  and self.router_w.device == x.device)
-        if exact and T <= 128 and 16 < self.e <= 256 and self.e % 4 == 0 \
-                and x.shape[1] >= 1024:
-            hip.moe_topk(experts, weights,
-                         hip.rows_tile_parts(x, self.router_w, 32, 4),
-                         bool(self.spec.norm_topk_prob))
-        elif exact and (self.e <= 64 or self.e <= 128 and T >= 2048):
+        plan = ops.router_plan(T, self.e, x.shape[1]) if exact else None
+        if exact and self.e <= 16:
             hip.moe_route(experts, weights, x, self.router_w,
                           bool(self.spec.norm_topk_prob))
+        elif plan:
+            hip.moe_topk(experts, weights,
+                         hip.rows_tile_parts(x, self.router_w, *plan),
+                         bool(self.spec.norm_topk_prob))
         else:
             rw = getattr(self, "_router_w_f32", None)
             if rw is None or rw.device != x.device:

@@ -420,6 +420,27 @@ def _rows_tile_plan(M: int, N: int, K: int):
     return plan if wins else None
 
 
+def router_plan(T: int, E: int, H: int):
+    """(columns of a tile, parts over k) of a router's product, whose parts the
+    choice of the experts adds up, or None. us for both launches against a
+    cast, an fp32 library product and the choice, at 64 / 1024 / 4068 / 16384
+    rows: 64 experts of 2048 10 / 13 / 17 / 33 against 16 / 21 / 39 / 87, 128
+    of 2048 13 / 16 / 21 / 41 against 18 / 24 / 57 / 125, 256 of 4096 18 / 23 /
+    38 / 91 against 21 / 40 / 109 / 317; 512 of 2048 22 / 27 / 37 / 102 against
+    23 / 39 / 96 / 311, but at 128 rows 25 against 24. Four parts of narrow
+    tiles fill the chip for few rows; later the parts' own traffic counts (128
+    experts at 16384 rows 57)."""
+    if E % 4 != 0 or H % 64 != 0 or H < 1024 or E > 512 or T == 0:
+        return None
+    if E > 256:
+        if 64 < T < 256:
+            return None
+        return (64, 2) if T <= 2048 else (128, 2)
+    if T * E <= 1 << 19:
+        return 32, 4
+    return (128, 2) if E >= 128 else (64, 2)
+
+
 def linear_auto(x, w):
     """Shape-gated GEMM dispatch: the products for few rows
     (_rows_tile_plan, _rows_gemm_wins), the split-K skinny kernel where it measured faster than

@@ -406,65 +406,53 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(
 }
 
 // The router's product and the choice in one launch, for bf16 rows and router
-// weights of up to 16 NT <= 128 experts: products of bf16 are exact in fp32,
-// so bf16 matrix instructions and their fp32 sums stand for the fp32 product
-// of the casted operands. A workgroup takes 16 rows, its 16 waves the 128-k
-// blocks in turn; the sums meet in the LDS, where each wave then chooses for
-// one row. Bound by latency and, over many rows, by the router's weights out
-// of the L2, once per 16 rows: 26 us at 4068 rows over 128 experts of 2048 (the
-// cast, the fp32 product and the choice apart 55), 10 at 4096 over 8 of 4096
-// (35).
-template <int NT>
+// weights of up to 16 experts: products of bf16 are exact in fp32, so bf16
+// matrix instructions and their fp32 sums stand for the fp32 product of the
+// casted operands. A workgroup takes 16 rows, its 16 waves the 128-k blocks in
+// turn; the sums meet in the LDS, where each wave then chooses for one row.
+// Bound by latency: 9 us at 64 rows over 8 experts of 4096, 12 at 4068 (cast,
+// fp32 product and choice apart: 15 and 40). With more experts the router's
+// weights, read again by every workgroup, take over (128 of 2048 at 64 rows
+// 25): those take the tiled product's parts and the choice above.
 __global__ __launch_bounds__(1024) void moe_route_kernel(
     int* __restrict__ experts,               // [T, k]
     float* __restrict__ weights,             // [T, k]
     const unsigned short* __restrict__ x,    // [T, H]
     const unsigned short* __restrict__ w,    // [E, H]
     int T, int E, int H, int k, int renorm) {
-  constexpr int COLS = 16 * NT, NV = (COLS + 63) / 64;
-  __shared__ float red[16 * 16 * COLS];
+  __shared__ float red[16 * 16 * 16];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE_SIZE);
   const int lc = lane & 15, lg = lane >> 4;
   const int t0 = blockIdx.x * 16;
   const unsigned short* xp = x + (long)min(t0 + lc, T - 1) * H + lg * 8;
-  const unsigned short* wp[NT];
-  f32x4 acc[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    wp[t] = w + (long)min(t * 16 + lc, E - 1) * H + lg * 8;
-    acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
+  const unsigned short* wp = w + (long)min(lc, E - 1) * H + lg * 8;
+  f32x4 acc{0.f, 0.f, 0.f, 0.f};
   for (int b = wave; b < H / 128; b += 16)
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const u32x4 fx = *reinterpret_cast<const u32x4*>(xp + b * 128 + c * 32);
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            __builtin_bit_cast(m_s16x8, fx),
-            __builtin_bit_cast(m_s16x8, *reinterpret_cast<const u32x4*>(
-                                            wp[t] + b * 128 + c * 32)),
-            acc[t], 0, 0, 0);
-    }
+    for (int c = 0; c < 4; ++c)
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+          __builtin_bit_cast(m_s16x8, *reinterpret_cast<const u32x4*>(
+                                          xp + b * 128 + c * 32)),
+          __builtin_bit_cast(m_s16x8, *reinterpret_cast<const u32x4*>(
+                                          wp + b * 128 + c * 32)),
+          acc, 0, 0, 0);
   // D[row = lg*4 + r][expert = lc]
 #pragma unroll
-  for (int t = 0; t < NT; ++t)
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      red[(wave * 16 + lg * 4 + r) * COLS + t * 16 + lc] = acc[t][r];
+  for (int r = 0; r < 4; ++r)
+    red[(wave * 16 + lg * 4 + r) * 16 + lc] = acc[r];
   __syncthreads();
-  for (int u = tid; u < 16 * COLS; u += 1024) {
+  if (tid < 256) {
     float v = 0.f;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) v += red[i * 16 * COLS + u];
-    red[u] = v;                              // read by this thread alone so far
+    for (int i = 0; i < 16; ++i) v += red[i * 256 + tid];
+    red[tid] = v;                            // read by this thread alone so far
   }
   __syncthreads();
   if (t0 + wave < T)
-    moe_topk_row<NV>(experts + (long)(t0 + wave) * k,
-                     weights + (long)(t0 + wave) * k, red + wave * COLS, lane,
-                     E, k, renorm);
+    moe_topk_row<1>(experts + (long)(t0 + wave) * k,
+                    weights + (long)(t0 + wave) * k, red + wave * 16, lane, E,
+                    k, renorm);
 }
 
 constexpr int MOE_MAX_E = 4096;
@@ -657,18 +645,12 @@ void moe_topk_launch(int* experts, float* weights, const float* logits, int T,
 void moe_route_launch(int* experts, float* weights, const void* x,
                       const void* w, int T, int E, int H, int k, int renorm,
                       int* err_unsupported, hipStream_t s) {
-  *err_unsupported = E < 1 || E > 128 || k < 1 || k > 64 || k > E ||
-                     H < 128 || H % 128 != 0;
+  *err_unsupported = E < 1 || E > 16 || k < 1 || k > E || H < 128 ||
+                     H % 128 != 0;
   if (*err_unsupported || T == 0) return;
-#define ROUTE(NT)                                                             \
-  hipLaunchKernelGGL((moe_route_kernel<NT>), dim3((T + 15) / 16), dim3(1024), \
-                     0, s, experts, weights, (const unsigned short*)x,        \
-                     (const unsigned short*)w, T, E, H, k, renorm)
-  if (E <= 16) ROUTE(1);
-  else if (E <= 32) ROUTE(2);
-  else if (E <= 64) ROUTE(4);
-  else ROUTE(8);
-#undef ROUTE
+  hipLaunchKernelGGL(moe_route_kernel, dim3((T + 15) / 16), dim3(1024), 0, s,
+                     experts, weights, (const unsigned short*)x,
+                     (const unsigned short*)w, T, E, H, k, renorm);
 }
 
 // hist: [slices, E] for moe_sort_slices(TK) > 0 of them, else unused

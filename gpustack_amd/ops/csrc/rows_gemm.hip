@@ -154,6 +154,7 @@ __global__ __launch_bounds__(256, 2) void rows_tile_kernel(
   __shared__ unsigned short lds[S * BUF];
   const int split = SPLIT ? blockIdx.x % splits : 0;
   const int n0 = (SPLIT ? blockIdx.x / splits : blockIdx.x) * 16 * NT;
+  const int m0 = blockIdx.y * 16 * MT;
   const int total = K / RT_K;
   const int from = SPLIT ? (int)((long)total * split / splits) : 0;
   const int n = (SPLIT ? (int)((long)total * (split + 1) / splits) : total) - from;
@@ -169,7 +170,8 @@ __global__ __launch_bounds__(256, 2) void rows_tile_kernel(
 #pragma unroll
   for (int i = 0; i < MT / 2; ++i) {
     const int row = (i * 4 + wave) * 8 + lane / 8;
-    xp[i] = x + (long)min(row, M - 1) * xs + ((lane & 7) ^ ((row >> 1) & 7)) * 8;
+    xp[i] = x + (long)min(m0 + row, M - 1) * xs +
+            ((lane & 7) ^ ((row >> 1) & 7)) * 8;
   }
 #pragma unroll
   for (int i = 0; i < NT / 2; ++i) {
@@ -237,7 +239,7 @@ __global__ __launch_bounds__(256, 2) void rows_tile_kernel(
   // D[column = lg*4 + r][row = lc] per 16x16 tile
 #pragma unroll
   for (int m = 0; m < MT / 2; ++m) {
-    const int row = (wm * MT / 2 + m) * 16 + lc;
+    const int row = m0 + (wm * MT / 2 + m) * 16 + lc;
     if (row >= M) continue;
 #pragma unroll
     for (int t = 0; t < NT / 2; ++t) {
@@ -275,7 +277,8 @@ void rows_tile(void* out, void* parts, const void* x, const void* w, int M,
                int N, int K, long xs, int splits, hipStream_t s) {
   const int nt = (N + 16 * NT - 1) / (16 * NT);
   if (splits > 1 || out == nullptr) {
-    hipLaunchKernelGGL((rows_tile_kernel<MT, NT, S, true>), dim3(nt * splits),
+    hipLaunchKernelGGL((rows_tile_kernel<MT, NT, S, true>),
+                       dim3(nt * splits, (M + 16 * MT - 1) / (16 * MT)),
                        dim3(256), 0, s, parts, (const unsigned short*)x,
                        (const unsigned short*)w, M, N, K, xs, splits);
     if (out == nullptr) return;
@@ -318,11 +321,13 @@ void rows_gemm_launch(void* out, const void* x, const void* w, int M, int N,
   }
 }
 
-// parts: fp32 [splits, M, N] where splits > 1, or the result where out is null
+// parts: fp32 [splits, M, N] where splits > 1, or the result, for any number of
+// rows, where out is null
 void rows_tile_launch(void* out, void* parts, const void* x, const void* w,
                       int M, int N, int K, long xs, int cols, int splits,
                       int* err_unsupported, hipStream_t s) {
-  *err_unsupported = K % RT_K != 0 || K == 0 || M > 128 || N % 4 != 0 ||
+  *err_unsupported = K % RT_K != 0 || K == 0 ||
+                     (M > 128 && out != nullptr) || N % 4 != 0 ||
                      splits < 1 || splits > K / RT_K ||
                      (cols != 32 && cols != 64 && cols != 128);
   if (*err_unsupported || M == 0 || N == 0) return;
@@ -332,7 +337,8 @@ void rows_tile_launch(void* out, void* parts, const void* x, const void* w,
   else rows_tile<MT, 8, S8>(out, parts, x, w, M, N, K, xs, splits, s);
   if (M <= 32) { RT(2, 8, 6, 4) }
   else if (M <= 64) { RT(4, 6, 5, 3) }
-  else if ((N + cols - 1) / cols * splits <= 256) {   // one workgroup a CU
+  else if ((N + cols - 1) / cols * splits * ((M + 127) / 128) <= 256) {
+    // one workgroup a CU
     if (M <= 96) { RT(6, 8, 7, 5) }
     else { RT(8, 7, 6, 4) }
   }
