@@ -25,6 +25,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
+from .. import ops
 from ..engine.config import EngineConfig
 from ..parallel import Communicator
 from .experts import DenseFF

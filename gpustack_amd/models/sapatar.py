@@ -23,6 +23,7 @@ from __future__ import annotations
 import torch
 from torch import nn
 
+from .. import ops
 from ..engine.config import EngineConfig
 from ..parallel import Communicator
 from .experts import RoutedFF
