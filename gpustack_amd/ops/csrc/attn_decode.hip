@@ -80,6 +80,10 @@ DEVICE_INLINE int part_tokens(int len, int nsplit) {
   return max((per + STEP - 1) / STEP * STEP, 4 * STEP);
 }
 
+DEVICE_INLINE int window_start(int len, int window) {
+  return window > 0 && len > window ? len - window : 0;
+}
+
 // EXT: sinks / sliding window / softcap (GPT-OSS and Gemma variants).
 template <int D, int GQ, bool FP8, bool EXT>
 __global__ __launch_bounds__(THREADS) void paged_attn_decode_kernel(
@@ -107,11 +111,12 @@ __global__ __launch_bounds__(THREADS) void paged_attn_decode_kernel(
   const int nsplit = gridDim.z;
   const int Hq = Hkv * GQ;
   const int len = seq_lens[seq];
-  const int span = part_tokens(len, nsplit);
   // sliding window (EXT): the query sits at position len - 1 and attends
-  // [max(0, len - window), len)
-  const int wstart = (EXT && window > 0 && len > window) ? len - window : 0;
-  const int t0 = (int)blockIdx.z * span;
+  // [max(0, len - window), len); the parts cut only that
+  const int wstart = EXT ? window_start(len, window) : 0;
+  const int from = wstart / STEP * STEP;
+  const int span = part_tokens(len - from, nsplit);
+  const int t0 = from + (int)blockIdx.z * span;
   const int t1 = min(len, t0 + span);
   if (nsplit > 1 && t0 >= len) return;     // the join skips it as well
 
@@ -149,9 +154,8 @@ __global__ __launch_bounds__(THREADS) void paged_attn_decode_kernel(
   const int* bt = block_tables + (long)seq * max_blocks;
   const int last_page = (len - 1) / BS;
   const float sc = scale * LOG2E;
-  const int first = EXT ? max(t0, wstart / STEP * STEP) : t0;
 
-  for (int c0 = first + wave * STEP; c0 < t1; c0 += NWAVES * STEP) {
+  for (int c0 = t0 + wave * STEP; c0 < t1; c0 += NWAVES * STEP) {
     const int page = c0 / BS;
     long at[2];
 #pragma unroll
@@ -327,12 +331,13 @@ __global__ __launch_bounds__(D) void paged_attn_join_kernel(
     unsigned short* __restrict__ out,       // [N, Hq, D]
     const float* __restrict__ part,         // [N, Hkv, nsplit, GQ, D + 2]
     const int* __restrict__ seq_lens, int GQ, int nsplit,
-    const float* __restrict__ sinks) {
+    const float* __restrict__ sinks, int window) {
   const int seq = blockIdx.x, hq = blockIdx.y, Hq = gridDim.y;
   const int h = hq / GQ, gq = hq % GQ, d = threadIdx.x;
   const int len = seq_lens[seq];
-  const int span = part_tokens(len, nsplit);
-  const int n = min(nsplit, (len + span - 1) / span);
+  const int keys = len - window_start(len, window) / STEP * STEP;
+  const int span = part_tokens(keys, nsplit);
+  const int n = min(nsplit, (keys + span - 1) / span);
   const float* pp = part +
       (((long)seq * (Hq / GQ) + h) * nsplit * GQ + gq) * (D + 2);
   const long step = (long)GQ * (D + 2);
@@ -355,16 +360,21 @@ __global__ __launch_bounds__(D) void paged_attn_join_kernel(
 
 }  // namespace
 
-// Parts per sequence. 256 CUs hold about 1024 of these workgroups at once:
-// below that the keys are cut until there are about 2048 (two rounds even out
-// unequal lengths), of at least 128 keys each — shorter parts save less than
-// their join costs. max_blocks is the width of the block table, so a captured
-// graph keeps its grid; parts behind a sequence's end return at once.
-int decode_splits(int N, int Hkv, int max_blocks) {
-  const long base = (long)N * Hkv;
-  if (base >= 1024) return 1;
-  long n = (2048 + base - 1) / base;
-  const long most = ((long)max_blocks * BS + 4 * STEP - 1) / (4 * STEP);
+// Parts per sequence. 256 CUs hold about 1024 of these workgroups at once, of
+// heads of 256 channels half as many: below that the keys are cut until there
+// are about twice as many (two rounds even out unequal lengths), of at least
+// 128 keys each — shorter parts save less than their join costs (a window of
+// 128 keys, 16 sequences: 22 us in parts of the whole length, 9 in one; 64
+// sequences of 300 keys at 256 channels: 50 cut, 36 whole). max_blocks is the
+// width of the block table, so a captured graph keeps its grid; parts behind a
+// sequence's end return at once.
+int decode_splits(int N, int Hkv, int max_blocks, int D, int window) {
+  const long base = (long)N * Hkv, held = D > 128 ? 512 : 1024;
+  if (base >= held) return 1;
+  long n = (2 * held + base - 1) / base;
+  long keys = (long)max_blocks * BS;
+  if (window > 0 && window < keys) keys = window;
+  const long most = (keys + 4 * STEP - 1) / (4 * STEP);
   if (n > most) n = most;
   return (int)(n < 1 ? 1 : n > 64 ? 64 : n);
 }
@@ -421,7 +431,7 @@ void paged_attn_decode_launch(void* out, const void* q, const void* kc,
 #define JOIN(DD)                                                              \
   hipLaunchKernelGGL((paged_attn_join_kernel<DD>), dim3(N, Hq), dim3(DD), 0,  \
                      s, (unsigned short*)out, part, seq_lens, GQ, nsplit,     \
-                     sinks)
+                     sinks, window)
   if (D == 128) JOIN(128);
   else if (D == 64) JOIN(64);
   else JOIN(256);

@@ -13,7 +13,7 @@ void reshape_and_cache_launch(const void*, const void*, void*, void*, const long
 void greedy_sample_launch(long*, const void*, int, int, hipStream_t);
 void mla_decode_launch(float*, const void*, const void*, const int*, const int*, int, int, int, int, int, int, float, int*, hipStream_t);
 void qkv_store_launch(void*, const void*, const void*, const float*, const long*, const long*, void*, void*, long, int, int, int, int, float, int, int*, hipStream_t);
-int decode_splits(int, int, int);
+int decode_splits(int, int, int, int, int);
 void paged_attn_decode_launch(void*, const void*, const void*, const void*, const int*, const int*, float*, int, int, int, int, int, int, float, long, int, const float*, int, float, int*, hipStream_t);
 void flash_prefill_launch(void*, const void*, const void*, const void*, const int*, const int*, const int*, int, int, int, int, int, float, long, long, long, const float*, int, float, int*, hipStream_t);
 void flash_prefill_paged_launch(void*, const void*, const void*, const void*, const int*, const int*, const int*, const int*, const int*, const int*, int, int, int, int, int, float, long, const float*, int, float, int*, hipStream_t);
@@ -235,7 +235,7 @@ void paged_attn_decode(at::Tensor out, at::Tensor q, at::Tensor k_cache,
   const int max_blocks = block_tables.size(1);
   const float* sink_ptr = sink_ptr_checked(sinks, Hq);
   int err = 0;
-  const int nsplit = decode_splits(N, Hkv, max_blocks);
+  const int nsplit = decode_splits(N, Hkv, max_blocks, D, (int)window);
   // this call's own workspace, from the stream's allocator
   at::Tensor part;
   if (nsplit > 1)

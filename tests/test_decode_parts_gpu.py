@@ -64,3 +64,32 @@ def test_parts_against_double(fp8, Hq, Hkv, lens):
     err = (out.double() - ref).abs()
     assert bool((err <= ref.abs() * 2.0 ** -8 + 1e-4).all()), \
         float((err - ref.abs() * 2.0 ** -8).max())
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("window", [1, 33, 128, 129, 1000])
+def test_parts_of_a_window(monkeypatch, D, window):
+    from gpustack_amd import ops
+
+    monkeypatch.setenv("GPUSTACK_AMD_OSS_KERNELS", "1")
+    lens = [4095, 1, 300, 1001, 1000, 160]
+    g = torch.Generator(device="cuda").manual_seed(window + D)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    nb = (max(lens) + 15) // 16
+    kc, vc = rnd(nb * len(lens), 2, 16, D), rnd(nb * len(lens), 2, 16, D)
+    bt = torch.arange(nb * len(lens), device="cuda").int().view(len(lens), nb)
+    q = rnd(len(lens), 8, D)
+    out = torch.empty_like(q)
+    scale = 1 / math.sqrt(D)
+    ops.paged_attn_decode(out, q, kc, vc, bt,
+                          torch.tensor(lens, dtype=torch.int32,
+                                       device="cuda"), scale, window=window)
+    for i, n in enumerate(lens):
+        j = torch.arange(max(0, n - window), n, device="cuda")
+        k = kc[bt[i, j // 16].long(), :, j % 16].double()
+        v = vc[bt[i, j // 16].long(), :, j % 16].double()
+        p = ((q[i].double() * k.repeat_interleave(4, 1)).sum(-1) * scale)
+        ref = (p.softmax(0)[:, :, None] * v.repeat_interleave(4, 1)).sum(0)
+        err = (out[i].double() - ref).abs()
+        # as above: one rounding to bf16, fp32 before it
+        assert bool((err <= ref.abs() * 2.0 ** -8 + 1e-4).all()), (i, n)
