@@ -382,12 +382,14 @@ def _rows_tile_plan(M: int, N: int, K: int):
     16384x2048 18.9 / 19.0 (18944 columns make 296 tiles, two for some CUs and
     one for most: 31 / 27 at 2560);
     up to 16 rows: 28672x4096 40 / 43 at one and 41 / 53 at 16, 4096x11008
-    17 / 31, 102400x4096 153 / 177, but 16384x4096 at one row 27 / 26."""
+    17 / 31, 22016x4096 32 / 39, 128256x4096 175 / 178, but 16384x4096 at one
+    row 27 / 26."""
     if not 0 < M <= 128 or K % 64 != 0 or N % 8 != 0 or min(N, K) < 1024:
         return None
     t64, t128 = -(-N // 64), -(-N // 128)
     if N > 10240:
-        if 256 < t64 < 400:
+        wide = 160 <= t128 <= 256 or t128 >= 500 or M > 64 and t128 > 256
+        if 256 < t64 < 400 and not wide:
             return None
         if M <= 16:
             wins = (N <= 32768 and K >= 2560 and (
@@ -397,7 +399,6 @@ def _rows_tile_plan(M: int, N: int, K: int):
             wins = K % 2048 == 0 and (K <= 8192 or N <= 32768)
         else:
             wins = K == 4096 and N >= 22016 or K == 2048 and N >= 51200
-        wide = 160 <= t128 <= 256 or t128 >= 500 or M > 64 and t128 > 256
         plan = (128 if wide else 64), 1
     elif K <= 2048:
         wins = 16 < M <= 64 and (K == 1024 and N >= 2560
