@@ -644,7 +644,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rows_tile_parts", &rows_tile_parts,
         "fp32 parts over k of a product of up to 128 rows");
   m.def("rows_tile", &rows_tile, "bf16 product of up to 128 rows in tiles");
-  m.def("rows_gemm", &rows_gemm, "bf16 product of up to 64 rows");
+  m.def("rows_gemm", &rows_gemm, "bf16 product of up to 16 rows");
   m.def("moe_route", &moe_route, "router product and choice");
   m.def("moe_topk", &moe_topk, "softmax routing, top k");
   m.def("moe_sort", &moe_sort, "assignments by expert, and the tile list");

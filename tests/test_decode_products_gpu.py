@@ -23,7 +23,7 @@ def _close(out, ref, size):
     assert bool((err <= bound).all()), float((err - bound).max())
 
 
-@pytest.mark.parametrize("M", [1, 15, 16, 17, 33, 64])
+@pytest.mark.parametrize("M", [1, 15, 16])
 @pytest.mark.parametrize("N,K", [(16, 128), (100, 1152), (4096, 1024),
                                  (16400, 256)])
 def test_rows_gemm(M, N, K):
