@@ -242,7 +242,18 @@ __global__ __launch_bounds__(THREADS) void paged_attn_decode_kernel(
         for (int j = 0; j < DV; ++j) acc[gq][j] *= c;
       }
     }
-    // values: lane = channels sub*DV .., keys (i/4)*16 + (i%4)*4 + g
+    // values: lane = channels sub*DV .., keys (i/4)*16 + (i%4)*4 + g. Rows that
+    // are not the sequence's (behind its end in its last page, in front of its
+    // window) may hold anything, and a weight of 0 does not undo a NaN
+    if (c0 + STEP > t1 || (EXT && c0 < wstart)) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int tok = c0 + (i / 4) * 16 + (i & 3) * 4 + g;
+        if (tok >= t1 || (EXT && tok < wstart))
+#pragma unroll
+          for (int w = 0; w < VW; ++w) vw[i][w] = 0;
+      }
+    }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       float pr[GQ], vf[DV];

@@ -49,6 +49,13 @@ def test_parts_against_double(fp8, Hq, Hkv, lens):
     for i, n in enumerate(need):
         bt[i, :n] = pages[at:at + n]
         at += n
+    # what lies behind a sequence's end in its last page is not its own
+    for i, n in enumerate(lens):
+        if n % 16:
+            for pool in (kc, vc):
+                (pool.view(torch.uint8) if fp8 else pool)[
+                    bt[i, need[i] - 1].long(), :, n % 16:] = \
+                    0x7f if fp8 else float("nan")
     q = rnd(len(lens), Hq, 128).bfloat16()
     out = torch.empty_like(q)
     scale = 1 / math.sqrt(128)
@@ -78,6 +85,12 @@ def test_parts_of_a_window(monkeypatch, D, window):
     nb = (max(lens) + 15) // 16
     kc, vc = rnd(nb * len(lens), 2, 16, D), rnd(nb * len(lens), 2, 16, D)
     bt = torch.arange(nb * len(lens), device="cuda").int().view(len(lens), nb)
+    # nothing outside the window counts: behind the end, in front of the first
+    for i, n in enumerate(lens):
+        j = torch.arange(nb * 16, device="cuda")
+        j = j[(j >= n) | (j < n - window)]
+        for pool in (kc, vc):
+            pool[bt[i, j // 16].long(), :, j % 16] = float("nan")
     q = rnd(len(lens), 8, D)
     out = torch.empty_like(q)
     scale = 1 / math.sqrt(D)
