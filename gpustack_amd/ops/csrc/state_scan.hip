@@ -205,6 +205,7 @@ __global__ __launch_bounds__(256) void state_scan_vec_kernel(
 
   u16x8 kreg[KV], qreg[KV], vreg[VV];
   float dreg = 0.f;
+  float odd = 0.f;                           // NaN behind a value that is not finite
   auto fetch = [&](int c0) {
     const int rows = min(CH, n - c0);
 #pragma unroll
@@ -379,12 +380,15 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
   const float dtb = dt_src != nullptr ? p.dt_bias[h] : 0.f;
   const float a_const = dt_src == nullptr ? p.decay[h] : 0.f;
   const bool neg = a_const < 0.f;            // (-1)^(t - s) beside |a|^(t - s)
-  // far enough down that e^it is 0 in fp32, and still exact in the sums
-  const float log_const = fmaxf(logf(fabsf(a_const)), -1e4f);
+  // far enough down that e^it is 0 in fp32, and still exact in the sums; a
+  // NaN stays one
+  auto low = [](float v) { return v < -1e4f ? -1e4f : v; };
+  const float log_const = low(logf(fabsf(a_const)));
   const u16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
 
   u16x8 kreg[KU], qreg[KU], vreg;
   float dreg = 0.f;
+  float odd = 0.f;                           // NaN behind a value that is not finite
   auto fetch = [&](int c0) {
     const int rows = min(C, n - c0);
 #pragma unroll
@@ -435,7 +439,7 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
       if (tid < rows) {
         if (dt_src != nullptr) {
           b = softplus_f(dreg + dtb);
-          la = fmaxf(-a_rate * b, -1e4f);
+          la = low(-a_rate * b);
         } else {
           b = 1.f;
           la = log_const;
@@ -511,6 +515,10 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
 #pragma unroll
       for (int j = 0; j < 4; ++j) vv[b][j] = vs[b * 16 + g * 4 + j][wave * 16 + lc];
 #pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) odd += vv[b][j] * 0.f;
+#pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int b = 0; b <= t; ++b) {
@@ -546,6 +554,38 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
           S[t] = mm(ks[sr][t * 16 + lc], bv, S[t]);
       }
     __syncthreads();
+  }
+  // A value that is infinite or NaN belongs to its own row and those behind
+  // it, but the weights of 0 above the diagonal carried it to the rows in
+  // front: such columns are walked again row by row, on the state in memory.
+  if (__any(odd != 0.f)) {
+    auto load = [&](const unsigned short* at) {
+      const float f = bf2f(*at);
+      return p.act ? silu_f(f) : f;
+    };
+#pragma unroll 1
+    for (int i = 0; i < n; ++i) {
+      const unsigned short* rp = src + (long)(first + i) * p.ld_src;
+      float a = a_const, b = 1.f, part = 0.f;
+      if (dt_src != nullptr) {
+        b = softplus_f(bf2f(dt_src[(long)(first + i) * p.ld_dt + p.col_dt + h])
+                       + dtb);
+        a = expf(-a_rate * b);
+      }
+      const float v = live ? load(rp + p.col_x + h * P + pc) : 0.f;
+#pragma unroll 1
+      for (int nn = g; nn < N && live; nn += 4) {
+        float* at = sp + (long)nn * P + pc;
+        const float old = i > 0 || hist > 0 ? *at : 0.f;
+        *at = a * old + b * load(rp + p.col_b + grp * N + nn) * v;
+        part += *at * load(rp + p.col_c + grp * N + nn);
+      }
+      part += __shfl_xor(part, 16, 64);
+      part += __shfl_xor(part, 32, 64);
+      if (g == 0 && live)
+        y[(long)(first + i) * p.H * P + h * P + pc] = part + skip * v;
+    }
+    return;
   }
 #pragma unroll
   for (int t = 0; t < NT; ++t)

@@ -77,3 +77,35 @@ def test_chunks(kind, H, G, N, P, news):
         scale = float(ref.abs().max())
         assert float((got.double() - ref).abs().max()) <= 4e-6 * scale
     assert torch.equal(st[6], state[6])
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("at", [5, 20, 47])
+def test_not_finite(bad, at):
+    """A value reaches its own row and the rows behind it, of its channel."""
+    from gpustack_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(at)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    T, H, N, P = 70, 2, 64, 96
+    src = rnd(T, H * (P + 2 * N)).bfloat16()
+    src[at, P + 70] = bad                      # head 1, channel 70
+    decay = torch.tensor([0.9, -0.97], device="cuda")
+    state = torch.zeros(2, H, N, P, device="cuda")
+    cb, cc = H * P, H * (P + N)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    y = torch.zeros(T, H * P, device="cuda")
+    ops.state_scan(y, src, 0, cb, cc, None, 0, H, H, N, P, False, None, None,
+                   None, decay, state, i32([0]), i32([T]), i32([0]),
+                   i32(list(range(T))))
+    a = decay.double().expand(T, H)
+    ref, ref_s = _walk(src, 0, cb, cc, H, H, N, P, False, a,
+                       torch.ones_like(a), None,
+                       torch.zeros(2, H, N, P, device="cuda"), [T], [0], [0])
+    for got, want in ((y, ref), (state, ref_s)):
+        ok = want.isfinite()
+        assert torch.equal(got.isfinite(), ok)
+        scale = float(want[ok].abs().max())    # fp32 sums, as above
+        assert float((got[ok].double() - want[ok]).abs().max()) <= 4e-6 * scale
+    assert bool(ref[:at].isfinite().all()) and not bool(
+        ref[at:, P + 70].isfinite().any())
