@@ -9,11 +9,13 @@ engine/control-plane logic testable without hardware.
 from __future__ import annotations
 
 import os
+from pathlib import Path
 
 import torch
 
 from . import torch_ref
 
+_HIP_SO = Path(__file__).resolve().parent / "_hip_ops.so"
 _HIP = None
 _HIP_ERR: str | None = None
 
@@ -24,9 +26,8 @@ def _load_hip():
         return _HIP
     try:
         import importlib.util
-        from pathlib import Path
 
-        so = Path(__file__).resolve().parent / "_hip_ops.so"
+        so = _HIP_SO
         if not so.exists():
             raise ImportError(
                 f"{so} not found — build it with `python -m gpustack_amd.ops.build` "
@@ -49,6 +50,14 @@ def hip_available() -> bool:
         return _load_hip() is not None
     except Exception:  # noqa: BLE001
         return False
+
+
+def _products():
+    """The main library, or None in a checkout without it: the models that
+    come with libraries of their own run there on the library's products."""
+    if _HIP is None and not _HIP_SO.exists():
+        return None
+    return _load_hip()
 
 
 def _backend(t: torch.Tensor):
@@ -458,6 +467,7 @@ def linear_auto(x, w):
         N = w.shape[0]
         plan = _rows_tile_plan(M, N, K)
         if ((plan or _rows_gemm_wins(M, N, K)) and M > 0
+                and _products() is not None
                 and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
                 and w.is_contiguous() and w.data_ptr() % 16 == 0
                 and x.stride(1) == 1 and x.stride(0) % 8 == 0
@@ -470,7 +480,7 @@ def linear_auto(x, w):
                 _load_hip().rows_gemm(out, x, w)
             return out
         if (N == 4096 and K >= 8192 and 384 <= M <= 1024
-                and K % 256 == 0
+                and K % 256 == 0 and _products() is not None
                 and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
                 and x.is_contiguous() and w.is_contiguous()):
             return skinny_gemm(x, w, splitk=4)

@@ -98,3 +98,25 @@ def test_argmax_of_a_row(V):
     for t in (x.bfloat16(), x):
         ref = torch.stack([(r == r.max()).nonzero()[0, 0] for r in t.float()])
         assert torch.equal(ops.greedy_sample(t), ref)
+
+
+@pytest.mark.parametrize("M,N,K", [(4, 4096, 2048), (48, 4096, 4096),
+                                   (512, 4096, 8192), (300, 256, 256)])
+def test_products_without_the_main_library(monkeypatch, M, N, K):
+    """A checkout that has built only the libraries of one model."""
+    from pathlib import Path
+
+    from gpustack_amd import ops
+
+    exists = Path.exists
+    monkeypatch.setattr(Path, "exists", lambda p: exists(p)
+                        and p.name != "_hip_ops.so")
+    monkeypatch.setattr(ops, "_HIP", None)
+    monkeypatch.setattr(ops, "_HIP_ERR", None)
+    x = torch.randn(M, K, device="cuda").bfloat16()
+    w = torch.randn(N, K, device="cuda").bfloat16()
+    for _ in range(2):
+        assert torch.equal(ops.linear_auto(x, w),
+                           torch.nn.functional.linear(x, w))
+    with pytest.raises(ImportError):
+        ops._load_hip()
