@@ -767,9 +767,9 @@ class MoEMLP(nn.Module):
         T = x.shape[0]
         fused = self._fused_ok(x)
         # softmax routing in one launch (a top-k, a sort and a softmax
-        # otherwise)
+        # otherwise): 16 logits a lane, and a lane for each chosen expert
         soft = fused and self.spec.router_mode != "sigmoid_bias" \
-            and self.e <= 1024
+            and self.e <= 1024 and self.top_k <= 64
         bias = self.router_bias if self.spec.router_logit_bias else None
         if soft:
             hip = ops._load_hip()

@@ -152,3 +152,45 @@ def test_route(T, E, H, k, renorm):
     # a logit off by eps moves a weight by 2 eps of itself; fp32 exp and sum
     assert bool(((weights.double() - want).abs()
                  <= want * (4 * eps + 2.0 ** -18) + 2.0 ** -30).all())
+
+
+def _moe(E, k, H, I, seed=0):
+    import dataclasses
+
+    from gpustack_amd.engine import EngineConfig
+    from gpustack_amd.models.llama import MoEMLP
+    from gpustack_amd.parallel import Communicator
+
+    spec = dataclasses.replace(
+        EngineConfig(model="qwen3-30b-a3b", device="cpu").spec,
+        num_experts=E, num_experts_per_tok=k, hidden_size=H,
+        moe_intermediate_size=I)
+    m = MoEMLP(spec, 1, Communicator(), torch.bfloat16).cuda()
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    for p in m.parameters():
+        p.data.copy_(torch.randn(p.shape, generator=g, device="cuda")
+                     * p.shape[-1] ** -0.5)
+    return m, g
+
+
+def _moe_reference(m, x):
+    """The layer in float64: routing, experts, weighted sum."""
+    x = x.double()
+    top, ex = torch.topk(x @ m.router_w.double().T, m.top_k, -1)
+    top = top.softmax(-1)
+    out = torch.zeros_like(x)
+    for e in range(m.e):
+        t, j = (ex == e).nonzero(as_tuple=True)
+        gu = x[t] @ m.gate_up_w[e].double().T
+        h = torch.nn.functional.silu(gu[:, :m.i]) * gu[:, m.i:]
+        out.index_add_(0, t, (h @ m.down_w[e].double().T) * top[t, j, None])
+    return out
+
+
+@pytest.mark.parametrize("k", [64, 65, 128])
+def test_more_experts_a_row_than_lanes(k):
+    m, g = _moe(128, k, 256, 128)
+    x = torch.randn(9, 256, generator=g, device="cuda").bfloat16()
+    ref = _moe_reference(m, x)
+    # bf16 activations and contributions: 2^-8 of each, of about equal size
+    assert float((m(x).double() - ref).norm() / ref.norm()) < 2.0 ** -7
