@@ -348,6 +348,7 @@ DEVICE_INLINE void moe_topk_row(int* experts, float* weights,
                                 int renorm, int parts = 1, long stride = 0) {
   float v[NV];
   unsigned taken = 0;
+  bool nan = false;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int e = i * 64 + lane;
@@ -355,7 +356,9 @@ DEVICE_INLINE void moe_topk_row(int* experts, float* weights,
     for (int p = 1; p < parts; ++p)
       if (e < E) v[i] += logits[p * stride + e];
     if (e >= E) taken |= 1u << i;
+    nan |= v[i] != v[i];
   }
+  const bool lost = __any(nan);        // one NaN is in every weight's sum
   float top = 0.f, mine = 0.f, sum = 0.f;
   for (int j = 0; j < k; ++j) {
     float best = -INFINITY;
@@ -389,7 +392,7 @@ DEVICE_INLINE void moe_topk_row(int* experts, float* weights,
     for (int i = 0; i < NV; ++i) all += __expf(v[i] - top);
     sum = wave_reduce_sum(all);
   }
-  if (lane < k) weights[lane] = mine / sum;
+  if (lane < k) weights[lane] = lost ? NAN : mine / sum;
 }
 
 template <int NV>

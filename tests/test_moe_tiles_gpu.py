@@ -104,6 +104,26 @@ def test_softmax_routing(renorm, T, E, k):
     torch.testing.assert_close(w.double(), ref, rtol=1e-5, atol=1e-7)
 
 
+@pytest.mark.parametrize("renorm", [False, True])
+@pytest.mark.parametrize("E,k", [(8, 2), (100, 4), (1000, 32)])
+def test_routing_of_logits_that_are_not_finite(renorm, E, k):
+    """As top-k and softmax have it: a row with a NaN or infinite logit has no
+    weights, one of minus infinity none for that expert; experts in range."""
+    inf, nan = float("inf"), float("nan")
+    logits = torch.randn(7, E, device="cuda")
+    logits[0, 3], logits[1, E - 1], logits[2, 5] = nan, inf, -inf
+    logits[3], logits[4], logits[5, 1:] = nan, -inf, -inf
+    ex = torch.full((7, k), -1, dtype=torch.int32, device="cuda")
+    w = torch.zeros(7, k, device="cuda")
+    _hip().moe_topk(ex, w, logits, renorm)
+    if renorm:
+        ref = torch.topk(logits, k, -1).values.softmax(-1)
+    else:
+        ref = torch.topk(logits.softmax(-1), k, -1).values
+    assert bool(((ex >= 0) & (ex < E)).all())
+    torch.testing.assert_close(w, ref, rtol=1e-5, atol=1e-7, equal_nan=True)
+
+
 @pytest.mark.parametrize("TK,E", [(65536, 4096), (4096, 128), (4097, 128),
                                   (32544, 128), (8192, 1025), (5000, 1)])
 def test_sort_of_a_long_list(TK, E):
