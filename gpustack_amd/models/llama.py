@@ -177,7 +177,9 @@ def qlinear(x, w, pack: "W4Pack | None", bias=None):
         hip = ops._load_hip()
         most = 1024 if _os.environ.get("GPUSTACK_AMD_W4_KERNEL", "0") == "1" \
             else 64
-        if 0 < x.shape[0] <= most and x.dim() == 2 and pack.shape[1] <= 131072:
+        # whole workgroups of 64 columns, scales that fit the LDS
+        if 0 < x.shape[0] <= most and x.dim() == 2 \
+                and pack.shape[0] % 64 == 0 and pack.shape[1] <= 131072:
             out = torch.empty(x.shape[0], pack.shape[0], dtype=x.dtype,
                               device=x.device)
             hip.w4_gemm(out, x.contiguous(), pack.qw, pack.sc, pack.zs)

@@ -120,3 +120,22 @@ def test_products_without_the_main_library(monkeypatch, M, N, K):
                            torch.nn.functional.linear(x, w))
     with pytest.raises(ImportError):
         ops._load_hip()
+
+
+@pytest.mark.parametrize("N,K", [(96, 256), (8, 128), (64, 256)])
+def test_packed_weights_of_any_column_count(N, K):
+    from gpustack_amd.models.llama import W4Pack, qlinear
+    from gpustack_amd.models.quantized import (dequant_w4_runtime,
+                                               pack_w4_runtime)
+
+    g = torch.Generator(device="cuda").manual_seed(N)
+    pack = W4Pack(*pack_w4_runtime(
+        torch.randint(0, 16, (N, K), generator=g, device="cuda"),
+        torch.rand(N, K // 128, generator=g, device="cuda") * 0.05 + 0.01,
+        torch.full((N, K // 128), 8.0, device="cuda"), 128))
+    x = torch.randn(5, K, generator=g, device="cuda").bfloat16()
+    w = dequant_w4_runtime(pack.qw, pack.sc, pack.zs).double()
+    size = x.double().abs() @ w.abs().T
+    # the expansion rounds a weight to bf16 (2^-9 of it), the result once more
+    err = (qlinear(x, None, pack).double() - x.double() @ w.T).abs()
+    assert bool((err <= size * 2.0 ** -7).all())
