@@ -935,6 +935,8 @@ class MoEMLP(nn.Module):
         T, k = experts.shape
         TK = T * k
         hip = ops._load_hip()
+        if x.data_ptr() % 16:          # the tiles' loads to the LDS
+            x = x.clone()
         flat = experts.reshape(-1).to(torch.int32)
         flat_w = weights.reshape(-1).float()
         order, s_tok, counts, offs, tiles, ntiles = hip.moe_sort(

@@ -214,3 +214,14 @@ def test_more_experts_a_row_than_lanes(k):
     ref = _moe_reference(m, x)
     # bf16 activations and contributions: 2^-8 of each, of about equal size
     assert float((m(x).double() - ref).norm() / ref.norm()) < 2.0 ** -7
+
+
+@pytest.mark.parametrize("T", [3, 130])
+def test_rows_at_any_address(T):
+    m, g = _moe(4, 2, 256, 128)
+    flat = torch.randn(T * 256 + 1, generator=g, device="cuda").bfloat16()
+    x = flat[1:].view(T, 256)
+    assert x.data_ptr() % 16
+    ref = _moe_reference(m, x)
+    # as above
+    assert float((m(x).double() - ref).norm() / ref.norm()) < 2.0 ** -7
