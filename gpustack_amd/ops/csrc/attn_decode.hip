@@ -7,7 +7,7 @@
 //  - a workgroup owns (sequence, kv head, part of the keys); the GQ = Hq/Hkv
 //    query heads of a kv head share its K/V stream, so each KV byte is read
 //    exactly once per step. The keys of a sequence are cut into parts when
-//    (sequences x kv heads) alone leaves CUs without work (decode_splits);
+//    (sequences x kv heads) alone leaves CUs without work (decode_parts);
 //    a second kernel joins the parts.
 //  - 4 waves per workgroup, 32 keys (two pages) per wave and step. Scores are
 //    a matrix product, S^T = K Q^T on mfma_f32_16x16x32_bf16: K rows are the
@@ -22,12 +22,16 @@
 //
 // Bound by the K/V stream: 32 keys cost a SIMD about 1300 cycles (GQ = 4),
 // 31 TB/s over the chip in bf16 and 15 TB/s in fp8, so memory sets the time
-// once enough of it is in flight (16 KB a wave, 16 waves a CU).
+// once enough of it is in flight (16 KB a wave in bf16 at 128 channels;
+// registers allow 3 waves a SIMD there with 4 to 8 heads, 4 in fp8 with 4 or
+// at 64 channels, 2 at 256).
 //
 // KV pool layout: [num_blocks, Hkv, BS, D] bf16 | fp8, BS = 16 tokens.
 #include "common.h"
 
 #include <type_traits>
+
+struct DecodeParts { int n, least; };   // of a sequence, and a part's keys
 
 namespace {
 
@@ -74,10 +78,10 @@ DEVICE_INLINE unsigned int pack_hi(float lo, float hi) {
                                0x07060302u);
 }
 
-// keys per part of a sequence of `len` tokens: whole steps, at least 128
-DEVICE_INLINE int part_tokens(int len, int nsplit) {
+// keys per part of a sequence of `len` tokens: whole steps, at least `least`
+DEVICE_INLINE int part_tokens(int len, int nsplit, int least) {
   const int per = (len + nsplit - 1) / nsplit;
-  return max((per + STEP - 1) / STEP * STEP, 4 * STEP);
+  return max((per + STEP - 1) / STEP * STEP, least);
 }
 
 DEVICE_INLINE int window_start(int len, int window) {
@@ -94,6 +98,7 @@ __global__ __launch_bounds__(THREADS) void paged_attn_decode_kernel(
     const int* __restrict__ block_tables,    // [N, max_blocks]
     const int* __restrict__ seq_lens,        // [N]
     float* __restrict__ part,                // [N, Hkv, nsplit, GQ, D + 2]
+    int least,                               // keys of a part (part_tokens)
     int Hkv, int max_blocks, float scale, long q_stride,
     const float* __restrict__ sinks,         // [Hq] or null (GPT-OSS)
     int window,                              // 0 = full attention
@@ -115,7 +120,7 @@ __global__ __launch_bounds__(THREADS) void paged_attn_decode_kernel(
   // [max(0, len - window), len); the parts cut only that
   const int wstart = EXT ? window_start(len, window) : 0;
   const int from = wstart / STEP * STEP;
-  const int span = part_tokens(len - from, nsplit);
+  const int span = part_tokens(len - from, nsplit, least);
   const int t0 = from + (int)blockIdx.z * span;
   const int t1 = min(len, t0 + span);
   if (nsplit > 1 && t0 >= len) return;     // the join skips it as well
@@ -341,13 +346,13 @@ template <int D>
 __global__ __launch_bounds__(D) void paged_attn_join_kernel(
     unsigned short* __restrict__ out,       // [N, Hq, D]
     const float* __restrict__ part,         // [N, Hkv, nsplit, GQ, D + 2]
-    const int* __restrict__ seq_lens, int GQ, int nsplit,
+    const int* __restrict__ seq_lens, int GQ, int nsplit, int least,
     const float* __restrict__ sinks, int window) {
   const int seq = blockIdx.x, hq = blockIdx.y, Hq = gridDim.y;
   const int h = hq / GQ, gq = hq % GQ, d = threadIdx.x;
   const int len = seq_lens[seq];
   const int keys = len - window_start(len, window) / STEP * STEP;
-  const int span = part_tokens(keys, nsplit);
+  const int span = part_tokens(keys, nsplit, least);
   const int n = min(nsplit, (keys + span - 1) / span);
   const float* pp = part +
       (((long)seq * (Hq / GQ) + h) * nsplit * GQ + gq) * (D + 2);
@@ -371,33 +376,54 @@ __global__ __launch_bounds__(D) void paged_attn_join_kernel(
 
 }  // namespace
 
-// Parts per sequence. 256 CUs hold about 1024 of these workgroups at once, of
-// heads of 256 channels half as many: below that the keys are cut until there
-// are about twice as many (two rounds even out unequal lengths), of at least
-// 128 keys each — shorter parts save less than their join costs (a window of
-// 128 keys, 16 sequences: 22 us in parts of the whole length, 9 in one; 64
-// sequences of 300 keys at 256 channels: 50 cut, 36 whole). max_blocks is the
-// width of the block table, so a captured graph keeps its grid; parts behind a
-// sequence's end return at once.
-int decode_splits(int N, int Hkv, int max_blocks, int D, int window) {
-  const long base = (long)N * Hkv, held = D > 128 ? 512 : 1024;
-  if (base >= held) return 1;
-  long n = (2 * held + base - 1) / base;
+// Parts per sequence, and the fewest keys of one: parts fill the chip when
+// sequences x kv heads (`base`) do not, and even out unequal lengths, but each
+// writes its sums to memory and the join is a launch. max_blocks is the width
+// of the block table, so a captured graph keeps its grid; parts behind a
+// sequence's end return at once. Measured with 1 to 64 parts, us, 32 heads on
+// 8 of 128 channels in bf16 unless said (parts chosen: time / others):
+//   one sequence, 4000 keys   16: 18.5 / 8: 17.8, 64: 38.8, 1: 51
+//   8, 200 to 8000            8: 38 / 4: 37, 32: 51, 1: 95
+//   16, 1000 to 8000          4: 62 / 1: 132, 16: 75
+//   32, 1000 to 8000          2: 125 / 1: 153, 8: 135; all of 300: 1: 12.7 / 2: 15.3
+//   48, 3500 to 7900          2: 218 / 1: 234, 6: 223
+//   64, 100 to 4000           1: 119 / 2: 136, 4: 131; all of 300: 1: 18 / 4: 29
+// Rows of 128 bytes (fp8, or 64 channels) spend relatively more on scores, so
+// they are cut for twice as many workgroups:
+//   fp8: 64, 100 to 4000      2: 84 / 1: 89; 32, 1000 to 8000 4: 83 / 1: 117, 2: 91
+//        96, 100 to 4000      1: 108 / 2: 123
+// So are heads of 256 channels, of which few workgroups fit at once, but not
+// into more than 8 parts (16 heads on 8):
+//        48, 3500 to 7900     3: 434 / 1: 480, 2: 438; 24, 200 to 2000 6: 45 / 1: 52
+//        64, 100 to 4000      1: 238 / 4: 233, 8: 249
+// A context of less than one part pays for the join's launch behind a wide
+// block table (one sequence of 100 keys, 8 heads on 8: 6.8 against 5.0).
+DecodeParts decode_parts(int N, int Hkv, int max_blocks, int D, int fp8,
+                         int window) {
+  const long base = (long)N * Hkv;
+  if (base < 1) return {1, 4 * STEP};
+  const bool narrow = D * (fp8 ? 1 : 2) <= 128;
+  long n = narrow    ? 1024 / base
+           : base >= 512 ? 1
+           : D > 128     ? (1024 + base - 1) / base
+                         : (512 + base - 1) / base;
+  const int least = base >= 256 ? 512 : base >= 128 ? 256 : 128;
   long keys = (long)max_blocks * BS;
   if (window > 0 && window < keys) keys = window;
-  const long most = (keys + 4 * STEP - 1) / (4 * STEP);
+  const long most = base >= 128 ? keys / least : (keys + least - 1) / least;
   if (n > most) n = most;
-  return (int)(n < 1 ? 1 : n > 64 ? 64 : n);
+  const long cap = D > 128 ? 8 : 16;
+  return {(int)(n < 1 ? 1 : n > cap ? cap : n), least};
 }
 
 void paged_attn_decode_launch(void* out, const void* q, const void* kc,
                               const void* vc, const int* block_tables,
-                              const int* seq_lens, float* part, int nsplit,
+                              const int* seq_lens, float* part, DecodeParts parts,
                               int N, int Hq, int Hkv, int D, int max_blocks,
                               float scale, long q_stride, int fp8,
                               const float* sinks, int window, float softcap,
                               int* err_unsupported, hipStream_t s) {
-  const int GQ = Hq / Hkv;
+  const int GQ = Hq / Hkv, nsplit = parts.n;
   dim3 grid(N, Hkv, nsplit);
   dim3 block(THREADS);
   *err_unsupported = 0;
@@ -407,8 +433,8 @@ void paged_attn_decode_launch(void* out, const void* q, const void* kc,
 #define LAUNCH_D(DD, G, F, E)                                                  \
   hipLaunchKernelGGL((paged_attn_decode_kernel<DD, G, F, E>), grid, block, 0,  \
                      s, (unsigned short*)out, (const unsigned short*)q, kc,    \
-                     vc, block_tables, seq_lens, part, Hkv, max_blocks, scale, \
-                     q_stride, sinks, window, softcap)
+                     vc, block_tables, seq_lens, part, parts.least, Hkv,       \
+                     max_blocks, scale, q_stride, sinks, window, softcap)
 #define LAUNCH_GQ2(G, F)                                                       \
   do {                                                                         \
     if (D == 128) {                                                            \
@@ -442,7 +468,7 @@ void paged_attn_decode_launch(void* out, const void* q, const void* kc,
 #define JOIN(DD)                                                              \
   hipLaunchKernelGGL((paged_attn_join_kernel<DD>), dim3(N, Hq), dim3(DD), 0,  \
                      s, (unsigned short*)out, part, seq_lens, GQ, nsplit,     \
-                     sinks, window)
+                     parts.least, sinks, window)
   if (D == 128) JOIN(128);
   else if (D == 64) JOIN(64);
   else JOIN(256);

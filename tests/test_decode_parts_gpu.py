@@ -30,7 +30,8 @@ def _reference(q, kc, vc, bt, lens, scale):
                                     (28, 4), (32, 4)])
 @pytest.mark.parametrize("lens", [
     [1], [31, 32, 33], [127, 128, 129], [4095, 1, 300], [2049],
-    [1 + 7 * i for i in range(300)]])
+    [1 + 7 * i for i in range(300)], [1 + 61 * i for i in range(70)],
+    [900 - 43 * i for i in range(20)]])
 def test_parts_against_double(fp8, Hq, Hkv, lens):
     from gpustack_amd import ops
 
