@@ -807,10 +807,10 @@ class MoEMLP(nn.Module):
                              bool(self.spec.norm_topk_prob))
             else:
                 weights, experts = self._route(logits)
-        if fused:
+        if fused and not self._library_wins(T):
             out = self._fused_dispatch(x, experts, weights)
             return self.comm.all_reduce(self._add_shared(x, out))
-        flat_exp = experts.reshape(-1)                            # [T*k]
+        flat_exp = experts.reshape(-1).long()                     # [T*k]
         flat_tok = torch.arange(T, device=x.device) \
             .repeat_interleave(self.top_k)
         flat_w32 = weights.reshape(-1)                            # f32
@@ -821,7 +821,8 @@ class MoEMLP(nn.Module):
         # router on near-ties (observed on HW).
         # Aligned sizes on the GPU run the grouped expert kernels above
         # (ops/csrc/moe_gemm.hip; no host sync, capturable); what is left
-        # here is the per-expert loop, and the padded batched product.
+        # here is the per-expert loop, also for long prompts of few large
+        # experts (_library_wins), and the padded batched product.
         flat_w = flat_w32.to(x.dtype)
         contrib = x.new_zeros(T * self.top_k, x.shape[1])
         # prefill-shaped on GPU with many experts: padded-bmm. The r2
@@ -926,6 +927,21 @@ class MoEMLP(nn.Module):
                 and act_ok
                 and self.i % 128 == 0 and x.shape[1] % 128 == 0
                 and self.e <= 4096 and ops.hip_available())
+
+    def _library_wins(self, T: int) -> bool:
+        """Long prompts of few large experts: the library's product of one
+        expert at a time (1100 to 1300 TFLOP/s) makes up for a loop that syncs
+        with the host and gathers the rows (about 130 us an expert) against
+        the tiles' 830. us of the layer, tiles against loop, at 4096 x 14336
+        and two experts a row: 8 experts 4096 rows 3630 / 3900, 6144 rows
+        5320 / 5160, 8192 rows 6980 / 6200, 16384 rows 14900 / 11700; 16
+        experts 12288 rows 10570 / 11070, 16384 rows 13860 / 12100; 8 of
+        4096 x 7168 12288 rows 5280 / 5460, 16384 rows 7160 / 5930. The line
+        is one number of multiplications an expert in all of them. A capture
+        cannot record the syncs."""
+        return (T * self.top_k * self.i * self.spec.hidden_size
+                >= 100_000_000_000 * self.e
+                and not torch.cuda.is_current_stream_capturing())
 
     def _fused_dispatch(self, x, experts, weights):
         """Sync-free grouped expert products: sort the assignments by expert

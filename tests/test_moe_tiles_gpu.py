@@ -225,3 +225,24 @@ def test_rows_at_any_address(T):
     ref = _moe_reference(m, x)
     # as above
     assert float((m(x).double() - ref).norm() / ref.norm()) < 2.0 ** -7
+
+
+@pytest.mark.parametrize("T,loop", [(12000, True), (11900, False)])
+def test_long_prompts_of_few_large_experts(monkeypatch, T, loop):
+    """Both sides of the line between the tiles and the library's loop."""
+    m, g = _moe(4, 2, 2048, 8192)
+    x = torch.randn(T, 2048, generator=g, device="cuda").bfloat16()
+    taken = []
+    for name in ("_fused_dispatch", "_loop_dispatch"):
+        real = getattr(m, name)
+        monkeypatch.setattr(m, name, lambda *a, r=real, n=name:
+                            (taken.append(n), r(*a))[1])
+    out = m(x)
+    assert taken == ["_loop_dispatch" if loop else "_fused_dispatch"]
+    part = torch.cat([torch.arange(64), torch.arange(T - 64, T)]).cuda()
+    ref = _moe_reference(m, x[part])
+    # as above, with one more rounding of the activation's operands
+    assert float((out[part].double() - ref).norm() / ref.norm()) < 2.0 ** -6
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing",
+                        lambda: True)
+    assert not m._library_wins(T)
