@@ -965,11 +965,16 @@ class MoEMLP(nn.Module):
         hip.moe_tile(False, act, x, self._bank("gate_up"), s_tok, tiles,
                      ntiles, offs, counts, bias=self.gate_up_b,
                      act_mode=act_mode)
-        # few workgroups of long rows: twice as many of 64 columns (8 experts
-        # of 4096 x 14336, us: 1 row 90 against 191, 8 rows 170 against 215,
-        # 64 rows 350 against 231; 128 of 2048 x 768: 64 rows 83 against 76)
-        if TK <= 16 * self.e and self.i > 2048 \
-                and min(TK, self.e) * (x.shape[1] // 128) < 512:
+        # Up to one workgroup a CU of long rows: twice as many of 64 columns,
+        # which read the weights again for every 16 rows of an expert. us,
+        # 64 columns against tiles, by assignments: 8 experts of 4096 x 14336
+        # 2: 90 / 192, 16: 179 / 230, 64: 195 / 231, 96: 276 / 231, 128:
+        # 315 / 231; 16 of 4096 x 6400 8: 99 / 103, 12: 129 / 110, 64:
+        # 146 / 134; 8 of 6144 x 16384 4: 114 / 225, 8: 228 / 240, 24:
+        # 320 / 290; 8 of 4096 x 3584 32: 47 / 58; but 64 of 2048 x 2816
+        # 8: 36 / 29, 16: 55 / 49
+        if TK <= 8 * self.e and self.i > 3072 \
+                and min(TK, self.e) * (x.shape[1] // 128) <= 256:
             hip.moe_down_scale(contrib, act, self._bank("down"), offs, counts,
                                order, flat_w, bias=db)
         else:

@@ -246,3 +246,22 @@ def test_long_prompts_of_few_large_experts(monkeypatch, T, loop):
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing",
                         lambda: True)
     assert not m._library_wins(T)
+
+
+@pytest.mark.parametrize("E,T,H,I,tiles", [
+    (8, 32, 256, 3200, False), (8, 33, 256, 3200, True),
+    (8, 8, 256, 3072, True), (40, 4, 4096, 3200, False),
+    (40, 5, 4096, 3200, True)])
+def test_down_product_of_few_rows(monkeypatch, E, T, H, I, tiles):
+    """Both sides of the lines between its two forms."""
+    m, g = _moe(E, 2, H, I)
+    x = torch.randn(T, H, generator=g, device="cuda").bfloat16()
+    hip, taken = _hip(), []
+    real = hip.moe_down_scale
+    monkeypatch.setattr(hip, "moe_down_scale",
+                        lambda *a, **k: (taken.append(1), real(*a, **k)))
+    out = m(x)
+    assert (not taken) == tiles
+    ref = _moe_reference(m, x)
+    # as above
+    assert float((out.double() - ref).norm() / ref.norm()) < 2.0 ** -7
