@@ -387,9 +387,16 @@ def _rows_tile_plan(M: int, N: int, K: int):
     13.5 / 12.8;
     more columns, where the library loses on rows a multiple of 4 KB apart:
     28672x4096 41.2 / 50.7 at 48 rows and 45.7 / 57.5 at 96, 128256x4096
-    182 / 254, 16384x2048 15.7 / 18.0, but 51200x3072 72 / 62 and at 96 rows
-    16384x2048 18.9 / 19.0 (18944 columns make 296 tiles, two for some CUs and
-    one for most: 31 / 27 at 2560);
+    182 / 254, 16384x2048 15.7 / 18.0, 65536x6144 144 / 178, 28672x8192
+    85 / 129, but 51200x3072 72 / 62, 40960x5120 97 / 91, 22016x2560 31 / 30
+    (18944 columns make 296 tiles, two for some CUs and one for most: 31 / 27
+    at 2560). At 96 rows: 16384x2048 18.3 / 18.8, 16384x4096 32 / 35,
+    65536x2048 60 / 70, 65536x4096 99 / 129, 51200x6144 137 / 147, 22016x8192
+    82 / 82, 128256x8192 372 / 416; rows of 5120, 3072 and 2560 lose (51200 of
+    each: 121 / 104, 73 / 68, 65 / 58), so do longer ones (51200x10240
+    224 / 200, 102400x12288 at 112 rows 557 / 504), 12288x4096 33 / 30, and
+    above 96 rows one and a bit rounds of tiles of long rows (40960x8192 at
+    128 160 / 154, where 40960x4096 is 86 / 87);
     up to 16 rows: 28672x4096 40 / 43 at one and 41 / 53 at 16, 4096x11008
     17 / 31, 22016x4096 32 / 39, 128256x4096 175 / 178, but 16384x4096 at one
     row 27 / 26."""
@@ -407,7 +414,8 @@ def _rows_tile_plan(M: int, N: int, K: int):
         elif M <= 64:
             wins = K % 2048 == 0 and (K <= 8192 or N <= 32768)
         else:
-            wins = K == 4096 and N >= 22016 or K == 2048 and N >= 51200
+            wins = K % 2048 == 0 and K <= 8192 and N >= 16384 and not (
+                M > 96 and K > 4096 and 256 < t128 < 500)
         plan = (128 if wide else 64), 1
     elif K <= 2048:
         wins = 16 < M <= 64 and (K == 1024 and N >= 2560

@@ -139,3 +139,19 @@ def test_packed_weights_of_any_column_count(N, K):
     # the expansion rounds a weight to bf16 (2^-9 of it), the result once more
     err = (qlinear(x, None, pack).double() - x.double() @ w.T).abs()
     assert bool((err <= size * 2.0 ** -7).all())
+
+
+@pytest.mark.parametrize("M,N,K,own", [
+    (65, 16384, 2048, True), (65, 16376, 2048, False),
+    (96, 22024, 6144, True), (97, 32896, 6144, False),
+    (97, 32768, 8192, True), (128, 16384, 10240, False),
+    (80, 16384, 3072, False)])
+def test_rule_of_tiles_for_many_columns(M, N, K, own):
+    from gpustack_amd import ops
+
+    assert (ops._rows_tile_plan(M, N, K) is not None) == own
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    x = torch.randn(M, K + 8, generator=g, device="cuda").bfloat16()[:, :K]
+    w = torch.randn(N, K, generator=g, device="cuda").bfloat16()
+    _close(ops.linear_auto(x, w), x.double() @ w.double().T,
+           x.double().abs() @ w.double().abs().T)
