@@ -107,3 +107,48 @@ def test_parts_of_a_window(monkeypatch, D, window):
         err = (out[i].double() - ref).abs()
         # as above: one rounding to bf16, fp32 before it
         assert bool((err <= ref.abs() * 2.0 ** -8 + 1e-4).all()), (i, n)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("D,Hq,Hkv", [(64, 16, 2), (128, 8, 2), (128, 2, 2),
+                                      (256, 8, 2)])
+@pytest.mark.parametrize("lens", [[100, 1, 77], [2500, 1, 300, 1001, 160]])
+@pytest.mark.parametrize("sink,window,softcap", [
+    (True, 0, 0.0), (True, 129, 0.0), (False, 0, 20.0), (True, 129, 20.0)])
+def test_sinks_and_softcap(monkeypatch, fp8, D, Hq, Hkv, lens, sink, window,
+                           softcap):
+    """In the one part of short sequences, and where the join adds the sink."""
+    from gpustack_amd import ops
+
+    monkeypatch.setenv("GPUSTACK_AMD_OSS_KERNELS", "1")
+    g = torch.Generator(device="cuda").manual_seed(D + Hq + lens[0])
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    nb = (max(lens) + 15) // 16
+    kc, vc = (rnd(nb * len(lens), Hkv, 16, D) for _ in range(2))
+    if fp8:
+        kc, vc = (t.to(torch.float8_e4m3fn) for t in (kc, vc))
+    bt = torch.randperm(nb * len(lens), generator=g, device="cuda").int() \
+        .view(len(lens), nb)
+    q = rnd(len(lens), Hq, D) * 3
+    sinks = torch.randn(Hq, generator=g, device="cuda") * 3 if sink else None
+    out = torch.empty_like(q)
+    scale = 1 / math.sqrt(D)
+    ops.paged_attn_decode(out, q, kc, vc, bt,
+                          torch.tensor(lens, dtype=torch.int32,
+                                       device="cuda"), scale, sinks=sinks,
+                          window=window, softcap=softcap)
+    rep = Hq // Hkv
+    for i, n in enumerate(lens):
+        j = torch.arange(max(0, n - window) if window else 0, n, device="cuda")
+        k, v = (t.float()[bt[i, j // 16].long(), :, j % 16].double()
+                .repeat_interleave(rep, 1) for t in (kc, vc))
+        s = (q[i].double() * k).sum(-1) * scale              # [keys, Hq]
+        if softcap:
+            s = torch.tanh(s / softcap) * softcap
+        if sink:
+            s = torch.cat([s, sinks.double()[None]])
+        p = s.softmax(0)[:len(j)]
+        ref = (p[:, :, None] * v).sum(0)
+        err = (out[i].double() - ref).abs()
+        # as above: one rounding to bf16, fp32 before it
+        assert bool((err <= ref.abs() * 2.0 ** -8 + 1e-4).all()), (i, n)

@@ -109,3 +109,117 @@ def test_tile_lists_of_either_size(rows):
         _check(out[at:at + n], q[at:at + n], k[at:at + n], v[at:at + n], 0,
                0.1)
         at += n
+
+
+def _check_variant(out, q, k, v, hist, scale, sinks, window, softcap):
+    """out [n, Hq, DV], q [n, Hq, D] of one sequence, k / v [hist + n, G, .]"""
+    n, Hq, _ = q.shape
+    rep = Hq // k.shape[1]
+    k, v = (t.double().repeat_interleave(rep, 1).transpose(0, 1)
+            for t in (k, v))
+    s = torch.matmul(q.double().transpose(0, 1),
+                     k.transpose(1, 2).contiguous()) * scale
+    if softcap:
+        s = torch.tanh(s / softcap) * softcap
+    at = torch.arange(hist, hist + n, device=q.device)[:, None]
+    kv = torch.arange(hist + n, device=q.device)[None, :]
+    hide = (kv > at) | (kv <= at - window if window else kv < 0)
+    s = s.masked_fill(hide, float("-inf"))
+    if sinks is not None:
+        s = torch.cat([s, sinks.double()[:, None, None].expand(Hq, n, 1)], -1)
+    p = s.softmax(-1)[:, :, :hist + n]
+    ref = torch.matmul(p, v).transpose(0, 1)
+    # as in _check
+    bound = torch.matmul(p, v.abs()).transpose(0, 1) * 2.0 ** -8 \
+        + ref.abs() * 2.0 ** -8 + 1e-4
+    err = (out.double() - ref).abs()
+    assert bool((err <= bound).all()), float((err - bound).max())
+
+
+_VARIANTS = pytest.mark.parametrize("sink,window,softcap", [
+    (False, 0, 0.0), (True, 0, 0.0), (False, 1, 0.0), (True, 128, 0.0),
+    (False, 65, 30.0), (True, 0, 30.0)])
+_HEADS = pytest.mark.parametrize("D,Hq,Hkv", [(64, 16, 2), (128, 8, 4),
+                                              (256, 4, 2)])
+
+
+@_VARIANTS
+@_HEADS
+@pytest.mark.parametrize("lens", [
+    [1], [31, 33, 64], [65, 77, 2], [127, 128, 129], [300]])
+def test_variants_of_whole_prompts(monkeypatch, D, Hq, Hkv, lens, sink, window,
+                                   softcap):
+    from gpustack_amd import ops
+
+    monkeypatch.setenv("GPUSTACK_AMD_OSS_KERNELS", "1")
+    g = torch.Generator(device="cuda").manual_seed(sum(lens) + D)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    T = sum(lens)
+    q, k, v = rnd(T, Hq, D) * 3, rnd(T, Hkv, D), rnd(T, Hkv, D)
+    sinks = torch.randn(Hq, generator=g, device="cuda") * 3 if sink else None
+    out = torch.full_like(q, 9.0)
+    scale = 1 / math.sqrt(D)
+    ops.varlen_prefill_attn(out, q, k, v, lens, scale, sinks=sinks,
+                            window=window, softcap=softcap)
+    at = 0
+    for n in lens:
+        r = slice(at, at + n)
+        _check_variant(out[r], q[r], k[r], v[r], 0, scale, sinks, window,
+                       softcap)
+        at += n
+
+
+@_VARIANTS
+@_HEADS
+@pytest.mark.parametrize("seqs", [
+    [(0, 1)], [(1, 127), (15, 129)], [(17, 33), (63, 1), (64, 64)],
+    [(500, 77), (0, 130)]])
+def test_variants_behind_history(monkeypatch, D, Hq, Hkv, seqs, sink, window,
+                                 softcap):
+    from gpustack_amd import ops
+
+    monkeypatch.setenv("GPUSTACK_AMD_OSS_KERNELS", "1")
+    g = torch.Generator(device="cuda").manual_seed(seqs[0][0] + D)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    nb = max((h + n + 15) // 16 for h, n in seqs)
+    kc, vc = (rnd(nb * len(seqs), Hkv, 16, D) for _ in range(2))
+    bt = torch.randperm(nb * len(seqs), generator=g, device="cuda").int() \
+        .view(len(seqs), nb)
+    starts = [sum(n for _, n in seqs[:i]) for i in range(len(seqs))]
+    # what lies behind a sequence's end in its last page is not its own
+    for i, (h, n) in enumerate(seqs):
+        j = torch.arange(h + n, (h + n + 15) // 16 * 16, device="cuda")
+        for pool in (kc, vc):
+            pool[bt[i, j // 16].long(), :, j % 16] = float("nan")
+    q = rnd(sum(n for _, n in seqs), Hq, D) * 3
+    sinks = torch.randn(Hq, generator=g, device="cuda") * 3 if sink else None
+    out = torch.full_like(q, 9.0)
+    scale = 1 / math.sqrt(D)
+    ops.paged_prefill_attn(out, q, kc, vc, bt, starts, [h for h, _ in seqs],
+                           [n for _, n in seqs], scale, sinks=sinks,
+                           window=window, softcap=softcap)
+    for i, (h, n) in enumerate(seqs):
+        j = torch.arange(h + n, device="cuda")
+        blk = bt[i, j // 16].long()
+        r = slice(starts[i], starts[i] + n)
+        _check_variant(out[r], q[r], kc[blk, :, j % 16], vc[blk, :, j % 16], h,
+                       scale, sinks, window, softcap)
+
+
+@pytest.mark.parametrize("lens", [[1], [33, 64, 65], [129, 200]])
+def test_keys_wider_than_values(monkeypatch, lens):
+    from gpustack_amd import ops
+
+    monkeypatch.setenv("GPUSTACK_AMD_MLA_KERNEL", "1")
+    g = torch.Generator(device="cuda").manual_seed(sum(lens))
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    T = sum(lens)
+    q, k, v = rnd(T, 16, 192) * 3, rnd(T, 16, 192), rnd(T, 16, 128)
+    out = torch.full_like(v, 9.0)
+    scale = 1 / math.sqrt(192)
+    ops.varlen_prefill_attn(out, q, k, v, lens, scale)
+    at = 0
+    for n in lens:
+        r = slice(at, at + n)
+        _check_variant(out[r], q[r], k[r], v[r], 0, scale, None, 0, 0.0)
+        at += n
