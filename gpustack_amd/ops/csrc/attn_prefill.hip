@@ -67,12 +67,14 @@ DEVICE_INLINE unsigned int pack_bf16(float lo, float hi) {
                             __builtin_convertvector(v, bf16x2));
 }
 
-// EXT: sinks / sliding window / softcap. PAGED: k / v are pools
-// [nblocks, Hkv, 16, D]; otherwise rows of the batch.
+// EXT: 1 sinks / sliding window, 2 softcap (and those). Forms of their own,
+// because a short prompt is one pass over the code (77 rows of 64 heads of 64
+// on 8, us: 7.3, 8.4 and 11.4; with all of it in one kernel 8.9, 8.9 and 14.6).
+// PAGED: k / v are pools [nblocks, Hkv, 16, D]; otherwise rows of the batch.
 // A tile: the sequence's first row in q and out, the tile's first row within
 // the sequence's rows, the cached tokens in front of them, their number, and
 // the sequence's row of the block tables.
-template <int D, int DVK, bool EXT, bool PAGED>
+template <int D, int DVK, int EXT, bool PAGED>
 __global__ __launch_bounds__(PF_THREADS, D > 128 ? 1 : 2)
 void flash_prefill_kernel(
     unsigned short* __restrict__ out,      // [T, Hq, DVK]
@@ -117,6 +119,15 @@ void flash_prefill_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
   const int lc = lane & 31;
   const int hf = lane >> 5;
+  // The lane's own part of every LDS and memory address does not change from
+  // tile to tile; at 256 channels keeping all of them took more than 512
+  // registers (284 bytes a lane in scratch, 77 rows 18.8 us; worked out anew in
+  // each tile 13.7, and 2000 rows 191 -> 126).
+  auto lane_again = [&] {
+    int l = lane;
+    if constexpr (D > 192) asm volatile("" : "+v"(l));
+    return l;
+  };
 
   // this wave's 32 query rows as the B operand
   const int qrow = q0 + wave * 32 + lc;            // within the new rows
@@ -142,13 +153,14 @@ void flash_prefill_kernel(
   const int kt_end = (kv_end + BK - 1) / BK;
   // the first tile any row of the workgroup can see
   int kt0 = 0;
-  if constexpr (EXT)
+  if constexpr (EXT > 0)
     if (window > 0) kt0 = max(0, hist + q0 - window + 1) / BK;
 
   u32x4 kst[KU], vst[VB][4];
 
   // wave w stages rows 16 w .. 16 w + 15 of a tile (one page of a pool)
   auto issue = [&](int kt) {
+    const int lane = lane_again();
     const int kv0 = kt * BK + wave * 16;
     const unsigned short *kp, *vp;
     long kstep, vstep;
@@ -192,6 +204,7 @@ void flash_prefill_kernel(
   };
 
   auto stash = [&](unsigned short* buf) {
+    const int lane = lane_again();
     unsigned short* vt = buf + K_ELEMS;
 #pragma unroll
     for (int i = 0; i < KU; ++i) {
@@ -222,7 +235,7 @@ void flash_prefill_kernel(
     }
   };
 
-  const float sc = scale * LOG2E;
+  const float sc = EXT == 2 ? scale / softcap : scale * LOG2E;
   issue(kt0);
   stash(lds);
   __syncthreads();
@@ -234,9 +247,10 @@ void flash_prefill_kernel(
     if (more) issue(kt + 1);
 
     bool live = kv0 <= lo_wave + 31;               // not above the diagonal
-    if constexpr (EXT)
+    if constexpr (EXT > 0)
       live = live && !(window > 0 && kv0 + BK <= lo_wave - window + 1);
     if (live) {
+      const int la = lane_again(), lc = la & 31, hf = la >> 5;
       f32x16 st[2];
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
@@ -252,20 +266,18 @@ void flash_prefill_kernel(
       }
       // scores in powers of two
       bool edge = kv0 + BK - 1 > lo_wave || kv0 + BK > len;
-      if constexpr (EXT) edge = edge || window > 0;
+      if constexpr (EXT > 0) edge = edge || window > 0;
       float mx = -INFINITY;
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           float x = st[t][r] * sc;
-          if constexpr (EXT)
-            if (softcap > 0.f)
-              x = tanhf(st[t][r] * scale / softcap) * (softcap * LOG2E);
+          if constexpr (EXT == 2) x = tanhf(x) * (softcap * LOG2E);
           if (edge) {
             const int kv = kv0 + t * 32 + 8 * (r >> 2) + 4 * hf + (r & 3);
             bool ok = kv <= qpos && kv < len;
-            if constexpr (EXT) ok = ok && (window <= 0 || kv > qpos - window);
+            if constexpr (EXT > 0) ok = ok && (window <= 0 || kv > qpos - window);
             x = ok ? x : -INFINITY;
           }
           st[t][r] = x;
@@ -318,7 +330,7 @@ void flash_prefill_kernel(
   // normalise; a SINK logit joins the denominator only
   l += __shfl_xor(l, 32, WAVE_SIZE);
   float num = 1.f;
-  if constexpr (EXT) {
+  if constexpr (EXT > 0) {
     if (sinks != nullptr) {
       const float sk = sinks[qh] * LOG2E;
       const float M = fmaxf(m, sk);
@@ -358,7 +370,7 @@ void flash_prefill_kernel(
   }
 }
 
-template <int D, int DVK, bool EXT, bool PAGED>
+template <int D, int DVK, int EXT, bool PAGED>
 void launch(void* out, const void* q, const void* k, const void* v,
             const int* bt, const int* start, const int* q0, const int* hist,
             const int* nnew, const int* seq, int ntiles, int Hq, int Hkv,
@@ -387,20 +399,19 @@ void flash_prefill_paged_launch(
     *err_unsupported = 1;
     return;
   }
-  const bool ext = (sinks != nullptr) || window > 0 || softcap > 0.f;
-#define PPG_LAUNCH(DD, E)                                                     \
+#define PPG_FORM(DD, E)                                                       \
   launch<DD, DD, E, true>(out, q, kc, vc, block_tables, tile_qstart, tile_q0, \
                           tile_hist, tile_new, tile_seq, ntiles, Hq, Hkv,     \
                           maxb, scale, qs, 0, 0, sinks, window, softcap, s)
-  if (D == 128) {
-    if (ext) PPG_LAUNCH(128, true);
-    else PPG_LAUNCH(128, false);
-  } else if (D == 64) {
-    PPG_LAUNCH(64, true);
-  } else {
-    PPG_LAUNCH(256, true);
-  }
+#define PPG_LAUNCH(DD)                                                        \
+  if (softcap > 0.f) PPG_FORM(DD, 2);                                         \
+  else if (sinks != nullptr || window > 0) PPG_FORM(DD, 1);                   \
+  else PPG_FORM(DD, 0);
+  if (D == 128) { PPG_LAUNCH(128) }
+  else if (D == 64) { PPG_LAUNCH(64) }
+  else { PPG_LAUNCH(256) }
 #undef PPG_LAUNCH
+#undef PPG_FORM
 }
 
 void flash_prefill_launch(void* out, const void* q, const void* k,
@@ -417,23 +428,22 @@ void flash_prefill_launch(void* out, const void* q, const void* k,
     *err_unsupported = 1;
     return;
   }
-  const bool ext = (sinks != nullptr) || window > 0 || softcap > 0.f;
-#define PF_LAUNCH(DD, E, DVV)                                                 \
+#define PF_FORM(DD, E, DVV)                                                   \
   launch<DD, DVV, E, false>(out, q, k, v, nullptr, tile_start, tile_q0,       \
                             nullptr, tile_len, nullptr, ntiles, Hq, Hkv, 0,   \
                             scale, qs, ks, vs, sinks, window, softcap, s)
+#define PF_LAUNCH(DD)                                                         \
+  if (softcap > 0.f) PF_FORM(DD, 2, DD);                                      \
+  else if (sinks != nullptr || window > 0) PF_FORM(DD, 1, DD);                \
+  else PF_FORM(DD, 0, DD);
   if (mla_dims) {
     // MLA expand-prefill (DeepSeek): 192-dim qk over 128-dim values
-    PF_LAUNCH(192, false, 128);
-  } else if (D == 128) {
-    if (ext) PF_LAUNCH(128, true, 128);
-    else PF_LAUNCH(128, false, 128);
-  } else if (D == 64) {
-    PF_LAUNCH(64, true, 64);
-  } else {
-    PF_LAUNCH(256, true, 256);
-  }
+    PF_FORM(192, 0, 128);
+  } else if (D == 128) { PF_LAUNCH(128) }
+  else if (D == 64) { PF_LAUNCH(64) }
+  else { PF_LAUNCH(256) }
 #undef PF_LAUNCH
+#undef PF_FORM
 }
 
 // ---------------------------------------------------------------------------
