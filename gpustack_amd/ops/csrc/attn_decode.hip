@@ -8,8 +8,11 @@
 //    query heads of a kv head share its K/V stream, so each KV byte is read
 //    exactly once per step. The keys of a sequence are cut into parts when
 //    (sequences x kv heads) alone leaves CUs without work (decode_parts);
-//    a second kernel joins the parts.
-//  - 4 waves per workgroup, 32 keys (two pages) per wave and step. Scores are
+//    a second kernel joins the parts where more than one has keys.
+//  - 4 waves per workgroup, 32 keys (two pages) per wave and step; the last
+//    step, and the only one of parts of up to 64 keys, may be of one page (us,
+//    8 heads on 8: 64 x 400 keys in a window of 128 9.5 -> 7.1, 512 x 40 20.1 ->
+//    18.2 and in fp8 18.7 -> 16.5). Scores are
 //    a matrix product, S^T = K Q^T on mfma_f32_16x16x32_bf16: K rows are the
 //    16-byte loads of the A operand as they lie in the page, the GQ query
 //    rows (zero rows up to 16) the B operand. One lane then holds one head's
@@ -23,8 +26,7 @@
 // Bound by the K/V stream: 32 keys cost a SIMD about 1300 cycles (GQ = 4),
 // 31 TB/s over the chip in bf16 and 15 TB/s in fp8, so memory sets the time
 // once enough of it is in flight (16 KB a wave in bf16 at 128 channels;
-// registers allow 3 waves a SIMD there with 4 to 8 heads, 4 in fp8 with 4 or
-// at 64 channels, 2 at 256).
+// decode_waves has the waves a SIMD).
 //
 // KV pool layout: [num_blocks, Hkv, BS, D] bf16 | fp8, BS = 16 tokens.
 #include "common.h"
@@ -88,9 +90,19 @@ DEVICE_INLINE int window_start(int len, int window) {
   return window > 0 && len > window ? len - window : 0;
 }
 
+// Waves that a SIMD holds beside each other. Left to itself the compiler takes
+// a few registers too many for four of them at 4 heads in fp8 and for three at
+// 8 in bf16 (us: 256 x 400 keys 43 -> 49, 93 -> 99).
+constexpr int decode_waves(int D, int GQ, bool fp8) {
+  return D == 64    ? (GQ <= 6 ? 5 : 4)
+         : D == 256 ? 2
+                    : (GQ <= 2 || (fp8 && GQ <= 5) ? 4 : 3);
+}
+
 // EXT: sinks / sliding window / softcap (GPT-OSS and Gemma variants).
 template <int D, int GQ, bool FP8, bool EXT>
-__global__ __launch_bounds__(THREADS) void paged_attn_decode_kernel(
+__global__ __launch_bounds__(THREADS, decode_waves(D, GQ, FP8))
+void paged_attn_decode_kernel(
     unsigned short* __restrict__ out,        // [N, Hq, D]
     const unsigned short* __restrict__ q,    // [N, Hq, D]
     const void* __restrict__ kc,             // [B, Hkv, BS, D] bf16|fp8
@@ -119,11 +131,13 @@ __global__ __launch_bounds__(THREADS) void paged_attn_decode_kernel(
   // sliding window (EXT): the query sits at position len - 1 and attends
   // [max(0, len - window), len); the parts cut only that
   const int wstart = EXT ? window_start(len, window) : 0;
-  const int from = wstart / STEP * STEP;
+  const int from = wstart / BS * BS;
   const int span = part_tokens(len - from, nsplit, least);
   const int t0 = from + (int)blockIdx.z * span;
   const int t1 = min(len, t0 + span);
   if (nsplit > 1 && t0 >= len) return;     // the join skips it as well
+  // the only part with keys is the result (one x 60 keys 8.5 -> 7.8)
+  const bool whole = nsplit == 1 || span >= len - from;
 
   const int lane = threadIdx.x & (WAVE_SIZE - 1);
   const int wave = threadIdx.x / WAVE_SIZE;
@@ -160,29 +174,30 @@ __global__ __launch_bounds__(THREADS) void paged_attn_decode_kernel(
   const int last_page = (len - 1) / BS;
   const float sc = scale * LOG2E;
 
-  for (int c0 = t0 + wave * STEP; c0 < t1; c0 += NWAVES * STEP) {
+  auto step = [&](auto pages, int c0) {
+    constexpr int PG = decltype(pages)::value, VR = 4 * PG;
     const int page = c0 / BS;
-    long at[2];
+    long at[PG];
 #pragma unroll
-    for (int p = 0; p < 2; ++p)
+    for (int p = 0; p < PG; ++p)
       at[p] = (long)bt[min(page + p, last_page)] * page_bytes;
-    unsigned int kw[2][QK][KW], vw[8][VW];
+    unsigned int kw[PG][QK][KW], vw[VR][VW];
 #pragma unroll
-    for (int p = 0; p < 2; ++p)
+    for (int p = 0; p < PG; ++p)
 #pragma unroll
       for (int kk = 0; kk < QK; ++kk)
         load_words<KW>(kw[p][kk],
                        kbase + at[p] + (sub * D + kk * 32 + g * 8) * ES);
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < VR; ++i)
       load_words<VW>(vw[i], vbase + at[i / 4] +
                                 (((i & 3) * 4 + g) * D + sub * DV) * ES);
 
     // scores: lane = head `sub`, keys c0 + p*16 + g*4 + r
-    float x[8];
+    float x[VR];
     float mx = -INFINITY;
 #pragma unroll
-    for (int p = 0; p < 2; ++p) {
+    for (int p = 0; p < PG; ++p) {
       f32x4 st{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int kk = 0; kk < QK; ++kk) {
@@ -225,13 +240,13 @@ __global__ __launch_bounds__(THREADS) void paged_attn_decode_kernel(
     m = nm;
     s *= corr;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < VR; ++i) {
       x[i] = __builtin_amdgcn_exp2f(x[i] - base);
       s += x[i];
     }
     if (sub < GQ) {
 #pragma unroll
-      for (int p = 0; p < 2; ++p)
+      for (int p = 0; p < PG; ++p)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
           lds_p[wave][p * 16 + g * 4 + r][sub] = x[p * 4 + r];
@@ -250,9 +265,9 @@ __global__ __launch_bounds__(THREADS) void paged_attn_decode_kernel(
     // values: lane = channels sub*DV .., keys (i/4)*16 + (i%4)*4 + g. Rows that
     // are not the sequence's (behind its end in its last page, in front of its
     // window) may hold anything, and a weight of 0 does not undo a NaN
-    if (c0 + STEP > t1 || (EXT && c0 < wstart)) {
+    if (c0 + PG * BS > t1 || (EXT && c0 < wstart)) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
+      for (int i = 0; i < VR; ++i) {
         const int tok = c0 + (i / 4) * 16 + (i & 3) * 4 + g;
         if (tok >= t1 || (EXT && tok < wstart))
 #pragma unroll
@@ -260,7 +275,7 @@ __global__ __launch_bounds__(THREADS) void paged_attn_decode_kernel(
       }
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < VR; ++i) {
       float pr[GQ], vf[DV];
 #pragma unroll
       for (int gq = 0; gq < GQ; ++gq)
@@ -280,7 +295,15 @@ __global__ __launch_bounds__(THREADS) void paged_attn_decode_kernel(
         for (int j = 0; j < DV; ++j) acc[gq][j] += pr[gq] * vf[j];
     }
     asm volatile("" ::: "memory");  // P is read before the next step's writes
-  }
+  };
+  // a page for each wave where that is all (one step of latency, and no wave
+  // without keys beside one with two pages), else two a step and a last one
+  const bool few = t1 - t0 <= NWAVES * BS;
+  int c0 = t0 + wave * (few ? BS : STEP);
+  if (!few)
+    for (; c0 + BS < t1; c0 += NWAVES * STEP)
+      step(std::integral_constant<int, 2>{}, c0);
+  if (c0 < t1) step(std::integral_constant<int, 1>{}, c0);
 
   // the four key groups of a wave, then the waves
   s += __shfl_xor(s, 16, WAVE_SIZE);
@@ -311,7 +334,7 @@ __global__ __launch_bounds__(THREADS) void paged_attn_decode_kernel(
     if constexpr (EXT) {
       // an attention sink joins the softmax denominator only; with several
       // parts the join adds it
-      if (sinks != nullptr && nsplit == 1) {
+      if (sinks != nullptr && whole) {
         const float sk = sinks[h * GQ + gq] * LOG2E;
         M = fmaxf(M, sk);
         extra = __builtin_amdgcn_exp2f(sk - M);
@@ -325,7 +348,7 @@ __global__ __launch_bounds__(THREADS) void paged_attn_decode_kernel(
       num += wt * lds_acc[w][gq][d];
       den += wt * lds_ms[w][gq][1];
     }
-    if (nsplit == 1) {
+    if (whole) {
       out[((long)seq * Hq + (long)h * GQ + gq) * D + d] =
           f2bf(den > 0.f ? num / den : 0.f);
     } else {
@@ -351,9 +374,10 @@ __global__ __launch_bounds__(D) void paged_attn_join_kernel(
   const int seq = blockIdx.x, hq = blockIdx.y, Hq = gridDim.y;
   const int h = hq / GQ, gq = hq % GQ, d = threadIdx.x;
   const int len = seq_lens[seq];
-  const int keys = len - window_start(len, window) / STEP * STEP;
+  const int keys = len - window_start(len, window) / BS * BS;
   const int span = part_tokens(keys, nsplit, least);
   const int n = min(nsplit, (keys + span - 1) / span);
+  if (n == 1) return;                      // the decode kernel's own result
   const float* pp = part +
       (((long)seq * (Hq / GQ) + h) * nsplit * GQ + gq) * (D + 2);
   const long step = (long)GQ * (D + 2);
@@ -380,24 +404,24 @@ __global__ __launch_bounds__(D) void paged_attn_join_kernel(
 // sequences x kv heads (`base`) do not, and even out unequal lengths, but each
 // writes its sums to memory and the join is a launch. max_blocks is the width
 // of the block table, so a captured graph keeps its grid; parts behind a
-// sequence's end return at once. Measured with 1 to 64 parts, us, 32 heads on
+// sequence's end return at once. Measured with 1 to 32 parts, us, 32 heads on
 // 8 of 128 channels in bf16 unless said (parts chosen: time / others):
-//   one sequence, 4000 keys   16: 18.5 / 8: 17.8, 64: 38.8, 1: 51
-//   8, 200 to 8000            8: 38 / 4: 37, 32: 51, 1: 95
-//   16, 1000 to 8000          4: 62 / 1: 132, 16: 75
-//   32, 1000 to 8000          2: 125 / 1: 153, 8: 135; all of 300: 1: 12.7 / 2: 15.3
-//   48, 3500 to 7900          2: 218 / 1: 234, 6: 223
-//   64, 100 to 4000           1: 119 / 2: 136, 4: 131; all of 300: 1: 18 / 4: 29
+//   one sequence, 4000 keys   16: 17 / 8: 16.5, 32: 23, 1: 49
+//   8, 200 to 8000            8: 37 / 4: 39, 32: 48, 1: 112
+//   16, 1000 to 8000          4: 66 / 1: 137, 16: 71; 300 to 1200 2: 18 / 1: 22
+//   32, 1000 to 8000          2: 134 / 1: 154, 8: 140; all of 300: 2: 12.5 / 1: 10.9
+//   48, 3500 to 7900          2: 219 / 1: 237, 6: 225; 100 to 600 2: 21 / 1: 19
+//   64, 100 to 4000           1: 125 / 2: 134, 4: 131; all of 300: 1: 16.7 / 4: 18.9
 // Rows of 128 bytes (fp8, or 64 channels) spend relatively more on scores, so
 // they are cut for twice as many workgroups:
-//   fp8: 64, 100 to 4000      2: 84 / 1: 89; 32, 1000 to 8000 4: 83 / 1: 117, 2: 91
-//        96, 100 to 4000      1: 108 / 2: 123
+//   fp8: 64, 100 to 4000      2: 86 / 1: 83, 4: 82; 32, 1000 to 8000 4: 90 / 1: 141, 2: 97
+//        96, 100 to 4000      1: 117 / 2: 132; 48, 3500 to 7900 2: 131 / 1: 179, 4: 150
 // So are heads of 256 channels, of which few workgroups fit at once, but not
 // into more than 8 parts (16 heads on 8):
-//        48, 3500 to 7900     3: 434 / 1: 480, 2: 438; 24, 200 to 2000 6: 45 / 1: 52
-//        64, 100 to 4000      1: 238 / 4: 233, 8: 249
+//        48, 3500 to 7900     3: 436 / 1: 486, 6: 414; 24, 200 to 2000 6: 48 / 1: 51
+//        64, 100 to 4000      1: 240 / 4: 247, 8: 259
 // A context of less than one part pays for the join's launch behind a wide
-// block table (one sequence of 100 keys, 8 heads on 8: 6.8 against 5.0).
+// block table (one sequence of 100 keys, 8 heads on 8: 5.8 against 4.4).
 DecodeParts decode_parts(int N, int Hkv, int max_blocks, int D, int fp8,
                          int window) {
   const long base = (long)N * Hkv;
