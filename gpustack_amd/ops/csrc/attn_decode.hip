@@ -80,6 +80,29 @@ DEVICE_INLINE unsigned int pack_hi(float lo, float hi) {
                                0x07060302u);
 }
 
+// A value and the one of the lane 16 or 32 away, in either order, without the
+// LDS: as shuffles these exchanges, most of them in the sums at the end, were
+// 12 % of the kernel over 240 shapes (16 heads of 256, us: 512 x 40 keys
+// 53.6 -> 42.0, one x 300 12.2 -> 11.1; 32 of 128: 64 x 400 21.0 -> 19.2).
+template <int M>
+DEVICE_INLINE f32x2 with_lane(float v) {
+  const unsigned int u = __builtin_bit_cast(unsigned int, v);
+  const auto r = M == 16 ? __builtin_amdgcn_permlane16_swap(u, u, false, false)
+                         : __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  const unsigned int x = r[0], y = r[1];
+  return f32x2{__builtin_bit_cast(float, x), __builtin_bit_cast(float, y)};
+}
+DEVICE_INLINE float sum_groups(float v) {
+  f32x2 p = with_lane<16>(v);
+  p = with_lane<32>(p[0] + p[1]);
+  return p[0] + p[1];
+}
+DEVICE_INLINE float max_groups(float v) {
+  f32x2 p = with_lane<16>(v);
+  p = with_lane<32>(fmaxf(p[0], p[1]));
+  return fmaxf(p[0], p[1]);
+}
+
 // keys per part of a sequence of `len` tokens: whole steps, at least `least`
 DEVICE_INLINE int part_tokens(int len, int nsplit, int least) {
   const int per = (len + nsplit - 1) / nsplit;
@@ -95,7 +118,7 @@ DEVICE_INLINE int window_start(int len, int window) {
 // 8 in bf16 (us: 256 x 400 keys 43 -> 49, 93 -> 99).
 constexpr int decode_waves(int D, int GQ, bool fp8) {
   return D == 64    ? (GQ <= 6 ? 5 : 4)
-         : D == 256 ? 2
+         : D == 256 ? (fp8 && GQ <= 2 ? 3 : 2)
                     : (GQ <= 2 || (fp8 && GQ <= 5) ? 4 : 3);
 }
 
@@ -232,8 +255,7 @@ void paged_attn_decode_kernel(
         mx = fmaxf(mx, v);
       }
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE_SIZE));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE_SIZE));
+    mx = max_groups(mx);
     const float nm = fmaxf(m, mx);
     const float base = nm == -INFINITY ? 0.f : nm;
     const float corr = __builtin_amdgcn_exp2f(m - base);
@@ -306,15 +328,12 @@ void paged_attn_decode_kernel(
   if (c0 < t1) step(std::integral_constant<int, 1>{}, c0);
 
   // the four key groups of a wave, then the waves
-  s += __shfl_xor(s, 16, WAVE_SIZE);
-  s += __shfl_xor(s, 32, WAVE_SIZE);
+  s = sum_groups(s);
 #pragma unroll
   for (int gq = 0; gq < GQ; ++gq) {
 #pragma unroll
     for (int j = 0; j < DV; ++j) {
-      float a = acc[gq][j];
-      a += __shfl_xor(a, 16, WAVE_SIZE);
-      a += __shfl_xor(a, 32, WAVE_SIZE);
+      const float a = sum_groups(acc[gq][j]);
       if (g == 0) lds_acc[wave][gq][sub * DV + j] = a;
     }
   }
