@@ -359,10 +359,11 @@ def _rows_gemm_wins(M: int, N: int, K: int) -> bool:
     15.6, 2048x4096 8.5 / 9.6 / 10.8 against 14.8, 5120x2048 8.0 / 9.0 / 10.6
     against 12.3 (24 rows of 4096x4096: 12.9 against 13.4; 6144x4096 13.0 /
     15.6 / 18.3 against 14.6);
-    many columns: 16384x2048 14 / 15 / 16 against 18, 22016x4096 36 / 39 / 41
-    against 52, 28672x4096 43 / 47 / 53 against 54, 49152x2048 34 / 37 / 42
-    against 47, 65536x4096 88 / 93 against 120 (49152x3072 at 16 rows 65
-    against 60, 16384x5120 34 / 37 / 42 against 34);
+    many columns (22016x4096 36 / 39 / 41 against 52 and 28672x4096 43 / 47 / 53
+    against 54, where the tiled product is better still): 16384x2048 14 / 15 /
+    16 against 18, 49152x2048 34 / 37 / 42 against 47, 65536x4096 88 / 93
+    against 120 (49152x3072 at 16 rows 65 against 60, 16384x5120 34 / 37 / 42
+    against 34);
     wide heads of narrow models: 102400x1536 71 / 77 / 80 against 115,
     151936x2048 127 / 135 / 144 against 205, 200064x2560 220 / 236 / 260
     against 325 (128256x3072 135 / 150 / 173 against 146, 102400x1024 50 / 52 /
@@ -390,13 +391,19 @@ def _rows_tile_plan(M: int, N: int, K: int):
     182 / 254, 16384x2048 15.7 / 18.0, 65536x6144 144 / 178, 28672x8192
     85 / 129, but 51200x3072 72 / 62, 40960x5120 97 / 91, 22016x2560 31 / 30
     (18944 columns make 296 tiles, two for some CUs and one for most: 31 / 27
-    at 2560). At 96 rows: 16384x2048 18.3 / 18.8, 16384x4096 32 / 35,
-    65536x2048 60 / 70, 65536x4096 99 / 129, 51200x6144 137 / 147, 22016x8192
-    82 / 82, 128256x8192 372 / 416; rows of 5120, 3072 and 2560 lose (51200 of
-    each: 121 / 104, 73 / 68, 65 / 58), so do longer ones (51200x10240
-    224 / 200, 102400x12288 at 112 rows 557 / 504), 12288x4096 33 / 30, and
-    above 96 rows one and a bit rounds of tiles of long rows (40960x8192 at
-    128 160 / 154, where 40960x4096 is 86 / 87);
+    at 2560), and a fourth or fifth round of tiles of long rows (49152x8192
+    137 / 149, 57344x8192 172 / 161, 69632x8192 230 / 224, 86016x8192 249 / 295;
+    57344x6144 142 / 147).
+    At 96 rows: 16384x2048 18.3 / 18.8, 16384x4096 32 / 35, 65536x2048 60 / 70,
+    65536x4096 99 / 129, 51200x6144 137 / 147, 22016x8192 82 / 82, 128256x8192
+    372 / 416; rows of 5120, 3072 and 2560 lose (51200 of each: 121 / 104,
+    73 / 68, 65 / 58), so do longer ones (51200x10240 224 / 200, 102400x12288 at
+    112 rows 557 / 504) and 12288x4096 33 / 30. Tiles of 128 columns fill the
+    256 CUs in rounds, and one that is not nearly full loses on rows of more
+    than 4096 (73728x8192 302 / 279, 77824x6144 250 / 237, 143360x8192 at 80
+    rows 477 / 428), above 96 rows on rows of 4096 too, where it is the second
+    or third (at 128: 36864x4096 84 / 75, 77824x4096 166 / 153, 40960x8192
+    160 / 154).
     up to 16 rows: 28672x4096 40 / 43 at one and 41 / 53 at 16, 4096x11008
     17 / 31, 22016x4096 32 / 39, 128256x4096 175 / 178, but 16384x4096 at one
     row 27 / 26."""
@@ -412,10 +419,13 @@ def _rows_tile_plan(M: int, N: int, K: int):
                 M > 4 or N >= 22016 or K >= 11008)
                 or N >= 100000 and K >= 3072)
         elif M <= 64:
-            wins = K % 2048 == 0 and (K <= 8192 or N <= 32768)
+            wins = K % 2048 == 0 and (K <= 8192 or N <= 32768) and not (
+                K > 6144 and 768 < t64 <= 1280)
         else:
             wins = K % 2048 == 0 and K <= 8192 and N >= 16384 and not (
-                M > 96 and K > 4096 and 256 < t128 < 500)
+                M > 96 and (K > 4096 and 256 < t128 < 500 or K > 2048 and (
+                    256 < t128 < 300 or 512 < t128 < 768))
+                or K > 4096 and (512 < t128 < 768 or 1024 < t128 < 1280))
         plan = (128 if wide else 64), 1
     elif K <= 2048:
         wins = 16 < M <= 64 and (K == 1024 and N >= 2560
@@ -461,15 +471,15 @@ def router_plan(T: int, E: int, H: int):
 
 def linear_auto(x, w):
     """Shape-gated GEMM dispatch: the products for few rows
-    (_rows_tile_plan, _rows_gemm_wins), the split-K skinny kernel where it measured faster than
-    hipBLASLt (scripts/bench_skinny_gemm.py on MI355X: down_proj-like N=4096
-    K>=8192 M>=384 at splitk=4, 824 TF vs hipBLASLt 680), F.linear everywhere
-    else."""
+    (_rows_tile_plan, _rows_gemm_wins), the split-K skinny kernel where it
+    measured faster than hipBLASLt (scripts/bench_skinny_gemm.py on MI355X:
+    down_proj-like N=4096 K>=8192 M>=384 at splitk=4, 824 TF vs hipBLASLt 680),
+    F.linear everywhere else."""
     import os
 
     import torch.nn.functional as F
 
-    if (x.is_cuda and x.dim() == 2
+    if (x.is_cuda and x.dim() == 2 and w.dim() == 2
             and os.environ.get("GPUSTACK_AMD_SKINNY_GEMM", "1") == "1"):
         M, K = x.shape
         N = w.shape[0]

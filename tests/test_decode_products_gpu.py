@@ -155,3 +155,18 @@ def test_rule_of_tiles_for_many_columns(M, N, K, own):
     w = torch.randn(N, K, generator=g, device="cuda").bfloat16()
     _close(ops.linear_auto(x, w), x.double() @ w.double().T,
            x.double().abs() @ w.double().abs().T)
+
+
+@pytest.mark.parametrize("M,N,K,own", [
+    (17, 49152, 8192, True), (64, 49160, 8192, False),
+    (32, 81920, 8192, False), (32, 81928, 8192, True),
+    (48, 57344, 6144, True), (65, 65536, 6144, True),
+    (65, 65544, 6144, False), (96, 98176, 8192, False),
+    (96, 98304, 8192, True), (65, 131080, 8192, False),
+    (96, 73728, 4096, True), (97, 73728, 4096, False),
+    (97, 32896, 4096, False), (128, 38400, 4096, True),
+    (128, 73728, 2048, True)])
+def test_rule_of_tiles_by_rounds(M, N, K, own):
+    from gpustack_amd import ops
+
+    assert (ops._rows_tile_plan(M, N, K) is not None) == own
