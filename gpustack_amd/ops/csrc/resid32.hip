@@ -465,9 +465,9 @@ __global__ __launch_bounds__(ROW_THREADS) void moe_combine_vec_kernel(
 }
 
 // 16 waves a row with four loads in flight each: bound by how fast one CU
-// takes a row in (128 KB at a 32000-word vocabulary)
-constexpr int AM_THREADS = 1024;
-
+// takes a row in (128 KB at a 32000-word vocabulary). 4 waves up to 4096 words,
+// where waves without any are what is left (512 rows of 1000, us: 4.6 -> 3.3).
+template <int AM_THREADS>
 __global__ __launch_bounds__(AM_THREADS) void argmax_f32_kernel(
     long* __restrict__ out, const float* __restrict__ logits, int V) {
   __shared__ float bv[AM_THREADS / 64];
@@ -649,5 +649,6 @@ void moe_combine_launch(void* out, const void* y, const int* inv,
 void argmax_f32_launch(long* out, const float* logits, int N, int V,
                        hipStream_t s) {
   if (N == 0) return;
-  argmax_f32_kernel<<<N, AM_THREADS, 0, s>>>(out, logits, V);
+  if (V <= 4096) argmax_f32_kernel<256><<<N, 256, 0, s>>>(out, logits, V);
+  else argmax_f32_kernel<1024><<<N, 1024, 0, s>>>(out, logits, V);
 }
