@@ -447,9 +447,10 @@ void flash_prefill_launch(void* out, const void* q, const void* k,
 }
 
 // ---------------------------------------------------------------------------
-// MFMA layout probe: D = A[16x32] * B[32x16] with the fragment layouts this
-// file assumes. The GPU unit test checks it against torch.matmul with random
-// asymmetric inputs (guide G9: transpose-detecting correctness checks).
+// MFMA layout probe: D = A[16x32] * B[32x16] on the 16x16x32 form, with the
+// fragment layouts that decode attention and the products of few rows assume
+// (the 32x32x16 form above is checked by the attention itself). Random
+// asymmetric inputs against torch.matmul show a transposed fragment.
 // ---------------------------------------------------------------------------
 namespace {
 __global__ void mfma_probe_kernel(float* __restrict__ d,

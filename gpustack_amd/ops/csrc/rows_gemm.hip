@@ -7,8 +7,8 @@
 // partial results in memory and no second kernel. A weight row's 16-byte
 // chunks are the MFMA operand as they lie; one block of them is in flight while
 // the block before is multiplied. x comes from the L2.
-// Bound by the weight stream (2 bytes a weight): 28672 x 4096 at one row 45 us
-// (5.2 TB/s), 4096 x 4096 9.5, which is latency.
+// Bound by the weight stream (2 bytes a weight): 65536 x 4096 at one row 88 us
+// (6.1 TB/s), 4096 x 4096 9.5, which is latency.
 #include "common.h"
 
 namespace {
