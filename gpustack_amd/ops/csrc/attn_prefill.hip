@@ -1,9 +1,11 @@
 // Causal flash attention of prompt rows for MI355X (gfx950) on MFMA: whole
 // prompts (keys and values in the step's own rows) and rows behind a cached
-// history (keys and values in the paged pool), one kernel template.
+// history (keys and values in the paged pool): flash_prefill_kernel for all head
+// sizes and options, flash_rows_kernel for heads of 128 channels without options.
 //
 // Replaces the prefill attention the reference gets from vLLM/SGLang.
 //
+// Of the first:
 //  - a workgroup owns 128 query rows of one head, 4 waves x 32 rows, and
 //    walks the keys 64 at a time; mfma_f32_32x32x16_bf16, lane layouts
 //      A: lane holds A[row = l&31][k = (l>>5)*8 + j]
@@ -65,6 +67,42 @@ DEVICE_INLINE unsigned int pack_bf16(float lo, float hi) {
   const f32x2 v{lo, hi};
   return __builtin_bit_cast(unsigned int,
                             __builtin_convertvector(v, bf16x2));
+}
+
+// A wave's 32 rows of the result (o: channels 32 n + 8 rr + 4 (l>>5) .. of row
+// l & 31) through its own part of the LDS to whole rows: unit u (4 channels) of
+// row r at u ^ (r & 15).
+template <int DVK>
+DEVICE_INLINE void store_rows(unsigned short* __restrict__ out,
+                              unsigned short* ol, const f32x16 (&o)[DVK / 32],
+                              float inv, int row0, int first, int nnew, int Hq,
+                              int qh, int lane) {
+  constexpr int OC = DVK / 8;              // 16-byte chunks of an output row
+  const int lc = lane & 31, hf = lane >> 5;
+#pragma unroll
+  for (int n = 0; n < DVK / 32; ++n)
+#pragma unroll
+    for (int rr = 0; rr < 4; ++rr) {
+      u32x2 w;
+      w[0] = pack_bf16(o[n][rr * 4] * inv, o[n][rr * 4 + 1] * inv);
+      w[1] = pack_bf16(o[n][rr * 4 + 2] * inv, o[n][rr * 4 + 3] * inv);
+      const int unit = n * 8 + rr * 2 + hf;
+      *reinterpret_cast<u32x2*>(ol + lc * DVK + (unit ^ (lc & 15)) * 4) = w;
+    }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < OC / 2; ++i) {
+    const int u = lane + i * WAVE_SIZE;
+    const int r = u / OC, c = u % OC;
+    const u32x2 a = *reinterpret_cast<const u32x2*>(
+        ol + r * DVK + ((2 * c) ^ (r & 15)) * 4);
+    const u32x2 b = *reinterpret_cast<const u32x2*>(
+        ol + r * DVK + ((2 * c + 1) ^ (r & 15)) * 4);
+    if (first + r < nnew)
+      *reinterpret_cast<u32x4*>(
+          out + ((long)(row0 + first + r) * Hq + qh) * DVK + c * 8) =
+          u32x4{a[0], a[1], b[0], b[1]};
+  }
 }
 
 // EXT: 1 sinks / sliding window, 2 softcap (and those). Forms of their own,
@@ -339,35 +377,290 @@ void flash_prefill_kernel(
     }
   }
   const float inv = l > 0.f ? num / l : 0.f;
-  // through the LDS to whole rows: unit u (4 channels) of row r at
-  // u ^ (r & 15), each wave its own 32 rows
-  unsigned short* ol = lds + wave * 32 * DVK;
+  store_rows<DVK>(out, lds + wave * 32 * DVK, o, inv, row0, q0 + wave * 32, nnew,
+                  Hq, qh, lane);
+}
+
+// The same attention without options for heads of 128 channels: whole prompts
+// and rows behind a history.
+//  - keys and values go from memory into the LDS by themselves
+//    (global_load_lds, 16 bytes a lane), rows as they are: no staging registers,
+//    no LDS writes and no packing. Chunks are permuted through the lanes'
+//    addresses: 16-byte chunks of a key row XORed with the row, 64-byte chunks
+//    of a value row with row & 3. V^T comes out of the LDS by the transposing
+//    read (ds_read_b64_tr_b16: 16 lanes read 4 keys x 16 channels and get 4 keys
+//    of a channel each), conflict-free with that order.
+//  - the loads are inline asm: behind the builtin the compiler puts a wait for
+//    all of them in front of the next transposing read, that is one memory
+//    latency a tile. The waits are in `advance`.
+//  - a wave works on 32 keys at a time: the scores of the next 32 are
+//    multiplied while the exponentials of these 32 run, and the maximum of the
+//    next is taken beside the second product, so that the matrix cores need not
+//    wait for the softmax. For that the K buffer of tile j holds keys
+//    64 j + 32 .. 64 j + 95, and the first 32 keys are multiplied before the
+//    loop. Whole unmasked tiles run two to a turn without a branch but the
+//    rescaling one; the rest, masked, 32 keys to a turn.
+//  - scores stay unscaled; the factor is in the exponential's fma.
+// Bound by the LDS reads (32 KB a wave and tile, half of the LDS rate at
+// 1000 TFLOP/s) and the products: 32 heads on 8, one prompt of 7999 rows 638 ->
+// 480 us (822 -> 1091 TFLOP/s), 2039 rows behind 6001 301 -> 233 (1007), 32 x 256
+// 60 -> 52, 77 rows 8.8 -> 7.1, 33 rows behind 1000 38 -> 23, one row 5.7 -> 4.5.
+// Eight waves on 256 rows: 493 and 238. An order of the instructions given with
+// sched_group_barrier: 486 to 547.
+typedef __attribute__((ext_vector_type(4))) short s16x4;
+
+DEVICE_INLINE u32x2 lds_read_tr(const unsigned short* p) {
+  return __builtin_bit_cast(
+      u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                 (__attribute__((address_space(3))) s16x4*)p));
+}
+
+// 16 bytes a lane from base + off to LDS address `to` + 16 * lane
+DEVICE_INLINE void load_to_lds(const unsigned short* base, unsigned int off,
+                               const unsigned short* to) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(
+          (unsigned int)(unsigned long)(
+              const __attribute__((address_space(3))) unsigned short*)to),
+      "v"(off), "s"(base)
+      : "memory");
+}
+
+template <bool PAGED>
+__global__ __launch_bounds__(PF_THREADS, 2) void flash_rows_kernel(
+    unsigned short* __restrict__ out,      // [T, Hq, 128]
+    const unsigned short* __restrict__ q, const unsigned short* __restrict__ k,
+    const unsigned short* __restrict__ v,
+    const int* __restrict__ block_tables,  // [nseq, maxb]
+    const int* __restrict__ tile_start, const int* __restrict__ tile_q0,
+    const int* __restrict__ tile_hist, const int* __restrict__ tile_new,
+    const int* __restrict__ tile_seq, int Hq, int Hkv, int maxb, float scale,
+    long qs, long ks, long vs) {
+  constexpr int D = 128, QK = D / 16, NT = D / 32;
+  constexpr int TILE = BK * D;             // elements of a buffer
+  constexpr int RW = BK / PF_WAVES;        // rows of a tile a wave brings
+  constexpr int NI = RW / 4;               // instructions, 4 rows each
+  constexpr int HB = 32;                   // keys of a turn
+  static_assert(RW == PP_BS, "a wave brings one page");
+  __shared__ __attribute__((aligned(1024))) unsigned short lds[4 * TILE];
+
+  int qh = blockIdx.x % Hq;
+  if (Hq % 8 == 0) qh = (qh % 8) * (Hq / 8) + qh / 8;
+  const int tile = (gridDim.x - 1 - blockIdx.x) / Hq;
+  const int kvh = qh / (Hq / Hkv);
+  const int row0 = tile_start[tile];
+  const int q0 = tile_q0[tile];
+  if (q0 % BQ != 0) return;          // the second half of a list of 64-row tiles
+  const int hist = PAGED ? tile_hist[tile] : 0;
+  const int nnew = tile_new[tile];
+  const int len = hist + nnew;
+  const int* bt = PAGED ? block_tables + (long)tile_seq[tile] * maxb : nullptr;
+
+  const int lane = threadIdx.x & (WAVE_SIZE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
+  const int lc = lane & 31, hf = lane >> 5;
+
+  const int qrow = q0 + wave * 32 + lc;            // within the new rows
+  const int qpos = hist + qrow;
+  u32x4 qf[QK];
+  {
+    const unsigned short* qp =
+        q + (long)(row0 + min(qrow, nnew - 1)) * qs + (long)qh * D + hf * 8;
 #pragma unroll
-  for (int n = 0; n < NT; ++n)
-#pragma unroll
-    for (int rr = 0; rr < 4; ++rr) {
-      u32x2 w;
-      w[0] = pack_bf16(o[n][rr * 4] * inv, o[n][rr * 4 + 1] * inv);
-      w[1] = pack_bf16(o[n][rr * 4 + 2] * inv, o[n][rr * 4 + 3] * inv);
-      const int unit = n * 8 + rr * 2 + hf;
-      *reinterpret_cast<u32x2*>(ol + lc * DVK + (unit ^ (lc & 15)) * 4) = w;
-    }
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  constexpr int OC = DVK / 8;              // 16-byte chunks of an output row
-#pragma unroll
-  for (int i = 0; i < OC / 2; ++i) {
-    const int u = lane + i * WAVE_SIZE;
-    const int r = u / OC, c = u % OC;
-    const u32x2 a = *reinterpret_cast<const u32x2*>(
-        ol + r * DVK + ((2 * c) ^ (r & 15)) * 4);
-    const u32x2 b = *reinterpret_cast<const u32x2*>(
-        ol + r * DVK + ((2 * c + 1) ^ (r & 15)) * 4);
-    const int row = q0 + wave * 32 + r;
-    if (row < nnew)
-      *reinterpret_cast<u32x4*>(
-          out + ((long)(row0 + row) * Hq + qh) * DVK + c * 8) =
-          u32x4{a[0], a[1], b[0], b[1]};
+    for (int kk = 0; kk < QK; ++kk)
+      qf[kk] = *reinterpret_cast<const u32x4*>(qp + kk * 16);
   }
+
+  float m = -INFINITY, l = 0.f;                    // m in powers of two
+  f32x16 o[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[t][r] = 0.f;
+
+  const int lo_wave = hist + q0 + wave * 32;       // this wave's first row
+  const bool idle = q0 + wave * 32 >= nnew;        // it has none
+  const int kv_end = min(len, hist + q0 + BQ);     // causal bound
+  const int nt = (kv_end + BK - 1) / BK;
+  const float sc = scale * LOG2E;
+
+  // the lanes' byte offsets in a wave's RW rows
+  const int lr = lane >> 4, ch = lane & 15;
+  const int r0 = wave * RW;
+  const int kstep = PAGED ? D : (int)ks, vstep = PAGED ? D : (int)vs;
+  unsigned int koffs[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+    koffs[i] = (unsigned)((i * 4 + lr) * kstep +
+                          (ch ^ ((r0 + i * 4 + lr) & 15)) * 8) * 2;
+  const unsigned int voffs = (unsigned)(lr * vstep + (ch ^ (lr << 2)) * 8) * 2;
+  // keys (or values) key0 .. key0 + 63 into a buffer; rows behind the
+  // sequence's end repeat its last, rows in front of its start stay out
+  auto stage = [&](bool isk, int key0, unsigned short* to) {
+    const int kv0 = key0 + r0;
+    if (kv0 < 0) return;
+    const int at = min(kv0, len - 1);
+    const int step = isk ? kstep : vstep;
+    const unsigned short* base;
+    if constexpr (PAGED)
+      base = (isk ? k : v) +
+             (((long)bt[at / PP_BS] * Hkv + kvh) * PP_BS + at % PP_BS) * D;
+    else
+      base = (isk ? k + (long)(row0 + at) * ks : v + (long)(row0 + at) * vs) +
+             (long)kvh * D;
+    to += r0 * D;
+    if (kv0 + RW <= len) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+        load_to_lds(isk ? base : base + i * 4 * step, isk ? koffs[i] : voffs,
+                    to + i * 4 * D);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int row = i * 4 + lr;
+        const int c = isk ? ch ^ ((r0 + row) & 15) : ch ^ (lr << 2);
+        load_to_lds(base, (unsigned)(min(row, len - 1 - at) * step + c * 8) * 2,
+                    to + i * 4 * D);
+      }
+    }
+  };
+  auto kbuf = [&](int j) { return lds + (j & 1) * TILE; };
+  auto vbuf = [&](int j) { return lds + (2 + (j & 1)) * TILE; };
+
+  // LDS places of the operands: K chunk kk, V channels 32 n
+  const int koff = lc * D + ((hf ^ (lc & 15)) * 8);
+  const int vrow = (lane & 15) >> 2;               // and its row & 3
+  const int voff =
+      (4 * hf + vrow) * D + ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
+  const unsigned short *ka[QK], *va[NT];
+#pragma unroll
+  for (int i = 0; i < QK; ++i) ka[i] = lds + (koff ^ (i * 16));
+#pragma unroll
+  for (int i = 0; i < NT; ++i) va[i] = lds + 2 * TILE + voff + ((i ^ vrow) * 32);
+
+  auto scores = [&](int at, f32x16& s) {           // at: elements from ka
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] = 0.f;
+#pragma unroll
+    for (int kk = 0; kk < QK; ++kk)
+      s = mfma32x32x16_bf16(*reinterpret_cast<const u32x4*>(ka[kk] + at),
+                            qf[kk], s);
+  };
+  auto row_max = [&](const f32x16& s) {            // in powers of two
+    float x = fmaxf(fmaxf(s[0], s[1]), s[2]);
+#pragma unroll
+    for (int r = 3; r < 15; r += 2) x = fmaxf(fmaxf(x, s[r]), s[r + 1]);
+    x = fmaxf(x, s[15]);
+    const unsigned int u = __builtin_bit_cast(unsigned int, x);
+    const u32x2 w = __builtin_bit_cast(
+        u32x2, __builtin_amdgcn_permlane32_swap(u, u, false, false));
+    return fmaxf(__builtin_bit_cast(float, w[0]),
+                 __builtin_bit_cast(float, w[1])) * sc;
+  };
+  auto rescale = [&](float mx) {
+    if (__any(mx > m + SLACK)) {
+      const float nm = fmaxf(m, mx);
+      const float corr =
+          nm == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - nm);
+      m = nm;
+      l *= corr;
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[t][r] *= corr;
+    }
+    return m == -INFINITY ? 0.f : m;
+  };
+  auto weights = [&](const f32x16& s, u32x4 (&pf)[2], float base) {
+    float sum = 0.f;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const float a = __builtin_amdgcn_exp2f(
+            __builtin_fmaf(s[t * 8 + w * 2], sc, -base));
+        const float b = __builtin_amdgcn_exp2f(
+            __builtin_fmaf(s[t * 8 + w * 2 + 1], sc, -base));
+        sum += a + b;
+        pf[t][w] = pack_bf16(a, b);
+      }
+    l += sum;
+  };
+  auto weigh = [&](int at, const u32x4 (&pf)[2]) {  // at: elements from va
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int n = 0; n < NT; ++n) {
+        const unsigned short* p = va[n] + at + t * 16 * D;
+        const u32x2 a = lds_read_tr(p), b = lds_read_tr(p + 8 * D);
+        o[n] = mfma32x32x16_bf16(u32x4{a[0], a[1], b[0], b[1]}, pf[t], o[n]);
+      }
+  };
+  // Tile j is in the LDS for every wave, and every wave is done with tile
+  // j - 1, whose buffers tile j + 1 takes.
+  auto advance = [&](int j) {
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if ((j + 1) * BK + HB < kv_end) stage(true, (j + 1) * BK + HB, kbuf(j + 1));
+    if (j + 1 < nt) stage(false, (j + 1) * BK, vbuf(j + 1));
+  };
+
+  stage(true, HB - BK, kbuf(1));
+  if (HB < kv_end) stage(true, HB, kbuf(0));
+  stage(false, 0, vbuf(0));
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  f32x16 st;
+  scores(TILE + HB * D, st);
+
+  // whole tiles, which no row of the wave needs a mask for
+  const int full = idle ? 0 : min(nt - 1, (lo_wave + 1) / BK);
+  float mx = full > 1 ? row_max(st) : 0.f;
+  auto whole = [&](int j, int p) {                 // p = j & 1, a constant
+    advance(j);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const float base = rescale(mx);
+      f32x16 next;
+      u32x4 pf[2];
+      scores(p * TILE + h * HB * D, next);
+      weights(st, pf, base);
+      weigh(p * TILE + h * HB * D, pf);
+      st = next;
+      mx = row_max(st);
+    }
+  };
+  int j = 0;
+  for (; j + 1 < full; j += 2) {
+    whole(j, 0);
+    whole(j + 1, 1);
+  }
+  for (; j < nt; ++j) {
+    advance(j);
+#pragma unroll 1
+    for (int h = 0; h < 2; ++h) {
+      const int kv0 = j * BK + h * HB;
+      if (kv0 > lo_wave + 31 || kv0 >= kv_end || idle) break;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int kv = kv0 + 8 * (r >> 2) + 4 * hf + (r & 3);
+        st[r] = kv <= qpos && kv < len ? st[r] : -INFINITY;
+      }
+      const float base = rescale(row_max(st));
+      const int at = (j & 1) * TILE + h * HB * D;
+      u32x4 pf[2];
+      weights(st, pf, base);
+      if (kv0 + HB < kv_end) scores(at, st);
+      weigh(at, pf);
+    }
+  }
+  __syncthreads();
+
+  l += __shfl_xor(l, 32, WAVE_SIZE);
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  store_rows<D>(out, lds + wave * 32 * D, o, inv, row0, q0 + wave * 32, nnew, Hq,
+                qh, lane);
 }
 
 template <int D, int DVK, int EXT, bool PAGED>
@@ -377,6 +670,23 @@ void launch(void* out, const void* q, const void* k, const void* v,
             int maxb, float scale, long qs, long ks, long vs,
             const float* sinks, int window, float softcap, hipStream_t s) {
   if (ntiles == 0) return;
+  // Rows that the loads to the LDS can take: aligned to them, offsets within 32
+  // bits; and a factor that a maximum of unscaled scores may be taken under.
+  // It was the faster one at every size measured (above).
+  if constexpr (D == 128 && DVK == 128 && EXT == 0) {
+    const unsigned long at = (unsigned long)k | (unsigned long)v |
+                             (unsigned long)(ks * 2) | (unsigned long)(vs * 2);
+    constexpr long FAR = 1l << 24;
+    if (at % 16 == 0 && ks >= 0 && vs >= 0 && ks < FAR && vs < FAR &&
+        scale > 0.f) {
+      hipLaunchKernelGGL((flash_rows_kernel<PAGED>), dim3((unsigned)ntiles * Hq),
+                         dim3(PF_THREADS), 0, s, (unsigned short*)out,
+                         (const unsigned short*)q, (const unsigned short*)k,
+                         (const unsigned short*)v, bt, start, q0, hist, nnew,
+                         seq, Hq, Hkv, maxb, scale, qs, ks, vs);
+      return;
+    }
+  }
   hipLaunchKernelGGL((flash_prefill_kernel<D, DVK, EXT, PAGED>),
                      dim3((unsigned)ntiles * Hq), dim3(PF_THREADS), 0, s,
                      (unsigned short*)out, (const unsigned short*)q,

@@ -111,6 +111,29 @@ def test_tile_lists_of_either_size(rows):
         at += n
 
 
+@pytest.mark.parametrize("pad,scale", [(0, 0.1), (8, 0.1), (4, 0.1), (1, 0.1),
+                                       (0, -0.1), (0, 0.0)])
+def test_rows_and_factors_of_either_kernel(pad, scale):
+    """Key and value rows at 16-byte addresses or not, and factors under which
+    the largest unscaled score is not the largest one."""
+    from gpustack_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(pad)
+    lens, Hq, Hkv = [1, 95, 96, 97, 385], 8, 2
+    qkv = torch.randn(sum(lens), (Hq + 2 * Hkv) * 128 + pad, generator=g,
+                      device="cuda").bfloat16()
+    q, k, v = (qkv[:, pad + a * 128:pad + b * 128].unflatten(1, (b - a, 128))
+               for a, b in ((0, Hq), (Hq, Hq + Hkv), (Hq + Hkv, Hq + 2 * Hkv)))
+    q = (q * 3).contiguous()
+    out = torch.full((sum(lens), Hq, 128), 9.0, device="cuda").bfloat16()
+    ops.varlen_prefill_attn(out, q, k, v, lens, scale)
+    at = 0
+    for n in lens:
+        _check(out[at:at + n], q[at:at + n], k[at:at + n], v[at:at + n], 0,
+               scale)
+        at += n
+
+
 def _check_variant(out, q, k, v, hist, scale, sinks, window, softcap):
     """out [n, Hq, DV], q [n, Hq, D] of one sequence, k / v [hist + n, G, .]"""
     n, Hq, _ = q.shape
