@@ -4,6 +4,7 @@ from __future__ import annotations
 
 import os
 
+import numpy as np
 import torch
 
 from .. import ops
@@ -552,12 +553,10 @@ class ModelRunner:
         )
         return tokens, meta
 
-    def _ragged_meta(self, batch: ScheduledBatch, positions) -> "RaggedMeta":
+    def _ragged_meta(self, batch: ScheduledBatch) -> "RaggedMeta":
         """The per-sequence (first row, cached tokens, rows) view of any
         batch kind plus each row's previous token (RaggedMeta)."""
         from ..models.llama import RaggedMeta
-
-        import numpy as np
 
         dev = self.device
         pos = np.asarray(batch.positions, dtype=np.int64)
@@ -580,35 +579,33 @@ class ModelRunner:
         row_seq = np.repeat(np.arange(len(news), dtype=np.int32), news)
         starts, hists = starts.tolist(), hists.tolist()
         maxb = max(len(s.block_table) for s in batch.seqs)
-        bt = torch.zeros(len(batch.seqs), maxb, dtype=torch.int32)
+        bt = np.zeros((len(batch.seqs), maxb), dtype=np.int32)
         for i, s in enumerate(batch.seqs):
-            bt[i, : len(s.block_table)] = torch.tensor(s.block_table,
-                                                       dtype=torch.int32)
-        rg = RaggedMeta(
-            block_tables=bt.to(dev),
-            row_seq=torch.from_numpy(row_seq).to(dev),
-            pos32=positions.to(torch.int32),
-            prev_tokens=torch.from_numpy(prev).to(dev),
-            seq_starts=starts, seq_hists=hists, seq_news=news,
-            max_ctx=max(h + n for h, n in zip(hists, news)))
-        if self.kv is not None and self.kv.state_allocator is not None:
+            bt[i, : len(s.block_table)] = s.block_table
+        i32 = torch.int32
+        parts = [(bt, i32), (row_seq, i32), (pos, i32), (prev, torch.long)]
+        slots = self.kv is not None and self.kv.state_allocator is not None
+        if slots:
             if any(s.state_slot < 0 for s in batch.seqs):
                 raise RuntimeError("a scheduled sequence holds no state slot")
-            per_seq = np.asarray(
-                [starts, news, [s.state_slot for s in batch.seqs]],
-                dtype=np.int32)
-            per_seq = torch.from_numpy(per_seq).to(dev)
-            rg.seq_first, rg.seq_rows, rg.state_slots = (
-                per_seq[0], per_seq[1], per_seq[2])
+            parts.append((np.asarray(
+                [starts, news, [s.state_slot for s in batch.seqs]]), i32))
+        up = ops.to_device(parts, dev)
+        rg = RaggedMeta(
+            block_tables=up[0], row_seq=up[1], pos32=up[2], prev_tokens=up[3],
+            seq_starts=starts, seq_hists=hists, seq_news=news,
+            max_ctx=max(h + n for h, n in zip(hists, news)))
+        if slots:
+            rg.seq_first, rg.seq_rows, rg.state_slots = up[4].unbind(0)
         return rg
 
     def _meta(self, batch: ScheduledBatch) -> tuple[torch.Tensor, ForwardMeta]:
         tokens, meta = self._meta_by_kind(batch)
         if batch.logit_rows is not None:
-            meta.logits_indices = torch.tensor(
-                batch.logit_rows, dtype=torch.long, device=self.device)
+            meta.logits_indices = ops.to_device(
+                [(batch.logit_rows, torch.long)], self.device)[0]
         if self.ragged:
-            meta.ragged = self._ragged_meta(batch, meta.positions)
+            meta.ragged = self._ragged_meta(batch)
         return tokens, meta
 
     @torch.inference_mode()
@@ -628,9 +625,21 @@ class ModelRunner:
         if self._cp_splittable(batch):
             return self._meta_cp(batch)
         dev = self.device
-        tokens = torch.as_tensor(batch.token_ids, dtype=torch.long).to(dev)
-        positions = torch.as_tensor(batch.positions, dtype=torch.long).to(dev)
-        slots = torch.as_tensor(batch.slot_mapping, dtype=torch.long).to(dev)
+        i32, i64 = torch.int32, torch.long
+        # what every kind of step has; each adds its own, all in one copy
+        parts = [(batch.token_ids, i64), (batch.positions, i64),
+                 (batch.slot_mapping, i64)]
+
+        def table(seqs, repeat=lambda i: 1):
+            bt = np.zeros((sum(repeat(i) for i in range(len(seqs))),
+                           max(len(s.block_table) for s in seqs)), np.int32)
+            r = 0
+            for i, s in enumerate(seqs):
+                n = repeat(i)
+                bt[r:r + n, : len(s.block_table)] = s.block_table
+                r += n
+            return bt
+
         if batch.is_prefill:
             # last token of each prefill sequence produces its logits row
             n_pre = batch.n_prefill_seqs or len(batch.seqs)
@@ -643,34 +652,26 @@ class ModelRunner:
             n_dec = len(batch.seqs) - n_pre
             # decode rows (mixed batch) produce logits directly
             idx.extend(range(tp, tp + n_dec))
-            tiles = ops.build_prefill_tiles(pre_lens, dev, ops.PREFILL_ROWS)
-            bt = None
-            dec_lens = None
-            if self.cfg.spec.kv_lora_rank and dev.type == "cuda":
+            parts += [(idx, i64)] + [
+                (a, i32) for a in ops.prefill_tile_rows(pre_lens,
+                                                        ops.PREFILL_ROWS)]
+            if n_dec:
+                parts += [(table(batch.seqs[n_pre:]), i32),
+                          (batch.decode_seq_lens, i32)]
+            elif self.cfg.spec.kv_lora_rank and dev.type == "cuda":
                 # MLA gated GPU path: the absorbed kernel reads the latent
                 # through per-seq block tables even for prefill rows
-                maxb_p = max(len(s.block_table) for s in batch.seqs[:n_pre])
-                btp = torch.zeros(n_pre, maxb_p, dtype=torch.int32)
-                for i, sq in enumerate(batch.seqs[:n_pre]):
-                    btp[i, : len(sq.block_table)] = torch.tensor(
-                        sq.block_table, dtype=torch.int32)
-                bt = btp.to(dev)
-            if n_dec:
-                maxb = max(len(s.block_table) for s in batch.seqs[n_pre:])
-                btc = torch.zeros(n_dec, maxb, dtype=torch.int32)
-                for i, s in enumerate(batch.seqs[n_pre:]):
-                    btc[i, : len(s.block_table)] = torch.tensor(s.block_table, dtype=torch.int32)
-                bt = btc.to(dev)
-                dec_lens = torch.tensor(batch.decode_seq_lens, dtype=torch.int32, device=dev)
+                parts.append((table(batch.seqs[:n_pre]), i32))
+            tokens, positions, slots, idx, *own = ops.to_device(parts, dev)
             meta = ForwardMeta(
                 is_prefill=True,
                 positions=positions,
                 slot_mapping=slots,
-                logits_indices=torch.tensor(idx, dtype=torch.long, device=dev),
+                logits_indices=idx,
                 seq_lens_list=pre_lens,
-                tile_start=tiles[0], tile_q0=tiles[1], tile_len=tiles[2],
-                block_tables=bt,
-                seq_lens=dec_lens,
+                tile_start=own[0], tile_q0=own[1], tile_len=own[2],
+                block_tables=own[3] if len(own) > 3 else None,
+                seq_lens=own[4] if len(own) > 4 else None,
                 num_prefill_tokens=tp,
             )
         elif batch.is_suffix:
@@ -696,59 +697,47 @@ class ModelRunner:
             else:  # torch_ref path handles any dtype/head_dim except fp8
                 use_pp = (self.kv is not None
                           and self.kv.kv_dtype != torch.float8_e4m3fn)
+            parts.append((idx, i64))
             if use_pp:
-                maxb = max(len(s.block_table) for s in batch.seqs)
-                bt = torch.zeros(len(batch.seqs), maxb, dtype=torch.int32)
-                for i, s in enumerate(batch.seqs):
-                    bt[i, : len(s.block_table)] = torch.tensor(
-                        s.block_table, dtype=torch.int32)
-                tiles = ops.build_paged_prefill_tiles(starts, hists, news, dev,
-                                                  ops.PREFILL_ROWS)
+                parts += [(table(batch.seqs), i32)] + [
+                    (a, i32) for a in ops.paged_prefill_tile_rows(
+                        starts, hists, news, ops.PREFILL_ROWS)]
+                tokens, positions, slots, idx, bt, *tiles = ops.to_device(
+                    parts, dev)
                 meta = ForwardMeta(
                     is_prefill=False,
                     positions=positions,
                     slot_mapping=slots,
-                    logits_indices=torch.tensor(idx, dtype=torch.long,
-                                                device=dev),
-                    block_tables=bt.to(dev),
-                    suffix_meta=(tiles, starts, hists, news),
+                    logits_indices=idx,
+                    block_tables=bt,
+                    suffix_meta=(tuple(tiles), starts, hists, news),
                 )
             else:
-                nrows = sum(batch.suffix_rows)
-                maxb = max(len(s.block_table) for s in batch.seqs)
-                bt = torch.zeros(nrows, maxb, dtype=torch.int32)
-                r = 0
-                for s, nr in zip(batch.seqs, batch.suffix_rows):
-                    row = torch.tensor(s.block_table, dtype=torch.int32)
-                    for _ in range(nr):
-                        bt[r, : len(s.block_table)] = row
-                        r += 1
+                parts += [(table(batch.seqs, lambda i: news[i]), i32),
+                          (batch.seq_lens, i32)]
+                tokens, positions, slots, idx, bt, lens = ops.to_device(
+                    parts, dev)
                 meta = ForwardMeta(
                     is_prefill=False,
                     positions=positions,
                     slot_mapping=slots,
-                    logits_indices=torch.tensor(idx, dtype=torch.long,
-                                                device=dev),
-                    block_tables=bt.to(dev),
-                    seq_lens=torch.tensor(batch.seq_lens, dtype=torch.int32,
-                                          device=dev),
+                    logits_indices=idx,
+                    block_tables=bt,
+                    seq_lens=lens,
                 )
         else:
             rps = batch.rows_per_seq
-            nrows = len(batch.seqs) * rps
-            maxb = max(len(s.block_table) for s in batch.seqs)
-            bt = torch.zeros(nrows, maxb, dtype=torch.int32)
-            for i, s in enumerate(batch.seqs):
-                row = torch.tensor(s.block_table, dtype=torch.int32)
-                for j in range(rps):
-                    bt[i * rps + j, : len(s.block_table)] = row
+            parts += [(table(batch.seqs, lambda i: rps), i32),
+                      (batch.seq_lens, i32)]
+            tokens, positions, slots, bt, lens = ops.to_device(parts, dev)
             meta = ForwardMeta(
                 is_prefill=False,
                 positions=positions,
                 slot_mapping=slots,
-                logits_indices=torch.arange(nrows, dtype=torch.long, device=dev),
-                block_tables=bt.to(dev),
-                seq_lens=torch.tensor(batch.seq_lens, dtype=torch.int32, device=dev),
+                logits_indices=torch.arange(len(batch.seqs) * rps,
+                                            dtype=torch.long, device=dev),
+                block_tables=bt,
+                seq_lens=lens,
             )
         slots = self._row_lora_slots(batch)
         if slots is not None:

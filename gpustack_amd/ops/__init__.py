@@ -52,6 +52,37 @@ def hip_available() -> bool:
         return False
 
 
+def to_device(parts, device) -> list[torch.Tensor]:
+    """Host integers on the device: `parts` is a list of (values, dtype), values
+    a list of ints, an array or a CPU tensor. On a GPU they go through pinned
+    memory in ONE copy that waits for nothing, so that the host can prepare a
+    step while the GPU works on the one before (torch's copies from ordinary
+    memory wait for the stream, each of them)."""
+    import array
+
+    import numpy as np
+
+    host = []
+    for v, dtype in parts:
+        if isinstance(v, list) and v and isinstance(v[0], int):
+            v = np.frombuffer(array.array("q", v), dtype=np.int64)
+        host.append(torch.as_tensor(v, dtype=dtype))
+    device = torch.device(device)
+    if device.type != "cuda":
+        return [t.to(device) for t in host]
+    at, n = [], 0
+    for t in host:                       # 16-byte places
+        at.append(n)
+        n += (t.numel() * t.element_size() + 15) // 16 * 16
+    pin = torch.empty(max(n, 16), dtype=torch.uint8, pin_memory=True)
+    part = lambda buf, t, o: buf[o:o + t.numel() * t.element_size()] \
+        .view(t.dtype).view(t.shape)
+    for t, o in zip(host, at):
+        part(pin, t, o).copy_(t)
+    dev = pin.to(device, non_blocking=True)
+    return [part(dev, t, o) for t, o in zip(host, at)]
+
+
 def _products():
     """The main library, or None in a checkout without it: the models that
     come with libraries of their own run there on the library's products."""
@@ -222,6 +253,13 @@ def build_prefill_tiles(seq_lens: list[int], device,
                         rows: int = _PREFILL_BQ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """Map varlen sequences to q tiles of `rows` (64 or PREFILL_ROWS) for the
     MFMA kernel."""
+    return tuple(to_device([(a, torch.int32) for a in
+                            prefill_tile_rows(seq_lens, rows)], device))
+
+
+def prefill_tile_rows(seq_lens: list[int], rows: int = _PREFILL_BQ):
+    """The lists of build_prefill_tiles: each tile's sequence's first row, its
+    own first row in the sequence, the sequence's length."""
     starts, q0s, lens = [], [], []
     tok = 0
     for L in seq_lens:
@@ -230,8 +268,7 @@ def build_prefill_tiles(seq_lens: list[int], device,
             q0s.append(q0)
             lens.append(L)
         tok += L
-    mk = lambda a: torch.tensor(a, dtype=torch.int32, device=device)
-    return mk(starts), mk(q0s), mk(lens)
+    return starts, q0s, lens
 
 
 def varlen_prefill_attn(out, q, k, v, seq_lens: list[int], scale: float,
@@ -264,6 +301,14 @@ def build_paged_prefill_tiles(seq_starts: list[int], seq_hists: list[int],
                               rows: int = _PREFILL_BQ):
     """Map per-seq suffix rows to q tiles of `rows` (64 or PREFILL_ROWS) for
     the paged prefill-with-history kernel (one entry set per (seq, q-tile))."""
+    return tuple(to_device([(a, torch.int32) for a in paged_prefill_tile_rows(
+        seq_starts, seq_hists, seq_news, rows)], device))
+
+
+def paged_prefill_tile_rows(seq_starts: list[int], seq_hists: list[int],
+                            seq_news: list[int], rows: int = _PREFILL_BQ):
+    """The lists of build_paged_prefill_tiles: each tile's sequence's first
+    row, its own first row there, cached tokens, new rows, sequence."""
     qstart, q0s, hists, news, seqi = [], [], [], [], []
     for i, (st, h, n) in enumerate(zip(seq_starts, seq_hists, seq_news)):
         for q0 in range(0, n, rows):
@@ -272,8 +317,7 @@ def build_paged_prefill_tiles(seq_starts: list[int], seq_hists: list[int],
             hists.append(h)
             news.append(n)
             seqi.append(i)
-    mk = lambda a: torch.tensor(a, dtype=torch.int32, device=device)
-    return mk(qstart), mk(q0s), mk(hists), mk(news), mk(seqi)
+    return qstart, q0s, hists, news, seqi
 
 
 def paged_prefill_attn(out, q, k_cache, v_cache, block_tables,
@@ -644,7 +688,7 @@ def build_latent_tiles(seq_starts, seq_hists, seq_news, heads: int, device):
         parts.append(t)
     tiles = (np.concatenate(parts) if parts
              else np.empty((0, 6), dtype=np.int32))
-    return torch.from_numpy(tiles).to(device)
+    return to_device([(tiles, torch.int32)], device)[0]
 
 
 def latent_attention_mfma_ok(cache) -> bool:
@@ -781,7 +825,7 @@ def build_page_groups(seq_starts, seq_hists, seq_news, block_size: int,
         hi = np.minimum(first + block_size, hist + new)
         parts.append(np.stack([st + lo - hist, hi - lo], axis=1))
     g = (np.concatenate(parts) if parts else np.empty((0, 2))).astype(np.int32)
-    return torch.from_numpy(g).to(device)
+    return to_device([(g, torch.int32)], device)[0]
 
 
 def rotary_norm_store(q_out, qkv, nq: int, nk: int, q_norm_w, k_norm_w,
@@ -843,7 +887,7 @@ def build_attn_tiles(seq_starts, seq_hists, seq_news, heads: int,
         parts.append(t)
     tiles = (np.concatenate(parts) if parts
              else np.empty((0, 6), dtype=np.int32))
-    return torch.from_numpy(tiles).to(device)
+    return to_device([(tiles, torch.int32)], device)[0]
 
 
 def paged_attention(out, q, k_cache, v_cache, block_tables, row_seq, positions,
@@ -1219,7 +1263,7 @@ def build_scan_chunks(seq_starts, seq_news, size: int, device):
         n += lo.size
         parts.append(t)
     c = np.concatenate(parts) if parts else np.empty((0, 4), dtype=np.int32)
-    return torch.from_numpy(c).to(device)
+    return to_device([(c, torch.int32)], device)[0]
 
 
 def gru_scan(y, src, col_z: int, col_u: int, col_g: int, z_b, u_b, state,
