@@ -30,7 +30,7 @@ void moe_route_launch(int*, float*, const void*, const void*, int, int, int, int
 int moe_sort_slices(int);
 void moe_sort_launch(int*, int*, int*, int*, int*, int*, int*, const int*, int, int, int, int*, hipStream_t);
 void moe_sum_launch(void*, const void*, long, int, int, hipStream_t);
-void moe_tile_launch(int, void*, const void*, const void*, const int*, const int*, const int*, const int*, const int*, const float*, const void*, int, int, int, int, int*, hipStream_t);
+void moe_tile_launch(int, void*, const void*, const void*, const int*, const int*, const int*, const int*, const int*, const float*, const void*, int, long, int, int, int, int*, hipStream_t);
 void rows_tile_launch(void*, void*, const void*, const void*, int, int, int, long, int, int, int*, hipStream_t);
 void rows_gemm_launch(void*, const void*, const void*, int, int, int, long, int*, hipStream_t);
 void w4_gemm_launch(void*, const void*, const void*, const void*, const void*, int, int, int, int*, hipStream_t);
@@ -487,7 +487,7 @@ void moe_tile(bool down, at::Tensor out, at::Tensor src, at::Tensor w,
   moe_tile_launch(down ? 1 : 0, out.data_ptr(), src.data_ptr(), w.data_ptr(),
                   rows.data_ptr<int>(), tiles.data_ptr<int>(),
                   ntiles.data_ptr<int>(), offs.data_ptr<int>(),
-                  counts.data_ptr<int>(), fw, bias_ptr, (int)act_mode,
+                  counts.data_ptr<int>(), fw, bias_ptr, (int)act_mode, src.size(0),
                   (int)(out.size(0) / 128 + E), (int)N, K, &err,
                   cur_stream(src));
   TORCH_CHECK(!err, "moe_tile: unsupported dims N=", N, " K=", K);

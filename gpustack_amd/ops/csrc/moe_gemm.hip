@@ -15,11 +15,13 @@
 // Launch grids do not depend on the routing outcome: workgroups without a tile
 // exit. Both products run in 128 x 128 tiles (below), from a few rows per
 // expert, where they are bound by the weight stream (128 experts x 1536 x 2048
-// at 64 rows: 146 us, 5.5 TB/s), to whole prompts. The down product has a
+// at 64 rows: 147 us, 5.5 TB/s), to whole prompts. The down product has a
 // second form for few workgroups of long rows (moe_down_scale, 64 columns):
 // 16-row MFMA 16x16x32 tiles, A staged through LDS in 512-element K chunks, B
 // streamed from HBM, once per 16 rows.
 #include "common.h"
+
+#include <type_traits>
 
 namespace {
 
@@ -130,25 +132,34 @@ __global__ __launch_bounds__(MOE_THREADS) void moe_down_scale_kernel(
 // Tile form. A tile is 128 rows of one expert x 128 weight rows (of gate and
 // up: 64 each, 32 + 32 beside each other per wave, so that a lane holds a
 // column's gate and up), four waves of 64 x 64 on mfma_f32_32x32x16_bf16, K in
-// steps of 64 through two LDS buffers that global_load_lds fills 16 bytes a
-// lane (the next step's loads fly under this step's products, one barrier a
-// step; 64 KB, two workgroups a CU). 16-byte chunks are XORed with (row >> 1):
-// eight chunks a row, conflict-free over 16 rows of one chunk. Weights are the
-// A operand: a lane ends with 4 neighbouring columns of a row, which go
-// through the LDS to whole 16-byte stores.
+// steps of 64 through LDS buffers that global_load_lds fills 16 bytes a lane,
+// one barrier a step: two for the rows, which come out of the L2 a step ahead,
+// three for the weights, which come out of memory two steps ahead (80 KB, two
+// workgroups a CU). 16-byte chunks are XORed with (row >> 1): eight chunks a
+// row, conflict-free over 16 rows of one chunk. Weights are the A operand: a
+// lane ends with 4 neighbouring columns of a row, which go through the LDS to
+// whole 16-byte stores.
 // The tile list (moe_sort) holds only tiles that exist; workgroups are dealt to
 // the XCDs in runs, and the tiles of an expert that share weight rows follow
 // each other, so that these are read once into one L2 (tile by tile instead,
 // 8 experts of 4096 x 14336 at 1024 rows each read 17 GB past the L2 and ran
 // at 597 TFLOP/s). Halves of a wave's rows that an expert does not fill are
-// not multiplied (64 rows over 128 experts: 146 us, as the weights take).
-// Bound by the products and the weight stream alike: 256 rows per expert of
-// 128 x (1536 + 768) x 2048 are 0.31 TFLOP and 1.2 GB a layer, 313 + 200 us
-// (658 and 516 TFLOP/s; 8 experts at 1024 rows: 840 and 762). Steps of 32 through a ring of five buffers, four of
-// them in flight, took 368 + 225: the LDS reads of 64 x 64 wave tiles and the
-// barriers set the pace, not the loads.
+// not multiplied: three forms of the loop, without a branch inside, so that a
+// 16-k's LDS reads fly under the products before it.
+// The loads are inline asm, because the compiler would wait for all of them in
+// front of LDS reads that it cannot tell from them; the weights' first ones leave before the tile's rows are known,
+// and what the end needs of the routing is read before the loop.
+// Bound by the products and the weight stream alike: 254 rows per expert of
+// 128 x (1536 + 768) x 2048 are 0.31 TFLOP and 1.2 GB a layer, 282 + 172 us (727
+// and 596 TFLOP/s; with two buffers of each, branches between the products and
+// the routing read at the end 312 + 198), 62 rows 155 + 96 (162 + 100), 4 rows
+// 147 + 76 (150 + 76); 8 experts of 4096 x 14336 at 256 rows 636 + 407 (720 +
+// 542). Tiles of 256 weight rows by eight waves, three buffers of each, one
+// workgroup a CU: 278 to 286 + 176 to 179; of 256 in steps of 32: 291 to 312 +
+// 181. Steps of 32 of 128 x 128 through three buffers: 322 to 330 + 187.
 // ---------------------------------------------------------------------------
 constexpr int MT_M = 128, MT_N = 128, MT_K = 64;
+constexpr int MT_WB = 3;                     // weight buffers
 
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
@@ -158,7 +169,23 @@ DEVICE_INLINE unsigned int moe_pack(float lo, float hi) {
   return __builtin_bit_cast(unsigned int, __builtin_convertvector(v, bf16x2));
 }
 
-template <bool DOWN, bool EXTM>
+// 16 bytes a lane to LDS address `to` + 16 * lane: from base + off, or from at
+DEVICE_INLINE unsigned int moe_lds(const unsigned short* p) {
+  return (unsigned int)(unsigned long)(
+      const __attribute__((address_space(3))) unsigned short*)p;
+}
+DEVICE_INLINE void moe_load(const unsigned short* base, unsigned int off,
+                            const unsigned short* to) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               ::"s"(moe_lds(to)), "v"(off), "s"(base) : "memory");
+}
+DEVICE_INLINE void moe_load(const unsigned short* at, const unsigned short* to) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+               ::"s"(moe_lds(to)), "v"(at) : "memory");
+}
+
+// FAR: rows of `src` lie further than 32 bits of bytes from its start.
+template <bool DOWN, bool EXTM, bool FAR>
 __global__ __launch_bounds__(MOE_THREADS, 2) void moe_tile_kernel(
     unsigned short* __restrict__ out,        // act [TK, I] | contrib [TK, H]
     const unsigned short* __restrict__ src,  // x [T, H] | act [TK, I]
@@ -170,10 +197,14 @@ __global__ __launch_bounds__(MOE_THREADS, 2) void moe_tile_kernel(
     const float* __restrict__ flat_w,        // DOWN: [TK] routing weights
     const unsigned short* __restrict__ bias, // [E, 2I] | [E, H] or null
     int act_mode, int N, int K) {            // N = I | H
-  constexpr int BUF = (MT_M + MT_N) * MT_K;  // elements of a buffer
-  __shared__ __attribute__((aligned(16))) unsigned short lds[2 * BUF];
+  constexpr int BUF = MT_M * MT_K;           // elements of a buffer
+  static_assert(MT_M == MT_N, "rows and weights share their layout");
+  // rows' buffers, then the weights'
+  __shared__ __attribute__((aligned(16))) unsigned short lds[(2 + MT_WB) * BUF];
+  constexpr int OW = DOWN ? MT_N : MT_N / 2; // columns of the result
+  constexpr int NI = MT_M / 8 / 4;           // loads of a wave, 8 rows each
 
-  const int nnt = N / (DOWN ? MT_N : MT_N / 2);
+  const int nnt = N / OW;
   const int nwg = ntiles[0] * nnt;
   int wg = blockIdx.x;
   if (wg >= nwg) return;
@@ -195,41 +226,63 @@ __global__ __launch_bounds__(MOE_THREADS, 2) void moe_tile_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE_SIZE);
   const int wm = wave >> 1, wn = wave & 1;
   const int lc = lane & 31, hf = lane >> 5;
-  const int mine = nrows - wm * 64;          // rows of this wave's half
 
-  // staging: a wave instruction fills 8 rows of 128 bytes; instruction i of
-  // wave w takes rows (i * 4 + w) * 8 ..
-  const unsigned short* ap[4];
-  const unsigned short* bp[4];
+  // A wave's load i brings rows (i * 4 + wave) * 8 .. of 128 bytes. Of gate and
+  // up, 32 rows of one and 32 of the other take turns: a load is of one of them.
+  const int nk = K / MT_K;
+  const unsigned short* wbase =
+      w + ((long)e * (DOWN ? N : 2 * N) + nt * OW) * K;
+  unsigned int woff[NI];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < NI; ++i) {
     const int row = (i * 4 + wave) * 8 + lane / 8;
     const int chunk = (lane & 7) ^ ((row >> 1) & 7);
-    const int at = first + min(row, nrows - 1);
-    const long arow = DOWN ? (long)at : (long)rows[at];
-    ap[i] = src + arow * K + chunk * 8;
-    long brow;
-    if constexpr (DOWN) {
-      brow = (long)e * N + nt * MT_N + row;
-    } else {
-      const int col = nt * 64 + (row >> 6) * 32 + (row & 31);
-      brow = (long)e * 2 * N + ((row & 32) ? N : 0) + col;
-    }
-    bp[i] = w + brow * K + chunk * 8;
+    const int col = DOWN ? row : (row >> 6) * 32 + (row & 31);
+    woff[i] = ((unsigned)col * K + chunk * 8) * 2;
   }
-  auto stage = [&](int buf, int k0) {
+  auto load_weights = [&](int kt) {
+    unsigned short* to = lds + (2 + kt % MT_WB) * BUF + wave * 8 * MT_K;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      unsigned short* d = lds + buf * BUF + (i * 4 + wave) * 8 * MT_K;
-      __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) unsigned int*)(ap[i] + k0),
-          (__attribute__((address_space(3))) unsigned int*)d, 16, 0, 0);
-      __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) unsigned int*)(bp[i] + k0),
-          (__attribute__((address_space(3))) unsigned int*)(d + MT_M * MT_K),
-          16, 0, 0);
+    for (int i = 0; i < NI; ++i)
+      moe_load(wbase + (DOWN ? 0 : (long)(i & 1) * N * K) + kt * MT_K, woff[i],
+               to + i * 32 * MT_K);
+  };
+  load_weights(0);
+  const unsigned short* rbase = DOWN ? src + (long)first * K : src;
+  std::conditional_t<FAR, unsigned long, unsigned int> roff[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int row = (i * 4 + wave) * 8 + lane / 8;
+    const int chunk = (lane & 7) ^ ((row >> 1) & 7);
+    const int at = min(row, nrows - 1);
+    roff[i] = DOWN ? at : rows[first + at];
+    roff[i] = (roff[i] * K + chunk * 8) * 2;
+  }
+  auto load_rows = [&](int kt) {
+    unsigned short* to = lds + (kt & 1) * BUF + wave * 8 * MT_K;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      if constexpr (FAR)
+        moe_load(rbase + roff[i] / 2 + kt * MT_K, to + i * 32 * MT_K);
+      else
+        moe_load(rbase + kt * MT_K, roff[i], to + i * 32 * MT_K);
     }
   };
+  // what the end needs of the routing
+  constexpr int OC = OW / 8;                 // 16-byte chunks of a result row
+  constexpr int NO = MT_M * OC / MOE_THREADS;
+  int orow[NO];
+  float rw[2] = {1.f, 1.f};
+  if constexpr (DOWN) {
+#pragma unroll
+    for (int i = 0; i < NO; ++i)
+      orow[i] = rows[first + min((tid + i * MOE_THREADS) / OC, nrows - 1)];
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+      rw[b] = flat_w[rows[first + min(wm * 64 + b * 32 + lc, nrows - 1)]];
+  }
+  load_rows(0);
+  if (nk > 1) load_weights(1);
 
   f32x16 acc[2][2];                          // [weight tile][row tile]
 #pragma unroll
@@ -239,51 +292,61 @@ __global__ __launch_bounds__(MOE_THREADS, 2) void moe_tile_kernel(
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
 
-  const int nk = K / MT_K;
-  stage(0, 0);
-  for (int kt = 0; kt < nk; ++kt) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (kt + 1 < nk) stage((kt + 1) & 1, (kt + 1) * MT_K);
-    const unsigned short* al = lds + (kt & 1) * BUF;
-    const unsigned short* bl = al + MT_M * MT_K;
-    if (mine > 0) {
-      // the step's operands first, then its products as they arrive
-      u32x4 fa[MT_K / 16][2], fb[MT_K / 16][2];
+  // NB: row tiles of this wave that hold rows
+  auto products = [&](auto nb) {
+    constexpr int NB = decltype(nb)::value;
+    for (int kt = 0; kt < nk; ++kt) {
+      // step kt is there: only the weights of the next were asked for later
+      if (kt + 1 < nk)
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(NI) : "memory");
+      else
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      if (kt + 1 < nk) load_rows(kt + 1);
+      if (kt + 2 < nk) load_weights(kt + 2);
+      const unsigned short* rl = lds + (kt & 1) * BUF;
+      const unsigned short* wl = lds + (2 + kt % MT_WB) * BUF;
+      if constexpr (NB > 0) {
+        __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-      for (int kk = 0; kk < MT_K / 16; ++kk)
+        for (int kk = 0; kk < MT_K / 16; ++kk) {
+          u32x4 fw[2], fr[NB];
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          const int rb = wn * 64 + t * 32 + lc, ra = wm * 64 + t * 32 + lc;
-          fb[kk][t] = *reinterpret_cast<const u32x4*>(
-              bl + rb * MT_K + ((kk * 2 + hf) ^ ((rb >> 1) & 7)) * 8);
-          if (t == 0 || mine > 32)
-            fa[kk][t] = *reinterpret_cast<const u32x4*>(
-                al + ra * MT_K + ((kk * 2 + hf) ^ ((ra >> 1) & 7)) * 8);
+          for (int t = 0; t < 2; ++t) {
+            const int at = wn * 64 + t * 32 + lc;
+            fw[t] = *reinterpret_cast<const u32x4*>(
+                wl + at * MT_K + ((kk * 2 + hf) ^ ((at >> 1) & 7)) * 8);
+          }
+#pragma unroll
+          for (int t = 0; t < NB; ++t) {
+            const int at = wm * 64 + t * 32 + lc;
+            fr[t] = *reinterpret_cast<const u32x4*>(
+                rl + at * MT_K + ((kk * 2 + hf) ^ ((at >> 1) & 7)) * 8);
+          }
+#pragma unroll
+          for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int a = 0; a < 2; ++a)
+              acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                  __builtin_bit_cast(m_s16x8, fw[a]),
+                  __builtin_bit_cast(m_s16x8, fr[b]), acc[a][b], 0, 0, 0);
         }
-#pragma unroll
-      for (int kk = 0; kk < MT_K / 16; ++kk)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-          if (b == 1 && mine <= 32) continue;
-#pragma unroll
-          for (int a = 0; a < 2; ++a)
-            acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                __builtin_bit_cast(m_s16x8, fb[kk][a]),
-                __builtin_bit_cast(m_s16x8, fa[kk][b]), acc[a][b], 0, 0, 0);
-        }
+        __builtin_amdgcn_s_setprio(0);
+      }
     }
-  }
+  };
+  const int mine = nrows - wm * 64;          // rows of this wave's half
+  if (mine > 32) products(std::integral_constant<int, 2>{});
+  else if (mine > 0) products(std::integral_constant<int, 1>{});
+  else products(std::integral_constant<int, 0>{});
   __syncthreads();
 
   // acc[a][b][r]: weight row 8 (r>>2) + 4 hf + (r&3) of tile a, row lc of
   // tile b. Rows of the result through the LDS, 8-byte units XORed with row.
-  constexpr int OW = DOWN ? MT_N : MT_N / 2; // columns of the result
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
     const int row = wm * 64 + b * 32 + lc;
-    float rw = 1.f;
-    if constexpr (DOWN) rw = flat_w[rows[first + min(row, nrows - 1)]];
 #pragma unroll
     for (int a = 0; a < (DOWN ? 2 : 1); ++a)
 #pragma unroll
@@ -298,7 +361,7 @@ __global__ __launch_bounds__(MOE_THREADS, 2) void moe_tile_kernel(
             if constexpr (EXTM)
               if (bias != nullptr)
                 bd = bf2f(bias[(long)e * N + nt * OW + c + j]);
-            v[j] = (acc[a][b][r] + bd) * rw;
+            v[j] = (acc[a][b][r] + bd) * rw[b];
           } else {
             float g = acc[0][b][r], u = acc[1][b][r];
             if constexpr (EXTM) {
@@ -321,9 +384,8 @@ __global__ __launch_bounds__(MOE_THREADS, 2) void moe_tile_kernel(
       }
   }
   __syncthreads();
-  constexpr int OC = OW / 8;
 #pragma unroll
-  for (int i = 0; i < MT_M * OC / MOE_THREADS; ++i) {
+  for (int i = 0; i < NO; ++i) {
     const int u = tid + i * MOE_THREADS;
     const int row = u / OC, c = u % OC;
     if (row >= nrows) continue;
@@ -331,8 +393,8 @@ __global__ __launch_bounds__(MOE_THREADS, 2) void moe_tile_kernel(
         lds + row * OW + ((2 * c) ^ (row & 15)) * 4);
     const u32x2 b = *reinterpret_cast<const u32x2*>(
         lds + row * OW + ((2 * c + 1) ^ (row & 15)) * 4);
-    const long orow = DOWN ? (long)rows[first + row] : (long)(first + row);
-    *reinterpret_cast<u32x4*>(out + orow * N + nt * OW + c * 8) =
+    const long to = DOWN ? (long)orow[i] : (long)(first + row);
+    *reinterpret_cast<u32x4*>(out + to * N + nt * OW + c * 8) =
         u32x4{a[0], a[1], b[0], b[1]};
   }
 }
@@ -696,25 +758,30 @@ void moe_sum_launch(void* out, const void* contrib, long T, int k, int H,
 void moe_tile_launch(int down, void* out, const void* src, const void* w,
                      const int* rows, const int* tiles, const int* ntiles,
                      const int* offs, const int* counts, const float* flat_w,
-                     const void* bias, int act_mode, int max_tiles, int N,
-                     int K, int* err_unsupported, hipStream_t s) {
+                     const void* bias, int act_mode, long src_rows,
+                     int max_tiles, int N, int K, int* err_unsupported,
+                     hipStream_t s) {
   const int ow = down ? MT_N : MT_N / 2;
   *err_unsupported = N % ow != 0 || K % MT_K != 0;
   if (*err_unsupported || max_tiles == 0) return;
   const bool extm = bias != nullptr || act_mode != 0;
-#define TILE(D, X)                                                            \
-  hipLaunchKernelGGL((moe_tile_kernel<D, X>),                                 \
+  const bool far = !down && src_rows * K * 2 >= 1l << 32;
+#define TILE(D, X, F)                                                         \
+  hipLaunchKernelGGL((moe_tile_kernel<D, X, F>),                              \
                      dim3((unsigned)max_tiles * (N / ow)), dim3(MOE_THREADS), \
                      0, s, (unsigned short*)out, (const unsigned short*)src,  \
                      (const unsigned short*)w, rows, tiles, ntiles, offs,     \
                      counts, flat_w, (const unsigned short*)bias, act_mode,   \
                      N, K)
   if (down) {
-    if (extm) TILE(true, true);
-    else TILE(true, false);
+    if (extm) TILE(true, true, false);
+    else TILE(true, false, false);
+  } else if (far) {
+    if (extm) TILE(false, true, true);
+    else TILE(false, false, true);
   } else {
-    if (extm) TILE(false, true);
-    else TILE(false, false);
+    if (extm) TILE(false, true, false);
+    else TILE(false, false, false);
   }
 #undef TILE
 }

@@ -265,3 +265,31 @@ def test_down_product_of_few_rows(monkeypatch, E, T, H, I, tiles):
     ref = _moe_reference(m, x)
     # as above
     assert float((out.double() - ref).norm() / ref.norm()) < 2.0 ** -7
+
+
+@pytest.mark.parametrize("K", [64, 128, 192, 320])
+@pytest.mark.parametrize("far", [False, True])
+def test_steps_and_far_rows(K, far):
+    """One to five steps of the K loop; rows of a source whose last lie past
+    what 32 bits of byte offset reach (only the first product's are gathered
+    from anywhere)."""
+    hip = _hip()
+    counts = [0, 33, 1, 130, 64]
+    E, TK, N = len(counts), sum(counts), 128
+    g = torch.Generator(device="cuda").manual_seed(K)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    ex = _experts(counts, 1, g).view(-1)
+    order, s_tok, cnt, offs, tiles, n = hip.moe_sort(ex, E, 1)
+    T = TK + (2 ** 31 // K if far else 0)
+    x = torch.empty(T, K, dtype=torch.bfloat16, device="cuda")
+    x[-TK:] = rnd(TK, K)
+    gu = (rnd(E, 2 * N, K) * K ** -0.5).bfloat16()
+    act = torch.full((TK, N), 9.0, device="cuda").bfloat16()
+    hip.moe_tile(False, act, x, gu, s_tok + (T - TK), tiles, n, offs, cnt)
+    rows = x[-TK:].double()[s_tok.long()]
+    e = ex.long()[order.long()]
+    h = torch.stack([gu[int(i)].double() @ r for i, r in zip(e, rows)])
+    ref = torch.nn.functional.silu(h[:, :N]) * h[:, N:]
+    # bf16 result; fp32 sums of K products of size K^-1/2 under 1e-4
+    assert bool(((act.double() - ref).abs()
+                 <= ref.abs() * 2.0 ** -8 + 2e-4).all())
