@@ -390,9 +390,7 @@ void flash_prefill_kernel(
 //    of a value row with row & 3. V^T comes out of the LDS by the transposing
 //    read (ds_read_b64_tr_b16: 16 lanes read 4 keys x 16 channels and get 4 keys
 //    of a channel each), conflict-free with that order.
-//  - the loads are inline asm: behind the builtin the compiler puts a wait for
-//    all of them in front of the next transposing read, that is one memory
-//    latency a tile. The waits are in `advance`.
+//  - the waits for the loads are in `advance`.
 //  - a wave works on 32 keys at a time: the scores of the next 32 are
 //    multiplied while the exponentials of these 32 run, and the maximum of the
 //    next is taken beside the second product, so that the matrix cores need not
@@ -413,17 +411,6 @@ DEVICE_INLINE u32x2 lds_read_tr(const unsigned short* p) {
   return __builtin_bit_cast(
       u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
                  (__attribute__((address_space(3))) s16x4*)p));
-}
-
-// 16 bytes a lane from base + off to LDS address `to` + 16 * lane
-DEVICE_INLINE void load_to_lds(const unsigned short* base, unsigned int off,
-                               const unsigned short* to) {
-  asm volatile(
-      "s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(
-          (unsigned int)(unsigned long)(
-              const __attribute__((address_space(3))) unsigned short*)to),
-      "v"(off), "s"(base)
-      : "memory");
 }
 
 template <bool PAGED>
@@ -551,11 +538,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void flash_rows_kernel(
 #pragma unroll
     for (int r = 3; r < 15; r += 2) x = fmaxf(fmaxf(x, s[r]), s[r + 1]);
     x = fmaxf(x, s[15]);
-    const unsigned int u = __builtin_bit_cast(unsigned int, x);
-    const u32x2 w = __builtin_bit_cast(
-        u32x2, __builtin_amdgcn_permlane32_swap(u, u, false, false));
-    return fmaxf(__builtin_bit_cast(float, w[0]),
-                 __builtin_bit_cast(float, w[1])) * sc;
+    return half_wave_max(x) * sc;
   };
   auto rescale = [&](float mx) {
     if (__any(mx > m + SLACK)) {

@@ -11,6 +11,7 @@
 #include <stdint.h>
 
 #define WAVE_SIZE 64
+#define DEVICE_INLINE __device__ __forceinline__
 
 typedef __attribute__((ext_vector_type(2))) unsigned short u16x2;
 typedef __attribute__((ext_vector_type(4))) unsigned short u16x4;
@@ -83,11 +84,42 @@ __device__ __forceinline__ float wave_reduce_max(float x) {
   return x;
 }
 
+// Maximum of a lane and lane ^ 32, in all lanes. The two operands of the swap are
+// kept apart: given one value twice the compiler takes both results for the same.
+DEVICE_INLINE float half_wave_max(float x) {
+  const unsigned int a = __builtin_bit_cast(unsigned int, x);
+  unsigned int b = a;
+  asm("" : "+v"(b));
+  const auto w = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  return fmaxf(__builtin_bit_cast(float, (unsigned int)w[0]),
+               __builtin_bit_cast(float, (unsigned int)w[1]));
+}
+
 // Reduction across a 16-lane subgroup (lanes with equal l>>4).
 __device__ __forceinline__ float group16_reduce_sum(float x) {
 #pragma unroll
   for (int m = 8; m >= 1; m >>= 1) x += __shfl_xor(x, m, WAVE_SIZE);
   return x;
+}
+
+// Loads from memory straight to LDS address `to` + 16 * lane, 16 bytes a lane,
+// from base + off bytes or from `at`; addresses are multiples of 16. Inline asm,
+// because the compiler puts a wait for all such loads of its builtin in front of
+// LDS reads that it cannot tell from them. They write no register; the kernel
+// waits for them itself (s_waitcnt vmcnt, then its barrier).
+DEVICE_INLINE unsigned int lds_address(const unsigned short* p) {
+  return (unsigned int)(unsigned long)(
+      const __attribute__((address_space(3))) unsigned short*)p;
+}
+DEVICE_INLINE void load_to_lds(const unsigned short* base, unsigned int off,
+                               const unsigned short* to) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               ::"s"(lds_address(to)), "v"(off), "s"(base) : "memory");
+}
+DEVICE_INLINE void load_to_lds(const unsigned short* at,
+                               const unsigned short* to) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+               ::"s"(lds_address(to)), "v"(at) : "memory");
 }
 
 #define HIP_CHECK_KERNEL()                                        \
@@ -98,7 +130,5 @@ __device__ __forceinline__ float group16_reduce_sum(float x) {
                   hipGetErrorString(e_));                         \
     }                                                             \
   } while (0)
-
-#define DEVICE_INLINE __device__ __forceinline__
 
 static inline int ceil_div(int a, int b) { return (a + b - 1) / b; }

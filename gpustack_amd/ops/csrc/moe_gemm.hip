@@ -146,9 +146,8 @@ __global__ __launch_bounds__(MOE_THREADS) void moe_down_scale_kernel(
 // at 597 TFLOP/s). Halves of a wave's rows that an expert does not fill are
 // not multiplied: three forms of the loop, without a branch inside, so that a
 // 16-k's LDS reads fly under the products before it.
-// The loads are inline asm, because the compiler would wait for all of them in
-// front of LDS reads that it cannot tell from them; the weights' first ones leave before the tile's rows are known,
-// and what the end needs of the routing is read before the loop.
+// The weights' first loads leave before the tile's rows are known, and what the
+// end needs of the routing is read before the loop.
 // Bound by the products and the weight stream alike: 254 rows per expert of
 // 128 x (1536 + 768) x 2048 are 0.31 TFLOP and 1.2 GB a layer, 282 + 172 us (727
 // and 596 TFLOP/s; with two buffers of each, branches between the products and
@@ -167,21 +166,6 @@ typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
 DEVICE_INLINE unsigned int moe_pack(float lo, float hi) {
   const f32x2 v{lo, hi};
   return __builtin_bit_cast(unsigned int, __builtin_convertvector(v, bf16x2));
-}
-
-// 16 bytes a lane to LDS address `to` + 16 * lane: from base + off, or from at
-DEVICE_INLINE unsigned int moe_lds(const unsigned short* p) {
-  return (unsigned int)(unsigned long)(
-      const __attribute__((address_space(3))) unsigned short*)p;
-}
-DEVICE_INLINE void moe_load(const unsigned short* base, unsigned int off,
-                            const unsigned short* to) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               ::"s"(moe_lds(to)), "v"(off), "s"(base) : "memory");
-}
-DEVICE_INLINE void moe_load(const unsigned short* at, const unsigned short* to) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-               ::"s"(moe_lds(to)), "v"(at) : "memory");
 }
 
 // FAR: rows of `src` lie further than 32 bits of bytes from its start.
@@ -244,7 +228,7 @@ __global__ __launch_bounds__(MOE_THREADS, 2) void moe_tile_kernel(
     unsigned short* to = lds + (2 + kt % MT_WB) * BUF + wave * 8 * MT_K;
 #pragma unroll
     for (int i = 0; i < NI; ++i)
-      moe_load(wbase + (DOWN ? 0 : (long)(i & 1) * N * K) + kt * MT_K, woff[i],
+      load_to_lds(wbase + (DOWN ? 0 : (long)(i & 1) * N * K) + kt * MT_K, woff[i],
                to + i * 32 * MT_K);
   };
   load_weights(0);
@@ -263,9 +247,9 @@ __global__ __launch_bounds__(MOE_THREADS, 2) void moe_tile_kernel(
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       if constexpr (FAR)
-        moe_load(rbase + roff[i] / 2 + kt * MT_K, to + i * 32 * MT_K);
+        load_to_lds(rbase + roff[i] / 2 + kt * MT_K, to + i * 32 * MT_K);
       else
-        moe_load(rbase + kt * MT_K, roff[i], to + i * 32 * MT_K);
+        load_to_lds(rbase + kt * MT_K, roff[i], to + i * 32 * MT_K);
     }
   };
   // what the end needs of the routing

@@ -134,6 +134,25 @@ def test_rows_and_factors_of_either_kernel(pad, scale):
         at += n
 
 
+@pytest.mark.parametrize("n", [40, 200])
+@pytest.mark.parametrize("at", range(0, 32, 4))
+def test_one_key_far_above_the_others(n, at):
+    """Four keys of 32 whose scores are 300 above all others (more than the
+    exponent of a float holds): whichever lanes hold them."""
+    from gpustack_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(at)
+    q, k, v = (torch.randn(n, h, 128, generator=g, device="cuda")
+               for h in (8, 2, 2))
+    q[..., 0] = 64.0
+    k[..., 0] = 0.0
+    k[at:at + 4, :, 0] = 64.0
+    q, k, v = q.bfloat16(), k.bfloat16(), v.bfloat16()
+    out = torch.full_like(q, 9.0)
+    ops.varlen_prefill_attn(out, q, k, v, [n], 0.1)
+    _check(out, q, k, v, 0, 0.1)
+
+
 def _check_variant(out, q, k, v, hist, scale, sinks, window, softcap):
     """out [n, Hq, DV], q [n, Hq, D] of one sequence, k / v [hist + n, G, .]"""
     n, Hq, _ = q.shape
