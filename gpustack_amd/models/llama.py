@@ -98,18 +98,41 @@ class RaggedMeta:
             self._tiles[key] = c
         return c
 
-    def attn_tiles(self, heads: int, kv_heads: int, maps: int):
+    def attn_tiles(self, heads: int, kv_heads: int, maps: int,
+                   short: bool = False):
         """Workgroup tile list for ops.paged_attention, cached per head
-        layout (layers of one model may differ in it)."""
+        layout (layers of one model may differ in it). `short`: of the
+        portions that prompt_tiles leaves out."""
         if self._tiles is None:
             self._tiles = {}
-        key = (heads, kv_heads, maps)
+        key = (heads, kv_heads, maps, short)
         t = self._tiles.get(key)
         if t is None:
-            t = ops.build_attn_tiles(self.seq_starts, self.seq_hists,
-                                     self.seq_news, heads, kv_heads, maps,
+            view = (self.seq_starts, self.seq_hists, self.seq_news)
+            if short:
+                # portions of no rows have no tiles
+                view = (*view[:2], [0 if n >= ops.PROMPT_PORTION else n
+                                    for n in view[2]])
+            t = ops.build_attn_tiles(*view, heads, kv_heads, maps,
                                      self.block_tables.device)
             self._tiles[key] = t
+        return t
+
+    def prompt_tiles(self, heads: int, window: int):
+        """Tile list of the portions of at least ops.PROMPT_PORTION rows for
+        ops.paged_attention's prompt kernel, or None where the tiles of 16
+        rows are the better ones (ops.prompt_kernel_wins)."""
+        if not ops.prompt_kernel_wins(self.seq_news, self.max_ctx, heads,
+                                      window):
+            return None
+        if self._tiles is None:
+            self._tiles = {}
+        t = self._tiles.get("prompt")
+        if t is None:
+            t = ops.build_prompt_tiles(self.seq_starts, self.seq_hists,
+                                       self.seq_news,
+                                       self.block_tables.device)
+            self._tiles["prompt"] = t
         return t
 
 

@@ -188,14 +188,18 @@ class PagedRotaryAttention(nn.Module):
         # two maps meet again in fp32 (their difference cancels digits)
         a = torch.empty(T, A, self.vw, device=h.device,
                         dtype=torch.float32 if m.maps == 2 else h.dtype)
+        prompt = rg.prompt_tiles(m.heads, m.window) if ops.prompt_attention_fits(
+            m.qk_dim, self.vw, m.maps, m.keep_first, m.softcap, m.chunk,
+            gate is not None, m.scale, k_cache) else None
         ops.paged_attention(
             a, q.view(T, A, m.qk_dim), k_cache, v_cache, rg.block_tables,
             rg.row_seq, rg.pos32, m.scale, maps=m.maps, window=m.window,
             keep_first=m.keep_first,
             sinks=self.zero_sinks if m.unit_sink else self.sinks,
-            tiles=rg.attn_tiles(m.heads, m.kv_heads, m.maps) if h.is_cuda
+            tiles=rg.attn_tiles(m.heads, m.kv_heads, m.maps,
+                                short=prompt is not None) if h.is_cuda
             else None, max_ctx=rg.max_ctx, slopes=self.slopes,
-            softcap=m.softcap, chunk=m.chunk, gate=gate)
+            softcap=m.softcap, chunk=m.chunk, gate=gate, prompt_tiles=prompt)
         if m.maps == 2:
             o = torch.empty(T, m.heads * self.vw, dtype=h.dtype,
                             device=h.device)

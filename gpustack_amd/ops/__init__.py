@@ -890,12 +890,53 @@ def build_attn_tiles(seq_starts, seq_hists, seq_news, heads: int,
     return to_device([(tiles, torch.int32)], device)[0]
 
 
+# Portions of at least this many rows go to the prompt kernel where it fits.
+PROMPT_PORTION = 32
+
+
+def prompt_kernel_wins(seq_news, max_ctx: int, heads: int, window: int) -> bool:
+    """Where the prompt kernel is the faster one: tiles of 16 rows cut a long
+    walk over the keys into parts, so they keep long histories of few rows.
+    us, 16-row tiles / prompt kernel, 16 heads on 4 unless said, slopes: one
+    whole prompt of 32 rows 7.6 / 5.7, 100 9.8 / 10.1, 200 14 / 12.5, six of
+    301 to 1900 in a window of 1024 240 / 85; 16 x 100 behind 100 37 / 16; in
+    a window of 1024 64 rows behind 3000 18 / 40, 200 27 / 45; 8 x 16 behind
+    2000, 32 heads on 8 (256 tiles) 41 / 40, 8 x 32 (512) 57 / 41, 8 x 200
+    207 / 64; without a window 200 behind 3001 (208 tiles) 59 / 97. Both grow
+    with the walk, so the line is the number of 16-row tiles."""
+    tiles = sum((n + 15) // 16 for n in seq_news if n >= PROMPT_PORTION) * heads
+    span = min(max_ctx, window) if window > 0 else max_ctx
+    return tiles >= 512 or (tiles > 0 and span < 512)
+
+
+def build_prompt_tiles(seq_starts, seq_hists, seq_news, device):
+    """Tiles of PREFILL_ROWS rows of every portion of at least PROMPT_PORTION
+    rows, int32 [5, ntiles]: the lists of paged_prefill_tile_rows."""
+    lists = paged_prefill_tile_rows(
+        seq_starts, seq_hists,
+        [n if n >= PROMPT_PORTION else 0 for n in seq_news], PREFILL_ROWS)
+    return to_device([([v for one in lists for v in one], torch.int32)],
+                     device)[0].view(5, -1)
+
+
+def prompt_attention_fits(q_dim: int, v_dim: int, maps: int, keep_first: int,
+                          softcap: float, chunk: int, gate: bool, scale: float,
+                          k_cache) -> bool:
+    """What the prompt kernel of paged_attention takes: heads of 128 channels
+    on values of 128 in bf16 pages of 16, one score map, a window, sinks and
+    slopes, and no other option."""
+    return (q_dim == 128 and v_dim == 128 and maps == 1 and keep_first == 0
+            and softcap == 0 and chunk == 0 and not gate and scale > 0
+            and k_cache.is_cuda and k_cache.dtype == torch.bfloat16
+            and k_cache.shape[2] == 16)
+
+
 def paged_attention(out, q, k_cache, v_cache, block_tables, row_seq, positions,
                     scale: float, maps: int = 1, window: int = 0,
                     keep_first: int = 0, sinks=None, tiles=None,
                     exact: bool = False, max_ctx: int = 0,
                     slopes=None, softcap: float = 0.0, chunk: int = 0,
-                    gate=None) -> None:
+                    gate=None, prompt_tiles=None) -> None:
     """q: [T, A, D], out: [T, A, VW] (A = heads * maps score maps; views
     whose last axis is contiguous). On the
     GPU the MFMA kernel runs for bf16 pools of fitting sizes, the fp32
@@ -905,12 +946,20 @@ def paged_attention(out, q, k_cache, v_cache, block_tables, row_seq, positions,
     `slopes` (fp32, per head): slope * distance is taken off every scaled
     score. `softcap` > 0: scaled scores pass softcap * tanh(s / softcap).
     `chunk` > 0: keys of the row's own chunk of positions only. `gate`
-    ([T, heads] view in q's dtype): a head's output times sigmoid(gate)."""
+    ([T, heads] view in q's dtype): a head's output times sigmoid(gate).
+    `prompt_tiles` (build_prompt_tiles; GPU, where prompt_attention_fits):
+    these portions' rows take the prompt kernel, `tiles` the others."""
     k = _paged_backend(q)
     if k is not None:
         if tiles is None:
             raise ValueError("paged_attention on GPU needs the tile list "
                              "(build_attn_tiles)")
+        if prompt_tiles is not None:
+            k.paged_prompt_attention(out, q, k_cache, v_cache, block_tables,
+                                     prompt_tiles, scale, window, sinks,
+                                     slopes)
+            if tiles.shape[0] == 0:
+                return
         nsplit = 1
         nt = tiles.shape[0]
         span = min(max_ctx, window + keep_first) if window > 0 else max_ctx

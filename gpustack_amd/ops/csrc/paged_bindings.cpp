@@ -18,6 +18,7 @@ void head_rope_store_launch(void*, const void*, long, int, int, int, const float
 void dual_rms_mix_launch(void*, const void*, const float*, const void*, const float*, int, int, float, int, hipStream_t);
 void head_gate_launch(void*, const void*, const void*, long, int, int, int, int, int, hipStream_t);
 void act_inplace_launch(void*, long, int, int, hipStream_t);
+void paged_prompt_attention_launch(void*, const void*, const void*, const void*, const int*, const int*, const float*, const float*, float, long, long, int, int, int, int, int, int, int, int, hipStream_t);
 int paged_attn_max_dim();
 int paged_attn_uses_mfma(int, int, int, int);
 
@@ -177,6 +178,53 @@ void rotary_norm_store(Tensor q_out, Tensor qkv, long nq, long nk,
                             cur_stream(qkv));
     HIP_CHECK_LAST();
   }
+}
+
+// Portions of many rows: heads of 128 channels on values of 128, one map.
+void paged_prompt_attention(Tensor out, Tensor q, Tensor k_cache,
+                            Tensor v_cache, Tensor block_tables, Tensor tiles,
+                            double scale, long window, OptTensor sinks,
+                            OptTensor slopes) {
+  chk(block_tables, "block_tables", at::kInt);
+  chk(tiles, "tiles", at::kInt);
+  TORCH_CHECK(view_kind(q, "q") && view_kind(out, "out") &&
+              act_kind(k_cache, "k_cache") && act_kind(v_cache, "v_cache"),
+              "q, out and the pools must be bf16");
+  const int T = q.size(0), A = q.size(1), G = k_cache.size(1);
+  TORCH_CHECK(k_cache.dim() == 4 && v_cache.dim() == 4 && G >= 1 &&
+              A % G == 0 && q.size(2) == 128 && k_cache.size(2) == 16 &&
+              k_cache.size(3) == 128 && v_cache.size(0) == k_cache.size(0) &&
+              v_cache.size(1) == G && v_cache.size(2) == 128 &&
+              v_cache.size(3) == 16 && k_cache.size(0) >= 1,
+              "pools must be [nblocks, G, 16, 128] and [nblocks, G, 128, 16]");
+  TORCH_CHECK(out.size(0) == T && out.size(1) == A && out.size(2) == 128);
+  for (auto* t : {&q, &out, &k_cache, &v_cache})
+    TORCH_CHECK(reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0,
+                "rows must start at 16-byte addresses");
+  for (auto* t : {&q, &out})
+    TORCH_CHECK(t->stride(1) == 128 && t->stride(0) % 8 == 0,
+                "heads must be packed, rows at 16-byte addresses");
+  TORCH_CHECK(tiles.dim() == 2 && tiles.size(0) == 5 &&
+              block_tables.dim() == 2 && block_tables.size(1) >= 1 &&
+              window >= 0 && scale > 0);
+  const float *sp = nullptr, *slp = nullptr;
+  if (sinks.has_value()) {
+    chk(*sinks, "sinks", at::kFloat);
+    TORCH_CHECK(sinks->numel() == A);
+    sp = sinks->data_ptr<float>();
+  }
+  if (slopes.has_value()) {
+    chk(*slopes, "slopes", at::kFloat);
+    TORCH_CHECK(slopes->numel() == A);
+    slp = slopes->data_ptr<float>();
+  }
+  paged_prompt_attention_launch(
+      out.data_ptr(), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
+      block_tables.data_ptr<int>(), tiles.data_ptr<int>(), sp, slp,
+      (float)scale, q.stride(0), out.stride(0), (int)tiles.size(1), T, A, G,
+      (int)block_tables.size(0), (int)block_tables.size(1),
+      (int)k_cache.size(0), (int)window, cur_stream(q));
+  HIP_CHECK_LAST();
 }
 
 void paged_attention(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache,
@@ -450,6 +498,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("post_w"), py::arg("mult"), py::arg("eps"), py::arg("extra"),
         py::arg("next_w"), py::arg("h"), py::arg("center") = false);
   m.def("rotary_norm_store", &rotary_norm_store);
+  m.def("paged_prompt_attention", &paged_prompt_attention,
+        "attention of prompt portions over the paged pool");
   m.def("paged_attention", &paged_attention, py::arg("out"), py::arg("q"),
         py::arg("k_cache"), py::arg("v_cache"), py::arg("block_tables"),
         py::arg("tiles"), py::arg("pos32"), py::arg("scale"), py::arg("maps"),

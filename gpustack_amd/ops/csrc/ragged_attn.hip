@@ -44,6 +44,8 @@
 // kernel is tested against.
 #include "common.h"
 
+#include <type_traits>
+
 namespace {
 
 constexpr int G16 = 16;       // (row, map) pairs per workgroup
@@ -533,6 +535,326 @@ __global__ __launch_bounds__(MERGE_THREADS) void paged_attn_merge_kernel(
   }
 }
 
+// ---- prompts ---------------------------------------------------------------
+// Portions of many rows, heads of 128 channels on values of 128, one map, pages
+// of 16 keys: a workgroup takes 128 rows of one head, 4 waves x 32 rows, and
+// walks the keys 64 at a time on v_mfma_f32_32x32x16_bf16, from the page pools.
+//  - S^T = K Q^T: a lane holds scores of one row; keys are multiplied in an order
+//    in which a lane's 8 of 16 are neighbours (key_of), so that the value pages,
+//    channel by channel as they lie in the pool, are the operand of O^T = V^T P^T
+//    with one 16-byte LDS read.
+//  - pages go to the LDS by themselves, a wave brings one page of keys (16-byte
+//    chunks XORed with the row) and one of values; two buffers of each, one
+//    barrier a tile.
+//  - a wave works on 32 keys at a time: the next 32 are multiplied while these
+//    are weighted, so the K buffer of tile j holds keys 64 j + 32 .. 64 j + 95 and
+//    the first 32 come before the loop. Pairs of whole tiles (no key of them
+//    hidden from any row of the wave) run without masks.
+//  - the running maximum is exact, as in the kernel above: the largest weight is
+//    1 and rounds to itself. Let 2^8 above it, as prompts of the other models
+//    do, the error of a row is 2.2e-3 instead of 1.5e-3 of its length.
+// Bound by the latency of a tile's loads and its chain (1.9 us a tile of 64 keys
+// where few workgroups run, 3.3 with two on every CU): 16 heads on 4, six prompts
+// of 301 to 1900 rows in a window of 1024 with slopes 240 -> 85 us a layer, 8 x 200
+// rows behind 2000 (32 heads on 8) 207 -> 64, 16 x 100 behind 100 37 -> 16.
+typedef __attribute__((ext_vector_type(16))) float pr_f32x16;
+typedef __attribute__((ext_vector_type(2))) unsigned int pr_u32x2;
+
+constexpr int PR_ROWS = 128;       // rows of a workgroup
+constexpr int PR_KEYS = 64;        // keys of a tile
+constexpr int PR_D = 128;
+constexpr float PR_LOG2E = 1.4426950408889634f;
+
+struct PromptArgs {
+  const int* block_tables;   // [nseq, maxb]
+  const int* tiles;          // [5, ntiles] sequence's first row, tile's first
+                             // row there, cached tokens, rows, sequence
+  const float* sinks;        // [A] or null
+  const float* slopes;       // [A] or null
+  float scale;
+  long q_st, o_st;           // row strides of q and out, heads packed
+  int ntiles, T, A, G, nseq, maxb, nblocks, window;
+};
+
+__global__ __launch_bounds__(THREADS, 2) void paged_prompt_kernel(
+    unsigned short* __restrict__ out, const unsigned short* __restrict__ q,
+    const unsigned short* __restrict__ k_cache,
+    const unsigned short* __restrict__ v_cache, PromptArgs p) {
+  constexpr int D = PR_D, BS = 16, QK = D / 16, NT = D / 32, HB = 32;
+  constexpr int TILE = PR_KEYS * D;        // elements of a buffer
+  constexpr int PAGE = BS * D;
+  __shared__ __attribute__((aligned(1024))) unsigned short lds[4 * TILE];
+
+  // heads of one kv head on one XCD (workgroups go round the 8 XCDs)
+  int a = blockIdx.x % p.A;
+  if (p.A % 8 == 0) a = (a % 8) * (p.A / 8) + a / 8;
+  const int tile = (gridDim.x - 1 - blockIdx.x) / p.A;
+  const int row0 = p.tiles[tile], q0 = p.tiles[p.ntiles + tile];
+  const int hist = p.tiles[2 * p.ntiles + tile];
+  const int nnew = p.tiles[3 * p.ntiles + tile];
+  const int seq = p.tiles[4 * p.ntiles + tile];
+  if (row0 < 0 || hist < 0 || nnew < 1 || row0 + nnew > p.T || q0 < 0 ||
+      q0 >= nnew || seq < 0 || seq >= p.nseq ||
+      (hist + nnew + BS - 1) / BS > p.maxb)
+    return;
+  const int g = a / (p.A / p.G);
+  const int len = hist + nnew;
+  const int* bt = p.block_tables + (long)seq * p.maxb;
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int lc = lane & 31, hf = lane >> 5;
+  const int qrow = q0 + wave * 32 + lc;            // within the new rows
+  const int qpos = hist + qrow;
+  u32x4 qf[QK];
+  {
+    const unsigned short* qp =
+        q + (long)(row0 + min(qrow, nnew - 1)) * p.q_st + (long)a * D + hf * 8;
+#pragma unroll
+    for (int kk = 0; kk < QK; ++kk)
+      qf[kk] = *reinterpret_cast<const u32x4*>(qp + kk * 16);
+  }
+  const float sc = p.scale * PR_LOG2E;
+  const float slope = p.slopes != nullptr ? p.slopes[a] / p.scale : 0.f;
+  float m = -INFINITY, l = 0.f;                    // m in powers of two
+  pr_f32x16 o[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[t][r] = 0.f;
+
+  const int lo_wave = hist + q0 + wave * 32;       // this wave's first row
+  const bool idle = q0 + wave * 32 >= nnew;        // it has none
+  const int kv_end = min(len, hist + q0 + PR_ROWS);
+  const int nt = (kv_end + PR_KEYS - 1) / PR_KEYS;
+  // first keys that any row of the workgroup, of the wave may see, and the
+  // first that all rows of the wave see
+  const int first = p.window > 0 ? max(0, hist + q0 - p.window + 1) : 0;
+  const int first_wave = p.window > 0 ? max(0, lo_wave - p.window + 1) : 0;
+  const int first_all = p.window > 0 ? max(0, lo_wave + 31 - p.window + 1) : 0;
+  const int kt0 = first / PR_KEYS;
+  // and what this lane's row sees
+  const int seen_lo = p.window > 0 ? qpos - p.window + 1 : 0;
+  const int seen_hi = min(qpos, len - 1);
+
+  const int lr = lane >> 4, ch = lane & 15;
+  const unsigned int koff = (unsigned)(lr * D + (ch ^ lr) * 8) * 2;
+  auto page_of = [&](int key) {
+    const int pg = min(key, len - 1) / BS;
+    return ((long)min(max(bt[pg], 0), p.nblocks - 1) * p.G + g) * PAGE;
+  };
+  // a page behind the sequence's end is its last one again
+  auto stage_keys = [&](int key0, unsigned short* to) {
+    const int key = key0 + wave * BS;
+    if (key < kt0 * PR_KEYS) return;
+    const unsigned short* base = k_cache + page_of(key);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      load_to_lds(base + i * 4 * D, koff ^ (i * 64), to + wave * PAGE + i * 4 * D);
+  };
+  auto stage_values = [&](int key0, unsigned short* to) {
+    const unsigned short* base = v_cache + page_of(key0 + wave * BS);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      load_to_lds(base + i * 512, (unsigned)lane * 16, to + wave * PAGE + i * 512);
+  };
+  auto kbuf = [&](int j) { return lds + (j & 1) * TILE; };
+  auto vbuf = [&](int j) { return lds + (2 + (j & 1)) * TILE; };
+
+  // row lc of the K operand is key key_of(lc) of 32: a lane's scores r are keys
+  // 16 (r>>3) + 8 hf + (r&7)
+  const int key_of = (lc >> 4) * 16 + ((lc >> 2) & 1) * 8 + ((lc >> 3) & 1) * 4 +
+                     (lc & 3);
+  const unsigned short *ka[QK], *va = lds + 2 * TILE + lc * BS + hf * 8;
+#pragma unroll
+  for (int i = 0; i < QK; ++i)
+    ka[i] = lds + key_of * D + (((i * 2 + hf) ^ (key_of & 15)) * 8);
+
+  // unscaled scores of keys kv0 .. kv0 + 31, on top of slope * distance / scale;
+  // at: elements from ka
+  auto scores = [&](int at, int kv0, pr_f32x16& s) {
+    const float near = slope * (float)(kv0 + 8 * hf - qpos);
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      s[r] = __builtin_fmaf(slope, (float)(16 * (r >> 3) + (r & 7)), near);
+#pragma unroll
+    for (int kk = 0; kk < QK; ++kk)
+      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+          __builtin_bit_cast(ra_s16x8,
+                             *reinterpret_cast<const u32x4*>(ka[kk] + at)),
+          __builtin_bit_cast(ra_s16x8, qf[kk]), s, 0, 0, 0);
+  };
+  auto row_max = [&](const pr_f32x16& s) {          // in powers of two
+    float x = fmaxf(fmaxf(s[0], s[1]), s[2]);
+#pragma unroll
+    for (int r = 3; r < 15; r += 2) x = fmaxf(fmaxf(x, s[r]), s[r + 1]);
+    x = fmaxf(x, s[15]);
+    return half_wave_max(x) * sc;
+  };
+  auto rescale = [&](float mx) {
+    if (__any(mx > m)) {
+      const float nm = fmaxf(m, mx);
+      const float corr =
+          nm == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - nm);
+      m = nm;
+      l *= corr;
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[t][r] *= corr;
+    }
+    return m == -INFINITY ? 0.f : m;
+  };
+  auto weights = [&](const pr_f32x16& s, u32x4 (&pf)[2], float base) {
+    float sum = 0.f;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const float x = __builtin_amdgcn_exp2f(
+            __builtin_fmaf(s[t * 8 + w * 2], sc, -base));
+        const float y = __builtin_amdgcn_exp2f(
+            __builtin_fmaf(s[t * 8 + w * 2 + 1], sc, -base));
+        sum += x + y;
+        const f32x2 xy{x, y};
+        pf[t][w] = __builtin_bit_cast(unsigned int,
+                                      __builtin_convertvector(xy, bf16x2));
+      }
+    l += sum;
+  };
+  // at: elements from va. CUT: only `left` keys of the 32 are the sequence's, and
+  // what lies behind them in its last page is not multiplied.
+  auto weigh = [&](int at, const u32x4 (&pf)[2], auto cut, int left) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int n = 0; n < NT; ++n) {
+        u32x4 v = *reinterpret_cast<const u32x4*>(va + at + t * PAGE + n * 512);
+        if constexpr (decltype(cut)::value) {
+          const int own = left - t * 16 - hf * 8;
+#pragma unroll
+          for (int w = 0; w < 4; ++w)
+            v[w] &= own > 2 * w + 1 ? 0xffffffffu : own > 2 * w ? 0xffffu : 0u;
+        }
+        o[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            __builtin_bit_cast(ra_s16x8, v),
+            __builtin_bit_cast(ra_s16x8, pf[t]), o[n], 0, 0, 0);
+      }
+  };
+  // Tile j is in the LDS for every wave, and every wave is done with tile
+  // j - 1, whose buffers tile j + 1 takes.
+  auto advance = [&](int j) {
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const int next = (j + 1) * PR_KEYS;
+    if (next + HB < kv_end) stage_keys(next + HB, kbuf(j + 1));
+    if (next < kv_end) stage_values(next, vbuf(j + 1));
+  };
+
+  const int k0 = kt0 * PR_KEYS;
+  stage_keys(k0 - HB, kbuf(kt0 + 1));
+  if (k0 + HB < kv_end) stage_keys(k0 + HB, kbuf(kt0));
+  stage_values(k0, vbuf(kt0));
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  pr_f32x16 st;
+  scores(((kt0 + 1) & 1) * TILE + HB * D, k0, st);
+
+  float mx = 0.f;
+  bool known = false;                              // mx is st's
+  auto whole = [&](int j, int par) {               // par = j & 1, a constant
+    advance(j);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const float base = rescale(mx);
+      pr_f32x16 next;
+      u32x4 pf[2];
+      scores(par * TILE + h * HB * D, j * PR_KEYS + (h + 1) * HB, next);
+      weights(st, pf, base);
+      weigh(par * TILE + h * 2 * PAGE, pf, std::false_type{}, 32);
+      st = next;
+      mx = row_max(st);
+    }
+  };
+  // tiles whose every key every row of the wave sees, and their next tile exists
+  const int whole_lo = (first_all + PR_KEYS - 1) / PR_KEYS;
+  const int whole_hi = idle ? 0 : min(nt - 1, (lo_wave + 1) / PR_KEYS);
+  for (int j = kt0; j < nt;) {
+    if (!(j & 1) && j >= whole_lo && j + 1 < whole_hi) {
+      if (!known) mx = row_max(st);
+      known = true;
+      whole(j, 0);
+      whole(j + 1, 1);
+      j += 2;
+      continue;
+    }
+    known = false;
+    advance(j);
+#pragma unroll 1
+    for (int h = 0; h < 2; ++h) {
+      const int kv0 = j * PR_KEYS + h * HB;
+      if (kv0 > lo_wave + 31 || kv0 >= kv_end || idle) break;
+      const int at = (j & 1) * TILE + h * HB * D;
+      if (kv0 + HB > first_wave) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int kv = kv0 + 16 * (r >> 3) + 8 * hf + (r & 7);
+          st[r] = kv >= seen_lo && kv <= seen_hi ? st[r] : -INFINITY;
+        }
+        const float base = rescale(row_max(st));
+        u32x4 pf[2];
+        weights(st, pf, base);
+        const int vat = (j & 1) * TILE + h * 2 * PAGE;
+        if (len - kv0 < HB) weigh(vat, pf, std::true_type{}, len - kv0);
+        else weigh(vat, pf, std::false_type{}, HB);
+      }
+      if (kv0 + HB < kv_end) scores(at, kv0 + HB, st);
+    }
+    ++j;
+  }
+  __syncthreads();
+
+  l += __shfl_xor(l, 32, 64);
+  float num = 1.f;
+  if (p.sinks != nullptr) {                        // no key, no value
+    const float sk = p.sinks[a] * PR_LOG2E;
+    const float M = fmaxf(m, sk);
+    num = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - M);
+    l = l * num + __builtin_amdgcn_exp2f(sk - M);
+  }
+  const float inv = l > 0.f ? num / l : 0.f;
+  // through the wave's own part of the LDS to whole rows
+  unsigned short* ol = lds + wave * 32 * D;
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+#pragma unroll
+    for (int rr = 0; rr < 4; ++rr) {
+      pr_u32x2 w;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const f32x2 xy{o[n][rr * 4 + c * 2] * inv, o[n][rr * 4 + c * 2 + 1] * inv};
+        w[c] = __builtin_bit_cast(unsigned int,
+                                  __builtin_convertvector(xy, bf16x2));
+      }
+      *reinterpret_cast<pr_u32x2*>(
+          ol + lc * D + ((n * 8 + rr * 2 + hf) ^ (lc & 15)) * 4) = w;
+    }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < D / 16; ++i) {
+    const int u = lane + i * 64, r = u / 16, c = u % 16;
+    const pr_u32x2 x = *reinterpret_cast<const pr_u32x2*>(
+        ol + r * D + ((2 * c) ^ (r & 15)) * 4);
+    const pr_u32x2 y = *reinterpret_cast<const pr_u32x2*>(
+        ol + r * D + ((2 * c + 1) ^ (r & 15)) * 4);
+    const int row = q0 + wave * 32 + r;
+    if (row < nnew)
+      *reinterpret_cast<u32x4*>(out + (long)(row0 + row) * p.o_st + (long)a * D +
+                                c * 8) = u32x4{x[0], x[1], y[0], y[1]};
+  }
+}
+
 template <int NT, typename TO>
 void launch_mfma(void* out, const void* q, const void* kc, const void* vc,
                  const AttnArgs& p, int ntiles, int nsplit, float* ws_acc,
@@ -642,4 +964,20 @@ void paged_attention_launch(void* out, const void* q, const void* k_cache,
   } else {
     dispatch_exact<float, float, float>(out, q, k_cache, v_cache, p, ntiles, s);
   }
+}
+
+void paged_prompt_attention_launch(
+    void* out, const void* q, const void* k_cache, const void* v_cache,
+    const int* block_tables, const int* tiles, const float* sinks,
+    const float* slopes, float scale, long q_st, long o_st, int ntiles, int T,
+    int A, int G, int nseq, int maxb, int nblocks, int window, hipStream_t s) {
+  if (ntiles == 0) return;
+  PromptArgs p;
+  p.block_tables = block_tables; p.tiles = tiles; p.sinks = sinks;
+  p.slopes = slopes; p.scale = scale; p.q_st = q_st; p.o_st = o_st;
+  p.ntiles = ntiles; p.T = T; p.A = A; p.G = G; p.nseq = nseq; p.maxb = maxb;
+  p.nblocks = nblocks; p.window = window;
+  paged_prompt_kernel<<<dim3((unsigned)ntiles * A), THREADS, 0, s>>>(
+      (unsigned short*)out, (const unsigned short*)q,
+      (const unsigned short*)k_cache, (const unsigned short*)v_cache, p);
 }
