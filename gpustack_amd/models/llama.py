@@ -98,6 +98,14 @@ class RaggedMeta:
             self._tiles[key] = c
         return c
 
+    def scan_runs(self, heads: int, n_state: int, vdim: int, dtype):
+        """Runs of rows for ops.state_scan, or None for a batch of short
+        portions or operands that its chunk kernel does not take."""
+        if dtype != torch.bfloat16 or not 32 <= n_state <= 128 or vdim < 32:
+            return None
+        rows = ops.scan_run_rows(self.seq_news, heads, vdim)
+        return self.scan_chunks(rows) if rows else None
+
     def attn_tiles(self, heads: int, kv_heads: int, maps: int,
                    short: bool = False):
         """Workgroup tile list for ops.paged_attention, cached per head

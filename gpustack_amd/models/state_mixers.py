@@ -93,7 +93,9 @@ class Mamba2Mixer(nn.Module):
                        m.heads, m.groups, m.state, m.vdim, False,
                        self.dt_bias, self.a_log, self.skip, None, ssm_state,
                        rg.seq_first, rg.seq_rows, rg.state_slots, rg.pos32,
-                       single=max(rg.seq_news, default=1) <= 1)
+                       single=max(rg.seq_news, default=1) <= 1,
+                       runs=rg.scan_runs(m.heads, m.state, m.vdim, h.dtype)
+                       if h.is_cuda else None)
         g = torch.empty(T, m.inner, dtype=h.dtype, device=h.device)
         ops.gated_group_norm(g, y, u[:, :m.inner], self.norm, m.norm_groups,
                              self.eps, True)
@@ -129,7 +131,9 @@ class LightningMixer(nn.Module):
                        m.heads, m.state, m.vdim, True, None, None, None,
                        self.decay, ssm_state, rg.seq_first, rg.seq_rows,
                        rg.state_slots, rg.pos32,
-                       single=max(rg.seq_news, default=1) <= 1)
+                       single=max(rg.seq_news, default=1) <= 1,
+                       runs=rg.scan_runs(m.heads, m.state, m.vdim, h.dtype)
+                       if h.is_cuda else None)
         g = torch.empty(T, m.inner, dtype=h.dtype, device=h.device)
         ops.gated_group_norm(g, y, u[:, 2 * self.nqk + m.inner:], self.norm,
                              1, self.eps, False)

@@ -1124,18 +1124,37 @@ def causal_conv_silu(out, src, col0: int, w, b, conv_state, seq_first,
                state_slots, row_seq, pos32)
 
 
+def scan_run_rows(seq_news, heads: int, vdim: int) -> int:
+    """Rows of a run for state_scan, or 0 where whole sequences do as well: up
+    to half of the chip's 512 places for workgroups (64 value channels of a
+    head) would work through the longest sequence alone. us whole / in runs of
+    an eighth of it and 64 rows: 64 heads of 64 channels, 1 x 4000 rows 723 /
+    266, 1 x 1000 191 / 107, 1 x 500 97 / 70, 1 x 250 50 / 50, 2 x 2000 364 /
+    259, six of 301 to 1900 433 / 353, but 8 x 500 141 / 250, 4 x 200 47 / 91;
+    16 heads of 128 1 x 4000 918 / 260, 1 x 500 121 / 77, the six 428 / 241,
+    8 x 500 133 / 173, 32 x 125 91 / 145."""
+    longest = max(seq_news, default=0)
+    groups = heads * ((vdim + 63) // 64)
+    if longest < 256 or longest * 256 <= sum(seq_news) * groups:
+        return 0
+    return (longest // 8 + 64 + 31) // 32 * 32
+
+
 def state_scan(y, src, col_x: int, col_b: int, col_c: int, dt_src,
                col_dt: int, heads: int, groups: int, n_state: int, vdim: int,
                act_silu: bool, dt_bias, a_log, skip, decay, state, seq_first,
-               seq_rows, state_slots, pos32, single: bool = False) -> None:
+               seq_rows, state_slots, pos32, single: bool = False,
+               runs=None) -> None:
     """`single` (a host-side hint): every sequence brings one row, as in a
-    decode step; the GPU then streams the states through its step kernel."""
+    decode step; the GPU then streams the states through its step kernel.
+    `runs` (build_scan_chunks; a prompt): the GPU cuts
+    the sequences into runs of rows that workgroups take side by side."""
     k = _state_backend(src)
     if k is not None:
         k.state_scan(y, src, col_x, col_b, col_c, dt_src, col_dt, heads,
                      groups, n_state, vdim, act_silu, dt_bias, a_log, skip,
                      decay, state, seq_first, seq_rows, state_slots, pos32,
-                     single)
+                     single, runs)
     else:
         torch_ref.state_scan(y, src, col_x, col_b, col_c, dt_src, col_dt,
                              heads, groups, n_state, vdim, act_silu, dt_bias,

@@ -13,7 +13,7 @@ void add_layer_norm_launch(float*, const void*, const float*, const float*, void
 void head_norm_store_launch(void*, void*, long, int, int, int, const float*, const float*, int, float, float, const int*, const void*, long, const float*, void*, void*, const long*, long, int, int, int, float, int, int, int, hipStream_t);
 void value_page_store_launch(const void*, long, int, void*, const long*, long, const int*, int, int, int, int, int, int, hipStream_t);
 void route_topk_launch(int*, float*, const float*, int, const float*, int, int, int, int, int, int, int, int, float, hipStream_t);
-int state_scan_launch(float*, const void*, long, int, int, int, const void*, long, int, int, int, int, int, int, const float*, const float*, const float*, const float*, float*, const int*, const int*, const int*, const int*, int, int, int, int, int, hipStream_t);
+int state_scan_launch(float*, const void*, long, int, int, int, const void*, long, int, int, int, int, int, int, const float*, const float*, const float*, const float*, float*, const int*, const int*, const int*, const int*, int, int, int, int, int, const int*, int, float*, float*, float*, hipStream_t);
 void gated_group_norm_launch(void*, const float*, const float*, const void*, long, const float*, int, int, int, float, int, int, int, hipStream_t);
 int delta_scan_launch(float*, const void*, long, int, int, int, const void*, long, int, int, int, int, int, int, const float*, const float*, float*, const int*, const int*, const int*, const int*, int, int, int, int, int, hipStream_t);
 int delta_scan_max_state();
@@ -218,7 +218,7 @@ void state_scan(Tensor y, Tensor src, long col_x, long col_b, long col_c,
                 long n_state, long vdim, bool act_silu, OptTensor dt_bias,
                 OptTensor a_log, OptTensor skip, OptTensor decay, Tensor state,
                 Tensor seq_first, Tensor seq_rows, Tensor state_slots,
-                Tensor pos32, bool single) {
+                Tensor pos32, bool single, OptTensor runs) {
   chk(y, "y", at::kFloat);
   chk(state, "state", at::kFloat);
   const int bf = view_kind(src, "src");
@@ -259,6 +259,19 @@ void state_scan(Tensor y, Tensor src, long col_x, long col_b, long col_c,
     sp = skip->data_ptr<float>();
   }
   const int nseq = seq_view(seq_first, seq_rows, state_slots, pos32, T);
+  const int* rp = nullptr;
+  int nruns = 0;
+  Tensor ends, scratch, falls;
+  if (runs.has_value()) {
+    chk(*runs, "runs", at::kInt);
+    TORCH_CHECK(runs->dim() == 2 && runs->size(1) == 4,
+                "runs must be [n, 4] (build_scan_chunks)");
+    rp = runs->data_ptr<int>();
+    nruns = (int)runs->size(0);
+    ends = at::empty({nruns, heads, n_state, vdim}, y.options());
+    scratch = at::empty_like(ends);
+    falls = at::empty({nruns, heads}, y.options());
+  }
   const int ok = state_scan_launch(
       y.data_ptr<float>(), src.data_ptr(), src.stride(0), (int)col_x,
       (int)col_b, (int)col_c, dtp, ld_dt, (int)col_dt, (int)heads, (int)groups,
@@ -266,7 +279,9 @@ void state_scan(Tensor y, Tensor src, long col_x, long col_b, long col_c,
       state.data_ptr<float>(), seq_first.data_ptr<int>(),
       seq_rows.data_ptr<int>(), state_slots.data_ptr<int>(),
       pos32.data_ptr<int>(), nseq, (int)state.size(0), T, bf, single ? 1 : 0,
-      cur_stream(src));
+      rp, nruns, nruns ? ends.data_ptr<float>() : nullptr,
+      nruns ? scratch.data_ptr<float>() : nullptr,
+      nruns ? falls.data_ptr<float>() : nullptr, cur_stream(src));
   TORCH_CHECK(ok, "state size unsupported");
   HIP_CHECK_LAST();
 }

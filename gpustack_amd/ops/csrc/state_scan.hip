@@ -55,6 +55,13 @@ struct ScanArgs {
   const int* state_slots;
   const int* pos32;
   int nslots, T;
+  // sequences cut into runs of rows (state_chunk_kernel), or null
+  const int* runs;         // [nruns, 4] first row, rows, sequence, the list
+                           // index of the sequence's first run
+  int nruns, nseq;
+  float* ends;             // [nruns, H, N, P] state behind a run
+  float* scratch;          // [nruns, H, N, P]
+  float* falls;            // [nruns, H] product of a run's decays
 };
 
 constexpr int CH = 16;     // rows staged per pass
@@ -337,44 +344,99 @@ __global__ __launch_bounds__(256) void state_scan_vec_kernel(
 //   - with that order the state, as the accumulators hold it (rows 4 g + r,
 //     column l & 15), is the operand of Q S: it never leaves the registers.
 //   - the next chunk's rows are fetched while this one is worked on; 48 KB.
-// Bound by the chain of chunks of the longest sequence (about 170 matrix
-// instructions of 32 cycles a wave and chunk).
+// Bound by the chain of chunks (about 170 matrix instructions of 32 cycles a wave
+// and chunk, 7.7 us). Where whole sequences leave the chip idle they are cut into
+// runs of chunks (RUNS): a first launch (ENDS) works out what each run but a
+// sequence's last adds to the state, from zero (the first run from the slot), and
+// how far the run lets a state fall; in the second (OUTPUTS) a run's workgroup
+// puts the state in front of it together from the runs before and goes through
+// its rows as above. The slot is read by the first launch (the second takes the
+// first run's state from `scratch`) and written by the last run in the second.
+// 64 heads of 128 x 64, one sequence of 4000 rows 723 -> 266 us, six of 301 to 1900
+// 433 -> 353; 16 heads of 128 x 128 918 -> 260 and 428 -> 241.
 typedef __attribute__((ext_vector_type(4))) float sc_f32x4;
 
-template <int NT>   // state rows / 16, padded
+enum ChunkPart { WHOLE, ENDS, OUTPUTS };
+
+template <int NT, int PART>   // state rows / 16, padded
 __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
     float* __restrict__ y, const unsigned short* __restrict__ src,
     const unsigned short* __restrict__ dt_src, ScanArgs p) {
   constexpr int C = 32, NP = NT * 16, KS = NP + 4, PB = 64, VS = PB + 4;
   constexpr int KU = C * NP / 8 / 256;       // 16-byte loads of k (and q)
   static_assert(KU >= 1 && C * NP / 8 % 256 == 0, "NT is 4 or 8");
-  __shared__ __attribute__((aligned(16))) float qs[C][KS];
+  constexpr int QR = PART == ENDS ? 1 : C;
+  __shared__ __attribute__((aligned(16))) float qs[QR][KS];
   __shared__ __attribute__((aligned(16))) float ks[C][KS];
   __shared__ __attribute__((aligned(16))) float vs[C][VS];
-  __shared__ __attribute__((aligned(16))) float as[C][C + 4];
+  __shared__ __attribute__((aligned(16))) float as[QR][C + 4];
   __shared__ double cs[C];
   __shared__ float bl[C], el[C], wl[C];
-  const int s = blockIdx.x, h = blockIdx.y, pb0 = blockIdx.z * PB;
+  int s = blockIdx.x;
+  const int h = blockIdx.y, pb0 = blockIdx.z * PB;
+  const int run = blockIdx.x;
+  int run0 = run, first, n;
+  bool ends = true;                          // the sequence ends with these rows
+  if constexpr (PART == WHOLE) {
+    first = p.seq_first[s];
+    n = p.seq_rows[s];
+  } else {
+    const int* r = p.runs + (long)run * 4;
+    first = r[0];
+    n = r[1];
+    s = r[2];
+    run0 = r[3];
+    if (s < 0 || s >= p.nseq || run0 < 0 || run0 > run) return;
+    ends = first + n >= p.seq_first[s] + p.seq_rows[s];
+    if (PART == ENDS && ends) return;
+  }
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lc = lane & 15, g = lane >> 4;
-  const int first = p.seq_first[s], n = p.seq_rows[s];
   if (first < 0 || n < 1 || first + n > p.T) return;
   const int slot = min(max(p.state_slots[s], 0), p.nslots - 1);
-  const int hist = p.pos32[first];
+  // a state in front of these rows
+  const int hist = run == run0 ? p.pos32[first] : PART == OUTPUTS;
   const int N = p.N, P = p.P;
   const int grp = h / (p.H / p.G);
   const int pc = pb0 + wave * 16 + lc;       // this lane's value channel
   const bool live = pc < P;
   float* sp = p.state + ((long)slot * p.H + h) * N * P;
+  const long NP_ = (long)N * P, stride = p.H * NP_;  // of a head, of a run
+  float odd = 0.f;                           // NaN behind a value that is not finite
   sc_f32x4 S[NT];                            // rows 16 t + 4 g + r, column pc
+  auto each = [&](auto f) {
 #pragma unroll
-  for (int t = 0; t < NT; ++t)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int nn = t * 16 + g * 4 + r;
-      S[t][r] = (hist > 0 && live && nn < N) ? sp[(long)nn * P + pc] : 0.f;
+      for (int r = 0; r < 4; ++r) {
+        const int nn = t * 16 + g * 4 + r;
+        if (live && nn < N) S[t][r] = f(S[t][r], (long)nn * P + pc);
+      }
+  };
+#pragma unroll
+  for (int t = 0; t < NT; ++t) S[t] = sc_f32x4{0.f, 0.f, 0.f, 0.f};
+  if (PART == OUTPUTS && run > run0) {
+    const float* at = p.ends + (long)run0 * stride + h * NP_;
+    each([&](float, long i) { return at[i]; });
+    for (int j = run0 + 1; j < run; ++j) {
+      const float fall = p.falls[(long)j * p.H + h];
+      at += stride;
+      // what is not finite outlives every decay
+      each([&](float x, long i) {
+        return (fall == 0.f && !(fabsf(x) < INFINITY) ? x : x * fall) + at[i];
+      });
     }
+    each([&](float x, long) { odd += x * 0.f; return x; });
+  } else if (hist > 0) {
+    const float* from = PART == OUTPUTS && !ends
+                            ? p.scratch + (long)run * stride + h * NP_ : sp;
+    each([&](float, long i) { return from[i]; });
+    if constexpr (PART == ENDS) {            // the last run writes the slot
+      float* to = p.scratch + (long)run * stride + h * NP_;
+      each([&](float x, long i) { return to[i] = x; });
+    }
+  }
   const float skip = p.skip != nullptr ? p.skip[h] : 0.f;
   const float a_rate = dt_src != nullptr ? expf(p.a_log[h]) : 0.f;
   const float dtb = dt_src != nullptr ? p.dt_bias[h] : 0.f;
@@ -388,7 +450,6 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
 
   u16x8 kreg[KU], qreg[KU], vreg;
   float dreg = 0.f;
-  float odd = 0.f;                           // NaN behind a value that is not finite
   auto fetch = [&](int c0) {
     const int rows = min(C, n - c0);
 #pragma unroll
@@ -399,7 +460,8 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
       if (r < rows && e < N) {
         const unsigned short* rp = src + (long)(first + c0 + r) * p.ld_src;
         kreg[u] = *reinterpret_cast<const u16x8*>(rp + p.col_b + grp * N + e);
-        qreg[u] = *reinterpret_cast<const u16x8*>(rp + p.col_c + grp * N + e);
+        if constexpr (PART != ENDS)
+          qreg[u] = *reinterpret_cast<const u16x8*>(rp + p.col_c + grp * N + e);
       }
     }
     const int r = tid / (PB / 8), e = tid % (PB / 8) * 8;
@@ -423,6 +485,7 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
   };
 
+  float fall = 1.f;
   fetch(0);
   for (int c0 = 0; c0 < n; c0 += C) {
     const int rows = min(C, n - c0);
@@ -430,7 +493,7 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
     for (int u = 0; u < KU; ++u) {
       const int i = tid + u * 256, r = i / (NP / 8), e = i % (NP / 8) * 8;
       put8(&ks[r][e], kreg[u]);
-      put8(&qs[r][e], qreg[u]);
+      if constexpr (PART != ENDS) put8(&qs[r][e], qreg[u]);
     }
     put8(&vs[tid / (PB / 8)][tid % (PB / 8) * 8], vreg);
     if (tid < C) {
@@ -462,6 +525,8 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
     __syncthreads();
     if (c0 + C < n) fetch(c0 + C);
 
+    sc_f32x4 o[2];
+    if constexpr (PART != ENDS) {
     // scores of 16 x 16 rows a wave, weighted
     const int ti = wave >> 1, si = wave & 1;
     if (si <= ti) {
@@ -490,7 +555,6 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
       }
     }
     // what the state brings
-    sc_f32x4 o[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) o[t] = sc_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -508,6 +572,7 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[t][r] *= el[t * 16 + g * 4 + r];
     __syncthreads();
+    }
     // what the chunk's own rows bring
     float vv[2][4];
 #pragma unroll
@@ -518,6 +583,7 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
     for (int b = 0; b < 2; ++b)
 #pragma unroll
       for (int j = 0; j < 4; ++j) odd += vv[b][j] * 0.f;
+    if constexpr (PART != ENDS) {
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -536,9 +602,11 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
           y[(long)(first + c0 + tr) * p.H * P + h * P + pc] =
               o[t][r] + skip * vs[tr][wave * 16 + lc];
       }
+    }
     // the state behind the chunk
     const float down = expf((float)cs[C - 1]) *
                        (neg && (rows & 1) ? -1.f : 1.f);
+    if constexpr (PART == ENDS) fall *= down;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -555,14 +623,36 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
       }
     __syncthreads();
   }
+  float* own = PART == WHOLE ? sp
+               : (PART == ENDS ? p.ends : p.scratch) + (long)run * stride + h * NP_;
+  if constexpr (PART == ENDS)
+    if (tid == 0 && pb0 == 0) p.falls[(long)run * p.H + h] = fall;
   // A value that is infinite or NaN belongs to its own row and those behind
   // it, but the weights of 0 above the diagonal carried it to the rows in
-  // front: such columns are walked again row by row, on the state in memory.
+  // front: such columns are walked again row by row, on the state in memory
+  // (the slot, or a run's own place).
   if (__any(odd != 0.f)) {
     auto load = [&](const unsigned short* at) {
       const float f = bf2f(*at);
       return p.act ? silu_f(f) : f;
     };
+    if (PART != WHOLE && hist > 0)
+#pragma unroll 1
+      for (int nn = g; nn < N && live; nn += 4) {
+        const long i = (long)nn * P + pc;
+        if (run == run0) {
+          if (PART == ENDS || ends) own[i] = sp[i];
+          continue;
+        }
+        const float* at = p.ends + (long)run0 * stride + h * NP_ + i;
+        float x = *at;
+        for (int j = run0 + 1; j < run; ++j) {
+          const float f = p.falls[(long)j * p.H + h];
+          at += stride;
+          x = (f == 0.f && !(fabsf(x) < INFINITY) ? x : x * f) + *at;
+        }
+        own[i] = x;
+      }
 #pragma unroll 1
     for (int i = 0; i < n; ++i) {
       const unsigned short* rp = src + (long)(first + i) * p.ld_src;
@@ -575,25 +665,28 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
       const float v = live ? load(rp + p.col_x + h * P + pc) : 0.f;
 #pragma unroll 1
       for (int nn = g; nn < N && live; nn += 4) {
-        float* at = sp + (long)nn * P + pc;
+        float* at = own + (long)nn * P + pc;
         const float old = i > 0 || hist > 0 ? *at : 0.f;
         *at = a * old + b * load(rp + p.col_b + grp * N + nn) * v;
-        part += *at * load(rp + p.col_c + grp * N + nn);
+        if constexpr (PART != ENDS)
+          part += *at * load(rp + p.col_c + grp * N + nn);
       }
-      part += __shfl_xor(part, 16, 64);
-      part += __shfl_xor(part, 32, 64);
-      if (g == 0 && live)
-        y[(long)(first + i) * p.H * P + h * P + pc] = part + skip * v;
+      if constexpr (PART != ENDS) {
+        part += __shfl_xor(part, 16, 64);
+        part += __shfl_xor(part, 32, 64);
+        if (g == 0 && live)
+          y[(long)(first + i) * p.H * P + h * P + pc] = part + skip * v;
+      }
     }
+    if (PART == OUTPUTS && ends)
+      for (int nn = g; nn < N && live; nn += 4)
+        sp[(long)nn * P + pc] = own[(long)nn * P + pc];
     return;
   }
-#pragma unroll
-  for (int t = 0; t < NT; ++t)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int nn = t * 16 + g * 4 + r;
-      if (live && nn < N) sp[(long)nn * P + pc] = S[t][r];
-    }
+  if (PART == ENDS || ends) {
+    float* to = PART == ENDS ? own : sp;
+    each([&](float x, long i) { return to[i] = x; });
+  }
 }
 
 // Single rows (decode): the state itself is the traffic, so one workgroup
@@ -844,13 +937,21 @@ bool scan_pick(float* y, const void* src, const void* dt, const ScanArgs& p,
   // channels and 16-row state tiles are not mostly padding
   if (sizeof(TS) == 2 && vec && p.N >= 32 && p.N <= 128 && p.P >= 32 &&
       (long)p.T >= (long)CHUNK_ROWS * nseq) {
-    const dim3 grid(nseq, p.H, (p.P + 63) / 64);
-    if (p.N <= 64)
-      state_chunk_kernel<4><<<grid, 256, 0, s>>>(
-          y, (const unsigned short*)src, (const unsigned short*)dt, p);
-    else
-      state_chunk_kernel<8><<<grid, 256, 0, s>>>(
-          y, (const unsigned short*)src, (const unsigned short*)dt, p);
+    const bool cut = p.nruns > nseq;
+    const dim3 grid(cut ? p.nruns : nseq, p.H, (p.P + 63) / 64);
+#define CHUNKS(NT, PART)                                                     \
+  state_chunk_kernel<NT, PART><<<grid, 256, 0, s>>>(                         \
+      y, (const unsigned short*)src, (const unsigned short*)dt, p)
+#define CHUNKS_NT(NT)                                                        \
+  if (cut) {                                                                 \
+    CHUNKS(NT, ENDS);                                                        \
+    CHUNKS(NT, OUTPUTS);                                                     \
+  } else {                                                                   \
+    CHUNKS(NT, WHOLE);                                                       \
+  }
+    if (p.N <= 64) { CHUNKS_NT(4) } else { CHUNKS_NT(8) }
+#undef CHUNKS_NT
+#undef CHUNKS
     return true;
   }
   // few workgroups (long portions of few sequences): more lanes per channel
@@ -888,6 +989,8 @@ int state_scan_max_state() { return 8 * 64; }
 
 // src_bf: src and dt_src are bf16 (else fp32). single: the caller expects
 // one row per sequence (a hint: any batch is still computed correctly).
+// runs (or null): the sequences cut into nruns > nseq runs of rows, for the
+// chunk kernel, with ends and scratch [nruns, H, N, P] and falls [nruns, H].
 // Returns 0 when no instantiation covers the sizes.
 int state_scan_launch(float* y, const void* src, long ld_src, int col_x,
                       int col_b, int col_c, const void* dt_src, long ld_dt,
@@ -897,9 +1000,12 @@ int state_scan_launch(float* y, const void* src, long ld_src, int col_x,
                       const int* seq_first, const int* seq_rows,
                       const int* state_slots, const int* pos32, int nseq,
                       int nslots, int T, int src_bf, int single,
-                      hipStream_t s) {
+                      const int* runs, int nruns, float* ends, float* scratch,
+                      float* falls, hipStream_t s) {
   if (T <= 0 || nseq <= 0) return 1;
   ScanArgs p;
+  p.runs = runs; p.nruns = nruns; p.nseq = nseq; p.ends = ends;
+  p.scratch = scratch; p.falls = falls;
   p.ld_src = ld_src; p.ld_dt = ld_dt; p.col_x = col_x; p.col_b = col_b;
   p.col_c = col_c; p.col_dt = col_dt; p.H = H; p.G = G; p.N = N; p.P = P;
   p.act = act; p.dt_bias = dt_bias; p.a_log = a_log; p.skip = skip;

@@ -79,6 +79,86 @@ def test_chunks(kind, H, G, N, P, news):
     assert torch.equal(st[6], state[6])
 
 
+@pytest.mark.parametrize("size", [32, 64, 96])
+@pytest.mark.parametrize("kind", ["steps", "wide steps", "constants"])
+@pytest.mark.parametrize("H,G,N,P", [(4, 2, 128, 64), (3, 3, 64, 128),
+                                     (2, 1, 40, 72)])
+@pytest.mark.parametrize("news", [[31, 65, 33, 1, 64], [200, 7], [97]])
+def test_runs(size, kind, H, G, N, P, news):
+    """Sequences cut into runs of rows (one to seven of them): as without."""
+    from gpustack_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(sum(news) + N)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    T, S = sum(news), len(news)
+    hists, slots = [7, 5, 0, 9, 3][:S], [3, 0, 5, 1, 2][:S]
+    cb, cc = 8 + H * P, 8 + H * P + G * N
+    cdt = cc + G * N
+    src = (rnd(T, (cdt + H + 15) // 8 * 8) * 0.7).bfloat16()
+    state = rnd(7, H, N, P)
+    if kind == "constants":
+        decay = torch.tensor([1.0, 0.0, -0.5, 0.97], device="cuda")[:H]
+        args = (None, 0, H, G, N, P, True, None, None, None, decay)
+        a = decay.double().expand(T, H)
+        b, skip = torch.ones_like(a), None
+    else:
+        a_log = rnd(H) * 0.5 + (4.0 if kind == "wide steps" else 0.0)
+        bias, skip = rnd(H) - 1, rnd(H)
+        args = (src, cdt, H, G, N, P, False, bias, a_log, skip, None)
+        b = torch.nn.functional.softplus(
+            src[:, cdt:cdt + H].double() + bias.double())
+        a = torch.exp(-torch.exp(a_log.double()) * b)
+    ref_y, ref_s = _walk(src, 8, cb, cc, H, G, N, P, kind == "constants", a, b,
+                         skip, state, news, hists, slots)
+    first = [sum(news[:i]) for i in range(S)]
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    pos = i32([h + j for h, n in zip(hists, news) for j in range(n)])
+    y = torch.zeros(T, H * P, device="cuda")
+    st = state.clone()
+    ops.state_scan(y, src, 8, cb, cc, *args, st, i32(first), i32(news),
+                   i32(slots), pos,
+                   runs=ops.build_scan_chunks(first, news, size, "cuda"))
+    # the bound of test_chunks: a state put together from runs has two more
+    # roundings a run
+    for got, ref in ((y, ref_y), (st, ref_s)):
+        scale = float(ref.abs().max())
+        assert float((got.double() - ref).abs().max()) <= 4e-6 * scale
+    assert torch.equal(st[6], state[6])
+
+
+@pytest.mark.parametrize("size", [0, 32])
+@pytest.mark.parametrize("decay", [0.9, 0.0])
+@pytest.mark.parametrize("hist", [0, 3])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("at", [5, 40, 90])
+def test_not_finite_in_runs(at, bad, hist, decay, size):
+    from gpustack_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(at)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    T, H, N, P = 130, 2, 64, 96
+    src = rnd(T, H * (P + 2 * N)).bfloat16()
+    src[at, P + 70] = bad
+    decay = torch.tensor([0.9, decay], device="cuda")
+    state = rnd(2, H, N, P)
+    cb, cc = H * P, H * (P + N)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    y = torch.zeros(T, H * P, device="cuda")
+    a = decay.double().expand(T, H)
+    ref, ref_s = _walk(src, 0, cb, cc, H, H, N, P, False, a,
+                       torch.ones_like(a), None, state, [T], [hist], [0])
+    ops.state_scan(y, src, 0, cb, cc, None, 0, H, H, N, P, False, None, None,
+                   None, decay, state, i32([0]), i32([T]), i32([0]),
+                   i32(list(range(hist, hist + T))),
+                   runs=ops.build_scan_chunks([0], [T], size, "cuda")
+                   if size else None)
+    for got, want in ((y, ref), (state, ref_s)):
+        ok = want.isfinite()
+        assert torch.equal(got.isfinite(), ok)
+        scale = float(want[ok].abs().max())    # fp32 sums, as above
+        assert float((got[ok].double() - want[ok]).abs().max()) <= 4e-6 * scale
+
+
 @pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
 @pytest.mark.parametrize("at", [5, 20, 47])
 def test_not_finite(bad, at):
