@@ -34,6 +34,8 @@ class DenseFF(nn.Module):
     block's output (a projection of the same input that someone else
     needs, a residual gate for instance)."""
 
+    out_parts = False      # the result may be a product's parts (linear_auto)
+
     def __init__(self, width: int, f: FeedForwardSpec, dtype, comm=None,
                  extra: int = 0):
         super().__init__()
@@ -63,7 +65,7 @@ class DenseFF(nn.Module):
             u = g
         else:
             ops.act_inplace(u, self.act)
-        return ops.linear_auto(u, self.down_w)
+        return ops.linear_auto(u, self.down_w, self.out_parts)
 
 
 class RoutedFF(nn.Module):

@@ -51,6 +51,11 @@ class LivasunLayer(nn.Module):
             cls = RoutedFF if ls.mlp.kind == "moe" else DenseFF
             self.mlp = cls(width, ls.mlp, dtype, comm)
             self.norm2_w, self.norm2_b = f32(), f32()
+        # ops.add_layer_norm, which closes both, adds parts up (of rows that
+        # its 16-byte form takes)
+        for m in (self.mixer, self.mlp):
+            if hasattr(m, "out_parts"):
+                m.out_parts = width % 8 == 0 and width <= 8192
 
 
 class LivasunForCausalLM(nn.Module):

@@ -190,8 +190,9 @@ class W4Pack:
         self.shape = (qw.shape[0], qw.shape[1] * 2)
 
 
-def qlinear(x, w, pack: "W4Pack | None", bias=None):
-    """F.linear with an optional W4 runtime pack.
+def qlinear(x, w, pack: "W4Pack | None", bias=None, parts: bool = False):
+    """F.linear with an optional W4 runtime pack. `parts` as in
+    ops.linear_auto.
 
     Packed weights stay RESIDENT packed (the capacity goal). Up to 64 rows
     the packed product (ops/csrc/w4_gemm.hip) reads them as they are; more
@@ -201,7 +202,8 @@ def qlinear(x, w, pack: "W4Pack | None", bias=None):
     (4096x14336: 20 / 50, 60 / 59, 110 / 70). GPUSTACK_AMD_W4_KERNEL=1 keeps
     the packed product up to 1024 rows."""
     if pack is None:
-        return ops.linear_auto(x, w) if bias is None else F.linear(x, w, bias)
+        return ops.linear_auto(x, w, parts) if bias is None \
+            else F.linear(x, w, bias)
     if x.is_cuda:
         import os as _os
 
@@ -291,9 +293,22 @@ class Attention(nn.Module):
                 self.q_norm = nn.Parameter(torch.empty(self.d, dtype=dtype), requires_grad=False)
                 self.k_norm = nn.Parameter(torch.empty(self.d, dtype=dtype), requires_grad=False)
 
-    def forward(self, x, meta: ForwardMeta, cos_sin, k_cache, v_cache):
+    def forward(self, x, meta: ForwardMeta, cos_sin, k_cache, v_cache,
+                parts: bool = False):
+        """`parts`: the result may be the parts of the output product
+        (ops.linear_auto)."""
         T = x.shape[0]
-        qkv = qlinear(x, self.qkv_w, self.qkv_pack, self.qkv_b)
+        head_norm = self.spec.qk_norm and not (
+            self.spec.qk_norm_full or self.spec.qk_norm_after_rope)
+        store = (meta.cp is None and self.use_rope
+                 and (head_norm or not self.spec.qk_norm))
+        qkv = qlinear(x, self.qkv_w, self.qkv_pack, self.qkv_b,
+                      parts=store and meta.lora is None and ops.qkv_store_ok(
+                          x, self.d, self.rot_dim, self.spec.rope_mode))
+        qkv_parts = None
+        if qkv.dim() == 3:
+            qkv_parts = qkv
+            qkv = torch.empty(qkv.shape[1:], dtype=x.dtype, device=x.device)
         if meta.lora is not None:
             qkv = qkv.contiguous()
             meta.lora.apply(self.layer_idx, x, qkv, self._qkv_projs)
@@ -303,17 +318,13 @@ class Attention(nn.Module):
         q = qkv[:, :nq].unflatten(1, (self.hq, self.d))
         k = qkv[:, nq:nq + nk].unflatten(1, (self.hkv, self.d))
         v = qkv[:, nq + nk:].unflatten(1, (self.hkv, self.d))
-        head_norm = self.spec.qk_norm and not (
-            self.spec.qk_norm_full or self.spec.qk_norm_after_rope)
-        if (meta.cp is None and self.use_rope
-                and (head_norm or not self.spec.qk_norm)
-                and ops.qkv_store_ok(qkv, self.d, self.rot_dim,
-                                     self.spec.rope_mode)):
+        if store and ops.qkv_store_ok(qkv, self.d, self.rot_dim,
+                                      self.spec.rope_mode):
             ops.qkv_store(qkv, self.hq, self.hkv,
                           self.q_norm if head_norm else None,
                           self.k_norm if head_norm else None, cos_sin,
                           meta.positions, meta.slot_mapping, k_cache, v_cache,
-                          self.spec.rms_norm_eps)
+                          self.spec.rms_norm_eps, qkv_parts)
         else:
             q, k, v = self._norm_rope_store(q, k, v, meta, cos_sin, k_cache,
                                             v_cache)
@@ -344,7 +355,8 @@ class Attention(nn.Module):
                 out, q, k_cache, v_cache, meta.block_tables, meta.seq_lens,
                 self.scale, **sw
             )
-        o = qlinear(out.view(T, -1), self.o_w, self.o_pack, self.o_b)
+        o = qlinear(out.view(T, -1), self.o_w, self.o_pack, self.o_b,
+                    parts=parts and meta.lora is None)
         if meta.lora is not None:
             meta.lora.apply(self.layer_idx, out.view(T, -1), o, self._o_projs)
         return self.comm.all_reduce(o)
@@ -672,7 +684,8 @@ class MLP(nn.Module):
         self._down_projs = [("down_proj", 0, h)]
         self.act = spec.mlp_act
 
-    def forward(self, x, meta: ForwardMeta | None = None):
+    def forward(self, x, meta: ForwardMeta | None = None,
+                parts: bool = False):
         gu = qlinear(x, self.gate_up_w, self.gate_up_pack)
         if meta is not None and meta.lora is not None:
             meta.lora.apply(self.layer_idx, x, gu, self._gu_projs)
@@ -690,8 +703,10 @@ class MLP(nn.Module):
             act = torch.empty(x.shape[0], self.i, dtype=x.dtype,
                               device=x.device)
             ops.silu_and_mul(act, gu)
-        down = qlinear(act, self.down_w, self.down_pack)
-        if meta is not None and meta.lora is not None:
+        lora = meta is not None and meta.lora is not None
+        down = qlinear(act, self.down_w, self.down_pack,
+                       parts=parts and not lora)
+        if lora:
             meta.lora.apply(self.layer_idx, act, down, self._down_projs)
         return self.comm.all_reduce(down)
 
@@ -1134,7 +1149,10 @@ class DecoderLayer(nn.Module):
         else:
             self.pre_ff_norm = self.post_ff_norm = None
 
-    def forward(self, x, residual, meta, cos_sin, k_cache, v_cache):
+    def forward(self, x, residual, meta, cos_sin, k_cache, v_cache,
+                parts: bool = False):
+        """`parts`: x and the result may be the parts of a product
+        (ops.linear_auto), to be added up by ops.add_rms_norm."""
         eps = self.spec.rms_norm_eps
         if self.spec.parallel_block:
             return self._forward_parallel(x, meta, cos_sin, k_cache,
@@ -1150,14 +1168,15 @@ class DecoderLayer(nn.Module):
             h = torch.empty_like(x)
             ops.rms_norm(h, x, self.input_norm, eps)
         else:
-            h = x
-            ops.fused_add_rms_norm(h, residual, self.input_norm, eps)
-        a = self.attn(h, meta, cos_sin, k_cache, v_cache)
+            h = ops.add_rms_norm(x, residual, self.input_norm, eps)
         rm = self.spec.residual_multiplier
+        kw = {"parts": True} if parts and not rm else {}
+        a = self.attn(h, meta, cos_sin, k_cache, v_cache,
+                      **(kw if isinstance(self.attn, Attention) else {}))
         if rm:  # Granite: scale sublayer outputs before the residual add
             a = a * rm
-        ops.fused_add_rms_norm(a, residual, self.post_attn_norm, eps)
-        m = self.mlp(a, meta)
+        a = ops.add_rms_norm(a, residual, self.post_attn_norm, eps)
+        m = self.mlp(a, meta, **(kw if isinstance(self.mlp, MLP) else {}))
         if rm:
             m = m * rm
         return m, residual
@@ -1304,6 +1323,8 @@ class LlamaForCausalLM(nn.Module):
                 x = x * torch.tensor(self.spec.embed_scale,
                                      dtype=x.dtype, device=x.device)
         residual = None
+        # whole rows of whole products: nothing between a product and its norm
+        parts = self.comm.pp_size == 1 and self.comm.tp_size == 1
         off = self.offload
         if off is not None:
             off.begin()
@@ -1313,7 +1334,8 @@ class LlamaForCausalLM(nn.Module):
             cs = (self.cos_sin_local
                   if (self.cos_sin_local is not None and layer.attn.window)
                   else self.cos_sin)
-            x, residual = layer(x, residual, meta, cs, kv.k_caches[i], kv.v_caches[i])
+            x, residual = layer(x, residual, meta, cs, kv.k_caches[i],
+                                kv.v_caches[i], parts=parts)
         if self.comm.pp_size > 1 and not self.comm.is_last_stage:
             if residual is None:  # sandwich layers carry the true stream
                 self.comm.send_hidden(x.contiguous())
@@ -1327,8 +1349,8 @@ class LlamaForCausalLM(nn.Module):
         elif residual is None:
             ops.rms_norm(x, x, self.final_norm, self.spec.rms_norm_eps)
         else:
-            ops.fused_add_rms_norm(x, residual, self.final_norm,
-                                   self.spec.rms_norm_eps)
+            x = ops.add_rms_norm(x, residual, self.final_norm,
+                                 self.spec.rms_norm_eps)
         if return_hidden:
             return x  # all rows, post final norm (embedding serving)
         hidden = x[meta.logits_indices]

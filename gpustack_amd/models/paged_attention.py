@@ -46,6 +46,8 @@ from ..engine.config import PagedMixerSpec
 
 
 class PagedRotaryAttention(nn.Module):
+    out_parts = False      # the result may be a product's parts (linear_auto)
+
     def __init__(self, width: int, m: PagedMixerSpec, eps: float, dtype,
                  comm=None, v_mix_first: bool = False):
         super().__init__()
@@ -207,5 +209,5 @@ class PagedRotaryAttention(nn.Module):
                              m.diff, self.eps)
         else:
             o = a.view(T, A * self.vw)
-        out = ops.linear_auto(o, self.o_w)
+        out = ops.linear_auto(o, self.o_w, self.out_parts)
         return self.comm.all_reduce(out) if self.comm is not None else out

@@ -58,6 +58,8 @@ def _mk(*shape, dt):
 
 
 class Mamba2Mixer(nn.Module):
+    out_parts = False      # the result may be a product's parts (linear_auto)
+
     def __init__(self, width: int, m: ScanMixerSpec, eps: float, dtype,
                  comm=None):
         super().__init__()
@@ -99,11 +101,13 @@ class Mamba2Mixer(nn.Module):
         g = torch.empty(T, m.inner, dtype=h.dtype, device=h.device)
         ops.gated_group_norm(g, y, u[:, :m.inner], self.norm, m.norm_groups,
                              self.eps, True)
-        out = ops.linear_auto(g, self.o_w)
+        out = ops.linear_auto(g, self.o_w, self.out_parts)
         return self.comm.all_reduce(out) if self.comm is not None else out
 
 
 class LightningMixer(nn.Module):
+    out_parts = False      # the result may be a product's parts (linear_auto)
+
     def __init__(self, width: int, m: ScanMixerSpec, eps: float, dtype,
                  comm=None):
         super().__init__()
@@ -137,7 +141,7 @@ class LightningMixer(nn.Module):
         g = torch.empty(T, m.inner, dtype=h.dtype, device=h.device)
         ops.gated_group_norm(g, y, u[:, 2 * self.nqk + m.inner:], self.norm,
                              1, self.eps, False)
-        out = ops.linear_auto(g, self.o_w)
+        out = ops.linear_auto(g, self.o_w, self.out_parts)
         return self.comm.all_reduce(out) if self.comm is not None else out
 
 

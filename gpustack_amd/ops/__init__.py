@@ -126,6 +126,17 @@ def rms_norm(out, x, weight, eps: float) -> None:
         torch_ref.rms_norm(out, x, weight, eps)
 
 
+def add_rms_norm(x, residual, weight, eps: float):
+    """residual += x and the norm of it, which is returned: in x, or where x is
+    the parts of a product (linear_auto with `parts`) in a tensor of its own."""
+    if x.dim() == 3:
+        out = torch.empty_like(residual)
+        _load_hip().fused_add_rms_norm(out, residual, weight, eps, x)
+        return out
+    fused_add_rms_norm(x, residual, weight, eps)
+    return x
+
+
 def fused_add_rms_norm(x, residual, weight, eps: float) -> None:
     hip = _backend(x)
     if hip is not None:
@@ -174,12 +185,14 @@ def qkv_store_ok(qkv, head_dim: int, rot_dim: int, mode: str) -> bool:
 
 
 def qkv_store(qkv, q_heads: int, kv_heads: int, q_norm, k_norm, cos_sin,
-              positions, slots, k_cache, v_cache, eps: float) -> None:
+              positions, slots, k_cache, v_cache, eps: float,
+              parts=None) -> None:
     """qkv [T, (q_heads + 2 kv_heads) * D]: weighted RMS norm of every q and k
     head (where weights are given), rotation of q and k in place, keys and
-    values to their slots (-1: none). GPU only (qkv_store_ok)."""
+    values to their slots (-1: none). `parts` (linear_auto): the rows are
+    their sum, and qkv is only written. GPU only (qkv_store_ok)."""
     _load_hip().qkv_store(qkv, q_heads, kv_heads, q_norm, k_norm, cos_sin,
-                          positions, slots, k_cache, v_cache, eps)
+                          positions, slots, k_cache, v_cache, eps, parts)
 
 
 def greedy_sample_into(out, logits) -> None:
@@ -513,12 +526,14 @@ def router_plan(T: int, E: int, H: int):
     return (128, 2) if E >= 128 else (64, 2)
 
 
-def linear_auto(x, w):
+def linear_auto(x, w, parts: bool = False):
     """Shape-gated GEMM dispatch: the products for few rows
     (_rows_tile_plan, _rows_gemm_wins), the split-K skinny kernel where it
     measured faster than hipBLASLt (scripts/bench_skinny_gemm.py on MI355X:
     down_proj-like N=4096 K>=8192 M>=384 at splitk=4, 824 TF vs hipBLASLt 680),
-    F.linear everywhere else."""
+    F.linear everywhere else. `parts`: a product that is cut over k may come
+    as its fp32 parts [n, M, N], for a consumer that adds them up itself
+    (add_rms_norm, qkv_store, add_layer_norm) and saves the join's launch."""
     import os
 
     import torch.nn.functional as F
@@ -535,6 +550,8 @@ def linear_auto(x, w):
                 and x.stride(1) == 1 and x.stride(0) % 8 == 0
                 and x.data_ptr() % 16 == 0
                 and not (x.requires_grad or w.requires_grad)):
+            if parts and plan and plan[1] > 1:
+                return _load_hip().rows_tile_parts(x, w, *plan)
             out = torch.empty(M, N, dtype=x.dtype, device=x.device)
             if plan:
                 _load_hip().rows_tile(out, x, w, *plan)
@@ -1076,6 +1093,8 @@ def embed_rows_scaled(x, tokens, embed, scale: float) -> None:
 
 
 def add_layer_norm(x, a, w, b, eps: float, h) -> None:
+    """x += a and h = its layer norm; a may be the parts of a product
+    (linear_auto)."""
     k = _state_backend(x)
     if k is not None:
         k.add_layer_norm(x, a, w, b, eps, h)

@@ -6,13 +6,13 @@
 
 // launchers (defined in the .hip translation units)
 void rms_norm_launch(void*, const void*, const void*, float, int, int, hipStream_t);
-void fused_add_rms_norm_launch(void*, void*, const void*, float, int, int, hipStream_t);
+void fused_add_rms_norm_launch(void*, void*, const void*, const float*, int, float, int, int, hipStream_t);
 void rope_neox_launch(const long*, void*, void*, const float*, int, int, int, int, int, long, long, hipStream_t);
 void silu_and_mul_launch(void*, const void*, long, int, hipStream_t);
 void reshape_and_cache_launch(const void*, const void*, void*, void*, const long*, int, int, int, int, long, long, int, hipStream_t);
 void greedy_sample_launch(long*, const void*, int, int, hipStream_t);
 void mla_decode_launch(float*, const void*, const void*, const int*, const int*, int, int, int, int, int, int, float, int*, hipStream_t);
-void qkv_store_launch(void*, const void*, const void*, const float*, const long*, const long*, void*, void*, long, int, int, int, int, float, int, int*, hipStream_t);
+void qkv_store_launch(void*, const float*, int, const void*, const void*, const float*, const long*, const long*, void*, void*, long, int, int, int, int, float, int, int*, hipStream_t);
 struct DecodeParts { int n, least; };
 DecodeParts decode_parts(int, int, int, int, int, int);
 void paged_attn_decode_launch(void*, const void*, const void*, const void*, const int*, const int*, float*, DecodeParts, int, int, int, int, int, float, long, int, const float*, int, float, int*, hipStream_t);
@@ -87,15 +87,29 @@ void rms_norm(at::Tensor out, at::Tensor input, at::Tensor weight, double eps) {
   HIP_CHECK_LAST();
 }
 
+// fp32 parts [n, rows, cols] of a product cut over k, not added up
+const float* check_parts(const at::Tensor& p, long rows, long cols) {
+  TORCH_CHECK(p.is_cuda() && p.scalar_type() == at::kFloat &&
+              p.is_contiguous() && p.dim() == 3 && p.size(0) >= 1 &&
+              p.size(1) == rows && p.size(2) == cols,
+              "parts must be fp32 [n, rows, cols]");
+  return p.data_ptr<float>();
+}
+
 void fused_add_rms_norm(at::Tensor x, at::Tensor residual, at::Tensor weight,
-                        double eps) {
+                        double eps, c10::optional<at::Tensor> parts) {
   check_bf16(x, "x"); check_bf16(residual, "residual"); check_bf16(weight, "weight");
   const int H = x.size(-1);
   const long T = x.numel() / H;
   TORCH_CHECK(H % 8 == 0, "hidden size must be a multiple of 8");
-  fused_add_rms_norm_launch(x.data_ptr(), residual.data_ptr(),
-                            weight.data_ptr(), (float)eps, (int)T, H,
-                            cur_stream(x));
+  TORCH_CHECK(!parts.has_value() || (residual.numel() == x.numel() &&
+                                     weight.numel() == H),
+              "fused_add_rms_norm shapes");
+  fused_add_rms_norm_launch(
+      x.data_ptr(), residual.data_ptr(), weight.data_ptr(),
+      parts.has_value() ? check_parts(*parts, T, H) : nullptr,
+      parts.has_value() ? (int)parts->size(0) : 0, (float)eps, (int)T, H,
+      cur_stream(x));
   HIP_CHECK_LAST();
 }
 
@@ -145,7 +159,8 @@ void qkv_store(at::Tensor qkv, long Hq, long Hk,
                c10::optional<at::Tensor> q_norm,
                c10::optional<at::Tensor> k_norm, at::Tensor cos_sin,
                at::Tensor positions, at::Tensor slots, at::Tensor k_cache,
-               at::Tensor v_cache, double eps) {
+               at::Tensor v_cache, double eps,
+               c10::optional<at::Tensor> parts) {
   check_bf16(qkv, "qkv");
   check_cache(k_cache, "k_cache"); check_cache(v_cache, "v_cache");
   const long T = qkv.size(0);
@@ -169,7 +184,10 @@ void qkv_store(at::Tensor qkv, long Hq, long Hk,
       nw[i] = (*given[i])->data_ptr();
     }
   int err = 0;
-  qkv_store_launch(qkv.data_ptr(), nw[0], nw[1], cos_sin.data_ptr<float>(),
+  qkv_store_launch(qkv.data_ptr(),
+                   parts.has_value() ? check_parts(*parts, T, qkv.size(1))
+                                     : nullptr,
+                   parts.has_value() ? (int)parts->size(0) : 0, nw[0], nw[1], cos_sin.data_ptr<float>(),
                    positions.data_ptr<long>(), slots.data_ptr<long>(),
                    k_cache.data_ptr(), v_cache.data_ptr(), T, (int)Hq,
                    (int)Hk, D, BS, (float)eps, is_fp8_cache(k_cache) ? 1 : 0,
@@ -496,14 +514,16 @@ void moe_tile(bool down, at::Tensor out, at::Tensor src, at::Tensor w,
 
 // fp32 parts [splits, M, N] of the product, not added up
 at::Tensor rows_tile_parts(at::Tensor x, at::Tensor w, long cols, long splits) {
-  check_bf16(x, "x"); check_bf16(w, "w");
+  check_bf16(w, "w");
+  TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 && x.dim() == 2
+              && x.stride(1) == 1 && x.stride(0) % 8 == 0, "x rows of bf16");
   const int M = x.size(0), K = x.size(1), N = w.size(0);
   TORCH_CHECK(w.size(1) == K && (uintptr_t)x.data_ptr() % 16 == 0 &&
               (uintptr_t)w.data_ptr() % 16 == 0, "rows_tile_parts shapes");
   at::Tensor parts = at::empty({splits, M, N}, x.options().dtype(at::kFloat));
   int err = 0;
   rows_tile_launch(nullptr, parts.data_ptr(), x.data_ptr(), w.data_ptr(), M, N,
-                   K, K, (int)cols, (int)splits, &err, cur_stream(x));
+                   K, x.stride(0), (int)cols, (int)splits, &err, cur_stream(x));
   TORCH_CHECK(!err, "rows_tile_parts: unsupported M=", M, " N=", N, " K=", K);
   HIP_CHECK_LAST();
   return parts;
@@ -615,12 +635,19 @@ at::Tensor mfma_probe(at::Tensor a, at::Tensor b) {
 #undef HIP_CHECK_LAST
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rms_norm", &rms_norm, "RMSNorm (bf16)");
-  m.def("fused_add_rms_norm", &fused_add_rms_norm, "residual+=x; x=norm(residual)*w");
+  m.def("fused_add_rms_norm", &fused_add_rms_norm,
+        "residual+=x (or the sum of parts); x=norm(residual)*w", py::arg("x"),
+        py::arg("residual"), py::arg("weight"), py::arg("eps"),
+        py::arg("parts") = py::none());
   m.def("rotary_embedding", &rotary_embedding, "in-place neox RoPE on q,k");
   m.def("silu_and_mul", &silu_and_mul, "silu(x[:d])*x[d:]");
   m.def("reshape_and_cache", &reshape_and_cache, "scatter K/V into paged pool");
   m.def("qkv_store", &qkv_store,
-        "head norms, rotation in place and cache write of a q|k|v row");
+        "head norms, rotation in place and cache write of a q|k|v row",
+        py::arg("qkv"), py::arg("q_heads"), py::arg("kv_heads"),
+        py::arg("q_norm"), py::arg("k_norm"), py::arg("cos_sin"),
+        py::arg("positions"), py::arg("slots"), py::arg("k_cache"),
+        py::arg("v_cache"), py::arg("eps"), py::arg("parts") = py::none());
   m.def("greedy_sample", &greedy_sample, "argmax over vocab");
   m.def("mla_decode", &mla_decode,
         "MLA absorbed decode over the paged latent cache (DeepSeek)");

@@ -71,6 +71,29 @@ __device__ __forceinline__ u16x8 f32_to_bf8(const float* in) {
   return v;
 }
 
+// Eight neighbours of a product cut over k: fp32 parts `stride` apart, added up in
+// their order and rounded, as the product's own join does it. Four parts are in
+// flight at a time.
+DEVICE_INLINE u16x8 join_parts8(const float* p, long stride, int parts) {
+  float sum[8];
+  for (int s0 = 0; s0 < parts; s0 += 4) {
+    f32x4 v[4][2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float* at = p + min(s0 + i, parts - 1) * stride;
+      v[i][0] = *reinterpret_cast<const f32x4*>(at);
+      v[i][1] = *reinterpret_cast<const f32x4*>(at + 4);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (s0 + i < parts)
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          sum[j] = s0 + i == 0 ? v[0][j / 4][j % 4] : sum[j] + v[i][j / 4][j % 4];
+  }
+  return f32_to_bf8(sum);
+}
+
 // Full-wave (64-lane) butterfly reductions.
 __device__ __forceinline__ float wave_reduce_sum(float x) {
 #pragma unroll

@@ -9,7 +9,7 @@
 #include <hip/hip_runtime.h>
 
 void embed_rows_scaled_launch(float*, const long*, const void*, int, int, long, float, int, hipStream_t);
-void add_layer_norm_launch(float*, const void*, const float*, const float*, void*, int, int, float, int, int, hipStream_t);
+int add_layer_norm_launch(float*, const void*, int, const float*, const float*, void*, int, int, float, int, int, hipStream_t);
 void head_norm_store_launch(void*, void*, long, int, int, int, const float*, const float*, int, float, float, const int*, const void*, long, const float*, void*, void*, const long*, long, int, int, int, float, int, int, int, hipStream_t);
 void value_page_store_launch(const void*, long, int, void*, const long*, long, const int*, int, int, int, int, int, int, hipStream_t);
 void route_topk_launch(int*, float*, const float*, int, const float*, int, int, int, int, int, int, int, int, float, hipStream_t);
@@ -84,10 +84,16 @@ void add_layer_norm(Tensor x, OptTensor a, OptTensor w, OptTensor b, double eps,
   const void* ap = nullptr;
   const float *wp = nullptr, *bp = nullptr;
   void* hp = nullptr;
-  int a_bf = 0, h_bf = 0;
+  int a_bf = 0, h_bf = 0, parts = 0;
   if (a.has_value()) {
     a_bf = act_kind(*a, "a");
-    TORCH_CHECK(a->sizes() == x.sizes());
+    if (a->dim() == 3) {
+      parts = (int)a->size(0);
+      TORCH_CHECK(!a_bf && parts >= 1 && a->size(1) == T && a->size(2) == W,
+                  "parts must be fp32 [n, T, W]");
+    } else {
+      TORCH_CHECK(a->sizes() == x.sizes());
+    }
     ap = a->data_ptr();
   }
   if (w.has_value()) {
@@ -101,8 +107,10 @@ void add_layer_norm(Tensor x, OptTensor a, OptTensor w, OptTensor b, double eps,
     bp = b->data_ptr<float>();
     hp = h->data_ptr();
   }
-  add_layer_norm_launch(x.data_ptr<float>(), ap, wp, bp, hp, T, W, (float)eps,
-                        a_bf, h_bf, cur_stream(x));
+  const int ok = add_layer_norm_launch(x.data_ptr<float>(), ap, parts, wp, bp,
+                                       hp, T, W, (float)eps, a_bf, h_bf,
+                                       cur_stream(x));
+  TORCH_CHECK(ok, "parts of rows of ", W, " at these addresses");
   HIP_CHECK_LAST();
 }
 

@@ -1,0 +1,102 @@
+"""Products cut over k whose parts the next kernel adds up: the same bits as
+the product's own join and that kernel; and the layer-norm rows of 16-byte
+loads at the edges of their lanes."""
+import pytest
+import torch
+
+from gpustack_amd import ops
+
+pytestmark = [pytest.mark.gpu,
+              pytest.mark.skipif(not torch.cuda.is_available(),
+                                 reason="needs a GPU")]
+
+
+def _gen(seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return lambda *s: torch.randn(*s, generator=g, device="cuda")
+
+
+def _joined(parts):
+    v = parts[0].clone()
+    for p in parts[1:]:
+        v += p
+    return v.bfloat16()
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 8, 11])
+@pytest.mark.parametrize("T,H", [(1, 64), (17, 2048), (48, 4096), (3, 8200)])
+def test_add_rms_norm(n, T, H):
+    rnd = _gen(n + T)
+    parts, res = rnd(n, T, H), rnd(T, H).bfloat16()
+    w = rnd(H).bfloat16()
+    x, r1, r2 = _joined(parts), res.clone(), res.clone()
+    ops.fused_add_rms_norm(x, r1, w, 1e-5)
+    got = ops.add_rms_norm(parts, r2, w, 1e-5)
+    assert torch.equal(got, x) and torch.equal(r1, r2)
+
+
+@pytest.mark.parametrize("n", [2, 4, 7])
+@pytest.mark.parametrize("D,Hq,Hk", [(64, 4, 4), (128, 32, 8), (256, 3, 1)])
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("kv", [torch.bfloat16, torch.float8_e4m3fn])
+def test_qkv_store(n, D, Hq, Hk, norm, kv):
+    rnd = _gen(n + D)
+    T = 21
+    parts = rnd(n, T, (Hq + 2 * Hk) * D)
+    qw, kw = (rnd(D).bfloat16(), rnd(D).bfloat16()) if norm else (None, None)
+    cs = ops.build_cos_sin_cache(D, D, 64).cuda()
+    pos = torch.arange(T, device="cuda") + 5
+    slots = torch.arange(T, device="cuda") * 2 - 1
+    slots[0] = -1
+    got = []
+    for given in (None, parts):
+        pools = [torch.zeros(8, Hk, 16, D, device="cuda").to(kv)
+                 for _ in range(2)]
+        qkv = _joined(parts) if given is None \
+            else torch.full(parts.shape[1:], 9.0, device="cuda").bfloat16()
+        ops.qkv_store(qkv, Hq, Hk, qw, kw, cs, pos, slots, *pools, 1e-5, given)
+        got.append([qkv] + [p.view(torch.uint8) for p in pools])
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+@pytest.mark.parametrize("T", [1, 65])
+@pytest.mark.parametrize("W", [8, 1000, 1004, 2048, 2056, 4096, 4104, 8192,
+                               8200])
+@pytest.mark.parametrize("add", ["nothing", "bf16", "fp32", "parts"])
+@pytest.mark.parametrize("out", [torch.bfloat16, torch.float32])
+def test_add_layer_norm(T, W, add, out):
+    rnd = _gen(W)
+    x = rnd(T, W) + 3
+    w, b = rnd(W), rnd(W)
+    a = {"nothing": None, "bf16": rnd(T, W).bfloat16(), "fp32": rnd(T, W),
+         "parts": rnd(3, T, W)}[add]
+    if add == "parts" and (W % 8 or W > 8192):
+        with pytest.raises(RuntimeError):
+            ops.add_layer_norm(x, a, w, b, 1e-5, torch.empty_like(x))
+        return
+    one = _joined(a) if add == "parts" else a
+    want = x.double() if one is None else x.double() + one.double()
+    ref = torch.nn.functional.layer_norm(want, (W,), w.double(), b.double(),
+                                         1e-5)
+    h = torch.full((T, W), 9.0, device="cuda").to(out)
+    ops.add_layer_norm(x, a, w, b, 1e-5, h)
+    # one fp32 addition; sums of W of them, then bf16 once
+    assert torch.equal(x, want.float()) if one is not None else True
+    err = (h.double() - ref).abs()
+    eps = 2.0 ** -8 if out == torch.bfloat16 else 0.0
+    assert bool((err <= ref.abs() * eps + 2e-5).all()), float(err.max())
+    y = x.clone()
+    ops.add_layer_norm(y, a, None, None, 1e-5, None)
+    if a is not None:
+        assert torch.equal(y, (x + one.float()))
+
+
+@pytest.mark.parametrize("M", [1, 17, 48, 128])
+@pytest.mark.parametrize("N,K", [(4096, 14336), (4096, 4096), (2048, 8192)])
+def test_products_come_in_parts(M, N, K):
+    rnd = _gen(M)
+    x, w = rnd(M, K).bfloat16(), (rnd(N, K) * K ** -0.5).bfloat16()
+    got = ops.linear_auto(x, w, parts=True)
+    if got.dim() == 3:
+        got = _joined(got)
+    assert torch.equal(got, ops.linear_auto(x, w))
