@@ -55,6 +55,10 @@ class DenseFF(nn.Module):
                                    requires_grad=False)
 
     def forward(self, h, x32=None):
+        if self.gated and self.act == "silu" and not self.extra:
+            g = ops.linear_silu(h, self.up_w)
+            if g is not None:
+                return ops.linear_auto(g, self.down_w, self.out_parts)
         u = ops.linear_auto(h, self.up_w)
         if self.gated:
             g = torch.empty(h.shape[0], self.ff, dtype=h.dtype,

@@ -686,8 +686,22 @@ class MLP(nn.Module):
 
     def forward(self, x, meta: ForwardMeta | None = None,
                 parts: bool = False):
+        lora = meta is not None and meta.lora is not None
+        act = None
+        if not (lora or self.no_gate or self.act == "gelu_tanh"
+                or self.gate_up_pack is not None):
+            act = ops.linear_silu(x, self.gate_up_w)
+        if act is None:
+            act = self._activated(x, meta if lora else None)
+        down = qlinear(act, self.down_w, self.down_pack,
+                       parts=parts and not lora)
+        if lora:
+            meta.lora.apply(self.layer_idx, act, down, self._down_projs)
+        return self.comm.all_reduce(down)
+
+    def _activated(self, x, meta):
         gu = qlinear(x, self.gate_up_w, self.gate_up_pack)
-        if meta is not None and meta.lora is not None:
+        if meta is not None:
             meta.lora.apply(self.layer_idx, x, gu, self._gu_projs)
         if self.no_gate:
             # Arcee: single up projection, relu^2 activation
@@ -703,12 +717,7 @@ class MLP(nn.Module):
             act = torch.empty(x.shape[0], self.i, dtype=x.dtype,
                               device=x.device)
             ops.silu_and_mul(act, gu)
-        lora = meta is not None and meta.lora is not None
-        down = qlinear(act, self.down_w, self.down_pack,
-                       parts=parts and not lora)
-        if lora:
-            meta.lora.apply(self.layer_idx, act, down, self._down_projs)
-        return self.comm.all_reduce(down)
+        return act
 
 
 class MoEMLP(nn.Module):

@@ -534,22 +534,13 @@ def linear_auto(x, w, parts: bool = False):
     F.linear everywhere else. `parts`: a product that is cut over k may come
     as its fp32 parts [n, M, N], for a consumer that adds them up itself
     (add_rms_norm, qkv_store, add_layer_norm) and saves the join's launch."""
-    import os
-
     import torch.nn.functional as F
 
-    if (x.is_cuda and x.dim() == 2 and w.dim() == 2
-            and os.environ.get("GPUSTACK_AMD_SKINNY_GEMM", "1") == "1"):
+    if _own_products(x, w):
         M, K = x.shape
         N = w.shape[0]
         plan = _rows_tile_plan(M, N, K)
-        if ((plan or _rows_gemm_wins(M, N, K)) and M > 0
-                and _products() is not None
-                and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
-                and w.is_contiguous() and w.data_ptr() % 16 == 0
-                and x.stride(1) == 1 and x.stride(0) % 8 == 0
-                and x.data_ptr() % 16 == 0
-                and not (x.requires_grad or w.requires_grad)):
+        if (plan or _rows_gemm_wins(M, N, K)) and _rows_take(x, w):
             if parts and plan and plan[1] > 1:
                 return _load_hip().rows_tile_parts(x, w, *plan)
             out = torch.empty(M, N, dtype=x.dtype, device=x.device)
@@ -564,6 +555,39 @@ def linear_auto(x, w, parts: bool = False):
                 and x.is_contiguous() and w.is_contiguous()):
             return skinny_gemm(x, w, splitk=4)
     return F.linear(x, w)
+
+
+def _own_products(x, w) -> bool:
+    import os
+
+    return (x.is_cuda and x.dim() == 2 and w.dim() == 2
+            and os.environ.get("GPUSTACK_AMD_SKINNY_GEMM", "1") == "1")
+
+
+def _rows_take(x, w) -> bool:
+    """Operands that the products for few rows take."""
+    return (x.shape[0] > 0 and _products() is not None
+            and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+            and w.is_contiguous() and w.data_ptr() % 16 == 0
+            and x.stride(1) == 1 and x.stride(0) % 8 == 0
+            and x.data_ptr() % 16 == 0
+            and not (x.requires_grad or w.requires_grad))
+
+
+def linear_silu(x, w):
+    """silu(gate) * up of the product with w = [gate rows; up rows], or None
+    where the activation is a launch of its own: the tiled product of up to
+    128 rows (_rows_tile_plan), not cut over k, ends in it."""
+    if not _own_products(x, w):
+        return None
+    plan = _rows_tile_plan(x.shape[0], w.shape[0], x.shape[1])
+    if not plan or plan[1] > 1 or plan[0] < 64 or w.shape[0] % 8 != 0 \
+            or not _rows_take(x, w):
+        return None
+    out = torch.empty(x.shape[0], w.shape[0] // 2, dtype=x.dtype,
+                      device=x.device)
+    _load_hip().rows_tile(out, x, w, *plan, silu=True)
+    return out
 
 
 def mfma_probe(a, b):

@@ -31,7 +31,7 @@ int moe_sort_slices(int);
 void moe_sort_launch(int*, int*, int*, int*, int*, int*, int*, const int*, int, int, int, int*, hipStream_t);
 void moe_sum_launch(void*, const void*, long, int, int, hipStream_t);
 void moe_tile_launch(int, void*, const void*, const void*, const int*, const int*, const int*, const int*, const int*, const float*, const void*, int, long, int, int, int, int*, hipStream_t);
-void rows_tile_launch(void*, void*, const void*, const void*, int, int, int, long, int, int, int*, hipStream_t);
+void rows_tile_launch(void*, void*, const void*, const void*, int, int, int, long, int, int, int, int*, hipStream_t);
 void rows_gemm_launch(void*, const void*, const void*, int, int, int, long, int*, hipStream_t);
 void w4_gemm_launch(void*, const void*, const void*, const void*, const void*, int, int, int, int*, hipStream_t);
 void w4_dequant_launch(void*, const void*, const void*, const void*, long, int, int*, hipStream_t);
@@ -523,20 +523,24 @@ at::Tensor rows_tile_parts(at::Tensor x, at::Tensor w, long cols, long splits) {
   at::Tensor parts = at::empty({splits, M, N}, x.options().dtype(at::kFloat));
   int err = 0;
   rows_tile_launch(nullptr, parts.data_ptr(), x.data_ptr(), w.data_ptr(), M, N,
-                   K, x.stride(0), (int)cols, (int)splits, &err, cur_stream(x));
+                   K, x.stride(0), (int)cols, (int)splits, 0, &err,
+                   cur_stream(x));
   TORCH_CHECK(!err, "rows_tile_parts: unsupported M=", M, " N=", N, " K=", K);
   HIP_CHECK_LAST();
   return parts;
 }
 
+// silu: w holds the gate's rows and behind them the up product's, out is
+// silu(gate) * up
 void rows_tile(at::Tensor out, at::Tensor x, at::Tensor w, long cols,
-               long splits) {
+               long splits, bool silu) {
   check_bf16(out, "out"); check_bf16(w, "w");
   TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 && x.dim() == 2
               && x.stride(1) == 1 && x.stride(0) % 8 == 0
               && (uintptr_t)x.data_ptr() % 16 == 0, "x rows of bf16");
-  const int M = x.size(0), K = x.size(1), N = w.size(0);
-  TORCH_CHECK(w.size(1) == K && out.size(0) == M && out.size(1) == N &&
+  const int M = x.size(0), K = x.size(1), N = out.size(1);
+  TORCH_CHECK(w.size(1) == K && out.size(0) == M &&
+              w.size(0) == (silu ? 2l * N : N) &&
               (uintptr_t)w.data_ptr() % 16 == 0, "rows_tile shapes");
   at::Tensor parts;
   if (splits > 1)
@@ -544,7 +548,7 @@ void rows_tile(at::Tensor out, at::Tensor x, at::Tensor w, long cols,
   int err = 0;
   rows_tile_launch(out.data_ptr(), splits > 1 ? parts.data_ptr() : nullptr,
                    x.data_ptr(), w.data_ptr(), M, N, K, x.stride(0),
-                   (int)cols, (int)splits, &err, cur_stream(x));
+                   (int)cols, (int)splits, silu ? 1 : 0, &err, cur_stream(x));
   TORCH_CHECK(!err, "rows_tile: unsupported M=", M, " N=", N, " K=", K);
   HIP_CHECK_LAST();
 }
@@ -674,7 +678,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_lab", &gemm_lab, "GEMM schedule lab variants (A/B vs hipBLASLt)");
   m.def("rows_tile_parts", &rows_tile_parts,
         "fp32 parts over k of a product of up to 128 rows");
-  m.def("rows_tile", &rows_tile, "bf16 product of up to 128 rows in tiles");
+  m.def("rows_tile", &rows_tile, "bf16 product of up to 128 rows in tiles",
+        py::arg("out"), py::arg("x"), py::arg("w"), py::arg("cols"),
+        py::arg("splits"), py::arg("silu") = false);
   m.def("rows_gemm", &rows_gemm, "bf16 product of up to 16 rows");
   m.def("moe_route", &moe_route, "router product and choice");
   m.def("moe_topk", &moe_topk, "softmax routing, top k");

@@ -100,3 +100,26 @@ def test_products_come_in_parts(M, N, K):
     if got.dim() == 3:
         got = _joined(got)
     assert torch.equal(got, ops.linear_auto(x, w))
+
+
+@pytest.mark.parametrize("M", [1, 16, 33, 64, 65, 96, 97, 128])
+@pytest.mark.parametrize("N,K,cols", [(128, 64, 64), (64, 256, 128),
+                                      (1000, 192, 64), (1000, 192, 128),
+                                      (36, 128, 128), (8192, 2048, 64)])
+def test_product_ends_in_the_activation(M, N, K, cols):
+    rnd = _gen(M + N)
+    x, w = rnd(M, K).bfloat16(), (rnd(2 * N, K) * K ** -0.5).bfloat16()
+    out = torch.full((M, N), 9.0, device="cuda").bfloat16()
+    ops._load_hip().rows_tile(out, x, w, cols, 1, silu=True)
+    h = x.double() @ w.double().T
+    ref = torch.nn.functional.silu(h[:, :N]) * h[:, N:]
+    # rounded to bf16 once; fp32 sums of K products of size K^-1/2
+    assert bool(((out.double() - ref).abs()
+                 <= ref.abs() * 2.0 ** -8 + 1e-4).all())
+
+
+def test_no_activation_where_there_is_no_such_product():
+    w = torch.zeros(64, 1024, device="cuda", dtype=torch.bfloat16)
+    x = torch.zeros(4, 1024, device="cuda", dtype=torch.bfloat16)
+    assert ops.linear_silu(x, w) is None
+    assert ops.linear_silu(x.cpu(), w.cpu()) is None
