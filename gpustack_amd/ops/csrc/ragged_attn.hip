@@ -313,8 +313,13 @@ constexpr int MKT = 64;            // keys per tile (16 per wave)
 constexpr int MSS = MKT + 4;       // fp32 score row stride
 constexpr int MPS = MKT + 8;       // bf16 weight row stride (16 B aligned)
 
-// NT: 16-channel n-tiles per wave (wave w owns n-tiles w, w+4, ...).
-template <int NT, typename TO>
+// NT: 16-channel n-tiles per wave (wave w owns n-tiles w, w+4, ...). DK: D / 32,
+// or 0 for any D. With DK a tile's values are asked for before its scores and
+// the next tile's keys, whose pages are known by then, behind them, so that a
+// tile waits for neither: 64 rows of 16 heads on 4 behind 200 to 3000 keys, with
+// the merge, in a window of 1024 36 -> 30 us, without one 67 -> 48, one row behind
+// 1000 16 -> 14.
+template <int NT, typename TO, int DK>
 __global__ __launch_bounds__(THREADS) void paged_attn_mfma_kernel(
     TO* __restrict__ out, const unsigned short* __restrict__ q,
     const unsigned short* __restrict__ k_cache,
@@ -369,23 +374,77 @@ __global__ __launch_bounds__(THREADS) void paged_attn_mfma_kernel(
   const KeyWalk walk = key_walk(lo, jmax, p.keep_first, MKT);
   const int per = (walk.n + nsplit - 1) / nsplit;
   const int v_end = min(walk.n, (split + 1) * per);
-  for (int v = split * per; v < v_end; ++v) {
+  auto page_at = [&](int pg) {
+    return (long)min(max(bt[min(pg, last_page)], 0), p.nblocks - 1);
+  };
+  // keys past jmax re-read key jmax (their weights are masked to zero below)
+  auto key_row = [&](int k0, long blk) {
+    const int key = min(k0 + wave * 16 + lc, jmax);
+    return k_cache + ((blk * p.G + g) * BS + (key & 15)) * (long)p.KW + koff +
+           lg * 8;
+  };
+  // 8 consecutive keys of one page; groups wholly past jmax read the last valid
+  // page (weights there are zero)
+  auto value_page = [&](int key, long blk) {
+    return v_cache + (blk * p.G + g) * (long)VW * BS + (key & 15);
+  };
+  u16x8 kreg[DK > 0 ? DK : 1], vreg[2][NT];
+  long vblk[2] = {0, 0};
+  const int v_begin = split * per;
+  if constexpr (DK > 0) {
+    if (v_begin < v_end) {
+      const int k0 = walk.tile(v_begin) * MKT;
+      const unsigned short* rowp = key_row(k0, page_at((k0 >> 4) + wave));
+#pragma unroll
+      for (int r = 0; r < DK; ++r)
+        kreg[r] = *reinterpret_cast<const u16x8*>(rowp + r * 32);
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+        vblk[ks] = page_at((k0 + ks * 32 + lg * 8) >> 4);
+    }
+  }
+  for (int v = v_begin; v < v_end; ++v) {
     const int k0 = walk.tile(v) * MKT;
     __syncthreads();   // Ql staged / previous tile's Pl and als consumed
     {
-      // scores: this wave's 16 keys; keys past jmax re-read key jmax (their
-      // weights are masked to zero below)
-      const int key = min(k0 + wave * 16 + lc, jmax);
-      const long blk = min(max(bt[key >> 4], 0), p.nblocks - 1);
-      const unsigned short* rowp =
-          k_cache + ((blk * p.G + g) * BS + (key & 15)) * (long)p.KW + koff;
       const unsigned short* qrow = Ql + lc * QS;
       f32x4 sacc{0.f, 0.f, 0.f, 0.f};
+      if constexpr (DK > 0) {
+        const int kn = walk.tile(min(v + 1, v_end - 1)) * MKT;
+        const long kblk = page_at((kn >> 4) + wave);
+        long vnext[2];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+          vnext[ks] = page_at((kn + ks * 32 + lg * 8) >> 4);
+          const unsigned short* pt =
+              value_page(k0 + ks * 32 + lg * 8, vblk[ks]);
+#pragma unroll
+          for (int i = 0; i < NT; ++i)
+            if ((wave + 4 * i) * 16 < VW)
+              vreg[ks][i] = *reinterpret_cast<const u16x8*>(
+                  pt + (long)((wave + 4 * i) * 16 + lc) * BS);
+        }
+#pragma unroll
+        for (int r = 0; r < DK; ++r)
+          sacc = ra_mfma(
+              *reinterpret_cast<const u16x8*>(qrow + r * 32 + lg * 8), kreg[r],
+              sacc);
+        if (v + 1 < v_end) {
+          const unsigned short* rowp = key_row(kn, kblk);
+#pragma unroll
+          for (int r = 0; r < DK; ++r)
+            kreg[r] = *reinterpret_cast<const u16x8*>(rowp + r * 32);
+        }
+        vblk[0] = vnext[0];
+        vblk[1] = vnext[1];
+      } else {
+        const unsigned short* rowp = key_row(k0, page_at((k0 >> 4) + wave));
 #pragma unroll 4
-      for (int r = 0; r < D; r += 32) {
-        const u16x8 a = *reinterpret_cast<const u16x8*>(qrow + r + lg * 8);
-        const u16x8 b = *reinterpret_cast<const u16x8*>(rowp + r + lg * 8);
-        sacc = ra_mfma(a, b, sacc);
+        for (int r = 0; r < D; r += 32) {
+          const u16x8 a = *reinterpret_cast<const u16x8*>(qrow + r + lg * 8);
+          const u16x8 b = *reinterpret_cast<const u16x8*>(rowp + r);
+          sacc = ra_mfma(a, b, sacc);
+        }
       }
 #pragma unroll
       for (int r = 0; r < 4; ++r)
@@ -438,18 +497,16 @@ __global__ __launch_bounds__(THREADS) void paged_attn_mfma_kernel(
       for (int ks = 0; ks < MKT; ks += 32) {
         const u16x8 a =
             *reinterpret_cast<const u16x8*>(Pl + lc * MPS + ks + lg * 8);
-        // 8 consecutive keys of one page; groups wholly past jmax read the
-        // last valid page (weights there are zero)
         const int keyb = k0 + ks + lg * 8;
-        const int pg = min(keyb >> 4, last_page);
-        const long blk = min(max(bt[pg], 0), p.nblocks - 1);
         const unsigned short* pt =
-            v_cache + (blk * p.G + g) * (long)VW * BS + (keyb & 15);
+            DK > 0 ? nullptr : value_page(keyb, page_at(keyb >> 4));
 #pragma unroll
         for (int i = 0; i < NT; ++i) {
           const int ch = (wave + 4 * i) * 16 + lc;
           if ((wave + 4 * i) * 16 < VW) {       // uniform over the wave
-            const u16x8 b = *reinterpret_cast<const u16x8*>(pt + (long)ch * BS);
+            u16x8 b;
+            if constexpr (DK > 0) b = vreg[ks / 32][i];
+            else b = *reinterpret_cast<const u16x8*>(pt + (long)ch * BS);
             acc[i] = ra_mfma(a, b, acc[i]);
           }
         }
@@ -861,7 +918,10 @@ void launch_mfma(void* out, const void* q, const void* kc, const void* vc,
                  float* ws_ml, hipStream_t s) {
   const size_t smem = (size_t)G16 * (p.D + 8) * 2 + (size_t)G16 * MPS * 2 +
                       (size_t)(G16 * MSS + 2 * G16) * sizeof(float);
-  paged_attn_mfma_kernel<NT, TO><<<dim3(ntiles, nsplit), THREADS, smem, s>>>(
+  const auto kern = NT == 2 && p.D == 128
+                        ? paged_attn_mfma_kernel<NT, TO, NT == 2 ? 4 : 0>
+                        : paged_attn_mfma_kernel<NT, TO, 0>;
+  kern<<<dim3(ntiles, nsplit), THREADS, smem, s>>>(
       (TO*)out, (const unsigned short*)q, (const unsigned short*)kc,
       (const unsigned short*)vc, p, ws_acc, ws_ml);
   if (nsplit > 1)
