@@ -110,6 +110,40 @@ def test_head_norm_store(dtype, mix, paged):
         assert (a.float() - b.float()).abs().max() <= tol
 
 
+@pytest.mark.parametrize("HQ,G,D,VW", [(4, 2, 64, 64), (16, 4, 128, 128),
+                                       (3, 3, 256, 24), (5, 1, 128, 136)])
+@pytest.mark.parametrize("mix", [False, True])
+@pytest.mark.parametrize("later", [False, True])
+@pytest.mark.parametrize("T", [1, 21])
+def test_head_norm_store_of_whole_lanes(HQ, G, D, VW, mix, later, T):
+    """Heads whose channels lanes of 8 share, value rows that end within one."""
+    nq, nk, nv, BS, nb = HQ * D, G * D, G * VW, 16, 5
+    qkv = _rand(T, nq + nk + nv, dtype=torch.bfloat16, std=2.0)
+    v_first = _rand(T, nq + nk + nv, dtype=torch.bfloat16, seed=9)[:, nq + nk:] \
+        if mix else None
+    lam = torch.tensor([0.3], device=DEV)
+    qw, kw = _rand(D, seed=1) + 1, _rand(D, seed=2) + 1
+    pos = _i32([(50 * t) % 2300 for t in range(T)])
+    slots = (torch.arange(T) * 3 + 1).to(DEV)
+    slots[-1] = -1
+    groups = _i32([[t, 1] for t in range(T)]) if later else None
+    outs = []
+    for impl in (ops, torch_ref):
+        q = torch.zeros(T, nq, dtype=torch.bfloat16, device=DEV)
+        kc = torch.zeros(nb, G, BS, D, dtype=torch.bfloat16, device=DEV)
+        vc = torch.zeros(nb, G, VW, BS, dtype=torch.bfloat16, device=DEV)
+        args = (q, qkv.clone(), nq, nk, qw, kw, D, 0.25, 1024, pos, v_first,
+                lam if mix else None, kc, vc, slots, 1e-5)
+        if impl is ops:
+            ops.head_norm_store(*args, page_groups=groups)
+        else:
+            torch_ref.head_norm_store(*args)
+        outs.append((q, kc, vc))
+    for a, b in zip(*outs):         # a bf16 rounding apart
+        a, b = a.float(), b.float()
+        assert bool(((a - b).abs() <= b.abs() * 2.0 ** -7 + 1e-5).all())
+
+
 @pytest.mark.parametrize("sigmoid", [True, False])
 @pytest.mark.parametrize("E,G,keep,gtop,top", [
     (8, 2, 1, 2, 3), (16, 1, 1, 1, 4), (12, 4, 2, 1, 5), (64, 8, 4, 2, 8),
