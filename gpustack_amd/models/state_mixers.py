@@ -88,7 +88,8 @@ class Mamba2Mixer(nn.Module):
         xbc = torch.empty(T, m.conv_channels, dtype=h.dtype, device=h.device)
         ops.causal_conv_silu(xbc, u, self.col_x, self.conv_w, self.conv_b,
                              conv_state, rg.seq_first, rg.seq_rows,
-                             rg.state_slots, rg.row_seq, rg.pos32)
+                             rg.state_slots, rg.row_seq, rg.pos32,
+                             single=rg.single)
         gn = m.groups * m.state
         y = torch.empty(T, m.inner, dtype=torch.float32, device=h.device)
         ops.state_scan(y, xbc, 0, m.inner, m.inner + gn, u, self.col_dt,

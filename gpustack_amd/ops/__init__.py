@@ -1160,11 +1160,12 @@ def short_conv(out, src, col0: int, w, b, conv_state, seq_first, seq_rows,
 
 
 def causal_conv_silu(out, src, col0: int, w, b, conv_state, seq_first,
-                     seq_rows, state_slots, row_seq, pos32) -> None:
+                     seq_rows, state_slots, row_seq, pos32,
+                     single: bool = False) -> None:
     if src.is_cuda:
         _load_state()       # models that call this run on that library
     short_conv(out, src, col0, w, b, conv_state, seq_first, seq_rows,
-               state_slots, row_seq, pos32)
+               state_slots, row_seq, pos32, single=single)
 
 
 def scan_run_rows(seq_news, heads: int, vdim: int) -> int:
