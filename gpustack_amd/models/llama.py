@@ -194,28 +194,28 @@ def qlinear(x, w, pack: "W4Pack | None", bias=None, parts: bool = False):
     """F.linear with an optional W4 runtime pack. `parts` as in
     ops.linear_auto.
 
-    Packed weights stay RESIDENT packed (the capacity goal). Up to 64 rows
+    Packed weights stay RESIDENT packed (the capacity goal). Up to 192 rows
     the packed product (ops/csrc/w4_gemm.hip) reads them as they are; more
     rows expand the weight into a transient bf16 tensor (allocator-cached)
-    and run the library GEMM at full MFMA rate. Measured on 28672x4096, us:
-    16 rows 21 against 98, 64 rows 77 against 102, 128 rows 134 against 107
-    (4096x14336: 20 / 50, 60 / 59, 110 / 70). GPUSTACK_AMD_W4_KERNEL=1 keeps
-    the packed product up to 1024 rows."""
+    and run the library GEMM at full MFMA rate. Measured, us, 64 rows:
+    28672x4096 33 against 105, 4096x14336 18 / 62, 128256x4096 134 / 584; 192
+    rows: 28672x4096 93 / 133, 4096x14336 48 / 104, 4096x4096 20 / 43; 256 rows
+    121 / 135, 63 / 74 and 25 / 34, but 10240x8192 reaches the expansion.
+    GPUSTACK_AMD_W4_KERNEL=1 keeps the packed product up to 1024 rows."""
     if pack is None:
         return ops.linear_auto(x, w, parts) if bias is None \
             else F.linear(x, w, bias)
     if x.is_cuda:
-        import os as _os
-
         hip = ops._load_hip()
-        most = 1024 if _os.environ.get("GPUSTACK_AMD_W4_KERNEL", "0") == "1" \
-            else 64
-        # whole workgroups of 64 columns, scales that fit the LDS
-        if 0 < x.shape[0] <= most and x.dim() == 2 \
-                and pack.shape[0] % 64 == 0 and pack.shape[1] <= 131072:
+        if _w4_takes(x, pack):
+            x = x.contiguous()
+            if parts and bias is None:
+                p = hip.w4_parts(x, pack.qw, pack.sc, pack.zs)
+                if p is not None:
+                    return p
             out = torch.empty(x.shape[0], pack.shape[0], dtype=x.dtype,
                               device=x.device)
-            hip.w4_gemm(out, x.contiguous(), pack.qw, pack.sc, pack.zs)
+            hip.w4_gemm(out, x, pack.qw, pack.sc, pack.zs)
             if bias is not None:
                 out += bias
             return out
@@ -226,6 +226,27 @@ def qlinear(x, w, pack: "W4Pack | None", bias=None, parts: bool = False):
 
     wt = dequant_w4_runtime(pack.qw, pack.sc, pack.zs).to(x.dtype)
     return F.linear(x, wt, bias)
+
+
+def _w4_takes(x, pack: "W4Pack") -> bool:
+    """True where the packed product takes x: rows up to its limit, whole
+    workgroups of 64 columns, scales that fit the LDS."""
+    import os
+
+    most = 1024 if os.environ.get("GPUSTACK_AMD_W4_KERNEL", "0") == "1" \
+        else 192
+    return (x.is_cuda and x.dim() == 2 and 0 < x.shape[0] <= most
+            and pack.shape[0] % 64 == 0 and pack.shape[1] <= 131072)
+
+
+def _gate_up_silu(x, w, pack: "W4Pack | None"):
+    """silu(gate) * up of the fused product where it ends in the activation,
+    else None."""
+    if pack is None:
+        return ops.linear_silu(x, w)
+    if not _w4_takes(x, pack):
+        return None
+    return ops._load_hip().w4_silu(x.contiguous(), pack.qw, pack.sc, pack.zs)
 
 
 class Attention(nn.Module):
@@ -688,9 +709,8 @@ class MLP(nn.Module):
                 parts: bool = False):
         lora = meta is not None and meta.lora is not None
         act = None
-        if not (lora or self.no_gate or self.act == "gelu_tanh"
-                or self.gate_up_pack is not None):
-            act = ops.linear_silu(x, self.gate_up_w)
+        if not (lora or self.no_gate or self.act == "gelu_tanh"):
+            act = _gate_up_silu(x, self.gate_up_w, self.gate_up_pack)
         if act is None:
             act = self._activated(x, meta if lora else None)
         down = qlinear(act, self.down_w, self.down_pack,

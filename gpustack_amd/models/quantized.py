@@ -129,9 +129,11 @@ def _frag_perm(K: int, device=None) -> torch.Tensor:
 
     Within each 128-k block, packed order is [lg(4)][chunk(4)][j(8)] while
     the source order is [chunk][lg][j] — this puts the 32 values of lane
-    lg's four MFMA B-fragments into one contiguous 16-byte load."""
-    arr = torch.arange(K, device=device).view(-1, 4, 4, 8)  # [blk, c, lg, j]
-    return arr.permute(0, 2, 1, 3).reshape(-1)
+    lg's four MFMA fragments into one contiguous 16-byte load. In a word the
+    even j fill the low half and the odd ones the high half: a shift and a
+    mask then leave two neighbours where a register of bf16 has them."""
+    arr = torch.arange(K, device=device).view(-1, 4, 4, 4, 2)
+    return arr.permute(0, 2, 1, 4, 3).reshape(-1)  # [blk, c, lg, j/2, j%2]
 
 
 def pack_w4_runtime(q: torch.Tensor, scales: torch.Tensor,

@@ -344,6 +344,14 @@ void rows_gemm_launch(void* out, const void* x, const void* w, int M, int N,
   else rows_gemm<1>(out, x, w, M, N, K, xs, s);
 }
 
+// out [MN] = the sum of the parts [splits, MN], MN a multiple of 4
+void rows_join_launch(void* out, const float* parts, long MN, int splits,
+                      hipStream_t s) {
+  if (MN == 0) return;
+  hipLaunchKernelGGL(rows_join_kernel, dim3((MN / 4 + 255) / 256), dim3(256), 0,
+                     s, (unsigned short*)out, parts, MN, splits);
+}
+
 // parts: fp32 [splits, M, N] where splits > 1, or the result, for any number of
 // rows, where out is null. silu: w is [2 N, K], out its activation [M, N].
 void rows_tile_launch(void* out, void* parts, const void* x, const void* w,

@@ -3,27 +3,45 @@
 // that prompt-sized products use in front of the library GEMM.
 //
 // Packed layout (models/quantized.py pack_w4_runtime): qw u8 [N, K/2] in
-// FRAGMENT ORDER — within each 128-k block, the 16 bytes lane group lg loads
-// hold exactly the 32 nibbles (4 MFMA k-chunks x 8 values) of its operand
-// fragments:
-//   nibble i (0..31) of lg's 16 bytes = q[row][blk*128 + (i/8)*32 + lg*8 + i%8]
+// FRAGMENT ORDER: within each 128-k block, the 16 bytes that lane group lg loads
+// hold the 32 weights (4 MFMA k-chunks x 8 values) of its operand fragments, word
+// c those of k = c*32 + lg*8 .. + 7. In a word value j is the nibble at bit
+// 4*(j/2) + 16*(j%2): neighbours lie 16 bits apart, as in a register of bf16.
 // Scales / zero-scales: bf16 [N, K/128], one group per 128-k block.
 // w = q * s - zs   (zs = zero * s, precomputed).
 //
-// Few rows (decode). A workgroup of 8 or 16 waves owns 16 NTW columns of up to
-// 64 rows; its waves take the k blocks in turn (neighbouring blocks of a row
-// are read together) and meet in the LDS at the end, so no second kernel and
-// no partial results in memory.
-//  - A nibble becomes bf16 without arithmetic: 0x4300 | q is 128 + q, two at
-//    a time (q_j beside q_{j+4}; x fragments are put in the same order with
-//    four v_perm). The products of a block are exact in q; its scale and
-//    offset are applied to the fp32 sums:
-//      out += s * (x . (128 + q)) - (128 s + zs) * sum(x),
-//    sum(x) coming from one more product with a fragment of ones, shared by
-//    the NTW column tiles. The weights are never rounded to bf16 here, as the
-//    expansion does.
-//  - 16-byte weight loads run one block ahead; scales are staged in the LDS.
-// Bound by the weight stream (0.5 bytes a weight).
+// A nibble becomes bf16 without arithmetic: 0x4300 | q is 128 + q, two at a time.
+// The products of a block are exact in q; its scale and offset are applied to the
+// fp32 sums:
+//   out += s * (x . (128 + q)) - (128 s + zs) * sum(x),
+// sum(x) coming from a product with a fragment of ones. The weights are never
+// rounded to bf16 here, as the expansion does.
+//
+// Tiles (w4_tile_kernel). 8 waves (4 where the columns are no multiple of 128)
+// have 16 columns each and all of up to 64 rows; more rows are more workgroups.
+// Steps of 256 k of x and of the weights go to two buffers in the LDS, whole
+// 128-byte lines of both by loads that write the LDS themselves, one step ahead.
+// 16-byte chunks are permuted through the lanes' addresses: of x's rows (512
+// bytes) XORed with the row, of the weights' (128 bytes) with (row >> 1). Weights
+// are the A operand: a lane ends with 4 neighbouring columns of a row. The sums of
+// x over a step's blocks are made once, by a wave each, and used a step later.
+// Narrow products are cut over k into fp32 parts, which the next kernel adds up.
+// What bounds it is the unpacking: some 150 vector instructions of a wave in a
+// step, two waves a SIMD, are most of the microsecond that it takes; at 64 rows the
+// reads of x from the LDS. Before, nibbles lay in order and x was permuted to fit
+// them, each wave made its own sums of x, and both came in pieces of 64 bytes, 16
+// rows an instruction, x again for every 16 to 64 columns. us, weights out of
+// memory, before -> now at 1 / 16 / 32 / 64 rows: 28672 x 4096 21 -> 21 / 23 -> 22
+// / 36 -> 23 / 81 -> 33, 4096 x 14336 12.8 -> 11.4 / 20 -> 12 / 33 -> 13 / 65 ->
+// 18, 6144 x 4096 7.3 -> 7.1 / 9.1 -> 7.4 / 14.3 -> 8.6 / 21 -> 12, 4096 x 4096
+// 6.0 -> 5.3 / 7.8 -> 5.7 / 12.3 -> 6.5 / 20 -> 8.8, 128256 x 4096 74 -> 61 / 83 ->
+// 64 / 138 -> 98 / 316 -> 134, 57344 x 8192 70 -> 65 / 79 -> 63 / - / 259 -> 125.
+// Two tiles of columns a wave, four waves: 27, 14, 9.1, 6.2, 73 at 16 rows and 42,
+// 22, 15, 9.9, 173 at 64; a third buffer in the LDS: no faster where one workgroup
+// fits a CU, 94 instead of 73 where it takes the second one's place.
+//
+// Rows (w4_rows_kernel): few rows of products that are narrow and have no consumer
+// for parts, and small ones. Straight from memory, k cut over the waves.
 #include "common.h"
 
 namespace {
@@ -37,7 +55,7 @@ DEVICE_INLINE f32x4 w4_mfma(u32x4 a, u32x4 b, f32x4 c) {
       __builtin_bit_cast(w4_s16x8, a), __builtin_bit_cast(w4_s16x8, b), c, 0, 0, 0);
 }
 
-// eight nibbles as bf16 128 + q in the order 0 4 1 5 2 6 3 7
+// eight nibbles as bf16 128 + q, in order
 DEVICE_INLINE u32x4 w4_bf16(unsigned int d) {
   u32x4 o;
 #pragma unroll
@@ -46,18 +64,205 @@ DEVICE_INLINE u32x4 w4_bf16(unsigned int d) {
   return o;
 }
 
-// eight bf16 in that order
-DEVICE_INLINE u32x4 w4_order(u32x4 v) {
-  u32x4 o;
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    o[2 * j] = __builtin_amdgcn_perm(v[2 + j], v[j], 0x05040100u);
-    o[2 * j + 1] = __builtin_amdgcn_perm(v[2 + j], v[j], 0x07060302u);
+constexpr int W4_SK = 2 * W4_KC;            // k of a step
+constexpr int W4_SZ = 32;                   // blocks of k whose scales are staged
+
+// What becomes of the sums: the result, fp32 parts [splits, M, N], or
+// silu(gate) * up in [M, N], qw then holding N gate rows and N up rows behind.
+enum W4Out { W4_ROWS, W4_PARTS, W4_SILU };
+
+template <int MT, int WAVES, W4Out OUT>
+__global__ __launch_bounds__(WAVES * WAVE_SIZE) void w4_tile_kernel(
+    void* __restrict__ out, const unsigned short* __restrict__ x,  // [M, K] bf16
+    const unsigned char* __restrict__ qw,   // [N, K/2] frag-ordered nibbles
+    const unsigned short* __restrict__ sc,  // [N, K/128] bf16 scale
+    const unsigned short* __restrict__ zs,  // [N, K/128] bf16 zero*scale
+    int M, int N, int K, int splits) {
+  constexpr int ROWS = 16 * MT, COLS = 16 * WAVES;
+  constexpr int XB = ROWS * W4_SK, BUF = XB + COLS * 64;  // elements of 2 bytes
+  constexpr int LX = 8 * MT / WAVES;        // loads of x of a wave in a step
+  constexpr int CT = OUT == W4_SILU ? COLS / 2 : COLS;    // columns of out
+  __shared__ __attribute__((aligned(1024))) unsigned short lds[2 * BUF];
+  __shared__ __attribute__((aligned(16))) unsigned int sz[W4_SZ * COLS];
+  __shared__ float xsum[2][2][ROWS];        // of a step's blocks, by its parity
+
+  const int nb = K / W4_KC, total = (nb + 1) / 2;
+  const int split = OUT == W4_PARTS ? blockIdx.x % splits : 0;
+  const int n0 = (OUT == W4_PARTS ? blockIdx.x / splits : blockIdx.x) * CT;
+  const int m0 = blockIdx.y * ROWS;
+  int from = 0, end = total;
+  if constexpr (OUT == W4_PARTS) {
+    from = (int)((long)total * split / splits);
+    end = (int)((long)total * (split + 1) / splits);
   }
-  return o;
+  const int tid = threadIdx.x, lane = tid & (WAVE_SIZE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE_SIZE);
+  const int lc = lane & 15, lg = lane >> 4;
+  // row of qw of one of the workgroup's columns: the first waves' are of the gate
+  auto at = [&](int c) {
+    return n0 + c + (OUT == W4_SILU && c >= CT ? N - CT : 0);
+  };
+
+  // an instruction brings 2 rows of x, or 8 of the weights, a wave its own
+  // columns; a step of one block (the last of an odd number) brings it twice
+  const unsigned short* xp[LX];
+  const unsigned char* wp[2];
+  int xc[LX], wc[2];
+#pragma unroll
+  for (int i = 0; i < LX; ++i) {
+    const int row = (wave * LX + i) * 2 + lane / 32;
+    xp[i] = x + (long)min(m0 + row, M - 1) * K;
+    xc[i] = (lane & 31) ^ (row & 15);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int row = i * 8 + lane / 8;
+    wp[i] = qw + (long)at(wave * 16 + row) * (K / 2);
+    wc[i] = (lane & 7) ^ ((row >> 1) & 7);
+  }
+
+  f32x4 acc[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const u32x4 ones = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
+  f32x4 z[2];                               // 128 s + zs of the step before
+  auto correct = [&](int i) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        const float xs = xsum[i & 1][h][m * 16 + lc];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[m][r] -= z[h][r] * xs;
+      }
+  };
+
+  for (; from < end; from += W4_SZ / 2) {    // once up to 4096 k
+    const int n = min(end - from, W4_SZ / 2);
+    // Steps start at the workgroup's own place in the row: rows lie a power of
+    // two apart, and workgroups that all read the same columns of their rows
+    // would meet on a few memory channels.
+    const int rot = blockIdx.x % n;
+    auto step = [&](int i) {
+      return from + (i + rot < n ? i + rot : i + rot - n);
+    };
+    auto stage = [&](int i) {
+      const int st = step(i);
+      const bool half = 2 * st + 1 >= nb;
+      unsigned short* to = lds + (i & 1) * BUF;
+#pragma unroll
+      for (int j = 0; j < LX; ++j)
+        load_to_lds(xp[j] + (long)st * W4_SK + (half ? xc[j] & 15 : xc[j]) * 8,
+                    to + (wave * LX + j) * 2 * W4_SK);
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        load_to_lds((const unsigned short*)(wp[j] + (long)st * W4_KC +
+                                            (half ? wc[j] & 3 : wc[j]) * 16),
+                    to + XB + (wave * 16 + j * 8) * 64);
+    };
+    stage(0);
+    // scale (low half) and offset of every column and block, 0 behind the last
+    const int b0 = 2 * from;
+    for (int u = tid; u < COLS * 2 * n; u += WAVES * WAVE_SIZE) {
+      const int c = u / (2 * n), b = u % (2 * n);
+      const long i = (long)at(c) * nb + b0 + b;
+      sz[b * COLS + c] =
+          b0 + b < nb ? (unsigned int)sc[i] | ((unsigned int)zs[i] << 16) : 0u;
+    }
+
+    for (int i = 0; i < n; ++i) {
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      if (i + 1 < n) stage(i + 1);
+      if (i > 0) correct(i - 1);
+      const unsigned short* xl = lds + (i & 1) * BUF + lc * W4_SK;
+      const unsigned short* wl =
+          lds + (i & 1) * BUF + XB + (wave * 16 + lc) * 64;
+      const int b = 2 * (step(i) - from);
+      // sums of x over the blocks, each by one of the waves for all
+#pragma unroll
+      for (int j = 0; j < (2 * MT + WAVES - 1) / WAVES; ++j) {
+        const int q = wave + j * WAVES, h = q / MT, m = q % MT;
+        if (q >= 2 * MT) break;
+        f32x4 xs = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          xs = w4_mfma(ones,
+                       *reinterpret_cast<const u32x4*>(
+                           xl + m * 16 * W4_SK + ((h * 16 + c * 4 + lg) ^ lc) * 8),
+                       xs);
+        if (lg == 0) xsum[i & 1][h][m * 16 + lc] = xs[0];
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const u32x4 w4 = *reinterpret_cast<const u32x4*>(
+            wl + ((h * 4 + lg) ^ ((lc >> 1) & 7)) * 8);
+        f32x4 p[MT];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const u32x4 wf = w4_bf16(w4[c]);
+#pragma unroll
+          for (int m = 0; m < MT; ++m)
+            p[m] = w4_mfma(wf,
+                           *reinterpret_cast<const u32x4*>(
+                               xl + m * 16 * W4_SK +
+                               ((h * 16 + c * 4 + lg) ^ lc) * 8),
+                           c ? p[m] : f32x4{0.f, 0.f, 0.f, 0.f});
+        }
+        const u32x4 v = *reinterpret_cast<const u32x4*>(
+            sz + (b + h) * COLS + wave * 16 + lg * 4);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float s = __builtin_bit_cast(float, v[r] << 16);
+          z[h][r] = 128.f * s + __builtin_bit_cast(float, v[r] & 0xffff0000u);
+#pragma unroll
+          for (int m = 0; m < MT; ++m) acc[m][r] += s * p[m][r];
+        }
+      }
+    }
+    __syncthreads();
+    correct(n - 1);
+    __syncthreads();                         // the buffers are done with
+  }
+
+  // D[column = lg*4 + r][row = lc]
+  constexpr int US = CT + 4;                 // the up product's rows in the LDS
+  float* up = reinterpret_cast<float*>(lds);
+  if constexpr (OUT == W4_SILU) {
+    if (wave >= WAVES / 2)
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+        *reinterpret_cast<f32x4*>(up + (m * 16 + lc) * US +
+                                  (wave - WAVES / 2) * 16 + lg * 4) = acc[m];
+    __syncthreads();
+    if (wave >= WAVES / 2) return;
+  }
+  const int col = n0 + wave * 16 + lg * 4;
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const int row = m0 + m * 16 + lc;
+    if (row >= M) continue;
+    f32x4 v = acc[m];
+    if constexpr (OUT == W4_PARTS) {
+      *reinterpret_cast<f32x4*>((float*)out + ((long)split * M + row) * N + col) =
+          v;
+    } else {
+      if constexpr (OUT == W4_SILU) {
+        const f32x4 u = *reinterpret_cast<const f32x4*>(
+            up + (m * 16 + lc) * US + wave * 16 + lg * 4);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = v[r] / (1.f + __expf(-v[r])) * u[r];
+      }
+      uint2 o;
+      o.x = (unsigned)f2bf(v[0]) | (unsigned)f2bf(v[1]) << 16;
+      o.y = (unsigned)f2bf(v[2]) | (unsigned)f2bf(v[3]) << 16;
+      *reinterpret_cast<uint2*>((unsigned short*)out + (long)row * N + col) = o;
+    }
+  }
 }
 
-template <int MT, int NTW, int WAVES>
+template <int NTW, int WAVES>
 __global__ __launch_bounds__(WAVES * WAVE_SIZE) void w4_rows_kernel(
     unsigned short* __restrict__ out,       // [M, N] bf16
     const unsigned short* __restrict__ x,   // [M, K] bf16
@@ -65,7 +270,7 @@ __global__ __launch_bounds__(WAVES * WAVE_SIZE) void w4_rows_kernel(
     const unsigned short* __restrict__ sc,  // [N, K/128] bf16 scale
     const unsigned short* __restrict__ zs,  // [N, K/128] bf16 zero*scale
     int M, int N, int K) {
-  constexpr int COLS = 16 * NTW, ROWS = 16 * MT;
+  constexpr int COLS = 16 * NTW, ROWS = 16;
   extern __shared__ __attribute__((aligned(16))) float w4_lds[];
   const int nb = K / W4_KC;
   // scales of the workgroup's columns, [nb][COLS] (s low half, zs high), then
@@ -84,10 +289,7 @@ __global__ __launch_bounds__(WAVES * WAVE_SIZE) void w4_rows_kernel(
 #pragma unroll
   for (int t = 0; t < NTW; ++t)
     wp[t] = qw + (long)(n0 + t * 16 + lc) * (K / 2) + lg * 16;
-  const unsigned short* xp[MT];
-#pragma unroll
-  for (int t = 0; t < MT; ++t)
-    xp[t] = x + (long)min(m0 + t * 16 + lc, M - 1) * K + lg * 8;
+  const unsigned short* xp = x + (long)min(m0 + lc, M - 1) * K + lg * 8;
 
   // block numbers start at the workgroup's own place in the row: rows lie a
   // power of two apart, and workgroups that all read the same columns of
@@ -107,47 +309,29 @@ __global__ __launch_bounds__(WAVES * WAVE_SIZE) void w4_rows_kernel(
   }
   __syncthreads();
 
-  f32x4 acc[MT][NTW];
+  f32x4 acc[NTW];
 #pragma unroll
-  for (int i = 0; i < MT; ++i)
-#pragma unroll
-    for (int t = 0; t < NTW; ++t) acc[i][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < NTW; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
   const u32x4 ones = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
 
   auto multiply = [&](int b) {
-    u32x4 xa[MT][4];
+    u32x4 xa[4];
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+    for (int c = 0; c < 4; ++c)
+      xa[c] = *reinterpret_cast<const u32x4*>(xp + b * W4_KC + c * 32);
+    f32x4 xs = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int c = 0; c < 4; ++c)
-        xa[i][c] = w4_order(*reinterpret_cast<const u32x4*>(
-            xp[i] + b * W4_KC + c * 32));
-    f32x4 xs[MT];
-#pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      xs[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int c = 0; c < 4; ++c) xs[i] = w4_mfma(xa[i][c], ones, xs[i]);
-    }
+    for (int c = 0; c < 4; ++c) xs = w4_mfma(xa[c], ones, xs);
 #pragma unroll
     for (int t = 0; t < NTW; ++t) {
-      f32x4 p[MT];
+      f32x4 p = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int i = 0; i < MT; ++i) p[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const u32x4 wf = w4_bf16(wc[t][c]);
-#pragma unroll
-        for (int i = 0; i < MT; ++i) p[i] = w4_mfma(xa[i][c], wf, p[i]);
-      }
+      for (int c = 0; c < 4; ++c) p = w4_mfma(xa[c], w4_bf16(wc[t][c]), p);
       const unsigned int v = sz[b * COLS + t * 16 + lc];
       const float s = __builtin_bit_cast(float, v << 16);
       const float z = 128.f * s + __builtin_bit_cast(float, v & 0xffff0000u);
 #pragma unroll
-      for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          acc[i][t][r] += s * p[i][r] - z * xs[i][r];
+      for (int r = 0; r < 4; ++r) acc[t][r] += s * p[r] - z * xs[r];
     }
   };
   int j = wave;
@@ -166,13 +350,10 @@ __global__ __launch_bounds__(WAVES * WAVE_SIZE) void w4_rows_kernel(
   // D[row = lg*4 + r][col = lc] per 16x16 tile
   float* red = w4_lds;
 #pragma unroll
-  for (int i = 0; i < MT; ++i)
+  for (int t = 0; t < NTW; ++t)
 #pragma unroll
-    for (int t = 0; t < NTW; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        red[(wave * ROWS + i * 16 + lg * 4 + r) * COLS + t * 16 + lc] =
-            acc[i][t][r];
+    for (int r = 0; r < 4; ++r)
+      red[(wave * ROWS + lg * 4 + r) * COLS + t * 16 + lc] = acc[t][r];
   __syncthreads();
   for (int u = tid; u < ROWS * COLS; u += WAVES * WAVE_SIZE) {
     const int row = m0 + u / COLS;
@@ -212,7 +393,7 @@ __global__ __launch_bounds__(256) void w4_dequant_kernel(
       unsigned short o[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j)
-        o[j] = f2bf((float)((d >> (4 * j)) & 0xF) * s - z);
+        o[j] = f2bf((float)((d >> (j / 2 * 4 + j % 2 * 16)) & 0xF) * s - z);
       *reinterpret_cast<u16x8*>(out + row * K + blk * 128 + c * 32 + lg * 8) =
           *reinterpret_cast<u16x8*>(o);
     }
@@ -236,50 +417,121 @@ void w4_dequant_launch(void* out, const void* qw, const void* sc,
 }
 
 namespace {
-template <int MT, int NTW, int WAVES>
+template <int NTW, int WAVES>
 void w4_rows(void* out, const void* x, const void* qw, const void* sc,
              const void* zs, int M, int N, int K, hipStream_t s) {
   const size_t scales = (size_t)(K / W4_KC) * 16 * NTW * 4;
-  const size_t sums = (size_t)WAVES * 16 * MT * 16 * NTW * 4;
-  hipLaunchKernelGGL((w4_rows_kernel<MT, NTW, WAVES>),
-                     dim3(N / (16 * NTW), (M + 16 * MT - 1) / (16 * MT)),
+  const size_t sums = (size_t)WAVES * 16 * 16 * NTW * 4;
+  hipLaunchKernelGGL((w4_rows_kernel<NTW, WAVES>),
+                     dim3(N / (16 * NTW), (M + 15) / 16),
                      dim3(WAVES * WAVE_SIZE), scales > sums ? scales : sums, s,
                      (unsigned short*)out, (const unsigned short*)x,
                      (const unsigned char*)qw, (const unsigned short*)sc,
                      (const unsigned short*)zs, M, N, K);
 }
+
+template <int MT, int WAVES, W4Out OUT>
+void w4_tile(void* out, const void* x, const void* qw, const void* sc,
+             const void* zs, int M, int N, int K, int splits, hipStream_t s) {
+  constexpr int CT = (OUT == W4_SILU ? 8 : 16) * WAVES;
+  hipLaunchKernelGGL((w4_tile_kernel<MT, WAVES, OUT>),
+                     dim3(N / CT * splits, (M + 16 * MT - 1) / (16 * MT)),
+                     dim3(WAVES * WAVE_SIZE), 0, s, out,
+                     (const unsigned short*)x, (const unsigned char*)qw,
+                     (const unsigned short*)sc, (const unsigned short*)zs, M, N,
+                     K, splits);
+}
+
+int w4_waves(int N) { return N % 128 == 0 ? 8 : 4; }
+
+template <W4Out OUT>
+void w4_tiles(void* out, const void* x, const void* qw, const void* sc,
+              const void* zs, int M, int N, int K, int splits, hipStream_t s) {
+#define W4_TILE(MT)                                                            \
+  do {                                                                         \
+    if (OUT == W4_SILU || w4_waves(N) == 8)                                    \
+      w4_tile<MT, 8, OUT>(out, x, qw, sc, zs, M, N, K, splits, s);             \
+    else if constexpr (OUT != W4_SILU)                                         \
+      w4_tile<MT, 4, OUT>(out, x, qw, sc, zs, M, N, K, splits, s);             \
+  } while (0)
+  if (M <= 16) W4_TILE(1);
+  else if (M <= 32) W4_TILE(2);
+  else W4_TILE(4);
+#undef W4_TILE
+}
 }  // namespace
 
-// The form by columns: workgroups of four column tiles per wave (two at 64
-// rows) from 448 of them on; of two from 160 on, with 16 waves while x is one
-// row tile (6144 x 4096, us at 16 rows: 9.1 against 12.3 with one tile, at 64
-// rows 21.5 against 33.7); else of one, which keeps every CU on the stream
-// (4096 x 4096 at 16 rows: 7.6 against 8.7 with two), with 16 waves for long
-// rows (4096 x 14336 at one row: 11.9 against 14.5). The scales of K / 128
-// blocks stay under 64 KB.
-void w4_gemm_launch(void* out, const void* x, const void* qw, const void* sc,
-                    const void* zs, int M, int N, int K,
-                    int* err_unsupported, hipStream_t s) {
-  *err_unsupported = 0;
-  if (N % 64 != 0 || K % W4_KC != 0 || K / W4_KC > 1024) {
-    *err_unsupported = 1;
-    return;
-  }
+// Shapes that have a product: whole workgroups of 64 columns, blocks of 128 k.
+bool w4_has(int N, int K) {
+  return N % 64 == 0 && K % W4_KC == 0 && K > 0 && K / W4_KC <= 1024;
+}
+
+// Parts over k: one workgroup a CU, up to 16 rows of long rows two, 8 parts at
+// most. us at 16 rows: 4096 x 14336 (32 groups) 4 parts 20, 8 12, 16 13; 6144 x
+// 4096 (48) 2 12, 5 7.4, 8 7.3; 8192 x 28672 (64) 4 37, 8 29; 10240 x 8192 (80) 3
+// 16, 6 15; at 64 rows: 6144 x 4096 5 12, 8 15; 10240 x 8192 3 25, 6 30.
+int w4_splits(int M, int N, int K) {
+  const int groups = N / (16 * w4_waves(N)), total = (K / W4_KC + 1) / 2;
+  int splits = (M <= 16 && K >= 8192 ? 512 : 256) / groups;
+  if (splits > 8) splits = 8;
+  if (splits > total) splits = total;
+  return splits > 1 ? splits : 1;
+}
+
+// Products for which parts do not pay even where the next kernel adds them up: few
+// rows of short ones (at one row 6144 x 4096 7.1 against 7.3 and 4096 x 4096 5.3
+// against 6.0, which their consumer's reading costs; 4096 x 14336 11.4 / 12.8,
+// 8192 x 28672 29 / 39), and small ones (6144 x 1920 at 16 rows 5.0 / 5.3).
+bool w4_cuts(int M, int N, int K) {
+  return (M >= 8 || K >= 8192) && (long)N * K > 12l << 20 &&
+         w4_splits(M, N, K) > 1;
+}
+
+// The whole result: rows where these are few and the product is narrow (28672 x
+// 4096 at one row 20.7 against 21.4; 57344 x 8192 70 / 65), unless k is long and
+// parts with a join (3 us) gain more (4096 x 14336 at 16 rows 20 against 12 + 3),
+// and for small products (6144 x 1920 at 64 rows 10 against 8 + 3).
+bool w4_by_rows(int M, int N, int K) {
+  if (M <= 16 && N < 32768 && !(M > 8 && K >= 8192)) return true;
+  return M <= 64 && (long)N * K <= 12l << 20;
+}
+
+// parts: fp32 [splits, M, N]. x, qw and parts at 16-byte addresses.
+void w4_parts_launch(float* parts, const void* x, const void* qw, const void* sc,
+                     const void* zs, int M, int N, int K, int splits,
+                     hipStream_t s) {
+  if (M > 0) w4_tiles<W4_PARTS>(parts, x, qw, sc, zs, M, N, K, splits, s);
+}
+
+// out [M, N] = silu(gate) * up, qw of N gate rows and N up rows, N a multiple of
+// 64. x, qw and out at 16-byte addresses.
+void w4_silu_launch(void* out, const void* x, const void* qw, const void* sc,
+                    const void* zs, int M, int N, int K, hipStream_t s) {
+  if (M > 0) w4_tiles<W4_SILU>(out, x, qw, sc, zs, M, N, K, 1, s);
+}
+
+// One launch. x, qw and out at 16-byte addresses.
+void w4_tile_launch(void* out, const void* x, const void* qw, const void* sc,
+                    const void* zs, int M, int N, int K, hipStream_t s) {
+  if (M > 0) w4_tiles<W4_ROWS>(out, x, qw, sc, zs, M, N, K, 1, s);
+}
+
+// The form by columns: workgroups of four column tiles per wave from 448 of them
+// on; of two from 160 on, with 16 waves (6144 x 4096, us at 16 rows: 9.1 against
+// 12.3 with one tile); else of one, which keeps every CU on the stream (4096 x
+// 4096 at 16 rows: 7.6 against 8.7 with two), with 16 waves for long rows (4096 x
+// 14336 at one row: 11.9 against 14.5). The scales of K / 128 blocks stay under
+// 64 KB.
+void w4_rows_launch(void* out, const void* x, const void* qw, const void* sc,
+                    const void* zs, int M, int N, int K, hipStream_t s) {
   if (M == 0) return;
   const int nb = K / W4_KC;
   const int ntw = N / 64 >= 448 && nb <= 256 ? 4
                   : N / 32 >= 160 && nb <= 512 ? 2 : 1;
 #define W4_ARGS out, x, qw, sc, zs, M, N, K, s
-#define W4_ROWS(MT)                                                          \
-  do {                                                                       \
-    if (ntw == 4) w4_rows<MT, (MT) == 4 ? 2 : 4, 8>(W4_ARGS);                \
-    else if (ntw == 2) w4_rows<MT, 2, (MT) == 1 ? 16 : 8>(W4_ARGS);          \
-    else if (nb >= 64 && (MT) <= 2) w4_rows<MT, 1, (MT) <= 2 ? 16 : 8>(W4_ARGS); \
-    else w4_rows<MT, 1, 8>(W4_ARGS);                                         \
-  } while (0)
-  if (M <= 16) W4_ROWS(1);
-  else if (M <= 32) W4_ROWS(2);
-  else W4_ROWS(4);
+  if (ntw == 4) w4_rows<4, 8>(W4_ARGS);
+  else if (ntw == 2) w4_rows<2, 16>(W4_ARGS);
+  else if (nb >= 64) w4_rows<1, 16>(W4_ARGS);
+  else w4_rows<1, 8>(W4_ARGS);
 #undef W4_ARGS
-#undef W4_ROWS
 }

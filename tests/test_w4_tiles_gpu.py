@@ -1,0 +1,83 @@
+"""Tiled product with packed int4 weights: rows at the edges of its row tiles and
+above one workgroup's 64, steps of one block at the end, several chunks of staged
+scales, four and eight waves, parts over k, and the activation behind it, against
+float64; the forms that the launch chooses between agree with each other."""
+import pytest
+import torch
+
+pytestmark = [pytest.mark.gpu,
+              pytest.mark.skipif(not torch.cuda.is_available(),
+                                 reason="needs a GPU")]
+
+
+def _hip():
+    from gpustack_amd import ops
+
+    return ops._load_hip()
+
+
+def _case(M, N, K, size=1.0):
+    """x, the packed weight, the weight in float64 and a bound for the sums: they
+    run over 128 + q and are corrected by 128 times the sum of x."""
+    import gpustack_amd.engine  # noqa: F401  (package import order)
+    from gpustack_amd.models.quantized import pack_w4_runtime
+
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    q = torch.randint(0, 16, (N, K), generator=g, device="cuda")
+    sc = (torch.rand(N, K // 128, generator=g, device="cuda") * 0.05 + 0.01) * size
+    zr = torch.randint(0, 16, (N, K // 128), generator=g, device="cuda").float()
+    pack = pack_w4_runtime(q, sc, zr, 128)
+    x = (torch.randn(M, K, generator=g, device="cuda") + 0.5).bfloat16()
+    wide = lambda t: t.double().repeat_interleave(128, 1)
+    s, z = wide(pack[1]), wide(pack[2])
+    return x, pack, q.double() * s - z, x.double().abs() @ (s * 144 + z.abs()).T
+
+
+@pytest.mark.parametrize("M", [1, 8, 16, 17, 32, 33, 64, 65, 130])
+@pytest.mark.parametrize("N,K", [(32768, 384), (33024, 4480), (32832, 2176),
+                                 (4096, 3328), (1088, 12416)])
+def test_product(M, N, K):
+    x, (qw, s, z), w, size = _case(M, N, K)
+    ref = x.double() @ w.T
+    out = torch.full((M, N), 9.0, device="cuda").bfloat16()
+    _hip().w4_gemm(out, x, qw, s, z)
+    # rounded to bf16 once; fp32 sums
+    assert bool(((out.double() - ref).abs()
+                 <= ref.abs() * 2.0 ** -8 + size * 2.0 ** -18).all())
+    parts = _hip().w4_parts(x, qw, s, z)
+    cut = N < 30000 and (M >= 8 or K >= 8192)
+    assert (parts is not None) == cut
+    if cut:
+        assert parts.dtype == torch.float32 and parts.shape[1:] == out.shape
+        assert bool(((parts.double().sum(0) - ref).abs()
+                     <= size * 2.0 ** -18).all())
+    # the general form, which operands at other than 16-byte addresses take
+    y = torch.empty(M * K + 4, device="cuda", dtype=torch.bfloat16)[4:].view(M, K)
+    y.copy_(x)
+    general = torch.full_like(out, 9.0)
+    _hip().w4_gemm(general, y, qw, s, z)
+    assert _hip().w4_parts(y, qw, s, z) is None
+    assert bool(((general.double() - ref).abs()
+                 <= ref.abs() * 2.0 ** -8 + size * 2.0 ** -18).all())
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 65])
+@pytest.mark.parametrize("N,K", [(22016, 384), (24576, 4352)])
+def test_product_ends_in_the_activation(M, N, K):
+    x, (qw, s, z), w, size = _case(M, N, K, 1 / 16)
+    act = _hip().w4_silu(x, qw, s, z)
+    h, n = x.double() @ w.T, N // 2
+    g, u = h[:, :n], h[:, n:]
+    ref = torch.nn.functional.silu(g) * u
+    eg, eu = (size[:, :n] * 2.0 ** -18, size[:, n:] * 2.0 ** -18)
+    # silu's slope is under 1.1 and it is no larger than its argument; the
+    # exponential's own error is a few units of fp32
+    bound = ref.abs() * (2.0 ** -8 + 2.0 ** -20) + 1.1 * eg * (u.abs() + eu) \
+        + g.abs() * eu
+    assert bool(((act.double() - ref).abs() <= bound).all())
+
+
+def test_none_where_there_is_no_such_form():
+    x, (qw, s, z), _, _ = _case(4, 192, 256)
+    assert _hip().w4_silu(x, qw, s, z) is None
+    assert _hip().w4_parts(x, qw, s, z) is None
