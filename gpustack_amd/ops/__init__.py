@@ -434,9 +434,9 @@ def _rows_gemm_wins(M: int, N: int, K: int) -> bool:
 
 
 def _rows_tile_plan(M: int, N: int, K: int):
-    """(columns of a tile, parts of K) where the tiled product of up to 128
+    """(columns of a tile, parts of K) where the tiled product of up to 512
     rows (rows_tile_kernel in ops/csrc/rows_gemm.hip) measured fastest, else
-    None. The split aims at one workgroup a CU (256); us against the library,
+    None. Above 128 rows _tall_tile_plan has the rule. The split aims at one workgroup a CU (256); us against the library,
     or up to 16 rows against the better of it and the decode product, weights
     out of HBM:
     up to 10240 columns, 48 rows: 4096x14336 26.0 / 36.3, 4096x4096 11.8 / 13.8,
@@ -464,8 +464,10 @@ def _rows_tile_plan(M: int, N: int, K: int):
     up to 16 rows: 28672x4096 40 / 43 at one and 41 / 53 at 16, 4096x11008
     17 / 31, 22016x4096 32 / 39, 128256x4096 175 / 178, but 16384x4096 at one
     row 27 / 26."""
-    if not 0 < M <= 128 or K % 64 != 0 or N % 8 != 0 or min(N, K) < 1024:
+    if not 0 < M <= 512 or K % 64 != 0 or N % 8 != 0 or min(N, K) < 1024:
         return None
+    if M > 128:
+        return _tall_tile_plan(M, N, K)
     t64, t128 = -(-N // 64), -(-N // 128)
     if N > 10240:
         wide = 160 <= t128 <= 256 or t128 >= 500 or M > 64 and t128 > 256
@@ -503,6 +505,34 @@ def _rows_tile_plan(M: int, N: int, K: int):
         else:
             plan = 128, 256 // t128
     return plan if wins else None
+
+
+def _tall_tile_plan(M: int, N: int, K: int):
+    """_rows_tile_plan for 129 to 512 rows: long rows of up to 10240 columns,
+    which leave the library's tiles few and its chip idle. Cut over k into up
+    to 8 parts, as many as two workgroups a CU take (4096x14336 at 256 rows:
+    four parts 45 without their join, eight 39). us against the library, with
+    the join, weights out of HBM:
+    160 rows: 4096x14336 44 / 82, 10240x9216 64 / 73, 1024x14336 21 / 33,
+    5120x5120 27 / 37; 256 rows: 4096x14336 49 / 60, 6144x12288 61 / 109,
+    8192x7168 51 / 68, 3072x6144 26 / 29, but 2560x6144 at 136 rows 22 / 20
+    and 8192x4096 at 176 34 / 28; 384 rows: 5120x14336 72 / 87, 2048x11008
+    34 / 46, but 4096x9216 55 / 51 and 6144x11008 88 / 90; 512 rows:
+    4096x14336 72 / 88, 4096x6144 38 / 44, but 5120x11008 95 / 93."""
+    rows = -(-M // 128)
+    if rows == 2:
+        wins = N <= 10240 and K >= (
+            7168 if 1024 < N < 3072 else 6144 if N < 3072 else 5120)
+    elif rows == 3:
+        wins = N <= 5120 and K >= (11008 if 2048 < N <= 4096 else 6144)
+    else:
+        wins = N <= 4096 and K >= 6144
+    if not wins:
+        return None
+    t128 = rows * -(-N // 128)
+    if t128 < 32:
+        return 64, 8
+    return 128, min(8, 512 // t128)
 
 
 def router_plan(T: int, E: int, H: int):

@@ -113,6 +113,10 @@ __global__ __launch_bounds__(RG_THREADS) void rows_gemm_kernel(
 // of conflicts for 16 rows of one chunk. Weights are the A operand, so a lane
 // ends with 4 neighbouring columns of a row. Few columns are cut over k as
 // well, into fp32 parts that rows_join_kernel adds up.
+// More than 128 rows are row tiles of their own, always in parts. (Row tiles of a
+// piece of the weights one behind the other on an XCD, for its L2, lost: 512 rows
+// of 4096 x 14336 64 -> 77 us; one behind the other in time the Infinity Cache
+// serves them, and 4 or 8 parts leave an XCD a quarter or less of x.)
 // Bound by the weight stream: 28672 x 4096 at 48 rows 41 us (5.7 TB/s; the
 // library 51), 4096 x 14336 in four
 // parts 26 with the join (36), 128256 x 4096 182 (254). One workgroup a CU
@@ -352,13 +356,13 @@ void rows_join_launch(void* out, const float* parts, long MN, int splits,
                      s, (unsigned short*)out, parts, MN, splits);
 }
 
-// parts: fp32 [splits, M, N] where splits > 1, or the result, for any number of
-// rows, where out is null. silu: w is [2 N, K], out its activation [M, N].
+// parts: fp32 [splits, M, N] where splits > 1, or the result where out is null;
+// both for any number of rows. silu: w is [2 N, K], out its activation [M, N].
 void rows_tile_launch(void* out, void* parts, const void* x, const void* w,
                       int M, int N, int K, long xs, int cols, int splits,
                       int silu, int* err_unsupported, hipStream_t s) {
   *err_unsupported = K % RT_K != 0 || K == 0 ||
-                     (M > 128 && out != nullptr) || N % 4 != 0 ||
+                     (M > 128 && out != nullptr && splits == 1) || N % 4 != 0 ||
                      splits < 1 || splits > K / RT_K ||
                      (cols != 32 && cols != 64 && cols != 128) ||
                      (silu && (splits != 1 || cols == 32 || out == nullptr));

@@ -123,3 +123,27 @@ def test_no_activation_where_there_is_no_such_product():
     x = torch.zeros(4, 1024, device="cuda", dtype=torch.bfloat16)
     assert ops.linear_silu(x, w) is None
     assert ops.linear_silu(x.cpu(), w.cpu()) is None
+
+
+@pytest.mark.parametrize("M", [129, 255, 257, 385, 512])
+@pytest.mark.parametrize("N,K", [(1024, 6144), (1032, 7168), (4096, 11008),
+                                 (5120, 6208)])
+def test_tall_products_in_parts(M, N, K):
+    plan = ops._rows_tile_plan(M, N, K)
+    wins = N <= 4096 or M < 385
+    assert (plan is not None) == wins
+    if not wins:
+        return
+    assert plan[1] > 1
+    rnd = _gen(M + N)
+    x, w = rnd(M, K).bfloat16(), (rnd(N, K) * K ** -0.5).bfloat16()
+    ref = x.double() @ w.double().T
+    size = x.double().abs() @ w.double().abs().T
+    parts = ops.linear_auto(x, w, parts=True)
+    assert parts.shape == (plan[1], M, N) and parts.dtype == torch.float32
+    # fp32 sums of terms that add up to `size`, then rounded to bf16 once
+    assert bool(((parts.double().sum(0) - ref).abs()
+                 <= size * 2.0 ** -18).all())
+    out = ops.linear_auto(x, w)
+    assert bool(((out.double() - ref).abs()
+                 <= ref.abs() * 2.0 ** -8 + size * 2.0 ** -18).all())
