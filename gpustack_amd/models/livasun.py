@@ -113,6 +113,7 @@ class LivasunForCausalLM(nn.Module):
                               spec.embed_scale or 1.0)
         shared: dict = {}
         n = len(self.layers)
+        last = None
         if n:
             first = self.layers[0]
             ops.add_layer_norm(x, None, first.norm1_w, first.norm1_b, eps, h)
@@ -131,15 +132,20 @@ class LivasunForCausalLM(nn.Module):
             if layer.mlp is not None:
                 ops.add_layer_norm(x, a, layer.norm2_w, layer.norm2_b, eps, h)
                 f = layer.mlp(h, None)
-                ops.add_layer_norm(x, f, nw, nb, eps, h)
             else:
-                ops.add_layer_norm(x, a, nw, nb, eps, h)
-        rows = x if return_hidden else x[meta.logits_indices].contiguous()
-        y = torch.empty(rows.shape, dtype=self.dtype, device=dev)
-        ops.add_layer_norm(rows, None, self.final_norm, self.final_norm_b,
-                           eps, y)
+                f = a
+            if nxt is None and not return_hidden:
+                last = f              # added where the final norm picks rows
+            else:
+                ops.add_layer_norm(x, f, nw, nb, eps, h)
         if return_hidden:
+            y = torch.empty(T, W, dtype=self.dtype, device=dev)
+            ops.add_layer_norm(x, None, self.final_norm, self.final_norm_b,
+                               eps, y)
             return y
+        y = ops.add_layer_norm_rows(x, last, self.final_norm,
+                                    self.final_norm_b, eps,
+                                    meta.logits_indices, self.dtype)
         logits = ops.linear_auto(y, self.lm_head).float()
         if return_both:
             return logits, y

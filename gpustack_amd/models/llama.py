@@ -1178,10 +1178,17 @@ class DecoderLayer(nn.Module):
         else:
             self.pre_ff_norm = self.post_ff_norm = None
 
+    def plain_start(self) -> bool:
+        """True where the layer starts with the RMS norm of its rows."""
+        spec = self.spec
+        return not (spec.parallel_block or spec.sandwich_norms
+                    or spec.norm_after)
+
     def forward(self, x, residual, meta, cos_sin, k_cache, v_cache,
-                parts: bool = False):
+                parts: bool = False, normed=None):
         """`parts`: x and the result may be the parts of a product
-        (ops.linear_auto), to be added up by ops.add_rms_norm."""
+        (ops.linear_auto), to be added up by ops.add_rms_norm. `normed`: x
+        under the first norm (plain_start, no residual)."""
         eps = self.spec.rms_norm_eps
         if self.spec.parallel_block:
             return self._forward_parallel(x, meta, cos_sin, k_cache,
@@ -1194,8 +1201,10 @@ class DecoderLayer(nn.Module):
                                             v_cache, eps)
         if residual is None:
             residual = x
-            h = torch.empty_like(x)
-            ops.rms_norm(h, x, self.input_norm, eps)
+            h = normed
+            if h is None:
+                h = torch.empty_like(x)
+                ops.rms_norm(h, x, self.input_norm, eps)
         else:
             h = ops.add_rms_norm(x, residual, self.input_norm, eps)
         rm = self.spec.residual_multiplier
@@ -1336,6 +1345,8 @@ class LlamaForCausalLM(nn.Module):
     @torch.inference_mode()
     def forward(self, token_ids: torch.Tensor, meta: ForwardMeta, kv,
                 return_hidden: bool = False, return_both: bool = False):
+        first = {}                # of the first layer: its rows under the norm
+        off = self.offload
         if self.comm.pp_size > 1 and not self.comm.is_first_stage:
             # previous stage sends the summed residual stream; starting the
             # local stack with residual=None reproduces the single-rank
@@ -1344,6 +1355,13 @@ class LlamaForCausalLM(nn.Module):
             x = self.comm.recv_hidden(
                 (token_ids.shape[0], self.spec.hidden_size),
                 self.dtype, self.device)
+        elif (len(self.layers) and not self.spec.embed_scale
+              and self.layers[0].plain_start()
+              and (off is None or off.first > 0)
+              and ops.embed_rms_norm_ok(token_ids, self.embed)):
+            x, first["normed"] = ops.embed_rms_norm(
+                token_ids, self.embed, self.layers[0].input_norm,
+                self.spec.rms_norm_eps)
         else:
             x = F.embedding(token_ids, self.embed)
             if self.spec.embed_scale:
@@ -1354,7 +1372,6 @@ class LlamaForCausalLM(nn.Module):
         residual = None
         # whole rows of whole products: nothing between a product and its norm
         parts = self.comm.pp_size == 1 and self.comm.tp_size == 1
-        off = self.offload
         if off is not None:
             off.begin()
         for i, layer in enumerate(self.layers):
@@ -1364,7 +1381,8 @@ class LlamaForCausalLM(nn.Module):
                   if (self.cos_sin_local is not None and layer.attn.window)
                   else self.cos_sin)
             x, residual = layer(x, residual, meta, cs, kv.k_caches[i],
-                                kv.v_caches[i], parts=parts)
+                                kv.v_caches[i], parts=parts, **first)
+            first = {}
         if self.comm.pp_size > 1 and not self.comm.is_last_stage:
             if residual is None:  # sandwich layers carry the true stream
                 self.comm.send_hidden(x.contiguous())
@@ -1377,12 +1395,17 @@ class LlamaForCausalLM(nn.Module):
             _layer_norm(x, x, self.final_norm, self.spec.rms_norm_eps)
         elif residual is None:
             ops.rms_norm(x, x, self.final_norm, self.spec.rms_norm_eps)
+        elif not return_hidden:
+            hidden = ops.add_rms_norm_rows(x, residual, self.final_norm,
+                                           self.spec.rms_norm_eps,
+                                           meta.logits_indices)
         else:
             x = ops.add_rms_norm(x, residual, self.final_norm,
                                  self.spec.rms_norm_eps)
         if return_hidden:
             return x  # all rows, post final norm (embedding serving)
-        hidden = x[meta.logits_indices]
+        if residual is None:
+            hidden = x[meta.logits_indices]
         logits = qlinear(hidden, self.lm_head, self.lm_head_pack)
         if self.spec.final_logit_softcap:
             cap = self.spec.final_logit_softcap

@@ -137,6 +137,35 @@ def add_rms_norm(x, residual, weight, eps: float):
     return x
 
 
+def add_rms_norm_rows(x, residual, weight, eps: float, rows):
+    """add_rms_norm's result at the given rows, residual left as it is or not:
+    the last norm, of the rows whose logits are asked for."""
+    if residual.is_cuda and residual.is_contiguous() and rows.is_cuda \
+            and rows.dim() == 1 and rows.is_contiguous() \
+            and residual.dtype == torch.bfloat16 and residual.dim() == 2 \
+            and residual.shape[0] > 0 and rows.dtype == torch.int64:
+        out = torch.empty(rows.shape[0], residual.shape[1],
+                          dtype=residual.dtype, device=residual.device)
+        _load_hip().add_rms_norm_rows(out, x, residual, weight, eps, rows)
+        return out
+    return add_rms_norm(x, residual, weight, eps)[rows]
+
+
+def embed_rms_norm(tokens, embed, weight, eps: float):
+    """(rows of the tokens, their norm). GPU only (embed_rms_norm_ok)."""
+    x = torch.empty(tokens.shape[0], embed.shape[1], dtype=embed.dtype,
+                    device=embed.device)
+    out = torch.empty_like(x)
+    _load_hip().embed_rms_norm(out, x, tokens, embed, weight, eps)
+    return x, out
+
+
+def embed_rms_norm_ok(tokens, embed) -> bool:
+    return (tokens.is_cuda and tokens.dim() == 1 and tokens.is_contiguous()
+            and tokens.dtype == torch.int64 and embed.is_contiguous()
+            and embed.dtype == torch.bfloat16 and embed.shape[1] % 8 == 0)
+
+
 def fused_add_rms_norm(x, residual, weight, eps: float) -> None:
     hip = _backend(x)
     if hip is not None:
@@ -1154,6 +1183,21 @@ def add_layer_norm(x, a, w, b, eps: float, h) -> None:
         k.add_layer_norm(x, a, w, b, eps, h)
     else:
         torch_ref.add_layer_norm(x, a, w, b, eps, h)
+
+
+def add_layer_norm_rows(x, a, w, b, eps: float, rows, dtype):
+    """The layer norm of the given rows of x + a, x getting the sum or not: the
+    end of a stream, of the rows whose logits are asked for."""
+    k = _state_backend(x)
+    h = torch.empty(rows.shape[0], x.shape[1], dtype=dtype, device=x.device)
+    if k is not None and a is not None and rows.is_cuda and x.shape[0] > 0 \
+            and rows.dtype == torch.int64 and rows.is_contiguous() \
+            and k.add_layer_norm(x, a, w, b, eps, h, rows):
+        return h
+    if a is not None:
+        add_layer_norm(x, a, None, None, eps, None)
+    add_layer_norm(x[rows].contiguous(), None, w, b, eps, h)
+    return h
 
 
 def head_norm_store(q_out, qkv, nq: int, nk: int, q_w, k_w, head_dim: int,

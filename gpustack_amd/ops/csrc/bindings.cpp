@@ -5,8 +5,8 @@
 #include <hip/hip_runtime.h>
 
 // launchers (defined in the .hip translation units)
-void rms_norm_launch(void*, const void*, const void*, float, int, int, hipStream_t);
-void fused_add_rms_norm_launch(void*, void*, const void*, const float*, int, float, int, int, hipStream_t);
+void rms_norm_launch(void*, const void*, const void*, const long*, void*, long, float, int, int, hipStream_t);
+void fused_add_rms_norm_launch(void*, const void*, void*, const void*, const float*, const long*, int, float, int, int, int, hipStream_t);
 void rope_neox_launch(const long*, void*, void*, const float*, int, int, int, int, int, long, long, hipStream_t);
 void silu_and_mul_launch(void*, const void*, long, int, hipStream_t);
 void reshape_and_cache_launch(const void*, const void*, void*, void*, const long*, int, int, int, int, long, long, int, hipStream_t);
@@ -90,8 +90,26 @@ void rms_norm(at::Tensor out, at::Tensor input, at::Tensor weight, double eps) {
   const int H = input.size(-1);
   const long T = input.numel() / H;
   TORCH_CHECK(H % 8 == 0, "hidden size must be a multiple of 8");
-  rms_norm_launch(out.data_ptr(), input.data_ptr(), weight.data_ptr(),
-                  (float)eps, (int)T, H, cur_stream(input));
+  rms_norm_launch(out.data_ptr(), input.data_ptr(), weight.data_ptr(), nullptr,
+                  nullptr, 0, (float)eps, (int)T, H, cur_stream(input));
+  HIP_CHECK_LAST();
+}
+
+// x = the rows of the tokens, out their norm
+void embed_rms_norm(at::Tensor out, at::Tensor x, at::Tensor tokens,
+                    at::Tensor embed, at::Tensor weight, double eps) {
+  check_bf16(out, "out"); check_bf16(x, "x"); check_bf16(embed, "embed");
+  check_bf16(weight, "weight");
+  const int H = embed.size(1);
+  const long T = tokens.numel();
+  TORCH_CHECK(tokens.is_cuda() && tokens.scalar_type() == at::kLong &&
+              tokens.is_contiguous(), "tokens must be int64 on GPU");
+  TORCH_CHECK(H % 8 == 0 && weight.numel() == H && x.numel() == T * H &&
+              out.numel() == T * H, "embed_rms_norm shapes");
+  if (T == 0) return;
+  rms_norm_launch(out.data_ptr(), embed.data_ptr(), weight.data_ptr(),
+                  tokens.data_ptr<long>(), x.data_ptr(), embed.size(0),
+                  (float)eps, (int)T, H, cur_stream(x));
   HIP_CHECK_LAST();
 }
 
@@ -114,10 +132,36 @@ void fused_add_rms_norm(at::Tensor x, at::Tensor residual, at::Tensor weight,
                                      weight.numel() == H),
               "fused_add_rms_norm shapes");
   fused_add_rms_norm_launch(
-      x.data_ptr(), residual.data_ptr(), weight.data_ptr(),
-      parts.has_value() ? check_parts(*parts, T, H) : nullptr,
-      parts.has_value() ? (int)parts->size(0) : 0, (float)eps, (int)T, H,
+      x.data_ptr(), x.data_ptr(), residual.data_ptr(), weight.data_ptr(),
+      parts.has_value() ? check_parts(*parts, T, H) : nullptr, nullptr,
+      parts.has_value() ? (int)parts->size(0) : 0, (float)eps, (int)T, (int)T, H,
       cur_stream(x));
+  HIP_CHECK_LAST();
+}
+
+// out = the norm of the rows `pick` of residual + a, a being rows or fp32 parts
+void add_rms_norm_rows(at::Tensor out, at::Tensor a, at::Tensor residual,
+                       at::Tensor weight, double eps, at::Tensor pick) {
+  check_bf16(out, "out"); check_bf16(residual, "residual");
+  check_bf16(weight, "weight");
+  const int H = residual.size(-1);
+  const long N = residual.numel() / H, T = pick.numel();
+  TORCH_CHECK(H % 8 == 0, "hidden size must be a multiple of 8");
+  TORCH_CHECK(pick.is_cuda() && pick.scalar_type() == at::kLong &&
+              pick.is_contiguous(), "pick must be int64 on GPU");
+  TORCH_CHECK(out.numel() == T * H && weight.numel() == H && N > 0,
+              "add_rms_norm_rows shapes");
+  const bool parts = a.dim() == 3;
+  if (!parts) {
+    check_bf16(a, "a");
+    TORCH_CHECK(a.numel() == residual.numel(), "add_rms_norm_rows shapes");
+  }
+  if (T == 0) return;
+  fused_add_rms_norm_launch(
+      out.data_ptr(), a.data_ptr(), residual.data_ptr(), weight.data_ptr(),
+      parts ? check_parts(a, N, H) : nullptr, pick.data_ptr<long>(),
+      parts ? (int)a.size(0) : 0, (float)eps, (int)T, (int)N, H,
+      cur_stream(residual));
   HIP_CHECK_LAST();
 }
 
@@ -705,6 +749,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "residual+=x (or the sum of parts); x=norm(residual)*w", py::arg("x"),
         py::arg("residual"), py::arg("weight"), py::arg("eps"),
         py::arg("parts") = py::none());
+  m.def("embed_rms_norm", &embed_rms_norm, "rows of tokens and their RMS norm");
+  m.def("add_rms_norm_rows", &add_rms_norm_rows,
+        "RMS norm of picked rows of residual + a");
   m.def("rotary_embedding", &rotary_embedding, "in-place neox RoPE on q,k");
   m.def("silu_and_mul", &silu_and_mul, "silu(x[:d])*x[d:]");
   m.def("reshape_and_cache", &reshape_and_cache, "scatter K/V into paged pool");

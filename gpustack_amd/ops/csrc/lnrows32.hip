@@ -116,15 +116,23 @@ __global__ __launch_bounds__(ROW_THREADS) void add_layer_norm_kernel(
 // to bf16 as its join would (4.7 us a launch).
 // Bound by the row's bytes, few rows by the launch: 7032 rows of 2048 45 -> 32 us
 // (5.4 TB/s), 64 rows 7.4 -> 4.9, in four parts 4.7 + 7.4 -> 5.0.
+// pick (or null): h's row t is the norm of row pick[t] of the N, and the sum goes
+// nowhere: the stream's end, of the rows whose logits are asked for. One launch
+// for the last sum, the gather and the norm: 64 rows of 2048 4.7 + 4.7 + 4.7 -> 5.
 enum AddFrom { NOTHING, ROWS16, ROWS32, PARTS };
 
 template <typename TH, int NV, int FROM>
 __global__ __launch_bounds__(ROW_THREADS) void add_layer_norm_vec_kernel(
     float* __restrict__ x, const void* __restrict__ a, int parts,
     const float* __restrict__ w, const float* __restrict__ b,
-    TH* __restrict__ h, int T, int W, float eps) {
+    TH* __restrict__ h, const long* __restrict__ pick, int N, int W, float eps) {
   __shared__ float red[4];
-  const long t = blockIdx.x;
+  long t = blockIdx.x;
+  if (pick != nullptr) {
+    t = pick[blockIdx.x];
+    if (t < 0) t += N;
+    t = t < 0 ? 0 : t < N ? t : N - 1;
+  }
   float* xr = x + t * W;
   float keep[NV][8];
   float sum = 0.f;
@@ -144,7 +152,7 @@ __global__ __launch_bounds__(ROW_THREADS) void add_layer_norm_vec_kernel(
 #pragma unroll
       for (int k = 0; k < 8; ++k) f[k] = ((const float*)a)[t * W + i + k];
     } else if constexpr (FROM == PARTS) {
-      bf8_to_f32(join_parts8((const float*)a + t * W + i, (long)T * W, parts), f);
+      bf8_to_f32(join_parts8((const float*)a + t * W + i, (long)N * W, parts), f);
     }
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
@@ -153,7 +161,7 @@ __global__ __launch_bounds__(ROW_THREADS) void add_layer_norm_vec_kernel(
       keep[j][k] = v;
       sum += v;
     }
-    if constexpr (FROM != NOTHING) {
+    if (FROM != NOTHING && pick == nullptr) {
       *reinterpret_cast<f32x4*>(xr + i) =
           f32x4{keep[j][0], keep[j][1], keep[j][2], keep[j][3]};
       *reinterpret_cast<f32x4*>(xr + i + 4) =
@@ -161,6 +169,7 @@ __global__ __launch_bounds__(ROW_THREADS) void add_layer_norm_vec_kernel(
     }
   }
   if (w == nullptr) return;
+  TH* hr = h + (long)blockIdx.x * W;
   const float mean = block_sum(sum, red) / (float)W;
   float sq = 0.f;
 #pragma unroll
@@ -180,10 +189,10 @@ __global__ __launch_bounds__(ROW_THREADS) void add_layer_norm_vec_kernel(
 #pragma unroll
     for (int k = 0; k < 8; ++k) f[k] = (keep[j][k] - mean) * inv * w[i + k] + b[i + k];
     if constexpr (sizeof(TH) == 2) {
-      *reinterpret_cast<u16x8*>(h + t * W + i) = f32_to_bf8(f);
+      *reinterpret_cast<u16x8*>(hr + i) = f32_to_bf8(f);
     } else {
-      *reinterpret_cast<f32x4*>(h + t * W + i) = f32x4{f[0], f[1], f[2], f[3]};
-      *reinterpret_cast<f32x4*>(h + t * W + i + 4) = f32x4{f[4], f[5], f[6], f[7]};
+      *reinterpret_cast<f32x4*>(hr + i) = f32x4{f[0], f[1], f[2], f[3]};
+      *reinterpret_cast<f32x4*>(hr + i + 4) = f32x4{f[4], f[5], f[6], f[7]};
     }
   }
 }
@@ -463,10 +472,11 @@ void aln_pick(float* x, const void* a, const float* w, const float* b, void* h,
 
 template <typename TH, int NV>
 void aln_vec(float* x, const void* a, int from, int parts, const float* w,
-             const float* b, void* h, int T, int W, float eps, hipStream_t s) {
+             const float* b, void* h, const long* pick, int T, int N, int W,
+             float eps, hipStream_t s) {
 #define ALN(F)                                                               \
   add_layer_norm_vec_kernel<TH, NV, F><<<T, ROW_THREADS, 0, s>>>(            \
-      x, a, parts, w, b, (TH*)h, T, W, eps)
+      x, a, parts, w, b, (TH*)h, pick, N, W, eps)
   if (from == NOTHING) ALN(NOTHING);
   else if (from == ROWS16) ALN(ROWS16);
   else if (from == ROWS32) ALN(ROWS32);
@@ -476,11 +486,13 @@ void aln_vec(float* x, const void* a, int from, int parts, const float* w,
 
 template <typename TH>
 void aln_vec_pick(float* x, const void* a, int from, int parts, const float* w,
-                  const float* b, void* h, int T, int W, float eps,
-                  hipStream_t s) {
-  if (W <= 2048) aln_vec<TH, 1>(x, a, from, parts, w, b, h, T, W, eps, s);
-  else if (W <= 4096) aln_vec<TH, 2>(x, a, from, parts, w, b, h, T, W, eps, s);
-  else aln_vec<TH, 4>(x, a, from, parts, w, b, h, T, W, eps, s);
+                  const float* b, void* h, const long* pick, int T, int N,
+                  int W, float eps, hipStream_t s) {
+#define ALN_ARGS x, a, from, parts, w, b, h, pick, T, N, W, eps, s
+  if (W <= 2048) aln_vec<TH, 1>(ALN_ARGS);
+  else if (W <= 4096) aln_vec<TH, 2>(ALN_ARGS);
+  else aln_vec<TH, 4>(ALN_ARGS);
+#undef ALN_ARGS
 }
 
 }  // namespace
@@ -499,22 +511,24 @@ void embed_rows_scaled_launch(float* x, const long* tokens, const void* embed,
         x, tokens, (const float*)embed, W, vocab, scale);
 }
 
-// parts: of a [parts, T, W] in fp32, or 0 for rows [T, W]. Returns 0 when
-// parts come with rows that only whole rows are taken of.
+// parts: of a [parts, N, W] in fp32, or 0 for rows [N, W]. pick: null (T = N),
+// or the T rows whose norm h gets, x being left as it is. Returns 0 when parts or
+// picked rows come with rows that only the general form takes.
 int add_layer_norm_launch(float* x, const void* a, int parts, const float* w,
-                          const float* b, void* h, int T, int W, float eps,
-                          int a_bf, int h_bf, hipStream_t s) {
+                          const float* b, void* h, const long* pick, int T,
+                          int N, int W, float eps, int a_bf, int h_bf,
+                          hipStream_t s) {
   if (T <= 0) return 1;
   const uintptr_t at = (uintptr_t)x | (uintptr_t)a | (uintptr_t)w |
                        (uintptr_t)b | (uintptr_t)h;
   if (W % 8 == 0 && W <= 8192 && at % 16 == 0) {
     const int from = a == nullptr ? NOTHING : parts > 0 ? PARTS
                    : a_bf ? ROWS16 : ROWS32;
-    if (h_bf) aln_vec_pick<unsigned short>(x, a, from, parts, w, b, h, T, W, eps, s);
-    else aln_vec_pick<float>(x, a, from, parts, w, b, h, T, W, eps, s);
+    if (h_bf) aln_vec_pick<unsigned short>(x, a, from, parts, w, b, h, pick, T, N, W, eps, s);
+    else aln_vec_pick<float>(x, a, from, parts, w, b, h, pick, T, N, W, eps, s);
     return 1;
   }
-  if (parts > 0) return 0;
+  if (parts > 0 || pick != nullptr) return 0;
   if (a_bf) {
     if (h_bf) aln_pick<unsigned short, unsigned short>(x, a, w, b, h, T, W, eps, s);
     else aln_pick<unsigned short, float>(x, a, w, b, h, T, W, eps, s);

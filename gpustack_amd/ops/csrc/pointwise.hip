@@ -17,18 +17,39 @@ namespace {
 constexpr int NORM_THREADS = 256;
 constexpr int NORM_MAX_VEC = 4; // u16x8 per thread held in registers
 
+// tokens (or null): `in` is a table of `vocab` rows, row t the one of tokens[t],
+// which `rows` gets as well. That is the embedding and the first norm in a launch:
+// 16 rows of 4096 12.5 + 4.6 -> 5.1 us, 48 4.7 + 4.7 -> 5.1. Tokens out of range
+// make a row of zeros.
 __global__ void rms_norm_kernel(unsigned short* __restrict__ out,
                                 const unsigned short* __restrict__ in,
                                 const unsigned short* __restrict__ w,
+                                const long* __restrict__ tokens,
+                                unsigned short* __restrict__ rows, long vocab,
                                 float eps, int T, int H) {
   const int nvec = H / 8; // H % 8 == 0 enforced on host
   const bool cached = nvec <= NORM_THREADS * NORM_MAX_VEC;
   for (int row = blockIdx.x; row < T; row += gridDim.x) {
     const unsigned short* rp = in + (long)row * H;
+    if (tokens != nullptr) {
+      const long id = tokens[row];
+      unsigned short* to = rows + (long)row * H;
+      rp = in + id * H;
+      if (id < 0 || id >= vocab) {           // the same for the workgroup
+        const u16x8 none = {0, 0, 0, 0, 0, 0, 0, 0};
+        for (int v = threadIdx.x; v < nvec; v += NORM_THREADS) {
+          *reinterpret_cast<u16x8*>(to + v * 8) = none;
+          *reinterpret_cast<u16x8*>(out + (long)row * H + v * 8) = none;
+        }
+        continue;
+      }
+    }
     float vals[NORM_MAX_VEC][8];
     float ss = 0.f;
     for (int v = threadIdx.x, slot = 0; v < nvec; v += NORM_THREADS, ++slot) {
       u16x8 u = *reinterpret_cast<const u16x8*>(rp + v * 8);
+      if (tokens != nullptr)
+        *reinterpret_cast<u16x8*>(rows + (long)row * H + v * 8) = u;
       float f[8];
       bf8_to_f32(u, f);
 #pragma unroll
@@ -71,24 +92,37 @@ __global__ void rms_norm_kernel(unsigned short* __restrict__ out,
 // PARTS: x is only written; what is added comes as the fp32 parts [parts, T, H]
 // of a product cut over k, rounded as its join would. That saves the join's
 // launch: 48 rows of 4096 in four parts 4.6 + 4.7 us -> 5.6.
+// pick (or null): row t is the norm of row pick[t] of N, the result goes to `out`
+// and the sum nowhere: the last norm, of the rows whose logits are asked for. That
+// saves the gather behind it (4.7 us).
 template <bool PARTS>
-__global__ void fused_add_rms_norm_kernel(unsigned short* __restrict__ x,
+__global__ void fused_add_rms_norm_kernel(unsigned short* out,
+                                          const unsigned short* x,
                                           unsigned short* __restrict__ residual,
                                           const unsigned short* __restrict__ w,
                                           const float* __restrict__ from,
-                                          int parts, float eps, int T, int H) {
+                                          const long* __restrict__ pick,
+                                          int parts, float eps, int T, int N,
+                                          int H) {
   const int nvec = H / 8;
   const bool cached = nvec <= NORM_THREADS * NORM_MAX_VEC;
   for (int row = blockIdx.x; row < T; row += gridDim.x) {
-    unsigned short* xp = x + (long)row * H;
-    unsigned short* rp = residual + (long)row * H;
+    long src = row;
+    if (pick != nullptr) {
+      src = pick[row];
+      if (src < 0) src += N;
+      src = src < 0 ? 0 : src < N ? src : N - 1;
+    }
+    unsigned short* op = out + (long)row * H;
+    const unsigned short* xp = x + src * H;
+    unsigned short* rp = residual + src * H;
     float vals[NORM_MAX_VEC][8];
     float ss = 0.f;
     for (int v = threadIdx.x, slot = 0; v < nvec; v += NORM_THREADS, ++slot) {
       u16x8 ur = *reinterpret_cast<const u16x8*>(rp + v * 8);
       u16x8 ux;
       if constexpr (PARTS)
-        ux = join_parts8(from + (long)row * H + v * 8, (long)T * H, parts);
+        ux = join_parts8(from + src * H + v * 8, (long)N * H, parts);
       else
         ux = *reinterpret_cast<const u16x8*>(xp + v * 8);
       float f[8];
@@ -97,7 +131,8 @@ __global__ void fused_add_rms_norm_kernel(unsigned short* __restrict__ x,
         f[i] = bf2f(ux[i]) + bf2f(ur[i]);
         ss += f[i] * f[i];
       }
-      *reinterpret_cast<u16x8*>(rp + v * 8) = f32_to_bf8(f);
+      if (pick == nullptr)
+        *reinterpret_cast<u16x8*>(rp + v * 8) = f32_to_bf8(f);
       if (cached && slot < NORM_MAX_VEC) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) vals[slot][i] = f[i];
@@ -120,12 +155,22 @@ __global__ void fused_add_rms_norm_kernel(unsigned short* __restrict__ x,
         // residual now holds the sum (bf16-rounded); re-read it.
         u16x8 u = *reinterpret_cast<const u16x8*>(rp + v * 8);
         bf8_to_f32(u, f);
+        if (pick != nullptr) {               // add again, and round like that
+          u16x8 ux;
+          if constexpr (PARTS)
+            ux = join_parts8(from + src * H + v * 8, (long)N * H, parts);
+          else
+            ux = *reinterpret_cast<const u16x8*>(xp + v * 8);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) f[i] += bf2f(ux[i]);
+          bf8_to_f32(f32_to_bf8(f), f);
+        }
       }
       u16x8 wv = *reinterpret_cast<const u16x8*>(w + v * 8);
       float o[8];
 #pragma unroll
       for (int i = 0; i < 8; ++i) o[i] = f[i] * inv * bf2f(wv[i]);
-      *reinterpret_cast<u16x8*>(xp + v * 8) = f32_to_bf8(o);
+      *reinterpret_cast<u16x8*>(op + v * 8) = f32_to_bf8(o);
     }
     __syncthreads();
   }
@@ -439,25 +484,30 @@ static inline int pw_grid(long total_threads_needed, int block) {
   return (int)blocks;
 }
 
-void rms_norm_launch(void* out, const void* in, const void* w, float eps,
+// tokens: null, or the rows of `in` [vocab, H] that `rows` gets
+void rms_norm_launch(void* out, const void* in, const void* w,
+                     const long* tokens, void* rows, long vocab, float eps,
                      int T, int H, hipStream_t s) {
   int grid = T < 8192 ? (T < 1 ? 1 : T) : 8192;
   hipLaunchKernelGGL(rms_norm_kernel, dim3(grid), dim3(NORM_THREADS), 0, s,
                      (unsigned short*)out, (const unsigned short*)in,
-                     (const unsigned short*)w, eps, T, H);
+                     (const unsigned short*)w, tokens, (unsigned short*)rows,
+                     vocab, eps, T, H);
 }
 
-// from: null, or the fp32 parts that are added instead of x
-void fused_add_rms_norm_launch(void* x, void* residual, const void* w,
-                               const float* from, int parts, float eps, int T,
-                               int H, hipStream_t s) {
+// out [T, H], x and residual [N, H]. from: null, or the fp32 parts that are added
+// instead of x. pick: null (T = N), or the rows that out has.
+void fused_add_rms_norm_launch(void* out, const void* x, void* residual,
+                               const void* w, const float* from,
+                               const long* pick, int parts, float eps, int T,
+                               int N, int H, hipStream_t s) {
   int grid = T < 8192 ? (T < 1 ? 1 : T) : 8192;
   hipLaunchKernelGGL(
       (from != nullptr ? fused_add_rms_norm_kernel<true>
                        : fused_add_rms_norm_kernel<false>),
-      dim3(grid), dim3(NORM_THREADS), 0, s, (unsigned short*)x,
-      (unsigned short*)residual, (const unsigned short*)w, from, parts, eps, T,
-      H);
+      dim3(grid), dim3(NORM_THREADS), 0, s, (unsigned short*)out,
+      (const unsigned short*)x, (unsigned short*)residual,
+      (const unsigned short*)w, from, pick, parts, eps, T, N, H);
 }
 
 void rope_neox_launch(const long* positions, void* q, void* k,

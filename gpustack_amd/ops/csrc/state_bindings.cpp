@@ -9,7 +9,7 @@
 #include <hip/hip_runtime.h>
 
 void embed_rows_scaled_launch(float*, const long*, const void*, int, int, long, float, int, hipStream_t);
-int add_layer_norm_launch(float*, const void*, int, const float*, const float*, void*, int, int, float, int, int, hipStream_t);
+int add_layer_norm_launch(float*, const void*, int, const float*, const float*, void*, const long*, int, int, int, float, int, int, hipStream_t);
 void head_norm_store_launch(void*, void*, long, int, int, int, const float*, const float*, int, float, float, const int*, const void*, long, const float*, void*, void*, const long*, long, int, int, int, float, int, int, int, hipStream_t);
 void value_page_store_launch(const void*, long, int, void*, const long*, long, const int*, int, int, int, int, int, int, hipStream_t);
 void route_topk_launch(int*, float*, const float*, int, const float*, int, int, int, int, int, int, int, int, float, hipStream_t);
@@ -76,11 +76,21 @@ void embed_rows_scaled(Tensor x, Tensor tokens, Tensor embed, double scale) {
   HIP_CHECK_LAST();
 }
 
-void add_layer_norm(Tensor x, OptTensor a, OptTensor w, OptTensor b, double eps,
-                    OptTensor h) {
+// With pick, h's rows are those of x + a, which x does not get; false then where
+// there is no such form.
+bool add_layer_norm(Tensor x, OptTensor a, OptTensor w, OptTensor b, double eps,
+                    OptTensor h, OptTensor pick) {
   chk(x, "x", at::kFloat);
   TORCH_CHECK(x.dim() == 2);
-  const int T = x.size(0), W = x.size(1);
+  const int N = x.size(0), W = x.size(1);
+  int T = N;
+  const long* rows = nullptr;
+  if (pick.has_value()) {
+    chk(*pick, "pick", at::kLong);
+    TORCH_CHECK(w.has_value() && N > 0, "pick wants a norm of rows");
+    T = (int)pick->numel();
+    rows = pick->data_ptr<long>();
+  }
   const void* ap = nullptr;
   const float *wp = nullptr, *bp = nullptr;
   void* hp = nullptr;
@@ -89,7 +99,7 @@ void add_layer_norm(Tensor x, OptTensor a, OptTensor w, OptTensor b, double eps,
     a_bf = act_kind(*a, "a");
     if (a->dim() == 3) {
       parts = (int)a->size(0);
-      TORCH_CHECK(!a_bf && parts >= 1 && a->size(1) == T && a->size(2) == W,
+      TORCH_CHECK(!a_bf && parts >= 1 && a->size(1) == N && a->size(2) == W,
                   "parts must be fp32 [n, T, W]");
     } else {
       TORCH_CHECK(a->sizes() == x.sizes());
@@ -102,16 +112,18 @@ void add_layer_norm(Tensor x, OptTensor a, OptTensor w, OptTensor b, double eps,
     chk(*b, "b", at::kFloat);
     TORCH_CHECK(w->numel() == W && b->numel() == W);
     h_bf = act_kind(*h, "h");
-    TORCH_CHECK(h->sizes() == x.sizes());
+    TORCH_CHECK(h->dim() == 2 && h->size(0) == T && h->size(1) == W);
     wp = w->data_ptr<float>();
     bp = b->data_ptr<float>();
     hp = h->data_ptr();
   }
   const int ok = add_layer_norm_launch(x.data_ptr<float>(), ap, parts, wp, bp,
-                                       hp, T, W, (float)eps, a_bf, h_bf,
+                                       hp, rows, T, N, W, (float)eps, a_bf, h_bf,
                                        cur_stream(x));
-  TORCH_CHECK(ok, "parts of rows of ", W, " at these addresses");
+  TORCH_CHECK(ok || rows != nullptr, "parts of rows of ", W,
+              " at these addresses");
   HIP_CHECK_LAST();
+  return ok;
 }
 
 void head_norm_store(Tensor q_out, Tensor qkv, long nq, long nk, Tensor q_w,
@@ -482,7 +494,9 @@ void gated_group_norm(Tensor out, Tensor y, Tensor gate, Tensor w, long groups,
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("embed_rows_scaled", &embed_rows_scaled);
-  m.def("add_layer_norm", &add_layer_norm);
+  m.def("add_layer_norm", &add_layer_norm, py::arg("x"), py::arg("a"),
+        py::arg("w"), py::arg("b"), py::arg("eps"), py::arg("h"),
+        py::arg("pick") = py::none());
   m.def("head_norm_store", &head_norm_store);
   m.def("route_topk", &route_topk);
   m.def("short_conv", &short_conv);

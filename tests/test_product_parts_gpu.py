@@ -147,3 +147,50 @@ def test_tall_products_in_parts(M, N, K):
     out = ops.linear_auto(x, w)
     assert bool(((out.double() - ref).abs()
                  <= ref.abs() * 2.0 ** -8 + size * 2.0 ** -18).all())
+
+
+@pytest.mark.parametrize("T,H", [(1, 64), (17, 4096), (3, 8200)])
+def test_embedding_under_the_first_norm(T, H):
+    rnd = _gen(T + H)
+    embed, w = rnd(50, H).bfloat16(), rnd(H).bfloat16()
+    ids = torch.arange(T, device="cuda") * 7 % 50
+    x, h = ops.embed_rms_norm(ids, embed, w, 1e-5)
+    ref = torch.empty_like(x)
+    ops.rms_norm(ref, embed[ids], w, 1e-5)
+    assert torch.equal(x, embed[ids]) and torch.equal(h, ref)
+    bad = ids.clone()
+    bad[-1] = 50
+    x, h = ops.embed_rms_norm(bad, embed, w, 1e-5)
+    assert torch.equal(x[:-1], embed[ids[:-1]]) and torch.equal(h[:-1], ref[:-1])
+    assert not x[-1].any() and not h[-1].any()
+
+
+@pytest.mark.parametrize("n", [0, 1, 3, 8])
+@pytest.mark.parametrize("T,H", [(1, 64), (17, 4096), (9, 8200)])
+def test_the_last_norm_of_picked_rows(n, T, H):
+    rnd = _gen(n + T)
+    res, w = rnd(T, H).bfloat16(), rnd(H).bfloat16()
+    a = rnd(n, T, H) if n else rnd(T, H).bfloat16()
+    rows = torch.tensor([T - 1, 0, -1], device="cuda")[: 1 + 2 * (T > 1)]
+    x, r = (_joined(a) if n else a.clone()), res.clone()
+    ops.fused_add_rms_norm(x, r, w, 1e-5)
+    got = ops.add_rms_norm_rows(a, res, w, 1e-5, rows)
+    assert torch.equal(got, x[rows])
+
+
+@pytest.mark.parametrize("kind", ["parts", "bf16", "fp32"])
+@pytest.mark.parametrize("T,W", [(1, 64), (17, 2048), (9, 8192), (5, 100)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_the_last_layer_norm_of_picked_rows(kind, T, W, dtype):
+    rnd = _gen(T + W)
+    x, w, b = rnd(T, W), rnd(W), rnd(W)
+    if kind == "parts" and W % 8:
+        return                         # products give such rows whole
+    a = rnd(3, T, W) if kind == "parts" else rnd(T, W)
+    if kind == "bf16":
+        a = a.bfloat16()
+    rows = torch.tensor([T - 1, 0, 0], device="cuda")
+    y, ref = x.clone(), torch.empty(T, W, device="cuda", dtype=dtype)
+    ops.add_layer_norm(y, a, w, b, 1e-5, ref)
+    got = ops.add_layer_norm_rows(x, a, w, b, 1e-5, rows, dtype)
+    assert torch.equal(got, ref[rows])
