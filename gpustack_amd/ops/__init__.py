@@ -564,6 +564,33 @@ def _tall_tile_plan(M: int, N: int, K: int):
     return 128, min(8, 512 // t128)
 
 
+def _parts_plan(M: int, N: int, K: int):
+    """(columns of a tile, parts of K) of a small product whose consumer adds
+    the parts up, where that beats the product of _rows_tile_plan, the library
+    or the decode product, else None: short rows leave whole tiles few and
+    their chain long. us with an RMS norm behind, 64 rows (24 rows; 16 rows):
+    2048x2048 9.4 against 14.9 (8.2 / 14.1; 8.0 / 9.2), 1536x1024 7.7 / 11.5
+    (7.0 / 11.2; 6.9 / 7.0), 4096x2048 13.0 / 16.3 (12.0 / 15.7; 11.6 / 11.1),
+    4096x3072 14.3 / 20.1 (12.6 / 15.3; 12.2 / 12.9), 6144x3072 18.8 / 23.4
+    (16.4 / 18.1; 16.0 / 17.5), 6144x2048 at 16 rows 13.7 / 16.0 but at 24
+    rows 13.9 / 13.7; 128 rows: 2048x2048 12.2 / 14.4, 4096x1024 14.3 / 16.7.
+    At one row 2048x3072 8.6 / 9.6, 2048x2048 7.7 / 7.7."""
+    if not 0 < M <= 128 or K % 64 != 0 or N % 8 != 0 or min(N, K) < 1024 \
+            or N > 6144 or K >= 4096:
+        return None
+    if M <= 16:
+        wins = N <= 2048 and (K >= 3072 or K >= 2048 and M >= 8) or \
+            N >= 5120 and (K >= 3072 or K >= 2048 and M >= 8)
+    elif N <= 4096:
+        wins = M > 64 and K < 3072 or M <= 64 and not (N >= 2560 and K == 1024) \
+            or N < 2048
+    else:
+        wins = K >= 3072 and M <= 64
+    if not wins:
+        return None
+    return (32 if N <= 2048 else 64 if N <= 4096 else 128), 4
+
+
 def router_plan(T: int, E: int, H: int):
     """(columns of a tile, parts over k) of a router's product, whose parts the
     choice of the experts adds up, or None. us for both launches against a
@@ -598,7 +625,7 @@ def linear_auto(x, w, parts: bool = False):
     if _own_products(x, w):
         M, K = x.shape
         N = w.shape[0]
-        plan = _rows_tile_plan(M, N, K)
+        plan = parts and _parts_plan(M, N, K) or _rows_tile_plan(M, N, K)
         if (plan or _rows_gemm_wins(M, N, K)) and _rows_take(x, w):
             if parts and plan and plan[1] > 1:
                 return _load_hip().rows_tile_parts(x, w, *plan)

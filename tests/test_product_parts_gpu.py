@@ -149,6 +149,25 @@ def test_tall_products_in_parts(M, N, K):
                  <= ref.abs() * 2.0 ** -8 + size * 2.0 ** -18).all())
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 1024, 3072), (8, 2048, 2048),
+                                   (17, 1032, 1024), (64, 2048, 1088),
+                                   (65, 4096, 1024), (128, 3072, 2048),
+                                   (33, 6136, 3136), (16, 5120, 2048)])
+def test_small_products_in_parts(M, N, K):
+    plan = ops._parts_plan(M, N, K)
+    assert plan is not None
+    rnd = _gen(M + N)
+    x, w = rnd(M, K).bfloat16(), (rnd(N, K) * K ** -0.5).bfloat16()
+    parts = ops.linear_auto(x, w, parts=True)
+    assert parts.shape == (plan[1], M, N) and parts.dtype == torch.float32
+    ref = x.double() @ w.double().T
+    size = x.double().abs() @ w.double().abs().T
+    # fp32 sums of terms that add up to `size`
+    assert bool(((parts.double().sum(0) - ref).abs()
+                 <= size * 2.0 ** -18).all())
+    assert ops.linear_auto(x, w).shape == (M, N)
+
+
 @pytest.mark.parametrize("T,H", [(1, 64), (17, 4096), (3, 8200)])
 def test_embedding_under_the_first_norm(T, H):
     rnd = _gen(T + H)
