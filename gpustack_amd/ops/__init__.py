@@ -574,13 +574,32 @@ def _parts_plan(M: int, N: int, K: int):
     4096x3072 14.3 / 20.1 (12.6 / 15.3; 12.2 / 12.9), 6144x3072 18.8 / 23.4
     (16.4 / 18.1; 16.0 / 17.5), 6144x2048 at 16 rows 13.7 / 16.0 but at 24
     rows 13.9 / 13.7; 128 rows: 2048x2048 12.2 / 14.4, 4096x1024 14.3 / 16.7.
-    At one row 2048x3072 8.6 / 9.6, 2048x2048 7.7 / 7.7."""
+    At one row 2048x3072 8.6 / 9.6, 2048x2048 7.7 / 7.7.
+    Up to 16 rows also longer ones, at one / 16 rows: 2048x5120 10 / 10 against
+    21 / 13, 4096x5120 15 / 16 against 24 / 23, 1024x8192 10 / 10 against 15 /
+    15, 6144x4096 19 / 19 against 21 / 20 (in four parts 22 / 23 at 7168x4096, in
+    three 21 / 21), 4096x4096 13.4 / 13.7 against 13.6 / 15.0, but 4096x8192
+    20.3 / 20.6 against 20.7 / 20.8; and 8192x3072 19 / 19 against 26 / 24, at
+    64 rows 22 / 25, 7168x10240 there 41 / 49."""
     if not 0 < M <= 128 or K % 64 != 0 or N % 8 != 0 or min(N, K) < 1024 \
-            or N > 6144 or K >= 4096:
+            or N > 8192:
+        return None
+    # four cuts of rows a multiple of 8 KB apart meet on a few memory channels
+    wide = 128, 3 if K % 4096 == 0 else 4
+    if N > 6144:
+        return wide if M <= 64 and 3072 <= K < 11008 else None
+    if M <= 16 and 4096 <= K < 11008:
+        if N > 5120:
+            return wide
+        if K % 8192 == 0 and 2048 < N <= 4096:
+            return None
+        cols = 32 if N <= 2048 else 64
+        return cols, min(8 if cols == 32 else 4, 256 // -(-N // cols))
+    if K >= 4096:
         return None
     if M <= 16:
-        wins = N <= 2048 and (K >= 3072 or K >= 2048 and M >= 8) or \
-            N >= 5120 and (K >= 3072 or K >= 2048 and M >= 8)
+        wins = (N <= 2048 or N >= 5120) and (
+            K >= 3072 or K >= 2048 and M >= 8)
     elif N <= 4096:
         wins = M > 64 and K < 3072 or M <= 64 and not (N >= 2560 and K == 1024) \
             or N < 2048
