@@ -838,7 +838,10 @@ class MoEMLP(nn.Module):
             weights, experts = torch.topk(probs, self.top_k, dim=-1)
         return weights, experts
 
-    def forward(self, x, meta: ForwardMeta | None = None):
+    def forward(self, x, meta: ForwardMeta | None = None,
+                parts: bool = False):
+        """`parts`: the result may be the rows of each row's experts [T, k, h],
+        to be added up by ops.add_rms_norm."""
         # MoE expert MLPs do not take LoRA (rejected at adapter load);
         # attention adapters still apply upstream
         T = x.shape[0]
@@ -883,6 +886,9 @@ class MoEMLP(nn.Module):
             else:
                 weights, experts = self._route(logits)
         if fused and not self._library_wins(T):
+            if parts and T > 0 and self.shared_gate_up_w is None:
+                return self._fused_contrib(x, experts, weights) \
+                    .view(T, self.top_k, -1)
             out = self._fused_dispatch(x, experts, weights)
             return self.comm.all_reduce(self._add_shared(x, out))
         flat_exp = experts.reshape(-1).long()                     # [T*k]
@@ -1019,8 +1025,15 @@ class MoEMLP(nn.Module):
                 and not torch.cuda.is_current_stream_capturing())
 
     def _fused_dispatch(self, x, experts, weights):
-        """Sync-free grouped expert products: sort the assignments by expert
-        on the device, run the two expert kernels, sum over the k axis. Every
+        """Sync-free grouped expert products, summed over the k axis."""
+        contrib = self._fused_contrib(x, experts, weights)
+        out = torch.empty_like(x)
+        ops._load_hip().moe_sum(out, contrib, experts.shape[1])
+        return out
+
+    def _fused_contrib(self, x, experts, weights):
+        """The weighted results of each row's experts [T * k, h]: sort the
+        assignments by expert on the device, run the two expert kernels. Every
         tensor shape here depends only on (T, k, E) — safe under hipGraph
         capture (reference capability: vLLM fused_moe)."""
         T, k = experts.shape
@@ -1055,9 +1068,7 @@ class MoEMLP(nn.Module):
         else:
             hip.moe_tile(True, contrib, act, self._bank("down"), order, tiles,
                          ntiles, offs, counts, flat_w, bias=db)
-        out = torch.empty_like(x)
-        hip.moe_sum(out, contrib, k)
-        return out
+        return contrib
 
     def _act_mul(self, gu):
         """[T', 2i] -> [T', i]: SiLU-mul (fused kernel/ref) or GPT-OSS
@@ -1214,7 +1225,8 @@ class DecoderLayer(nn.Module):
         if rm:  # Granite: scale sublayer outputs before the residual add
             a = a * rm
         a = ops.add_rms_norm(a, residual, self.post_attn_norm, eps)
-        m = self.mlp(a, meta, **(kw if isinstance(self.mlp, MLP) else {}))
+        m = self.mlp(a, meta, **(kw if isinstance(self.mlp, (MLP, MoEMLP))
+                                else {}))
         if rm:
             m = m * rm
         return m, residual

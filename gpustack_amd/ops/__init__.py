@@ -128,7 +128,8 @@ def rms_norm(out, x, weight, eps: float) -> None:
 
 def add_rms_norm(x, residual, weight, eps: float):
     """residual += x and the norm of it, which is returned: in x, or where x is
-    the parts of a product (linear_auto with `parts`) in a tensor of its own."""
+    the parts of a product (linear_auto with `parts`) or the bf16 rows of each
+    row's experts [T, k, H], in a tensor of its own."""
     if x.dim() == 3:
         out = torch.empty_like(residual)
         _load_hip().fused_add_rms_norm(out, residual, weight, eps, x)

@@ -6,7 +6,7 @@
 
 // launchers (defined in the .hip translation units)
 void rms_norm_launch(void*, const void*, const void*, const long*, void*, long, float, int, int, hipStream_t);
-void fused_add_rms_norm_launch(void*, const void*, void*, const void*, const float*, const long*, int, float, int, int, int, hipStream_t);
+void fused_add_rms_norm_launch(void*, const void*, void*, const void*, const void*, int, const long*, int, float, int, int, int, hipStream_t);
 void rope_neox_launch(const long*, void*, void*, const float*, int, int, int, int, int, long, long, hipStream_t);
 void silu_and_mul_launch(void*, const void*, long, int, hipStream_t);
 void reshape_and_cache_launch(const void*, const void*, void*, void*, const long*, int, int, int, int, long, long, int, hipStream_t);
@@ -122,6 +122,19 @@ const float* check_parts(const at::Tensor& p, long rows, long cols) {
   return p.data_ptr<float>();
 }
 
+// what a norm adds to its stream besides rows: fp32 parts [n, rows, cols], or bf16
+// rows of a row's experts [rows, n, cols]
+struct Addend { const void* data; int chosen, n; };
+
+Addend norm_addend(const at::Tensor& p, long rows, long cols) {
+  if (p.scalar_type() == at::kFloat)
+    return {check_parts(p, rows, cols), 0, (int)p.size(0)};
+  check_bf16(p, "experts' rows");
+  TORCH_CHECK(p.dim() == 3 && p.size(0) == rows && p.size(1) >= 1 &&
+              p.size(2) == cols, "experts' rows must be [rows, n, cols]");
+  return {p.data_ptr(), 1, (int)p.size(1)};
+}
+
 void fused_add_rms_norm(at::Tensor x, at::Tensor residual, at::Tensor weight,
                         double eps, c10::optional<at::Tensor> parts) {
   check_bf16(x, "x"); check_bf16(residual, "residual"); check_bf16(weight, "weight");
@@ -131,15 +144,17 @@ void fused_add_rms_norm(at::Tensor x, at::Tensor residual, at::Tensor weight,
   TORCH_CHECK(!parts.has_value() || (residual.numel() == x.numel() &&
                                      weight.numel() == H),
               "fused_add_rms_norm shapes");
-  fused_add_rms_norm_launch(
-      x.data_ptr(), x.data_ptr(), residual.data_ptr(), weight.data_ptr(),
-      parts.has_value() ? check_parts(*parts, T, H) : nullptr, nullptr,
-      parts.has_value() ? (int)parts->size(0) : 0, (float)eps, (int)T, (int)T, H,
-      cur_stream(x));
+  Addend from{nullptr, 0, 0};
+  if (parts.has_value()) from = norm_addend(*parts, T, H);
+  fused_add_rms_norm_launch(x.data_ptr(), x.data_ptr(), residual.data_ptr(),
+                            weight.data_ptr(), from.data, from.chosen, nullptr,
+                            from.n, (float)eps, (int)T, (int)T, H,
+                            cur_stream(x));
   HIP_CHECK_LAST();
 }
 
-// out = the norm of the rows `pick` of residual + a, a being rows or fp32 parts
+// out = the norm of the rows `pick` of residual + a, a being rows or what
+// norm_addend takes
 void add_rms_norm_rows(at::Tensor out, at::Tensor a, at::Tensor residual,
                        at::Tensor weight, double eps, at::Tensor pick) {
   check_bf16(out, "out"); check_bf16(residual, "residual");
@@ -151,17 +166,18 @@ void add_rms_norm_rows(at::Tensor out, at::Tensor a, at::Tensor residual,
               pick.is_contiguous(), "pick must be int64 on GPU");
   TORCH_CHECK(out.numel() == T * H && weight.numel() == H && N > 0,
               "add_rms_norm_rows shapes");
-  const bool parts = a.dim() == 3;
-  if (!parts) {
+  Addend from{nullptr, 0, 0};
+  if (a.dim() == 3) {
+    from = norm_addend(a, N, H);
+  } else {
     check_bf16(a, "a");
     TORCH_CHECK(a.numel() == residual.numel(), "add_rms_norm_rows shapes");
   }
   if (T == 0) return;
-  fused_add_rms_norm_launch(
-      out.data_ptr(), a.data_ptr(), residual.data_ptr(), weight.data_ptr(),
-      parts ? check_parts(a, N, H) : nullptr, pick.data_ptr<long>(),
-      parts ? (int)a.size(0) : 0, (float)eps, (int)T, (int)N, H,
-      cur_stream(residual));
+  fused_add_rms_norm_launch(out.data_ptr(), a.data_ptr(), residual.data_ptr(),
+                            weight.data_ptr(), from.data, from.chosen,
+                            pick.data_ptr<long>(), from.n, (float)eps, (int)T,
+                            (int)N, H, cur_stream(residual));
   HIP_CHECK_LAST();
 }
 

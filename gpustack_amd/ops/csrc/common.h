@@ -94,6 +94,27 @@ DEVICE_INLINE u16x8 join_parts8(const float* p, long stride, int parts) {
   return f32_to_bf8(sum);
 }
 
+// Eight neighbours of k bf16 rows `stride` apart, added up in fp32 in their order and
+// rounded. Four rows are in flight at a time.
+DEVICE_INLINE u16x8 sum_rows8(const unsigned short* p, long stride, int k) {
+  float sum[8];
+  for (int j0 = 0; j0 < k; j0 += 4) {
+    u16x8 v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      v[i] = *reinterpret_cast<const u16x8*>(p + min(j0 + i, k - 1) * stride);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float f[8];
+      bf8_to_f32(v[i], f);
+      if (j0 + i < k)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) sum[j] = j0 + i == 0 ? f[j] : sum[j] + f[j];
+    }
+  }
+  return f32_to_bf8(sum);
+}
+
 // Full-wave (64-lane) butterfly reductions.
 __device__ __forceinline__ float wave_reduce_sum(float x) {
 #pragma unroll

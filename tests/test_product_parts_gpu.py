@@ -222,3 +222,18 @@ def test_the_last_layer_norm_of_picked_rows(kind, T, W, dtype):
     ops.add_layer_norm(y, a, w, b, 1e-5, ref)
     got = ops.add_layer_norm_rows(x, a, w, b, 1e-5, rows, dtype)
     assert torch.equal(got, ref[rows])
+
+
+@pytest.mark.parametrize("k", [1, 3, 4, 8, 9])
+@pytest.mark.parametrize("T,H", [(1, 64), (17, 2048), (3, 8200)])
+def test_the_norm_adds_up_the_experts(k, T, H):
+    rnd = _gen(k + T)
+    rows, res, w = rnd(T, k, H).bfloat16(), rnd(T, H).bfloat16(), rnd(H).bfloat16()
+    x = torch.empty_like(res)
+    ops._load_hip().moe_sum(x, rows.view(T * k, H), k)
+    pick = torch.tensor([T - 1, 0], device="cuda")
+    picked = ops.add_rms_norm_rows(rows, res, w, 1e-5, pick)
+    r1, r2 = res.clone(), res.clone()
+    ops.fused_add_rms_norm(x, r1, w, 1e-5)
+    assert torch.equal(ops.add_rms_norm(rows, r2, w, 1e-5), x)
+    assert torch.equal(r1, r2) and torch.equal(picked, x[pick])
