@@ -13,6 +13,7 @@ scratch, never in live KV.
 """
 from __future__ import annotations
 
+import gc
 import os
 
 import torch
@@ -124,6 +125,20 @@ class DecodeGraphRunner:
         return meta
 
     def capture(self) -> None:
+        """Capture every bucket. The cyclic collector stays off meanwhile: an
+        engine that was dropped is a cycle, and when the collector meets it
+        inside a capture its graphs, events and pinned memory are given back by
+        calls that a capture forbids, from destructors that end the process."""
+        gc.collect()
+        collecting = gc.isenabled()
+        gc.disable()
+        try:
+            self._capture()
+        finally:
+            if collecting:
+                gc.enable()
+
+    def _capture(self) -> None:
         model, kv = self.runner.model, self.runner.kv
         pool = torch.cuda.graph_pool_handle()
         for bs in reversed(self.buckets):  # largest first reserves the pool
