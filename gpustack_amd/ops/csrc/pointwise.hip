@@ -112,8 +112,8 @@ DEVICE_INLINE u16x8 norm_addend(const unsigned short* x, const void* from,
     return *reinterpret_cast<const u16x8*>(x + row * H + v * 8);
 }
 
-template <int FROM>
-__global__ void fused_add_rms_norm_kernel(unsigned short* out,
+template <int FROM, int THREADS>
+__global__ __launch_bounds__(THREADS) void fused_add_rms_norm_kernel(unsigned short* out,
                                           const unsigned short* x,
                                           unsigned short* __restrict__ residual,
                                           const unsigned short* __restrict__ w,
@@ -122,7 +122,7 @@ __global__ void fused_add_rms_norm_kernel(unsigned short* out,
                                           int parts, float eps, int T, int N,
                                           int H) {
   const int nvec = H / 8;
-  const bool cached = nvec <= NORM_THREADS * NORM_MAX_VEC;
+  const bool cached = nvec <= THREADS * NORM_MAX_VEC;
   for (int row = blockIdx.x; row < T; row += gridDim.x) {
     long src = row;
     if (pick != nullptr) {
@@ -134,7 +134,7 @@ __global__ void fused_add_rms_norm_kernel(unsigned short* out,
     unsigned short* rp = residual + src * H;
     float vals[NORM_MAX_VEC][8];
     float ss = 0.f;
-    for (int v = threadIdx.x, slot = 0; v < nvec; v += NORM_THREADS, ++slot) {
+    for (int v = threadIdx.x, slot = 0; v < nvec; v += THREADS, ++slot) {
       u16x8 ur = *reinterpret_cast<const u16x8*>(rp + v * 8);
       const u16x8 ux = norm_addend<FROM>(x, from, src, v, parts, N, H);
       float f[8];
@@ -150,15 +150,15 @@ __global__ void fused_add_rms_norm_kernel(unsigned short* out,
         for (int i = 0; i < 8; ++i) vals[slot][i] = f[i];
       }
     }
-    __shared__ float red[NORM_THREADS / WAVE_SIZE];
+    __shared__ float red[THREADS / WAVE_SIZE];
     ss = wave_reduce_sum(ss);
     if ((threadIdx.x & (WAVE_SIZE - 1)) == 0) red[threadIdx.x / WAVE_SIZE] = ss;
     __syncthreads();
     float tot = 0.f;
 #pragma unroll
-    for (int i = 0; i < NORM_THREADS / WAVE_SIZE; ++i) tot += red[i];
+    for (int i = 0; i < THREADS / WAVE_SIZE; ++i) tot += red[i];
     const float inv = rsqrtf(tot / H + eps);
-    for (int v = threadIdx.x, slot = 0; v < nvec; v += NORM_THREADS, ++slot) {
+    for (int v = threadIdx.x, slot = 0; v < nvec; v += THREADS, ++slot) {
       float f[8];
       if (cached && slot < NORM_MAX_VEC) {
 #pragma unroll
@@ -503,6 +503,22 @@ void rms_norm_launch(void* out, const void* in, const void* w,
                      vocab, eps, T, H);
 }
 
+namespace {
+template <int THREADS>
+void norm_launch(void* out, const void* x, void* residual, const void* w,
+                 const void* from, int chosen, const long* pick, int parts,
+                 float eps, int T, int N, int H, hipStream_t s) {
+  int grid = T < 8192 ? (T < 1 ? 1 : T) : 8192;
+  hipLaunchKernelGGL(
+      (from == nullptr ? fused_add_rms_norm_kernel<ROWS, THREADS>
+       : chosen        ? fused_add_rms_norm_kernel<CHOSEN, THREADS>
+                       : fused_add_rms_norm_kernel<PARTS, THREADS>),
+      dim3(grid), dim3(THREADS), 0, s, (unsigned short*)out,
+      (const unsigned short*)x, (unsigned short*)residual,
+      (const unsigned short*)w, from, pick, parts, eps, T, N, H);
+}
+}  // namespace
+
 // out [T, H], x and residual [N, H]. from: null, or what is added instead of x:
 // fp32 parts [parts, N, H] or, with chosen, bf16 rows [N, parts, H]. pick: null
 // (T = N), or the rows that out has.
@@ -510,14 +526,16 @@ void fused_add_rms_norm_launch(void* out, const void* x, void* residual,
                                const void* w, const void* from, int chosen,
                                const long* pick, int parts, float eps, int T,
                                int N, int H, hipStream_t s) {
-  int grid = T < 8192 ? (T < 1 ? 1 : T) : 8192;
-  hipLaunchKernelGGL(
-      (from == nullptr ? fused_add_rms_norm_kernel<ROWS>
-       : chosen        ? fused_add_rms_norm_kernel<CHOSEN>
-                       : fused_add_rms_norm_kernel<PARTS>),
-      dim3(grid), dim3(NORM_THREADS), 0, s, (unsigned short*)out,
-      (const unsigned short*)x, (unsigned short*)residual,
-      (const unsigned short*)w, from, pick, parts, eps, T, N, H);
+  // Few rows of more than 2048: 512 threads, one chunk of 8 a thread up to 4096,
+  // for the latency of a row's loads (us back to back, 256 -> 512 threads: 16 rows
+  // of 4096 3.4 -> 2.8, in 8 parts 4.9 -> 3.8, of 8192 4.8 -> 3.7 and 7.6 -> 5.6;
+  // 512 rows of 4096 4.7 -> 4.5); more rows fill the CUs with 256.
+  if (T <= 512 && H > 2048)
+    norm_launch<512>(out, x, residual, w, from, chosen, pick, parts, eps, T, N, H,
+                     s);
+  else
+    norm_launch<NORM_THREADS>(out, x, residual, w, from, chosen, pick, parts, eps,
+                              T, N, H, s);
 }
 
 void rope_neox_launch(const long* positions, void* q, void* k,
