@@ -99,12 +99,23 @@ class RaggedMeta:
         return c
 
     def scan_runs(self, heads: int, n_state: int, vdim: int, dtype):
-        """Runs of rows for ops.state_scan, or None for a batch of short
+        """ops.state_scan's `runs` and `cut`, or nothing for a batch of short
         portions or operands that its chunk kernel does not take."""
         if dtype != torch.bfloat16 or not 32 <= n_state <= 128 or vdim < 32:
-            return None
+            return {}
         rows = ops.scan_run_rows(self.seq_news, heads, vdim)
-        return self.scan_chunks(rows) if rows else None
+        if not rows:
+            return {}
+        if self._tiles is None:
+            self._tiles = {}
+        key = ("runs", rows)
+        r = self._tiles.get(key)
+        if r is None:
+            runs, cut = ops.build_scan_runs(self.seq_starts, self.seq_news,
+                                            rows, self.block_tables.device)
+            r = {"runs": runs, "cut": cut} if cut else {}
+            self._tiles[key] = r
+        return r
 
     def attn_tiles(self, heads: int, kv_heads: int, maps: int,
                    short: bool = False):

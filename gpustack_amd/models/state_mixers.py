@@ -97,8 +97,8 @@ class Mamba2Mixer(nn.Module):
                        self.dt_bias, self.a_log, self.skip, None, ssm_state,
                        rg.seq_first, rg.seq_rows, rg.state_slots, rg.pos32,
                        single=max(rg.seq_news, default=1) <= 1,
-                       runs=rg.scan_runs(m.heads, m.state, m.vdim, h.dtype)
-                       if h.is_cuda else None)
+                       **(rg.scan_runs(m.heads, m.state, m.vdim, h.dtype)
+                          if h.is_cuda else {}))
         g = torch.empty(T, m.inner, dtype=h.dtype, device=h.device)
         ops.gated_group_norm(g, y, u[:, :m.inner], self.norm, m.norm_groups,
                              self.eps, True)
@@ -137,8 +137,8 @@ class LightningMixer(nn.Module):
                        self.decay, ssm_state, rg.seq_first, rg.seq_rows,
                        rg.state_slots, rg.pos32,
                        single=max(rg.seq_news, default=1) <= 1,
-                       runs=rg.scan_runs(m.heads, m.state, m.vdim, h.dtype)
-                       if h.is_cuda else None)
+                       **(rg.scan_runs(m.heads, m.state, m.vdim, h.dtype)
+                          if h.is_cuda else {}))
         g = torch.empty(T, m.inner, dtype=h.dtype, device=h.device)
         ops.gated_group_norm(g, y, u[:, 2 * self.nqk + m.inner:], self.norm,
                              1, self.eps, False)

@@ -1289,6 +1289,11 @@ def causal_conv_silu(out, src, col0: int, w, b, conv_state, seq_first,
                state_slots, row_seq, pos32, single=single)
 
 
+# Rows a sequence, on average, from which state_scan takes its chunk kernel
+# (CHUNK_ROWS in ops/csrc/state_scan.hip)
+SCAN_CHUNK_ROWS = 24
+
+
 def scan_run_rows(seq_news, heads: int, vdim: int) -> int:
     """Rows of a run for state_scan, or 0 where whole sequences do as well: up
     to half of the chip's 512 places for workgroups (64 value channels of a
@@ -1297,10 +1302,13 @@ def scan_run_rows(seq_news, heads: int, vdim: int) -> int:
     266, 1 x 1000 191 / 107, 1 x 500 97 / 70, 1 x 250 50 / 50, 2 x 2000 364 /
     259, six of 301 to 1900 433 / 353, but 8 x 500 141 / 250, 4 x 200 47 / 91;
     16 heads of 128 1 x 4000 918 / 260, 1 x 500 121 / 77, the six 428 / 241,
-    8 x 500 133 / 173, 32 x 125 91 / 145."""
-    longest = max(seq_news, default=0)
+    8 x 500 133 / 173, 32 x 125 91 / 145. Batches of so many short sequences
+    that no chunk kernel runs have none either."""
+    longest, rows = max(seq_news, default=0), sum(seq_news)
     groups = heads * ((vdim + 63) // 64)
-    if longest < 256 or longest * 256 <= sum(seq_news) * groups:
+    if longest < 256 or longest * 256 <= rows * groups:
+        return 0
+    if rows < SCAN_CHUNK_ROWS * len(seq_news):
         return 0
     return (longest // 8 + 64 + 31) // 32 * 32
 
@@ -1309,17 +1317,19 @@ def state_scan(y, src, col_x: int, col_b: int, col_c: int, dt_src,
                col_dt: int, heads: int, groups: int, n_state: int, vdim: int,
                act_silu: bool, dt_bias, a_log, skip, decay, state, seq_first,
                seq_rows, state_slots, pos32, single: bool = False,
-               runs=None) -> None:
+               runs=None, cut: int | None = None) -> None:
     """`single` (a host-side hint): every sequence brings one row, as in a
     decode step; the GPU then streams the states through its step kernel.
-    `runs` (build_scan_chunks; a prompt): the GPU cuts
-    the sequences into runs of rows that workgroups take side by side."""
+    `runs` (build_scan_runs; a prompt): the GPU cuts the sequences into runs of
+    rows that workgroups take side by side. `cut`: how many of the list, its
+    first, belong to sequences of several runs (None: all may); two states of
+    all heads are kept for each of these during the call."""
     k = _state_backend(src)
     if k is not None:
         k.state_scan(y, src, col_x, col_b, col_c, dt_src, col_dt, heads,
                      groups, n_state, vdim, act_silu, dt_bias, a_log, skip,
                      decay, state, seq_first, seq_rows, state_slots, pos32,
-                     single, runs)
+                     single, runs, cut)
     else:
         torch_ref.state_scan(y, src, col_x, col_b, col_c, dt_src, col_dt,
                              heads, groups, n_state, vdim, act_silu, dt_bias,
@@ -1483,10 +1493,26 @@ def build_scan_chunks(seq_starts, seq_news, size: int, device):
     """Runs of at most `size` rows of one sequence in order, for scans that
     split a prompt over workgroups: int32 [n, 4] = first row, rows,
     sequence, list index of the sequence's first run."""
+    return to_device([(_scan_chunks(seq_starts, seq_news, size,
+                                    range(len(seq_news))), torch.int32)],
+                     device)[0]
+
+
+def build_scan_runs(seq_starts, seq_news, size: int, device):
+    """(build_scan_chunks' list with the sequences of one run at its end, the
+    number of entries in front of them)."""
+    order = sorted(range(len(seq_news)), key=lambda i: seq_news[i] <= size)
+    runs = to_device([(_scan_chunks(seq_starts, seq_news, size, order),
+                       torch.int32)], device)[0]
+    return runs, sum(-(-n // size) for n in seq_news if n > size)
+
+
+def _scan_chunks(seq_starts, seq_news, size: int, order):
     import numpy as np
 
     parts, n = [], 0
-    for i, (st, new) in enumerate(zip(seq_starts, seq_news)):
+    for i in order:
+        st, new = seq_starts[i], seq_news[i]
         lo = np.arange(0, new, size)
         t = np.empty((lo.size, 4), dtype=np.int32)
         t[:, 0] = st + lo
@@ -1495,8 +1521,7 @@ def build_scan_chunks(seq_starts, seq_news, size: int, device):
         t[:, 3] = n
         n += lo.size
         parts.append(t)
-    c = np.concatenate(parts) if parts else np.empty((0, 4), dtype=np.int32)
-    return to_device([(c, torch.int32)], device)[0]
+    return np.concatenate(parts) if parts else np.empty((0, 4), dtype=np.int32)
 
 
 def gru_scan(y, src, col_z: int, col_u: int, col_g: int, z_b, u_b, state,

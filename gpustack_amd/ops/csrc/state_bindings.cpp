@@ -13,7 +13,8 @@ int add_layer_norm_launch(float*, const void*, int, const float*, const float*, 
 void head_norm_store_launch(void*, void*, long, int, int, int, const float*, const float*, int, float, float, const int*, const void*, long, const float*, void*, void*, const long*, long, int, int, int, float, int, int, int, hipStream_t);
 void value_page_store_launch(const void*, long, int, void*, const long*, long, const int*, int, int, int, int, int, int, hipStream_t);
 void route_topk_launch(int*, float*, const float*, int, const float*, int, int, int, int, int, int, int, int, float, hipStream_t);
-int state_scan_launch(float*, const void*, long, int, int, int, const void*, long, int, int, int, int, int, int, const float*, const float*, const float*, const float*, float*, const int*, const int*, const int*, const int*, int, int, int, int, int, const int*, int, float*, float*, float*, hipStream_t);
+int state_scan_launch(float*, const void*, long, int, int, int, const void*, long, int, int, int, int, int, int, const float*, const float*, const float*, const float*, float*, const int*, const int*, const int*, const int*, int, int, int, int, int, const int*, int, int, float*, float*, float*, hipStream_t);
+bool state_scan_cuts(int, int, int, int, long, int, int, int, long, int);
 void gated_group_norm_launch(void*, const float*, const float*, const void*, long, const float*, int, int, int, float, int, int, int, hipStream_t);
 int delta_scan_launch(float*, const void*, long, int, int, int, const void*, long, int, int, int, int, int, int, const float*, const float*, float*, const int*, const int*, const int*, const int*, int, int, int, int, int, hipStream_t);
 int delta_scan_max_state();
@@ -238,7 +239,8 @@ void state_scan(Tensor y, Tensor src, long col_x, long col_b, long col_c,
                 long n_state, long vdim, bool act_silu, OptTensor dt_bias,
                 OptTensor a_log, OptTensor skip, OptTensor decay, Tensor state,
                 Tensor seq_first, Tensor seq_rows, Tensor state_slots,
-                Tensor pos32, bool single, OptTensor runs) {
+                Tensor pos32, bool single, OptTensor runs,
+                c10::optional<long> cut) {
   chk(y, "y", at::kFloat);
   chk(state, "state", at::kFloat);
   const int bf = view_kind(src, "src");
@@ -280,17 +282,27 @@ void state_scan(Tensor y, Tensor src, long col_x, long col_b, long col_c,
   }
   const int nseq = seq_view(seq_first, seq_rows, state_slots, pos32, T);
   const int* rp = nullptr;
-  int nruns = 0;
+  int nruns = 0, ncut = 0;
   Tensor ends, scratch, falls;
   if (runs.has_value()) {
     chk(*runs, "runs", at::kInt);
     TORCH_CHECK(runs->dim() == 2 && runs->size(1) == 4,
                 "runs must be [n, 4] (build_scan_chunks)");
-    rp = runs->data_ptr<int>();
-    nruns = (int)runs->size(0);
-    ends = at::empty({nruns, heads, n_state, vdim}, y.options());
-    scratch = at::empty_like(ends);
-    falls = at::empty({nruns, heads}, y.options());
+    TORCH_CHECK(!cut.has_value() || (*cut >= 0 && *cut <= runs->size(0)),
+                "more runs cut than there are");
+    // places for what the kernel hands over, only where it takes runs
+    if (runs->size(0) > nseq &&
+        state_scan_cuts(bf, single ? 1 : 0, (int)n_state, (int)vdim, src.stride(0),
+                        (int)col_x, (int)col_b, (int)col_c, T, nseq)) {
+      rp = runs->data_ptr<int>();
+      nruns = (int)runs->size(0);
+      ncut = cut.has_value() ? (int)*cut : nruns;
+    }
+    if (ncut > 0) {
+      ends = at::empty({ncut, heads, n_state, vdim}, y.options());
+      scratch = at::empty_like(ends);
+      falls = at::empty({ncut, heads}, y.options());
+    }
   }
   const int ok = state_scan_launch(
       y.data_ptr<float>(), src.data_ptr(), src.stride(0), (int)col_x,
@@ -299,9 +311,9 @@ void state_scan(Tensor y, Tensor src, long col_x, long col_b, long col_c,
       state.data_ptr<float>(), seq_first.data_ptr<int>(),
       seq_rows.data_ptr<int>(), state_slots.data_ptr<int>(),
       pos32.data_ptr<int>(), nseq, (int)state.size(0), T, bf, single ? 1 : 0,
-      rp, nruns, nruns ? ends.data_ptr<float>() : nullptr,
-      nruns ? scratch.data_ptr<float>() : nullptr,
-      nruns ? falls.data_ptr<float>() : nullptr, cur_stream(src));
+      rp, nruns, ncut, ncut ? ends.data_ptr<float>() : nullptr,
+      ncut ? scratch.data_ptr<float>() : nullptr,
+      ncut ? falls.data_ptr<float>() : nullptr, cur_stream(src));
   TORCH_CHECK(ok, "state size unsupported");
   HIP_CHECK_LAST();
 }
@@ -500,7 +512,15 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("head_norm_store", &head_norm_store);
   m.def("route_topk", &route_topk);
   m.def("short_conv", &short_conv);
-  m.def("state_scan", &state_scan);
+  m.def("state_scan", &state_scan, py::arg("y"), py::arg("src"),
+        py::arg("col_x"), py::arg("col_b"), py::arg("col_c"),
+        py::arg("dt_src"), py::arg("col_dt"), py::arg("heads"),
+        py::arg("groups"), py::arg("n_state"), py::arg("vdim"),
+        py::arg("act_silu"), py::arg("dt_bias"), py::arg("a_log"),
+        py::arg("skip"), py::arg("decay"), py::arg("state"),
+        py::arg("seq_first"), py::arg("seq_rows"), py::arg("state_slots"),
+        py::arg("pos32"), py::arg("single"), py::arg("runs"),
+        py::arg("cut") = py::none());
   m.def("delta_scan", &delta_scan);
   m.def("memory_scan", &memory_scan);
   m.def("rope_table", &rope_table);

@@ -59,9 +59,11 @@ struct ScanArgs {
   const int* runs;         // [nruns, 4] first row, rows, sequence, the list
                            // index of the sequence's first run
   int nruns, nseq;
-  float* ends;             // [nruns, H, N, P] state behind a run
-  float* scratch;          // [nruns, H, N, P]
-  float* falls;            // [nruns, H] product of a run's decays
+  int ncut;                // runs in front of the list that have places below;
+                           // only sequences of one run may lie behind them
+  float* ends;             // [ncut, H, N, P] state behind a run
+  float* scratch;          // [ncut, H, N, P]
+  float* falls;            // [ncut, H] product of a run's decays
 };
 
 constexpr int CH = 16;     // rows staged per pass
@@ -352,6 +354,8 @@ __global__ __launch_bounds__(256) void state_scan_vec_kernel(
 // puts the state in front of it together from the runs before and goes through
 // its rows as above. The slot is read by the first launch (the second takes the
 // first run's state from `scratch`) and written by the last run in the second.
+// Sequences of one run need none of that: they lie at the end of the list, without
+// places, and the first launch leaves them out.
 // 64 heads of 128 x 64, one sequence of 4000 rows 723 -> 266 us, six of 301 to 1900
 // 433 -> 353; 16 heads of 128 x 128 918 -> 260 and 428 -> 241.
 typedef __attribute__((ext_vector_type(4))) float sc_f32x4;
@@ -389,6 +393,7 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
     if (s < 0 || s >= p.nseq || run0 < 0 || run0 > run) return;
     ends = first + n >= p.seq_first[s] + p.seq_rows[s];
     if (PART == ENDS && ends) return;
+    if (run >= p.ncut && (run != run0 || !ends)) return;
   }
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -623,14 +628,16 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
       }
     __syncthreads();
   }
-  float* own = PART == WHOLE ? sp
-               : (PART == ENDS ? p.ends : p.scratch) + (long)run * stride + h * NP_;
+  float* own = PART == WHOLE || (PART == OUTPUTS && ends)
+                   ? sp
+                   : (PART == ENDS ? p.ends : p.scratch) + (long)run * stride +
+                         h * NP_;
   if constexpr (PART == ENDS)
     if (tid == 0 && pb0 == 0) p.falls[(long)run * p.H + h] = fall;
   // A value that is infinite or NaN belongs to its own row and those behind
   // it, but the weights of 0 above the diagonal carried it to the rows in
   // front: such columns are walked again row by row, on the state in memory
-  // (the slot, or a run's own place).
+  // (the slot, or the own place of a run that is not its sequence's last).
   if (__any(odd != 0.f)) {
     auto load = [&](const unsigned short* at) {
       const float f = bf2f(*at);
@@ -640,8 +647,8 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
 #pragma unroll 1
       for (int nn = g; nn < N && live; nn += 4) {
         const long i = (long)nn * P + pc;
-        if (run == run0) {
-          if (PART == ENDS || ends) own[i] = sp[i];
+        if (run == run0) {                   // of OUTPUTS it is there already
+          if (PART == ENDS) own[i] = sp[i];
           continue;
         }
         const float* at = p.ends + (long)run0 * stride + h * NP_ + i;
@@ -678,15 +685,9 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
           y[(long)(first + i) * p.H * P + h * P + pc] = part + skip * v;
       }
     }
-    if (PART == OUTPUTS && ends)
-      for (int nn = g; nn < N && live; nn += 4)
-        sp[(long)nn * P + pc] = own[(long)nn * P + pc];
     return;
   }
-  if (PART == ENDS || ends) {
-    float* to = PART == ENDS ? own : sp;
-    each([&](float x, long i) { return to[i] = x; });
-  }
+  if (PART == ENDS || ends) each([&](float x, long i) { return own[i] = x; });
 }
 
 // Single rows (decode): the state itself is the traffic, so one workgroup
@@ -922,32 +923,46 @@ void scan_launch(float* y, const void* src, const void* dt, const ScanArgs& p,
 // than the head has.
 constexpr int CHUNK_ROWS = 24;
 
+// 16-byte staging: bf16 rows whose sizes and columns are multiples of 8
+bool vec_rows(int N, int P, long ld_src, int col_x, int col_b, int col_c) {
+  return N % 8 == 0 && P % 8 == 0 && ld_src % 8 == 0 && col_x % 8 == 0 &&
+         col_b % 8 == 0 && col_c % 8 == 0;
+}
+
+// Chunks on the matrix instructions from CHUNK_ROWS rows a sequence on (on
+// average: the sizes themselves are on the device), where a wave's 16 value
+// channels and 16-row state tiles are not mostly padding
+bool chunk_rows(int bf, bool vec, int N, int P, long T, int nseq) {
+  return bf && vec && N >= 32 && N <= 128 && P >= 32 &&
+         T >= (long)CHUNK_ROWS * nseq;
+}
+
+// batches of single rows: the streaming step kernel, when the value size splits
+// a workgroup evenly into 16-byte columns
+bool step_rows(int single, int N, int P) {
+  const int P4 = P / 4;
+  return single && P % 4 == 0 && P4 >= 1 && P4 <= 256 && 256 % P4 == 0 &&
+         (size_t)(2 * N + P + (256 / P4) * P) * sizeof(float) <= 48 * 1024;
+}
+
 template <typename TS, typename TD>
 bool scan_pick(float* y, const void* src, const void* dt, const ScanArgs& p,
                int nseq, hipStream_t s) {
   int tpp = 1;
   while (tpp < 8 && ((p.N + tpp - 1) / tpp > 32 || 64 / tpp > max(p.P, 8)))
     tpp *= 2;
-  // 16-byte staging: bf16 rows whose sizes and columns are multiples of 8
-  const bool vec = p.N % 8 == 0 && p.P % 8 == 0 &&
-                   p.ld_src % 8 == 0 && p.col_x % 8 == 0 && p.col_b % 8 == 0 &&
-                   p.col_c % 8 == 0;
-  // Chunks on the matrix instructions from CHUNK_ROWS rows a sequence on (on
-  // average: the sizes themselves are on the device), where a wave's 16 value
-  // channels and 16-row state tiles are not mostly padding
-  if (sizeof(TS) == 2 && vec && p.N >= 32 && p.N <= 128 && p.P >= 32 &&
-      (long)p.T >= (long)CHUNK_ROWS * nseq) {
-    const bool cut = p.nruns > nseq;
-    const dim3 grid(cut ? p.nruns : nseq, p.H, (p.P + 63) / 64);
-#define CHUNKS(NT, PART)                                                     \
-  state_chunk_kernel<NT, PART><<<grid, 256, 0, s>>>(                         \
-      y, (const unsigned short*)src, (const unsigned short*)dt, p)
+  const bool vec = vec_rows(p.N, p.P, p.ld_src, p.col_x, p.col_b, p.col_c);
+  if (chunk_rows(sizeof(TS) == 2, vec, p.N, p.P, p.T, nseq)) {
+#define CHUNKS(NT, PART, GROUPS)                                             \
+  state_chunk_kernel<NT, PART>                                               \
+      <<<dim3(GROUPS, p.H, (p.P + 63) / 64), 256, 0, s>>>(                   \
+          y, (const unsigned short*)src, (const unsigned short*)dt, p)
 #define CHUNKS_NT(NT)                                                        \
-  if (cut) {                                                                 \
-    CHUNKS(NT, ENDS);                                                        \
-    CHUNKS(NT, OUTPUTS);                                                     \
+  if (p.ncut > 0) {                                                          \
+    CHUNKS(NT, ENDS, p.ncut);                                                \
+    CHUNKS(NT, OUTPUTS, p.nruns);                                            \
   } else {                                                                   \
-    CHUNKS(NT, WHOLE);                                                       \
+    CHUNKS(NT, WHOLE, nseq);                                                 \
   }
     if (p.N <= 64) { CHUNKS_NT(4) } else { CHUNKS_NT(8) }
 #undef CHUNKS_NT
@@ -987,10 +1002,19 @@ bool scan_pick(float* y, const void* src, const void* dt, const ScanArgs& p,
 
 int state_scan_max_state() { return 8 * 64; }
 
+// Whether a call of these sizes may be cut into runs: the chunk kernel takes it.
+bool state_scan_cuts(int src_bf, int single, int N, int P, long ld_src, int col_x,
+                     int col_b, int col_c, long T, int nseq) {
+  return !step_rows(single, N, P) &&
+         chunk_rows(src_bf, vec_rows(N, P, ld_src, col_x, col_b, col_c), N, P, T,
+                    nseq);
+}
+
 // src_bf: src and dt_src are bf16 (else fp32). single: the caller expects
 // one row per sequence (a hint: any batch is still computed correctly).
-// runs (or null): the sequences cut into nruns > nseq runs of rows, for the
-// chunk kernel, with ends and scratch [nruns, H, N, P] and falls [nruns, H].
+// runs: the sequences cut into nruns runs of rows, where state_scan_cuts; the
+// first ncut of them (0: no runs) with ends and scratch [ncut, H, N, P] and falls
+// [ncut, H].
 // Returns 0 when no instantiation covers the sizes.
 int state_scan_launch(float* y, const void* src, long ld_src, int col_x,
                       int col_b, int col_c, const void* dt_src, long ld_dt,
@@ -1000,11 +1024,12 @@ int state_scan_launch(float* y, const void* src, long ld_src, int col_x,
                       const int* seq_first, const int* seq_rows,
                       const int* state_slots, const int* pos32, int nseq,
                       int nslots, int T, int src_bf, int single,
-                      const int* runs, int nruns, float* ends, float* scratch,
+                      const int* runs, int nruns, int ncut, float* ends,
+                      float* scratch,
                       float* falls, hipStream_t s) {
   if (T <= 0 || nseq <= 0) return 1;
   ScanArgs p;
-  p.runs = runs; p.nruns = nruns; p.nseq = nseq; p.ends = ends;
+  p.runs = runs; p.nruns = nruns; p.nseq = nseq; p.ncut = ncut; p.ends = ends;
   p.scratch = scratch; p.falls = falls;
   p.ld_src = ld_src; p.ld_dt = ld_dt; p.col_x = col_x; p.col_b = col_b;
   p.col_c = col_c; p.col_dt = col_dt; p.H = H; p.G = G; p.N = N; p.P = P;
@@ -1012,11 +1037,8 @@ int state_scan_launch(float* y, const void* src, long ld_src, int col_x,
   p.decay = decay; p.state = state; p.seq_first = seq_first;
   p.seq_rows = seq_rows; p.state_slots = state_slots; p.pos32 = pos32;
   p.nslots = nslots; p.T = T;
-  // batches of single rows: the streaming step kernel, when the value size
-  // splits a workgroup evenly into 16-byte columns
-  const int P4 = P / 4;
-  if (single && P % 4 == 0 && P4 >= 1 && P4 <= 256 && 256 % P4 == 0 &&
-      (size_t)(2 * N + P + (256 / P4) * P) * sizeof(float) <= 48 * 1024) {
+  if (step_rows(single, N, P)) {
+    const int P4 = P / 4;
     const size_t smem = (size_t)(2 * N + P + (256 / P4) * P) * sizeof(float);
     if (src_bf)
       state_step_kernel<unsigned short><<<dim3(nseq, H), 256, smem, s>>>(

@@ -189,3 +189,42 @@ def test_not_finite(bad, at):
         assert float((got[ok].double() - want[ok]).abs().max()) <= 4e-6 * scale
     assert bool(ref[:at].isfinite().all()) and not bool(
         ref[at:, P + 70].isfinite().any())
+
+
+@pytest.mark.parametrize("bad", [None, float("inf"), float("nan")])
+@pytest.mark.parametrize("news", [[20, 130, 64, 200, 31], [96, 97, 1, 60]])
+def test_whole_sequences_behind_the_runs(news, bad):
+    """Sequences of one run have no places in the workspace, also where their
+    columns are walked again on the slot."""
+    from gpustack_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(sum(news))
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    T, S, H, N, P = sum(news), len(news), 2, 64, 96
+    hists, slots = [7, 5, 0, 9, 3][:S], [3, 0, 5, 1, 2][:S]
+    src = rnd(T, H * (P + 2 * N)).bfloat16()
+    first = [sum(news[:i]) for i in range(S)]
+    if bad is not None:
+        for f, n in zip(first, news):
+            src[f + n // 2, P + 70] = bad
+    decay = torch.tensor([0.9, -0.97], device="cuda")
+    state = rnd(7, H, N, P)
+    cb, cc = H * P, H * (P + N)
+    a = decay.double().expand(T, H)
+    ref, ref_s = _walk(src, 0, cb, cc, H, H, N, P, False, a,
+                       torch.ones_like(a), None, state, news, hists, slots)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    y = torch.zeros(T, H * P, device="cuda")
+    runs, cut = ops.build_scan_runs(first, news, 64, "cuda")
+    assert 0 < cut < len(runs)
+    spare = state[6].clone()
+    ops.state_scan(y, src, 0, cb, cc, None, 0, H, H, N, P, False, None, None,
+                   None, decay, state, i32(first), i32(news), i32(slots),
+                   i32([h + j for h, n in zip(hists, news) for j in range(n)]),
+                   runs=runs, cut=cut)
+    for got, want in ((y, ref), (state, ref_s)):
+        ok = want.isfinite()
+        assert torch.equal(got.isfinite(), ok)
+        scale = float(want[ok].abs().max())    # fp32 sums, as above
+        assert float((got[ok].double() - want[ok]).abs().max()) <= 4e-6 * scale
+    assert torch.equal(state[6], spare)
