@@ -109,6 +109,7 @@ class DecodeGraphRunner:
             logits_indices=self.logits_idx[:bs],
             block_tables=self.block_tables[:bs],
             seq_lens=self.seq_lens[:bs],
+            checked=True,         # by run, or by the sampler that feeds them
         )
         if self.ragged:
             meta.ragged = RaggedMeta(
@@ -169,7 +170,7 @@ class DecodeGraphRunner:
         bucket = next(b for b in self.buckets if b >= bs)
         # host staging (numpy views over pinned memory)
         if token_src is None:
-            self.n_tokens[:bs] = batch.token_ids
+            self.n_tokens[:bs] = self.runner.in_vocab(batch.token_ids)
         self.n_positions[:bs] = batch.positions
         self.n_slots[:bs] = batch.slot_mapping
         self.n_seq_lens[:bs] = np.asarray(batch.seq_lens, dtype=np.int32)

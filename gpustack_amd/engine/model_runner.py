@@ -496,6 +496,7 @@ class ModelRunner:
             self.cp_suffixes += 1
         dev = self.device
         comm = self.comm
+        self.in_vocab(batch.token_ids)
         if batch.is_suffix:
             # chunk-continuation / suffix rows: split each seq's NEW rows;
             # this rank's history = the seq's cached tokens + the chunk
@@ -550,6 +551,7 @@ class ModelRunner:
             block_tables=bt.to(dev),
             suffix_meta=(tiles, starts, hists, news),
             cp=CPMeta(comm, pad_rows, perm.to(dev)),
+            checked=True,
         )
         return tokens, meta
 
@@ -599,9 +601,24 @@ class ModelRunner:
             rg.seq_first, rg.seq_rows, rg.state_slots = up[4].unbind(0)
         return rg
 
+    def in_vocab(self, ids) -> np.ndarray:
+        """Token ids as an array, refused where the vocabulary has no such id:
+        ForwardMeta.checked promises it for them. (The models with a ragged
+        view have an embedding of their own, which takes any id.)"""
+        ids = np.asarray(ids, dtype=np.int64)
+        # negative ids are the largest unsigned ones
+        if not self.ragged and ids.size \
+                and int(ids.view(np.uint64).max()) >= self.cfg.spec.vocab_size:
+            raise IndexError("a token id outside the vocabulary of "
+                             f"{self.cfg.spec.vocab_size}")
+        return ids
+
     def _meta(self, batch: ScheduledBatch) -> tuple[torch.Tensor, ForwardMeta]:
         tokens, meta = self._meta_by_kind(batch)
         if batch.logit_rows is not None:
+            T = tokens.shape[0]
+            if any(not -T <= r < T for r in batch.logit_rows):
+                raise IndexError(f"a logit row outside the batch's {T} rows")
             meta.logits_indices = ops.to_device(
                 [(batch.logit_rows, torch.long)], self.device)[0]
         if self.ragged:
@@ -627,7 +644,7 @@ class ModelRunner:
         dev = self.device
         i32, i64 = torch.int32, torch.long
         # what every kind of step has; each adds its own, all in one copy
-        parts = [(batch.token_ids, i64), (batch.positions, i64),
+        parts = [(self.in_vocab(batch.token_ids), i64), (batch.positions, i64),
                  (batch.slot_mapping, i64)]
 
         def table(seqs, repeat=lambda i: 1):
@@ -739,6 +756,7 @@ class ModelRunner:
                 block_tables=bt,
                 seq_lens=lens,
             )
+        meta.checked = True
         slots = self._row_lora_slots(batch)
         if slots is not None:
             from ..models.lora import BatchLora
@@ -760,7 +778,7 @@ class ModelRunner:
         for p, L in zip(prompts, lens):
             flat.extend(p[:L])
             positions.extend(range(L))
-        tokens = torch.tensor(flat, dtype=torch.long, device=dev)
+        tokens = torch.tensor(self.in_vocab(flat), device=dev)
         pos = torch.tensor(positions, dtype=torch.long, device=dev)
         slots = torch.full((len(flat),), -1, dtype=torch.long, device=dev)
         tiles = ops.build_prefill_tiles(lens, dev, ops.PREFILL_ROWS)
@@ -773,6 +791,7 @@ class ModelRunner:
             logits_indices=torch.tensor(idx, dtype=torch.long, device=dev),
             seq_lens_list=lens,
             tile_start=tiles[0], tile_q0=tiles[1], tile_len=tiles[2],
+            checked=True,
         )
         logits = self.model(tokens, meta, self.kv)
         if self.comm.pp_size > 1:
@@ -797,7 +816,7 @@ class ModelRunner:
         for p, L in zip(prompts, lens):
             flat.extend(p[:L])
             positions.extend(range(L))
-        tokens = torch.tensor(flat, dtype=torch.long, device=dev)
+        tokens = torch.tensor(self.in_vocab(flat), device=dev)
         pos = torch.tensor(positions, dtype=torch.long, device=dev)
         slots = torch.full((len(flat),), -1, dtype=torch.long, device=dev)
         tiles = ops.build_prefill_tiles(lens, dev, ops.PREFILL_ROWS)
@@ -806,6 +825,7 @@ class ModelRunner:
             logits_indices=torch.zeros(1, dtype=torch.long, device=dev),
             seq_lens_list=lens,
             tile_start=tiles[0], tile_q0=tiles[1], tile_len=tiles[2],
+            checked=True,
         )
         hidden = self.model(tokens, meta, self.kv, return_hidden=True)
         if self.comm.pp_size > 1:

@@ -134,7 +134,7 @@ class LivasunForCausalLM(nn.Module):
                 f = layer.mlp(h, None)
             else:
                 f = a
-            if nxt is None and not return_hidden:
+            if nxt is None and meta.checked and not return_hidden:
                 last = f              # added where the final norm picks rows
             else:
                 ops.add_layer_norm(x, f, nw, nb, eps, h)

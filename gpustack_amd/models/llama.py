@@ -188,6 +188,10 @@ class ForwardMeta:
     # stay local-row)
     cp: object | None = None
     ragged: RaggedMeta | None = None
+    # the host has seen that every token id lies in the vocabulary and every
+    # entry of logits_indices among the rows: kernels may gather by them that,
+    # unlike torch's gathers, do not refuse others
+    checked: bool = False
 
 
 class W4Pack:
@@ -1378,7 +1382,7 @@ class LlamaForCausalLM(nn.Module):
             x = self.comm.recv_hidden(
                 (token_ids.shape[0], self.spec.hidden_size),
                 self.dtype, self.device)
-        elif (len(self.layers) and not self.spec.embed_scale
+        elif (meta.checked and len(self.layers) and not self.spec.embed_scale
               and self.layers[0].plain_start()
               and (off is None or off.first > 0)
               and ops.embed_rms_norm_ok(token_ids, self.embed)):
@@ -1418,13 +1422,14 @@ class LlamaForCausalLM(nn.Module):
             _layer_norm(x, x, self.final_norm, self.spec.rms_norm_eps)
         elif residual is None:
             ops.rms_norm(x, x, self.final_norm, self.spec.rms_norm_eps)
-        elif not return_hidden:
+        elif meta.checked and not return_hidden:
             hidden = ops.add_rms_norm_rows(x, residual, self.final_norm,
                                            self.spec.rms_norm_eps,
                                            meta.logits_indices)
         else:
             x = ops.add_rms_norm(x, residual, self.final_norm,
                                  self.spec.rms_norm_eps)
+            residual = None
         if return_hidden:
             return x  # all rows, post final norm (embedding serving)
         if residual is None:

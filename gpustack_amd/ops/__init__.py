@@ -140,7 +140,8 @@ def add_rms_norm(x, residual, weight, eps: float):
 
 def add_rms_norm_rows(x, residual, weight, eps: float, rows):
     """add_rms_norm's result at the given rows, residual left as it is or not:
-    the last norm, of the rows whose logits are asked for."""
+    the last norm, of the rows whose logits are asked for. The caller has seen
+    that there are such rows: the GPU clamps others."""
     if residual.is_cuda and residual.is_contiguous() and rows.is_cuda \
             and rows.dim() == 1 and rows.is_contiguous() \
             and residual.dtype == torch.bfloat16 and residual.dim() == 2 \
@@ -153,7 +154,8 @@ def add_rms_norm_rows(x, residual, weight, eps: float, rows):
 
 
 def embed_rms_norm(tokens, embed, weight, eps: float):
-    """(rows of the tokens, their norm). GPU only (embed_rms_norm_ok)."""
+    """(rows of the tokens, their norm). GPU only (embed_rms_norm_ok). The
+    caller has seen that the table has such rows: others come out as zeros."""
     x = torch.empty(tokens.shape[0], embed.shape[1], dtype=embed.dtype,
                     device=embed.device)
     out = torch.empty_like(x)
@@ -1234,7 +1236,8 @@ def add_layer_norm(x, a, w, b, eps: float, h) -> None:
 
 def add_layer_norm_rows(x, a, w, b, eps: float, rows, dtype):
     """The layer norm of the given rows of x + a, x getting the sum or not: the
-    end of a stream, of the rows whose logits are asked for."""
+    end of a stream, of the rows whose logits are asked for. With an `a` the
+    caller has seen that there are such rows: the GPU clamps others."""
     k = _state_backend(x)
     h = torch.empty(rows.shape[0], x.shape[1], dtype=dtype, device=x.device)
     if k is not None and a is not None and rows.is_cuda and x.shape[0] > 0 \

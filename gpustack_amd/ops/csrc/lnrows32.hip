@@ -119,6 +119,7 @@ __global__ __launch_bounds__(ROW_THREADS) void add_layer_norm_kernel(
 // pick (or null): h's row t is the norm of row pick[t] of the N, and the sum goes
 // nowhere: the stream's end, of the rows whose logits are asked for. One launch
 // for the last sum, the gather and the norm: 64 rows of 2048 4.7 + 4.7 + 4.7 -> 5.
+// Picks out of range, which the caller refuses (ForwardMeta.checked), are clamped.
 enum AddFrom { NOTHING, ROWS16, ROWS32, PARTS };
 
 template <typename TH, int NV, int FROM>

@@ -19,8 +19,9 @@ constexpr int NORM_MAX_VEC = 4; // u16x8 per thread held in registers
 
 // tokens (or null): `in` is a table of `vocab` rows, row t the one of tokens[t],
 // which `rows` gets as well. That is the embedding and the first norm in a launch:
-// 16 rows of 4096 12.5 + 4.6 -> 5.1 us, 48 4.7 + 4.7 -> 5.1. Tokens out of range
-// make a row of zeros.
+// 16 rows of 4096 12.5 + 4.6 -> 5.1 us, 48 4.7 + 4.7 -> 5.1. The caller refuses
+// tokens out of range (ForwardMeta.checked); here they only read nothing outside
+// the table and make a row of zeros.
 __global__ void rms_norm_kernel(unsigned short* __restrict__ out,
                                 const unsigned short* __restrict__ in,
                                 const unsigned short* __restrict__ w,
@@ -97,7 +98,8 @@ __global__ void rms_norm_kernel(unsigned short* __restrict__ out,
 // us -> 5.4, 4068 rows 27 + 15 -> 34 (5.3 TB/s).
 // pick (or null): row t is the norm of row pick[t] of N, the result goes to `out`
 // and the sum nowhere: the last norm, of the rows whose logits are asked for. That
-// saves the gather behind it (4.7 us).
+// saves the gather behind it (4.7 us). Picks out of range, which the caller
+// refuses, are clamped.
 enum NormFrom { ROWS, PARTS, CHOSEN };
 
 template <int FROM>

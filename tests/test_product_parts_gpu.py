@@ -186,6 +186,7 @@ def test_embedding_under_the_first_norm(T, H):
     ref = torch.empty_like(x)
     ops.rms_norm(ref, embed[ids], w, 1e-5)
     assert torch.equal(x, embed[ids]) and torch.equal(h, ref)
+    # callers refuse such ids (test_refused_ids.py); the kernel stays in bounds
     bad = ids.clone()
     bad[-1] = 50
     x, h = ops.embed_rms_norm(bad, embed, w, 1e-5)
