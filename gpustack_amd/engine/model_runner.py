@@ -591,7 +591,8 @@ class ModelRunner:
             if any(s.state_slot < 0 for s in batch.seqs):
                 raise RuntimeError("a scheduled sequence holds no state slot")
             parts.append((np.asarray(
-                [starts, news, [s.state_slot for s in batch.seqs]]), i32))
+                [starts, news, [s.state_slot for s in batch.seqs]],
+                dtype=np.int32), i32))
         up = ops.to_device(parts, dev)
         rg = RaggedMeta(
             block_tables=up[0], row_seq=up[1], pos32=up[2], prev_tokens=up[3],

@@ -62,10 +62,13 @@ def to_device(parts, device) -> list[torch.Tensor]:
 
     import numpy as np
 
+    kinds = {torch.int32: ("i", np.int32), torch.int64: ("q", np.int64)}
     host = []
     for v, dtype in parts:
-        if isinstance(v, list) and v and isinstance(v[0], int):
-            v = np.frombuffer(array.array("q", v), dtype=np.int64)
+        if isinstance(v, list) and v and isinstance(v[0], int) \
+                and dtype in kinds:
+            # refuses what the type does not hold, as torch.tensor does
+            v = np.frombuffer(array.array(kinds[dtype][0], v), kinds[dtype][1])
         host.append(torch.as_tensor(v, dtype=dtype))
     device = torch.device(device)
     if device.type != "cuda":

@@ -26,6 +26,18 @@ def test_values_and_types(device, n):
                for g, w in zip(got, want))
 
 
+@pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("value", [2 ** 31, -2 ** 31 - 1, 2 ** 40])
+def test_values_that_a_type_does_not_hold(device, value):
+    """Refused, as torch.tensor refuses them, not wrapped."""
+    with pytest.raises(RuntimeError):
+        torch.tensor([3, value], dtype=torch.int32)
+    with pytest.raises((RuntimeError, OverflowError)):
+        ops.to_device([([3, value], torch.int32)], device)
+    ends = [2 ** 31 - 1, -2 ** 31]
+    assert ops.to_device([(ends, torch.int32)], device)[0].tolist() == ends
+
+
 @pytest.mark.gpu
 @pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")
 def test_copies_queued_behind_work_keep_their_values():
