@@ -124,7 +124,10 @@ __global__ __launch_bounds__(THREADS) void fused_add_rms_norm_kernel(unsigned sh
                                           int parts, float eps, int T, int N,
                                           int H) {
   const int nvec = H / 8;
-  const bool cached = nvec <= THREADS * NORM_MAX_VEC;
+  // Rows of more than 8192 read the rounded sum back, with 512 threads too, which
+  // could hold it: else a row's rounding would depend on the rows beside it.
+  const bool cached = nvec <= NORM_THREADS * NORM_MAX_VEC;
+  constexpr int SLOTS = NORM_THREADS * NORM_MAX_VEC / THREADS;
   for (int row = blockIdx.x; row < T; row += gridDim.x) {
     long src = row;
     if (pick != nullptr) {
@@ -134,7 +137,7 @@ __global__ __launch_bounds__(THREADS) void fused_add_rms_norm_kernel(unsigned sh
     }
     unsigned short* op = out + (long)row * H;
     unsigned short* rp = residual + src * H;
-    float vals[NORM_MAX_VEC][8];
+    float vals[SLOTS][8];
     float ss = 0.f;
     for (int v = threadIdx.x, slot = 0; v < nvec; v += THREADS, ++slot) {
       u16x8 ur = *reinterpret_cast<const u16x8*>(rp + v * 8);
@@ -147,7 +150,7 @@ __global__ __launch_bounds__(THREADS) void fused_add_rms_norm_kernel(unsigned sh
       }
       if (pick == nullptr)
         *reinterpret_cast<u16x8*>(rp + v * 8) = f32_to_bf8(f);
-      if (cached && slot < NORM_MAX_VEC) {
+      if (cached && slot < SLOTS) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) vals[slot][i] = f[i];
       }
@@ -162,7 +165,7 @@ __global__ __launch_bounds__(THREADS) void fused_add_rms_norm_kernel(unsigned sh
     const float inv = rsqrtf(tot / H + eps);
     for (int v = threadIdx.x, slot = 0; v < nvec; v += THREADS, ++slot) {
       float f[8];
-      if (cached && slot < NORM_MAX_VEC) {
+      if (cached && slot < SLOTS) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) f[i] = vals[slot][i];
       } else {
