@@ -83,12 +83,15 @@ DEVICE_INLINE unsigned int pack_hi(float lo, float hi) {
 // A value and the one of the lane 16 or 32 away, in either order, without the
 // LDS: as shuffles these exchanges, most of them in the sums at the end, were
 // 12 % of the kernel over 240 shapes (16 heads of 256, us: 512 x 40 keys
-// 53.6 -> 42.0, one x 300 12.2 -> 11.1; 32 of 128: 64 x 400 21.0 -> 19.2).
+// 53.6 -> 42.0, one x 300 12.2 -> 11.1; 32 of 128: 64 x 400 21.0 -> 19.2). The two
+// operands are kept apart, as in half_wave_max.
 template <int M>
 DEVICE_INLINE f32x2 with_lane(float v) {
-  const unsigned int u = __builtin_bit_cast(unsigned int, v);
-  const auto r = M == 16 ? __builtin_amdgcn_permlane16_swap(u, u, false, false)
-                         : __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  const unsigned int a = __builtin_bit_cast(unsigned int, v);
+  unsigned int b = a;
+  asm("" : "+v"(b));
+  const auto r = M == 16 ? __builtin_amdgcn_permlane16_swap(a, b, false, false)
+                         : __builtin_amdgcn_permlane32_swap(a, b, false, false);
   const unsigned int x = r[0], y = r[1];
   return f32x2{__builtin_bit_cast(float, x), __builtin_bit_cast(float, y)};
 }
