@@ -149,22 +149,27 @@ __device__ __forceinline__ float group16_reduce_sum(float x) {
 // Loads from memory straight to LDS address `to` + 16 * lane, 16 bytes a lane,
 // from base + off bytes or from `at`; addresses are multiples of 16. Inline asm,
 // because the compiler puts a wait for all such loads of its builtin in front of
-// LDS reads that it cannot tell from them. They write no register; the kernel
-// waits for them itself (s_waitcnt vmcnt, then its barrier).
+// LDS reads that it cannot tell from them. They write no register but m0, which
+// the compiler is told; the kernel waits for them itself (s_waitcnt vmcnt, then its
+// barrier).
 DEVICE_INLINE unsigned int lds_address(const unsigned short* p) {
   return (unsigned int)(unsigned long)(
       const __attribute__((address_space(3))) unsigned short*)p;
 }
+// (m0 is reserved, which clang warns about where it is named as written to.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 DEVICE_INLINE void load_to_lds(const unsigned short* base, unsigned int off,
                                const unsigned short* to) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               ::"s"(lds_address(to)), "v"(off), "s"(base) : "memory");
+               ::"s"(lds_address(to)), "v"(off), "s"(base) : "m0", "memory");
 }
 DEVICE_INLINE void load_to_lds(const unsigned short* at,
                                const unsigned short* to) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-               ::"s"(lds_address(to)), "v"(at) : "memory");
+               ::"s"(lds_address(to)), "v"(at) : "m0", "memory");
 }
+#pragma clang diagnostic pop
 
 #define HIP_CHECK_KERNEL()                                        \
   do {                                                            \
