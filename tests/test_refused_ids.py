@@ -54,6 +54,23 @@ def test_ids_outside_the_vocabulary(device, bad, prefill):
     assert eng.runner.forward_logits(_batch(eng, [0, V - 1])).shape[-1] == V
 
 
+def test_long_lists_and_arrays_of_ids():
+    import numpy as np
+
+    run = _engine().runner
+    V = run.cfg.spec.vocab_size
+    for n in (0, 1, 512, 513, 5000):
+        ids = [i % V for i in range(n)]
+        for form in (ids, np.asarray(ids, dtype=np.int64)):
+            assert list(run.in_vocab(form)) == ids
+        for bad in (-1, V):
+            for at in {0, n // 2, n - 1} if n else ():
+                wrong = ids[:at] + [bad] + ids[at + 1:]
+                for form in (wrong, np.asarray(wrong)):
+                    with pytest.raises(IndexError):
+                        run.in_vocab(form)
+
+
 def test_a_captured_step_refuses_them():
     eng = _engine()
     graphs = DecodeGraphRunner(eng.runner)
