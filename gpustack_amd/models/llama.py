@@ -259,9 +259,10 @@ def _gate_up_silu(x, w, pack: "W4Pack | None"):
     else None."""
     if pack is None:
         return ops.linear_silu(x, w)
-    if not _w4_takes(x, pack):
+    hip = ops._load_hip() if _w4_takes(x, pack) else None
+    if hip is None or not hip.w4_silu_wins(x.shape[0], *pack.shape):
         return None
-    return ops._load_hip().w4_silu(x.contiguous(), pack.qw, pack.sc, pack.zs)
+    return hip.w4_silu(x.contiguous(), pack.qw, pack.sc, pack.zs)
 
 
 class Attention(nn.Module):

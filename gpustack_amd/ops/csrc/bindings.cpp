@@ -36,6 +36,7 @@ void rows_gemm_launch(void*, const void*, const void*, int, int, int, long, int*
 bool w4_has(int, int);
 bool w4_cuts(int, int, int);
 bool w4_by_rows(int, int, int);
+bool w4_silu_wins(int, int, int);
 int w4_splits(int, int, int);
 void w4_parts_launch(float*, const void*, const void*, const void*, const void*, int, int, int, int, hipStream_t);
 void w4_silu_launch(void*, const void*, const void*, const void*, const void*, int, int, int, hipStream_t);
@@ -706,14 +707,13 @@ c10::optional<at::Tensor> w4_parts(at::Tensor x, at::Tensor qw, at::Tensor sc,
 }
 
 // silu(gate) * up of the product, qw holding the gate's rows and behind them the
-// up product's; none where the activation is a launch of its own: a product that
-// is not cut over k takes 18 us for 4096 k however narrow it is (28672 columns at
-// 16 rows 22 against 23 and 2.5 for the activation, at 22016 20 / 18 + 2.5)
+// up product's; none where there is no such form (w4_silu_wins says where it is the
+// faster one)
 c10::optional<at::Tensor> w4_silu(at::Tensor x, at::Tensor qw, at::Tensor sc,
                                   at::Tensor zs) {
   check_w4(x, qw, sc, zs);
   const int M = x.size(0), K = x.size(1), N = qw.size(0);
-  if (!w4_has(N, K) || N % 128 != 0 || N < 22016 || !at_16(x) || !at_16(qw))
+  if (!w4_has(N, K) || N % 128 != 0 || !at_16(x) || !at_16(qw))
     return c10::nullopt;
   at::Tensor out = at::empty({M, N / 2}, x.options());
   w4_silu_launch(out.data_ptr(), x.data_ptr(), qw.data_ptr(), sc.data_ptr(),
@@ -832,6 +832,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "fp32 parts of a W4A16 product that is cut over k, or None");
   m.def("w4_silu", &w4_silu,
         "silu(gate) * up of a W4A16 product, or None");
+  m.def("w4_silu_wins",
+        [](long M, long N, long K) { return w4_silu_wins(M, N, K); },
+        "whether that beats the product and an activation behind it");
   m.def("w4_dequant", &w4_dequant,
         "packed-int4 -> bf16 weight expansion (prefill transient)");
 }

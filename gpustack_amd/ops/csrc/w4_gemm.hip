@@ -496,6 +496,24 @@ bool w4_by_rows(int M, int N, int K) {
   return M <= 64 && (long)N * K <= 12l << 20;
 }
 
+// Whether a product of N columns (gate and up) ends in the activation. Where the
+// product is one launch of whole tiles by itself it does, and saves the
+// activation's launch (us without / with, 28672 x 4096 at 17 rows 28 / 26, 64 rows
+// 36 / 34, 192 rows 97 / 95; 17920 x 2048 at 64 rows 21 / 18). Products cut over k
+// do not: their chain of k would run whole on less than one workgroup a CU (16384 x
+// 4096 at 64 rows 27 / 33, 22016 x 8192 at 16 rows 36 / 43).
+// In the place of the rows' form, up to 16 rows, the tiles pay for a chain of a
+// microsecond for every 256 k, however few rows there are, and the rows' form for
+// its columns and for x, which it reads again in every workgroup: the line grows
+// with both (22016 x 2048 at one row 12.5 / 12.7, x 4096 18.6 / 23.1, at 12 rows 22.1
+// / 21.8, at 16 24.3 / 22.4; 28672 x 3072 at one row 20.1 / 19.5, x 4096 24.2 / 24.8,
+// at 8 rows 24.7 / 24.0; 24576 x 3072 at 4 rows, right on it, 16.8 / 17.9).
+bool w4_silu_wins(int M, int N, int K) {
+  if (w4_by_rows(M, N, K))
+    return M <= 16 && N > 16384 && K <= 256 * (M + 4) + (N - 16384) / 8;
+  return w4_splits(M, N, K) == 1;
+}
+
 // parts: fp32 [splits, M, N]. x, qw and parts at 16-byte addresses.
 void w4_parts_launch(float* parts, const void* x, const void* qw, const void* sc,
                      const void* zs, int M, int N, int K, int splits,

@@ -77,6 +77,36 @@ def test_product_ends_in_the_activation(M, N, K):
     assert bool(((act.double() - ref).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("M,N,K,wins", [
+    (17, 16640, 4096, True), (192, 22016, 12288, True),   # whole tiles anyway
+    (1, 32768, 4096, True), (1, 32768, 8192, False),      # cut from 8192 k on
+    (64, 16384, 4096, False), (16, 22016, 8192, False),   # cut over k
+    (1, 22016, 4096, False), (2, 28672, 4096, False),     # the rows' form
+    (16, 22016, 4096, True), (8, 28672, 4096, True), (1, 28672, 2048, True),
+    (1, 8192, 128, False)])
+def test_where_it_ends_in_the_activation(monkeypatch, M, N, K, wins):
+    """The route, and both ways the same result up to the rounding of the
+    product that the activation reads."""
+    from gpustack_amd import ops
+    from gpustack_amd.models.llama import W4Pack, _gate_up_silu, qlinear
+
+    assert _hip().w4_silu_wins(M, N, K) == wins
+    if N * K > 1 << 27:
+        return                             # the two forms have tests above
+    x, (qw, s, z), _, _ = _case(M, N, K, 1 / 16)
+    pack = W4Pack(qw, s, z)
+    got = _gate_up_silu(x, None, pack)
+    assert (got is not None) == wins
+    if not wins:
+        return
+    want = torch.empty(M, N // 2, device="cuda", dtype=torch.bfloat16)
+    ops.silu_and_mul(want, qlinear(x, None, pack))
+    # gate and up rounded to bf16 here and not there, the result in both; silu's
+    # slope is under 1.1
+    assert float((got.double() - want.double()).norm()
+                 / want.double().norm()) < 3 * 2.0 ** -8
+
+
 def test_none_where_there_is_no_such_form():
     x, (qw, s, z), _, _ = _case(4, 192, 256)
     assert _hip().w4_silu(x, qw, s, z) is None
