@@ -544,30 +544,33 @@ def _rows_tile_plan(M: int, N: int, K: int):
 
 def _tall_tile_plan(M: int, N: int, K: int):
     """_rows_tile_plan for 129 to 512 rows: long rows of up to 10240 columns,
-    which leave the library's tiles few and its chip idle. Cut over k into up
-    to 8 parts, as many as two workgroups a CU take (4096x14336 at 256 rows:
-    four parts 45 without their join, eight 39). us against the library, with
-    the join, weights out of HBM:
-    160 rows: 4096x14336 44 / 82, 10240x9216 64 / 73, 1024x14336 21 / 33,
-    5120x5120 27 / 37; 256 rows: 4096x14336 49 / 60, 6144x12288 61 / 109,
-    8192x7168 51 / 68, 3072x6144 26 / 29, but 2560x6144 at 136 rows 22 / 20
-    and 8192x4096 at 176 34 / 28; 384 rows: 5120x14336 72 / 87, 2048x11008
-    34 / 46, but 4096x9216 55 / 51 and 6144x11008 88 / 90; 512 rows:
-    4096x14336 72 / 88, 4096x6144 38 / 44, but 5120x11008 95 / 93."""
+    which leave the library's tiles few and its chip idle; more row tiles leave
+    it less so, and the lines come down with their number. Cut over k into as
+    many parts as two workgroups a CU take, at most 8 (4096x14336 at 256 rows:
+    four parts 45 without their join, eight 39), and into 5 or 7 nowhere: the 8
+    XCDs take workgroups in turn, so that an odd number of parts brings all of x
+    to each of their L2s, an even one half of it or less (176 rows of 4608x9216
+    in 7 parts 48, in 6 37; 240 of 5632x11008 in 5 78, in 4 54; 384 of
+    4096x11008 66, 54; but 136 of 6144x8192 39, 43). us against the library,
+    with the join, weights out of HBM:
+    160 rows: 4096x14336 42 / 82, 4608x9216 36 / 57, 5120x5120 26 / 36; 176
+    rows: 4608x9216 37 / 41, 2560x6144 22.4 / 22.5, 8192x5120 36 / 34 (x4096 34 /
+    28); 256 rows: 4096x14336 48 / 61, 6144x12288 63 / 110, 1032x6144 17 / 22,
+    2048x6144 20 / 23, but 10240x10240 100 / 89; 384 rows: 5120x14336 71 / 88,
+    4096x11008 54 / 63, 2560x6144 27 / 28; 512 rows: 4096x14336 71 / 82,
+    4096x6144 38 / 43, 3072x7168 40 / 42, but 5120x11008 97 / 93. The library is
+    uneven in M: between 4608 and 5120 columns it is up to a tenth the faster one
+    at 136 to 152 and at 168 to 184 rows (184 rows of 4864x8192 43 / 36), and half
+    as fast as the tiles at 160 and from 192 on (192 of 5120x8192 .62)."""
     rows = -(-M // 128)
-    if rows == 2:
-        wins = N <= 10240 and K >= (
-            7168 if 1024 < N < 3072 else 6144 if N < 3072 else 5120)
-    elif rows == 3:
-        wins = N <= 5120 and K >= (11008 if 2048 < N <= 4096 else 6144)
-    else:
-        wins = N <= 4096 and K >= 6144
-    if not wins:
+    if N > (10240, 5120, 4096)[rows - 2] \
+            or K < (5120 if rows == 2 and N >= 3072 else 6144):
         return None
     t128 = rows * -(-N // 128)
     if t128 < 32:
         return 64, 8
-    return 128, min(8, 512 // t128)
+    parts = min(8, 512 // t128)
+    return 128, parts - parts % 2 if parts > 4 else parts
 
 
 def _parts_plan(M: int, N: int, K: int):
