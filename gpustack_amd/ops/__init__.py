@@ -577,46 +577,53 @@ def _parts_plan(M: int, N: int, K: int):
     """(columns of a tile, parts of K) of a small product whose consumer adds
     the parts up, where that beats the product of _rows_tile_plan, the library
     or the decode product, else None: short rows leave whole tiles few and
-    their chain long. us with an RMS norm behind, 64 rows (24 rows; 16 rows):
-    2048x2048 9.4 against 14.9 (8.2 / 14.1; 8.0 / 9.2), 1536x1024 7.7 / 11.5
-    (7.0 / 11.2; 6.9 / 7.0), 4096x2048 13.0 / 16.3 (12.0 / 15.7; 11.6 / 11.1),
-    4096x3072 14.3 / 20.1 (12.6 / 15.3; 12.2 / 12.9), 6144x3072 18.8 / 23.4
-    (16.4 / 18.1; 16.0 / 17.5), 6144x2048 at 16 rows 13.7 / 16.0 but at 24
-    rows 13.9 / 13.7; 128 rows: 2048x2048 12.2 / 14.4, 4096x1024 14.3 / 16.7.
-    At one row 2048x3072 8.6 / 9.6, 2048x2048 7.7 / 7.7.
-    Up to 16 rows also longer ones, at one / 16 rows: 2048x5120 10 / 10 against
-    21 / 13, 4096x5120 15 / 16 against 24 / 23, 1024x8192 10 / 10 against 15 /
-    15, 6144x4096 19 / 19 against 21 / 20 (in four parts 22 / 23 at 7168x4096, in
-    three 21 / 21), 4096x4096 13.4 / 13.7 against 13.6 / 15.0, but 4096x8192
-    20.3 / 20.6 against 20.7 / 20.8; and 8192x3072 19 / 19 against 26 / 24, at
-    64 rows 22 / 25, 7168x10240 there 41 / 49."""
+    their chain long. us with an RMS norm behind, parts against the best of the
+    others.
+    Up to 16 rows, against the decode product (which wants k in 128s, and whose
+    workgroups of 16 columns fill the chip from 2049 to 4096 of these) from 3072
+    k there and from 2048 k elsewhere: at one row 2048x2048 7.7 / 7.8, 2048x3072
+    8.6 / 9.6, 4608x2048 10.8 / 11.8, but 4096x3072 11.2 / 10.9; at 16 rows 8.1 /
+    9.3, -, 11.4 / 14.3, 11.5 / 12.2; 4096x2048 at 8 rows 10.4 / 9.7. Where only
+    the library is beside it, at any k: 3072x1088 at 8 rows 8.1 / 12.5, 2048x5120
+    at one 11 / 21, 4096x5120 14 / 23, 1024x8192 10 / 15, 6144x4096 17 / 20,
+    4096x8192 19.4 / 20.8, 8192x3072 at 16 rows 17 / 24, and about even on 5632
+    to 7168 columns of 8192 k (28 / 29 at one row, 31 / 30 at 16).
+    More rows: up to 4096 columns at any k, beyond from where whole tiles of 32
+    columns stop (2048 k): 24 rows of 2048x2048 8.2 / 14.0, 3072x1024 8.3 / 8.6,
+    6144x2112 13.4 / 19.5, but 6144x2048 12.9 / 12.5; 64 rows of 3072x1024 9.6 /
+    9.9, x1088 9.7 / 14.9, 4096x2048 12.2 / 15.9, but 4608x1024 12.2 / 10.8; 128
+    rows of 2048x2048 12.3 / 14.5. Above 64 rows _rows_tile_plan cuts rows from
+    3072 k on itself, from as many columns (128 rows of 2560x3072 16 / 24), and
+    up to 64 rows those from 4096 k on, up to 6144 columns (64 rows of 7168x10240
+    38 / 49)."""
     if not 0 < M <= 128 or K % 64 != 0 or N % 8 != 0 or min(N, K) < 1024 \
-            or N > 8192:
-        return None
-    # four cuts of rows a multiple of 8 KB apart meet on a few memory channels
-    wide = 128, 3 if K % 4096 == 0 else 4
-    if N > 6144:
-        return wide if M <= 64 and 3072 <= K < 11008 else None
-    if M <= 16 and 4096 <= K < 11008:
-        if N > 5120:
-            return wide
-        if K % 8192 == 0 and 2048 < N <= 4096:
-            return None
-        cols = 32 if N <= 2048 else 64
-        return cols, min(8 if cols == 32 else 4, 256 // -(-N // cols))
-    if K >= 4096:
+            or N > 8192 or K >= 11008:
         return None
     if M <= 16:
-        wins = (N <= 2048 or N >= 5120) and (
-            K >= 3072 or K >= 2048 and M >= 8)
-    elif N <= 4096:
-        wins = M > 64 and K < 3072 or M <= 64 and not (N >= 2560 and K == 1024) \
-            or N < 2048
+        wins = K >= (3072 if 2048 < N <= 4096 else 2048) \
+            or not _rows_gemm_wins(M, N, K)
+    elif K >= 4096:
+        wins = N > 6144 and M <= 64
+    elif M > 64 and K >= 3072:
+        wins = N < 3072
     else:
-        wins = K >= 3072 and M <= 64
+        wins = N <= 4096 or K > 2048
     if not wins:
         return None
-    return (32 if N <= 2048 else 64 if N <= 4096 else 128), 4
+    if M <= 16 and K >= 4096 and N <= 5120:
+        # long rows: as many parts as leave one workgroup a CU. Cuts of 4 KB
+        # meet on few memory channels, the more workgroups the more (3 / 4
+        # parts at 8192 k: 4096 columns .91, 3840 .96, 3584 1.03, 3072 1.13)
+        if N <= 2048:
+            return 32, min(8, 256 // -(-N // 32))
+        if K % 8192 == 0 and N > 3584:
+            return 64, 3
+        return 64, min(4, 256 // -(-N // 64))
+    if N <= 4096:
+        return 32 if N <= 2048 else 64, 4
+    # the same for four cuts of rows a multiple of 8 KB apart (8192 columns: .88
+    # at 4096 k, .77 at 8192, but 1.02 at 4032 and 1.0 at 8320)
+    return 128, 3 if K % 4096 == 0 else 4
 
 
 def router_plan(T: int, E: int, H: int):

@@ -161,7 +161,10 @@ def test_tall_products_in_parts(M, N, K):
                                    (65, 4096, 1024), (128, 3072, 2048),
                                    (33, 6136, 3136), (16, 5120, 2048),
                                    (16, 1160, 4160), (2, 6144, 4096),
-                                   (64, 8192, 8192), (5, 5000, 10240)])
+                                   (64, 8192, 8192), (5, 5000, 10240),
+                                   (3, 3072, 1088), (1, 2304, 8192),
+                                   (16, 3600, 8192), (24, 6144, 2112),
+                                   (96, 2560, 3072), (128, 8192, 2112)])
 def test_small_products_in_parts(M, N, K):
     plan = ops._parts_plan(M, N, K)
     assert plan is not None

@@ -23,3 +23,27 @@ def test_tall_products_from_some_length_and_up_to_some_width(M, K):
     changes = sum(a != b for a, b in zip(cut, cut[1:]))
     # at 5120 k two row tiles want 3072 columns besides
     assert changes <= (2 if K < 6144 else 1), changes
+
+
+@pytest.mark.parametrize("M", [1, 8, 16])
+@pytest.mark.parametrize("N", [1024, 2048, 2304, 3072, 4096, 4104, 5120, 6144,
+                               8192])
+def test_parts_of_long_rows_at_every_length(M, N):
+    """From 4096 k to where the whole product is cut anyway."""
+    for K in range(4096, 11008, 64):
+        plan = ops._parts_plan(M, N, K)
+        assert plan is not None, K
+        assert 1 < plan[1] <= 8 and plan[1] <= K // 64
+        assert plan[1] * -(-N // plan[0]) <= 256
+
+
+@pytest.mark.parametrize("M", [1, 8, 16, 17, 24, 64, 65, 128])
+def test_parts_of_short_rows_at_every_width(M):
+    """Products that only the library is beside are cut up to 4096 columns; with
+    the decode product, from one length of rows on."""
+    for N in range(1024, 4097, 8):
+        for K in (1088, 1984, 2624):
+            assert ops._parts_plan(M, N, K) is not None, (N, K)
+        for K in range(1024, 4096, 128):
+            if M > 16 and (M <= 64 or K < 3072) or M <= 16 and K >= 3072:
+                assert ops._parts_plan(M, N, K) is not None, (N, K)
