@@ -506,11 +506,13 @@ bool w4_by_rows(int M, int N, int K) {
 // microsecond for every 256 k, however few rows there are, and the rows' form for
 // its columns and for x, which it reads again in every workgroup: the line grows
 // with both (22016 x 2048 at one row 12.5 / 12.7, x 4096 18.6 / 23.1, at 12 rows 22.1
-// / 21.8, at 16 24.3 / 22.4; 28672 x 3072 at one row 20.1 / 19.5, x 4096 24.2 / 24.8,
-// at 8 rows 24.7 / 24.0; 24576 x 3072 at 4 rows, right on it, 16.8 / 17.9).
+// / 21.8, at 16 24.3 / 22.4; 28672 x 4096 at one row 24.2 / 24.8, at 8 rows 24.7 /
+// 24.0; 24576 x 4096 at 2 rows, right on it, 19.5 / 23.2). It lies where the tiles
+// take 1.5 us more in these loops: in a captured step the activation costs that
+// much besides (a step of 4 layers at one row 372 / 368, at 4 rows 380 / 371).
 bool w4_silu_wins(int M, int N, int K) {
   if (w4_by_rows(M, N, K))
-    return M <= 16 && N > 16384 && K <= 256 * (M + 4) + (N - 16384) / 8;
+    return M <= 16 && N > 16384 && K < 256 * (M + 6) + (N - 16384) / 4;
   return w4_splits(M, N, K) == 1;
 }
 
