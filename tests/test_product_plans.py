@@ -25,6 +25,19 @@ def test_tall_products_from_some_length_and_up_to_some_width(M, K):
     assert changes <= (2 if K < 6144 else 1), changes
 
 
+@pytest.mark.parametrize("M", [1, 8, 16, 17, 64, 65, 128])
+def test_tiles_that_end_in_the_activation(M):
+    """Uncut tiles of 64 or 128 columns do; of 64 not where two runs of 32 rows
+    meet on the memory channels."""
+    for N in range(8192, 65537, 256):
+        for K in (2048, 4096, 6144, 8192):
+            plan = ops._rows_tile_plan(M, N, K)
+            whole = plan is not None and plan[1] == 1 and plan[0] >= 64
+            meet = whole and plan[0] == 64 and K == 4096
+            assert ops._silu_plan(M, N, K) == (
+                plan if whole and not meet else None)
+
+
 @pytest.mark.parametrize("M", [1, 8, 16])
 @pytest.mark.parametrize("N", [1024, 2048, 2304, 3072, 4096, 4104, 5120, 6144,
                                8192])
