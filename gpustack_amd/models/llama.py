@@ -215,8 +215,9 @@ def qlinear(x, w, pack: "W4Pack | None", bias=None, parts: bool = False):
     and run the library GEMM at full MFMA rate. Measured, us, 64 rows:
     28672x4096 33 against 105, 4096x14336 18 / 62, 128256x4096 134 / 584; 192
     rows: 28672x4096 93 / 133, 4096x14336 48 / 104, 4096x4096 20 / 43; 256 rows
-    121 / 135, 63 / 74 and 25 / 34, but 10240x8192 reaches the expansion.
-    GPUSTACK_AMD_W4_KERNEL=1 keeps the packed product up to 1024 rows."""
+    121 / 135, 63 / 74 and 25 / 34, but 10240x8192 reaches the expansion; above
+    128 rows a few columns more than two workgroups a CU take expand as well
+    (_w4_takes). GPUSTACK_AMD_W4_KERNEL=1 keeps the packed product up to 1024 rows."""
     if pack is None:
         return ops.linear_auto(x, w, parts) if bias is None \
             else F.linear(x, w, bias)
@@ -245,13 +246,21 @@ def qlinear(x, w, pack: "W4Pack | None", bias=None, parts: bool = False):
 
 def _w4_takes(x, pack: "W4Pack") -> bool:
     """True where the packed product takes x: rows up to its limit, whole
-    workgroups of 64 columns, scales that fit the LDS."""
+    workgroups of 64 columns, scales that fit the LDS. Above 128 rows, three
+    tiles of rows, some widths leave a last round of a few workgroups behind the
+    512 that two a CU make; up to 4096 k the expansion is the faster one there
+    (us, own / expansion, 160 rows: 22016x4096 93 / 81, x3072 70 / 64, 23552x4096
+    93 / 89, but x2048 49 / 50, x5120 118 / 119, 24576x4096 94 / 93 and, below
+    them, 21760x4096 71 / 82)."""
     import os
 
-    most = 1024 if os.environ.get("GPUSTACK_AMD_W4_KERNEL", "0") == "1" \
-        else 192
-    return (x.is_cuda and x.dim() == 2 and 0 < x.shape[0] <= most
-            and pack.shape[0] % 64 == 0 and pack.shape[1] <= 131072)
+    always = os.environ.get("GPUSTACK_AMD_W4_KERNEL", "0") == "1"
+    M, (N, K) = x.shape[0], pack.shape
+    if 128 < M and not always and K <= 4096 and N % 128 == 0 \
+            and 512 < 3 * (N // 128) <= 552:
+        return False
+    return (x.is_cuda and x.dim() == 2 and 0 < M <= (1024 if always else 192)
+            and N % 64 == 0 and K <= 131072)
 
 
 def _gate_up_silu(x, w, pack: "W4Pack | None"):
