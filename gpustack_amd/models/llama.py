@@ -1038,13 +1038,15 @@ class MoEMLP(nn.Module):
         """Long prompts of few large experts: the library's product of one
         expert at a time (1100 to 1300 TFLOP/s) makes up for a loop that syncs
         with the host and gathers the rows (about 130 us an expert) against
-        the tiles' 830. us of the layer, tiles against loop, at 4096 x 14336
-        and two experts a row: 8 experts 4096 rows 3630 / 3900, 6144 rows
-        5320 / 5160, 8192 rows 6980 / 6200, 16384 rows 14900 / 11700; 16
-        experts 12288 rows 10570 / 11070, 16384 rows 13860 / 12100; 8 of
-        4096 x 7168 12288 rows 5280 / 5460, 16384 rows 7160 / 5930. The line
-        is one number of multiplications an expert in all of them. A capture
-        cannot record the syncs."""
+        the tiles' 850. us of the layer, tiles against loop, at 4096 x 14336
+        and two experts a row: 8 experts 4096 rows 3330 / 3790, 6656 rows
+        5650 / 5740, 7168 rows 6190 / 5670, 8192 rows 7170 / 6340, 16384 rows
+        15250 / 11210; 16 experts 12288 rows 10580 / 10990, 13632 rows 11960 /
+        11000; 8 of 4096 x 7168 8192 rows 3400 / 3570, 12288 rows 5560 / 5300,
+        16384 rows 7870 / 5590; 4 of 2048 x 8192 8192 rows 2060 / 2250, 11900
+        rows 2890 / 2740. The line is one number of multiplications an expert
+        in all of them (6812, 13624, 13624 and 11921 rows). A capture cannot
+        record the syncs."""
         return (T * self.top_k * self.i * self.spec.hidden_size
                 >= 100_000_000_000 * self.e
                 and not torch.cuda.is_current_stream_capturing())

@@ -802,8 +802,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm8", &gemm8, "8-phase pipelined 256x256 GEMM (bf16, f32 accum)");
   m.def("gemm_lab", &gemm_lab, "GEMM schedule lab variants (A/B vs hipBLASLt)");
   m.def("rows_tile_parts", &rows_tile_parts,
-        "fp32 parts over k of a product of up to 128 rows");
-  m.def("rows_tile", &rows_tile, "bf16 product of up to 128 rows in tiles",
+        "fp32 parts over k of a bf16 product of any number of rows");
+  m.def("rows_tile", &rows_tile,
+        "bf16 product in tiles: up to 128 rows, more where it is cut over k",
         py::arg("out"), py::arg("x"), py::arg("w"), py::arg("cols"),
         py::arg("splits"), py::arg("silu") = false);
   m.def("rows_gemm", &rows_gemm, "bf16 product of up to 16 rows");

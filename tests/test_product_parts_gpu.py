@@ -92,12 +92,19 @@ def test_add_layer_norm(T, W, add, out):
 
 
 @pytest.mark.parametrize("M", [1, 17, 48, 128])
-@pytest.mark.parametrize("N,K", [(4096, 14336), (4096, 4096), (2048, 8192)])
+@pytest.mark.parametrize("N,K", [(4096, 14336), (4096, 4096), (2048, 8192),
+                                 (1024, 1024), (16384, 2048)])
 def test_products_come_in_parts(M, N, K):
     rnd = _gen(M)
     x, w = rnd(M, K).bfloat16(), (rnd(N, K) * K ** -0.5).bfloat16()
     got = ops.linear_auto(x, w, parts=True)
-    if got.dim() == 3:
+    # parts exactly where the plan cuts the product: of its own for consumers of
+    # parts, or the product's
+    plan = ops._parts_plan(M, N, K) or ops._rows_tile_plan(M, N, K)
+    if plan is None or plan[1] == 1:
+        assert got.shape == (M, N) and got.dtype == torch.bfloat16
+    else:
+        assert got.shape == (plan[1], M, N) and got.dtype == torch.float32
         got = _joined(got)
     if ops._parts_plan(M, N, K) is None:
         assert torch.equal(got, ops.linear_auto(x, w))
@@ -210,14 +217,14 @@ def test_the_last_norm_of_picked_rows(n, T, H):
     assert torch.equal(got, x[rows])
 
 
-@pytest.mark.parametrize("kind", ["parts", "bf16", "fp32"])
-@pytest.mark.parametrize("T,W", [(1, 64), (17, 2048), (9, 8192), (5, 100)])
+@pytest.mark.parametrize("kind,T,W", [
+    (kind, T, W) for kind in ("parts", "bf16", "fp32")
+    for T, W in ((1, 64), (17, 2048), (9, 8192), (5, 100))
+    if kind != "parts" or W % 8 == 0])     # products give other rows whole
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_the_last_layer_norm_of_picked_rows(kind, T, W, dtype):
     rnd = _gen(T + W)
     x, w, b = rnd(T, W), rnd(W), rnd(W)
-    if kind == "parts" and W % 8:
-        return                         # products give such rows whole
     a = rnd(3, T, W) if kind == "parts" else rnd(T, W)
     if kind == "bf16":
         a = a.bfloat16()
