@@ -1071,18 +1071,21 @@ PROMPT_PORTION = 32
 
 
 def prompt_kernel_wins(seq_news, max_ctx: int, heads: int, window: int) -> bool:
-    """Where the prompt kernel is the faster one: tiles of 16 rows cut a long
-    walk over the keys into parts, so they keep long histories of few rows.
-    us, 16-row tiles / prompt kernel, 16 heads on 4 unless said, slopes: one
-    whole prompt of 32 rows 7.6 / 5.7, 100 9.8 / 10.1, 200 14 / 12.5, six of
-    301 to 1900 in a window of 1024 240 / 85; 16 x 100 behind 100 37 / 16; in
-    a window of 1024 64 rows behind 3000 18 / 40, 200 27 / 45; 8 x 16 behind
-    2000, 32 heads on 8 (256 tiles) 41 / 40, 8 x 32 (512) 57 / 41, 8 x 200
-    207 / 64; without a window 200 behind 3001 (208 tiles) 59 / 97. Both grow
-    with the walk, so the line is the number of 16-row tiles."""
+    """Where the prompt kernel is the faster one. Tiles of 16 rows are many
+    workgroups that may cut a long walk over the keys into parts, tiles of 128
+    few that read every key once, so the line is the number of 16-row tiles, two
+    workgroups a CU, and a quarter more where the walk is long; a whole prompt
+    of up to 64 rows is one tile either way. us, 16-row tiles / prompt kernel, 16
+    heads on 4 unless said: one whole prompt of 64 rows 8.7 / 8.8, two of 32 in 64
+    heads 8.7 / 7.1, 100 10.2 / 11.6, 300 15.4 / 15.9; 100 behind 200 14.7 / 18.4;
+    512 rows (512 tiles) 33 / 23, behind 1000 56 / 55, behind 4000 117 / 138,
+    behind 8000 195 / 276, in a window of 1024 there 50 / 45; 2 x 300 (608) behind
+    8000 242 / 265; 1000 rows (1008) behind 8000 359 / 290; 200 (208) behind 4000
+    58 / 126; 32 heads on 8, 8 x 200 behind 1000 182 / 66."""
     tiles = sum((n + 15) // 16 for n in seq_news if n >= PROMPT_PORTION) * heads
     span = min(max_ctx, window) if window > 0 else max_ctx
-    return tiles >= 512 or (tiles > 0 and span < 512)
+    return tiles >= 640 or tiles >= 512 and span <= 2048 \
+        or tiles > 0 and span <= 64
 
 
 def build_prompt_tiles(seq_starts, seq_hists, seq_news, device):

@@ -42,6 +42,16 @@ def test_every_row_and_head_has_one_tile(seqs, heads, kv_heads, window):
     assert bool((seen == 1).all())
 
 
+@pytest.mark.parametrize("news,ctx,heads,window,wins", [
+    ([512], 1512, 16, 0, True), ([512], 4512, 16, 0, False),
+    ([512], 8512, 16, 1024, True), ([1000], 9000, 16, 0, True),
+    ([128] * 8, 8128, 8, 0, False), ([100], 300, 16, 0, False),
+    ([300], 300, 16, 0, False), ([64], 64, 16, 0, True), ([31], 31, 64, 0, False),
+    ([1] * 512, 9000, 64, 0, False)])
+def test_where_the_prompt_kernel_runs(news, ctx, heads, window, wins):
+    assert ops.prompt_kernel_wins(news, ctx, heads, window) == wins
+
+
 @pytest.mark.parametrize("heads,kv_heads", [(16, 4), (3, 1)])
 @pytest.mark.parametrize("window", [0, 1, 33, 64, 200])
 @pytest.mark.parametrize("option", ["", "slopes", "sinks"])
