@@ -1335,8 +1335,10 @@ def scan_run_rows(seq_news, heads: int, vdim: int) -> int:
     266, 1 x 1000 191 / 107, 1 x 500 97 / 70, 1 x 250 50 / 50, 2 x 2000 364 /
     259, six of 301 to 1900 433 / 353, but 8 x 500 141 / 250, 4 x 200 47 / 91;
     16 heads of 128 1 x 4000 918 / 260, 1 x 500 121 / 77, the six 428 / 241,
-    8 x 500 133 / 173, 32 x 125 91 / 145. Batches of so many short sequences
-    that no chunk kernel runs have none either."""
+    8 x 500 133 / 173, 32 x 125 91 / 145. Of 345 batches that it cuts 20 take
+    longer, most at about 256 rows (49 / 54), at worst where the others fill the
+    chip anyway (400 beside 12 x 200 rows of 32 heads 93 / 115). Batches of so many
+    short sequences that no chunk kernel runs have none either."""
     longest, rows = max(seq_news, default=0), sum(seq_news)
     groups = heads * ((vdim + 63) // 64)
     if longest < 256 or longest * 256 <= rows * groups:
