@@ -710,18 +710,46 @@ def _silu_plan(M: int, N: int, K: int):
     return plan
 
 
+def _wide_silu_wins(M: int, N: int, K: int) -> bool:
+    """Where the product of many rows that ends in the activation
+    (wide_silu_kernel in ops/csrc/wide_tiles.hip) measured faster than the
+    library's product and the activation behind it; N columns, gate and up. Its
+    256 workgroups take tiles of 256 rows and 128 columns of the result in rounds,
+    so what decides is the share of its rounds' rows and columns that are filled;
+    short rows, of whose time the activation is more, want less of it. Of 1171
+    sizes (768 to 24576 columns of the result, 1024 to 8192 k, 136 to 8192 rows,
+    weights out of HBM) 438 are taken, two of them slower by more than 3 % (1280
+    rows of 11264 columns and 8192 k 1.06, 2048 of 11264 and 4096 1.04), .84 of the
+    other's time in the middle; 91 that would gain more than 5 % are not. us,
+    library and activation / this, 4096 k: 512 rows of 28672 105 / 94, 2048 381 /
+    355, 8192 1379 / 1282; 2048 of 22016 431 / 260; but 512 of 11264 57 / 72, and
+    640 of 28672, two rounds for one and a third, 146 / 164."""
+    if N % 16 != 0 or K % 64 != 0 or K < 128 or M <= 128 \
+            or (2 * N + 512) * K >= 1 << 31:
+        return False
+    tiles = -(-M // 256) * -(-N // 256)
+    filled = M * N / (-(-tiles // 256) * 256 * 256 * 256)
+    return filled >= (.5 if K <= 1024 else .6 if K <= 2048
+                      else .68 if K <= 4096 else .78)
+
+
 def linear_silu(x, w):
     """silu(gate) * up of the product with w = [gate rows; up rows], or None
     where the activation is a launch of its own: the tiled product of up to
-    128 rows (_rows_tile_plan), not cut over k, ends in it."""
+    128 rows (_rows_tile_plan), not cut over k, and the one of many rows
+    (_wide_silu_wins) end in it."""
     if not _own_products(x, w):
         return None
-    plan = _silu_plan(x.shape[0], w.shape[0], x.shape[1])
-    if plan is None or not _rows_take(x, w):
+    M, K = x.shape
+    plan = _silu_plan(M, w.shape[0], K)
+    wide = plan is None and _wide_silu_wins(M, w.shape[0], K)
+    if not (plan or wide) or not _rows_take(x, w):
         return None
-    out = torch.empty(x.shape[0], w.shape[0] // 2, dtype=x.dtype,
-                      device=x.device)
-    _load_hip().rows_tile(out, x, w, *plan, silu=True)
+    out = torch.empty(M, w.shape[0] // 2, dtype=x.dtype, device=x.device)
+    if wide:
+        _load_hip().wide_silu(out, x, w)
+    else:
+        _load_hip().rows_tile(out, x, w, *plan, silu=True)
     return out
 
 
