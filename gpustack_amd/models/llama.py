@@ -1070,16 +1070,28 @@ class MoEMLP(nn.Module):
             x = x.clone()
         flat = experts.reshape(-1).to(torch.int32)
         flat_w = weights.reshape(-1).float()
-        order, s_tok, counts, offs, tiles, ntiles = hip.moe_sort(
-            flat, self.e, k)
         act_mode = 1 if self.spec.moe_act == "clamped_swiglu" else 0
         # down bias on tp rank 0 only: the TP all-reduce must sum it once
         db = self.down_b if self.comm.tp_rank == 0 else None
+        h = x.shape[1]
+        wide_up = act_mode == 0 and self.gate_up_b is None \
+            and ops.moe_wide_wins(TK, self.e, self.i, h, False)
+        wide_down = db is None and ops.moe_wide_wins(TK, self.e, h, self.i, True)
+        order, s_tok, counts, offs, tiles, ntiles, *s_w = hip.moe_sort(
+            flat, self.e, k, weights=flat_w if wide_down else None)
         act = x.new_empty(TK, self.i)
-        contrib = x.new_empty(TK, x.shape[1])
-        hip.moe_tile(False, act, x, self._bank("gate_up"), s_tok, tiles,
-                     ntiles, offs, counts, bias=self.gate_up_b,
-                     act_mode=act_mode)
+        contrib = x.new_empty(TK, h)
+        if wide_up:
+            hip.moe_wide(False, act, x, self._bank("gate_up"), s_tok, offs,
+                         counts)
+        else:
+            hip.moe_tile(False, act, x, self._bank("gate_up"), s_tok, tiles,
+                         ntiles, offs, counts, bias=self.gate_up_b,
+                         act_mode=act_mode)
+        if wide_down:
+            hip.moe_wide(True, contrib, act, self._bank("down"), order, offs,
+                         counts, s_w[0])
+            return contrib
         # Up to one workgroup a CU of long rows: twice as many of 64 columns,
         # which read the weights again for every 16 rows of an expert. us,
         # 64 columns against tiles, by assignments: 8 experts of 4096 x 14336

@@ -8,6 +8,7 @@ engine/control-plane logic testable without hardware.
 """
 from __future__ import annotations
 
+import math
 import os
 from pathlib import Path
 
@@ -645,6 +646,33 @@ def router_plan(T: int, E: int, H: int):
     if T * E <= 1 << 19:
         return 32, 4
     return (128, 2) if E >= 128 else (64, 2)
+
+
+def moe_wide_wins(rows: int, E: int, N: int, K: int, down: bool) -> bool:
+    """Where an expert product of `rows` assignments in tiles of up to 320 rows
+    (ops/csrc/moe_wide.hip) measured faster than tiles of 128 (moe_gemm.hip). From
+    128 rows an expert, where these begin to read its weights twice, and where its
+    256 workgroups' rounds are filled, but for one round, or rows that fill the
+    tiles. us, 128-row tiles / this, first and second product: 128 experts of 2048
+    x 768 at 112 rows each 172 / 169 + 106 / 113, 128 198 / 173 + 119 / 116, 256
+    283 / 209 + 176 / 149, 340 (two tiles for each) 340 / 296 + 209 / 194, 800
+    721 / 539 + 434 / 383; 8 of 4096 x 14336 at 128 492 / 387 + 301 / 246, at 320,
+    two rounds of .69, 748 / 624 + 413 / 516: the second stays. Of 108 pairs of
+    products from 128 to 800 rows an expert, of ten models' sizes, 99 and 95 are
+    taken, none of them slower by more than 3 %."""
+    if E < 1 or E > 256 or rows < 128 * E or K % 64 != 0 or K < 192 or N % 8 != 0 \
+            or rows >= 1 << 30:
+        return False
+    # offsets of 32 bits of bytes
+    if ((1 if down else 2) * N + 192) * K >= (1 << 31) - (1 << 19) \
+            or rows * (N if down else K) >= (1 << 31) - (1 << 19) \
+            or 320 * max(N, K) >= (1 << 31) - (1 << 19):
+        return False
+    mean = rows // E
+    parts = -(-(mean + math.isqrt(mean)) // 320)   # some experts have more rows
+    tiles = E * parts * -(-N // (192 if down else 96))
+    rounds = -(-tiles // 256)
+    return rounds == 1 or tiles >= .8 * 256 * rounds or mean >= 240 * parts
 
 
 def linear_auto(x, w, parts: bool = False):

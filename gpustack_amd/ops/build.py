@@ -18,8 +18,9 @@ CSRC = PKG_DIR / "csrc"
 SO_PATH = PKG_DIR / "_hip_ops.so"
 ARCH = os.environ.get("GPUSTACK_AMD_ARCH", "gfx950")
 
-HIP_SOURCES = ["pointwise.hip", "attn_decode.hip", "attn_prefill.hip", "skinny_gemm.hip", "gemm8.hip", "gemm8_lab.hip", "moe_gemm.hip", "w4_gemm.hip", "rows_gemm.hip", "wide_tiles.hip", "mla_decode.hip"]
+HIP_SOURCES = ["pointwise.hip", "attn_decode.hip", "attn_prefill.hip", "skinny_gemm.hip", "gemm8.hip", "gemm8_lab.hip", "moe_gemm.hip", "moe_wide.hip", "w4_gemm.hip", "rows_gemm.hip", "wide_tiles.hip", "mla_decode.hip"]
 CPP_SOURCES = ["bindings.cpp"]
+HEADERS = ["common.h", "wide_tiles.h"]
 # the fp32-residual op family lives in its own small library: a checkout
 # that serves only such a model compiles these few files and nothing else
 LATENT_SO_PATH = PKG_DIR / "_hip_latent.so"
@@ -97,7 +98,7 @@ def build(verbose: bool = False, force: bool = False) -> Path:
 
     objs = []
     newest_src = 0.0
-    for src in HIP_SOURCES + CPP_SOURCES + ["common.h"]:
+    for src in HIP_SOURCES + CPP_SOURCES + HEADERS:
         p = CSRC / src
         if p.exists():
             newest_src = max(newest_src, p.stat().st_mtime)
@@ -113,7 +114,8 @@ def build(verbose: bool = False, force: bool = False) -> Path:
             not force
             and obj.exists()
             and obj.stat().st_mtime >= srcp.stat().st_mtime
-            and obj.stat().st_mtime >= (CSRC / "common.h").stat().st_mtime
+            and all(obj.stat().st_mtime >= (CSRC / h).stat().st_mtime
+                    for h in HEADERS)
         ):
             objs.append(str(obj))
             continue

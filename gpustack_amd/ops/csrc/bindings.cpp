@@ -28,7 +28,9 @@ void moe_down_scale_launch(void*, const void*, const void*, const int*, const in
 void moe_topk_launch(int*, float*, const float*, int, int, int, int, int, int*, hipStream_t);
 void moe_route_launch(int*, float*, const void*, const void*, int, int, int, int, int, int*, hipStream_t);
 int moe_sort_slices(int);
-void moe_sort_launch(int*, int*, int*, int*, int*, int*, int*, const int*, int, int, int, int*, hipStream_t);
+void moe_sort_launch(int*, int*, float*, const float*, int*, int*, int*, int*, int*, const int*, int, int, int, int*, hipStream_t);
+bool moe_wide_takes(int, long, long, int, int, int);
+void moe_wide_launch(int, void*, const void*, const void*, const int*, const float*, const int*, const int*, long, long, int, int, int, hipStream_t);
 void moe_sum_launch(void*, const void*, long, int, int, hipStream_t);
 void moe_tile_launch(int, void*, const void*, const void*, const int*, const int*, const int*, const int*, const int*, const float*, const void*, int, long, int, int, int, int*, hipStream_t);
 void rows_tile_launch(void*, void*, const void*, const void*, int, int, int, long, int, int, int, int*, hipStream_t);
@@ -508,10 +510,19 @@ void moe_route(at::Tensor experts, at::Tensor weights, at::Tensor x,
   HIP_CHECK_LAST();
 }
 
-// -> (order, s_tok, counts, offs, tiles, ntiles)
-std::vector<at::Tensor> moe_sort(at::Tensor experts, long E, long k) {
+// -> (order, s_tok, counts, offs, tiles, ntiles), and the weights in the order of the
+// sorted rows where they are given
+std::vector<at::Tensor> moe_sort(at::Tensor experts, long E, long k,
+                                 c10::optional<at::Tensor> weights) {
   const long TK = experts.numel();
   check_i32(experts, TK, "experts");
+  at::Tensor s_w;
+  if (weights.has_value()) {
+    TORCH_CHECK(weights->is_cuda() && weights->scalar_type() == at::kFloat &&
+                weights->is_contiguous() && weights->numel() == TK,
+                "weights [TK] fp32");
+    s_w = at::empty({TK}, weights->options());
+  }
   TORCH_CHECK(TK < (1L << 30) && k >= 1 && E >= 1, "moe_sort sizes");
   auto o = experts.options();
   at::Tensor order = at::empty({TK}, o), s_tok = at::empty({TK}, o);
@@ -521,13 +532,51 @@ std::vector<at::Tensor> moe_sort(at::Tensor experts, long E, long k) {
   at::Tensor hist = at::empty({slices * E}, o);
   int err = 0;
   moe_sort_launch(order.data_ptr<int>(), s_tok.data_ptr<int>(),
+                  s_w.defined() ? s_w.data_ptr<float>() : nullptr,
+                  s_w.defined() ? weights->data_ptr<float>() : nullptr,
                   counts.data_ptr<int>(), offs.data_ptr<int>(),
                   tiles.data_ptr<int>(), n.data_ptr<int>(),
                   hist.data_ptr<int>(), experts.data_ptr<int>(), (int)TK, (int)E, (int)k, &err,
                   cur_stream(experts));
   TORCH_CHECK(!err, "moe_sort: unsupported E=", E);
   HIP_CHECK_LAST();
+  if (s_w.defined()) return {order, s_tok, counts, offs, tiles, n, s_w};
   return {order, s_tok, counts, offs, tiles, n};
+}
+
+// moe_tile without bias or another activation, in tiles of up to 320 rows; s_w: the
+// weights that moe_sort sorted
+void moe_wide(bool down, at::Tensor out, at::Tensor src, at::Tensor w,
+              at::Tensor rows, at::Tensor offs, at::Tensor counts,
+              c10::optional<at::Tensor> s_w) {
+  check_bf16(out, "out"); check_bf16(src, "src"); check_bf16(w, "w");
+  TORCH_CHECK(w.dim() == 3 && src.dim() == 2 && out.dim() == 2, "moe_wide shapes");
+  const long E = w.size(0), K = w.size(2), TK = out.size(0);
+  const long N = down ? w.size(1) : w.size(1) / 2;
+  check_i32(rows, TK, "rows");
+  check_i32(offs, E, "offs");
+  check_i32(counts, E, "counts");
+  TORCH_CHECK(src.size(1) == K && out.size(1) == N &&
+              w.size(1) == (down ? N : 2 * N) && (!down || src.size(0) == TK),
+              "moe_wide shapes");
+  TORCH_CHECK((uintptr_t)src.data_ptr() % 16 == 0 &&
+              (uintptr_t)w.data_ptr() % 16 == 0 &&
+              (uintptr_t)out.data_ptr() % 16 == 0, "moe_wide addresses");
+  const float* sw = nullptr;
+  if (down) {
+    TORCH_CHECK(s_w.has_value() && s_w->is_cuda() &&
+                s_w->scalar_type() == at::kFloat && s_w->is_contiguous() &&
+                s_w->numel() == TK, "s_w [TK] fp32");
+    sw = s_w->data_ptr<float>();
+  }
+  TORCH_CHECK(N < (1l << 30) && K < (1l << 30) &&
+              moe_wide_takes(down ? 1 : 0, src.size(0), TK, (int)E, (int)N, (int)K),
+              "moe_wide: unsupported E=", E, " N=", N, " K=", K);
+  moe_wide_launch(down ? 1 : 0, out.data_ptr(), src.data_ptr(), w.data_ptr(),
+                  rows.data_ptr<int>(), sw, offs.data_ptr<int>(),
+                  counts.data_ptr<int>(), src.size(0), TK, (int)E, (int)N, (int)K,
+                  cur_stream(src));
+  HIP_CHECK_LAST();
 }
 
 void moe_sum(at::Tensor out, at::Tensor contrib, long k) {
@@ -830,7 +879,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rows_gemm", &rows_gemm, "bf16 product of up to 16 rows");
   m.def("moe_route", &moe_route, "router product and choice");
   m.def("moe_topk", &moe_topk, "softmax routing, top k");
-  m.def("moe_sort", &moe_sort, "assignments by expert, and the tile list");
+  m.def("moe_sort", &moe_sort, "assignments by expert, and the tile list",
+        py::arg("experts"), py::arg("E"), py::arg("k"),
+        py::arg("weights") = py::none());
+  m.def("moe_wide", &moe_wide, "expert products in tiles of up to 320 rows",
+        py::arg("down"), py::arg("out"), py::arg("src"), py::arg("w"),
+        py::arg("rows"), py::arg("offs"), py::arg("counts"),
+        py::arg("s_w") = py::none());
   m.def("moe_sum", &moe_sum, "sum of a row's expert contributions");
   m.def("moe_tile", &moe_tile, "expert products in 128x128 tiles",
         py::arg("down"), py::arg("out"), py::arg("src"), py::arg("w"),

@@ -506,8 +506,8 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(
 
 constexpr int MOE_MAX_E = 4096;
 
-// Counting sort of the assignments by expert: counts, offsets, the sorted rows
-// and the tile list. The order within an expert is free: a row's result does
+// Counting sort of the assignments by expert: counts, offsets, the sorted rows,
+// their weights where these are given, and the tile list. The order within an expert is free: a row's result does
 // not depend on its place. A short list is one workgroup's (about 5 us at 512
 // assignments; a radix sort, a scatter and the casts around them took 100).
 // Longer ones (32544 took it 37 us) are cut into slices of MOE_SLICE: a first
@@ -545,6 +545,7 @@ __global__ __launch_bounds__(1024) void moe_count_kernel(
 // gridDim.x slices with their counts in `hist`, or one workgroup without.
 __global__ __launch_bounds__(1024) void moe_sort_kernel(
     int* __restrict__ order, int* __restrict__ s_tok,  // [TK]
+    float* __restrict__ s_w, const float* __restrict__ flat_w,  // [TK] or null
     int* __restrict__ counts, int* __restrict__ offs,  // [E]
     int* __restrict__ tiles, int* __restrict__ ntiles,
     const int* __restrict__ experts, const int* __restrict__ hist, int TK,
@@ -628,6 +629,7 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(
     const int at = atomicAdd(&cnt[e], 1);
     order[at] = i;
     s_tok[at] = i / k;
+    if (s_w != nullptr) s_w[at] = flat_w[i];
   });
 }
 
@@ -707,10 +709,10 @@ int moe_sort_slices(int TK) {
   return TK > 2 * MOE_SLICE ? (TK + MOE_SLICE - 1) / MOE_SLICE : 0;
 }
 
-void moe_sort_launch(int* order, int* s_tok, int* counts, int* offs,
-                     int* tiles, int* ntiles, int* hist, const int* experts,
-                     int TK, int E, int k, int* err_unsupported,
-                     hipStream_t s) {
+void moe_sort_launch(int* order, int* s_tok, float* s_w, const float* flat_w,
+                     int* counts, int* offs, int* tiles, int* ntiles, int* hist,
+                     const int* experts, int TK, int E, int k,
+                     int* err_unsupported, hipStream_t s) {
   *err_unsupported = E < 1 || E > MOE_MAX_E;
   if (*err_unsupported) return;
   const int slices = moe_sort_slices(TK);
@@ -718,8 +720,8 @@ void moe_sort_launch(int* order, int* s_tok, int* counts, int* offs,
     hipLaunchKernelGGL(moe_count_kernel, dim3(slices), dim3(1024), 0, s, hist,
                        experts, TK, E);
   hipLaunchKernelGGL(moe_sort_kernel, dim3(slices > 0 ? slices : 1),
-                     dim3(1024), 0, s, order, s_tok, counts, offs, tiles,
-                     ntiles, experts, slices > 0 ? hist : nullptr, TK, E, k);
+                     dim3(1024), 0, s, order, s_tok, s_w, flat_w, counts, offs,
+                     tiles, ntiles, experts, slices > 0 ? hist : nullptr, TK, E, k);
 }
 
 void moe_tiles_launch(int* tiles, int* ntiles, const int* counts, int E,

@@ -24,9 +24,7 @@
 // 8192 rows of 28672 x 4096 with the activation 1228 us (1566 TFLOP/s), 2039 rows 348
 // (3.5 rounds of tiles in the time of four), 512 rows 86 (1403); the library's product
 // and the activation behind it 1290 + 127, 353 + 31, 85 + 11.
-#include "common.h"
-
-#include <type_traits>
+#include "wide_tiles.h"
 
 namespace {
 
@@ -34,33 +32,6 @@ constexpr int WT_ROWS = 256, WT_K = 64;
 constexpr int WT_BUF = WT_ROWS * WT_K;      // elements of a buffer
 constexpr int WT_BYTES = WT_BUF * 2;
 constexpr int WT_CUS = 256;                 // workgroups of a launch
-
-typedef __attribute__((ext_vector_type(4))) int i32x4;
-
-DEVICE_INLINE unsigned wt_pack(float lo, float hi) {
-  const f32x2 v{lo, hi};
-  return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
-}
-
-// Descriptor of `bytes` bytes at p; loads beyond them bring no memory.
-DEVICE_INLINE i32x4 wt_rsrc(const void* p, unsigned bytes) {
-  const unsigned long a = (unsigned long)p;
-  return i32x4{(int)a, (int)(a >> 32) & 0xffff, (int)bytes, 0x00020000};
-}
-
-DEVICE_INLINE float wt_silu(float g, float u) {
-  return g * u * __builtin_amdgcn_rcpf(1.f + __expf(-g));
-}
-
-// A sum out of its accumulation register, in the order of the program: read where the
-// compiler likes, all at once, they do not fit beside the operands of the next tile.
-DEVICE_INLINE float wt_sum(float acc) {
-  float v;
-  asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(acc));
-  return v;
-}
-
-template <int I> using wt_int = std::integral_constant<int, I>;
 
 // out [M, N] = silu(x Wg^T) * (x Wu^T), w [2 N, K] = Wg, then Wu
 __global__ __launch_bounds__(256, 1) void wide_silu_kernel(
