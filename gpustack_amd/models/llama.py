@@ -98,12 +98,14 @@ class RaggedMeta:
             self._tiles[key] = c
         return c
 
-    def scan_runs(self, heads: int, n_state: int, vdim: int, dtype):
+    def scan_runs(self, heads: int, n_state: int, vdim: int, dtype,
+                  exact: bool = False):
         """ops.state_scan's `runs` and `cut`, or nothing for a batch of short
-        portions or operands that its chunk kernel does not take."""
+        portions or operands that its chunk kernel does not take. `exact`: its
+        rows are taken as they are, without an activation."""
         if dtype != torch.bfloat16 or not 32 <= n_state <= 128 or vdim < 32:
             return {}
-        rows = ops.scan_run_rows(self.seq_news, heads, vdim)
+        rows = ops.scan_run_rows(self.seq_news, heads, vdim, exact)
         if not rows:
             return {}
         if self._tiles is None:

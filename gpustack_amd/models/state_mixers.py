@@ -97,7 +97,7 @@ class Mamba2Mixer(nn.Module):
                        self.dt_bias, self.a_log, self.skip, None, ssm_state,
                        rg.seq_first, rg.seq_rows, rg.state_slots, rg.pos32,
                        single=max(rg.seq_news, default=1) <= 1,
-                       **(rg.scan_runs(m.heads, m.state, m.vdim, h.dtype)
+                       **(rg.scan_runs(m.heads, m.state, m.vdim, h.dtype, True)
                           if h.is_cuda else {}))
         g = torch.empty(T, m.inner, dtype=h.dtype, device=h.device)
         ops.gated_group_norm(g, y, u[:, :m.inner], self.norm, m.norm_groups,

@@ -1383,7 +1383,8 @@ def causal_conv_silu(out, src, col0: int, w, b, conv_state, seq_first,
 SCAN_CHUNK_ROWS = 24
 
 
-def scan_run_rows(seq_news, heads: int, vdim: int) -> int:
+def scan_run_rows(seq_news, heads: int, vdim: int,
+                  exact: bool = False) -> int:
     """Rows of a run for state_scan, or 0 where whole sequences do as well: up
     to half of the chip's 512 places for workgroups (64 value channels of a
     head) would work through the longest sequence alone. us whole / in runs of
@@ -1394,9 +1395,23 @@ def scan_run_rows(seq_news, heads: int, vdim: int) -> int:
     8 x 500 133 / 173, 32 x 125 91 / 145. Of 345 batches that it cuts 20 take
     longer, most at about 256 rows (49 / 54), at worst where the others fill the
     chip anyway (400 beside 12 x 200 rows of 32 heads 93 / 115). Batches of so many
-    short sequences that no chunk kernel runs have none either."""
+    short sequences that no chunk kernel runs have none either.
+    `exact`: rows that no activation is put on, whose chunks take a quarter to half
+    of the time. Runs pay for the second walk later, and want to be longer: as long
+    as the longest sequence's root has it, or as many as the chip has places.
+    64 heads of 64, 1 x 500 rows 37 / 43, 1 x 1000 69 / 51, 1 x 4000 254 / 120, 2 x
+    2000 130 / 98, but 3 x 2000 132 / 149, six of 301 to 1900 155 / 187; 16 heads of
+    128 the six 124 / 97, 4 x 1000 69 / 62; 8 of 64 4 x 4000 253 / 105. Over 194
+    batches 1.8 % above the best of eleven lengths each, at worst 1.27 (2600 rows,
+    1000 of them of one sequence, 64 heads 73 / 93)."""
     longest, rows = max(seq_news, default=0), sum(seq_news)
     groups = heads * ((vdim + 63) // 64)
+    if exact:
+        if longest < 640 or longest * 160 <= rows * groups \
+                or rows < SCAN_CHUNK_ROWS * len(seq_news):
+            return 0
+        size = max(12 * math.sqrt(longest), rows * groups / 512)
+        return (int(size) + 31) // 32 * 32
     if longest < 256 or longest * 256 <= rows * groups:
         return 0
     if rows < SCAN_CHUNK_ROWS * len(seq_news):

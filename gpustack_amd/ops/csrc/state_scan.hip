@@ -358,11 +358,78 @@ __global__ __launch_bounds__(256) void state_scan_vec_kernel(
 // places, and the first launch leaves them out.
 // 64 heads of 128 x 64, one sequence of 4000 rows 723 -> 266 us, six of 301 to 1900
 // 433 -> 353; 16 heads of 128 x 128 918 -> 260 and 428 -> 241.
+//
+// EXACT: without an activation q, k and v are bf16 values, and the bf16 instructions
+// multiply them as they are, at sixteen times the rate: 16 cycles for 32 k where fp32
+// takes 32 for 4. The other operand (state, weighted scores, weighted v) is split into
+// three bf16 parts whose sum it is, bit for bit, so that the products are the exact ones
+// and only the sums round, in fp32 as before: error against 64 bits of y .76 and of the
+// state .95 to .99 of what the fp32 instructions leave (decays of a few tenths a row), .55
+// and .65 (of a hundredth); only the state of decays that leave nothing of the row
+// before is off by 6.4e-8 for 5.0e-8.
+//   - the state stays in the accumulators; its parts are made a chunk, 32 rows at a time.
+//   - scores are multiplied transposed, so that they lie as the operand of the product
+//     with v; every wave has them all, and no barrier stands between.
+//   - k and v are read down their columns (ds_read_b64_tr_b16); rows of two chunks in
+//     the LDS, one barrier a chunk. Rows of q and k lie permuted, 16 bytes a lane: as two
+//     reads of 8 a chunk takes 2.7 us instead of 2.1.
+//   - decays and the weights e^(c_t - c_s) b_s are made for four chunks at a time, by all
+//     threads: for one at a time by 32 of them a chunk takes 3.9 us.
+//   - where anything is not finite its split is NaN; it shows in the rows or the state,
+//     and the columns are walked again as below.
+// Bound by the vector instructions (500 a wave and chunk, 72 % of the time with two
+// waves a SIMD; 66 matrix ones): 64 heads of 128 x 64, whole 4000 rows 547 -> 254 us, the
+// six 303 -> 155, 8 x 500 91 -> 58 (fp32 instructions: 723, 433, 141).
 typedef __attribute__((ext_vector_type(4))) float sc_f32x4;
 
 enum ChunkPart { WHOLE, ENDS, OUTPUTS };
 
-template <int NT, int PART>   // state rows / 16, padded
+// An fp32 value as three bf16 ones that add up to it: its significant bits eight by
+// eight. Pairs, high halves first.
+struct Split8 { u32x4 part[3]; };
+DEVICE_INLINE Split8 split8(const float* x) {
+  Split8 s;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    unsigned u[2], v[2], w[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const float a = x[2 * i + j];
+      u[j] = __builtin_bit_cast(unsigned, a);
+      const float b = a - __builtin_bit_cast(float, u[j] & 0xffff0000u);
+      v[j] = __builtin_bit_cast(unsigned, b);
+      const float c = b - __builtin_bit_cast(float, v[j] & 0xffff0000u);
+      w[j] = __builtin_bit_cast(unsigned, c);
+    }
+    s.part[0][i] = __builtin_amdgcn_perm(u[1], u[0], 0x07060302u);
+    s.part[1][i] = __builtin_amdgcn_perm(v[1], v[0], 0x07060302u);
+    s.part[2][i] = __builtin_amdgcn_perm(w[1], w[0], 0x07060302u);
+  }
+  return s;
+}
+typedef __attribute__((ext_vector_type(8))) short sc_s16x8;
+typedef __attribute__((ext_vector_type(4))) short sc_s16x4;
+typedef __attribute__((ext_vector_type(2))) unsigned int sc_u32x2;
+DEVICE_INLINE sc_f32x4 mm_bf(const u32x4 a, const u32x4 b, sc_f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+      __builtin_bit_cast(sc_s16x8, a), __builtin_bit_cast(sc_s16x8, b), c, 0, 0, 0);
+}
+// a x the value whose parts s are, smallest first
+DEVICE_INLINE sc_f32x4 mm_split(const u32x4 a, const Split8& s, sc_f32x4 c) {
+  return mm_bf(a, s.part[0], mm_bf(a, s.part[1], mm_bf(a, s.part[2], c)));
+}
+DEVICE_INLINE sc_f32x4 mm_split(const Split8& s, const u32x4 b, sc_f32x4 c) {
+  return mm_bf(s.part[0], b, mm_bf(s.part[1], b, mm_bf(s.part[2], b, c)));
+}
+// 16 lanes read 4 rows of 16 neighbours, a lane gets four rows of its own
+DEVICE_INLINE sc_u32x2 read_down(const unsigned short* p) {
+  return __builtin_bit_cast(
+      sc_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (__attribute__((address_space(3))) sc_s16x4*)p));
+}
+
+// EXACT: q, k and v are the bf16 values of src (no activation here).
+template <int NT, int PART, bool EXACT>   // state rows / 16, padded
 __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
     float* __restrict__ y, const unsigned short* __restrict__ src,
     const unsigned short* __restrict__ dt_src, ScanArgs p) {
@@ -370,12 +437,25 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
   constexpr int KU = C * NP / 8 / 256;       // 16-byte loads of k (and q)
   static_assert(KU >= 1 && C * NP / 8 % 256 == 0, "NT is 4 or 8");
   constexpr int QR = PART == ENDS ? 1 : C;
-  __shared__ __attribute__((aligned(16))) float qs[QR][KS];
-  __shared__ __attribute__((aligned(16))) float ks[C][KS];
-  __shared__ __attribute__((aligned(16))) float vs[C][VS];
-  __shared__ __attribute__((aligned(16))) float as[QR][C + 4];
-  __shared__ double cs[C];
-  __shared__ float bl[C], el[C], wl[C];
+  // fp32 rows of one chunk, or bf16 ones of two
+  constexpr int F = EXACT ? 1 : C, FQ = EXACT ? 1 : QR;
+  __shared__ __attribute__((aligned(16))) float qs[FQ][KS];
+  __shared__ __attribute__((aligned(16))) float ks[F][KS];
+  __shared__ __attribute__((aligned(16))) float vs[F][VS];
+  __shared__ __attribute__((aligned(16))) float as[FQ][C + 4];
+  constexpr int HS = NP + 16, WS = PB + 8, B = EXACT ? C : 1;
+  __shared__ __attribute__((aligned(16))) unsigned short qh[2][EXACT ? QR : 1][HS];
+  __shared__ __attribute__((aligned(16))) unsigned short kh[2][B][HS];
+  __shared__ __attribute__((aligned(16))) unsigned short vh[2][B][WS];
+  // decays and weights, of EXACT for SB chunks at a time
+  constexpr int SB = EXACT ? 4 : 1, EB = EXACT && PART != ENDS ? SB : 1;
+  // e^(c_t - c_s) b_s of row t, column s <= t
+  __shared__ __attribute__((aligned(16))) float es[EB][EB > 1 ? C : 1][C + 4];
+  __shared__ double cs2[SB][C];
+  __shared__ float scal[SB][3][C];
+  __shared__ float fell[SB];                 // EXACT: a chunk's product of decays
+  double* cs = cs2[0];
+  float *bl = scal[0][0], *el = scal[0][1], *wl = scal[0][2];
   int s = blockIdx.x;
   const int h = blockIdx.y, pb0 = blockIdx.z * PB;
   const int run = blockIdx.x;
@@ -437,6 +517,7 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
     const float* from = PART == OUTPUTS && !ends
                             ? p.scratch + (long)run * stride + h * NP_ : sp;
     each([&](float, long i) { return from[i]; });
+    if constexpr (EXACT) each([&](float x, long) { odd += x * 0.f; return x; });
     if constexpr (PART == ENDS) {            // the last run writes the slot
       float* to = p.scratch + (long)run * stride + h * NP_;
       each([&](float x, long i) { return to[i] = x; });
@@ -457,6 +538,33 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
   float dreg = 0.f;
   auto fetch = [&](int c0) {
     const int rows = min(C, n - c0);
+    if constexpr (EXACT) {
+      // rows behind the last one and columns of no row come as zeros
+      const unsigned ld2 = (unsigned)p.ld_src * 2u;
+      const unsigned short* at = src + (long)(first + c0) * p.ld_src;
+      auto rsrc = [&](const unsigned short* from, int width) {
+        return __builtin_amdgcn_make_buffer_rsrc(
+            (void*)from, 0, (unsigned)(rows - 1) * ld2 + (unsigned)width * 2u,
+            0x00020000);
+      };
+      const auto rk = rsrc(at + p.col_b + grp * N, N);
+      const auto rq = rsrc(at + p.col_c + grp * N, N);
+      const auto rv = rsrc(at + p.col_x + h * P, P);
+      auto load8 = [&](const __amdgpu_buffer_rsrc_t& rs, int r, int e, int width) {
+        return __builtin_bit_cast(
+            u16x8, __builtin_amdgcn_raw_buffer_load_b128(
+                       rs, e < width ? (unsigned)r * ld2 + (unsigned)e * 2u : 0xffffff00u,
+                       0, 0));
+      };
+#pragma unroll
+      for (int u = 0; u < KU; ++u) {
+        const int i = tid + u * 256, r = i / (NP / 8), e = i % (NP / 8) * 8;
+        kreg[u] = load8(rk, r, e, N);
+        if constexpr (PART != ENDS) qreg[u] = load8(rq, r, e, N);
+      }
+      vreg = load8(rv, tid / (PB / 8), pb0 + tid % (PB / 8) * 8, P);
+      return;
+    }
 #pragma unroll
     for (int u = 0; u < KU; ++u) {
       const int i = tid + u * 256, r = i / (NP / 8), e = i % (NP / 8) * 8;
@@ -490,10 +598,91 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
   };
 
+  // Eight neighbours of state rows, e .. e + 7. Of 32 rows a lane group takes 4 g ..
+  // 4 g + 3 and 16 further on, as the state's accumulators hold them: those lie
+  // together.
+  auto put_bf = [&](unsigned short* row, int e, const u16x8 from) {
+    const u32x4 w = __builtin_bit_cast(u32x4, from);
+    unsigned short* at = row + (e & ~31) + (e & 8) * 2 + (e & 16) / 4;
+    *reinterpret_cast<sc_u32x2*>(at) = sc_u32x2{w[0], w[1]};
+    *reinterpret_cast<sc_u32x2*>(at + 8) = sc_u32x2{w[2], w[3]};
+  };
+
+  // Decays and weights of the rows from c0 on, a row a thread, chunks of 32 apart.
+  auto scalars = [&](int c0) {
+    const int rows = n - c0, row = tid & (C - 1), chunk = EXACT ? tid / C : 0;
+    // rows behind the last one: decay 1, weight 0
+    float la = 0.f, b = 0.f;
+    if (tid < rows) {
+      if (dt_src != nullptr) {
+        b = softplus_f(dreg + dtb);
+        la = low(-a_rate * b);
+      } else {
+        b = 1.f;
+        la = log_const;
+      }
+    }
+    double c = la;
+#pragma unroll
+    for (int m = 1; m < C; m <<= 1) {
+      const double o = __shfl_up(c, m, 32);
+      if (row >= m) c += o;
+    }
+    const double all = __shfl(c, C - 1, 32);
+    if (EXACT && chunk >= SB) return;
+    const int in = min(C, rows - chunk * C), last = in - 1;
+    // EXACT takes powers of two of the differences
+    cs2[chunk][row] = EXACT ? c * 1.4426950408889634 : c;
+    if (EXACT && row == C - 1)
+      fell[chunk] = expf((float)c) * (neg && (in & 1) ? -1.f : 1.f);
+    scal[chunk][0][row] = b;
+    scal[chunk][1][row] = expf((float)c) * (neg && !(row & 1) ? -1.f : 1.f);
+    scal[chunk][2][row] = b * expf((float)(all - c)) *
+                          (neg && ((last - row) & 1) ? -1.f : 1.f);
+  };
+  auto fetch_dt = [&](int c0) {              // EXACT: for the next SB chunks
+    if (dt_src != nullptr && tid < SB * C && c0 + tid < n)
+      dreg = bf2f(dt_src[(long)(first + c0 + tid) * p.ld_dt + p.col_dt + h]);
+  };
+
   float fall = 1.f;
   fetch(0);
+  if constexpr (EXACT) fetch_dt(0);
   for (int c0 = 0; c0 < n; c0 += C) {
     const int rows = min(C, n - c0);
+    const int buf = EXACT ? (c0 / C) & 1 : 0, at = c0 / C % SB;
+    if constexpr (EXACT) {
+      if (at == 0) {
+        if (c0 > 0) __syncthreads();         // the last of the SB before is read
+        scalars(c0);
+        fetch_dt(c0 + SB * C);
+        if constexpr (PART != ENDS) {
+          __syncthreads();
+          const int tr = tid >> 4, sr = tid & 15;
+#pragma unroll 1
+          for (int b = 0; b < SB; ++b)
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {    // 16 x 16 on and below the diagonal
+              const int t = (i > 0) * 16 + tr, sc = (i > 1) * 16 + sr;
+              const bool behind = i == 1 || sr <= tr;
+              float x = scal[b][0][sc] *
+                        __builtin_amdgcn_exp2f(
+                            behind ? (float)(cs2[b][t] - cs2[b][sc]) : 0.f);
+              if (neg && ((t - sc) & 1)) x = -x;
+              es[b][t][sc] = behind ? x : 0.f;
+            }
+        }
+      }
+      el = scal[at][1];
+      wl = scal[at][2];
+#pragma unroll
+      for (int u = 0; u < KU; ++u) {
+        const int i = tid + u * 256, r = i / (NP / 8), e = i % (NP / 8) * 8;
+        put_bf(kh[buf][r], e, kreg[u]);
+        if constexpr (PART != ENDS) put_bf(qh[buf][r], e, qreg[u]);
+      }
+      *reinterpret_cast<u16x8*>(&vh[buf][tid / (PB / 8)][tid % (PB / 8) * 8]) = vreg;
+    } else {
 #pragma unroll
     for (int u = 0; u < KU; ++u) {
       const int i = tid + u * 256, r = i / (NP / 8), e = i % (NP / 8) * 8;
@@ -501,35 +690,117 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
       if constexpr (PART != ENDS) put8(&qs[r][e], qreg[u]);
     }
     put8(&vs[tid / (PB / 8)][tid % (PB / 8) * 8], vreg);
-    if (tid < C) {
-      // rows behind the last one: decay 1, weight 0
-      float la = 0.f, b = 0.f;
-      if (tid < rows) {
-        if (dt_src != nullptr) {
-          b = softplus_f(dreg + dtb);
-          la = low(-a_rate * b);
-        } else {
-          b = 1.f;
-          la = log_const;
-        }
-      }
-      double c = la;
-#pragma unroll
-      for (int m = 1; m < C; m <<= 1) {
-        const double o = __shfl_up(c, m, 32);
-        if (tid >= m) c += o;
-      }
-      const double all = __shfl(c, C - 1, 32);
-      const int last = rows - 1;
-      cs[tid] = c;
-      bl[tid] = b;
-      el[tid] = expf((float)c) * (neg && !(tid & 1) ? -1.f : 1.f);
-      wl[tid] = b * expf((float)(all - c)) *
-                (neg && ((last - tid) & 1) ? -1.f : 1.f);
     }
+    if (!EXACT && tid < C) scalars(c0);
     __syncthreads();
     if (c0 + C < n) fetch(c0 + C);
 
+    if constexpr (EXACT) {
+      // rows 4 g + j and 16 + 4 g + j of this lane's value channel
+      const unsigned short* vp = &vh[buf][g * 4 + (lc >> 2)][wave * 16 + (lc & 3) * 4];
+      const sc_u32x2 v0 = read_down(vp), v1 = read_down(vp + 16 * WS);
+      const u32x4 vb{v0[0], v0[1], v1[0], v1[1]};
+      float vf[8];
+      bf8_to_f32(__builtin_bit_cast(u16x8, vb), vf);
+      if constexpr (PART != ENDS) {
+        u32x4 qf[2][NT / 2];
+        sc_f32x4 o[2], o2[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          o[t] = o2[t] = sc_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int kb = 0; kb < NT / 2; ++kb)
+            qf[t][kb] = *reinterpret_cast<const u32x4*>(
+                &qh[buf][t * 16 + lc][kb * 32 + g * 8]);
+        }
+        // scores, transposed: row s = 4 g + r, column t = lc; weighted they are the
+        // operand of the product with v as they lie
+        float w[2][8];
+#pragma unroll
+        for (int si = 0; si < 2; ++si) {
+          sc_f32x4 a[2];
+#pragma unroll
+          for (int t = 0; t < 2; ++t) a[t] = sc_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int kb = 0; kb < NT / 2; ++kb) {
+            const u32x4 kf = *reinterpret_cast<const u32x4*>(
+                &kh[buf][si * 16 + lc][kb * 32 + g * 8]);
+#pragma unroll
+            for (int t = si; t < 2; ++t) a[t] = mm_bf(kf, qf[t][kb], a[t]);
+          }
+#pragma unroll
+          for (int t = 0; t < 2; ++t) {
+            if (si > t) {
+#pragma unroll
+              for (int r = 0; r < 4; ++r) w[t][si * 4 + r] = 0.f;
+              continue;
+            }
+            const sc_f32x4 e4 = *reinterpret_cast<const sc_f32x4*>(
+                &es[at][t * 16 + lc][si * 16 + g * 4]);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) w[t][si * 4 + r] = a[t][r] * e4[r];
+          }
+        }
+        // what the state brings
+#pragma unroll
+        for (int kb = 0; kb < NT / 2; ++kb) {
+          float x[8];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            x[r] = S[2 * kb][r];
+            x[4 + r] = S[2 * kb + 1][r];
+          }
+          const Split8 sp8 = split8(x);
+          // two chains a tile: the large parts and the small ones
+#pragma unroll
+          for (int t = 0; t < 2; ++t) {
+            o[t] = mm_bf(qf[t][kb], sp8.part[0], o[t]);
+            o2[t] = mm_bf(qf[t][kb], sp8.part[1],
+                          mm_bf(qf[t][kb], sp8.part[2], o2[t]));
+          }
+        }
+        const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(
+            y + (long)(first + c0) * p.H * P + h * P, 0,
+            ((unsigned)(rows - 1) * (unsigned)p.H + 1u) * (unsigned)P * 4u, 0x00020000);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            o[t][r] = (o[t][r] + o2[t][r]) * el[t * 16 + g * 4 + r];
+          // and the chunk's own rows
+          o[t] = mm_split(split8(w[t]), vb, o[t]);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            odd += o[t][r] * 0.f;
+            // rows behind the last and channels of no head are not stored
+            const unsigned off =
+                ((unsigned)(t * 16 + g * 4 + r) * (unsigned)p.H * (unsigned)P +
+                 (unsigned)pc) * 4u;
+            __builtin_amdgcn_raw_buffer_store_b32(
+                __builtin_bit_cast(unsigned, o[t][r] + skip * vf[t * 4 + r]), ry,
+                live ? off : 0xffffff00u, 0, 0);
+          }
+        }
+      }
+      // the state behind the chunk
+      const float down = fell[at];
+      if constexpr (PART == ENDS) fall *= down;
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[t][r] *= down;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) vf[j] *= wl[(j >> 2) * 16 + g * 4 + (j & 3)];
+      const Split8 bv = split8(vf);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const unsigned short* kp =
+            &kh[buf][g * 4 + (lc >> 2)][t / 2 * 32 + (lc & 3) * 8 + (t & 1) * 4];
+        const sc_u32x2 k0 = read_down(kp), k1 = read_down(kp + 16 * HS);
+        S[t] = mm_split(u32x4{k0[0], k0[1], k1[0], k1[1]}, bv, S[t]);
+      }
+      continue;
+    }
     sc_f32x4 o[2];
     if constexpr (PART != ENDS) {
     // scores of 16 x 16 rows a wave, weighted
@@ -628,6 +899,13 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
       }
     __syncthreads();
   }
+  // Of EXACT what is not finite, and splits into NaN, shows in the rows (q, k) or in
+  // the state (k, v), which keeps it.
+  if constexpr (EXACT)
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) odd += S[t][r] * 0.f;
   float* own = PART == WHOLE || (PART == OUTPUTS && ends)
                    ? sp
                    : (PART == ENDS ? p.ends : p.scratch) + (long)run * stride +
@@ -953,10 +1231,13 @@ bool scan_pick(float* y, const void* src, const void* dt, const ScanArgs& p,
     tpp *= 2;
   const bool vec = vec_rows(p.N, p.P, p.ld_src, p.col_x, p.col_b, p.col_c);
   if (chunk_rows(sizeof(TS) == 2, vec, p.N, p.P, p.T, nseq)) {
-#define CHUNKS(NT, PART, GROUPS)                                             \
-  state_chunk_kernel<NT, PART>                                               \
+#define CHUNKS_AS(NT, PART, GROUPS, EXACT)                                   \
+  state_chunk_kernel<NT, PART, EXACT>                                        \
       <<<dim3(GROUPS, p.H, (p.P + 63) / 64), 256, 0, s>>>(                   \
           y, (const unsigned short*)src, (const unsigned short*)dt, p)
+#define CHUNKS(NT, PART, GROUPS)                                             \
+  if (p.act) CHUNKS_AS(NT, PART, GROUPS, false);                             \
+  else CHUNKS_AS(NT, PART, GROUPS, true)
 #define CHUNKS_NT(NT)                                                        \
   if (p.ncut > 0) {                                                          \
     CHUNKS(NT, ENDS, p.ncut);                                                \
@@ -967,6 +1248,7 @@ bool scan_pick(float* y, const void* src, const void* dt, const ScanArgs& p,
     if (p.N <= 64) { CHUNKS_NT(4) } else { CHUNKS_NT(8) }
 #undef CHUNKS_NT
 #undef CHUNKS
+#undef CHUNKS_AS
     return true;
   }
   // few workgroups (long portions of few sequences): more lanes per channel
