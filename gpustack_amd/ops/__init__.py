@@ -627,6 +627,27 @@ def _parts_plan(M: int, N: int, K: int):
     return 128, 3 if K % 4096 == 0 else 4
 
 
+def _wide_parts(M: int, N: int, K: int) -> int:
+    """Parts over k of a product of many rows whose consumer adds them up
+    (wide_kernel in ops/csrc/wide_tiles.hip), or 0. As many as let its 256
+    workgroups have one tile of 256 x 256 each, where three quarters of them are
+    filled, from 11008 k on half; with rows that _tall_tile_plan cuts from 14336 k
+    on. us with an RMS norm behind, weights out of HBM, before / so: 4096x14336 at
+    400 rows 69 / 63, 640 143 / 84, 1024 159 / 107, 2039 217 / 197; 8192x8192 at 512
+    84 / 75; 5120x11008 at 512 .71 of the time, 7168x7168 .88; 4096x7168 at 512 1.09
+    (not taken), 6144x4096 at 512 43 / 46. Of 994 sizes (2048 to 10240 columns, 4096
+    to 14336 k, 264 to 4000 rows) 417 are taken, two of them slower by 4 %, .83 of
+    the time on average."""
+    if M <= 256 or K < 7168 or K % 64 != 0 or N % 8 != 0 \
+            or (N + 512) * K >= 1 << 31:
+        return 0
+    parts = min(8, 256 // (-(-M // 256) * -(-N // 256)))
+    if parts < 2 or K < 14336 and M <= 512 and _tall_tile_plan(M, N, K):
+        return 0
+    filled = M * N * parts / (256 * 256 * 256)
+    return parts if filled >= (.75 if K < 11008 else .55) else 0
+
+
 def router_plan(T: int, E: int, H: int):
     """(columns of a tile, parts over k) of a router's product, whose parts the
     choice of the experts adds up, or None. us for both launches against a
@@ -688,6 +709,9 @@ def linear_auto(x, w, parts: bool = False):
     if _own_products(x, w):
         M, K = x.shape
         N = w.shape[0]
+        wide = _wide_parts(M, N, K) if parts else 0
+        if wide and _rows_take(x, w):
+            return _load_hip().wide_parts(x, w, wide)
         plan = parts and _parts_plan(M, N, K) or _rows_tile_plan(M, N, K)
         if (plan or _rows_gemm_wins(M, N, K)) and _rows_take(x, w):
             if parts and plan and plan[1] > 1:
@@ -740,7 +764,7 @@ def _silu_plan(M: int, N: int, K: int):
 
 def _wide_silu_wins(M: int, N: int, K: int) -> bool:
     """Where the product of many rows that ends in the activation
-    (wide_silu_kernel in ops/csrc/wide_tiles.hip) measured faster than the
+    (wide_kernel in ops/csrc/wide_tiles.hip) measured faster than the
     library's product and the activation behind it; N columns, gate and up. Its
     256 workgroups take tiles of 256 rows and 128 columns of the result in rounds,
     so what decides is the share of its rounds' rows and columns that are filled;

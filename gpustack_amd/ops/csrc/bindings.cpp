@@ -39,7 +39,7 @@ bool w4_has(int, int);
 bool w4_cuts(int, int, int);
 bool w4_by_rows(int, int, int);
 bool w4_silu_wins(int, int, int);
-void wide_silu_launch(void*, const void*, const void*, int, int, int, long, int*, hipStream_t);
+void wide_launch(void*, const void*, const void*, int, int, int, long, int, int*, hipStream_t);
 int w4_splits(int, int, int);
 void w4_parts_launch(float*, const void*, const void*, const void*, const void*, int, int, int, int, hipStream_t);
 void w4_silu_launch(void*, const void*, const void*, const void*, const void*, int, int, int, hipStream_t);
@@ -687,23 +687,44 @@ void rows_gemm(at::Tensor out, at::Tensor x, at::Tensor w) {
   HIP_CHECK_LAST();
 }
 
-// out = silu(gate) * up of many rows, w holding the gate's rows and behind them the
-// up product's
-void wide_silu(at::Tensor out, at::Tensor x, at::Tensor w) {
-  check_bf16(out, "out"); check_bf16(w, "w");
+// operands of a product of many rows -> M, N weight rows, K
+void check_wide(const at::Tensor& x, const at::Tensor& w) {
+  check_bf16(w, "w");
   TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 && x.dim() == 2
               && x.stride(1) == 1 && x.stride(0) % 8 == 0
               && (uintptr_t)x.data_ptr() % 16 == 0, "x rows of bf16");
-  const long M = x.size(0), K = x.size(1), N = out.size(1);
-  TORCH_CHECK(w.dim() == 2 && w.size(0) == 2 * N && w.size(1) == K &&
-              out.size(0) == M && (uintptr_t)w.data_ptr() % 16 == 0 &&
-              (uintptr_t)out.data_ptr() % 16 == 0 && M < (1l << 31) &&
-              N < (1l << 30) && K < (1l << 30), "wide_silu shapes");
+  TORCH_CHECK(w.dim() == 2 && w.size(1) == x.size(1) &&
+              (uintptr_t)w.data_ptr() % 16 == 0 && x.size(0) < (1l << 31) &&
+              w.size(0) < (1l << 30) && x.size(1) < (1l << 30), "wide shapes");
+}
+
+// out = silu(gate) * up of many rows, w holding the gate's rows and behind them the
+// up product's
+void wide_silu(at::Tensor out, at::Tensor x, at::Tensor w) {
+  check_bf16(out, "out");
+  check_wide(x, w);
+  const long M = x.size(0), N = out.size(1), K = x.size(1);
+  TORCH_CHECK(out.dim() == 2 && out.size(0) == M && w.size(0) == 2 * N &&
+              (uintptr_t)out.data_ptr() % 16 == 0, "wide_silu shapes");
   int err = 0;
-  wide_silu_launch(out.data_ptr(), x.data_ptr(), w.data_ptr(), (int)M, (int)N,
-                   (int)K, x.stride(0), &err, cur_stream(x));
+  wide_launch(out.data_ptr(), x.data_ptr(), w.data_ptr(), (int)M, (int)N, (int)K,
+              x.stride(0), 0, &err, cur_stream(x));
   TORCH_CHECK(!err, "wide_silu: unsupported M=", M, " N=", N, " K=", K);
   HIP_CHECK_LAST();
+}
+
+// fp32 parts [splits, M, N] of the product, not added up
+at::Tensor wide_parts(at::Tensor x, at::Tensor w, long splits) {
+  check_wide(x, w);
+  const long M = x.size(0), N = w.size(0), K = x.size(1);
+  TORCH_CHECK(splits >= 1 && splits <= K / 128, "wide_parts: parts of K=", K);
+  at::Tensor parts = at::empty({splits, M, N}, x.options().dtype(at::kFloat));
+  int err = 0;
+  wide_launch(parts.data_ptr(), x.data_ptr(), w.data_ptr(), (int)M, (int)N,
+              (int)K, x.stride(0), (int)splits, &err, cur_stream(x));
+  TORCH_CHECK(!err, "wide_parts: unsupported M=", M, " N=", N, " K=", K);
+  HIP_CHECK_LAST();
+  return parts;
 }
 
 // the up product from counts and offsets that the caller sorted by
@@ -894,6 +915,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("bias") = py::none(), py::arg("act_mode") = 0);
   m.def("wide_silu", &wide_silu,
         "silu(x Wg^T) * (x Wu^T) of many rows (bf16, f32 accum)");
+  m.def("wide_parts", &wide_parts, "fp32 parts of a product of many rows");
   m.def("moe_gate_up_silu", &moe_gate_up_silu,
         py::arg("act"), py::arg("x"), py::arg("w"), py::arg("s_tok"),
         py::arg("offs"), py::arg("counts"), py::arg("bias") = py::none(),

@@ -1,5 +1,5 @@
 // Products of many rows for MI355X (gfx950) in tiles of 256 rows and 256 weight
-// rows: silu(x Wg^T) * (x Wu^T) in one launch.
+// rows: silu(x Wg^T) * (x Wu^T) in one launch, or x W^T cut over k.
 //
 // One workgroup a CU walks its tiles; four waves of 128 x 128 on
 // mfma_f32_16x16x32_bf16 (of random numbers 2.1 PFLOP/s before the card's power
@@ -21,9 +21,13 @@
 // them to other registers and copies, all 256 being taken. It does not see the products
 // in the asm, so the waits before their results are read stand here (s_nop), and a loop
 // of one body keeps it from copying them in between.
-// 8192 rows of 28672 x 4096 with the activation 1228 us (1566 TFLOP/s), 2039 rows 348
-// (3.5 rounds of tiles in the time of four), 512 rows 86 (1403); the library's product
-// and the activation behind it 1290 + 127, 353 + 31, 85 + 11.
+// 8192 rows of 28672 x 4096 with the activation 1228 us (1566 TFLOP/s), 2039 rows 345
+// (3.5 rounds of tiles in the time of four), 512 rows 86 (1403), 91 out of HBM; the
+// library's product and the activation behind it 1290 + 127, 353 + 31, 85 + 11.
+// A product of fewer columns leaves workgroups without a tile: cut over k it fills them,
+// and what reads it adds the fp32 parts up: with an RMS norm behind, 4096 x 14336 at 512
+// rows 69 us (before 73), 640 84 (143), 1024 107 (159), 2039 197 (217).
+// Without the activation and whole, the tiles are 1.00 to 1.05 of the library's time.
 #include "wide_tiles.h"
 
 namespace {
@@ -33,48 +37,67 @@ constexpr int WT_BUF = WT_ROWS * WT_K;      // elements of a buffer
 constexpr int WT_BYTES = WT_BUF * 2;
 constexpr int WT_CUS = 256;                 // workgroups of a launch
 
-// out [M, N] = silu(x Wg^T) * (x Wu^T), w [2 N, K] = Wg, then Wu
-__global__ __launch_bounds__(256, 1) void wide_silu_kernel(
-    unsigned short* __restrict__ out, const unsigned short* __restrict__ x,
-    const unsigned short* __restrict__ w, int M, int N, int K, long xs) {
-  constexpr int COLS = WT_ROWS / 2;         // columns of a tile
-  constexpr int STORES = 16;                // of a wave at the end of a tile
+// SILU: out [M, N] = silu(x Wg^T) * (x Wu^T), w [2 N, K] = Wg, then Wu. PARTS: out
+// [splits, M, N] = x W^T in fp32, each of its own steps of k, w [N, K].
+enum WideOut { SILU, PARTS };
+
+template <int OUT>
+__global__ __launch_bounds__(256, 1) void wide_kernel(
+    void* __restrict__ out_, const unsigned short* __restrict__ x,
+    const unsigned short* __restrict__ w, int M, int N, int K, long xs, int splits) {
+  constexpr int COLS = OUT == SILU ? WT_ROWS / 2 : WT_ROWS;  // columns of a tile
+  constexpr int HC = COLS / 2;              // of a wave
+  // of a wave at the end of a tile; what a wait can count
+  constexpr int STORES = OUT == SILU ? 16 : 55;
   // rows' buffers, then the weights'
   __shared__ __attribute__((aligned(16))) unsigned short lds[5 * WT_BUF];
   const int tid = threadIdx.x, lane = tid & (WAVE_SIZE - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE_SIZE);
   const int wm = wave >> 1, wn = wave & 1;
   const int lc = lane & 15, lg = lane >> 4;
-  const int n = K / WT_K;
+  const int steps = K / WT_K;
+  const int WN = OUT == SILU ? 2 * N : N;   // weight rows
   const int mt = (M + WT_ROWS - 1) / WT_ROWS, nt = (N + COLS - 1) / COLS;
 
   // An XCD's tiles follow each other in blocks of 8 tiles of rows by all columns,
-  // rows first, so that its L2 serves 8 workgroups a weight and 4 a row.
+  // rows first, so that its L2 serves 8 workgroups a weight and 4 a row; one part of
+  // k behind the other.
   const int xcd = blockIdx.x & 7, per = WT_CUS / 8, slot = blockIdx.x >> 3;
-  const int q = mt * nt / 8, r = mt * nt % 8;
+  const int all = mt * nt * (OUT == PARTS ? splits : 1);
+  const int q = all / 8, r = all % 8;
   const int count = xcd < r ? q + 1 : q;    // tiles of this XCD
   const int start = xcd * q + min(xcd, r);
   if (slot >= count) return;
   const int rounds = (count - slot + per - 1) / per;
-  struct Place { int m0, n0; };
+  struct Place { int m0, n0, part, from, n; };  // n: steps, the first is `from`
+  auto one = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
   auto place = [&](int round) {
-    const int t = start + round * per + slot;
+    int t = start + round * per + slot;
+    Place p{0, 0, 0, 0, steps};
+    if constexpr (OUT == PARTS) {
+      p.part = t / (mt * nt);
+      t -= p.part * (mt * nt);
+      p.from = one((int)((long)steps * p.part / splits));
+      p.n = one((int)((long)steps * (p.part + 1) / splits)) - p.from;
+    }
     const int g = t / (8 * nt), in = t % (8 * nt), high = min(8, mt - g * 8);
-    return Place{(g * 8 + in % high) * WT_ROWS, in / high * COLS};
+    p.m0 = one((g * 8 + in % high) * WT_ROWS);
+    p.n0 = one(in / high * COLS);
+    return p;
   };
 
-  // A wave's load i brings rows (i * 4 + wave) * 8 .. of 128 bytes to the LDS. Of the
-  // 128 weight rows of a wave 64 are the gate's and 64 the up product's; row 4 g + j
-  // of tiles 2 p and 2 p + 1 is column 32 p + 8 g + j and + 4, so that a lane ends
-  // with eight neighbouring columns.
+  // A wave's load i brings rows (i * 4 + wave) * 8 .. of 128 bytes to the LDS. Row
+  // 4 g + j of a wave's tiles 2 p and 2 p + 1 is column 32 p + 8 g + j and + 4, so that
+  // a lane ends with eight neighbouring columns; of SILU tiles 0 to 3 are the gate's, 4
+  // to 7 the up product's.
   unsigned ox[8], ow[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int row = (i * 4 + wave) * 8 + lane / 8;
     const int at = ((lane & 7) ^ ((row >> 1) & 7)) * 8;
-    const int b = (row >> 4) & 3, ii = row & 15;
-    const int col = (row >> 7) * 64 + (b >> 1) * 32 + (ii >> 2) * 8 + (b & 1) * 4 +
-                    (ii & 3) + (row & 64 ? N : 0);
+    const int b = (row >> 4) & (OUT == SILU ? 3 : 7), ii = row & 15;
+    const int col = (row >> 7) * HC + (b >> 1) * 32 + (ii >> 2) * 8 + (b & 1) * 4 +
+                    (ii & 3) + (OUT == SILU && (row & 64) ? N : 0);
     ox[i] = ((unsigned)row * (unsigned)xs + at) * 2;
     ow[i] = ((unsigned)col * (unsigned)K + at) * 2;
   }
@@ -82,22 +105,35 @@ __global__ __launch_bounds__(256, 1) void wide_silu_kernel(
   const unsigned short* wl = lds + (2 * WT_ROWS + wn * 128) * WT_K;
   const unsigned to = lds_address(lds) + wave * 8 * WT_K * 2;
 
-  // The step that is loaded next: lk of the tile of round `lr`.
-  int lr = 0, lk = 0;
+  // The step that is loaded next: of the tile of round `lr`, with `left` steps to come;
+  // k0: its bytes from the start of a row. Weight rows lie a power of two apart, and
+  // workgroups at one place of theirs meet on a few memory channels: each XCD begins an
+  // eighth of the row further on (512 rows of 28672 x 4096 out of HBM 97 -> 91 us; each
+  // column tile at a place of its own 96, and 1327 for 1250 at 8192 rows, whose rows
+  // then miss the L2). Of no use in more rows, which compute longer than they load
+  // (7122 x 8192 x 2048 330 -> 331), and parts begin elsewhere anyway.
+  const int turn = OUT == SILU && M <= 2048 ? xcd * steps / 8 : 0;
+  int lr = 0, left = 0;
+  unsigned k0 = 0;
   i32x4 rx{}, rw{};
   auto point = [&]() {
     if (lr < rounds) {
       const Place p = place(lr);
+      left = p.n;
+      k0 = (unsigned)(OUT == PARTS ? p.from : turn) * (WT_K * 2);
       rx = wt_rsrc(x + p.m0 * xs, ((unsigned)min(WT_ROWS, M - p.m0) - 1) *
                                           (unsigned)xs * 2 + (unsigned)K * 2);
-      rw = wt_rsrc(w + (long)p.n0 * K, (unsigned)(2 * N - p.n0) * (unsigned)K * 2);
+      rw = wt_rsrc(w + (long)p.n0 * K, (unsigned)(WN - p.n0) * (unsigned)K * 2);
     } else {
+      left = steps;
+      k0 = 0;
       rx[2] = rw[2] = 0;
     }
   };
   auto advance = [&]() {
-    if (++lk == n) {
-      lk = 0;
+    k0 += WT_K * 2;
+    if (OUT == SILU && k0 == (unsigned)K * 2) k0 = 0;
+    if (--left == 0) {
       ++lr;
       point();
     }
@@ -105,7 +141,7 @@ __global__ __launch_bounds__(256, 1) void wide_silu_kernel(
   auto load = [&](unsigned at, unsigned off, const i32x4& rs) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
                  "buffer_load_dwordx4 %1, %2, %3 offen lds"
-                 ::"s"(at), "v"(off), "s"(rs), "s"(lk * (WT_K * 2))
+                 ::"s"(at), "v"(off), "s"(rs), "s"(k0)
                  : "m0", "memory");
   };
   point();
@@ -137,7 +173,6 @@ __global__ __launch_bounds__(256, 1) void wide_silu_kernel(
   auto half = [&](auto h, const unsigned short* rn, const unsigned short* wnx,
                   const i32x4& rs, unsigned dst, const unsigned* off) {
     constexpr int H = decltype(h)::value;
-    const unsigned k0 = lk * (WT_K * 2);
 #pragma unroll
     for (int i = 0; i < 64; ++i) {
       const int a = i / 8, b = i % 8;
@@ -172,8 +207,9 @@ __global__ __launch_bounds__(256, 1) void wide_silu_kernel(
 #pragma unroll
       for (int b = 0; b < 8; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
     asm volatile("s_nop 7" ::: "memory");
+    const Place p = place(round);
 #pragma unroll 1
-    for (int s = 0; s < n; ++s) {
+    for (int s = 0; s < p.n; ++s) {
       const int next = bw == 2 ? 0 : bw + 1, over = bw == 0 ? 2 : bw - 1;
       half(wt_int<0>{}, rl + bx * WT_BUF + at1, wl + bw * WT_BUF + at1, rw,
            to + (2 + over) * WT_BYTES, ow);
@@ -194,32 +230,46 @@ __global__ __launch_bounds__(256, 1) void wide_silu_kernel(
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
 
     // acc[a][b][j]: column 4 lg + j of tile b, row lc of tile a
-    const Place p = place(round);
+    constexpr unsigned SIZE = OUT == PARTS ? 4 : 2;
     const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
-        out + (long)p.m0 * N + p.n0, 0,
-        ((unsigned)min(WT_ROWS, M - p.m0) - 1) * (unsigned)N * 2 +
-            (unsigned)min(COLS, N - p.n0) * 2,
+        (char*)out_ + (((long)p.part * M + p.m0) * N + p.n0) * SIZE, 0,
+        ((unsigned)min(WT_ROWS, M - p.m0) - 1) * (unsigned)N * SIZE +
+            (unsigned)min(COLS, N - p.n0) * SIZE,
         0x00020000);
-    unsigned row = (unsigned)(wm * 128 + lc) * (unsigned)N * 2;
+    unsigned row = (unsigned)(wm * 128 + lc) * (unsigned)N * SIZE;
     asm volatile("" : "+v"(row));           // not a register for every row
 #pragma unroll
     for (int a = 0; a < 8; ++a) {
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int b = 0; b < 4; b += 2) {
-        u32x4 o;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const f32x4 g = acc[a][b + j / 2], u = acc[a][b + 4 + j / 2];
-          const int e = j % 2 * 2;
-          o[j] = wt_pack(wt_silu(wt_sum(g[e]), wt_sum(u[e])),
-                         wt_silu(wt_sum(g[e + 1]), wt_sum(u[e + 1])));
-        }
+      for (int b = 0; b < HC / 16; b += 2) {
         // columns and rows beyond the result are not stored
-        const int col = wn * 64 + b * 16 + lg * 8;
-        const unsigned off = row + (unsigned)a * 32u * (unsigned)N + col * 2;
-        __builtin_amdgcn_raw_buffer_store_b128(
-            o, ro, p.n0 + col < N ? off : 0xffffff00u, 0, 0);
+        const int col = wn * HC + b * 16 + lg * 8;
+        const unsigned off = p.n0 + col < N ? row + (unsigned)a * 16u * SIZE * (unsigned)N +
+                                                  col * SIZE
+                                            : 0xffffff00u;
+        if constexpr (OUT == PARTS) {
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            u32x4 o;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              o[j] = __builtin_bit_cast(unsigned, wt_sum(acc[a][b + i][j]));
+            __builtin_amdgcn_raw_buffer_store_b128(
+                o, ro, p.n0 + col < N ? off + i * 16 : 0xffffff00u, 0, 0);
+          }
+        } else {
+          u32x4 o;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int e = j % 2 * 2;
+            const f32x4 g = acc[a][b + j / 2];
+            const f32x4 u = acc[a][b + 4 + j / 2];
+            o[j] = wt_pack(wt_silu(wt_sum(g[e]), wt_sum(u[e])),
+                           wt_silu(wt_sum(g[e + 1]), wt_sum(u[e + 1])));
+          }
+          __builtin_amdgcn_raw_buffer_store_b128(o, ro, off, 0, 0);
+        }
       }
     }
   }
@@ -229,15 +279,22 @@ __global__ __launch_bounds__(256, 1) void wide_silu_kernel(
 
 }  // namespace
 
-// x [M, K] of row stride xs; offsets inside a tile's operands are 32 bits of bytes
-void wide_silu_launch(void* out, const void* x, const void* w, int M, int N, int K,
-                      long xs, int* err_unsupported, hipStream_t s) {
-  const long far = 1l << 32;
+// x [M, K] of row stride xs; offsets inside a tile's operands are 32 bits of bytes.
+// splits 0: the activation of the product (w [2 N, K]), else the product in fp32 parts,
+// each of two steps of k or more.
+void wide_launch(void* out, const void* x, const void* w, int M, int N, int K, long xs,
+                 int splits, int* err_unsupported, hipStream_t s) {
+  const long far = 1l << 32, wn = splits == 0 ? 2l * N : N;
   *err_unsupported = K % WT_K != 0 || K < 2 * WT_K || N % 8 != 0 ||
-                     (2l * N + WT_ROWS) * K * 2 >= far ||
-                     (xs + K) * WT_ROWS * 2 >= far || 2l * N * (WT_ROWS + 1) >= far - 256;
+                     (wn + WT_ROWS) * K * 2 >= far || (xs + K) * WT_ROWS * 2 >= far ||
+                     4l * N * (WT_ROWS + 1) >= far - 256 || splits < 0 ||
+                     (splits > 0 && K / WT_K / splits < 2);
   if (*err_unsupported || M == 0 || N == 0) return;
-  hipLaunchKernelGGL(wide_silu_kernel, dim3(WT_CUS), dim3(256), 0, s,
-                     (unsigned short*)out, (const unsigned short*)x,
-                     (const unsigned short*)w, M, N, K, xs);
+#define WIDE(OUT)                                                               \
+  hipLaunchKernelGGL(wide_kernel<OUT>, dim3(WT_CUS), dim3(256), 0, s, out,      \
+                     (const unsigned short*)x, (const unsigned short*)w, M, N, K, xs, \
+                     splits)
+  if (splits == 0) WIDE(SILU);
+  else WIDE(PARTS);
+#undef WIDE
 }

@@ -69,6 +69,62 @@ def test_linear_silu_takes_it():
     _check(ops.linear_silu(x, w), x, w)
 
 
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")
+@pytest.mark.parametrize("M,N,K,parts,pad", [
+    (1, 8, 128, 1, 0), (257, 264, 64 * 17, 8, 8),     # parts of two and three steps
+    (300, 1000, 1024, 3, 0), (513, 520, 4096, 5, 0),
+    (2100, 2056, 64 * 11, 5, 64)])                    # 405 tiles: two a workgroup
+def test_product_in_parts(M, N, K, parts, pad):
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    x = torch.randn(M, K + pad, generator=g, device="cuda").bfloat16()[:, :K]
+    w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).bfloat16()
+    got = ops._load_hip().wide_parts(x, w, parts)
+    assert got.shape == (parts, M, N) and got.dtype == torch.float32
+    n = K // 64
+    for p in range(parts):
+        k = slice(n * p // parts * 64, n * (p + 1) // parts * 64)
+        a, b = x[:, k].double(), w[:, k].double().T.contiguous()
+        # fp32 sums, each off by 2^-24 of its terms' sizes a step at most
+        bound = torch.matmul(a.abs(), b.abs()) * (K * 2.0 ** -24) + 1e-30
+        assert bool(((got[p].double() - torch.matmul(a, b)).abs() <= bound).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")
+@pytest.mark.parametrize("M", [640, 1100])
+def test_the_norm_behind_adds_the_parts_up(M):
+    N, K = 4096, 11008
+    g = torch.Generator(device="cuda").manual_seed(M)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    x, res = rnd(M, K).bfloat16(), rnd(M, N).bfloat16()
+    w, nw = (rnd(N, K) * K ** -0.5).bfloat16(), rnd(N).bfloat16()
+    parts = ops.linear_auto(x, w, True)
+    assert parts.shape == (ops._wide_parts(M, N, K), M, N)
+    total = torch.matmul(x.double(), w.double().T.contiguous())
+    assert float((parts.double().sum(0) - total).abs().max()) < 1e-4
+    got, ref = ops.add_rms_norm(parts, res.clone(), nw, 1e-5), \
+        ops.add_rms_norm(parts.sum(0).bfloat16(), res.clone(), nw, 1e-5)
+    for a, b in zip(got, ref):
+        # the same but for the order of the parts' sum, half an ulp at a rounding
+        assert float(((a.float() - b.float()).abs()
+                      > b.float().abs() * 2.0 ** -7 + 2.0 ** -7).sum()) == 0
+
+
+@pytest.mark.parametrize("M", [257, 400, 512, 513, 700, 1024, 2048, 4000])
+@pytest.mark.parametrize("K", [4096, 7168, 8192, 11008, 14336])
+def test_parts_fill_the_workgroups_once(M, K):
+    for N in range(1024, 10752, 256):
+        parts = ops._wide_parts(M, N, K)
+        tiles = -(-M // 256) * -(-N // 256)
+        if parts:
+            assert K >= 7168 and 2 <= parts <= 8 and tiles * parts <= 256
+            assert M * N * parts * 4 <= 67 << 20          # bytes of the parts
+            assert K // 64 // parts >= 2
+    assert not ops._wide_parts(256, 4096, K)
+    assert not ops._wide_parts(1024, 4096, K + 32)
+
+
 @pytest.mark.parametrize("K", [1024, 2048, 4096, 8192])
 def test_rule_by_filled_rounds(K):
     """Full rounds are taken, rounds for the sake of a few tiles not."""
