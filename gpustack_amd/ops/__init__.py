@@ -8,6 +8,7 @@ engine/control-plane logic testable without hardware.
 """
 from __future__ import annotations
 
+import functools
 import math
 import os
 from pathlib import Path
@@ -698,7 +699,8 @@ def moe_wide_wins(rows: int, E: int, N: int, K: int, down: bool) -> bool:
 
 def linear_auto(x, w, parts: bool = False):
     """Shape-gated GEMM dispatch: the products for few rows
-    (_rows_tile_plan, _rows_gemm_wins), the split-K skinny kernel where it
+    (_rows_tile_plan, _rows_gemm_wins) and for many (_wide_parts,
+    _wide_rows_tile), the split-K skinny kernel where it
     measured faster than hipBLASLt (scripts/bench_skinny_gemm.py on MI355X:
     down_proj-like N=4096 K>=8192 M>=384 at splitk=4, 824 TF vs hipBLASLt 680),
     F.linear everywhere else. `parts`: a product that is cut over k may come
@@ -710,9 +712,14 @@ def linear_auto(x, w, parts: bool = False):
         M, K = x.shape
         N = w.shape[0]
         wide = _wide_parts(M, N, K) if parts else 0
-        if wide and _rows_take(x, w):
+        if wide and _wide_take(x, w):
             return _load_hip().wide_parts(x, w, wide)
         plan = parts and _parts_plan(M, N, K) or _rows_tile_plan(M, N, K)
+        wide = None if parts and plan and plan[1] > 1 else _wide_rows_tile(M, N, K)
+        if wide and _wide_take(x, w):
+            out = torch.empty(M, N, dtype=x.dtype, device=x.device)
+            _load_hip().wide_rows(out, x, w, *wide)
+            return out
         if (plan or _rows_gemm_wins(M, N, K)) and _rows_take(x, w):
             if parts and plan and plan[1] > 1:
                 return _load_hip().rows_tile_parts(x, w, *plan)
@@ -747,6 +754,12 @@ def _rows_take(x, w) -> bool:
             and not (x.requires_grad or w.requires_grad))
 
 
+def _wide_take(x, w) -> bool:
+    """Operands that the products of many rows take: _rows_take, and offsets inside
+    a tile's rows within 32 bits of bytes."""
+    return x.stride(0) <= 1 << 22 and _rows_take(x, w)
+
+
 def _silu_plan(M: int, N: int, K: int):
     """_rows_tile_plan of a product of N columns, gate and up, that ends in the
     activation, else None. Tiles of 64 columns bring 32 rows of each, which for
@@ -762,44 +775,87 @@ def _silu_plan(M: int, N: int, K: int):
     return plan
 
 
-def _wide_silu_wins(M: int, N: int, K: int) -> bool:
-    """Where the product of many rows that ends in the activation
-    (wide_kernel in ops/csrc/wide_tiles.hip) measured faster than the
-    library's product and the activation behind it; N columns, gate and up. Its
-    256 workgroups take tiles of 256 rows and 128 columns of the result in rounds,
-    so what decides is the share of its rounds' rows and columns that are filled;
-    short rows, of whose time the activation is more, want less of it. Of 1171
-    sizes (768 to 24576 columns of the result, 1024 to 8192 k, 136 to 8192 rows,
-    weights out of HBM) 438 are taken, two of them slower by more than 3 % (1280
-    rows of 11264 columns and 8192 k 1.06, 2048 of 11264 and 4096 1.04), .84 of the
-    other's time in the middle; 91 that would gain more than 5 % are not. us,
-    library and activation / this, 4096 k: 512 rows of 28672 105 / 94, 2048 381 /
-    355, 8192 1379 / 1282; 2048 of 22016 431 / 260; but 512 of 11264 57 / 72, and
-    640 of 28672, two rounds for one and a third, 146 / 164."""
-    if N % 16 != 0 or K % 64 != 0 or K < 128 or M <= 128 \
-            or (2 * N + 512) * K >= 1 << 31:
-        return False
-    tiles = -(-M // 256) * -(-N // 256)
-    filled = M * N / (-(-tiles // 256) * 256 * 256 * 256)
-    return filled >= (.5 if K <= 1024 else .6 if K <= 2048
-                      else .68 if K <= 4096 else .78)
+# Tiles of wide_kernel (ops/csrc/wide_tiles.hip), in 32 rows and 32 weight rows: us of
+# a round's end, of a round's step of 64 k, and what a step takes more where all 256
+# workgroups have a tile (the card's power). Fitted to 6600 sizes, off by 4 % of a time
+# on average (8 x 8) to 9 % (4 x 2); the tile of the least time by them costs .6 % more
+# than the best of them with the activation and 1.4 % without.
+_WIDE_TILES = {
+    (8, 8): (5.7, .92, .43), (8, 7): (6.2, .82, .37), (8, 6): (4.4, .73, .31),
+    (8, 5): (3.9, .67, .24), (8, 4): (3.1, .56, .22), (6, 8): (4.2, .77, .29),
+    (6, 6): (3.4, .65, .20), (4, 6): (2.1, .51, .17), (4, 4): (1.3, .38, .15),
+    (4, 2): (.4, .26, .10)}
+_WIDE_SILU = ((8, 8), (8, 7), (8, 6), (8, 5), (8, 4), (6, 8))
+_WIDE_ROWS = ((8, 8), (8, 7), (8, 6), (8, 4), (6, 8), (6, 6), (4, 6), (4, 4), (4, 2))
+
+
+def _wide_tile(M: int, N: int, K: int, tiles, base: float):
+    """The tile of the least time for N weight rows, where that is no more than the
+    library takes for its fixed part, `base`, its bytes at 6 TB/s and its products at
+    1250 TFLOP/s (the root of their squares), else None."""
+    if K % 64 != 0 or K < 128 or (N + 512) * K >= 1 << 31 \
+            or N >= 1 << 21 or M * max(N, K) >= 1 << 40:
+        return None
+
+    def time(tile):
+        end, step, full = _WIDE_TILES[tile]
+        n = -(-M // (32 * tile[0])) * -(-N // (32 * tile[1]))
+        rounds = -(-n // 256)
+        return 2 + end * rounds + K / 64 * (step * rounds + full * n / 256)
+
+    best = min(tiles, key=time)
+    moved = 2 * (N * K + M * (N + K)) / 6e6
+    return best if time(best) <= base + math.hypot(moved, 2 * M * N * K / 1250e6) \
+        else None
+
+
+@functools.lru_cache(maxsize=4096)
+def _wide_silu_tile(M: int, N: int, K: int):
+    """The tile of a product of many rows that ends in the activation, or None where
+    the library's product and the activation behind it are as good; N columns, gate
+    and up. Of 3927 sizes (1024 to 24576 columns of the result, 1024 to 8192 k, 136 to
+    8192 rows, weights out of HBM) 3016 are taken, one of them slower by more than 3 %
+    (.96), .79 of the other's time on average; 404 that would gain more than 5 % are
+    not. us, library and activation / this, 4096 k: 512 rows of 28672 108 / 93, 2039
+    411 / 337, 8192 1422 / 1286; 512 of 22016 99 / 80; but 136 of 16384 columns and
+    3072 k are left, .91."""
+    if N % 16 != 0 or M <= 128:
+        return None
+    return _wide_tile(M, N, K, _WIDE_SILU, 13)
+
+
+@functools.lru_cache(maxsize=4096)
+def _wide_rows_tile(M: int, N: int, K: int):
+    """The tile of a product of many rows, or None for the library. Whole tiles of 256
+    x 256 that fill their rounds are the library's too, and as often slower (.84 to 1.2
+    of its time): those are left to it, what fills smaller tiles better is taken. Of
+    2688 sizes (1024 to 24576 columns, 1024 to 14336 k, 264 to 8192 rows) 1529, 21 of
+    them slower by more than 3 % (768 rows of 18432 x 1024 the worst, 1.1), .84 of the
+    time of what took them before on average. us, before / this: 2039 rows of
+    6144x4096 84 / 75, of 4096x4096 62 / 56, 4188 of 5120x2048 82 / 77, of 2048x4096 65
+    / 58; but 512 of 4096x2560 and long rows of few columns (384 rows of 3584x7168 35 /
+    47) are left."""
+    if M <= 256 or N % 8 != 0:
+        return None
+    tile = _wide_tile(M, N, K, _WIDE_ROWS, 9)
+    return None if tile == (8, 8) else tile
 
 
 def linear_silu(x, w):
     """silu(gate) * up of the product with w = [gate rows; up rows], or None
     where the activation is a launch of its own: the tiled product of up to
     128 rows (_rows_tile_plan), not cut over k, and the one of many rows
-    (_wide_silu_wins) end in it."""
+    (_wide_silu_tile) end in it."""
     if not _own_products(x, w):
         return None
     M, K = x.shape
     plan = _silu_plan(M, w.shape[0], K)
-    wide = plan is None and _wide_silu_wins(M, w.shape[0], K)
-    if not (plan or wide) or not _rows_take(x, w):
+    wide = None if plan else _wide_silu_tile(M, w.shape[0], K)
+    if not (plan or wide) or not (_wide_take if wide else _rows_take)(x, w):
         return None
     out = torch.empty(M, w.shape[0] // 2, dtype=x.dtype, device=x.device)
     if wide:
-        _load_hip().wide_silu(out, x, w)
+        _load_hip().wide_rows(out, x, w, *wide, silu=True)
     else:
         _load_hip().rows_tile(out, x, w, *plan, silu=True)
     return out

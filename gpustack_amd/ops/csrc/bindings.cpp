@@ -39,7 +39,7 @@ bool w4_has(int, int);
 bool w4_cuts(int, int, int);
 bool w4_by_rows(int, int, int);
 bool w4_silu_wins(int, int, int);
-void wide_launch(void*, const void*, const void*, int, int, int, long, int, int*, hipStream_t);
+void wide_launch(int, void*, const void*, const void*, int, int, int, long, int, int, int, int*, hipStream_t);
 int w4_splits(int, int, int);
 void w4_parts_launch(float*, const void*, const void*, const void*, const void*, int, int, int, int, hipStream_t);
 void w4_silu_launch(void*, const void*, const void*, const void*, const void*, int, int, int, hipStream_t);
@@ -698,18 +698,21 @@ void check_wide(const at::Tensor& x, const at::Tensor& w) {
               w.size(0) < (1l << 30) && x.size(1) < (1l << 30), "wide shapes");
 }
 
-// out = silu(gate) * up of many rows, w holding the gate's rows and behind them the
-// up product's
-void wide_silu(at::Tensor out, at::Tensor x, at::Tensor w) {
+// out = x w^T of many rows in tiles of 32 rf x 32 cf; silu: silu(gate) * up, w holding
+// the gate's rows and behind them the up product's
+void wide_rows(at::Tensor out, at::Tensor x, at::Tensor w, int64_t rf, int64_t cf,
+               bool silu) {
   check_bf16(out, "out");
   check_wide(x, w);
   const long M = x.size(0), N = out.size(1), K = x.size(1);
-  TORCH_CHECK(out.dim() == 2 && out.size(0) == M && w.size(0) == 2 * N &&
-              (uintptr_t)out.data_ptr() % 16 == 0, "wide_silu shapes");
+  TORCH_CHECK(out.dim() == 2 && out.size(0) == M && w.size(0) == (silu ? 2 : 1) * N &&
+              (uintptr_t)out.data_ptr() % 16 == 0, "wide_rows shapes");
+  TORCH_CHECK(rf >= 0 && rf <= 9 && cf >= 0 && cf <= 9, "wide_rows tiles");
   int err = 0;
-  wide_launch(out.data_ptr(), x.data_ptr(), w.data_ptr(), (int)M, (int)N, (int)K,
-              x.stride(0), 0, &err, cur_stream(x));
-  TORCH_CHECK(!err, "wide_silu: unsupported M=", M, " N=", N, " K=", K);
+  wide_launch(silu ? 0 : 1, out.data_ptr(), x.data_ptr(), w.data_ptr(), (int)M, (int)N,
+              (int)K, x.stride(0), 1, (int)rf, (int)cf, &err, cur_stream(x));
+  TORCH_CHECK(!err, "wide_rows: unsupported M=", M, " N=", N, " K=", K, " tiles ", rf,
+              " x ", cf);
   HIP_CHECK_LAST();
 }
 
@@ -720,8 +723,8 @@ at::Tensor wide_parts(at::Tensor x, at::Tensor w, long splits) {
   TORCH_CHECK(splits >= 1 && splits <= K / 128, "wide_parts: parts of K=", K);
   at::Tensor parts = at::empty({splits, M, N}, x.options().dtype(at::kFloat));
   int err = 0;
-  wide_launch(parts.data_ptr(), x.data_ptr(), w.data_ptr(), (int)M, (int)N,
-              (int)K, x.stride(0), (int)splits, &err, cur_stream(x));
+  wide_launch(2, parts.data_ptr(), x.data_ptr(), w.data_ptr(), (int)M, (int)N, (int)K,
+              x.stride(0), (int)splits, 8, 8, &err, cur_stream(x));
   TORCH_CHECK(!err, "wide_parts: unsupported M=", M, " N=", N, " K=", K);
   HIP_CHECK_LAST();
   return parts;
@@ -913,8 +916,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("rows"), py::arg("tiles"), py::arg("ntiles"), py::arg("offs"),
         py::arg("counts"), py::arg("flat_w") = py::none(),
         py::arg("bias") = py::none(), py::arg("act_mode") = 0);
-  m.def("wide_silu", &wide_silu,
-        "silu(x Wg^T) * (x Wu^T) of many rows (bf16, f32 accum)");
+  m.def("wide_rows", &wide_rows,
+        "x W^T, or silu(x Wg^T) * (x Wu^T), of many rows (bf16, f32 accum)",
+        pybind11::arg("out"), pybind11::arg("x"), pybind11::arg("w"),
+        pybind11::arg("rf"), pybind11::arg("cf"), pybind11::arg("silu") = false);
   m.def("wide_parts", &wide_parts, "fp32 parts of a product of many rows");
   m.def("moe_gate_up_silu", &moe_gate_up_silu,
         py::arg("act"), py::arg("x"), py::arg("w"), py::arg("s_tok"),

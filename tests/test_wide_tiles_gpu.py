@@ -1,10 +1,10 @@
-"""The product of many rows that ends in silu(gate) * up, at the edges of its tiles
-(256 rows, 128 columns, steps of 64 k), and the rule that takes it."""
+"""Products of many rows, whole, ended in silu(gate) * up or in fp32 parts, at the edges
+of their tiles (32 rows and 32 weight rows times a tile's numbers, steps of 64 k), and
+the rules that take them."""
 import pytest
 import torch
 
 from gpustack_amd import ops
-
 
 
 def _operands(M, N, K, pad=0):
@@ -30,21 +30,43 @@ def _check(out, x, w):
     assert bool((err <= bound).all()), float((err - bound).max())
 
 
-@pytest.mark.parametrize("M,N,K,pad", [
+SIZES = [
     (1, 8, 128, 0),               # one row, one store of a lane
     (255, 120, 128, 8), (256, 128, 192, 0), (257, 136, 256, 64),
     (300, 1000, 64 * 7, 0), (513, 384, 4096, 0),
-    # two and three rounds of tiles: 9 x 33, 17 x 33
-    (2100, 4104, 128, 0), (4100, 4200, 192, 0)])
+    # two and three rounds of 256 x 256: 9 x 33, 17 x 33
+    (2100, 4104, 128, 0), (4100, 4200, 192, 0)]
+
+
+@pytest.mark.parametrize("M,N,K,pad", SIZES)
+@pytest.mark.parametrize("tile", ops._WIDE_SILU)
 @pytest.mark.gpu
 @pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")
-def test_product_ends_in_the_activation(M, N, K, pad):
+def test_product_ends_in_the_activation(M, N, K, pad, tile):
     x, w = _operands(M, N, K, pad)
     # rows beyond the result keep what they hold
     room = torch.full((M + 2, N), 7.0, device="cuda", dtype=torch.bfloat16)
-    ops._load_hip().wide_silu(room[1:M + 1], x, w)
+    ops._load_hip().wide_rows(room[1:M + 1], x, w, *tile, silu=True)
     assert bool((room[0] == 7).all()) and bool((room[M + 1] == 7).all())
     _check(room[1:M + 1], x, w)
+
+
+@pytest.mark.parametrize("M,N,K,pad", SIZES)
+@pytest.mark.parametrize("tile", [t for t in ops._WIDE_ROWS if t != (8, 8)])
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")
+def test_product(M, N, K, pad, tile):
+    x, w = _operands(M, N, K, pad)
+    w = w[:N]
+    room = torch.full((M + 2, N), 7.0, device="cuda", dtype=torch.bfloat16)
+    ops._load_hip().wide_rows(room[1:M + 1], x, w, *tile)
+    assert bool((room[0] == 7).all()) and bool((room[M + 1] == 7).all())
+    xd, wd = x.double(), w.double().T.contiguous()
+    ref = torch.matmul(xd, wd)
+    # an fp32 sum of K products, off by K 2^-24 of its terms' sizes at most, rounded
+    bound = torch.matmul(xd.abs(), wd.abs()) * (K * 2.0 ** -24) \
+        + ref.abs() * 2.0 ** -8 + 1e-30
+    assert bool(((room[1:M + 1].double() - ref).abs() <= bound).all())
 
 
 @pytest.mark.gpu
@@ -53,10 +75,12 @@ def test_refused_operands():
     x, w = _operands(256, 128, 128)
     out = torch.empty(256, 128, device="cuda", dtype=torch.bfloat16)
     hip = ops._load_hip()
-    for bad in (lambda: hip.wide_silu(out, x[:, :64], w[:, :64].contiguous()),
-                lambda: hip.wide_silu(out, x[:255], w),
-                lambda: hip.wide_silu(out, x.float(), w),
-                lambda: hip.wide_silu(out[:, :124], x, w[:248])):
+    for bad in (lambda: hip.wide_rows(out, x[:, :64], w[:, :64].contiguous(), 8, 8, True),
+                lambda: hip.wide_rows(out, x[:255], w, 8, 8, True),
+                lambda: hip.wide_rows(out, x.float(), w, 8, 8, True),
+                lambda: hip.wide_rows(out[:, :124], x, w[:248], 8, 8, True),
+                lambda: hip.wide_rows(out, x, w[:128], 8, 8),
+                lambda: hip.wide_rows(out, x, w, 8, 3, True)):
         with pytest.raises(RuntimeError):
             bad()
 
@@ -65,7 +89,7 @@ def test_refused_operands():
 @pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")
 def test_linear_silu_takes_it():
     x, w = _operands(512, 8192, 1024)
-    assert ops._wide_silu_wins(512, 16384, 1024)
+    assert ops._wide_silu_tile(512, 16384, 1024)
     _check(ops.linear_silu(x, w), x, w)
 
 
@@ -125,19 +149,47 @@ def test_parts_fill_the_workgroups_once(M, K):
     assert not ops._wide_parts(1024, 4096, K + 32)
 
 
-@pytest.mark.parametrize("K", [1024, 2048, 4096, 8192])
-def test_rule_by_filled_rounds(K):
-    """Full rounds are taken, rounds for the sake of a few tiles not."""
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")
+def test_linear_auto_takes_it():
+    x, w = _operands(2039, 2048, 4096)
+    assert ops._wide_rows_tile(2039, 4096, 4096)
+    got = ops.linear_auto(x, w)
+    ref = torch.matmul(x.double(), w.double().T.contiguous())
+    assert float((got.double() - ref).abs().max()) < 2.0 ** -8 * float(ref.abs().max())
+    # rows further apart than a tile's offsets reach are the library's
+    far = torch.empty((1 << 22) + 8192, device="cuda", dtype=torch.bfloat16) \
+        .as_strided((2, 4096), ((1 << 22) + 8, 1))
+    assert not ops._wide_take(far, w) and ops._wide_take(x, w)
+
+
+@pytest.mark.parametrize("rule,tiles", [(ops._wide_silu_tile, ops._WIDE_SILU),
+                                        (ops._wide_rows_tile, ops._WIDE_ROWS)])
+@pytest.mark.parametrize("K", [1024, 2048, 4096, 14336])
+def test_the_tile_fills_its_rounds(rule, tiles, K):
+    def filled(tile, M, N):
+        n = -(-M // (32 * tile[0])) * -(-N // (32 * tile[1]))
+        return M * N / (-(-n // 256) * 256 * 1024 * tile[0] * tile[1])
+
+    taken = 0
     for N in range(1024, 57345, 512):
-        cols = N // 2 / 128
-        for M in (129, 256, 512, 1000, 2048, 4096, 8192):
-            got = ops._wide_silu_wins(M, N, K)
-            tiles = -(-M // 256) * -(-int(cols * 128) // 128)
-            filled = M * (N // 2) / (256 * 128 * 256 * -(-tiles // 256))
-            assert got or filled < .8
-            assert not got or filled >= .5
-    assert not ops._wide_silu_wins(128, 28672, K)
-    assert not ops._wide_silu_wins(8192, 28672, K + 32)
-    assert not ops._wide_silu_wins(8192, 28672 + 8, K)
+        for M in (264, 512, 1000, 2048, 4096, 8192):
+            tile = rule(M, N, K)
+            taken += tile is not None
+            if tile:
+                assert tile in tiles
+                # no larger one that fills its rounds as well
+                assert all(filled(tile, M, N) > .93 * filled(t, M, N) for t in tiles
+                           if t[0] >= tile[0] and t[1] >= tile[1])
+            if rule is ops._wide_silu_tile and filled((8, 8), M, N) > .8 \
+                    and M * N > 1 << 23:
+                assert tile
+            if rule is ops._wide_rows_tile:
+                assert tile != (8, 8)
+    assert taken > 100
+    assert rule(8192, 28672 + 16, K)
+    assert rule(128, 28672, K) is None
+    assert rule(8192, 28672, K + 32) is None
+    assert rule(8192, 28672 + 4, K) is None
     # offsets inside the weights are 32 bits of bytes
-    assert not ops._wide_silu_wins(8192, 1 << 20, 8192)
+    assert rule(8192, 1 << 21, K) is None
