@@ -628,27 +628,6 @@ def _parts_plan(M: int, N: int, K: int):
     return 128, 3 if K % 4096 == 0 else 4
 
 
-def _wide_parts(M: int, N: int, K: int) -> int:
-    """Parts over k of a product of many rows whose consumer adds them up
-    (wide_kernel in ops/csrc/wide_tiles.hip), or 0. As many as let its 256
-    workgroups have one tile of 256 x 256 each, where three quarters of them are
-    filled, from 11008 k on half; with rows that _tall_tile_plan cuts from 14336 k
-    on. us with an RMS norm behind, weights out of HBM, before / so: 4096x14336 at
-    400 rows 69 / 63, 640 143 / 84, 1024 159 / 107, 2039 217 / 197; 8192x8192 at 512
-    84 / 75; 5120x11008 at 512 .71 of the time, 7168x7168 .88; 4096x7168 at 512 1.09
-    (not taken), 6144x4096 at 512 43 / 46. Of 994 sizes (2048 to 10240 columns, 4096
-    to 14336 k, 264 to 4000 rows) 417 are taken, two of them slower by 4 %, .83 of
-    the time on average."""
-    if M <= 256 or K < 7168 or K % 64 != 0 or N % 8 != 0 \
-            or (N + 512) * K >= 1 << 31:
-        return 0
-    parts = min(8, 256 // (-(-M // 256) * -(-N // 256)))
-    if parts < 2 or K < 14336 and M <= 512 and _tall_tile_plan(M, N, K):
-        return 0
-    filled = M * N * parts / (256 * 256 * 256)
-    return parts if filled >= (.75 if K < 11008 else .55) else 0
-
-
 def router_plan(T: int, E: int, H: int):
     """(columns of a tile, parts over k) of a router's product, whose parts the
     choice of the experts adds up, or None. us for both launches against a
@@ -699,8 +678,8 @@ def moe_wide_wins(rows: int, E: int, N: int, K: int, down: bool) -> bool:
 
 def linear_auto(x, w, parts: bool = False):
     """Shape-gated GEMM dispatch: the products for few rows
-    (_rows_tile_plan, _rows_gemm_wins) and for many (_wide_parts,
-    _wide_rows_tile), the split-K skinny kernel where it
+    (_rows_tile_plan, _rows_gemm_wins) and for many
+    (_wide_parts_plan, _wide_rows_tile), the split-K skinny kernel where it
     measured faster than hipBLASLt (scripts/bench_skinny_gemm.py on MI355X:
     down_proj-like N=4096 K>=8192 M>=384 at splitk=4, 824 TF vs hipBLASLt 680),
     F.linear everywhere else. `parts`: a product that is cut over k may come
@@ -711,9 +690,9 @@ def linear_auto(x, w, parts: bool = False):
     if _own_products(x, w):
         M, K = x.shape
         N = w.shape[0]
-        wide = _wide_parts(M, N, K) if parts else 0
+        wide = _wide_parts_plan(M, N, K) if parts else None
         if wide and _wide_take(x, w):
-            return _load_hip().wide_parts(x, w, wide)
+            return _load_hip().wide_parts(x, w, wide[1], *wide[0])
         plan = parts and _parts_plan(M, N, K) or _rows_tile_plan(M, N, K)
         wide = None if parts and plan and plan[1] > 1 else _wide_rows_tile(M, N, K)
         if wide and _wide_take(x, w):
@@ -787,6 +766,14 @@ _WIDE_TILES = {
     (4, 2): (.4, .26, .10)}
 _WIDE_SILU = ((8, 8), (8, 7), (8, 6), (8, 5), (8, 4), (6, 8))
 _WIDE_ROWS = ((8, 8), (8, 7), (8, 6), (8, 4), (6, 8), (6, 6), (4, 6), (4, 4), (4, 2))
+_WIDE_PARTS = ((8, 8), (8, 6), (8, 4), (6, 8), (6, 6), (4, 6), (4, 4))
+
+
+def _wide_time(M: int, N: int, K: int, tile, parts: int = 1) -> float:
+    end, step, full = _WIDE_TILES[tile]
+    n = -(-M // (32 * tile[0])) * -(-N // (32 * tile[1])) * parts
+    rounds = -(-n // 256)
+    return 2 + end * rounds + math.ceil(K / 64 / parts) * (step * rounds + full * n / 256)
 
 
 def _wide_tile(M: int, N: int, K: int, tiles, base: float):
@@ -797,16 +784,9 @@ def _wide_tile(M: int, N: int, K: int, tiles, base: float):
             or N >= 1 << 21 or M * max(N, K) >= 1 << 40:
         return None
 
-    def time(tile):
-        end, step, full = _WIDE_TILES[tile]
-        n = -(-M // (32 * tile[0])) * -(-N // (32 * tile[1]))
-        rounds = -(-n // 256)
-        return 2 + end * rounds + K / 64 * (step * rounds + full * n / 256)
-
-    best = min(tiles, key=time)
+    time, best = min((_wide_time(M, N, K, tile), tile) for tile in tiles)
     moved = 2 * (N * K + M * (N + K)) / 6e6
-    return best if time(best) <= base + math.hypot(moved, 2 * M * N * K / 1250e6) \
-        else None
+    return best if time <= base + math.hypot(moved, 2 * M * N * K / 1250e6) else None
 
 
 @functools.lru_cache(maxsize=4096)
@@ -822,6 +802,41 @@ def _wide_silu_tile(M: int, N: int, K: int):
     if N % 16 != 0 or M <= 128:
         return None
     return _wide_tile(M, N, K, _WIDE_SILU, 13)
+
+
+@functools.lru_cache(maxsize=4096)
+def _wide_parts_plan(M: int, N: int, K: int):
+    """(tile, parts over k) of a product of many rows whose consumer adds the parts up
+    (wide_kernel in ops/csrc/wide_tiles.hip), or None. As many parts as let its 256
+    workgroups have one tile each, at most 8, or half as many: the tile and the parts of
+    the least time with the parts' own bytes, where that is 3 % (up to 256 rows 5) less
+    than a whole product's; both with the norm behind, which reads 4 bytes a part and
+    element. Not below 2560 k, where a part is hardly more than its start, nor what
+    _tall_tile_plan cuts but for 14336 k of more than 2048 columns. us with an RMS norm behind, weights out of
+    HBM, before / so: 512 rows of 4096x4096 38 / 33, of 6144x4096 49 / 42, of 4096x14336
+    73 / 66, 264 of 4096x14336 64 / 53, 136 of 4096x4096 30 / 21, 640 of 4096x14336 143 /
+    84, 1024 159 / 107, 2039 217 / 197; but 1024 rows of 4096x4096 47 / 48. Of 2808
+    sizes (1024 to 10240 columns, 2560 to 14336 k, 136 to 4096 rows) 1640 are taken, 18
+    of them slower by more than 3 % (1536 rows of 5376x14336 the worst, 1.07), .86 of the
+    time on average."""
+    if M <= 128 or K < 2560 or K % 64 != 0 or N % 8 != 0 \
+            or (N + 512) * K >= 1 << 31 or N >= 1 << 21 \
+            or M <= 512 and (N <= 2048 or K < 14336) and _tall_tile_plan(M, N, K):
+        return None
+    out = M * N / 1e6
+    best = None
+    for tile in _WIDE_PARTS:
+        n = -(-M // (32 * tile[0])) * -(-N // (32 * tile[1]))
+        most = min(8, 256 // n, K // 128)
+        for parts in {most, -(-most // 2)}:
+            if parts >= 2:
+                plan = _wide_time(M, N, K, tile, parts) + parts * out, tile, parts
+                best = min(best or plan, plan)
+    behind = 10 + N * K / 20e6 + .85 * out
+    whole = min(_wide_time(M, N, K, tile) for tile in _WIDE_ROWS) + .3 * out
+    if best is None or best[0] + behind > (.97 if M > 256 else .95) * (whole + behind):
+        return None
+    return best[1:]
 
 
 @functools.lru_cache(maxsize=4096)

@@ -717,15 +717,18 @@ void wide_rows(at::Tensor out, at::Tensor x, at::Tensor w, int64_t rf, int64_t c
 }
 
 // fp32 parts [splits, M, N] of the product, not added up
-at::Tensor wide_parts(at::Tensor x, at::Tensor w, long splits) {
+at::Tensor wide_parts(at::Tensor x, at::Tensor w, int64_t splits, int64_t rf,
+                      int64_t cf) {
   check_wide(x, w);
+  TORCH_CHECK(rf >= 0 && rf <= 9 && cf >= 0 && cf <= 9, "wide_parts tiles");
   const long M = x.size(0), N = w.size(0), K = x.size(1);
   TORCH_CHECK(splits >= 1 && splits <= K / 128, "wide_parts: parts of K=", K);
   at::Tensor parts = at::empty({splits, M, N}, x.options().dtype(at::kFloat));
   int err = 0;
   wide_launch(2, parts.data_ptr(), x.data_ptr(), w.data_ptr(), (int)M, (int)N, (int)K,
-              x.stride(0), (int)splits, 8, 8, &err, cur_stream(x));
-  TORCH_CHECK(!err, "wide_parts: unsupported M=", M, " N=", N, " K=", K);
+              x.stride(0), (int)splits, (int)rf, (int)cf, &err, cur_stream(x));
+  TORCH_CHECK(!err, "wide_parts: unsupported M=", M, " N=", N, " K=", K, " tiles ", rf,
+              " x ", cf);
   HIP_CHECK_LAST();
   return parts;
 }
@@ -918,9 +921,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("bias") = py::none(), py::arg("act_mode") = 0);
   m.def("wide_rows", &wide_rows,
         "x W^T, or silu(x Wg^T) * (x Wu^T), of many rows (bf16, f32 accum)",
-        pybind11::arg("out"), pybind11::arg("x"), pybind11::arg("w"),
-        pybind11::arg("rf"), pybind11::arg("cf"), pybind11::arg("silu") = false);
-  m.def("wide_parts", &wide_parts, "fp32 parts of a product of many rows");
+        py::arg("out"), py::arg("x"), py::arg("w"), py::arg("rf"), py::arg("cf"),
+        py::arg("silu") = false);
+  m.def("wide_parts", &wide_parts, "fp32 parts of a product of many rows",
+        py::arg("x"), py::arg("w"), py::arg("splits"), py::arg("rf"), py::arg("cf"));
   m.def("moe_gate_up_silu", &moe_gate_up_silu,
         py::arg("act"), py::arg("x"), py::arg("w"), py::arg("s_tok"),
         py::arg("offs"), py::arg("counts"), py::arg("bias") = py::none(),

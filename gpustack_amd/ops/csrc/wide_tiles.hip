@@ -34,8 +34,8 @@
 // whole tiles of 256 x 256 fill the rounds it is the library's own tile, .91 to 1.1 of
 // its time.
 // Products whose consumer adds fp32 parts up fill the workgroups cut over k: with an RMS
-// norm behind, 4096 x 14336 at 512 rows 69 us (before 73), 640 84 (143), 1024 107 (159),
-// 2039 197 (217).
+// norm behind, 4096 x 14336 at 512 rows 66 us (before 73), 640 84 (143), 1024 107 (159),
+// 2039 197 (217); 512 rows of 6144 x 4096 42 (49), of 4096 x 4096 33 (38).
 #include "wide_tiles.h"
 
 namespace {
@@ -349,7 +349,8 @@ void wide_launch(int kind, void* out, const void* x, const void* w, int M, int N
     WIDE(SILU, 8, 4); WIDE(SILU, 6, 8);
     WIDE(ROWS, 8, 7); WIDE(ROWS, 8, 6); WIDE(ROWS, 8, 4); WIDE(ROWS, 6, 8);
     WIDE(ROWS, 6, 6); WIDE(ROWS, 4, 6); WIDE(ROWS, 4, 4); WIDE(ROWS, 4, 2);
-    WIDE(PARTS, 8, 8);
+    WIDE(PARTS, 8, 8); WIDE(PARTS, 8, 6); WIDE(PARTS, 8, 4); WIDE(PARTS, 6, 8);
+    WIDE(PARTS, 6, 6); WIDE(PARTS, 4, 6); WIDE(PARTS, 4, 4);
 #undef WIDE
     default: *err_unsupported = 1;
   }

@@ -95,15 +95,16 @@ def test_linear_silu_takes_it():
 
 @pytest.mark.gpu
 @pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")
+@pytest.mark.parametrize("tile", ops._WIDE_PARTS)
 @pytest.mark.parametrize("M,N,K,parts,pad", [
     (1, 8, 128, 1, 0), (257, 264, 64 * 17, 8, 8),     # parts of two and three steps
     (300, 1000, 1024, 3, 0), (513, 520, 4096, 5, 0),
-    (2100, 2056, 64 * 11, 5, 64)])                    # 405 tiles: two a workgroup
-def test_product_in_parts(M, N, K, parts, pad):
+    (2100, 2056, 64 * 11, 5, 64)])                    # two tiles a workgroup and more
+def test_product_in_parts(M, N, K, parts, pad, tile):
     g = torch.Generator(device="cuda").manual_seed(M + N)
     x = torch.randn(M, K + pad, generator=g, device="cuda").bfloat16()[:, :K]
     w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).bfloat16()
-    got = ops._load_hip().wide_parts(x, w, parts)
+    got = ops._load_hip().wide_parts(x, w, parts, *tile)
     assert got.shape == (parts, M, N) and got.dtype == torch.float32
     n = K // 64
     for p in range(parts):
@@ -116,15 +117,15 @@ def test_product_in_parts(M, N, K, parts, pad):
 
 @pytest.mark.gpu
 @pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")
-@pytest.mark.parametrize("M", [640, 1100])
-def test_the_norm_behind_adds_the_parts_up(M):
-    N, K = 4096, 11008
+@pytest.mark.parametrize("M,N,K", [(136, 4096, 4096), (512, 6144, 4096),
+                                   (640, 4096, 11008), (1100, 4096, 11008)])
+def test_the_norm_behind_adds_the_parts_up(M, N, K):
     g = torch.Generator(device="cuda").manual_seed(M)
     rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
     x, res = rnd(M, K).bfloat16(), rnd(M, N).bfloat16()
     w, nw = (rnd(N, K) * K ** -0.5).bfloat16(), rnd(N).bfloat16()
     parts = ops.linear_auto(x, w, True)
-    assert parts.shape == (ops._wide_parts(M, N, K), M, N)
+    assert parts.shape == (ops._wide_parts_plan(M, N, K)[1], M, N)
     total = torch.matmul(x.double(), w.double().T.contiguous())
     assert float((parts.double().sum(0) - total).abs().max()) < 1e-4
     got, ref = ops.add_rms_norm(parts, res.clone(), nw, 1e-5), \
@@ -135,18 +136,23 @@ def test_the_norm_behind_adds_the_parts_up(M):
                       > b.float().abs() * 2.0 ** -7 + 2.0 ** -7).sum()) == 0
 
 
-@pytest.mark.parametrize("M", [257, 400, 512, 513, 700, 1024, 2048, 4000])
-@pytest.mark.parametrize("K", [4096, 7168, 8192, 11008, 14336])
+@pytest.mark.parametrize("M", [129, 257, 400, 512, 513, 700, 1024, 2048, 4000])
+@pytest.mark.parametrize("K", [2048, 2560, 4096, 7168, 8192, 11008, 14336])
 def test_parts_fill_the_workgroups_once(M, K):
+    taken = 0
     for N in range(1024, 10752, 256):
-        parts = ops._wide_parts(M, N, K)
-        tiles = -(-M // 256) * -(-N // 256)
-        if parts:
-            assert K >= 7168 and 2 <= parts <= 8 and tiles * parts <= 256
+        plan = ops._wide_parts_plan(M, N, K)
+        if plan:
+            tile, parts = plan
+            tiles = -(-M // (32 * tile[0])) * -(-N // (32 * tile[1]))
+            assert K >= 2560 and 2 <= parts <= 8 and tiles * parts <= 256
+            assert tile in ops._WIDE_PARTS and K // 64 // parts >= 2
             assert M * N * parts * 4 <= 67 << 20          # bytes of the parts
-            assert K // 64 // parts >= 2
-    assert not ops._wide_parts(256, 4096, K)
-    assert not ops._wide_parts(1024, 4096, K + 32)
+            taken += 1
+    assert taken or K < 4096 or M == 4000
+    assert not ops._wide_parts_plan(128, 4096, K)
+    assert not ops._wide_parts_plan(512, 4096, K + 32)
+    assert not ops._wide_parts_plan(512, 4100, K)
 
 
 @pytest.mark.gpu
