@@ -812,13 +812,13 @@ def _wide_parts_plan(M: int, N: int, K: int):
     the least time with the parts' own bytes, where that is 3 % (up to 256 rows 5) less
     than a whole product's; both with the norm behind, which reads 4 bytes a part and
     element. Not below 2560 k, where a part is hardly more than its start, nor what
-    _tall_tile_plan cuts but for 14336 k of more than 2048 columns. us with an RMS norm behind, weights out of
-    HBM, before / so: 512 rows of 4096x4096 38 / 33, of 6144x4096 49 / 42, of 4096x14336
-    73 / 66, 264 of 4096x14336 64 / 53, 136 of 4096x4096 30 / 21, 640 of 4096x14336 143 /
-    84, 1024 159 / 107, 2039 217 / 197; but 1024 rows of 4096x4096 47 / 48. Of 2808
-    sizes (1024 to 10240 columns, 2560 to 14336 k, 136 to 4096 rows) 1640 are taken, 18
-    of them slower by more than 3 % (1536 rows of 5376x14336 the worst, 1.07), .86 of the
-    time on average."""
+    _tall_tile_plan cuts but for 14336 k of more than 2048 columns. us with an RMS norm
+    behind, weights out of HBM, before / so: 512 rows of 4096x4096 38 / 33, of 6144x4096
+    49 / 42, of 4096x14336 73 / 66, 264 of 4096x14336 64 / 53, 136 of 4096x4096 30 / 21,
+    640 of 4096x14336 143 / 84, 1024 159 / 107, 2039 217 / 197; but 1024 rows of
+    4096x4096 47 / 48. Of 2808 sizes (1024 to 10240 columns, 2560 to 14336 k, 136 to 4096
+    rows) 1352 are taken, 12 of them slower by more than 3 % (1536 rows of 5376x14336
+    the worst, 1.08), .85 of the time on average."""
     if M <= 128 or K < 2560 or K % 64 != 0 or N % 8 != 0 \
             or (N + 512) * K >= 1 << 31 or N >= 1 << 21 \
             or M <= 512 and (N <= 2048 or K < 14336) and _tall_tile_plan(M, N, K):

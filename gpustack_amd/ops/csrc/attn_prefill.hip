@@ -404,13 +404,29 @@ void flash_prefill_kernel(
 // 480 us (822 -> 1091 TFLOP/s), 2039 rows behind 6001 301 -> 233 (1007), 32 x 256
 // 60 -> 52, 77 rows 8.8 -> 7.1, 33 rows behind 1000 38 -> 23, one row 5.7 -> 4.5.
 // Eight waves on 256 rows: 493 and 238. An order of the instructions given with
-// sched_group_barrier: 486 to 547.
+// sched_group_barrier: 486 to 547. Of the long prompt the matrix cores are 58 % busy, at
+// the 1.75 GHz that the card's power leaves. One wave a SIMD on 64 rows, which reads half
+// as much from the LDS: 521; alone it issues an instruction every 5.5 cycles.
 typedef __attribute__((ext_vector_type(4))) short s16x4;
 
 DEVICE_INLINE u32x2 lds_read_tr(const unsigned short* p) {
   return __builtin_bit_cast(
       u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
                  (__attribute__((address_space(3))) s16x4*)p));
+}
+
+// The tile of this workgroup, two of which run on a CU. The tiles with the most keys
+// start first; but where one launch fills the chip no more than twice over, workgroups i
+// and 256 + i share a CU from the start to the end: the first 256 then begin with the
+// smallest of them, next to the largest of the others. us, largest first / so: 32 heads,
+// two prompts of 1024 rows 34.5 / 29.4, four of 512 22.8 / 20.5, one of 2039 48.1 / 47.2
+// (behind 6001 245 / 238, 2048 behind 2000 113 / 108), 16 heads, 4000 rows 85.4 / 83.8,
+// 8 heads, 7999 158 / 155. Heads that do not divide 256 gain or lose by the list (28
+// heads, 2039 rows 45.4 / 43.9, three prompts of 700 24.6 / 26.0) and stay.
+DEVICE_INLINE int tile_of(int Hq) {
+  const int n = gridDim.x / Hq, at = blockIdx.x / Hq, chip = 256 / Hq;
+  const bool twice = 256 % Hq == 0 && n > chip && n <= 2 * chip;
+  return twice && at < chip ? n - chip + at : n - 1 - at;
 }
 
 template <bool PAGED>
@@ -433,7 +449,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void flash_rows_kernel(
 
   int qh = blockIdx.x % Hq;
   if (Hq % 8 == 0) qh = (qh % 8) * (Hq / 8) + qh / 8;
-  const int tile = (gridDim.x - 1 - blockIdx.x) / Hq;
+  const int tile = tile_of(Hq);
   const int kvh = qh / (Hq / Hkv);
   const int row0 = tile_start[tile];
   const int q0 = tile_q0[tile];

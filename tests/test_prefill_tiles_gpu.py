@@ -265,3 +265,12 @@ def test_keys_wider_than_values(monkeypatch, lens):
         r = slice(at, at + n)
         _check_variant(out[r], q[r], k[r], v[r], 0, scale, None, 0, 0.0)
         at += n
+
+
+# launches of one tile more than the chip takes at a time, of twice as many and one more
+# (256 workgroups, a tile is one a head), whose tiles start in another order
+@pytest.mark.parametrize("Hq,Hkv,lens", [
+    (32, 8, [1025]), (32, 8, [700, 1, 1200]), (32, 8, [2048]), (32, 8, [2049]),
+    (64, 8, [513]), (64, 8, [500, 500]), (16, 2, [4100]), (28, 4, [1300])])
+def test_every_tile_of_a_launch_that_fills_the_chip(Hq, Hkv, lens):
+    test_whole_prompts(Hq, Hkv, lens)
