@@ -1296,11 +1296,20 @@ def paged_attention(out, q, k_cache, v_cache, block_tables, row_seq, positions,
         if chunk > 0:
             span = min(span, chunk)
         if span >= 512 and 0 < nt < 2048:
-            # 1024 workgroups, or up to 2048 while the split stays <= 4 (a
-            # wider split pays more for the merge than it gains in
-            # occupancy), each of at least 128 keys
-            nsplit = max(1, min(16, span // 128,
-                                max(1024 // nt, min(4, 2048 // nt))))
+            if (q.shape[-1] == 128 and 64 < out.shape[-1] <= 128
+                    and q.dtype == torch.bfloat16):
+                # paged_attn_waves_kernel: one workgroup a CU, each of at least 256
+                # keys; more parts only cost their merge. us at 1 / 2 / 4 / 8, 16
+                # heads on 4: 64 rows in a window of 1024 26 / 31 / 36 / 42, 16 rows
+                # 19.4 / 16.9 / 16.5 / 19.0, 8 rows behind 200 to 3000 keys 38 / 26 /
+                # 20 / 19, one behind 1000 16.0 / 13.3 / 11.5 / 12.2
+                nsplit = max(1, min(16, -(-span // 256), 256 // nt))
+            else:
+                # 1024 workgroups, or up to 2048 while the split stays <= 4 (a
+                # wider split pays more for the merge than it gains in
+                # occupancy), each of at least 128 keys
+                nsplit = max(1, min(16, span // 128,
+                                    max(1024 // nt, min(4, 2048 // nt))))
         k.paged_attention(out, q, k_cache, v_cache, block_tables, tiles,
                           positions, scale, maps, window, keep_first, sinks,
                           exact, nsplit, slopes, softcap, chunk, gate)

@@ -36,7 +36,8 @@
 // wave w multiplies the 16 pairs with keys 16w..16w+15 (B operand straight
 // from the key pool, 16 B per lane), scores meet in LDS for the online
 // softmax, then wave w owns the output channels of n-tiles w, w+4, ... and
-// multiplies P (A operand, LDS) with the transposed value pages. With few
+// multiplies P (A operand, LDS) with the transposed value pages; heads of 128
+// channels have a kernel of their own (paged_attn_waves_kernel). With few
 // tiles over long contexts (decode) gridDim.y workgroups split a tile's
 // keys and a merge kernel joins the partial (acc, m, l) triples. The exact
 // path keeps everything fp32 on the vector ALUs, for pools of bf16 or fp32
@@ -313,13 +314,8 @@ constexpr int MKT = 64;            // keys per tile (16 per wave)
 constexpr int MSS = MKT + 4;       // fp32 score row stride
 constexpr int MPS = MKT + 8;       // bf16 weight row stride (16 B aligned)
 
-// NT: 16-channel n-tiles per wave (wave w owns n-tiles w, w+4, ...). DK: D / 32,
-// or 0 for any D. With DK a tile's values are asked for before its scores and
-// the next tile's keys, whose pages are known by then, behind them, so that a
-// tile waits for neither: 64 rows of 16 heads on 4 behind 200 to 3000 keys, with
-// the merge, in a window of 1024 36 -> 30 us, without one 67 -> 48, one row behind
-// 1000 16 -> 14.
-template <int NT, typename TO, int DK>
+// NT: 16-channel n-tiles per wave (wave w owns n-tiles w, w+4, ...).
+template <int NT, typename TO>
 __global__ __launch_bounds__(THREADS) void paged_attn_mfma_kernel(
     TO* __restrict__ out, const unsigned short* __restrict__ q,
     const unsigned short* __restrict__ k_cache,
@@ -388,63 +384,18 @@ __global__ __launch_bounds__(THREADS) void paged_attn_mfma_kernel(
   auto value_page = [&](int key, long blk) {
     return v_cache + (blk * p.G + g) * (long)VW * BS + (key & 15);
   };
-  u16x8 kreg[DK > 0 ? DK : 1], vreg[2][NT];
-  long vblk[2] = {0, 0};
-  const int v_begin = split * per;
-  if constexpr (DK > 0) {
-    if (v_begin < v_end) {
-      const int k0 = walk.tile(v_begin) * MKT;
-      const unsigned short* rowp = key_row(k0, page_at((k0 >> 4) + wave));
-#pragma unroll
-      for (int r = 0; r < DK; ++r)
-        kreg[r] = *reinterpret_cast<const u16x8*>(rowp + r * 32);
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks)
-        vblk[ks] = page_at((k0 + ks * 32 + lg * 8) >> 4);
-    }
-  }
-  for (int v = v_begin; v < v_end; ++v) {
+  for (int v = split * per; v < v_end; ++v) {
     const int k0 = walk.tile(v) * MKT;
     __syncthreads();   // Ql staged / previous tile's Pl and als consumed
     {
       const unsigned short* qrow = Ql + lc * QS;
       f32x4 sacc{0.f, 0.f, 0.f, 0.f};
-      if constexpr (DK > 0) {
-        const int kn = walk.tile(min(v + 1, v_end - 1)) * MKT;
-        const long kblk = page_at((kn >> 4) + wave);
-        long vnext[2];
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-          vnext[ks] = page_at((kn + ks * 32 + lg * 8) >> 4);
-          const unsigned short* pt =
-              value_page(k0 + ks * 32 + lg * 8, vblk[ks]);
-#pragma unroll
-          for (int i = 0; i < NT; ++i)
-            if ((wave + 4 * i) * 16 < VW)
-              vreg[ks][i] = *reinterpret_cast<const u16x8*>(
-                  pt + (long)((wave + 4 * i) * 16 + lc) * BS);
-        }
-#pragma unroll
-        for (int r = 0; r < DK; ++r)
-          sacc = ra_mfma(
-              *reinterpret_cast<const u16x8*>(qrow + r * 32 + lg * 8), kreg[r],
-              sacc);
-        if (v + 1 < v_end) {
-          const unsigned short* rowp = key_row(kn, kblk);
-#pragma unroll
-          for (int r = 0; r < DK; ++r)
-            kreg[r] = *reinterpret_cast<const u16x8*>(rowp + r * 32);
-        }
-        vblk[0] = vnext[0];
-        vblk[1] = vnext[1];
-      } else {
-        const unsigned short* rowp = key_row(k0, page_at((k0 >> 4) + wave));
+      const unsigned short* rowp = key_row(k0, page_at((k0 >> 4) + wave));
 #pragma unroll 4
-        for (int r = 0; r < D; r += 32) {
-          const u16x8 a = *reinterpret_cast<const u16x8*>(qrow + r + lg * 8);
-          const u16x8 b = *reinterpret_cast<const u16x8*>(rowp + r);
-          sacc = ra_mfma(a, b, sacc);
-        }
+      for (int r = 0; r < D; r += 32) {
+        const u16x8 a = *reinterpret_cast<const u16x8*>(qrow + r + lg * 8);
+        const u16x8 b = *reinterpret_cast<const u16x8*>(rowp + r);
+        sacc = ra_mfma(a, b, sacc);
       }
 #pragma unroll
       for (int r = 0; r < 4; ++r)
@@ -498,15 +449,12 @@ __global__ __launch_bounds__(THREADS) void paged_attn_mfma_kernel(
         const u16x8 a =
             *reinterpret_cast<const u16x8*>(Pl + lc * MPS + ks + lg * 8);
         const int keyb = k0 + ks + lg * 8;
-        const unsigned short* pt =
-            DK > 0 ? nullptr : value_page(keyb, page_at(keyb >> 4));
+        const unsigned short* pt = value_page(keyb, page_at(keyb >> 4));
 #pragma unroll
         for (int i = 0; i < NT; ++i) {
           const int ch = (wave + 4 * i) * 16 + lc;
           if ((wave + 4 * i) * 16 < VW) {       // uniform over the wave
-            u16x8 b;
-            if constexpr (DK > 0) b = vreg[ks / 32][i];
-            else b = *reinterpret_cast<const u16x8*>(pt + (long)ch * BS);
+            const u16x8 b = *reinterpret_cast<const u16x8*>(pt + (long)ch * BS);
             acc[i] = ra_mfma(a, b, acc[i]);
           }
         }
@@ -545,6 +493,203 @@ __global__ __launch_bounds__(THREADS) void paged_attn_mfma_kernel(
     for (int i = 0; i < NT; ++i) {
       const int ch = (wave + 4 * i) * 16 + lc;
       if (ch < VW) stf(op + ch, acc[i][r] * inv);
+    }
+  }
+}
+
+// Heads of 128 channels on values of 80 to 128: every wave takes keys of its own, 32
+// at a time, with a maximum and a sum of its own, and the four meet once, at the end,
+// so that nothing waits at a barrier and a wave's next keys and these values (16 KB)
+// are under way all the time. S^T = K Q^T in an order of the key rows (key_at) in which
+// a lane's 8 weights of 32 keys are neighbours, as the value pages hold them: the
+// weights stay in its registers. Bound by memory: 64 rows of 16 heads on 4 behind 200 to
+// 3000 keys 55 us (230 MB), in a window of 1024 26 (121 MB; a workgroup to a tile of 64
+// keys, its scores and weights through the LDS with three barriers, 63 and 34), 256 rows
+// behind 100 to 1500 100 (117), 16 in the window 16 (19), one behind 7000 21 (26).
+template <typename TO>
+__global__ __launch_bounds__(THREADS, 2) void paged_attn_waves_kernel(
+    TO* __restrict__ out, const unsigned short* __restrict__ q,
+    const unsigned short* __restrict__ k_cache,
+    const unsigned short* __restrict__ v_cache, AttnArgs p,
+    float* __restrict__ ws_acc, float* __restrict__ ws_ml) {
+  constexpr int BS = 16, D = 128, DK = D / 32, VT = 8, WKT = 32, QS = D + 8;
+  constexpr int OS = D + 4;                           // fp32 row of the sums
+  __shared__ __attribute__((aligned(16))) unsigned short Ql[G16 * QS];
+  __shared__ __attribute__((aligned(16))) float os[4][G16 * OS];
+  __shared__ float ms[4][G16], ls[4][G16];
+  __shared__ int e_pos[G16], e_lo[G16], e_row[G16], e_a[G16];
+
+  int n_ent, seq, g, koff;
+  if (!tile_setup(p, blockIdx.x, e_pos, e_lo, e_row, e_a, n_ent, seq, g, koff))
+    return;
+  __syncthreads();
+  const int VW = p.VW;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lc = lane & 15, lg = lane >> 4;
+  int jmax = -1, lo = 1 << 30;
+#pragma unroll
+  for (int e = 0; e < G16; ++e) {
+    jmax = max(jmax, e_pos[e]);
+    lo = min(lo, e_lo[e]);
+  }
+  jmax = __builtin_amdgcn_readfirstlane(jmax);
+  lo = __builtin_amdgcn_readfirstlane(lo);
+  for (int e = wave; e < G16; e += 4) {
+    const bool ok = e < n_ent;
+    const unsigned short* qp =
+        q + (long)e_row[e] * p.q_st + (long)e_a[e] * p.q_sa;
+    for (int r = lane; r < D; r += 64)
+      Ql[e * QS + r] = ok ? qp[r] : (unsigned short)0;
+  }
+  __syncthreads();
+  u16x8 qf[DK];
+#pragma unroll
+  for (int r = 0; r < DK; ++r)
+    qf[r] = *reinterpret_cast<const u16x8*>(Ql + lc * QS + r * 32 + lg * 8);
+
+  const int my_pos = e_pos[lc], my_lo = e_lo[lc];
+  const int nsplit = gridDim.y, split = blockIdx.y;
+  float m_run = -INFINITY, l_run = 0.f;               // l: of this lane's keys
+  if (p.sinks != nullptr && my_pos >= 0 && split == 0 && wave == 0) {
+    m_run = p.sinks[e_a[lc] / p.maps];
+    l_run = lg == 0 ? 1.f : 0.f;
+  }
+  const float slope = p.slopes != nullptr ? p.slopes[e_a[lc] / p.maps] : 0.f;
+  f32x4 acc[VT];                                      // channels 16 c + 4 lg .. of pair lc
+#pragma unroll
+  for (int c = 0; c < VT; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const int* bt = p.block_tables + (long)seq * p.maxb;
+  const int last_page = jmax >> 4;
+  const KeyWalk walk = key_walk(lo, jmax, p.keep_first, WKT);
+  const int part = split * 4 + wave, parts = nsplit * 4;
+  const int v_begin = (int)((long)walk.n * part / parts);
+  const int v_end = (int)((long)walk.n * (part + 1) / parts);
+  auto page_at = [&](int pg) {
+    return min(max(bt[min(pg, last_page)], 0), p.nblocks - 1);
+  };
+  // key of row lc of product t; keys past jmax re-read key jmax (their weights are 0)
+  auto key_at = [&](int t) { return (lc >> 2) * 8 + t * 4 + (lc & 3); };
+  u16x8 kreg[2][DK], vreg[VT];
+  auto keys = [&](int k0, int pg0, int pg1) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int key = min(k0 + key_at(t), jmax);
+      const long blk = lc >= 8 ? pg1 : pg0;
+      const unsigned short* rowp =
+          k_cache + ((blk * p.G + g) * BS + (key & 15)) * (long)p.KW + koff + lg * 8;
+#pragma unroll
+      for (int r = 0; r < DK; ++r)
+        kreg[t][r] = *reinterpret_cast<const u16x8*>(rowp + r * 32);
+    }
+  };
+  int pg0 = 0, pg1 = 0;                               // pages of the tile at hand
+  if (v_begin < v_end) {
+    const int k0 = walk.tile(v_begin) * WKT;
+    pg0 = page_at(k0 >> 4);
+    pg1 = page_at((k0 >> 4) + 1);
+    keys(k0, pg0, pg1);
+  }
+  for (int v = v_begin; v < v_end; ++v) {
+    const int k0 = walk.tile(v) * WKT;
+    const int kn = walk.tile(min(v + 1, v_end - 1)) * WKT;
+    const int nx0 = page_at(kn >> 4), nx1 = page_at((kn >> 4) + 1);
+    {
+      // 8 neighbouring keys of one page; those past jmax weigh nothing
+      const long blk = lg >= 2 ? pg1 : pg0;
+      const unsigned short* pt =
+          v_cache + (blk * p.G + g) * (long)VW * BS + (lg & 1) * 8 + lc * BS;
+#pragma unroll
+      for (int c = 0; c < VT; ++c)
+        if (c * 16 < VW) vreg[c] = *reinterpret_cast<const u16x8*>(pt + c * 16 * BS);
+    }
+    f32x4 s[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int r = 0; r < DK; ++r) s[t] = ra_mfma(kreg[t][r], qf[r], s[t]);
+    }
+    if (v + 1 < v_end) keys(kn, nx0, nx1);
+    pg0 = nx0;
+    pg1 = nx1;
+    float sv[8], mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int j = k0 + lg * 8 + i;
+      sv[i] = key_visible(j, my_pos, my_lo, p.keep_first)
+                  ? scaled_score(s[i >> 2][i & 3], p) - slope * (float)(my_pos - j)
+                  : -INFINITY;
+      mx = fmaxf(mx, sv[i]);
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE_SIZE));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE_SIZE));
+    const float m_new = fmaxf(m_run, mx);
+    const bool any = m_new != -INFINITY;
+    const float alpha = any ? __expf(m_run - m_new) : 1.f;
+    u16x8 w;
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float pv = any ? __expf(sv[i] - m_new) : 0.f;
+      w[i] = f2bf(pv);
+      sum += pv;
+    }
+    l_run = l_run * alpha + sum;
+    m_run = m_new;
+    if (__any(alpha != 1.f)) {
+#pragma unroll
+      for (int c = 0; c < VT; ++c)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[c][r] *= alpha;
+    }
+#pragma unroll
+    for (int c = 0; c < VT; ++c)
+      if (c * 16 < VW) acc[c] = ra_mfma(vreg[c], w, acc[c]);
+  }
+  l_run += __shfl_xor(l_run, 16, WAVE_SIZE);
+  l_run += __shfl_xor(l_run, 32, WAVE_SIZE);
+  if (lg == 0) {
+    ms[wave][lc] = m_run;
+    ls[wave][lc] = l_run;
+  }
+  if (lc < n_ent) {
+#pragma unroll
+    for (int c = 0; c < VT; ++c)
+      *reinterpret_cast<f32x4*>(&os[wave][lc * OS + c * 16 + lg * 4]) = acc[c];
+  }
+  __syncthreads();
+  for (int i = tid; i < n_ent * (D / 4); i += THREADS) {
+    const int e = i / (D / 4), ch = i % (D / 4) * 4;
+    if (ch >= VW) continue;
+    float M = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) M = fmaxf(M, ms[u][e]);
+    float L = 0.f;
+    f32x4 o{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (ms[u][e] != -INFINITY) {
+        const float f = __expf(ms[u][e] - M);
+        L += ls[u][e] * f;
+        const f32x4 x = *reinterpret_cast<const f32x4*>(&os[u][e * OS + ch]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[r] += x[r] * f;
+      }
+    if (nsplit > 1) {
+      const long slot = (long)blockIdx.x * nsplit + split;
+      if (ch == 0) {
+        ws_ml[(slot * G16 + e) * 2] = M;
+        ws_ml[(slot * G16 + e) * 2 + 1] = L;
+      }
+      *reinterpret_cast<f32x4*>(ws_acc + (slot * G16 + e) * VW + ch) = o;
+    } else {
+      const float inv = (L > 0.f ? 1.0f / L : 0.f) *
+                        head_gate_of<unsigned short>(p, e_row[e], e_a[e]);
+      TO* op = out + (long)e_row[e] * p.o_st + (long)e_a[e] * p.o_sa + ch;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) stf(op + r, o[r] * inv);
     }
   }
 }
@@ -918,12 +1063,18 @@ void launch_mfma(void* out, const void* q, const void* kc, const void* vc,
                  float* ws_ml, hipStream_t s) {
   const size_t smem = (size_t)G16 * (p.D + 8) * 2 + (size_t)G16 * MPS * 2 +
                       (size_t)(G16 * MSS + 2 * G16) * sizeof(float);
-  const auto kern = NT == 2 && p.D == 128
-                        ? paged_attn_mfma_kernel<NT, TO, NT == 2 ? 4 : 0>
-                        : paged_attn_mfma_kernel<NT, TO, 0>;
-  kern<<<dim3(ntiles, nsplit), THREADS, smem, s>>>(
-      (TO*)out, (const unsigned short*)q, (const unsigned short*)kc,
-      (const unsigned short*)vc, p, ws_acc, ws_ml);
+  bool alone = false;
+  if constexpr (NT == 2) {
+    alone = p.D == 128;
+    if (alone)
+      paged_attn_waves_kernel<TO><<<dim3(ntiles, nsplit), THREADS, 0, s>>>(
+          (TO*)out, (const unsigned short*)q, (const unsigned short*)kc,
+          (const unsigned short*)vc, p, ws_acc, ws_ml);
+  }
+  if (!alone)
+    paged_attn_mfma_kernel<NT, TO><<<dim3(ntiles, nsplit), THREADS, smem, s>>>(
+        (TO*)out, (const unsigned short*)q, (const unsigned short*)kc,
+        (const unsigned short*)vc, p, ws_acc, ws_ml);
   if (nsplit > 1)
     paged_attn_merge_kernel<TO><<<dim3(ntiles, G16), MERGE_THREADS, 0, s>>>(
         (TO*)out, p, ws_acc, ws_ml, nsplit);

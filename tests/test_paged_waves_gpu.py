@@ -1,0 +1,82 @@
+"""Paged attention of heads of 128 channels, a wave to its own 32 keys: contexts at the
+edges of the tiles and of the waves' shares, against the fp32 path, with every option of
+the two, and the number of parts that a batch takes."""
+import pytest
+import torch
+
+from gpustack_amd import ops
+
+gpu = [pytest.mark.gpu, pytest.mark.skipif(not torch.cuda.is_available(),
+                                           reason="needs a GPU")]
+
+
+def _run(hists, news, H, G, VW, nsplit, maps=1, fp32=False, **kw):
+    D, A = 128, H * maps
+    g = torch.Generator(device="cuda").manual_seed(sum(hists) + VW + nsplit)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    pages = [(h + n + 15) // 16 for h, n in zip(hists, news)]
+    kc, vc = (rnd(sum(pages) + 1, G, *s).bfloat16()
+              for s in ((16, maps * D), (VW, 16)))
+    bt = torch.zeros(len(hists), max(pages), dtype=torch.int32)
+    order = torch.randperm(sum(pages), generator=torch.Generator().manual_seed(1))
+    at = starts = 0
+    start = []
+    for i, n in enumerate(pages):
+        bt[i, :n] = order[at:at + n].int()
+        at += n
+        start.append(starts)
+        starts += news[i]
+    q = rnd(starts, A, D).bfloat16()
+    pos = torch.tensor([h + j for h, n in zip(hists, news) for j in range(n)],
+                       dtype=torch.int32, device="cuda")
+    tiles = ops.build_attn_tiles(start, hists, news, H, G, maps, "cuda")
+    outs = []
+    k = ops._paged_backend(q)
+    for exact in (False, True):
+        out = torch.full((starts, A, VW), 7.0, device="cuda",
+                         dtype=torch.float32 if fp32 else torch.bfloat16)
+        k.paged_attention(out, q, kc, vc, bt.cuda(), tiles, pos, D ** -0.5, maps,
+                          kw.get("window", 0), kw.get("keep_first", 0),
+                          kw.get("sinks"), exact, nsplit, kw.get("slopes"),
+                          kw.get("softcap", 0.0), kw.get("chunk", 0), kw.get("gate"))
+        outs.append(out.double())
+    # weights rounded to bf16 (2^-8 of each at most, of values up to 6), results too
+    assert float((outs[0] - outs[1]).abs().max()) < 6 * 2.0 ** -8 \
+        + 2.0 ** -8 * float(outs[1].abs().max())
+    rel = float((outs[0] - outs[1]).norm() / outs[1].norm())
+    assert rel < 2.0 ** -7, rel
+
+
+@pytest.mark.parametrize("hists", [[0], [30, 31, 32, 33], [126, 127, 128, 129],
+                                   [15, 16, 63, 64, 65], [1000, 3, 517]])
+@pytest.mark.parametrize("nsplit", [1, 2, 5])
+@pytest.mark.parametrize("H,G,VW", [(16, 4, 128), (4, 4, 80), (32, 2, 112)])
+class TestEdges:
+    pytestmark = gpu
+
+    def test_decode_rows(self, hists, nsplit, H, G, VW):
+        _run(hists, [1] * len(hists), H, G, VW, nsplit)
+
+    def test_a_few_rows(self, hists, nsplit, H, G, VW):
+        _run(hists, [3 + 20 * (i % 2) for i in range(len(hists))], H, G, VW, nsplit)
+
+
+@pytest.mark.parametrize("nsplit", [1, 3])
+@pytest.mark.parametrize("kw", [
+    {"window": 100}, {"window": 64, "keep_first": 5}, {"chunk": 96}, {"softcap": 20.0},
+    {"maps": 2}, {"fp32": True}, {"sinks": True}, {"slopes": True}, {"gate": True}],
+    ids=str)
+class TestOptions:
+    pytestmark = gpu
+
+    def test_as_the_fp32_path(self, nsplit, kw):
+        hists, news, H = [0, 97, 411, 1300], [1, 5, 1, 33], 16
+        g = torch.Generator(device="cuda").manual_seed(4)
+        per_head = lambda: torch.rand(H, generator=g, device="cuda")
+        kw = dict(kw)
+        if kw.get("gate"):
+            kw["gate"] = torch.randn(sum(news), H, generator=g, device="cuda").bfloat16()
+        for name in ("sinks", "slopes"):
+            if name in kw:
+                kw[name] = per_head()
+        _run(hists, news, H, 4, 128, nsplit, **kw)
