@@ -20,25 +20,22 @@
 // Tiles (w4_tile_kernel). 8 waves (4 where the columns are no multiple of 128)
 // have 16 columns each and all of up to 64 rows; more rows are more workgroups.
 // Steps of 256 k of x and of the weights go to two buffers in the LDS, whole
-// 128-byte lines of both by loads that write the LDS themselves, one step ahead.
+// 128-byte lines of both by loads that write the LDS themselves, one step ahead; or 16
+// waves, two to a column tile with half a step each, whose sums meet at the end.
 // 16-byte chunks are permuted through the lanes' addresses: of x's rows (512
 // bytes) XORed with the row, of the weights' (128 bytes) with (row >> 1). Weights
 // are the A operand: a lane ends with 4 neighbouring columns of a row. The sums of
 // x over a step's blocks are made once, by a wave each, and used a step later.
 // Narrow products are cut over k into fp32 parts, which the next kernel adds up.
-// What bounds it is the unpacking: some 150 vector instructions of a wave in a
-// step, two waves a SIMD, are most of the microsecond that it takes; at 64 rows the
-// reads of x from the LDS. Before, nibbles lay in order and x was permuted to fit
-// them, each wave made its own sums of x, and both came in pieces of 64 bytes, 16
-// rows an instruction, x again for every 16 to 64 columns. us, weights out of
-// memory, before -> now at 1 / 16 / 32 / 64 rows: 28672 x 4096 21 -> 21 / 23 -> 22
-// / 36 -> 23 / 81 -> 33, 4096 x 14336 12.8 -> 11.4 / 20 -> 12 / 33 -> 13 / 65 ->
-// 18, 6144 x 4096 7.3 -> 7.1 / 9.1 -> 7.4 / 14.3 -> 8.6 / 21 -> 12, 4096 x 4096
-// 6.0 -> 5.3 / 7.8 -> 5.7 / 12.3 -> 6.5 / 20 -> 8.8, 128256 x 4096 74 -> 61 / 83 ->
-// 64 / 138 -> 98 / 316 -> 134, 57344 x 8192 70 -> 65 / 79 -> 63 / - / 259 -> 125.
+// What bounds it is a wave's chain in a step, LDS, unpacking, products and scales, of
+// which four waves a SIMD hide more than two; at 64 rows the reads of x from the LDS. us,
+// weights out of memory, 8 waves with scales one by one -> now at 8 / 16 / 32 / 64 rows:
+// 28672 x 4096 with the activation 21.3 -> 17.2 / 22.2 -> 18.3 / 23.7 -> 21.2 / 32.9 ->
+// 27.3, 57344 x 8192 59 -> 55 / 67 -> 59 / 87 -> 78 / 120 -> 100, 128256 x 4096 61 -> 57
+// / 61 -> 58 / 95 -> 83 / 128 -> 107, 8192 x 28672 28 -> 28.6 / 29.7 -> 29.0 / 43 -> 37.5
+// / 57 -> 49, 4096 x 14336 11.7 -> 10.9 / 11.8 -> 11.2 / 13.0 -> 13.1 / 17.6 -> 17.0.
 // Two tiles of columns a wave, four waves: 27, 14, 9.1, 6.2, 73 at 16 rows and 42,
-// 22, 15, 9.9, 173 at 64; a third buffer in the LDS: no faster where one workgroup
-// fits a CU, 94 instead of 73 where it takes the second one's place.
+// 22, 15, 9.9, 173 at 64 (28672 x 4096, 4096 x 14336, 6144 x, 4096 x, 128256 x 4096).
 //
 // Rows (w4_rows_kernel): few rows of products that are narrow and have no consumer
 // for parts, and small ones. Straight from memory, k cut over the waves.
@@ -55,12 +52,20 @@ DEVICE_INLINE f32x4 w4_mfma(u32x4 a, u32x4 b, f32x4 c) {
       __builtin_bit_cast(w4_s16x8, a), __builtin_bit_cast(w4_s16x8, b), c, 0, 0, 0);
 }
 
-// eight nibbles as bf16 128 + q, in order
+// eight nibbles as bf16 128 + q, in order. FUSED: the mask in a scalar and the exponents
+// in a vector register, both hidden from the compiler, which else takes two instructions
+// for the v_and_or_b32 that has no room for two constants (with 16 waves 3 to 8 %; where
+// a workgroup has 8, waves wait for the memory, and 128256 columns took 65 us for 61).
+template <bool FUSED = false>
 DEVICE_INLINE u32x4 w4_bf16(unsigned int d) {
+  unsigned int mask = 0x000f000fu, high = 0x43004300u;
+  if constexpr (FUSED) {
+    asm("" : "+s"(mask));
+    asm("" : "+v"(high));
+  }
   u32x4 o;
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
-    o[j] = ((d >> (4 * j)) & 0x000f000fu) | 0x43004300u;
+  for (int j = 0; j < 4; ++j) o[j] = ((d >> (4 * j)) & mask) | high;
   return o;
 }
 
@@ -71,8 +76,9 @@ constexpr int W4_SZ = 32;                   // blocks of k whose scales are stag
 // silu(gate) * up in [M, N], qw then holding N gate rows and N up rows behind.
 enum W4Out { W4_ROWS, W4_PARTS, W4_SILU };
 
-template <int MT, int WAVES, W4Out OUT>
-__global__ __launch_bounds__(WAVES * WAVE_SIZE) void w4_tile_kernel(
+// KW 2: twice the waves, each with one of a step's two blocks. NB: buffers in the LDS.
+template <int MT, int WAVES, int KW, int NB, W4Out OUT>
+__global__ __launch_bounds__(WAVES * KW * WAVE_SIZE) void w4_tile_kernel(
     void* __restrict__ out, const unsigned short* __restrict__ x,  // [M, K] bf16
     const unsigned char* __restrict__ qw,   // [N, K/2] frag-ordered nibbles
     const unsigned short* __restrict__ sc,  // [N, K/128] bf16 scale
@@ -80,13 +86,16 @@ __global__ __launch_bounds__(WAVES * WAVE_SIZE) void w4_tile_kernel(
     int M, int N, int K, int splits) {
   constexpr int ROWS = 16 * MT, COLS = 16 * WAVES;
   constexpr int XB = ROWS * W4_SK, BUF = XB + COLS * 64;  // elements of 2 bytes
-  constexpr int LX = 8 * MT / WAVES;        // loads of x of a wave in a step
+  constexpr int ALL = WAVES * KW;
+  constexpr int LX = (8 * MT + ALL - 1) / ALL;  // loads of x of a wave in a step
+  constexpr int LW = 2 / KW;                // of its weights
   constexpr int CT = OUT == W4_SILU ? COLS / 2 : COLS;    // columns of out
-  __shared__ __attribute__((aligned(1024))) unsigned short lds[2 * BUF];
+  __shared__ __attribute__((aligned(1024))) unsigned short lds[NB * BUF];
   __shared__ __attribute__((aligned(16))) unsigned int sz[W4_SZ * COLS];
   __shared__ float xsum[2][2][ROWS];        // of a step's blocks, by its parity
 
   const int nb = K / W4_KC, total = (nb + 1) / 2;
+  const bool pairs = nb % 2 == 0 && ((unsigned long)sc | (unsigned long)zs) % 4 == 0;
   const int split = OUT == W4_PARTS ? blockIdx.x % splits : 0;
   const int n0 = (OUT == W4_PARTS ? blockIdx.x / splits : blockIdx.x) * CT;
   const int m0 = blockIdx.y * ROWS;
@@ -96,7 +105,8 @@ __global__ __launch_bounds__(WAVES * WAVE_SIZE) void w4_tile_kernel(
     end = (int)((long)total * (split + 1) / splits);
   }
   const int tid = threadIdx.x, lane = tid & (WAVE_SIZE - 1);
-  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE_SIZE);
+  const int any = __builtin_amdgcn_readfirstlane(tid / WAVE_SIZE);
+  const int wave = any % WAVES, kw = any / WAVES;  // columns, and half of a step
   const int lc = lane & 15, lg = lane >> 4;
   // row of qw of one of the workgroup's columns: the first waves' are of the gate
   auto at = [&](int c) {
@@ -106,17 +116,17 @@ __global__ __launch_bounds__(WAVES * WAVE_SIZE) void w4_tile_kernel(
   // an instruction brings 2 rows of x, or 8 of the weights, a wave its own
   // columns; a step of one block (the last of an odd number) brings it twice
   const unsigned short* xp[LX];
-  const unsigned char* wp[2];
-  int xc[LX], wc[2];
+  const unsigned char* wp[LW];
+  int xc[LX], wc[LW];
 #pragma unroll
   for (int i = 0; i < LX; ++i) {
-    const int row = (wave * LX + i) * 2 + lane / 32;
+    const int row = (any * LX + i) * 2 + lane / 32;
     xp[i] = x + (long)min(m0 + row, M - 1) * K;
     xc[i] = (lane & 31) ^ (row & 15);
   }
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int row = i * 8 + lane / 8;
+  for (int i = 0; i < LW; ++i) {
+    const int row = (kw * LW + i) * 8 + lane / 8;
     wp[i] = qw + (long)at(wave * 16 + row) * (K / 2);
     wc[i] = (lane & 7) ^ ((row >> 1) & 7);
   }
@@ -125,13 +135,14 @@ __global__ __launch_bounds__(WAVES * WAVE_SIZE) void w4_tile_kernel(
 #pragma unroll
   for (int m = 0; m < MT; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
   const u32x4 ones = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
-  f32x4 z[2];                               // 128 s + zs of the step before
+  constexpr int HB = 2 / KW;                // blocks of a step that are the wave's
+  f32x4 z[HB];                              // 128 s + zs of the step before
   auto correct = [&](int i) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int h = 0; h < HB; ++h)
 #pragma unroll
       for (int m = 0; m < MT; ++m) {
-        const float xs = xsum[i & 1][h][m * 16 + lc];
+        const float xs = xsum[i & 1][kw * HB + h][m * 16 + lc];
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[m][r] -= z[h][r] * xs;
       }
@@ -149,41 +160,60 @@ __global__ __launch_bounds__(WAVES * WAVE_SIZE) void w4_tile_kernel(
     auto stage = [&](int i) {
       const int st = step(i);
       const bool half = 2 * st + 1 >= nb;
-      unsigned short* to = lds + (i & 1) * BUF;
+      unsigned short* to = lds + i % NB * BUF;
 #pragma unroll
       for (int j = 0; j < LX; ++j)
-        load_to_lds(xp[j] + (long)st * W4_SK + (half ? xc[j] & 15 : xc[j]) * 8,
-                    to + (wave * LX + j) * 2 * W4_SK);
+        if (8 * MT >= ALL || any * LX + j < 8 * MT)
+          load_to_lds(xp[j] + (long)st * W4_SK + (half ? xc[j] & 15 : xc[j]) * 8,
+                      to + (any * LX + j) * 2 * W4_SK);
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < LW; ++j)
         load_to_lds((const unsigned short*)(wp[j] + (long)st * W4_KC +
                                             (half ? wc[j] & 3 : wc[j]) * 16),
-                    to + XB + (wave * 16 + j * 8) * 64);
+                    to + XB + (wave * 16 + (kw * LW + j) * 8) * 64);
     };
-    stage(0);
-    // scale (low half) and offset of every column and block, 0 behind the last
+    for (int i = 0; i < NB - 1 && i < n; ++i) stage(i);
+    // scale (low half) and offset of every column and block, 0 behind the last; two
+    // blocks at a time where they lie so (28672 x 4096 22 -> 20 us)
     const int b0 = 2 * from;
-    for (int u = tid; u < COLS * 2 * n; u += WAVES * WAVE_SIZE) {
-      const int c = u / (2 * n), b = u % (2 * n);
-      const long i = (long)at(c) * nb + b0 + b;
-      sz[b * COLS + c] =
-          b0 + b < nb ? (unsigned int)sc[i] | ((unsigned int)zs[i] << 16) : 0u;
+    if (pairs) {
+#pragma unroll 4
+      for (int u = tid; u < COLS * n; u += ALL * WAVE_SIZE) {
+        const int c = u / n, b = u % n;
+        const long i = ((long)at(c) * nb + b0) / 2 + b;
+        const unsigned int p = reinterpret_cast<const unsigned int*>(sc)[i];
+        const unsigned int q = reinterpret_cast<const unsigned int*>(zs)[i];
+        sz[2 * b * COLS + c] = (p & 0xffffu) | (q << 16);
+        sz[(2 * b + 1) * COLS + c] = (p >> 16) | (q & 0xffff0000u);
+      }
+    } else {
+      for (int u = tid; u < COLS * 2 * n; u += ALL * WAVE_SIZE) {
+        const int c = u / (2 * n), b = u % (2 * n);
+        const long i = (long)at(c) * nb + b0 + b;
+        sz[b * COLS + c] =
+            b0 + b < nb ? (unsigned int)sc[i] | ((unsigned int)zs[i] << 16) : 0u;
+      }
     }
 
     for (int i = 0; i < n; ++i) {
-      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      // the steps asked for behind this one; a wave may have no rows of x to bring
+      if (NB > 2 && i > 0 && i + NB - 2 < n)
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)"
+                     ::"n"((NB - 2) * (8 * MT >= ALL ? LX + LW : LW)) : "memory");
+      else
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
-      if (i + 1 < n) stage(i + 1);
+      if (i + NB - 1 < n) stage(i + NB - 1);
       if (i > 0) correct(i - 1);
-      const unsigned short* xl = lds + (i & 1) * BUF + lc * W4_SK;
+      const unsigned short* xl = lds + i % NB * BUF + lc * W4_SK;
       const unsigned short* wl =
-          lds + (i & 1) * BUF + XB + (wave * 16 + lc) * 64;
+          lds + i % NB * BUF + XB + (wave * 16 + lc) * 64;
       const int b = 2 * (step(i) - from);
       // sums of x over the blocks, each by one of the waves for all
 #pragma unroll
-      for (int j = 0; j < (2 * MT + WAVES - 1) / WAVES; ++j) {
-        const int q = wave + j * WAVES, h = q / MT, m = q % MT;
+      for (int j = 0; j < (2 * MT + ALL - 1) / ALL; ++j) {
+        const int q = any + j * ALL, h = q / MT, m = q % MT;
         if (q >= 2 * MT) break;
         f32x4 xs = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -195,13 +225,14 @@ __global__ __launch_bounds__(WAVES * WAVE_SIZE) void w4_tile_kernel(
         if (lg == 0) xsum[i & 1][h][m * 16 + lc] = xs[0];
       }
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
+      for (int hh = 0; hh < HB; ++hh) {
+        const int h = kw * HB + hh;
         const u32x4 w4 = *reinterpret_cast<const u32x4*>(
             wl + ((h * 4 + lg) ^ ((lc >> 1) & 7)) * 8);
         f32x4 p[MT];
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-          const u32x4 wf = w4_bf16(w4[c]);
+          const u32x4 wf = w4_bf16<KW == 2>(w4[c]);
 #pragma unroll
           for (int m = 0; m < MT; ++m)
             p[m] = w4_mfma(wf,
@@ -215,7 +246,7 @@ __global__ __launch_bounds__(WAVES * WAVE_SIZE) void w4_tile_kernel(
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const float s = __builtin_bit_cast(float, v[r] << 16);
-          z[h][r] = 128.f * s + __builtin_bit_cast(float, v[r] & 0xffff0000u);
+          z[hh][r] = 128.f * s + __builtin_bit_cast(float, v[r] & 0xffff0000u);
 #pragma unroll
           for (int m = 0; m < MT; ++m) acc[m][r] += s * p[m][r];
         }
@@ -226,11 +257,28 @@ __global__ __launch_bounds__(WAVES * WAVE_SIZE) void w4_tile_kernel(
     __syncthreads();                         // the buffers are done with
   }
 
+  // the halves of the steps together
+  if constexpr (KW == 2) {
+    f32x4* other = reinterpret_cast<f32x4*>(lds) + wave * MT * WAVE_SIZE + lane;
+    if (kw == 1)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) other[m * WAVE_SIZE] = acc[m];
+    __syncthreads();
+    if (kw == 0)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        const f32x4 v = other[m * WAVE_SIZE];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[m][r] += v[r];
+      }
+    __syncthreads();
+  }
+
   // D[column = lg*4 + r][row = lc]
   constexpr int US = CT + 4;                 // the up product's rows in the LDS
   float* up = reinterpret_cast<float*>(lds);
   if constexpr (OUT == W4_SILU) {
-    if (wave >= WAVES / 2)
+    if (wave >= WAVES / 2 && kw == 0)
 #pragma unroll
       for (int m = 0; m < MT; ++m)
         *reinterpret_cast<f32x4*>(up + (m * 16 + lc) * US +
@@ -238,6 +286,7 @@ __global__ __launch_bounds__(WAVES * WAVE_SIZE) void w4_tile_kernel(
     __syncthreads();
     if (wave >= WAVES / 2) return;
   }
+  if (kw > 0) return;
   const int col = n0 + wave * 16 + lg * 4;
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
@@ -430,13 +479,13 @@ void w4_rows(void* out, const void* x, const void* qw, const void* sc,
                      (const unsigned short*)zs, M, N, K);
 }
 
-template <int MT, int WAVES, W4Out OUT>
+template <int MT, int WAVES, int KW, int NB, W4Out OUT>
 void w4_tile(void* out, const void* x, const void* qw, const void* sc,
              const void* zs, int M, int N, int K, int splits, hipStream_t s) {
   constexpr int CT = (OUT == W4_SILU ? 8 : 16) * WAVES;
-  hipLaunchKernelGGL((w4_tile_kernel<MT, WAVES, OUT>),
+  hipLaunchKernelGGL((w4_tile_kernel<MT, WAVES, KW, NB, OUT>),
                      dim3(N / CT * splits, (M + 16 * MT - 1) / (16 * MT)),
-                     dim3(WAVES * WAVE_SIZE), 0, s, out,
+                     dim3(WAVES * KW * WAVE_SIZE), 0, s, out,
                      (const unsigned short*)x, (const unsigned char*)qw,
                      (const unsigned short*)sc, (const unsigned short*)zs, M, N,
                      K, splits);
@@ -447,12 +496,25 @@ int w4_waves(int N) { return N % 128 == 0 ? 8 : 4; }
 template <W4Out OUT>
 void w4_tiles(void* out, const void* x, const void* qw, const void* sc,
               const void* zs, int M, int N, int K, int splits, hipStream_t s) {
-#define W4_TILE(MT)                                                            \
-  do {                                                                         \
-    if (OUT == W4_SILU || w4_waves(N) == 8)                                    \
-      w4_tile<MT, 8, OUT>(out, x, qw, sc, zs, M, N, K, splits, s);             \
-    else if constexpr (OUT != W4_SILU)                                         \
-      w4_tile<MT, 4, OUT>(out, x, qw, sc, zs, M, N, K, splits, s);             \
+  // Sixteen waves for eight from four steps a workgroup on (us, eight / sixteen, 16 rows
+  // and 64: 28672 x 4096 20.2 / 20.3 and 30.7 / 27.3, 57344 x 8192 63 / 59 and 113 / 100,
+  // 128256 x 4096 65 / 58 and 123 / 107; but 4096 x 4096, two steps, 5.7 / 5.9), with two
+  // more buffers where every workgroup has a CU of its own (28672 x 4096 20.3 / 18.3, at
+  // 57344 x 8192 59 / 66).
+  const int groups = (OUT == W4_SILU ? N / 64 : N / (16 * w4_waves(N))) * splits;
+  const bool half = (K / W4_KC + 1) / 2 / splits >= 4, own = groups <= 256;
+#define W4_TILE(MT)                                                                \
+  do {                                                                             \
+    if (OUT != W4_SILU && w4_waves(N) == 4) {                                      \
+      if constexpr (OUT != W4_SILU)                                                \
+        w4_tile<MT, 4, 1, 2, OUT>(out, x, qw, sc, zs, M, N, K, splits, s);         \
+    } else if (!half) {                                                            \
+      w4_tile<MT, 8, 1, 2, OUT>(out, x, qw, sc, zs, M, N, K, splits, s);           \
+    } else if (MT == 1 && own) {                                                   \
+      w4_tile<MT, 8, 2, MT == 1 ? 4 : 2, OUT>(out, x, qw, sc, zs, M, N, K, splits, s); \
+    } else {                                                                       \
+      w4_tile<MT, 8, 2, 2, OUT>(out, x, qw, sc, zs, M, N, K, splits, s);           \
+    }                                                                              \
   } while (0)
   if (M <= 16) W4_TILE(1);
   else if (M <= 32) W4_TILE(2);

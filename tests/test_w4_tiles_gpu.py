@@ -111,3 +111,26 @@ def test_none_where_there_is_no_such_form():
     x, (qw, s, z), _, _ = _case(4, 192, 256)
     assert _hip().w4_silu(x, qw, s, z) is None
     assert _hip().w4_parts(x, qw, s, z) is None
+
+
+# about the four steps of 256 k from which two waves share a step, the four buffers that
+# a workgroup with a CU of its own has, and the 16 steps whose scales are staged at once
+@pytest.mark.parametrize("M", [1, 16, 32, 64])
+@pytest.mark.parametrize("K", [768, 896, 1024, 1152, 1280, 4096, 4224, 4736, 8320])
+def test_steps_of_a_workgroup(M, K):
+    test_product_ends_in_the_activation(M, 8192, K)
+
+
+@pytest.mark.parametrize("M", [5, 64])
+def test_scales_that_lie_one_by_one(M):
+    x, (qw, s, z), w, size = _case(M, 33024, 2048)
+    odd = lambda t: torch.cat([t.flatten()[:1], t.flatten()])[1:].view(t.shape)
+    out = torch.full((M, 33024), 9.0, device="cuda").bfloat16()
+    same = torch.full_like(out, 9.0)
+    assert odd(s).data_ptr() % 4 == 2
+    _hip().w4_gemm(out, x, qw, odd(s), odd(z))
+    _hip().w4_gemm(same, x, qw, s, z)
+    assert torch.equal(out, same)
+    ref = x.double() @ w.T
+    assert bool(((out.double() - ref).abs()
+                 <= ref.abs() * 2.0 ** -8 + size * 2.0 ** -18).all())
