@@ -19,9 +19,10 @@ DEVICE_INLINE i32x4 wt_rsrc(const void* p, unsigned bytes) {
   return i32x4{(int)a, (int)(a >> 32) & 0xffff, (int)bytes, 0x00020000};
 }
 
-DEVICE_INLINE float wt_silu(float g, float u) {
-  return g * u * __builtin_amdgcn_rcpf(1.f + __expf(-g));
-}
+// The gate is divided first, as in every other form: g * u may leave fp32 where the
+// quotient is 0. A division costs the end of a tile nothing that shows (8192 rows of
+// 28672 x 4096 1254 us, with the reciprocal 1254).
+DEVICE_INLINE float wt_silu(float g, float u) { return g / (1.f + __expf(-g)) * u; }
 
 // A sum out of its accumulation register, in the order of the program: read where the
 // compiler likes, all at once, they do not fit beside the operands of the next tile.

@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from gpustack_amd import ops
+from test_wide_tiles_gpu import check_large, large_pairs
 
 needs_gpu = pytest.mark.skipif(not torch.cuda.is_available(),
                                reason="needs a GPU")
@@ -61,6 +62,25 @@ def _run(counts, k, H, I, weights=True):
     ([0] * 100 + [97] * 30, 2, 2048, 768)])
 def test_tiles(counts, k, H, I):
     _run(counts, k, H, I)
+
+
+@pytest.mark.gpu
+@needs_gpu
+@pytest.mark.parametrize("rows", [64, 320])
+def test_gate_and_up_beyond_fp32(rows):
+    hip = ops._load_hip()
+    g, u, ref = large_pairs()
+    I, H = -(-len(g) // 8) * 8, 192
+    x = torch.zeros(rows, H, dtype=torch.bfloat16)
+    x[:, 0] = 1
+    w = torch.zeros(1, 2 * I, H, dtype=torch.bfloat16)
+    w[0, :len(g), 0], w[0, I:I + len(u), 0] = g, u
+    act = torch.empty(rows, I, device="cuda", dtype=torch.bfloat16)
+    _, s_tok, counts, offs, _, _ = hip.moe_sort(
+        torch.zeros(rows, device="cuda", dtype=torch.int32), 1, 1)
+    hip.moe_wide(False, act, x.cuda(), w.cuda(), s_tok, offs, counts)
+    for row in (0, rows - 1):
+        check_large(act[row, :len(g)], ref)
 
 
 @pytest.mark.gpu

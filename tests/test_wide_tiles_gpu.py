@@ -51,6 +51,47 @@ def test_product_ends_in_the_activation(M, N, K, pad, tile):
     _check(room[1:M + 1], x, w)
 
 
+def large_pairs():
+    """Gates and ups whose product leaves fp32, or that are not finite, all by all in
+    bf16, and silu(gate) * up of them; e^-g is infinite where it leaves fp32."""
+    inf, nan = float("inf"), float("nan")
+    g = torch.tensor([-inf, -1e38, -1e30, -1e3, -100., -60., -1., 0., 1., 60., 1e30,
+                      inf, nan]).bfloat16()
+    u = torch.tensor([0., 1., -3., 1e30, -1e36, 1e37, inf, -inf, nan]).bfloat16()
+    g, u = (t.flatten() for t in torch.meshgrid(g, u, indexing="ij"))
+    gd, ud = g.double(), u.double()
+    return g, u, (gd / (1 + torch.exp(-gd).float().double()) * ud).float()
+
+
+def check_large(out, ref):
+    """`out` against large_pairs' `ref`: rounded to bf16 once, its functions 2^-20 of
+    it; e^-g of 60 is off by 60 2^-24 of it."""
+    out, ref = out.double().cpu(), ref.double()
+    assert torch.equal(out.isnan(), ref.isnan())
+    # no finite result becomes infinite or the other way round
+    assert torch.equal(out.isinf(), ref.isinf())
+    ok = ref.isfinite()
+    assert torch.equal(out[~ok & ~ref.isnan()], ref[~ok & ~ref.isnan()])
+    bound = ref.abs() * (2.0 ** -8 + 2.0 ** -17) + 1e-38
+    assert bool(((out - ref).abs() <= bound)[ok].all())
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")
+@pytest.mark.parametrize("tile", ops._WIDE_SILU)
+def test_gate_and_up_beyond_fp32(tile):
+    g, u, ref = large_pairs()
+    N, K = -(-len(g) // 16) * 16, 128
+    x = torch.zeros(130, K, dtype=torch.bfloat16)
+    x[:, 0] = 1
+    w = torch.zeros(2 * N, K, dtype=torch.bfloat16)
+    w[:len(g), 0], w[N:N + len(u), 0] = g, u
+    out = torch.empty(130, N, device="cuda", dtype=torch.bfloat16)
+    ops._load_hip().wide_rows(out, x.cuda(), w.cuda(), *tile, silu=True)
+    for row in (0, 129):
+        check_large(out[row, :len(g)], ref)
+
+
 @pytest.mark.parametrize("M,N,K,pad", SIZES)
 @pytest.mark.parametrize("tile", [t for t in ops._WIDE_ROWS if t != (8, 8)])
 @pytest.mark.gpu
