@@ -135,12 +135,15 @@ __global__ __launch_bounds__(256, 1) void wide_kernel(
 
   // The step that is loaded next: of the tile of round `lr`, with `left` steps to come;
   // k0: its bytes from the start of a row. Weight rows lie a power of two apart, and
-  // workgroups at one place of theirs meet on a few memory channels: each XCD begins an
-  // eighth of the row further on (512 rows of 28672 x 4096 out of HBM 97 -> 91 us; each
-  // column tile at a place of its own 96, and 1327 for 1250 at 8192 rows, whose rows
-  // then miss the L2). Of no use in more rows, which compute longer than they load
-  // (7122 x 8192 x 2048 330 -> 331), and parts begin elsewhere anyway.
-  const int turn = OUT != PARTS && M <= 2048 ? xcd * steps / 8 : 0;
+  // workgroups at one place of theirs meet on a few memory channels: each eighth of the
+  // columns, about an XCD's, begins an eighth of the row further on (512 rows of 28672 x
+  // 4096 out of HBM 97 -> 91 us; each column tile at a place of its own 96, and 1327 for
+  // 1250 at 8192 rows, whose rows then miss the L2). A column's rows all begin at one
+  // place: equal ones get equal sums. Of no use in more rows, which compute longer than
+  // they load (7122 x 8192 x 2048 330 -> 331), and parts begin elsewhere anyway.
+  auto turn = [&](const Place& p) {
+    return OUT != PARTS && M <= 2048 ? one(p.n0 / COLS * 8 / nt * steps / 8) : p.from;
+  };
   int lr = 0, left = 0;
   unsigned k0 = 0;
   i32x4 rx{}, rw{};
@@ -148,7 +151,7 @@ __global__ __launch_bounds__(256, 1) void wide_kernel(
     if (lr < rounds) {
       const Place p = place(lr);
       left = p.n;
-      k0 = (unsigned)(OUT == PARTS ? p.from : turn) * (WT_K * 2);
+      k0 = (unsigned)turn(p) * (WT_K * 2);
       rx = wt_rsrc(x + p.m0 * xs, ((unsigned)min(MT, M - p.m0) - 1) *
                                           (unsigned)xs * 2 + (unsigned)K * 2);
       rw = wt_rsrc(w + (long)p.n0 * K, (unsigned)(WN - p.n0) * (unsigned)K * 2);

@@ -112,6 +112,22 @@ def test_product(M, N, K, pad, tile):
 
 @pytest.mark.gpu
 @pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")
+@pytest.mark.parametrize("M,N,tile,silu", [
+    (700, 2008, (8, 6), True), (2000, 1080, (8, 4), True), (520, 2136, (6, 8), True),
+    (2000, 1032, (4, 4), False), (1500, 1032, (6, 6), False), (700, 5000, (8, 7), False)])
+def test_equal_rows_are_equal_anywhere(M, N, tile, silu):
+    # tiles of one column on two XCDs, eight row tiles a block and more; sums of which
+    # nothing but their roundings is left
+    x, w = _operands(1, N, 2048)
+    x = torch.cat([x, x], 1).expand(M, 4096).contiguous()
+    w = torch.cat([w, -w], 1)
+    out = torch.empty(M, N, device="cuda", dtype=torch.bfloat16)
+    ops._load_hip().wide_rows(out, x, w if silu else w[:N], *tile, silu=silu)
+    assert bool((out == out[:1]).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")
 def test_refused_operands():
     x, w = _operands(256, 128, 128)
     out = torch.empty(256, 128, device="cuda", dtype=torch.bfloat16)
