@@ -362,11 +362,10 @@ __global__ __launch_bounds__(256) void state_scan_vec_kernel(
 // EXACT: without an activation q, k and v are bf16 values, and the bf16 instructions
 // multiply them as they are, at sixteen times the rate: 16 cycles for 32 k where fp32
 // takes 32 for 4. The other operand (state, weighted scores, weighted v) is split into
-// three bf16 parts whose sum it is, bit for bit, so that the products are the exact ones
-// and only the sums round, in fp32 as before: error against 64 bits of y .76 and of the
-// state .95 to .99 of what the fp32 instructions leave (decays of a few tenths a row), .55
-// and .65 (of a hundredth); only the state of decays that leave nothing of the row
-// before is off by 6.4e-8 for 5.0e-8.
+// three bf16 parts whose sum it is to 26 bits and more, so that the products are the
+// exact ones and only the sums round, in fp32 as before: error against 64 bits of y .66
+// to .89 and of the state .82 to 1.00 of what the fp32 instructions leave (decays of e^-.1
+// a row to ones that leave nothing), .53 and .62 (of a hundredth).
 //   - the state stays in the accumulators; its parts are made a chunk, 32 rows at a time.
 //   - scores are multiplied transposed, so that they lie as the operand of the product
 //     with v; every wave has them all, and no barrier stands between.
@@ -378,32 +377,38 @@ __global__ __launch_bounds__(256) void state_scan_vec_kernel(
 //   - where anything is not finite its split is NaN; it shows in the rows or the state,
 //     and the columns are walked again as below.
 // Bound by the vector instructions (500 a wave and chunk, 72 % of the time with two
-// waves a SIMD; 66 matrix ones): 64 heads of 128 x 64, whole 4000 rows 547 -> 254 us, the
-// six 303 -> 155, 8 x 500 91 -> 58 (fp32 instructions: 723, 433, 141).
+// waves a SIMD; 66 matrix ones): 64 heads of 128 x 64, whole 4000 rows 741 -> 262 us, the
+// six 439 -> 165, 8 x 500 135 -> 60.
 typedef __attribute__((ext_vector_type(4))) float sc_f32x4;
+typedef __attribute__((ext_vector_type(2))) __bf16 sc_bf16x2;
 
 enum ChunkPart { WHOLE, ENDS, OUTPUTS };
 
-// An fp32 value as three bf16 ones that add up to it: its significant bits eight by
-// eight. Pairs, high halves first.
+// An fp32 value as three bf16 ones that add up to it. PRODUCT: of products, which the
+// compiler subtracts from before it rounds them (fma): up to 32 bits are left, and each
+// part is the nearest to what the ones before leave. Cut, the last one lost up to an ulp,
+// always towards 0, and the state of strong decays was off by 1.16 of what the fp32 form
+// leaves. Values that are held are their significant bits eight by eight, which takes as
+// many instructions but is the faster one (16 heads of 128 x 128, 4 x 1000 67.5 / 68.5).
 struct Split8 { u32x4 part[3]; };
+template <bool PRODUCT>
 DEVICE_INLINE Split8 split8(const float* x) {
   Split8 s;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    unsigned u[2], v[2], w[2];
+    float a = x[2 * i], b = x[2 * i + 1];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const float a = x[2 * i + j];
-      u[j] = __builtin_bit_cast(unsigned, a);
-      const float b = a - __builtin_bit_cast(float, u[j] & 0xffff0000u);
-      v[j] = __builtin_bit_cast(unsigned, b);
-      const float c = b - __builtin_bit_cast(float, v[j] & 0xffff0000u);
-      w[j] = __builtin_bit_cast(unsigned, c);
+    for (int part = 0; part < 3; ++part) {
+      const f32x2 v{a, b};
+      const unsigned u = __builtin_bit_cast(unsigned, a);
+      const unsigned w = __builtin_bit_cast(unsigned, b);
+      const unsigned both =
+          PRODUCT ? __builtin_bit_cast(unsigned, __builtin_convertvector(v, sc_bf16x2))
+                  : __builtin_amdgcn_perm(w, u, 0x07060302u);
+      s.part[part][i] = both;
+      a -= __builtin_bit_cast(float, PRODUCT ? both << 16 : u & 0xffff0000u);
+      b -= __builtin_bit_cast(float, (PRODUCT ? both : w) & 0xffff0000u);
     }
-    s.part[0][i] = __builtin_amdgcn_perm(u[1], u[0], 0x07060302u);
-    s.part[1][i] = __builtin_amdgcn_perm(v[1], v[0], 0x07060302u);
-    s.part[2][i] = __builtin_amdgcn_perm(w[1], w[0], 0x07060302u);
   }
   return s;
 }
@@ -750,7 +755,7 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
             x[r] = S[2 * kb][r];
             x[4 + r] = S[2 * kb + 1][r];
           }
-          const Split8 sp8 = split8(x);
+          const Split8 sp8 = split8<false>(x);
           // two chains a tile: the large parts and the small ones
 #pragma unroll
           for (int t = 0; t < 2; ++t) {
@@ -768,7 +773,7 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
           for (int r = 0; r < 4; ++r)
             o[t][r] = (o[t][r] + o2[t][r]) * el[t * 16 + g * 4 + r];
           // and the chunk's own rows
-          o[t] = mm_split(split8(w[t]), vb, o[t]);
+          o[t] = mm_split(split8<true>(w[t]), vb, o[t]);
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             odd += o[t][r] * 0.f;
@@ -791,7 +796,7 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
         for (int r = 0; r < 4; ++r) S[t][r] *= down;
 #pragma unroll
       for (int j = 0; j < 8; ++j) vf[j] *= wl[(j >> 2) * 16 + g * 4 + (j & 3)];
-      const Split8 bv = split8(vf);
+      const Split8 bv = split8<true>(vf);
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         const unsigned short* kp =

@@ -99,6 +99,34 @@ def test_decays_beyond_one(N, P, size):
                 <= 330 * 2.0 ** -24 * float(b.abs().max())
 
 
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")
+@pytest.mark.parametrize("N,P,T", [(128, 128, 96), (64, 64, 90), (72, 40, 101)])
+def test_weighted_values_are_rounded_not_cut(N, P, T):
+    # decays that leave nothing of the row before: the state is one product, k v b
+    g = torch.Generator(device="cuda").manual_seed(N)
+    H = 4
+    cb, cc, cdt = H * P, H * (P + N), H * (P + 2 * N)
+    src = torch.randn(T, (cdt + H + 15) // 8 * 8, generator=g,
+                      device="cuda").bfloat16()
+    src[:, cdt:] = 0
+    bias = 20 + torch.rand(H, generator=g, device="cuda") * 10   # softplus(b) = b
+    state = torch.zeros(1, H, N, P, device="cuda")
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    ops.state_scan(torch.zeros(T, H * P, device="cuda"), src, 0, cb, cc, src, cdt,
+                   H, H, N, P, False, bias, torch.full((H,), 5., device="cuda"),
+                   None, None, state, i32([0]), i32([T]), i32([0]),
+                   i32(list(range(5, 5 + T))))
+    v = src[-1, :cb].double().view(H, 1, P) * bias.double()[:, None, None]
+    ref = src[-1, cb:cc].double().view(H, N, 1) * v
+    ulp = torch.exp2(torch.floor(torch.log2(ref.abs().clamp(min=1e-30))) - 23)
+    off = (state[0].double() - ref) * ref.sign() / ulp
+    # half an ulp at the sum's end, half where its small terms meet the large one, a
+    # quarter of v b's parts; towards 0 as often as away from it
+    assert float(off.abs().max()) <= 1.25
+    assert abs(float(off.mean())) < 0.05
+
+
 def test_runs_of_exact_rows():
     rule = lambda news, heads, vdim: ops.scan_run_rows(news, heads, vdim, True)
     for n in (640, 1000, 4000, 8000, 100000):
