@@ -1261,6 +1261,27 @@ def prompt_attention_fits(q_dim: int, v_dim: int, maps: int, keep_first: int,
             and k_cache.shape[2] == 16)
 
 
+@functools.lru_cache(maxsize=4096)
+def _paged_wave_parts(nt: int, span: int) -> int:
+    """Parts of `span` keys for `nt` tiles of paged_attn_waves_kernel, each of 128
+    keys and more and no more than 2048 workgroups in all: those of the least time by 8
+    us for a thousand keys on the CU with the most workgroups (on an average one for half
+    of it: contexts differ, and the others make up for it), 2 us for a merge and .6 for
+    each part in it. us at 1 / 2 / 3 / 4 / 6 parts, 16 heads on 4, and of a workgroup to a
+    tile of 64 keys, with scores through the LDS: 33 rows behind 1000 to 8000 keys 113 /
+    103 / 83 / 86 / 75 (5 taken, 78; 85), 40 rows 116 / 106 / 92 / 92 / 91 (3; 95), 33
+    behind 200 to 3000 46 / 37 / 39 / 38 / 38 (3; 41), 64 of them in a window of 1024 27 /
+    31 / 32 / 37 / 39 (1; 35), 300 rows of a prompt behind 8000 153 / 125 / 114 / 108 /
+    116 (5, 107; 147). Of 307 batches of 1 to 200 sequences one is slower than that by more
+    than 2 % (65 / 64), .83 of its time on average, 1.2 % above the best number of each."""
+    def time(parts):
+        most = nt * parts / 256
+        return 4e-3 * span * (math.ceil(most) + max(most, 1)) / parts \
+            + (parts > 1) * (2 + .6 * parts)
+
+    return min(range(1, max(1, min(16, span // 128, 2048 // nt)) + 1), key=time)
+
+
 def paged_attention(out, q, k_cache, v_cache, block_tables, row_seq, positions,
                     scale: float, maps: int = 1, window: int = 0,
                     keep_first: int = 0, sinks=None, tiles=None,
@@ -1298,12 +1319,7 @@ def paged_attention(out, q, k_cache, v_cache, block_tables, row_seq, positions,
         if span >= 512 and 0 < nt < 2048:
             if (q.shape[-1] == 128 and 64 < out.shape[-1] <= 128
                     and q.dtype == torch.bfloat16):
-                # paged_attn_waves_kernel: one workgroup a CU, each of at least 256
-                # keys; more parts only cost their merge. us at 1 / 2 / 4 / 8, 16
-                # heads on 4: 64 rows in a window of 1024 26 / 31 / 36 / 42, 16 rows
-                # 19.4 / 16.9 / 16.5 / 19.0, 8 rows behind 200 to 3000 keys 38 / 26 /
-                # 20 / 19, one behind 1000 16.0 / 13.3 / 11.5 / 12.2
-                nsplit = max(1, min(16, -(-span // 256), 256 // nt))
+                nsplit = _paged_wave_parts(nt, span)
             else:
                 # 1024 workgroups, or up to 2048 while the split stays <= 4 (a
                 # wider split pays more for the merge than it gains in

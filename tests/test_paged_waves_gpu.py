@@ -80,3 +80,29 @@ class TestOptions:
             if name in kw:
                 kw[name] = per_head()
         _run(hists, news, H, 4, 128, nsplit, **kw)
+
+
+@pytest.mark.parametrize("ctx,window", [(8000, 0), (3000, 0), (20000, 4096)])
+def test_parts_leave_few_cus_without_work(monkeypatch, ctx, window):
+    taken = []
+
+    class Kernel:
+        def paged_attention(self, *a):
+            taken.append(a[13])
+
+    monkeypatch.setattr(ops, "_paged_backend", lambda t: Kernel())
+    q = torch.zeros(1, 4, 128, dtype=torch.bfloat16)
+    span = min(ctx, window or ctx)
+    for nt in [1, 4, 60, 100, *range(128, 260, 4), 300, 400, 520, 800, 1500, 2047]:
+        ops.paged_attention(q, q, None, None, None, None, None, 1., window=window,
+                            tiles=torch.zeros(nt, 6, dtype=torch.int32), max_ctx=ctx)
+        parts = taken.pop()
+        assert 1 <= parts <= 16 and span // parts >= 128
+        # partial sums of no more workgroups than with 64 keys to a tile
+        assert parts == 1 or nt * parts <= 2048
+        # whole rounds of the 256 CUs; a few tiles have a CU each
+        rounds = -(-nt * parts // 256)
+        assert nt * parts >= .7 * 256 * rounds or nt < 60
+    ops.paged_attention(q, q, None, None, None, None, None, 1., max_ctx=500,
+                        tiles=torch.zeros(132, 6, dtype=torch.int32))
+    assert taken == [1]
