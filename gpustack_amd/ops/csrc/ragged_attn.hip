@@ -626,13 +626,16 @@ __global__ __launch_bounds__(THREADS, 2) void paged_attn_waves_kernel(
     mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE_SIZE));
     mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE_SIZE));
     const float m_new = fmaxf(m_run, mx);
+    // before any key was seen from 0: those hidden weigh 0, a score that is no number
+    // (the maximum leaves it out) shows
     const bool any = m_new != -INFINITY;
-    const float alpha = any ? __expf(m_run - m_new) : 1.f;
+    const float m_ref = any ? m_new : 0.f;
+    const float alpha = any ? __expf(m_run - m_ref) : 1.f;
     u16x8 w;
     float sum = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const float pv = any ? __expf(sv[i] - m_new) : 0.f;
+      const float pv = __expf(sv[i] - m_ref);
       w[i] = f2bf(pv);
       sum += pv;
     }
@@ -666,17 +669,17 @@ __global__ __launch_bounds__(THREADS, 2) void paged_attn_waves_kernel(
     float M = -INFINITY;
 #pragma unroll
     for (int u = 0; u < 4; ++u) M = fmaxf(M, ms[u][e]);
+    const float ref = M == -INFINITY ? 0.f : M;
     float L = 0.f;
     f32x4 o{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
-      if (ms[u][e] != -INFINITY) {
-        const float f = __expf(ms[u][e] - M);
-        L += ls[u][e] * f;
-        const f32x4 x = *reinterpret_cast<const f32x4*>(&os[u][e * OS + ch]);
+    for (int u = 0; u < 4; ++u) {            // without a maximum: 0, or no number
+      const float f = __expf(ms[u][e] - ref);
+      L += ls[u][e] * f;
+      const f32x4 x = *reinterpret_cast<const f32x4*>(&os[u][e * OS + ch]);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] += x[r] * f;
-      }
+      for (int r = 0; r < 4; ++r) o[r] += x[r] * f;
+    }
     if (nsplit > 1) {
       const long slot = (long)blockIdx.x * nsplit + split;
       if (ch == 0) {
@@ -717,10 +720,13 @@ __global__ __launch_bounds__(MERGE_THREADS) void paged_attn_merge_kernel(
   float M = -INFINITY;
   for (int s = 0; s < nsplit; ++s)
     M = fmaxf(M, ws_ml[((base + s) * G16 + e) * 2]);
+  // a part without a maximum saw no key and is 0, or has only scores that are no
+  // numbers and is none itself
+  const float ref = M == -INFINITY ? 0.f : M;
   float L = 0.f;
   for (int s = 0; s < nsplit; ++s) {
     const float* ml = ws_ml + ((base + s) * G16 + e) * 2;
-    if (ml[0] != -INFINITY) L += ml[1] * __expf(ml[0] - M);
+    L += ml[1] * __expf(ml[0] - ref);
   }
   const int row = row0 + e / n_a, a = a0 + (e % n_a) * a_step;
   const float inv = (L > 0.f ? 1.0f / L : 0.f) *
@@ -728,11 +734,9 @@ __global__ __launch_bounds__(MERGE_THREADS) void paged_attn_merge_kernel(
   TO* op = out + (long)row * p.o_st + (long)a * p.o_sa;
   for (int ch = threadIdx.x; ch < VW; ch += MERGE_THREADS) {
     float v = 0.f;
-    for (int s = 0; s < nsplit; ++s) {
-      const float m = ws_ml[((base + s) * G16 + e) * 2];
-      if (m != -INFINITY)
-        v += ws_acc[((base + s) * G16 + e) * VW + ch] * __expf(m - M);
-    }
+    for (int s = 0; s < nsplit; ++s)
+      v += ws_acc[((base + s) * G16 + e) * VW + ch] *
+           __expf(ws_ml[((base + s) * G16 + e) * 2] - ref);
     stf(op + ch, v * inv);
   }
 }

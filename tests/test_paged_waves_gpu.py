@@ -82,6 +82,30 @@ class TestOptions:
         _run(hists, news, H, 4, 128, nsplit, **kw)
 
 
+@pytest.mark.parametrize("nsplit", [1, 2, 5])
+@pytest.mark.parametrize("last", [32, 64, 96, 192])
+class TestNotANumber:
+    pytestmark = gpu
+
+    @pytest.mark.parametrize("first", [True, False])
+    def test_a_key_alone_in_a_share_shows(self, nsplit, last, first):
+        """Key `last` begins a tile of 32: with no other in it, it may be the only
+        one of a wave's share or of a part."""
+        g = torch.Generator(device="cuda").manual_seed(last)
+        rnd = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+        H, G, n, at = 4, 2, last // 16 + 1, 0 if first else last
+        kc, vc, q = rnd(2 * n, G, 16, 128), rnd(2 * n, G, 128, 16), rnd(2, H, 128)
+        kc[at // 16, :, at % 16] = float("nan")
+        bt = torch.arange(2 * n, dtype=torch.int32, device="cuda").view(2, n)
+        pos = torch.full((2,), last, dtype=torch.int32, device="cuda")
+        tiles = ops.build_attn_tiles([0, 1], [last, last], [1, 1], H, G, 1, "cuda")
+        out = torch.zeros(2, H, 128, device="cuda", dtype=torch.bfloat16)
+        ops._paged_backend(q).paged_attention(
+            out, q, kc, vc, bt, tiles, pos, 128 ** -0.5, 1, 0, 0, None, False, nsplit,
+            None, 0.0, 0, None)
+        assert bool(out[0].isnan().all()) and bool(out[1].isfinite().all())
+
+
 @pytest.mark.parametrize("ctx,window", [(8000, 0), (3000, 0), (20000, 4096)])
 def test_parts_leave_few_cus_without_work(monkeypatch, ctx, window):
     taken = []
