@@ -808,26 +808,33 @@ def _wide_silu_tile(M: int, N: int, K: int):
 def _wide_parts_plan(M: int, N: int, K: int):
     """(tile, parts over k) of a product of many rows whose consumer adds the parts up
     (wide_kernel in ops/csrc/wide_tiles.hip), or None. As many parts as let its 256
-    workgroups have one tile each, at most 8, or half as many: the tile and the parts of
-    the least time with the parts' own bytes, where that is 3 % (up to 256 rows 5) less
-    than a whole product's; both with the norm behind, which reads 4 bytes a part and
-    element. Not below 2560 k, where a part is hardly more than its start, nor what
-    _tall_tile_plan cuts but for 14336 k of more than 2048 columns. us with an RMS norm
-    behind, weights out of HBM, before / so: 512 rows of 4096x4096 38 / 33, of 6144x4096
-    49 / 42, of 4096x14336 73 / 66, 264 of 4096x14336 64 / 53, 136 of 4096x4096 30 / 21,
-    640 of 4096x14336 143 / 84, 1024 159 / 107, 2039 217 / 197; but 1024 rows of
-    4096x4096 47 / 48. Of 2808 sizes (1024 to 10240 columns, 2560 to 14336 k, 136 to 4096
-    rows) 1352 are taken, 12 of them slower by more than 3 % (1536 rows of 5376x14336
-    the worst, 1.08), .85 of the time on average."""
-    if M <= 128 or K < 2560 or K % 64 != 0 or N % 8 != 0 \
-            or (N + 512) * K >= 1 << 31 or N >= 1 << 21 \
-            or M <= 512 and (N <= 2048 or K < 14336) and _tall_tile_plan(M, N, K):
+    workgroups have one tile each, at most 8 and each of 1024 k and more, or half as many:
+    the tile and the parts of the least time with the parts' own bytes, where that is 3 %
+    (up to 256 rows 5) less than a whole product's; both with the norm behind, which reads
+    4 bytes a part and element. Not below 3584 k, where a part is hardly more than its
+    start (3072 k, us with an RMS norm behind, before / so: 256 rows of 1024 columns 13.3 /
+    17.4, of 2048 19.2 / 22.8), up to 512 rows of 2048 columns and fewer, which the
+    library fills with small tiles, not below 5120 (256 of 1024x4096 15.2 / 18.0).
+    Up to 512 rows it takes the place of _tall_tile_plan: of 2568 sizes of 1408 to 10240
+    columns and 5120 to 28672 k .89 of its time on average, from .96 at 5120 k to .83 at
+    28672, 38 of them slower by more than 3 %, most at 11008 and 16384 k (192 rows of
+    8192x16384 the worst, 90 / 106); but of fewer columns a third loses (1024 1.02 on
+    average, 1152 .96, 1280 .97, 1408 .88).
+    us with the norm, weights out of HBM, before / so: 512 rows of 4096x4096 36 / 34, of
+    6144x4096 49 / 42, of 4096x14336 73 / 66, 264 of 4096x14336 64 / 53, 136 of 4096x4096
+    27 / 22, 640 of 4096x14336 143 / 84, 1024 159 / 107, 2039 217 / 197; but 1024 rows of
+    4096x4096 47 / 48. Of 3026 drawn sizes that it takes (1024 to 10240 columns, to 15360
+    k, 129 to 8192 rows) 31 are slower than before by more than 3 % (228 rows of 1024x5120
+    the worst, 1.14), .83 of the time on average."""
+    if M <= 128 or K < (5120 if M <= 512 and N <= 2048 else 3584) or K % 64 != 0 \
+            or N % 8 != 0 or (N + 512) * K >= 1 << 31 or N >= 1 << 21 \
+            or M <= 512 and N <= 1280 and _tall_tile_plan(M, N, K):
         return None
     out = M * N / 1e6
     best = None
     for tile in _WIDE_PARTS:
         n = -(-M // (32 * tile[0])) * -(-N // (32 * tile[1]))
-        most = min(8, 256 // n, K // 128)
+        most = min(8, 256 // n, K // 1024)
         for parts in {most, -(-most // 2)}:
             if parts >= 2:
                 plan = _wide_time(M, N, K, tile, parts) + parts * out, tile, parts

@@ -149,12 +149,14 @@ def test_tall_products_in_parts(M, N, K):
     if not wins:
         return
     assert plan[1] > 1
+    wide = ops._wide_parts_plan(M, N, K)
+    assert (wide is not None) == (N > 1280)
     rnd = _gen(M + N)
     x, w = rnd(M, K).bfloat16(), (rnd(N, K) * K ** -0.5).bfloat16()
     ref = x.double() @ w.double().T
     size = x.double().abs() @ w.double().abs().T
     parts = ops.linear_auto(x, w, parts=True)
-    assert parts.shape == (plan[1], M, N) and parts.dtype == torch.float32
+    assert parts.shape == ((wide or plan)[1], M, N) and parts.dtype == torch.float32
     # fp32 sums of terms that add up to `size`, then rounded to bf16 once
     assert bool(((parts.double().sum(0) - ref).abs()
                  <= size * 2.0 ** -18).all())

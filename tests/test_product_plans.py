@@ -25,6 +25,27 @@ def test_tall_products_from_some_length_and_up_to_some_width(M, K):
     assert changes <= (2 if K < 6144 else 1), changes
 
 
+@pytest.mark.parametrize("M", [129, 192, 256, 264, 384, 400, 512])
+@pytest.mark.parametrize("N", [1408, 2056, 2560, 4096, 5120, 6144, 8192])
+def test_parts_of_the_wide_tiles_have_no_line_in_long_rows(M, N):
+    """What the tiles of few rows cut over k, the wide ones do at any length."""
+    for K in range(5120, 16385, 512):
+        if ops._tall_tile_plan(M, N, K):
+            assert ops._wide_parts_plan(M, N, K), K
+    # narrow products stay with the others
+    assert ops._wide_parts_plan(M, 1280, 6144) is None
+
+
+@pytest.mark.parametrize("M", [129, 256, 400, 512, 640, 1024])
+def test_no_parts_of_less_than_1024_k(M):
+    for N in range(1024, 8193, 256):
+        assert not ops._wide_parts_plan(M, N, 3520)
+        for K in range(3584, 8193, 256):
+            plan = ops._wide_parts_plan(M, N, K)
+            assert plan is None or K // plan[1] >= 1024
+            assert plan is None or M > 512 or N > 2048 or K >= 5120
+
+
 @pytest.mark.parametrize("M", [1, 8, 16, 17, 64, 65, 128])
 def test_tiles_that_end_in_the_activation(M):
     """Uncut tiles of 64 or 128 columns do; of 64 not where two runs of 32 rows
