@@ -776,17 +776,20 @@ def _wide_time(M: int, N: int, K: int, tile, parts: int = 1) -> float:
     return 2 + end * rounds + math.ceil(K / 64 / parts) * (step * rounds + full * n / 256)
 
 
-def _wide_tile(M: int, N: int, K: int, tiles, base: float):
+def _wide_tile(M: int, N: int, K: int, tiles, base: float, rate: float = 1250e6,
+               end: int = 0):
     """The tile of the least time for N weight rows, where that is no more than the
     library takes for its fixed part, `base`, its bytes at 6 TB/s and its products at
-    1250 TFLOP/s (the root of their squares), else None."""
+    `rate`, with `end` k more for the end of its tiles (the root of their squares), else
+    None."""
     if K % 64 != 0 or K < 128 or (N + 512) * K >= 1 << 31 \
             or N >= 1 << 21 or M * max(N, K) >= 1 << 40:
         return None
 
     time, best = min((_wide_time(M, N, K, tile), tile) for tile in tiles)
     moved = 2 * (N * K + M * (N + K)) / 6e6
-    return best if time <= base + math.hypot(moved, 2 * M * N * K / 1250e6) else None
+    library = base + math.hypot(moved, 2 * M * N * (K + end) / rate)
+    return best if time <= library else None
 
 
 @functools.lru_cache(maxsize=4096)
@@ -850,16 +853,21 @@ def _wide_parts_plan(M: int, N: int, K: int):
 def _wide_rows_tile(M: int, N: int, K: int):
     """The tile of a product of many rows, or None for the library. Whole tiles of 256
     x 256 that fill their rounds are the library's too, and as often slower (.84 to 1.2
-    of its time): those are left to it, what fills smaller tiles better is taken. Of
-    2688 sizes (1024 to 24576 columns, 1024 to 14336 k, 264 to 8192 rows) 1529, 21 of
-    them slower by more than 3 % (768 rows of 18432 x 1024 the worst, 1.1), .84 of the
-    time of what took them before on average. us, before / this: 2039 rows of
-    6144x4096 84 / 75, of 4096x4096 62 / 56, 4188 of 5120x2048 82 / 77, of 2048x4096 65
-    / 58; but 512 of 4096x2560 and long rows of few columns (384 rows of 3584x7168 35 /
-    47) are left."""
+    of its time): those are left to it, what fills smaller tiles better is taken.
+    The library is uneven: by `_wide_tile`'s sum its times spread by 12 %, and rows and
+    columns that its tiles divide are its fast ones, so the sum is that of its better
+    third. By 9 us and 1250 TFLOP/s, its average, 161 of 1698 taken sizes of a grid of
+    such numbers were slower than before by more than 3 %, to 1.27 (384 rows of
+    3584x2560, us, before / this, 18.4 / 23.3; 5000 of 4096x11008 355 / 380).
+    Of that grid (1024 to 24576 columns, 1024 to 14336 k, 264 to 8192 rows) 1127 are
+    taken, 47 of them slower by more than 3 % (4000 rows of 2560x2048 the worst, 1.10),
+    .90 of the time of what took them before on average; of 3937 drawn sizes 66 (1.10),
+    .86. us, weights out of HBM, before / this: 2039 rows of 6144x4096 99 / 89, of
+    4096x4096 72 / 64, of 4096x14336 216 / 191; but 512 of 4096x2560 and long rows of
+    few columns (384 rows of 3584x7168 35 / 47) are left."""
     if M <= 256 or N % 8 != 0:
         return None
-    tile = _wide_tile(M, N, K, _WIDE_ROWS, 9)
+    tile = _wide_tile(M, N, K, _WIDE_ROWS, 6, 1400e6, 192)
     return None if tile == (8, 8) else tile
 
 

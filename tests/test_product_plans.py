@@ -46,6 +46,17 @@ def test_no_parts_of_less_than_1024_k(M):
             assert plan is None or M > 512 or N > 2048 or K >= 5120
 
 
+def test_products_that_the_library_fills_are_its_own():
+    """Sizes at which it is the faster one, and ones at which it is not."""
+    for M, N, K in ((384, 3584, 2560), (768, 2048, 2560), (1536, 1024, 2560),
+                    (512, 1536, 2048), (1024, 1024, 2048), (384, 8192, 3072),
+                    (640, 1536, 2048), (2560, 3584, 7168), (5000, 4096, 11008)):
+        assert ops._wide_rows_tile(M, N, K) is None, (M, N, K)
+    for M, N, K in ((768, 1536, 1024), (2039, 4096, 4096), (2039, 6144, 4096),
+                    (7000, 3584, 2560), (300, 24576, 7168), (5000, 8192, 14336)):
+        assert ops._wide_rows_tile(M, N, K), (M, N, K)
+
+
 @pytest.mark.parametrize("M", [1, 8, 16, 17, 64, 65, 128])
 def test_tiles_that_end_in_the_activation(M):
     """Uncut tiles of 64 or 128 columns do; of 64 not where two runs of 32 rows
