@@ -796,15 +796,17 @@ def _wide_tile(M: int, N: int, K: int, tiles, base: float, rate: float = 1250e6,
 def _wide_silu_tile(M: int, N: int, K: int):
     """The tile of a product of many rows that ends in the activation, or None where
     the library's product and the activation behind it are as good; N columns, gate
-    and up. Of 3927 sizes (1024 to 24576 columns of the result, 1024 to 8192 k, 136 to
-    8192 rows, weights out of HBM) 3016 are taken, one of them slower by more than 3 %
-    (.96), .79 of the other's time on average; 404 that would gain more than 5 % are
-    not. us, library and activation / this, 4096 k: 512 rows of 28672 108 / 93, 2039
-    411 / 337, 8192 1422 / 1286; 512 of 22016 99 / 80; but 136 of 16384 columns and
-    3072 k are left, .91."""
+    and up. Of 6668 drawn sizes that it takes (1024 to 30000 weight rows, 1024 to 15360 k,
+    129 to 8192 rows, weights out of HBM) 63 are slower by more than 3 %, most beyond
+    6912 k (256 rows of 19712x15104 the worst, 1.12), .80 of the other's time on average.
+    With 13 us for the library's fixed part and the activation's small products lost,
+    164 of 4404 (512 rows of 1280x1024 11.8 / 15.1, 256 of 4096x1024 14.7 / 16.8). us,
+    library and activation / this, 4096 k: 512 rows of 28672 108 / 93, 2039 411 / 337,
+    8192 1422 / 1286; 512 of 22016 99 / 80; but 136 of 16384 columns and 3072 k are
+    left, .91."""
     if N % 16 != 0 or M <= 128:
         return None
-    return _wide_tile(M, N, K, _WIDE_SILU, 13)
+    return _wide_tile(M, N, K, _WIDE_SILU, 11)
 
 
 @functools.lru_cache(maxsize=4096)

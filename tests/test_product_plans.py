@@ -57,6 +57,15 @@ def test_products_that_the_library_fills_are_its_own():
         assert ops._wide_rows_tile(M, N, K), (M, N, K)
 
 
+def test_small_products_keep_the_activation_behind():
+    for M, N, K in ((512, 1280, 1024), (830, 1040, 1024), (768, 1344, 1024),
+                    (2048, 1024, 1280), (192, 2688, 1024), (256, 4096, 1024)):
+        assert ops._wide_silu_tile(M, N, K) is None, (M, N, K)
+    for M, N, K in ((512, 28672, 4096), (2039, 28672, 4096), (200, 22016, 4096),
+                    (1024, 8192, 2048), (4096, 2816, 1024)):
+        assert ops._wide_silu_tile(M, N, K), (M, N, K)
+
+
 @pytest.mark.parametrize("M", [1, 8, 16, 17, 64, 65, 128])
 def test_tiles_that_end_in_the_activation(M):
     """Uncut tiles of 64 or 128 columns do; of 64 not where two runs of 32 rows
