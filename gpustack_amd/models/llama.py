@@ -1037,10 +1037,11 @@ class MoEMLP(nn.Module):
                 and self.e <= 4096 and ops.hip_available())
 
     def _library_wins(self, T: int) -> bool:
-        """Long prompts of few large experts: the library's product of one
-        expert at a time (1100 to 1300 TFLOP/s) makes up for a loop that syncs
-        with the host and gathers the rows (about 130 us an expert) against
-        the tiles' 850. us of the layer, tiles against loop, at 4096 x 14336
+        """Long prompts of few large experts that tiles of 128 take (_wide_products
+        refuses one of the two products, for biases or another activation): the
+        library's product of one expert at a time (1100 to 1300 TFLOP/s) makes up for a
+        loop that syncs with the host and gathers the rows (about 130 us an expert)
+        against these tiles' 850. us of the layer, tiles against loop, at 4096 x 14336
         and two experts a row: 8 experts 4096 rows 3330 / 3790, 6656 rows
         5650 / 5740, 7168 rows 6190 / 5670, 8192 rows 7170 / 6340, 16384 rows
         15250 / 11210; 16 experts 12288 rows 10580 / 10990, 13632 rows 11960 /
@@ -1048,10 +1049,25 @@ class MoEMLP(nn.Module):
         16384 rows 7870 / 5590; 4 of 2048 x 8192 8192 rows 2060 / 2250, 11900
         rows 2890 / 2740. The line is one number of multiplications an expert
         in all of them (6812, 13624, 13624 and 11921 rows). A capture cannot
-        record the syncs."""
-        return (T * self.top_k * self.i * self.spec.hidden_size
-                >= 100_000_000_000 * self.e
-                and not torch.cuda.is_current_stream_capturing())
+        record the syncs.
+        Tiles of up to 320 rows are the faster ones on both sides of it: 8 experts 7168
+        rows 4240 / 5320, 8192 4600 / 5730, 16384 9350 / 10290, 32768 20120 / 19870; 16
+        experts 13632 rows 7980 / 10240, 32768 18570 / 19870; 8 of 4096 x 7168 16384
+        rows 4670 / 5640, 32768 10440 / 10500; 4 of 2048 x 8192 12000 rows 2110 / 2760,
+        32768 5810 / 6470; 2 of 4096 x 14336 4096 rows 2400 / 2520."""
+        rows = T * self.top_k
+        return (rows * self.i * self.spec.hidden_size >= 100_000_000_000 * self.e
+                and not torch.cuda.is_current_stream_capturing()
+                and not all(self._wide_products(rows, self.spec.hidden_size)))
+
+    def _wide_products(self, rows: int, h: int):
+        """Whether the first and the second product of `rows` assignments take tiles of
+        up to 320 rows (ops.moe_wide_wins), which know no bias and one activation."""
+        # down bias on tp rank 0 only
+        bias = self.down_b if self.comm.tp_rank == 0 else None
+        return (self.spec.moe_act != "clamped_swiglu" and self.gate_up_b is None
+                and ops.moe_wide_wins(rows, self.e, self.i, h, False),
+                bias is None and ops.moe_wide_wins(rows, self.e, h, self.i, True))
 
     def _fused_dispatch(self, x, experts, weights):
         """Sync-free grouped expert products, summed over the k axis."""
@@ -1076,9 +1092,7 @@ class MoEMLP(nn.Module):
         # down bias on tp rank 0 only: the TP all-reduce must sum it once
         db = self.down_b if self.comm.tp_rank == 0 else None
         h = x.shape[1]
-        wide_up = act_mode == 0 and self.gate_up_b is None \
-            and ops.moe_wide_wins(TK, self.e, self.i, h, False)
-        wide_down = db is None and ops.moe_wide_wins(TK, self.e, h, self.i, True)
+        wide_up, wide_down = self._wide_products(TK, h)
         order, s_tok, counts, offs, tiles, ntiles, *s_w = hip.moe_sort(
             flat, self.e, k, weights=flat_w if wide_down else None)
         act = x.new_empty(TK, self.i)

@@ -227,10 +227,16 @@ def test_rows_at_any_address(T):
     assert float((m(x).double() - ref).norm() / ref.norm()) < 2.0 ** -7
 
 
-@pytest.mark.parametrize("T,loop", [(12000, True), (11900, False)])
-def test_long_prompts_of_few_large_experts(monkeypatch, T, loop):
-    """Both sides of the line between the tiles and the library's loop."""
+@pytest.mark.parametrize("T,loop,wide", [(12000, True, False), (11900, False, False),
+                                         (12000, False, True)])
+def test_long_prompts_of_few_large_experts(monkeypatch, T, loop, wide):
+    """Both sides of the line between the tiles of 128 rows and the library's loop, and
+    tiles of up to 320 rows, which have none."""
+    from gpustack_amd import ops
+
     m, g = _moe(4, 2, 2048, 8192)
+    if not wide:
+        monkeypatch.setattr(ops, "moe_wide_wins", lambda *a: False)
     x = torch.randn(T, 2048, generator=g, device="cuda").bfloat16()
     taken = []
     for name in ("_fused_dispatch", "_loop_dispatch"):
