@@ -1241,19 +1241,18 @@ PROMPT_PORTION = 32
 def prompt_kernel_wins(seq_news, max_ctx: int, heads: int, window: int) -> bool:
     """Where the prompt kernel is the faster one. Tiles of 16 rows are many
     workgroups that may cut a long walk over the keys into parts, tiles of 128
-    few that read every key once, so the line is the number of 16-row tiles, two
-    workgroups a CU, and a quarter more where the walk is long; a whole prompt
-    of up to 64 rows is one tile either way. us, 16-row tiles / prompt kernel, 16
-    heads on 4 unless said: one whole prompt of 64 rows 8.7 / 8.8, two of 32 in 64
-    heads 8.7 / 7.1, 100 10.2 / 11.6, 300 15.4 / 15.9; 100 behind 200 14.7 / 18.4;
-    512 rows (512 tiles) 33 / 23, behind 1000 56 / 55, behind 4000 117 / 138,
-    behind 8000 195 / 276, in a window of 1024 there 50 / 45; 2 x 300 (608) behind
-    8000 242 / 265; 1000 rows (1008) behind 8000 359 / 290; 200 (208) behind 4000
-    58 / 126; 32 heads on 8, 8 x 200 behind 1000 182 / 66."""
+    few that read every key once, so the line is the number of 16-row tiles, three
+    workgroups a CU; a whole prompt of up to 64 rows is one tile either way. us, 16-row
+    tiles (paged_attn_waves_kernel) / prompt kernel, 16 heads on 4: one whole prompt of
+    64 rows 8.6 / 8.6, 100 8.9 / 11.6, 300 11.9 / 15.7; 100 behind 200 11.4 / 18.1; 512
+    rows (512 tiles) 16 / 23, behind 1000 35 / 54, behind 4000 90 / 133, behind 8000 162
+    / 248, in a window of 1024 there 28 / 44; 2 x 300 (608) behind 8000 210 / 239; 700
+    (704) behind 1000 49 / 57, behind 8000 237 / 248; 1000 rows (1008) behind 1000 69 /
+    67, behind 8000 319 / 262; 200 (208) behind 4000 53 / 124. Of 940 batches (8 to 64
+    heads, 32 to 2000 rows) 16 are on the wrong side by more than 3 %, to 1.22."""
     tiles = sum((n + 15) // 16 for n in seq_news if n >= PROMPT_PORTION) * heads
     span = min(max_ctx, window) if window > 0 else max_ctx
-    return tiles >= 640 or tiles >= 512 and span <= 2048 \
-        or tiles > 0 and span <= 64
+    return tiles >= 768 or tiles > 0 and span <= 64
 
 
 def build_prompt_tiles(seq_starts, seq_hists, seq_news, device):

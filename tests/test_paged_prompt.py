@@ -43,8 +43,10 @@ def test_every_row_and_head_has_one_tile(seqs, heads, kv_heads, window):
 
 
 @pytest.mark.parametrize("news,ctx,heads,window,wins", [
-    ([512], 1512, 16, 0, True), ([512], 4512, 16, 0, False),
-    ([512], 8512, 16, 1024, True), ([1000], 9000, 16, 0, True),
+    ([512], 1512, 16, 0, False), ([512], 4512, 16, 0, False),
+    ([512], 8512, 16, 1024, False), ([1000], 9000, 16, 0, True),
+    ([700], 1700, 16, 0, False), ([300, 300], 8300, 16, 0, False),
+    ([768], 1768, 16, 0, True), ([200] * 8, 2200, 8, 1024, True),
     ([128] * 8, 8128, 8, 0, False), ([100], 300, 16, 0, False),
     ([300], 300, 16, 0, False), ([64], 64, 16, 0, True), ([31], 31, 64, 0, False),
     ([1] * 512, 9000, 64, 0, False)])
