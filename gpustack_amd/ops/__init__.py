@@ -1537,13 +1537,17 @@ def scan_run_rows(seq_news, heads: int, vdim: int,
     as the longest sequence's root has it, or as many as the chip has places.
     64 heads of 64, 1 x 500 rows 37 / 43, 1 x 1000 69 / 51, 1 x 4000 254 / 120, 2 x
     2000 130 / 98, but 3 x 2000 132 / 149, six of 301 to 1900 155 / 187; 16 heads of
-    128 the six 124 / 97, 4 x 1000 69 / 62; 8 of 64 4 x 4000 253 / 105. Over 194
-    batches 1.8 % above the best of eleven lengths each, at worst 1.27 (2600 rows,
-    1000 of them of one sequence, 64 heads 73 / 93)."""
+    128 the six 124 / 97, 4 x 1000 69 / 62; 8 of 64 4 x 4000 253 / 105. Whole ones pay
+    where a long sequence stands among many short ones: up to 185 places of a row of
+    the longest the sum of 12 uneven batches is .86 of it in runs (24 sequences, 1389 of
+    3928 rows in one, 311 / 146; but 657 of 913 70 / 84), beyond about even. Of 261
+    uneven batches none takes longer than on fp32 instructions by more than 1 %, .57 on average,
+    1.05 of the best of ten lengths each; at worst 2.1 (3322 of 5527 rows in one of 8,
+    128 heads 593 / 280)."""
     longest, rows = max(seq_news, default=0), sum(seq_news)
     groups = heads * ((vdim + 63) // 64)
     if exact:
-        if longest < 640 or longest * 160 <= rows * groups \
+        if longest < 640 or longest * 185 <= rows * groups \
                 or rows < SCAN_CHUNK_ROWS * len(seq_news):
             return 0
         size = max(12 * math.sqrt(longest), rows * groups / 512)

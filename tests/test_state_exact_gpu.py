@@ -140,3 +140,6 @@ def test_runs_of_exact_rows():
     assert rule([301, 1900, 821, 1340, 1660, 1100], 16, 128) > 0
     # too few rows a sequence for chunks
     assert rule([1900] + [1] * 85, 64, 64) == 0
+    # a long one among many short ones is cut
+    assert rule([87, 1, 19, 19, 33, 1389, 235, 2, 51, 13, 1, 1, 1, 1159, 5, 32, 4, 1,
+                 345, 12, 34, 18, 313, 153], 64, 64) == 512
