@@ -214,12 +214,13 @@ def qlinear(x, w, pack: "W4Pack | None", bias=None, parts: bool = False):
     Packed weights stay RESIDENT packed (the capacity goal). Up to 192 rows
     the packed product (ops/csrc/w4_gemm.hip) reads them as they are; more
     rows expand the weight into a transient bf16 tensor (allocator-cached)
-    and run the library GEMM at full MFMA rate. Measured, us, 64 rows:
-    28672x4096 33 against 105, 4096x14336 18 / 62, 128256x4096 134 / 584; 192
-    rows: 28672x4096 93 / 133, 4096x14336 48 / 104, 4096x4096 20 / 43; 256 rows
-    121 / 135, 63 / 74 and 25 / 34, but 10240x8192 reaches the expansion; above
-    128 rows a few columns more than two workgroups a CU take expand as well
-    (_w4_takes). GPUSTACK_AMD_W4_KERNEL=1 keeps the packed product up to 1024 rows."""
+    and run the library GEMM at full MFMA rate. us, weights out of memory, own /
+    expansion, 128 rows: 28672x4096 58 / 112, 4096x14336 37 / 69, 4096x4096 23 / 30; 192
+    rows: 82 / 132, 55 / 78 and 29 / 31, 22016x4096, whose last round has four
+    workgroups, 78 / 87; 256 rows: 105 / 135, 71 / 80, but 35 / 31. Of 231 sizes at 136 to
+    192 rows 3 are slower, 2048x2048 (to 1.17). At 200 to 256 rows most
+    would still gain (.6 to .95), products of 2048 to 6144 columns and up to 5120 k not
+    (to 1.28). GPUSTACK_AMD_W4_KERNEL=1 keeps the packed product up to 1024 rows."""
     if pack is None:
         return ops.linear_auto(x, w, parts) if bias is None \
             else F.linear(x, w, bias)
@@ -248,19 +249,11 @@ def qlinear(x, w, pack: "W4Pack | None", bias=None, parts: bool = False):
 
 def _w4_takes(x, pack: "W4Pack") -> bool:
     """True where the packed product takes x: rows up to its limit, whole
-    workgroups of 64 columns, scales that fit the LDS. Above 128 rows, three
-    tiles of rows, some widths leave a last round of a few workgroups behind the
-    512 that two a CU make; up to 4096 k the expansion is the faster one there
-    (us, own / expansion, 160 rows: 22016x4096 93 / 81, x3072 70 / 64, 23552x4096
-    93 / 89, but x2048 49 / 50, x5120 118 / 119, 24576x4096 94 / 93 and, below
-    them, 21760x4096 71 / 82)."""
+    workgroups of 64 columns, scales that fit the LDS."""
     import os
 
     always = os.environ.get("GPUSTACK_AMD_W4_KERNEL", "0") == "1"
     M, (N, K) = x.shape[0], pack.shape
-    if 128 < M and not always and K <= 4096 and N % 128 == 0 \
-            and 512 < 3 * (N // 128) <= 552:
-        return False
     return (x.is_cuda and x.dim() == 2 and 0 < M <= (1024 if always else 192)
             and N % 64 == 0 and K <= 131072)
 

@@ -529,9 +529,10 @@ bool w4_has(int N, int K) {
 }
 
 // Parts over k: one workgroup a CU, up to 16 rows of long rows two, 8 parts at
-// most. us at 16 rows: 4096 x 14336 (32 groups) 4 parts 20, 8 12, 16 13; 6144 x
-// 4096 (48) 2 12, 5 7.4, 8 7.3; 8192 x 28672 (64) 4 37, 8 29; 10240 x 8192 (80) 3
-// 16, 6 15; at 64 rows: 6144 x 4096 5 12, 8 15; 10240 x 8192 3 25, 6 30.
+// most. us at 16 rows in 8 waves: 4096 x 14336 (32 groups) 4 parts 20, 8 12, 16 13;
+// 6144 x 4096 (48) 2 12, 5 7.4, 8 7.3; 8192 x 28672 (64) 4 37, 8 29; 10240 x 8192 (80)
+// 3 16, 6 15; at 64 rows: 6144 x 4096 5 12, 8 15; 10240 x 8192 3 25, 6 30. In 16 waves
+// those taken are 12.0, 7.8, 30.7, 16.6, 12.4 and 23.0.
 int w4_splits(int M, int N, int K) {
   const int groups = N / (16 * w4_waves(N)), total = (K / W4_KC + 1) / 2;
   int splits = (M <= 16 && K >= 8192 ? 512 : 256) / groups;
@@ -541,40 +542,46 @@ int w4_splits(int M, int N, int K) {
 }
 
 // Products for which parts do not pay even where the next kernel adds them up: few
-// rows of short ones (at one row 6144 x 4096 7.1 against 7.3 and 4096 x 4096 5.3
-// against 6.0, which their consumer's reading costs; 4096 x 14336 11.4 / 12.8,
-// 8192 x 28672 29 / 39), and small ones (6144 x 1920 at 16 rows 5.0 / 5.3).
+// rows of short ones (at one row, with a norm behind, 6144 x 4096 10.0 against 12.3 and
+// 4096 x 4096 7.8 against 10.1, but 8192 x 28672 43 / 36), and small ones (6144 x 1920
+// at 16 rows 5.0 / 5.3). Of 640 sizes 81 of those that are cut take more than 3 % longer
+// than whole, to 1.28 (one row of 4096 x 8192 10.9 / 14.0), 44 of the others would gain
+// that (48 rows of 3072 x 4096 19 / 14).
 bool w4_cuts(int M, int N, int K) {
   return (M >= 8 || K >= 8192) && (long)N * K > 12l << 20 &&
          w4_splits(M, N, K) > 1;
 }
 
-// The whole result: rows where these are few and the product is narrow (28672 x
-// 4096 at one row 20.7 against 21.4; 57344 x 8192 70 / 65), unless k is long and
-// parts with a join (3 us) gain more (4096 x 14336 at 16 rows 20 against 12 + 3),
-// and for small products (6144 x 1920 at 64 rows 10 against 8 + 3).
+// The whole result: rows where these are few and the product is narrow, as far as a
+// wave of the rows' form has two column tiles (w4_rows_launch; us against the tiles, 24576
+// x 4096 at one row 16.5 / 17.4, at 8 18.4 / 17.2; with four tiles 28672 x 4096 21.1 /
+// 17.7 and 22.1 / 18.0), unless k is long and parts with a join (3 us) gain more (4096
+// x 14336 at 16 rows 20 against 12 + 3), and for small products (6144 x 1920 at 64 rows
+// 10 against 8 + 3). Left on the wrong side: more than 8 rows of 12288 columns and more
+// that do not end in the activation (24576 x 4096 at 16 rows 22.4 / 17.6), 10240 columns
+// and more of 8192 k and more at any (8 rows of 10240 x 14336 38 / 25).
 bool w4_by_rows(int M, int N, int K) {
-  if (M <= 16 && N < 32768 && !(M > 8 && K >= 8192)) return true;
+  if (M <= 16 && N < 28672 && !(M > 8 && K >= 8192)) return true;
   return M <= 64 && (long)N * K <= 12l << 20;
 }
 
 // Whether a product of N columns (gate and up) ends in the activation. Where the
 // product is one launch of whole tiles by itself it does, and saves the
-// activation's launch (us without / with, 28672 x 4096 at 17 rows 28 / 26, 64 rows
-// 36 / 34, 192 rows 97 / 95; 17920 x 2048 at 64 rows 21 / 18). Products cut over k
-// do not: their chain of k would run whole on less than one workgroup a CU (16384 x
-// 4096 at 64 rows 27 / 33, 22016 x 8192 at 16 rows 36 / 43).
-// In the place of the rows' form, up to 16 rows, the tiles pay for a chain of a
-// microsecond for every 256 k, however few rows there are, and the rows' form for
+// activation's launch (us without / with, 28672 x 4096 at 16 rows 20.6 / 18.2, 24 rows
+// 24.4 / 21.9, 64 rows 31.5 / 28.0, 192 rows 85 / 80; 17920 x 2048 at 64 rows 18.7 /
+// 15.7). Products cut over k do not: their chain of k would run whole on less than one
+// workgroup a CU (16384 x 4096 at 64 rows 25 / 27; 22016 x 8192 at 16 rows, right on
+// it, 33.9 / 33.5).
+// In the place of the rows' form, up to 16 rows, the tiles pay for a chain of .8
+// microseconds for every 256 k, however few rows there are, and the rows' form for
 // its columns and for x, which it reads again in every workgroup: the line grows
-// with both (22016 x 2048 at one row 12.5 / 12.7, x 4096 18.6 / 23.1, at 12 rows 22.1
-// / 21.8, at 16 24.3 / 22.4; 28672 x 4096 at one row 24.2 / 24.8, at 8 rows 24.7 /
-// 24.0; 24576 x 4096 at 2 rows, right on it, 19.5 / 23.2). It lies where the tiles
-// take 1.5 us more in these loops: in a captured step the activation costs that
-// much besides (a step of 4 layers at one row 372 / 368, at 4 rows 380 / 371).
+// with both (22016 columns at one row x 2048 12.4 / 10.7, x 4096 18.2 / 17.0, x 5120,
+// right on it, 21.5 / 22.3, x 8192 31.2 / 33.0; 17920 x 5120 at 2 rows 21.0 / 21.6, at 8
+// rows 23.9 / 21.6). It lies where the tiles take .8 us more in these loops: in a captured step
+// the activation costs 1.5 us more besides.
 bool w4_silu_wins(int M, int N, int K) {
   if (w4_by_rows(M, N, K))
-    return M <= 16 && N > 16384 && K < 256 * (M + 6) + (N - 16384) / 4;
+    return M <= 16 && N > 16384 && K < 256 * (M + 16) + (N - 16384) / 4;
   return w4_splits(M, N, K) == 1;
 }
 

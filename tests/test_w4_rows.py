@@ -17,8 +17,8 @@ def _takes(M, N, K, **kw):
     (193, 28672, 4096, False), (64, 96, 128, False), (64, 64, 131072, True),
     (64, 64, 131200, False),
     # a last round of 4 to 40 workgroups behind 512
-    (128, 22016, 4096, True), (129, 22016, 4096, False),
-    (192, 21888, 2048, False), (160, 23552, 4096, False),
+    (128, 22016, 4096, True), (129, 22016, 4096, True),
+    (192, 21888, 2048, True), (160, 23552, 4096, True),
     (160, 21760, 4096, True), (160, 24576, 4096, True),
     (160, 22016, 5120, True)])
 def test_rows_of_a_packed_product(monkeypatch, M, N, K, takes):

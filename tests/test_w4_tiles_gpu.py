@@ -81,7 +81,8 @@ def test_product_ends_in_the_activation(M, N, K):
     (17, 16640, 4096, True), (192, 22016, 12288, True),   # whole tiles anyway
     (1, 32768, 4096, True), (1, 32768, 8192, False),      # cut from 8192 k on
     (64, 16384, 4096, False), (16, 22016, 8192, False),   # cut over k
-    (1, 22016, 4096, False), (2, 24576, 4096, False),     # the rows' form
+    (1, 22016, 6144, False), (2, 17920, 5120, False),     # the rows' form
+    (1, 22016, 4096, True), (2, 24576, 4096, True), (8, 17920, 5120, True),
     (16, 22016, 4096, True), (1, 28672, 4096, True), (1, 22016, 2048, True),
     (1, 8192, 128, False)])
 def test_where_it_ends_in_the_activation(monkeypatch, M, N, K, wins):
