@@ -422,7 +422,10 @@ DEVICE_INLINE u32x2 lds_read_tr(const unsigned short* p) {
 // two prompts of 1024 rows 34.5 / 29.4, four of 512 22.8 / 20.5, one of 2039 48.1 / 47.2
 // (behind 6001 245 / 238, 2048 behind 2000 113 / 108), 16 heads, 4000 rows 85.4 / 83.8,
 // 8 heads, 7999 158 / 155. Heads that do not divide 256 gain or lose by the list (28
-// heads, 2039 rows 45.4 / 43.9, three prompts of 700 24.6 / 26.0) and stay.
+// heads, 2039 rows 45.4 / 43.9, three prompts of 700 24.6 / 26.0) and stay. Several
+// prompts lie in the batch's order, not by size, and gain or lose by that: of 43 drawn
+// batches 1.00 of the time, .79 (six of 231 rows behind 0 to 4000 113 / 89) to 1.16 (1354
+// and five of 48 to 506 32 / 37); of 35 single prompts .98, .96 to 1.04.
 DEVICE_INLINE int tile_of(int Hq) {
   const int n = gridDim.x / Hq, at = blockIdx.x / Hq, chip = 256 / Hq;
   const bool twice = 256 % Hq == 0 && n > chip && n <= 2 * chip;

@@ -21,7 +21,7 @@
 // two steps ahead of the rows is as far as the weights get. 128 experts of 1536 +
 // 2048 x 2048 + 768 at 254 rows each: 202 + 153 us, 141 + 100 without the memory, 165
 // + 111 without the loads (tiles of 128: 283 + 180); 188 rows 187 + 133 (232 + 149); 8
-// of 4096 x 14336 at 1024 rows 1560 + 830 (2160 + 1200), 1230 TFLOP/s.
+// of 4096 x 14336 at 1024 rows 1630 + 830 (2160 + 1200), 1170 TFLOP/s.
 // Tried: the loads of a step in one half, weights a step further ahead 1600 -> 1680;
 // tiles of every 32 rows no faster; whole parts of 320 and a rest, large ones dealt
 // first: even at 254 rows, 250 -> 266 at 500.

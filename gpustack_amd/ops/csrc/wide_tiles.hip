@@ -26,7 +26,7 @@
 // them to other registers and copies, all 256 being taken. It does not see the products
 // in the asm, so the waits before their results are read stand here (s_nop), and a loop
 // of one body keeps it from copying them in between.
-// With the activation, 28672 x 4096: 8192 rows 1228 us (1566 TFLOP/s), 2039 rows 337 in
+// With the activation, 28672 x 4096: 8192 rows 1278 us (1505 TFLOP/s), 2039 rows 341 in
 // tiles of 256 x 224 (256 x 256, whose last round is half empty, 354), 512 rows out of
 // HBM 91 (94); the library's product and the activation behind it 1290 + 127, 353 + 31,
 // 97 + 11. Without: 2039 rows of 6144 x 4096 in tiles of 256 x 192 75 (library 84), of
