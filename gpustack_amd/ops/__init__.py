@@ -692,13 +692,11 @@ def linear_auto(x, w, parts: bool = False):
     if _own_products(x, w):
         M, K = x.shape
         N = w.shape[0]
-        eager = M > 128 and not torch.cuda.is_current_stream_capturing()
-        wide = _wide_parts_plan(M, N, K, eager) if parts else None
+        wide = _wide_parts_plan(M, N, K) if parts else None
         if wide and _wide_take(x, w):
             return _load_hip().wide_parts(x, w, wide[1], *wide[0])
         plan = parts and _parts_plan(M, N, K) or _rows_tile_plan(M, N, K)
-        wide = None if parts and plan and plan[1] > 1 \
-            else _wide_rows_tile(M, N, K, eager)
+        wide = None if parts and plan and plan[1] > 1 else _wide_rows_tile(M, N, K)
         if wide and _wide_take(x, w):
             out = torch.empty(M, N, dtype=x.dtype, device=x.device)
             _load_hip().wide_rows(out, x, w, *wide)
@@ -780,18 +778,17 @@ def _wide_time(M: int, N: int, K: int, tile, parts: int = 1) -> float:
     return 2 + end * rounds + math.ceil(K / 64 / parts) * (step * rounds + full * n / 256)
 
 
-# us of a product that is bound by the host outside of a capture: a call of the library
-# costs it 18 to 20, one of these 7, and a step of a few hundred rows is such calls (a
-# prompt of 312 rows in the hybrid stack 847 us with the library's products of 2048 k,
-# 754 with these). Less than that by as much as _wide_time is below the times (1.2 to 1.45).
-_HOST_US = 14
-
-
 def _wide_tile(M: int, N: int, K: int, tiles, base: float, products: float,
-               host: float = 0):
+               host: float):
     """The tile of the least time for N weight rows, where that is no more than the
     library takes for its fixed part, `base`, its bytes at 6 TB/s and its products (the
-    root of their squares), or than its call costs the host, else None."""
+    root of their squares), else None.
+    Short products wait for the host where the step is not captured: a call of the library
+    costs it 18 to 20 us, one of these 7, and a step of a few hundred rows is such calls (a
+    prompt of 312 rows in the hybrid stack 847 us with the library's products of 2048 k,
+    754 with these). Their fixed part is `host`, up to 5 us more as _wide_time has them,
+    which is 1.2 to 1.45 below their times. Captured steps take the same kernels as their
+    warm-up, though some take the device longer: 512 rows of 1536x2048 12.5 / 15.3."""
     if K % 64 != 0 or K < 128 or (N + 512) * K >= 1 << 31 \
             or N >= 1 << 21 or M * max(N, K) >= 1 << 40:
         return None
@@ -799,29 +796,30 @@ def _wide_tile(M: int, N: int, K: int, tiles, base: float, products: float,
     time, best = min((_wide_time(M, N, K, tile), tile) for tile in tiles)
     moved = 2 * (N * K + M * (N + K)) / 6e6
     library = base + math.hypot(moved, products)
-    return best if time <= max(library, host) else None
+    short = host + min(5, math.hypot(moved, 2 * M * N * K / 1250e6))
+    return best if time <= max(library, short) else None
 
 
 @functools.lru_cache(maxsize=4096)
-def _wide_silu_tile(M: int, N: int, K: int, eager: bool = False):
+def _wide_silu_tile(M: int, N: int, K: int):
     """The tile of a product of many rows that ends in the activation, or None where
     the library's product and the activation behind it are as good; N columns, gate
-    and up. Of 6668 drawn sizes that it takes (1024 to 30000 weight rows, 1024 to 15360 k,
+    and up. Of 6668 drawn sizes that it takes by 11 (1024 to 30000 weight rows, 1024 to 15360 k,
     129 to 8192 rows, weights out of HBM) 63 are slower by more than 3 %, most beyond
     6912 k (256 rows of 19712x15104 the worst, 1.12), .80 of the other's time on average.
-    With 13 us for the library's fixed part and the activation's small products lost,
-    164 of 4404 (512 rows of 1280x1024 11.8 / 15.1, 256 of 4096x1024 14.7 / 16.8). us,
+    Short ones, with 13 us for the library's fixed part and the activation's, are slower on
+    the device as often as not, where both calls cost the host 25 (512 rows of 1280x1024
+    11.8 / 15.1, 256 of 4096x1024 14.7 / 16.8). us,
     library and activation / this, 4096 k: 512 rows of 28672 108 / 93, 2039 411 / 337,
     8192 1422 / 1286; 512 of 22016 99 / 80; but 136 of 16384 columns and 3072 k are
-    left, .91. `eager`: not captured, where the two calls cost the host more than that."""
+    left, .91."""
     if N % 16 != 0 or M <= 128:
         return None
-    return _wide_tile(M, N, K, _WIDE_SILU, 11, 2 * M * N * K / 1250e6,
-                      eager and _HOST_US + 3)
+    return _wide_tile(M, N, K, _WIDE_SILU, 11, 2 * M * N * K / 1250e6, 13)
 
 
 @functools.lru_cache(maxsize=4096)
-def _wide_parts_plan(M: int, N: int, K: int, eager: bool = False):
+def _wide_parts_plan(M: int, N: int, K: int):
     """(tile, parts over k) of a product of many rows whose consumer adds the parts up
     (wide_kernel in ops/csrc/wide_tiles.hip), or None. As many parts as let its 256
     workgroups have one tile each, at most 8 and each of 1024 k and more, or half as many:
@@ -841,11 +839,8 @@ def _wide_parts_plan(M: int, N: int, K: int, eager: bool = False):
     27 / 22, 640 of 4096x14336 143 / 84, 1024 159 / 107, 2039 217 / 197; but 1024 rows of
     4096x4096 47 / 48. Of 3026 drawn sizes that it takes (1024 to 10240 columns, to 15360
     k, 129 to 8192 rows) 31 are slower than before by more than 3 % (228 rows of 1024x5120
-    the worst, 1.14), .83 of the time on average.
-    `eager`: not captured, where up to 256 rows shorter products than the library's call
-    are taken from 2560 k on; of more rows _wide_rows_tile has them."""
-    short = K < (5120 if M <= 512 and N <= 2048 else 3584)
-    if M <= 128 or short and not (eager and M <= 256 and K >= 2560) or K % 64 != 0 \
+    the worst, 1.14), .83 of the time on average."""
+    if M <= 128 or K < (5120 if M <= 512 and N <= 2048 else 3584) or K % 64 != 0 \
             or N % 8 != 0 or (N + 512) * K >= 1 << 31 or N >= 1 << 21 \
             or M <= 512 and N <= 1280 and _tall_tile_plan(M, N, K):
         return None
@@ -858,8 +853,6 @@ def _wide_parts_plan(M: int, N: int, K: int, eager: bool = False):
             if parts >= 2:
                 plan = _wide_time(M, N, K, tile, parts) + parts * out, tile, parts
                 best = min(best or plan, plan)
-    if short:
-        return best[1:] if best and best[0] <= _HOST_US else None
     behind = 10 + N * K / 20e6 + .85 * out
     whole = min(_wide_time(M, N, K, tile) for tile in _WIDE_ROWS) + .3 * out
     if best is None or best[0] + behind > (.97 if M > 256 else .95) * (whole + behind):
@@ -868,28 +861,27 @@ def _wide_parts_plan(M: int, N: int, K: int, eager: bool = False):
 
 
 @functools.lru_cache(maxsize=4096)
-def _wide_rows_tile(M: int, N: int, K: int, eager: bool = False):
+def _wide_rows_tile(M: int, N: int, K: int):
     """The tile of a product of many rows, or None for the library. Whole tiles of 256
     x 256 that fill their rounds are the library's too, and as often slower (.84 to 1.2
     of its time): those are left to it, what fills smaller tiles better is taken.
     The library is uneven: its times spread by 14 % around any such sum, and rows and
     columns that its tiles divide are its fast ones. The sum is that of whole tiles of 128
     x 256, each with 192 k for its end, at 1250 TFLOP/s, and 6 us beside. (By M N K, and
-    9 us, 343 of 6383 drawn sizes that were taken were slower than the library by more
-    than 3 %, 85 by more than 10, to 1.33: 384 rows of 3584x2560, us, library / this,
-    18.4 / 23.3.) Of 7762 drawn sizes (1024 to 30000 columns, 1024 to 15360 k, 257 to 8192
-    rows) 6390 are taken, 237 of them slower by more than 3 %, 10 by more than 10, to
-    1.21, .87 of the library's time on average; of a grid of numbers that its tiles divide
-    1539 of 1698, 107 and 7, to 1.12, .91 (5000 rows of 4096x11008 355 / 380).
+    9 us, it lost more where products are longer than the library's call: 384 rows of
+    3584x2560 18.4 / 23.3 us, library / this.) Of 7762 drawn sizes (1024 to 30000 columns,
+    1024 to 15360 k, 257 to 8192 rows) 6390 are taken by that, 237 of them slower on the
+    device by more than 3 %, 10 by more than 10, to 1.21, .87 of the library's time on
+    average, and 257 short ones, 121 of them slower by more than 3 %, to 1.33;
+    of a grid of numbers that its tiles divide 1539 of 1698, 107 and 7, to 1.12, .91 (5000
+    rows of 4096x11008 355 / 380), and 42, 21 of them, to 1.23.
     us, weights out of HBM, before / this: 2039 rows of 6144x4096 99 / 89, of 4096x4096
     72 / 64, of 4096x14336 216 / 191; but 512 of 4096x2560 and long rows of few columns
-    (384 rows of 3584x7168 35 / 47) are left. `eager`: not captured, where products
-    shorter than the library's call are taken, too."""
+    (384 rows of 3584x7168 35 / 47) are left."""
     if M <= 256 or N % 8 != 0:
         return None
     rows, columns = (M + 127) // 128 * 128, (N + 255) // 256 * 256
-    tile = _wide_tile(M, N, K, _WIDE_ROWS, 6, 2 * rows * columns * (K + 192) / 1250e6,
-                      eager and _HOST_US)
+    tile = _wide_tile(M, N, K, _WIDE_ROWS, 6, 2 * rows * columns * (K + 192) / 1250e6, 9)
     return None if tile == (8, 8) else tile
 
 
@@ -902,8 +894,7 @@ def linear_silu(x, w):
         return None
     M, K = x.shape
     plan = _silu_plan(M, w.shape[0], K)
-    wide = None if plan else _wide_silu_tile(
-        M, w.shape[0], K, not torch.cuda.is_current_stream_capturing())
+    wide = None if plan else _wide_silu_tile(M, w.shape[0], K)
     if not (plan or wide) or not (_wide_take if wide else _rows_take)(x, w):
         return None
     out = torch.empty(M, w.shape[0] // 2, dtype=x.dtype, device=x.device)

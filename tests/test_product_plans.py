@@ -49,38 +49,21 @@ def test_no_parts_of_less_than_1024_k(M):
 def test_products_that_the_library_fills_are_its_own():
     """Sizes at which it is the faster one, and ones at which it is not."""
     for M, N, K in ((384, 3584, 2560), (768, 2048, 2560), (1536, 1024, 2560),
-                    (512, 1536, 2048), (1024, 1024, 2048), (384, 8192, 3072)):
+                    (384, 8192, 3072)):
         assert ops._wide_rows_tile(M, N, K) is None, (M, N, K)
     for M, N, K in ((768, 1536, 1024), (2039, 4096, 4096), (2039, 6144, 4096),
                     (7000, 3584, 2560), (300, 24576, 7168), (5000, 8192, 14336)):
         assert ops._wide_rows_tile(M, N, K), (M, N, K)
 
 
-@pytest.mark.parametrize("rule,first", [(ops._wide_rows_tile, 257),
-                                        (ops._wide_silu_tile, 129),
-                                        (ops._wide_parts_plan, 129)])
-def test_products_shorter_than_a_call_of_the_library(rule, first):
-    """Outside of a capture they are taken as well, long ones by the one line."""
-    for M in (first, 256 if first == 129 else 312, 600, 1000, 4000):
-        for N in range(1024, 16385, 512):
-            for K in (1024, 2048, 2560, 3072, 4096, 7168, 14336):
-                captured, eager = rule(M, N, K), rule(M, N, K, True)
-                assert not captured or eager == captured
-                # 17 us at the rate of the matrix cores
-                assert eager == captured or 2 * M * N * K < 17 * 2500e6
-    for M, N, K in ((312, 3072, 2048), (312, 1536, 2048), (512, 2048, 2048)):
-        assert ops._wide_rows_tile(M, N, K, True), (M, N, K)
-    assert ops._wide_silu_tile(256, 4096, 1024, True)
-    assert ops._wide_parts_plan(256, 2048, 3072, True)
-
-
-def test_small_products_keep_the_activation_behind():
-    for M, N, K in ((512, 1280, 1024), (830, 1040, 1024), (768, 1344, 1024),
-                    (2048, 1024, 1280), (192, 2688, 1024), (256, 4096, 1024)):
-        assert ops._wide_silu_tile(M, N, K) is None, (M, N, K)
-    for M, N, K in ((512, 28672, 4096), (2039, 28672, 4096), (200, 22016, 4096),
-                    (1024, 8192, 2048), (4096, 2816, 1024)):
-        assert ops._wide_silu_tile(M, N, K), (M, N, K)
+def test_products_shorter_than_a_call_of_the_library():
+    """They are taken though some take the device a little longer."""
+    for M, N, K in ((312, 3072, 2048), (500, 3072, 2048), (646, 2048, 2048)):
+        assert ops._wide_rows_tile(M, N, K), (M, N, K)
+    assert ops._wide_silu_tile(768, 1344, 1024)
+    # longer ones, by the device alone
+    assert ops._wide_rows_tile(384, 4096, 2560) is None
+    assert ops._wide_silu_tile(144, 11264, 1536) is None
 
 
 @pytest.mark.parametrize("M", [1, 8, 16, 17, 64, 65, 128])
