@@ -13,8 +13,8 @@ void reshape_and_cache_launch(const void*, const void*, void*, void*, const long
 void greedy_sample_launch(long*, const void*, int, int, hipStream_t);
 void mla_decode_launch(float*, const void*, const void*, const int*, const int*, int, int, int, int, int, int, float, int*, hipStream_t);
 void qkv_store_launch(void*, const float*, int, const void*, const void*, const float*, const long*, const long*, void*, void*, long, int, int, int, int, float, int, int*, hipStream_t);
-struct DecodeParts { int n, least; };
-DecodeParts decode_parts(int, int, int, int, int, int);
+struct DecodeParts { int n, least, grouped; };
+DecodeParts decode_parts(int, int, int, int, int, int, int, int);
 void paged_attn_decode_launch(void*, const void*, const void*, const void*, const int*, const int*, float*, DecodeParts, int, int, int, int, int, float, long, int, const float*, int, float, int*, hipStream_t);
 void flash_prefill_launch(void*, const void*, const void*, const void*, const int*, const int*, const int*, int, int, int, int, int, float, long, long, long, const float*, int, float, int*, hipStream_t);
 void flash_prefill_paged_launch(void*, const void*, const void*, const void*, const int*, const int*, const int*, const int*, const int*, const int*, int, int, int, int, int, float, long, const float*, int, float, int*, hipStream_t);
@@ -326,9 +326,11 @@ void paged_attn_decode(at::Tensor out, at::Tensor q, at::Tensor k_cache,
   const int max_blocks = block_tables.size(1);
   const float* sink_ptr = sink_ptr_checked(sinks, Hq);
   int err = 0;
-  const DecodeParts parts = decode_parts(N, Hkv, max_blocks, D,
+  const int aligned = ((reinterpret_cast<uintptr_t>(k_cache.data_ptr()) |
+                        reinterpret_cast<uintptr_t>(v_cache.data_ptr())) & 15) == 0;
+  const DecodeParts parts = decode_parts(N, Hq, Hkv, max_blocks, D,
                                          is_fp8_cache(k_cache) ? 1 : 0,
-                                         (int)window);
+                                         (int)window, aligned);
   const int nsplit = parts.n;
   // this call's own workspace, from the stream's allocator
   at::Tensor part;
