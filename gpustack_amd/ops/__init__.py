@@ -631,22 +631,32 @@ def _parts_plan(M: int, N: int, K: int):
 def router_plan(T: int, E: int, H: int):
     """(columns of a tile, parts over k) of a router's product, whose parts the
     choice of the experts adds up, or None. us for both launches against a
-    cast, an fp32 library product and the choice, at 64 / 1024 / 4068 / 16384
-    rows: 64 experts of 2048 10 / 13 / 17 / 33 against 16 / 21 / 39 / 87, 128
-    of 2048 13 / 16 / 21 / 41 against 18 / 24 / 57 / 125, 256 of 4096 18 / 23 /
-    38 / 91 against 21 / 40 / 109 / 317; 512 of 2048 22 / 27 / 37 / 102 against
-    23 / 39 / 96 / 311, but at 128 rows 25 against 24. Four parts of narrow
-    tiles fill the chip for few rows; later the parts' own traffic counts (128
-    experts at 16384 rows 57)."""
+    cast, an fp32 library product and the choice, at 64 / 1024 / 4188 / 16384
+    rows: 64 experts of 2048 8.1 / 9.8 / 14.5 / 26 against 12 / 17 / 36 / 77, 128
+    of 2048 8.5 / 11 / 18 / 34 against 14 / 20 / 53 / 115, 256 of 4096 12 / 17 / 30 / 73
+    against 13 / 30 / 102 / 297; 512 of 2048 (with a choice that took 4 more) 22 / 27 / 37 /
+    102 against 23 / 39 / 96 / 311, but at 128 rows 25 against 24. Eight parts of narrow
+    tiles fill the chip for few rows (32 experts of 4096, eight / four parts: 64 rows 7.8
+    / 9.4, 8000 19.7 / 22.3; 64 of 2048 8.1 / 8.6, 2000 rows 11.4 / 11.8; 128 of 2048 at
+    1024 11.3 / 12.2, but 2000 14.8 / 13.5, 256 of 4096 at 64 14.0 / 11.6); later the
+    parts' own traffic counts (4188 rows of 64 experts 64 x 4 14.5, 32 x 4 16.5; of 128
+    64 x 2 17.7, 32 x 4 19.4, 128 x 2 21.7; of 256 128 x 4 30, 128 x 2 34), and one
+    is the best of 256 experts at 16384 (73, two 82)."""
     if E % 4 != 0 or H % 64 != 0 or H < 1024 or E > 512 or T == 0:
         return None
     if E > 256:
         if 64 < T < 256:
             return None
         return (64, 2) if T <= 2048 else (128, 2)
-    if T * E <= 1 << 19:
-        return 32, 4
-    return (128, 2) if E >= 128 else (64, 2)
+    if E <= 32:
+        return 32, 8
+    if E <= 64:
+        return (32, 8) if T <= 2500 else (64, 4) if T <= 12000 else (64, 2)
+    if E <= 128:
+        return (32, 8) if T <= 1400 else (32, 4) if T <= 2500 \
+            else (64, 2) if T <= 6000 else (128, 2)
+    return (32, 4) if T <= 2500 else (128, 4) if T <= 6000 \
+        else (128, 2) if T <= 12000 else (128, 1)
 
 
 def moe_wide_wins(rows: int, E: int, N: int, K: int, down: bool) -> bool:
