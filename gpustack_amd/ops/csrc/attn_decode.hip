@@ -102,21 +102,10 @@ DEVICE_INLINE f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
                                                  0, 0, 0);
 }
 
-// A value and the one of the lane 16 or 32 away, in either order, without the
-// LDS: as shuffles these exchanges, most of them in the sums at the end, were
-// 12 % of the kernel over 240 shapes (16 heads of 256, us: 512 x 40 keys
-// 53.6 -> 42.0, one x 300 12.2 -> 11.1; 32 of 128: 64 x 400 21.0 -> 19.2). The two
-// operands are kept apart, as in half_wave_max.
-template <int M>
-DEVICE_INLINE f32x2 with_lane(float v) {
-  const unsigned int a = __builtin_bit_cast(unsigned int, v);
-  unsigned int b = a;
-  asm("" : "+v"(b));
-  const auto r = M == 16 ? __builtin_amdgcn_permlane16_swap(a, b, false, false)
-                         : __builtin_amdgcn_permlane32_swap(a, b, false, false);
-  const unsigned int x = r[0], y = r[1];
-  return f32x2{__builtin_bit_cast(float, x), __builtin_bit_cast(float, y)};
-}
+// Sums and maxima over the key groups without the LDS: as shuffles these exchanges, most
+// of them in the sums at the end, were 12 % of the kernel over 240 shapes (16 heads of
+// 256, us: 512 x 40 keys 53.6 -> 42.0, one x 300 12.2 -> 11.1; 32 of 128: 64 x 400 21.0
+// -> 19.2).
 DEVICE_INLINE float sum_groups(float v) {
   f32x2 p = with_lane<16>(v);
   p = with_lane<32>(p[0] + p[1]);
@@ -783,13 +772,15 @@ void paged_attn_decode_kernel(
 }
 
 // Joins the parts of one (sequence, query head): a few KB that the decode
-// kernel left in the L2, bound by the launch.
+// kernel left in the L2, bound by the launch and two round trips, the length's and the
+// parts', of which eight at a time are on their way.
 template <int D>
 __global__ __launch_bounds__(D) void paged_attn_join_kernel(
     unsigned short* __restrict__ out,       // [N, Hq, D]
     const float* __restrict__ part,         // [N, Hkv, nsplit, GQ, D + 2]
     const int* __restrict__ seq_lens, int GQ, int nsplit, int least,
     const float* __restrict__ sinks, int window) {
+  constexpr int U = 8;
   const int seq = blockIdx.x, hq = blockIdx.y, Hq = gridDim.y;
   const int h = hq / GQ, gq = hq % GQ, d = threadIdx.x;
   const int len = seq_lens[seq];
@@ -800,19 +791,34 @@ __global__ __launch_bounds__(D) void paged_attn_join_kernel(
   const float* pp = part +
       (((long)seq * (Hq / GQ) + h) * nsplit * GQ + gq) * (D + 2);
   const long step = (long)GQ * (D + 2);
-  float M = -INFINITY;
-  for (int i = 0; i < n; ++i) M = fmaxf(M, pp[i * step + D]);
-  float num = 0.f, den = 0.f;
+  float M = -INFINITY, num = 0.f, den = 0.f;
   if (sinks != nullptr) {
-    const float sk = sinks[hq] * LOG2E;
-    M = fmaxf(M, sk);
-    den = __builtin_amdgcn_exp2f(sk - M);
+    M = sinks[hq] * LOG2E;
+    den = 1.f;
   }
-  const float base = M == -INFINITY ? 0.f : M;
-  for (int i = 0; i < n; ++i) {
-    const float wt = __builtin_amdgcn_exp2f(pp[i * step + D] - base);
-    num += wt * pp[i * step + d];
-    den += wt * pp[i * step + D + 1];
+  for (int i0 = 0; i0 < n; i0 += U) {
+    float v[U], mx[U], dn[U], top = M;
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      const float* at = pp + min(i0 + i, n - 1) * step;
+      v[i] = at[d];
+      mx[i] = at[D];
+      dn[i] = at[D + 1];
+    }
+#pragma unroll
+    for (int i = 0; i < U; ++i) top = fmaxf(top, mx[i]);   // the last one again
+    const float base = top == -INFINITY ? 0.f : top;
+    const float was = __builtin_amdgcn_exp2f(M - base);
+    num *= was;
+    den *= was;
+    M = top;
+#pragma unroll
+    for (int i = 0; i < U; ++i)
+      if (i0 + i < n) {
+        const float wt = __builtin_amdgcn_exp2f(mx[i] - base);
+        num += wt * v[i];
+        den += wt * dn[i];
+      }
   }
   out[((long)seq * Hq + hq) * D + d] = f2bf(den > 0.f ? num / den : 0.f);
 }

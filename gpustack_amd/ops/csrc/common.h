@@ -71,24 +71,30 @@ __device__ __forceinline__ u16x8 f32_to_bf8(const float* in) {
 
 // Eight neighbours of a product cut over k: fp32 parts `stride` apart, added up in
 // their order and rounded, as the product's own join does it. Four parts are in
-// flight at a time.
-DEVICE_INLINE u16x8 join_parts8(const float* p, long stride, int parts) {
-  float sum[8];
-  for (int s0 = 0; s0 < parts; s0 += 4) {
-    f32x4 v[4][2];
+// flight at a time, or eight where there are more: what adds a few rows up waits for
+// the memory once or twice and does little else.
+template <int U>
+DEVICE_INLINE void add_parts8(float* sum, const float* p, long stride, int parts) {
+  for (int s0 = 0; s0 < parts; s0 += U) {
+    f32x4 v[U][2];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < U; ++i) {
       const float* at = p + min(s0 + i, parts - 1) * stride;
       v[i][0] = *reinterpret_cast<const f32x4*>(at);
       v[i][1] = *reinterpret_cast<const f32x4*>(at + 4);
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < U; ++i)
       if (s0 + i < parts)
 #pragma unroll
         for (int j = 0; j < 8; ++j)
           sum[j] = s0 + i == 0 ? v[0][j / 4][j % 4] : sum[j] + v[i][j / 4][j % 4];
   }
+}
+DEVICE_INLINE u16x8 join_parts8(const float* p, long stride, int parts) {
+  float sum[8];
+  if (parts > 4) add_parts8<8>(sum, p, stride, parts);
+  else add_parts8<4>(sum, p, stride, parts);
   return f32_to_bf8(sum);
 }
 
@@ -113,35 +119,63 @@ DEVICE_INLINE u16x8 sum_rows8(const unsigned short* p, long stride, int k) {
   return f32_to_bf8(sum);
 }
 
-// Full-wave (64-lane) butterfly reductions.
+// A value and that of the lane 32 (M = 32) or 16 away, in either order, without the
+// LDS. The two operands of the swap are kept apart: given one value twice the compiler
+// takes both results for the same.
+template <int M>
+DEVICE_INLINE f32x2 with_lane(float v) {
+  const unsigned int a = __builtin_bit_cast(unsigned int, v);
+  unsigned int b = a;
+  asm("" : "+v"(b));
+  const auto r = M == 16 ? __builtin_amdgcn_permlane16_swap(a, b, false, false)
+                         : __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  const unsigned int x = r[0], y = r[1];
+  return f32x2{__builtin_bit_cast(float, x), __builtin_bit_cast(float, y)};
+}
+
+// The value of the lane N places on in a row of 16 lanes, around its end.
+template <int N>
+DEVICE_INLINE float row_turned(float v) {
+  return __builtin_bit_cast(
+      float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x120 + N,
+                                         0xf, 0xf, true));
+}
+
+// Full-wave (64-lane) reductions, in the order and to the bit of a butterfly (lanes 32,
+// 16, 8, 4, 2, 1 apart; once lanes 2 N apart agree, N on and N apart are the same), but
+// not through the LDS, whose six exchanges are most of a microsecond in a row kernel.
 __device__ __forceinline__ float wave_reduce_sum(float x) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) x += __shfl_xor(x, m, WAVE_SIZE);
-  return x;
+  f32x2 p = with_lane<32>(x);
+  p = with_lane<16>(p[0] + p[1]);
+  x = p[0] + p[1];
+  x += row_turned<8>(x);
+  x += row_turned<4>(x);
+  x += row_turned<2>(x);
+  return x + row_turned<1>(x);
 }
 
 __device__ __forceinline__ float wave_reduce_max(float x) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) x = fmaxf(x, __shfl_xor(x, m, WAVE_SIZE));
-  return x;
+  f32x2 p = with_lane<32>(x);
+  p = with_lane<16>(fmaxf(p[0], p[1]));
+  x = fmaxf(p[0], p[1]);
+  x = fmaxf(x, row_turned<8>(x));
+  x = fmaxf(x, row_turned<4>(x));
+  x = fmaxf(x, row_turned<2>(x));
+  return fmaxf(x, row_turned<1>(x));
 }
 
-// Maximum of a lane and lane ^ 32, in all lanes. The two operands of the swap are
-// kept apart: given one value twice the compiler takes both results for the same.
+// Maximum of a lane and lane ^ 32, in all lanes.
 DEVICE_INLINE float half_wave_max(float x) {
-  const unsigned int a = __builtin_bit_cast(unsigned int, x);
-  unsigned int b = a;
-  asm("" : "+v"(b));
-  const auto w = __builtin_amdgcn_permlane32_swap(a, b, false, false);
-  return fmaxf(__builtin_bit_cast(float, (unsigned int)w[0]),
-               __builtin_bit_cast(float, (unsigned int)w[1]));
+  const f32x2 p = with_lane<32>(x);
+  return fmaxf(p[0], p[1]);
 }
 
 // Reduction across a 16-lane subgroup (lanes with equal l>>4).
 __device__ __forceinline__ float group16_reduce_sum(float x) {
-#pragma unroll
-  for (int m = 8; m >= 1; m >>= 1) x += __shfl_xor(x, m, WAVE_SIZE);
-  return x;
+  x += row_turned<8>(x);
+  x += row_turned<4>(x);
+  x += row_turned<2>(x);
+  return x + row_turned<1>(x);
 }
 
 // Loads from memory straight to LDS address `to` + 16 * lane, 16 bytes a lane,

@@ -136,6 +136,8 @@ __global__ __launch_bounds__(ROW_THREADS) void add_layer_norm_vec_kernel(
   }
   float* xr = x + t * W;
   float keep[NV][8];
+  // the weights come with the row and not behind its sums
+  f32x4 wk[NV][2], bk[NV][2];
   float sum = 0.f;
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
@@ -143,6 +145,13 @@ __global__ __launch_bounds__(ROW_THREADS) void add_layer_norm_vec_kernel(
 #pragma unroll
     for (int k = 0; k < 8; ++k) keep[j][k] = 0.f;
     if (i >= W) continue;
+    if (w != nullptr) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        wk[j][k / 4][k % 4] = w[i + k];
+        bk[j][k / 4][k % 4] = b[i + k];
+      }
+    }
     const f32x4 lo = *reinterpret_cast<const f32x4*>(xr + i);
     const f32x4 hi = *reinterpret_cast<const f32x4*>(xr + i + 4);
     float f[8];
@@ -188,7 +197,8 @@ __global__ __launch_bounds__(ROW_THREADS) void add_layer_norm_vec_kernel(
     if (i >= W) continue;
     float f[8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) f[k] = (keep[j][k] - mean) * inv * w[i + k] + b[i + k];
+    for (int k = 0; k < 8; ++k) 
+      f[k] = (keep[j][k] - mean) * inv * wk[j][k / 4][k % 4] + bk[j][k / 4][k % 4];
     if constexpr (sizeof(TH) == 2) {
       *reinterpret_cast<u16x8*>(hr + i) = f32_to_bf8(f);
     } else {

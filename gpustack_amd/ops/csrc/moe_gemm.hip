@@ -383,27 +383,6 @@ __global__ __launch_bounds__(MOE_THREADS, 2) void moe_tile_kernel(
   }
 }
 
-// Maximum of the 64 lanes, in all of them (a NaN loses): rotations of 16 lanes in the
-// operands, then the lane swaps, whose operands are kept apart as in half_wave_max.
-DEVICE_INLINE float moe_wave_max(float x) {
-  auto turned = [](float v, auto by) {
-    return __builtin_bit_cast(
-        float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v),
-                                           0x120 + decltype(by)::value, 0xf, 0xf,
-                                           true));
-  };
-  x = fmaxf(x, turned(x, std::integral_constant<int, 8>{}));
-  x = fmaxf(x, turned(x, std::integral_constant<int, 4>{}));
-  x = fmaxf(x, turned(x, std::integral_constant<int, 2>{}));
-  x = fmaxf(x, turned(x, std::integral_constant<int, 1>{}));
-  const unsigned int a = __builtin_bit_cast(unsigned int, x);
-  unsigned int b = a;
-  asm("" : "+v"(b));
-  const auto w = __builtin_amdgcn_permlane16_swap(a, b, false, false);
-  return half_wave_max(fmaxf(__builtin_bit_cast(float, (unsigned int)w[0]),
-                             __builtin_bit_cast(float, (unsigned int)w[1])));
-}
-
 // Softmax routing: the k largest logits of a row in descending order (lowest
 // index first among equals) and their weights: softmax over the chosen ones
 // (renorm) or their share of the softmax over all. One wave per row, NV
@@ -445,7 +424,7 @@ DEVICE_INLINE void moe_topk_row(int* experts, float* weights,
 #pragma unroll
     for (int i = 0; i < NV; ++i)
       best = fmaxf(best, taken >> i & 1 ? -INFINITY : v[i]);
-    best = moe_wave_max(best);
+    best = wave_reduce_max(best);
     int at = E - 1;                    // rows of NaN: any expert, in range
 #pragma unroll
     for (int i = NV - 1; i >= 0; --i) {

@@ -1,0 +1,35 @@
+"""Row kernels whose sums cross the wave without the LDS, at widths that leave lanes,
+waves and register chunks without numbers, with one to eight parts and more."""
+import pytest
+import torch
+
+pytestmark = [pytest.mark.gpu,
+              pytest.mark.skipif(not torch.cuda.is_available(),
+                                 reason="needs a GPU")]
+
+
+@pytest.mark.parametrize("H", [8, 72, 512, 2048, 2056, 4104, 8192, 8200])
+@pytest.mark.parametrize("T,parts", [(1, 1), (3, 4), (3, 5), (2, 8), (2, 9),
+                                     (600, 2)])
+def test_norm_of_parts(H, T, parts):
+    from gpustack_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(H + T + parts)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    p, res, w = rnd(parts, T, H), rnd(T, H).bfloat16(), rnd(H).bfloat16()
+    # the parts are added in their order and rounded, as a product's join does it
+    x = p[0].clone()
+    for i in range(1, parts):
+        x += p[i]
+    s = x.bfloat16().double() + res.double()
+    want = s * torch.rsqrt((s * s).mean(1, keepdim=True) + 1e-5) * w.double()
+    res2 = res.clone()
+    out = ops.add_rms_norm(p, res2, w, 1e-5)
+    assert torch.equal(res2, s.float().bfloat16())
+    # rows of more than 8192 are normed from the rounded sum (2^-8 of a value)
+    eps = 2.0 ** -8 if H <= 8192 else 2.0 ** -7
+    assert bool(((out.double() - want).abs() <= want.abs() * eps + 1e-6).all())
+    plain = x.bfloat16()
+    res3 = res.clone()
+    ops.fused_add_rms_norm(plain, res3, w, 1e-5)
+    assert torch.equal(plain, out) and torch.equal(res3, res2)
