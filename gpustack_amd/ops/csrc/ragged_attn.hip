@@ -502,17 +502,23 @@ __global__ __launch_bounds__(THREADS) void paged_attn_mfma_kernel(
 // so that nothing waits at a barrier and a wave's next keys and these values (16 KB)
 // are under way all the time. S^T = K Q^T in an order of the key rows (key_at) in which
 // a lane's 8 weights of 32 keys are neighbours, as the value pages hold them: the
-// weights stay in its registers. Bound by memory: 64 rows of 16 heads on 4 behind 200 to
-// 3000 keys 55 us (230 MB), in a window of 1024 26 (121 MB; a workgroup to a tile of 64
-// keys, its scores and weights through the LDS with three barriers, 63 and 34), 256 rows
-// behind 100 to 1500 100 (117), 16 in the window 16 (19), one behind 7000 21 (26).
-template <typename TO>
+// weights stay in its registers. VT tiles of 16 channels, all of them loaded: behind a
+// branch for each that VW may leave out, the wait for the keys took in the values asked
+// for behind them, and a step cost two latencies. Bound by memory, us, with the branches
+// / now: 64 rows of 16 heads on 4 behind 200 to 3000 keys 54.5 / 51.4 (210 MB, cold), in
+// a window of 1024 29.1 / 27.7 (118 MB; a workgroup to a tile of 64 keys, its scores and
+// weights through the LDS with three barriers, took 34), 33 rows behind 1000 to 8000 in
+// the window 26.1 / 23.6, 16 behind 300 to 1200 15.8 / 14.8, one behind 7000 20.8 /
+// 19.2; where every CU has four workgroups they ask for more than it takes: 256 rows
+// behind 100 to 1500 90.4 / 91.0, in the window 82 / 85.5. Eight waves for four, of half
+// the keys each, are no faster (27.7, 11.6 for 12.0 behind 7000 in the window, 102 for 94).
+template <typename TO, int VT>
 __global__ __launch_bounds__(THREADS, 2) void paged_attn_waves_kernel(
     TO* __restrict__ out, const unsigned short* __restrict__ q,
     const unsigned short* __restrict__ k_cache,
     const unsigned short* __restrict__ v_cache, AttnArgs p,
     float* __restrict__ ws_acc, float* __restrict__ ws_ml) {
-  constexpr int BS = 16, D = 128, DK = D / 32, VT = 8, WKT = 32, QS = D + 8;
+  constexpr int BS = 16, D = 128, DK = D / 32, WKT = 32, QS = D + 8;
   constexpr int OS = D + 4;                           // fp32 row of the sums
   __shared__ __attribute__((aligned(16))) unsigned short Ql[G16 * QS];
   __shared__ __attribute__((aligned(16))) float os[4][G16 * OS];
@@ -601,8 +607,8 @@ __global__ __launch_bounds__(THREADS, 2) void paged_attn_waves_kernel(
       const unsigned short* pt =
           v_cache + (blk * p.G + g) * (long)VW * BS + (lg & 1) * 8 + lc * BS;
 #pragma unroll
-      for (int c = 0; c < VT; ++c)
-        if (c * 16 < VW) vreg[c] = *reinterpret_cast<const u16x8*>(pt + c * 16 * BS);
+      for (int c = 0; c < VT; ++c)           // the last ones once more behind VW
+        vreg[c] = *reinterpret_cast<const u16x8*>(pt + min(c * 16, VW - 16) * BS);
     }
     f32x4 s[2];
 #pragma unroll
@@ -616,10 +622,15 @@ __global__ __launch_bounds__(THREADS, 2) void paged_attn_waves_kernel(
     pg1 = nx1;
     float sv[8], mx = -INFINITY;
 #pragma unroll
+    for (int i = 0; i < 8; ++i) sv[i] = s[i >> 2][i & 3] * p.scale;
+    if (p.softcap > 0.f)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) sv[i] = p.softcap * tanhf(sv[i] / p.softcap);
+#pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int j = k0 + lg * 8 + i;
       sv[i] = key_visible(j, my_pos, my_lo, p.keep_first)
-                  ? scaled_score(s[i >> 2][i & 3], p) - slope * (float)(my_pos - j)
+                  ? sv[i] - slope * (float)(my_pos - j)
                   : -INFINITY;
       mx = fmaxf(mx, sv[i]);
     }
@@ -648,8 +659,7 @@ __global__ __launch_bounds__(THREADS, 2) void paged_attn_waves_kernel(
         for (int r = 0; r < 4; ++r) acc[c][r] *= alpha;
     }
 #pragma unroll
-    for (int c = 0; c < VT; ++c)
-      if (c * 16 < VW) acc[c] = ra_mfma(vreg[c], w, acc[c]);
+    for (int c = 0; c < VT; ++c) acc[c] = ra_mfma(vreg[c], w, acc[c]);
   }
   l_run += __shfl_xor(l_run, 16, WAVE_SIZE);
   l_run += __shfl_xor(l_run, 32, WAVE_SIZE);
@@ -1070,8 +1080,12 @@ void launch_mfma(void* out, const void* q, const void* kc, const void* vc,
   bool alone = false;
   if constexpr (NT == 2) {
     alone = p.D == 128;
-    if (alone)
-      paged_attn_waves_kernel<TO><<<dim3(ntiles, nsplit), THREADS, 0, s>>>(
+    if (alone && p.VW > 96)
+      paged_attn_waves_kernel<TO, 8><<<dim3(ntiles, nsplit), THREADS, 0, s>>>(
+          (TO*)out, (const unsigned short*)q, (const unsigned short*)kc,
+          (const unsigned short*)vc, p, ws_acc, ws_ml);
+    else if (alone)
+      paged_attn_waves_kernel<TO, 6><<<dim3(ntiles, nsplit), THREADS, 0, s>>>(
           (TO*)out, (const unsigned short*)q, (const unsigned short*)kc,
           (const unsigned short*)vc, p, ws_acc, ws_ml);
   }
