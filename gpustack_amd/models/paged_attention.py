@@ -145,8 +145,17 @@ class PagedRotaryAttention(nn.Module):
         m = self.m
         T = h.shape[0]
         rg = meta.ragged
-        qkv = ops.linear_auto(h, self.qkv_w) if self.qkv_b is None \
-            else F.linear(h, self.qkv_w, self.qkv_b)
+        parts = None
+        if self.qkv_b is not None:
+            qkv = F.linear(h, self.qkv_w, self.qkv_b)
+        else:
+            qkv = ops.linear_auto(
+                h, self.qkv_w, m.head_norm and not self.rope_rows
+                and ops.head_norm_parts_ok(T, m.qk_dim, self.nv))
+            if qkv.dim() == 3:
+                parts = qkv
+                qkv = torch.empty(T, parts.shape[2], dtype=h.dtype,
+                                  device=h.device)
         gate = qkv[:, self.col_gate:self.col_gate + m.heads] \
             if m.out_gate else None
         if m.conv:
@@ -177,7 +186,7 @@ class PagedRotaryAttention(nn.Module):
                                 self.k_head_norm, m.qk_dim, coef, every,
                                 rg.pos32, v_first, self.v_lam, k_cache,
                                 v_cache, meta.slot_mapping, self.eps,
-                                page_groups=groups)
+                                page_groups=groups, parts=parts)
             if self.v_mix_first:
                 shared["v_first"] = qkv[:, self.nq + self.nk:]
         else:

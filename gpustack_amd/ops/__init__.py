@@ -1494,17 +1494,26 @@ def add_layer_norm_rows(x, a, w, b, eps: float, rows, dtype):
     return h
 
 
+def head_norm_parts_ok(T: int, head_dim: int, nv: int) -> bool:
+    """Whether head_norm_store adds a projection's parts up: whole lanes of 8
+    channels, rows whose weights bound the product (64 rows of 3072 x 2048 12.0 us
+    in the library, 6.5 cut over k)."""
+    return T <= 128 and head_dim in (64, 128, 256) and nv % 8 == 0
+
+
 def head_norm_store(q_out, qkv, nq: int, nk: int, q_w, k_w, head_dim: int,
                     temp_coef: float, temp_every: float, pos32, v_first, lam,
                     k_cache, v_cache, slots, eps: float,
-                    page_groups=None) -> None:
+                    page_groups=None, parts=None) -> None:
     """`page_groups` (build_page_groups; GPU, prompts): the value rows are
-    written page by page instead of row by row."""
+    written page by page instead of row by row. `parts` (linear_auto; GPU,
+    head_norm_parts_ok): the rows are their sum, of which qkv is left the
+    values."""
     k = _state_backend(qkv)
     if k is not None:
         k.head_norm_store(q_out, qkv, nq, nk, q_w, k_w, head_dim, temp_coef,
                           temp_every, pos32, v_first, lam, k_cache, v_cache,
-                          slots, eps, page_groups)
+                          slots, eps, page_groups, parts)
     else:
         torch_ref.head_norm_store(q_out, qkv, nq, nk, q_w, k_w, head_dim,
                                   temp_coef, temp_every, pos32, v_first, lam,

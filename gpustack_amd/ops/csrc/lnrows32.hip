@@ -275,10 +275,12 @@ __global__ __launch_bounds__(ROW_THREADS) void head_norm_store_kernel(
 // rows a workgroup. What a lane brings it reads once. Bound by the row's bytes,
 // few rows by the launch: 64 rows of 16 + 2 x 4 heads of 128 11.6 -> 5.2 us,
 // 7032 rows 48 -> 25 (a wave a head at a time, 2 bytes a lane, two passes).
-template <int LPH>
+// PARTS: the rows are fp32 parts of the projection, `stride` apart, added up in their
+// order and rounded as the product's own join does it; the values are left in qkv.
+template <int LPH, bool PARTS>
 __global__ __launch_bounds__(ROW_THREADS) void head_norm_store_vec_kernel(
     unsigned short* __restrict__ q_out, unsigned short* __restrict__ qkv,
-    long ld_qkv, int nq, int nk, int nv, const float* __restrict__ q_w,
+    const float* __restrict__ parts, long stride, int nparts, long ld_qkv, int nq, int nk, int nv, const float* __restrict__ q_w,
     const float* __restrict__ k_w, float temp_coef, float temp_every,
     const int* __restrict__ pos32, const unsigned short* __restrict__ v_first,
     long ld_vf, const float* __restrict__ lam,
@@ -297,8 +299,14 @@ __global__ __launch_bounds__(ROW_THREADS) void head_norm_store_vec_kernel(
   const long blk = keep ? slot / BS : 0;
   const int off = keep ? (int)(slot % BS) : 0;
   float f[8];
+  auto mine = [&](int col) {
+    if constexpr (PARTS)
+      return join_parts8(parts + t * (nq + nk + nv) + col, stride, nparts);
+    else
+      return *reinterpret_cast<const u16x8*>(row + col);
+  };
   if (h < HQ + G) {
-    bf8_to_f32(*reinterpret_cast<const u16x8*>(row + (long)h * D + c), f);
+    bf8_to_f32(mine(h * D + c), f);
     float ss = 0.f;
 #pragma unroll
     for (int k = 0; k < 8; ++k) ss += f[k] * f[k];
@@ -327,9 +335,9 @@ __global__ __launch_bounds__(ROW_THREADS) void head_norm_store_vec_kernel(
   }
   const int vc = (h - HQ - G) * D + c;
   const bool later = flags & 1;
-  if (vc >= nv || (later && v_first == nullptr)) return;
+  if (vc >= nv || (!PARTS && later && v_first == nullptr)) return;
   unsigned short* vr = row + nq + nk + vc;
-  u16x8 v = *reinterpret_cast<const u16x8*>(vr);
+  u16x8 v = mine(nq + nk + vc);
   if (v_first != nullptr) {
     const float l = lam[0];
     float g[8];
@@ -339,9 +347,8 @@ __global__ __launch_bounds__(ROW_THREADS) void head_norm_store_vec_kernel(
     for (int k = 0; k < 8; ++k) f[k] = (1.f - l) * f[k] + l * g[k];
     v = f32_to_bf8(f);
   }
-  if (later) {
-    *reinterpret_cast<u16x8*>(vr) = v;
-  } else if (keep) {
+  if (later || PARTS) *reinterpret_cast<u16x8*>(vr) = v;
+  if (!later && keep) {
 #pragma unroll
     for (int k = 0; k < 8; ++k)
       v_cache[((blk * G + (vc + k) / VW) * (long)VW + (vc + k) % VW) * BS + off] =
@@ -550,16 +557,19 @@ int add_layer_norm_launch(float* x, const void* a, int parts, const float* w,
   return 1;
 }
 
-void head_norm_store_launch(void* q_out, void* qkv, long ld_qkv, int nq, int nk,
-                            int nv, const float* q_w, const float* k_w, int D,
-                            float temp_coef, float temp_every, const int* pos32,
-                            const void* v_first, long ld_vf, const float* lam,
-                            void* k_cache, void* v_cache, const long* slots,
-                            long nslots, int G, int BS, int VW, float eps,
-                            int flags, int T, int bf, hipStream_t s) {
-  if (T <= 0) return;
+// parts: the rows [T, nq + nk + nv] as fp32 parts [nparts, T, ..], or null. Returns 0
+// where they are given and the kernel of whole lanes does not take the call.
+int head_norm_store_launch(void* q_out, void* qkv, const float* parts, int nparts,
+                           long ld_qkv, int nq, int nk, int nv, const float* q_w,
+                           const float* k_w, int D, float temp_coef,
+                           float temp_every, const int* pos32,
+                           const void* v_first, long ld_vf, const float* lam,
+                           void* k_cache, void* v_cache, const long* slots,
+                           long nslots, int G, int BS, int VW, float eps,
+                           int flags, int T, int bf, hipStream_t s) {
+  if (T <= 0) return 1;
   const uintptr_t at = (uintptr_t)q_out | (uintptr_t)qkv | (uintptr_t)v_first |
-                       (uintptr_t)k_cache |
+                       (uintptr_t)k_cache | (uintptr_t)parts |
                        (uintptr_t)(ld_qkv * 2) |
                        (uintptr_t)(v_first != nullptr ? ld_vf * 2 : 0);
   if (bf && (D == 64 || D == 128 || D == 256) && nq % D == 0 && nk == G * D &&
@@ -568,18 +578,27 @@ void head_norm_store_launch(void* q_out, void* qkv, long ld_qkv, int nq, int nk,
     const long units = (long)T * H;
     const int per = ROW_THREADS / (D / 8);
     const dim3 grid((unsigned)((units + per - 1) / per));
-#define HNS(L)                                                               \
-  head_norm_store_vec_kernel<L><<<grid, ROW_THREADS, 0, s>>>(                \
-      (unsigned short*)q_out, (unsigned short*)qkv, ld_qkv, nq, nk, nv, q_w, \
-      k_w, temp_coef, temp_every, pos32, (const unsigned short*)v_first,     \
-      ld_vf, lam, (unsigned short*)k_cache, (unsigned short*)v_cache, slots, \
+#define HNS(L, P)                                                            \
+  head_norm_store_vec_kernel<L, P><<<grid, ROW_THREADS, 0, s>>>(             \
+      (unsigned short*)q_out, (unsigned short*)qkv, parts,                   \
+      (long)T * (nq + nk + nv), nparts, ld_qkv, nq, nk, nv, q_w, k_w,        \
+      temp_coef, temp_every, pos32, (const unsigned short*)v_first, ld_vf,   \
+      lam, (unsigned short*)k_cache, (unsigned short*)v_cache, slots,        \
       nslots, G, BS, VW, eps, flags, units, H)
-    if (D == 64) HNS(8);
-    else if (D == 128) HNS(16);
-    else HNS(32);
+#define HNS_D(P)                                                             \
+  if (D == 64) HNS(8, P);                                                    \
+  else if (D == 128) HNS(16, P);                                             \
+  else HNS(32, P)
+    if (parts != nullptr) {
+      HNS_D(true);
+    } else {
+      HNS_D(false);
+    }
+#undef HNS_D
 #undef HNS
-    return;
+    return 1;
   }
+  if (parts != nullptr) return 0;
   if (bf)
     head_norm_store_kernel<unsigned short, unsigned short>
         <<<T, ROW_THREADS, 0, s>>>(
@@ -593,6 +612,7 @@ void head_norm_store_launch(void* q_out, void* qkv, long ld_qkv, int nq, int nk,
         (float*)q_out, (float*)qkv, ld_qkv, nq, nk, nv, q_w, k_w, D, temp_coef,
         temp_every, pos32, (const float*)v_first, ld_vf, lam, (float*)k_cache,
         (float*)v_cache, slots, nslots, G, BS, VW, eps, flags);
+  return 1;
 }
 
 void route_topk_launch(int* experts, float* weights, const float* logits,

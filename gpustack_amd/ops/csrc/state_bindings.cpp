@@ -10,7 +10,7 @@
 
 void embed_rows_scaled_launch(float*, const long*, const void*, int, int, long, float, int, hipStream_t);
 int add_layer_norm_launch(float*, const void*, int, const float*, const float*, void*, const long*, int, int, int, float, int, int, hipStream_t);
-void head_norm_store_launch(void*, void*, long, int, int, int, const float*, const float*, int, float, float, const int*, const void*, long, const float*, void*, void*, const long*, long, int, int, int, float, int, int, int, hipStream_t);
+int head_norm_store_launch(void*, void*, const float*, int, long, int, int, int, const float*, const float*, int, float, float, const int*, const void*, long, const float*, void*, void*, const long*, long, int, int, int, float, int, int, int, hipStream_t);
 void value_page_store_launch(const void*, long, int, void*, const long*, long, const int*, int, int, int, int, int, int, hipStream_t);
 void route_topk_launch(int*, float*, const float*, int, const float*, int, int, int, int, int, int, int, int, float, hipStream_t);
 int state_scan_launch(float*, const void*, long, int, int, int, const void*, long, int, int, int, int, int, int, const float*, const float*, const float*, const float*, float*, const int*, const int*, const int*, const int*, int, int, int, int, int, const int*, int, int, float*, float*, float*, hipStream_t);
@@ -131,7 +131,7 @@ void head_norm_store(Tensor q_out, Tensor qkv, long nq, long nk, Tensor q_w,
                      Tensor k_w, long head_dim, double temp_coef,
                      double temp_every, Tensor pos32, OptTensor v_first,
                      OptTensor lam, Tensor k_cache, Tensor v_cache, Tensor slots,
-                     double eps, OptTensor page_groups) {
+                     double eps, OptTensor page_groups, OptTensor parts) {
   const int bf = act_kind(q_out, "q_out");
   TORCH_CHECK(act_kind(qkv, "qkv") == bf && act_kind(k_cache, "k_cache") == bf &&
               act_kind(v_cache, "v_cache") == bf,
@@ -167,15 +167,23 @@ void head_norm_store(Tensor q_out, Tensor qkv, long nq, long nk, Tensor q_w,
     ld_vf = v_first->stride(0);
     lp = lam->data_ptr<float>();
   }
+  if (parts.has_value()) {
+    chk(*parts, "parts", at::kFloat);
+    TORCH_CHECK(parts->dim() == 3 && parts->size(0) >= 1 &&
+                parts->size(1) == T && parts->size(2) == qkv.size(1),
+                "parts must be fp32 [n, T, nq + nk + nv]");
+  }
   // slots outside [0, nblocks*BS) are skipped inside the kernels
-  head_norm_store_launch(q_out.data_ptr(), qkv.data_ptr(), qkv.stride(0),
-                         (int)nq, (int)nk, (int)nv, q_w.data_ptr<float>(),
-                         k_w.data_ptr<float>(), D, (float)temp_coef,
-                         (float)temp_every, pos32.data_ptr<int>(), vf, ld_vf, lp,
-                         k_cache.data_ptr(), v_cache.data_ptr(),
-                         slots.data_ptr<long>(), k_cache.size(0) * (long)BS, G,
-                         BS, VW, (float)eps, page_groups.has_value() ? 1 : 0, T,
-                         bf, cur_stream(qkv));
+  const int ok = head_norm_store_launch(
+      q_out.data_ptr(), qkv.data_ptr(),
+      parts.has_value() ? parts->data_ptr<float>() : nullptr,
+      parts.has_value() ? (int)parts->size(0) : 0, qkv.stride(0), (int)nq,
+      (int)nk, (int)nv, q_w.data_ptr<float>(), k_w.data_ptr<float>(), D,
+      (float)temp_coef, (float)temp_every, pos32.data_ptr<int>(), vf, ld_vf, lp,
+      k_cache.data_ptr(), v_cache.data_ptr(), slots.data_ptr<long>(),
+      k_cache.size(0) * (long)BS, G, BS, VW, (float)eps,
+      page_groups.has_value() ? 1 : 0, T, bf, cur_stream(qkv));
+  TORCH_CHECK(ok, "parts of heads of ", D, " at these addresses");
   HIP_CHECK_LAST();
   if (page_groups.has_value()) {
     // the value rows leave page by page (runs of rows inside one page)
