@@ -874,10 +874,10 @@ class ModelRunner:
             logits = self.model(tokens, meta, self.kv)
         from .. import ops
 
-        ops.greedy_sample_into(self._sampled_dev[:bs], logits)
         slot = self._pin_idx
         self._pin_idx ^= 1
-        self._sampled_pin[slot][:bs].copy_(self._sampled_dev[:bs], non_blocking=True)
+        ops.greedy_sample_into(self._sampled_dev[:bs], logits,
+                               self._sampled_pin[slot][:bs])
         if self.device.type == "cuda":
             ev = torch.cuda.Event()
             ev.record()

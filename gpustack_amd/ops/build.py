@@ -20,7 +20,7 @@ ARCH = os.environ.get("GPUSTACK_AMD_ARCH", "gfx950")
 
 HIP_SOURCES = ["pointwise.hip", "attn_decode.hip", "attn_prefill.hip", "skinny_gemm.hip", "gemm8.hip", "gemm8_lab.hip", "moe_gemm.hip", "moe_wide.hip", "w4_gemm.hip", "rows_gemm.hip", "wide_tiles.hip", "mla_decode.hip"]
 CPP_SOURCES = ["bindings.cpp"]
-HEADERS = ["common.h", "wide_tiles.h"]
+HEADERS = ["common.h", "wide_tiles.h", "pinned_words.h"]
 # the fp32-residual op family lives in its own small library: a checkout
 # that serves only such a model compiles these few files and nothing else
 LATENT_SO_PATH = PKG_DIR / "_hip_latent.so"

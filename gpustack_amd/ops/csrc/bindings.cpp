@@ -4,13 +4,15 @@
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime.h>
 
+#include "pinned_words.h"
+
 // launchers (defined in the .hip translation units)
 void rms_norm_launch(void*, const void*, const void*, const long*, void*, long, float, int, int, hipStream_t);
 void fused_add_rms_norm_launch(void*, const void*, void*, const void*, const void*, int, const long*, int, float, int, int, int, hipStream_t);
 void rope_neox_launch(const long*, void*, void*, const float*, int, int, int, int, int, long, long, hipStream_t);
 void silu_and_mul_launch(void*, const void*, long, int, hipStream_t);
 void reshape_and_cache_launch(const void*, const void*, void*, void*, const long*, int, int, int, int, long, long, int, hipStream_t);
-void greedy_sample_launch(long*, const void*, int, int, hipStream_t);
+void greedy_sample_launch(long*, long*, const void*, int, int, hipStream_t);
 void mla_decode_launch(float*, const void*, const void*, const int*, const int*, int, int, int, int, int, int, float, int*, hipStream_t);
 void qkv_store_launch(void*, const float*, int, const void*, const void*, const float*, const long*, const long*, void*, void*, long, int, int, int, int, float, int, int*, hipStream_t);
 struct DecodeParts { int n, least, grouped; };
@@ -268,11 +270,15 @@ void qkv_store(at::Tensor qkv, long Hq, long Hk,
   HIP_CHECK_LAST();
 }
 
-void greedy_sample(at::Tensor out, at::Tensor logits) {
+// host: the words once more, in pinned memory
+void greedy_sample(at::Tensor out, at::Tensor logits,
+                   c10::optional<at::Tensor> host) {
   check_bf16(logits, "logits");
   TORCH_CHECK(out.scalar_type() == at::kLong && out.is_contiguous());
   const int N = logits.size(0), V = logits.size(1);
-  greedy_sample_launch(out.data_ptr<long>(), logits.data_ptr(), N, V,
+  greedy_sample_launch(out.data_ptr<long>(),
+                       pinned_words(host, N),
+                       logits.data_ptr(), N, V,
                        cur_stream(logits));
   HIP_CHECK_LAST();
 }
@@ -875,7 +881,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("q_norm"), py::arg("k_norm"), py::arg("cos_sin"),
         py::arg("positions"), py::arg("slots"), py::arg("k_cache"),
         py::arg("v_cache"), py::arg("eps"), py::arg("parts") = py::none());
-  m.def("greedy_sample", &greedy_sample, "argmax over vocab");
+  m.def("greedy_sample", &greedy_sample, "argmax over vocab", py::arg("out"),
+        py::arg("logits"), py::arg("host") = py::none());
   m.def("mla_decode", &mla_decode,
         "MLA absorbed decode over the paged latent cache (DeepSeek)");
   m.def("paged_attn_decode", &paged_attn_decode, "paged GQA decode attention",

@@ -5,6 +5,8 @@
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime.h>
 
+#include "pinned_words.h"
+
 void embed_pair_hash_launch(float*, void*, const long*, const long*, const void*, const void*, int, int, long, long, long, long, int, hipStream_t);
 void rms_scale_add_launch(float*, const void*, const float*, const float*, void*, int, int, float, int, hipStream_t);
 void rms_norm_f32_launch(void*, const float*, const float*, int, int, float, int, hipStream_t);
@@ -13,7 +15,7 @@ void act_inplace_launch(void*, long, int, int, hipStream_t);
 void softcap_launch(float*, long, float, hipStream_t);
 void route_grouped_topk_launch(int*, float*, const float*, int, int, int, int, int, int, float, hipStream_t);
 void moe_combine_launch(void*, const void*, const int*, const float*, const void*, const float*, int, int, int, int, int, int, int, hipStream_t);
-void argmax_f32_launch(long*, const float*, int, int, hipStream_t);
+void argmax_f32_launch(long*, long*, const float*, int, int, hipStream_t);
 void latent_attention_launch(void*, const void*, const void*, const int*, const int*, const int*, int, float, int, int, int, int, int, int, int, int, int, int, int, long, long, long, long, int, float*, float*, hipStream_t);
 int latent_attn_max_rank();
 void grouped_up_act_launch(void*, const void*, const void*, const int*, const int*, const int*, int, int, int, int, int, int, int, hipStream_t);
@@ -312,11 +314,14 @@ void grouped_down(Tensor y, Tensor u, Tensor down, Tensor offs, Tensor counts) {
   HIP_CHECK_LAST();
 }
 
-void argmax_f32(Tensor out, Tensor logits) {
+// host: the words once more, in pinned memory
+void argmax_f32(Tensor out, Tensor logits, OptTensor host) {
   chk(out, "out", at::kLong);
   chk(logits, "logits", at::kFloat);
   TORCH_CHECK(logits.dim() == 2 && out.numel() == logits.size(0));
-  argmax_f32_launch(out.data_ptr<long>(), logits.data_ptr<float>(),
+  argmax_f32_launch(out.data_ptr<long>(),
+                    pinned_words(host, logits.size(0)),
+                    logits.data_ptr<float>(),
                     (int)logits.size(0), (int)logits.size(1),
                     cur_stream(logits));
   HIP_CHECK_LAST();
@@ -335,7 +340,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("softcap", &softcap);
   m.def("route_grouped_topk", &route_grouped_topk);
   m.def("moe_combine", &moe_combine);
-  m.def("argmax_f32", &argmax_f32);
+  m.def("argmax_f32", &argmax_f32, py::arg("out"), py::arg("logits"),
+        py::arg("host") = py::none());
   m.def("grouped_up_act", &grouped_up_act);
   m.def("grouped_down", &grouped_down);
 }

@@ -6,13 +6,15 @@
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime.h>
 
+#include "pinned_words.h"
+
 void embed_rows_f32_launch(float*, const long*, const void*, int, int, long, int, hipStream_t);
 void sandwich_add_norm_launch(float*, const void*, const float*, float, const float*, const float*, void*, int, int, float, int, int, int, hipStream_t);
 void rotary_norm_store_launch(void*, const void*, long, int, int, int, const float*, const float*, const float*, int, const int*, int, void*, void*, const long*, long, int, int, int, int, float, int, int, int, hipStream_t);
 void value_page_store_launch(const void*, long, int, void*, const long*, long, const int*, int, int, int, int, int, int, hipStream_t);
 void diff_combine_launch(void*, const float*, const float*, float, float, long, int, int, hipStream_t);
 void act_and_mul_launch(void*, const void*, long, long, int, int, int, hipStream_t);
-void argmax_f32_launch(long*, const float*, int, int, hipStream_t);
+void argmax_f32_launch(long*, long*, const float*, int, int, hipStream_t);
 void paged_attention_launch(void*, const void*, const void*, const void*, const int*, const int*, const int*, const float*, const float*, float, float, long, long, long, long, int, int, int, int, int, int, int, int, int, int, int, int, int, int, int, int, const void*, long, int, int, int, int, float*, float*, hipStream_t);
 void head_rope_store_launch(void*, const void*, long, int, int, int, const float*, int, int, int, int, int, const float*, int, int, int, const float*, int, int, float, const int*, void*, void*, const long*, long, int, int, float, int, int, int, hipStream_t);
 void dual_rms_mix_launch(void*, const void*, const float*, const void*, const float*, int, int, float, int, hipStream_t);
@@ -480,11 +482,14 @@ void act_inplace(Tensor x, long mode) {
   HIP_CHECK_LAST();
 }
 
-void argmax_f32(Tensor out, Tensor logits) {
+// host: the words once more, in pinned memory
+void argmax_f32(Tensor out, Tensor logits, OptTensor host) {
   chk(out, "out", at::kLong);
   chk(logits, "logits", at::kFloat);
   TORCH_CHECK(logits.dim() == 2 && out.numel() == logits.size(0));
-  argmax_f32_launch(out.data_ptr<long>(), logits.data_ptr<float>(),
+  argmax_f32_launch(out.data_ptr<long>(),
+                    pinned_words(host, logits.size(0)),
+                    logits.data_ptr<float>(),
                     (int)logits.size(0), (int)logits.size(1),
                     cur_stream(logits));
   HIP_CHECK_LAST();
@@ -514,5 +519,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("head_gate", &head_gate);
   m.def("act_inplace", &act_inplace);
   m.def("act_and_mul", &act_and_mul);
-  m.def("argmax_f32", &argmax_f32);
+  m.def("argmax_f32", &argmax_f32, py::arg("out"), py::arg("logits"),
+        py::arg("host") = py::none());
 }

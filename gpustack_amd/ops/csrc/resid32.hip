@@ -464,28 +464,40 @@ __global__ __launch_bounds__(ROW_THREADS) void moe_combine_vec_kernel(
   }
 }
 
-// 16 waves a row with four loads in flight each: bound by how fast one CU
-// takes a row in (128 KB at a 32000-word vocabulary). 4 waves up to 4096 words,
-// where waves without any are what is left (512 rows of 1000, us: 4.6 -> 3.3).
+// 16 waves a row with eight 16-byte loads in flight each: bound by the round trip and
+// the joins (64 rows of 32000 4.7 us; four loads of 4 bytes, ten round trips, 5.2). 4
+// waves up to 4096 words, where waves without any are what is left (512 rows of 1000,
+// us: 4.6 -> 3.3). The words are also left in `host` (pinned memory, or null).
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+
 template <int AM_THREADS>
 __global__ __launch_bounds__(AM_THREADS) void argmax_f32_kernel(
-    long* __restrict__ out, const float* __restrict__ logits, int V) {
+    long* __restrict__ out, long* __restrict__ host,
+    const float* __restrict__ logits, int V) {
+  constexpr int U = 8;
   __shared__ float bv[AM_THREADS / 64];
   __shared__ int bi[AM_THREADS / 64];
   const long t = blockIdx.x;
   const float* z = logits + t * V;
   float v = -INFINITY;
   int idx = 0x7fffffff;
-  int i = threadIdx.x;
-  for (; i + 3 * AM_THREADS < V; i += 4 * AM_THREADS) {
-    float f[4];
+  const int nvec = V / 4;
+  for (int i0 = threadIdx.x; i0 < nvec; i0 += U * AM_THREADS) {
+    f32x4_any f[U];                    // the last ones once more behind the end
 #pragma unroll
-    for (int j = 0; j < 4; ++j) f[j] = z[i + j * AM_THREADS];
+    for (int j = 0; j < U; ++j)
+      f[j] = *reinterpret_cast<const f32x4_any*>(
+          z + min(i0 + j * AM_THREADS, nvec - 1) * 4);
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (f[j] > v) { v = f[j]; idx = i + j * AM_THREADS; }
+    for (int j = 0; j < U; ++j)
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (f[j][k] > v) {
+          v = f[j][k];
+          idx = min(i0 + j * AM_THREADS, nvec - 1) * 4 + k;
+        }
   }
-  for (; i < V; i += AM_THREADS)
+  for (int i = nvec * 4 + threadIdx.x; i < V; i += AM_THREADS)
     if (z[i] > v) { v = z[i]; idx = i; }
   wave_argmax(v, idx);
   if ((threadIdx.x & 63) == 0) { bv[threadIdx.x >> 6] = v; bi[threadIdx.x >> 6] = idx; }
@@ -493,7 +505,9 @@ __global__ __launch_bounds__(AM_THREADS) void argmax_f32_kernel(
   if (threadIdx.x == 0) {
     for (int w = 1; w < AM_THREADS / 64; ++w)
       if (bv[w] > v || (bv[w] == v && bi[w] < idx)) { v = bv[w]; idx = bi[w]; }
-    out[t] = idx == 0x7fffffff ? 0 : idx;
+    const long word = idx == 0x7fffffff ? 0 : idx;
+    out[t] = word;
+    if (host != nullptr) host[t] = word;
   }
 }
 
@@ -646,9 +660,9 @@ void moe_combine_launch(void* out, const void* y, const int* inv,
         ld_gate, gate_col, W, top, T * top);
 }
 
-void argmax_f32_launch(long* out, const float* logits, int N, int V,
+void argmax_f32_launch(long* out, long* host, const float* logits, int N, int V,
                        hipStream_t s) {
   if (N == 0) return;
-  if (V <= 4096) argmax_f32_kernel<256><<<N, 256, 0, s>>>(out, logits, V);
-  else argmax_f32_kernel<1024><<<N, 1024, 0, s>>>(out, logits, V);
+  if (V <= 4096) argmax_f32_kernel<256><<<N, 256, 0, s>>>(out, host, logits, V);
+  else argmax_f32_kernel<1024><<<N, 1024, 0, s>>>(out, host, logits, V);
 }
