@@ -36,6 +36,8 @@ class DecodeGraphRunner:
         dev = runner.device
         spec = getattr(cfg, "speculative", None)
         rps = 1 + int(spec.get("num_draft_tokens", 3)) if spec else 1
+        # no drafted rows: the captured steps may store and attend in one launch
+        self.own_rows = rps == 1
         self.max_bs = min(cfg.max_num_seqs * rps, BUCKETS[-1])
         self.buckets = [b for b in BUCKETS if b <= self.max_bs]
         if self.buckets[-1] != self.max_bs:
@@ -110,6 +112,7 @@ class DecodeGraphRunner:
             block_tables=self.block_tables[:bs],
             seq_lens=self.seq_lens[:bs],
             checked=True,         # by run, or by the sampler that feeds them
+            own_rows=self.own_rows,
         )
         if self.ragged:
             meta.ragged = RaggedMeta(
@@ -159,6 +162,7 @@ class DecodeGraphRunner:
     def can_run(self, batch: ScheduledBatch) -> bool:
         return ((not batch.is_prefill)
                 and not batch.is_suffix
+                and (batch.rows_per_seq == 1 or not self.own_rows)
                 and len(batch.seqs) * batch.rows_per_seq <= self.max_bs
                 and bool(self.graphs))
 

@@ -190,6 +190,9 @@ class ForwardMeta:
     # stay local-row)
     cp: object | None = None
     ragged: RaggedMeta | None = None
+    # decode: every row is the last of a sequence of its own, whose earlier keys
+    # no row of this step writes (drafted rows of one sequence are not)
+    own_rows: bool = False
     # the host has seen that every token id lies in the vocabulary and every
     # entry of logits_indices among the rows: kernels may gather by them that,
     # unlike torch's gathers, do not refuse others
@@ -346,6 +349,21 @@ class Attention(nn.Module):
         qkv = qlinear(x, self.qkv_w, self.qkv_pack, self.qkv_b,
                       parts=store and meta.lora is None and ops.qkv_store_ok(
                           x, self.d, self.rot_dim, self.spec.rope_mode))
+        if store and meta.own_rows and meta.lora is None \
+                and not (self.sinks is not None or self.window or self.softcap) \
+                and ops.qkv_store_ok(x, self.d, self.rot_dim, self.spec.rope_mode) \
+                and ops.paged_attn_decode_rows_ok(x, self.hq, self.hkv, self.d,
+                                                  k_cache, v_cache,
+                                                  meta.block_tables):
+            out = torch.empty(T, self.hq, self.d, dtype=x.dtype, device=x.device)
+            ops.paged_attn_decode_rows(
+                out, qkv, self.hq, self.hkv, self.q_norm if head_norm else None,
+                self.k_norm if head_norm else None, cos_sin, meta.positions,
+                meta.slot_mapping, k_cache, v_cache, meta.block_tables,
+                meta.seq_lens, self.spec.rms_norm_eps, self.scale)
+            return self.comm.all_reduce(
+                qlinear(out.view(T, -1), self.o_w, self.o_pack, self.o_b,
+                        parts=parts))
         qkv_parts = None
         if qkv.dim() == 3:
             qkv_parts = qkv

@@ -285,6 +285,38 @@ def paged_attn_decode(out, q, k_cache, v_cache, block_tables, seq_lens,
                                     window=window, softcap=softcap)
 
 
+def paged_attn_decode_rows_ok(rows, q_heads: int, kv_heads: int, head_dim: int,
+                              k_cache, v_cache, block_tables) -> bool:
+    """Whether paged_attn_decode_rows takes a step: heads of 128 channels, two to
+    eight of them (not three) a kv head, without sinks, window or score cap; and
+    where it is the faster one. It saves 1.2 to 2.7 us up to four workgroups a CU
+    whatever the lengths (128 rows of 8 kv heads 14.5 -> 13.4 at 40 keys, 41.9 ->
+    39.2 at 256 to 383). Behind them it loses contexts under 80 keys (256 rows of 40
+    to 58 21.9 -> 22.8, 512 36.8 -> 40.7) and gains longer ones (80 to 109 54.5 ->
+    54.7, 100 to 149 67.6 -> 64.5): it is taken where the block table has room for
+    128. fp8 pages, whose steps are shorter, up to two a CU (64 rows 9.8 -> 8.4 and
+    17.0 -> 15.3; 128 15.7 -> 17.1 at 80 to 109 keys, 27.2 -> 26.8 at 256 to 383)."""
+    group = q_heads // kv_heads
+    groups, pages = block_tables.shape[0] * kv_heads, block_tables.shape[1]
+    return (rows.is_cuda and head_dim == 128 and q_heads % kv_heads == 0
+            and group in (2, 4, 5, 6, 7, 8)
+            and (groups <= 512 if k_cache.element_size() == 1
+                 else groups <= 1024 or pages >= 8)
+            and k_cache.data_ptr() % 16 == 0 and v_cache.data_ptr() % 16 == 0)
+
+
+def paged_attn_decode_rows(out, rows, q_heads: int, kv_heads: int, q_norm, k_norm,
+                           cos_sin, positions, slots, k_cache, v_cache,
+                           block_tables, seq_lens, eps: float, scale: float) -> None:
+    """qkv_store and paged_attn_decode in one launch, for batches of ONE row a
+    sequence, each the last of its sequence: rows is the projection [N, (q_heads + 2
+    kv_heads) * 128] or its fp32 parts (linear_auto). GPU only
+    (paged_attn_decode_rows_ok)."""
+    _load_hip().paged_attn_decode_rows(
+        out, rows, q_heads, kv_heads, q_norm, k_norm, cos_sin, positions, slots,
+        k_cache, v_cache, block_tables, seq_lens, eps, scale)
+
+
 def mla_decode(ctx_out, q_cat, lat_cache, block_tables, seq_lens,
                scale: float) -> None:
     """MLA absorbed decode (DeepSeek): ctx_out[N,H,512] f32 = softmax

@@ -32,6 +32,18 @@
 // parts of a sequence, a part's keys, and whether a kv head's query heads go together
 struct DecodeParts { int n, least, grouped; };
 
+// The step's rows as they leave the projection, where the kernel norms, rotates and
+// stores them itself: q | k | v in bf16, or (rows null) as fp32 parts of it.
+struct NewRows {
+  const unsigned short* rows;         // [N, (Hq + 2 Hkv) * D]
+  const float* parts;                 // [nparts, N, (Hq + 2 Hkv) * D]
+  int nparts;
+  const unsigned short *q_norm, *k_norm;   // [D] or null
+  const float* cos_sin;               // [positions, D]
+  const long *positions, *slots;      // [N]
+  float eps;
+};
+
 namespace {
 
 constexpr int BS = 16;       // tokens per KV block (page)
@@ -426,7 +438,17 @@ constexpr int ring_bytes(int D, bool fp8, int pages) {
 // 64 keys (16 heads on 8, three x 64 keys 5.5 -> 6.1): a workgroup of one step is its
 // latencies, of which the LDS adds one.
 // EXT: sinks / sliding window / softcap (GPT-OSS and Gemma variants).
-template <int D, bool FP8, bool EXT, int PGS>
+// NEW: q is not there yet, nor the step's own key and value in the pools. Each workgroup
+// makes its query heads from the projection's row, and the one whose part ends with the
+// sequence the kv head's key and value; it stores them and, since its loads from the pool
+// are under way, puts them over the row that these bring into the LDS. All of it, in the
+// order and to the bit of the row kernel (qkv_store), while the first pages come, so that
+// a launch and a round trip are saved. us, in two launches / in one, 32 heads on 8: one
+// row of 1000 keys 11.9 / 10.2, 16 of 300 to 1200 20.5 / 18.3, 512 of 256 to 383 142 /
+// 137, 48 of 3500 to 7900 in fp8 127.6 / 125.4; 64 x 200 to 2000 of 32 on 4 with norms
+// 37.3 / 35.5. Where a CU works through many workgroups of one step each, the row's
+// chain stands in front of every one: 512 x 40 to 58 36.8 / 40.7, in fp8 34 / 42.
+template <int D, bool FP8, bool EXT, int PGS, bool NEW>
 __global__ __launch_bounds__(THREADS, D == 256 || ring_bytes(D, FP8, PGS) > 8192 ? 2 : 3)
 void paged_attn_decode_kernel(
     unsigned short* __restrict__ out,        // [N, Hq, D]
@@ -440,7 +462,8 @@ void paged_attn_decode_kernel(
     int Hkv, int GQ, int max_blocks, float scale, long q_stride,
     const float* __restrict__ sinks,         // [Hq] or null (GPT-OSS)
     int window,                              // 0 = full attention
-    float softcap) {                         // 0 = off (Gemma-2 tanh cap)
+    float softcap,                           // 0 = off (Gemma-2 tanh cap)
+    NewRows nr) {
   constexpr int RB = FP8 ? D : 2 * D;   // bytes of a row
   constexpr int CPR = RB / 16;          // 16-byte chunks of a row
   constexpr int RPI = 64 / CPR;         // rows of a load
@@ -455,6 +478,9 @@ void paged_attn_decode_kernel(
   static_assert(RING >= 8 * OS * 4, "8 heads' sums");
   __shared__ __attribute__((aligned(1024))) char lds[NWAVES * RING];
   __shared__ float lds_ms[NWAVES][16][2];
+  constexpr int QS = D + 8;             // row of q in the LDS
+  __shared__ __attribute__((aligned(16))) unsigned short new_q[NEW ? 8 * QS : 8];
+  __shared__ __attribute__((aligned(16))) char new_kv[2][NEW ? RB : 16];
 
   const int seq = blockIdx.x;
   const int h = blockIdx.y;         // kv head
@@ -467,11 +493,18 @@ void paged_attn_decode_kernel(
 
   // Q as the B operand: column `sub` = head, rows g*8 .. g*8+7 of each chunk
   u32x4 qf[QK];
+  if constexpr (!NEW) {
 #pragma unroll
-  for (int kk = 0; kk < QK; ++kk) {
-    qf[kk] = *reinterpret_cast<const u32x4*>(
-        q + (long)seq * q_stride + ((long)h * GQ + min(sub, GQ - 1)) * D +
-        kk * 32 + g * 8);
+    for (int kk = 0; kk < QK; ++kk) {
+      qf[kk] = *reinterpret_cast<const u32x4*>(
+          q + (long)seq * q_stride + ((long)h * GQ + min(sub, GQ - 1)) * D +
+          kk * 32 + g * 8);
+    }
+  }
+  long pos = 0, slot = -1;
+  if constexpr (NEW) {
+    pos = nr.positions[seq];
+    slot = nr.slots[seq];
   }
 
   // Orders of a row's chunks in the LDS, through the lanes' addresses, so that 16
@@ -567,22 +600,131 @@ void paged_attn_decode_kernel(
 #pragma unroll
     for (int p = 0; p < PGS; ++p) page[p] = bt[max(min(c0 / BS + p, last_page), 0)];
   }
+  // the part that ends with the sequence stores its key and value
+  const bool owner = len > 0 ? t0 < len && len <= t0 + span : blockIdx.z == 0;
+  if (NEW && nsplit > 1 && t0 >= len && !owner) return;
+  int last_block = 0;
+  if constexpr (NEW) last_block = bt[max(last_page, 0)];
   // both are there before the loads that the compiler does not count
+  asm volatile("" ::"s"(page[0]), "s"(page[1]));
+  if constexpr (!NEW) {
 #pragma unroll
-  for (int kk = 0; kk < QK; ++kk) {
-    asm volatile("" : "+v"(qf[kk]) : "s"(page[0]), "s"(page[1]));
-    if (sub >= GQ) qf[kk] = u32x4{0, 0, 0, 0};
+    for (int kk = 0; kk < QK; ++kk) {
+      asm volatile("" : "+v"(qf[kk]));
+      if (sub >= GQ) qf[kk] = u32x4{0, 0, 0, 0};
+    }
   }
   if (c0 < t1) {
     stage_k(page, np);
     stage_v(page, np);
   }
+  if constexpr (NEW) {
+    constexpr int LPH = D / 16, HALF = D / 2;   // lanes of a head: 8 channels twice
+    const int u = threadIdx.x / LPH, c = threadIdx.x % LPH * 8;
+    if (u < GQ + 2) {
+      const int head = u < GQ ? h * GQ + u : Hq + (u - GQ) * Hkv + h;
+      const long row = (long)(Hq + 2 * Hkv) * D, at = seq * row + head * D + c;
+      const float* cs = nr.cos_sin + pos * D + c;
+      u16x8 a, b;
+      float co[8], si[8];
+      if (u <= GQ) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          co[i] = cs[i];
+          si[i] = cs[HALF + i];
+        }
+      }
+      if (nr.rows != nullptr) {
+        a = *reinterpret_cast<const u16x8*>(nr.rows + at);
+        b = *reinterpret_cast<const u16x8*>(nr.rows + at + HALF);
+      } else {
+        a = join_parts8(nr.parts + at, gridDim.x * row, nr.nparts);
+        b = join_parts8(nr.parts + at + HALF, gridDim.x * row, nr.nparts);
+      }
+      if (u <= GQ) {
+        float x[8], y[8], o[8];
+        bf8_to_f32(a, x);
+        bf8_to_f32(b, y);
+        const unsigned short* w = u < GQ ? nr.q_norm : nr.k_norm;
+        if (w != nullptr) {
+          float ss = 0.f, wx[8], wy[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) ss += x[i] * x[i] + y[i] * y[i];
+#pragma unroll
+          for (int i = LPH / 2; i >= 1; i >>= 1) ss += __shfl_xor(ss, i, 64);
+          const float inv = rsqrtf(ss / D + nr.eps);
+          bf8_to_f32(*reinterpret_cast<const u16x8*>(w + c), wx);
+          bf8_to_f32(*reinterpret_cast<const u16x8*>(w + c + HALF), wy);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            x[i] *= inv * wx[i];
+            y[i] *= inv * wy[i];
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          o[i] = x[i] * co[i] - y[i] * si[i];
+          y[i] = y[i] * co[i] + x[i] * si[i];
+        }
+        a = f32_to_bf8(o);
+        b = f32_to_bf8(y);
+      }
+      if (u < GQ) {
+        *reinterpret_cast<u16x8*>(new_q + u * QS + c) = a;
+        *reinterpret_cast<u16x8*>(new_q + u * QS + c + HALF) = b;
+      } else {
+        char* own = new_kv[u - GQ];
+        char* pool = const_cast<char*>(u == GQ ? kc : vc);
+        const bool store = owner && slot >= 0;
+        const long to = ((slot / BS * Hkv + h) * BS + slot % BS) * D + c;
+        if constexpr (FP8) {
+          u8x8 qa, qb;
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            qa[i] = f32_to_fp8(bf2f(a[i]));
+            qb[i] = f32_to_fp8(bf2f(b[i]));
+          }
+          *reinterpret_cast<u8x8*>(own + c) = qa;
+          *reinterpret_cast<u8x8*>(own + c + HALF) = qb;
+          if (store) {
+            *reinterpret_cast<u8x8*>(pool + to) = qa;
+            *reinterpret_cast<u8x8*>(pool + to + HALF) = qb;
+          }
+        } else {
+          *reinterpret_cast<u16x8*>(own + c * 2) = a;
+          *reinterpret_cast<u16x8*>(own + (c + HALF) * 2) = b;
+          if (store) {
+            *reinterpret_cast<u16x8*>(pool + to * 2) = a;
+            *reinterpret_cast<u16x8*>(pool + (to + HALF) * 2) = b;
+          }
+        }
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int kk = 0; kk < QK; ++kk) {
+      qf[kk] = *reinterpret_cast<const u32x4*>(new_q + min(sub, GQ - 1) * QS +
+                                               kk * 32 + g * 8);
+      if (sub >= GQ) qf[kk] = u32x4{0, 0, 0, 0};
+    }
+  }
+  // whether the row stored is the sequence's last (a slot elsewhere, or none, leaves what
+  // the pool holds there)
+  const int last = len - 1;
+  const bool mine = NEW && slot == (long)last_block * BS + last % BS;
   while (c0 < t1) {
     const int cn = c0 + stride;
     const int nn = cn < t1 ? pages_at(cn) : 0;
 #pragma unroll
     for (int p = 0; p < PGS; ++p) next[p] = bt[min(cn / BS + p, last_page)];
     wait(np);
+    const bool own = mine && c0 <= last && last < c0 + np * BS;
+    if constexpr (NEW) {
+      const int p = (last - c0) / BS, r = last % BS;
+      if (own && lane < CPR)
+        *reinterpret_cast<u32x4*>(kl + p * PAGE + r * RB + key_chunk(lane, r) * 16) =
+            *reinterpret_cast<const u32x4*>(new_kv[0] + lane * 16);
+    }
     // scores: lane = head `sub`, keys c0 + p*16 + g*4 + r
     f32x4 st[PGS];
 #pragma unroll
@@ -651,6 +793,13 @@ void paged_attn_decode_kernel(
     // of its window) may hold anything, and a weight of 0 does not undo a NaN
     const bool edge = np < PGS || c0 + PGS * BS > t1 || (EXT && c0 < wstart);
     wait(nn);
+    if constexpr (NEW) {
+      const int p = (last - c0) / BS, r = last % BS;
+      if (own && lane < CPR)
+        *reinterpret_cast<u32x4*>(vl + p * PAGE + r * RB +
+                                  value_chunk(lane, p * BS + r) * 16) =
+            *reinterpret_cast<const u32x4*>(new_kv[1] + lane * 16);
+    }
     auto weigh = [&](auto masked) {
       u32x4 keep;
       if constexpr (masked.value) {
@@ -898,17 +1047,18 @@ struct DecodeArgs {
   const float* sinks;
   int window;
   float softcap;
+  NewRows rows;             // or none of it, slots null
   hipStream_t s;
 };
 
 template <int D, bool FP8, bool EXT>
 void decode_launch(const DecodeArgs& a) {
   const int GQ = a.Hq / a.Hkv;
-  auto run = [&](auto kernel, int heads) {
+  auto run = [&](auto kernel, int heads, auto... extra) {
     hipLaunchKernelGGL(kernel, dim3(a.N, heads, a.parts.n), dim3(THREADS), 0, a.s,
                        a.out, a.q, a.kc, a.vc, a.block_tables, a.seq_lens, a.part,
                        a.parts.least, a.Hkv, GQ, a.max_blocks, a.scale, a.q_stride,
-                       a.sinks, a.window, a.softcap);
+                       a.sinks, a.window, a.softcap, extra...);
   };
   if (!a.parts.grouped) {
     run(paged_attn_heads_kernel<D, FP8, EXT>, a.Hq);
@@ -921,32 +1071,45 @@ void decode_launch(const DecodeArgs& a) {
   // (40 x 300 to 1200 32.1 / 34.4, 64 x 500 29.5 / 33.0, 512 x 40 to 60 26.1 / 33.9, but
   // 384 x 200 to 400 93 / 88).
   constexpr bool ONE = !FP8 && D >= 128, TWO = FP8 || D <= 128;
+  constexpr bool FUSED = D == 128 && !EXT;
   if constexpr (ONE) {
     if (!TWO || (long)a.N * a.Hkv > 256) {
-      run(paged_attn_decode_kernel<D, FP8, EXT, 1>, a.Hkv);
+      if (FUSED && a.rows.slots != nullptr)
+        run(paged_attn_decode_kernel<D, FP8, EXT, 1, FUSED>, a.Hkv, a.rows);
+      else
+        run(paged_attn_decode_kernel<D, FP8, EXT, 1, false>, a.Hkv, a.rows);
       return;
     }
   }
-  if constexpr (TWO) run(paged_attn_decode_kernel<D, FP8, EXT, 2>, a.Hkv);
+  if constexpr (TWO) {
+    if (FUSED && a.rows.slots != nullptr)
+      run(paged_attn_decode_kernel<D, FP8, EXT, 2, FUSED>, a.Hkv, a.rows);
+    else
+      run(paged_attn_decode_kernel<D, FP8, EXT, 2, false>, a.Hkv, a.rows);
+  }
 }
 }  // namespace
 
+// rows: where q is null, the step's own (heads of 128 channels, several of them a kv head,
+// no option); every sequence has one row.
 void paged_attn_decode_launch(void* out, const void* q, const void* kc,
                               const void* vc, const int* block_tables,
                               const int* seq_lens, float* part, DecodeParts parts,
                               int N, int Hq, int Hkv, int D, int max_blocks,
                               float scale, long q_stride, int fp8,
                               const float* sinks, int window, float softcap,
-                              int* err_unsupported, hipStream_t s) {
+                              const NewRows* rows, int* err_unsupported,
+                              hipStream_t s) {
   const int GQ = Hq / Hkv, nsplit = parts.n;
-  *err_unsupported = (D != 128 && D != 64 && D != 256) || GQ < 1 || GQ > 8 ||
-                     GQ == 3 || (D == 256 && GQ > 4);
-  if (*err_unsupported) return;
   const bool ext = (sinks != nullptr) || window > 0 || softcap > 0.f;
+  *err_unsupported = (D != 128 && D != 64 && D != 256) || GQ < 1 || GQ > 8 ||
+                     GQ == 3 || (D == 256 && GQ > 4) ||
+                     (rows != nullptr && (D != 128 || ext || !parts.grouped));
+  if (*err_unsupported || N == 0) return;
   const DecodeArgs a{(unsigned short*)out, (const unsigned short*)q,
                      (const char*)kc, (const char*)vc, block_tables, seq_lens,
                      part, parts, N, Hq, Hkv, max_blocks, scale, q_stride, sinks,
-                     window, softcap, s};
+                     window, softcap, rows != nullptr ? *rows : NewRows{}, s};
   if (D == 128 && !ext) (fp8 ? decode_launch<128, true, false> : decode_launch<128, false, false>)(a);
   else if (D == 128) (fp8 ? decode_launch<128, true, true> : decode_launch<128, false, true>)(a);
   else if (D == 64) (fp8 ? decode_launch<64, true, true> : decode_launch<64, false, true>)(a);

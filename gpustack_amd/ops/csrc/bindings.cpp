@@ -16,8 +16,17 @@ void greedy_sample_launch(long*, long*, const void*, int, int, hipStream_t);
 void mla_decode_launch(float*, const void*, const void*, const int*, const int*, int, int, int, int, int, int, float, int*, hipStream_t);
 void qkv_store_launch(void*, const float*, int, const void*, const void*, const float*, const long*, const long*, void*, void*, long, int, int, int, int, float, int, int*, hipStream_t);
 struct DecodeParts { int n, least, grouped; };
+struct NewRows {
+  const unsigned short* rows;
+  const float* parts;
+  int nparts;
+  const unsigned short *q_norm, *k_norm;
+  const float* cos_sin;
+  const long *positions, *slots;
+  float eps;
+};
 DecodeParts decode_parts(int, int, int, int, int, int, int, int);
-void paged_attn_decode_launch(void*, const void*, const void*, const void*, const int*, const int*, float*, DecodeParts, int, int, int, int, int, float, long, int, const float*, int, float, int*, hipStream_t);
+void paged_attn_decode_launch(void*, const void*, const void*, const void*, const int*, const int*, float*, DecodeParts, int, int, int, int, int, float, long, int, const float*, int, float, const NewRows*, int*, hipStream_t);
 void flash_prefill_launch(void*, const void*, const void*, const void*, const int*, const int*, const int*, int, int, int, int, int, float, long, long, long, const float*, int, float, int*, hipStream_t);
 void flash_prefill_paged_launch(void*, const void*, const void*, const void*, const int*, const int*, const int*, const int*, const int*, const int*, int, int, int, int, int, float, long, const float*, int, float, int*, hipStream_t);
 void mfma_probe_launch(float*, const void*, const void*, hipStream_t);
@@ -120,6 +129,8 @@ void embed_rms_norm(at::Tensor out, at::Tensor x, at::Tensor tokens,
 }
 
 // fp32 parts [n, rows, cols] of a product cut over k, not added up
+bool at_16(const at::Tensor& t) { return (uintptr_t)t.data_ptr() % 16 == 0; }
+
 const float* check_parts(const at::Tensor& p, long rows, long cols) {
   TORCH_CHECK(p.is_cuda() && p.scalar_type() == at::kFloat &&
               p.is_contiguous() && p.dim() == 3 && p.size(0) >= 1 &&
@@ -350,9 +361,80 @@ void paged_attn_decode(at::Tensor out, at::Tensor q, at::Tensor k_cache,
                            parts, N, Hq, Hkv, D, max_blocks,
                            (float)scale, qstride,
                            is_fp8_cache(k_cache) ? 1 : 0, sink_ptr,
-                           (int)window, (float)softcap, &err, cur_stream(q));
+                           (int)window, (float)softcap, nullptr, &err, cur_stream(q));
   TORCH_CHECK(!err, "paged_attn_decode: unsupported head_dim/GQ combination: D=",
               D, " Hq=", Hq, " Hkv=", Hkv);
+  HIP_CHECK_LAST();
+}
+
+// The step's rows from the projection to attention in one launch: qkv_store and
+// paged_attn_decode of one row a sequence. rows [N, (Hq + 2 Hkv) D] in bf16, or its fp32
+// parts [n, N, ..].
+void paged_attn_decode_rows(at::Tensor out, at::Tensor rows, long Hq, long Hkv,
+                            c10::optional<at::Tensor> q_norm,
+                            c10::optional<at::Tensor> k_norm, at::Tensor cos_sin,
+                            at::Tensor positions, at::Tensor slots,
+                            at::Tensor k_cache, at::Tensor v_cache,
+                            at::Tensor block_tables, at::Tensor seq_lens,
+                            double eps, double scale) {
+  check_bf16(out, "out");
+  check_cache(k_cache, "k_cache"); check_cache(v_cache, "v_cache");
+  TORCH_CHECK(out.dim() == 3 && out.size(1) == Hq && Hkv > 0 && Hq % Hkv == 0,
+              "out [N, Hq, D]");
+  const long N = out.size(0);
+  const int D = out.size(2);
+  TORCH_CHECK(k_cache.dim() == 4 && k_cache.size(1) == Hkv && k_cache.size(2) == 16 &&
+                  k_cache.size(3) == D && k_cache.sizes() == v_cache.sizes() &&
+                  k_cache.scalar_type() == v_cache.scalar_type(),
+              "pools [blocks, Hkv, 16, D]");
+  for (const at::Tensor* t : {&block_tables, &seq_lens})
+    TORCH_CHECK(t->is_cuda() && t->scalar_type() == at::kInt && t->is_contiguous(),
+                "block_tables and seq_lens are int32");
+  for (const at::Tensor* t : {&positions, &slots})
+    TORCH_CHECK(t->is_cuda() && t->scalar_type() == at::kLong && t->is_contiguous() &&
+                    t->numel() == N, "positions and slots [N]");
+  TORCH_CHECK(block_tables.dim() == 2 && block_tables.size(0) == N &&
+              block_tables.size(1) > 0 && seq_lens.numel() == N);
+  TORCH_CHECK(cos_sin.is_cuda() && cos_sin.scalar_type() == at::kFloat
+              && cos_sin.is_contiguous() && cos_sin.size(1) == D);
+  const long W = (Hq + 2 * Hkv) * D;
+  NewRows nr{};
+  if (rows.dim() == 3) {
+    nr.parts = check_parts(rows, N, W);
+    nr.nparts = (int)rows.size(0);
+  } else {
+    check_bf16(rows, "rows");
+    TORCH_CHECK(rows.dim() == 2 && rows.size(0) == N && rows.size(1) == W &&
+                    at_16(rows), "rows [N, (Hq + 2 Hkv) D]");
+    nr.rows = (const unsigned short*)rows.data_ptr();
+  }
+  const c10::optional<at::Tensor>* given[2] = {&q_norm, &k_norm};
+  const unsigned short** norms[2] = {&nr.q_norm, &nr.k_norm};
+  for (int i = 0; i < 2; ++i)
+    if (given[i]->has_value()) {
+      check_bf16(**given[i], "head norm");
+      TORCH_CHECK((*given[i])->numel() == D && at_16(**given[i]), "head norm [D]");
+      *norms[i] = (const unsigned short*)(*given[i])->data_ptr();
+    }
+  nr.cos_sin = cos_sin.data_ptr<float>();
+  nr.positions = positions.data_ptr<long>();
+  nr.slots = slots.data_ptr<long>();
+  nr.eps = (float)eps;
+  const int fp8 = is_fp8_cache(k_cache) ? 1 : 0;
+  const int max_blocks = block_tables.size(1);
+  const DecodeParts parts = decode_parts(N, Hq, Hkv, max_blocks, D, fp8, 0,
+                                         at_16(k_cache) && at_16(v_cache));
+  at::Tensor part;
+  if (parts.n > 1)
+    part = at::empty({N * Hq * parts.n * (D + 2)}, out.options().dtype(at::kFloat));
+  int err = 0;
+  paged_attn_decode_launch(out.data_ptr(), nullptr, k_cache.data_ptr(),
+                           v_cache.data_ptr(), block_tables.data_ptr<int>(),
+                           seq_lens.data_ptr<int>(),
+                           parts.n > 1 ? part.data_ptr<float>() : nullptr, parts, N,
+                           Hq, Hkv, D, max_blocks, (float)scale, 0, fp8, nullptr, 0,
+                           0.f, &nr, &err, cur_stream(out));
+  TORCH_CHECK(!err, "paged_attn_decode_rows: D=", D, " Hq=", Hq, " Hkv=", Hkv);
   HIP_CHECK_LAST();
 }
 
@@ -767,7 +849,6 @@ void check_w4(const at::Tensor& x, const at::Tensor& qw, const at::Tensor& sc,
   TORCH_CHECK(sc.size(0) == N && sc.size(1) == K / 128);
 }
 
-bool at_16(const at::Tensor& t) { return (uintptr_t)t.data_ptr() % 16 == 0; }
 
 void w4_gemm(at::Tensor out, at::Tensor x, at::Tensor qw, at::Tensor sc,
              at::Tensor zs) {
@@ -885,6 +966,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("logits"), py::arg("host") = py::none());
   m.def("mla_decode", &mla_decode,
         "MLA absorbed decode over the paged latent cache (DeepSeek)");
+  m.def("paged_attn_decode_rows", &paged_attn_decode_rows,
+        "head norms, rotation, cache write and paged attention of a step's rows");
   m.def("paged_attn_decode", &paged_attn_decode, "paged GQA decode attention",
         py::arg("out"), py::arg("q"), py::arg("k_cache"), py::arg("v_cache"),
         py::arg("block_tables"), py::arg("seq_lens"), py::arg("scale"),
