@@ -724,9 +724,65 @@ def moe_wide_wins(rows: int, E: int, N: int, K: int, down: bool) -> bool:
     return rounds == 1 or tiles >= .8 * 256 * rounds or mean >= 240 * parts
 
 
+# us of rows_tile_kernel's whole products by tile of 32, 64 and 128 columns, and of
+# rows_gemm_kernel (0), for up to so many rows: a launch, and for every 64 k (r: workgroups
+# by 256) with one workgroup a CU the second and r^3 times the third, with more the fourth,
+# r times the fifth and ceil(r / 2) times the sixth; of rows_gemm_kernel the second and r
+# times the third where its workgroups have 16 columns, the fourth and r times the fifth
+# where they have 32. Fitted to 3000 sizes of 1024 to 4096 k, weights out of HBM (3 to 6 %
+# off on average, 25 at most).
+_FEW_TIMES = {
+    8: {32: (2.41, .157, .043, .055, .133, .081), 64: (2.04, .271, .104, .088, .262, .159), 128: (2.08, .358, .476, .134, .546, .285), 0: (2.01, .045, .095, .066, .178, 0)},
+    16: {32: (2.42, .157, .043, .046, .146, .081), 64: (2.11, .272, .102, .073, .275, .167), 128: (2.1, .375, .458, .118, .563, .311), 0: (2.06, .05, .123, .05, .21, 0)},
+    32: {32: (2.42, .162, .048, .04, .163, .083), 64: (2.23, .274, .108, .063, .295, .165), 128: (2.22, .399, .439, .089, .563, .364)},
+    64: {32: (2.33, .246, .037, .067, .181, .133), 64: (2.52, .306, .107, .057, .331, .177), 128: (2.87, .484, .344, .055, .564, .455)},
+}
+
+
+def _few_time(rows: int, cols: int, N: int, K: int) -> float:
+    base, one, full, two, each, pair = _FEW_TIMES[rows][cols]
+    steps = K / 64
+    if cols == 0:
+        narrow = N // 32 < 512
+        r = -(-N // (16 if narrow else 32)) / 256
+        return base + steps * (one + r * full if narrow else two + r * each)
+    r = -(-N // cols) / 256
+    return base + steps * (one + r ** 3 * full if r <= 1 else
+                           two + r * each + math.ceil(r / 2) * pair)
+
+
+@functools.lru_cache(maxsize=4096)
+def _few_rows_plan(M: int, N: int, K: int, plan, rows: bool):
+    """(tile plan, whether rows_gemm) of a whole product of up to 64 rows of 1024 to 4096
+    k, given what _rows_tile_plan and _rows_gemm_wins say: the form of the least time
+    (_few_time), where it is 8 % less than that of theirs; in the library's place one of
+    the two, but beyond 16 rows only where it is no more than the library takes at its
+    best (8 us and 5.4 TB/s), and neither up to 8192 columns of 4096 k. Of 2233 such sizes
+    these take 1.024 of the time of the best form, where the two rules alone took 1.114:
+    728 take less by more than 4 %, 41 more, most of them of 2560 k beside the library, 8
+    by more than 8 %, to 1.13. us: 16 rows of 151936 x 2048 130 -> 117, 8 of 10304 x 2048
+    14.7 -> 12.5, 16 of 8192 x 2048 11.0 -> 8.3, 16 of 102400 x 1536 71 -> 63, 32 of 14336
+    x 1024 21.4 -> 7.7."""
+    if not (0 < M <= 64 and 1024 <= K <= 4096 and N >= 1024) or K % 64 or N % 8 \
+            or plan and plan[1] > 1:
+        return plan, rows
+    upto = next(m for m in _FEW_TIMES if m >= M)
+    forms = [c for c in _FEW_TIMES[upto] if c or K % 128 == 0]
+    time = {c: _few_time(upto, c, N, K) for c in forms}
+    best = min(time, key=time.get)
+    now = plan[0] if plan else 0 if rows else None
+    if now is None:
+        if N <= 8192 and K == 4096 \
+                or M > 16 and time[best] > 8 + 2e-6 * N * K / 5.4:
+            return plan, rows
+    elif time[best] >= .92 * time[now]:
+        return plan, rows
+    return ((best, 1), False) if best else (None, True)
+
+
 def linear_auto(x, w, parts: bool = False):
     """Shape-gated GEMM dispatch: the products for few rows
-    (_rows_tile_plan, _rows_gemm_wins) and for many
+    (_rows_tile_plan, _rows_gemm_wins, _few_rows_plan) and for many
     (_wide_parts_plan, _wide_rows_tile), the split-K skinny kernel where it
     measured faster than hipBLASLt (scripts/bench_skinny_gemm.py on MI355X:
     down_proj-like N=4096 K>=8192 M>=384 at splitk=4, 824 TF vs hipBLASLt 680),
@@ -742,12 +798,13 @@ def linear_auto(x, w, parts: bool = False):
         if wide and _wide_take(x, w):
             return _load_hip().wide_parts(x, w, wide[1], *wide[0])
         plan = parts and _parts_plan(M, N, K) or _rows_tile_plan(M, N, K)
+        plan, rows = _few_rows_plan(M, N, K, plan, _rows_gemm_wins(M, N, K))
         wide = None if parts and plan and plan[1] > 1 else _wide_rows_tile(M, N, K)
         if wide and _wide_take(x, w):
             out = torch.empty(M, N, dtype=x.dtype, device=x.device)
             _load_hip().wide_rows(out, x, w, *wide)
             return out
-        if (plan or _rows_gemm_wins(M, N, K)) and _rows_take(x, w):
+        if (plan or rows) and _rows_take(x, w):
             if parts and plan and plan[1] > 1:
                 return _load_hip().rows_tile_parts(x, w, *plan)
             out = torch.empty(M, N, dtype=x.dtype, device=x.device)
