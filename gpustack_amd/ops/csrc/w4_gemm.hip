@@ -34,12 +34,20 @@
 // 27.3, 57344 x 8192 59 -> 55 / 67 -> 59 / 87 -> 78 / 120 -> 100, 128256 x 4096 61 -> 57
 // / 61 -> 58 / 95 -> 83 / 128 -> 107, 8192 x 28672 28 -> 28.6 / 29.7 -> 29.0 / 43 -> 37.5
 // / 57 -> 49, 4096 x 14336 11.7 -> 10.9 / 11.8 -> 11.2 / 13.0 -> 13.1 / 17.6 -> 17.0.
+// A step's addresses are a number the wave shares and 32 bits of offset a lane, and its
+// buffer is a constant of the code (64-bit addresses of each lane, made anew in every
+// step -> this, at 16 / 32 / 64 / 100 rows: 57344 x 8192 62 -> 57 / 84 -> 82 / 106 -> 103
+// / 208 -> 191, 128256 x 4096 63 -> 60 / 88.7 -> 89 / 114 -> 110 / 221 -> 211, 4096 x
+// 14336 12.4 -> 12.1 / 14.1 -> 14.2 / 17.6 -> 17.3 / 32 -> 30.6, in four waves 5184 x
+// 8192 10.9 / 16.3 -> 15.1 / 22.9 -> 20.9 / 42.5 -> 38.3).
 // Two tiles of columns a wave, four waves: 27, 14, 9.1, 6.2, 73 at 16 rows and 42,
 // 22, 15, 9.9, 173 at 64 (28672 x 4096, 4096 x 14336, 6144 x, 4096 x, 128256 x 4096).
 //
 // Rows (w4_rows_kernel): few rows of products that are narrow and have no consumer
 // for parts, and small ones. Straight from memory, k cut over the waves.
 #include "common.h"
+
+#include <type_traits>
 
 namespace {
 
@@ -114,22 +122,23 @@ __global__ __launch_bounds__(WAVES * KW * WAVE_SIZE) void w4_tile_kernel(
   };
 
   // an instruction brings 2 rows of x, or 8 of the weights, a wave its own
-  // columns; a step of one block (the last of an odd number) brings it twice
-  const unsigned short* xp[LX];
-  const unsigned char* wp[LW];
+  // columns; a step of one block (the last of an odd number) brings it twice. Lanes keep
+  // offsets, what changes from step to step is the wave's.
+  unsigned int xo[LX], wo[LW];
   int xc[LX], wc[LW];
 #pragma unroll
   for (int i = 0; i < LX; ++i) {
     const int row = (any * LX + i) * 2 + lane / 32;
-    xp[i] = x + (long)min(m0 + row, M - 1) * K;
     xc[i] = (lane & 31) ^ (row & 15);
+    xo[i] = ((unsigned)min(row, M - 1 - m0) * (unsigned)K + xc[i] * 8) * 2;
   }
 #pragma unroll
   for (int i = 0; i < LW; ++i) {
     const int row = (kw * LW + i) * 8 + lane / 8;
-    wp[i] = qw + (long)at(wave * 16 + row) * (K / 2);
     wc[i] = (lane & 7) ^ ((row >> 1) & 7);
+    wo[i] = (unsigned)row * (unsigned)(K / 2) + wc[i] * 16;
   }
+  const unsigned char* wbase = qw + (long)at(wave * 16) * (K / 2);
 
   f32x4 acc[MT];
 #pragma unroll
@@ -157,22 +166,28 @@ __global__ __launch_bounds__(WAVES * KW * WAVE_SIZE) void w4_tile_kernel(
     auto step = [&](int i) {
       return from + (i + rot < n ? i + rot : i + rot - n);
     };
-    auto stage = [&](int i) {
+    auto stage = [&](int i, int in) {
       const int st = step(i);
       const bool half = 2 * st + 1 >= nb;
-      unsigned short* to = lds + i % NB * BUF;
+      unsigned short* to = lds + in * BUF;
+      const unsigned short* xb = x + (long)m0 * K + (long)st * W4_SK;
+      const unsigned short* wb =
+          reinterpret_cast<const unsigned short*>(wbase + (long)st * W4_KC);
+      auto bring = [&](auto twice) {
 #pragma unroll
-      for (int j = 0; j < LX; ++j)
-        if (8 * MT >= ALL || any * LX + j < 8 * MT)
-          load_to_lds(xp[j] + (long)st * W4_SK + (half ? xc[j] & 15 : xc[j]) * 8,
-                      to + (any * LX + j) * 2 * W4_SK);
+        for (int j = 0; j < LX; ++j)
+          if (8 * MT >= ALL || any * LX + j < 8 * MT)
+            load_to_lds(xb, twice.value ? xo[j] - (xc[j] & 16) * 16 : xo[j],
+                        to + (any * LX + j) * 2 * W4_SK);
 #pragma unroll
-      for (int j = 0; j < LW; ++j)
-        load_to_lds((const unsigned short*)(wp[j] + (long)st * W4_KC +
-                                            (half ? wc[j] & 3 : wc[j]) * 16),
-                    to + XB + (wave * 16 + (kw * LW + j) * 8) * 64);
+        for (int j = 0; j < LW; ++j)
+          load_to_lds(wb, twice.value ? wo[j] - (wc[j] & 4) * 16 : wo[j],
+                      to + XB + (wave * 16 + (kw * LW + j) * 8) * 64);
+      };
+      if (half) bring(std::true_type{});
+      else bring(std::false_type{});
     };
-    for (int i = 0; i < NB - 1 && i < n; ++i) stage(i);
+    for (int i = 0; i < NB - 1 && i < n; ++i) stage(i, i);
     // scale (low half) and offset of every column and block, 0 behind the last; two
     // blocks at a time where they lie so (28672 x 4096 22 -> 20 us)
     const int b0 = 2 * from;
@@ -195,7 +210,9 @@ __global__ __launch_bounds__(WAVES * KW * WAVE_SIZE) void w4_tile_kernel(
       }
     }
 
-    for (int i = 0; i < n; ++i) {
+    // step i, in a buffer of the LDS whose number is a constant of the code
+    auto work = [&](int i, auto in) {
+      constexpr int B = decltype(in)::value;
       // the steps asked for behind this one; a wave may have no rows of x to bring
       if (NB > 2 && i > 0 && i + NB - 2 < n)
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)"
@@ -204,11 +221,11 @@ __global__ __launch_bounds__(WAVES * KW * WAVE_SIZE) void w4_tile_kernel(
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
-      if (i + NB - 1 < n) stage(i + NB - 1);
+      if (i + NB - 1 < n) stage(i + NB - 1, (B + NB - 1) % NB);
       if (i > 0) correct(i - 1);
-      const unsigned short* xl = lds + i % NB * BUF + lc * W4_SK;
+      const unsigned short* xl = lds + B * BUF + lc * W4_SK;
       const unsigned short* wl =
-          lds + i % NB * BUF + XB + (wave * 16 + lc) * 64;
+          lds + B * BUF + XB + (wave * 16 + lc) * 64;
       const int b = 2 * (step(i) - from);
       // sums of x over the blocks, each by one of the waves for all
 #pragma unroll
@@ -250,6 +267,14 @@ __global__ __launch_bounds__(WAVES * KW * WAVE_SIZE) void w4_tile_kernel(
 #pragma unroll
           for (int m = 0; m < MT; ++m) acc[m][r] += s * p[m][r];
         }
+      }
+    };
+    for (int i = 0; i < n; i += NB) {
+      work(i, std::integral_constant<int, 0>{});
+      if (i + 1 < n) work(i + 1, std::integral_constant<int, 1>{});
+      if constexpr (NB > 2) {
+        if (i + 2 < n) work(i + 2, std::integral_constant<int, 2>{});
+        if (i + 3 < n) work(i + 3, std::integral_constant<int, 3>{});
       }
     }
     __syncthreads();
