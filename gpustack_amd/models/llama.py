@@ -903,13 +903,18 @@ class MoEMLP(nn.Module):
                  and (x.data_ptr() | self.router_w.data_ptr()) % 16 == 0
                  and self.router_w.device == x.device)
         plan = ops.router_plan(T, self.e, x.shape[1]) if exact else None
+        lists = None                       # the assignments by expert
         if exact and self.e <= 16:
             hip.moe_route(experts, weights, x, self.router_w,
                           bool(self.spec.norm_topk_prob))
         elif plan:
-            hip.moe_topk(experts, weights,
-                         hip.rows_tile_parts(x, self.router_w, *plan),
-                         bool(self.spec.norm_topk_prob))
+            logits = hip.rows_tile_parts(x, self.router_w, *plan)
+            if ops.choose_sorts(T, self.e):
+                lists = hip.moe_choose(experts, weights, logits,
+                                       bool(self.spec.norm_topk_prob))
+            else:
+                hip.moe_topk(experts, weights, logits,
+                             bool(self.spec.norm_topk_prob))
         else:
             rw = getattr(self, "_router_w_f32", None)
             if rw is None or rw.device != x.device:
@@ -925,9 +930,9 @@ class MoEMLP(nn.Module):
                 weights, experts = self._route(logits)
         if fused and not self._library_wins(T):
             if parts and T > 0 and self.shared_gate_up_w is None:
-                return self._fused_contrib(x, experts, weights) \
+                return self._fused_contrib(x, experts, weights, lists) \
                     .view(T, self.top_k, -1)
-            out = self._fused_dispatch(x, experts, weights)
+            out = self._fused_dispatch(x, experts, weights, lists)
             return self.comm.all_reduce(self._add_shared(x, out))
         flat_exp = experts.reshape(-1).long()                     # [T*k]
         flat_tok = torch.arange(T, device=x.device) \
@@ -1080,32 +1085,34 @@ class MoEMLP(nn.Module):
                 and ops.moe_wide_wins(rows, self.e, self.i, h, False),
                 bias is None and ops.moe_wide_wins(rows, self.e, h, self.i, True))
 
-    def _fused_dispatch(self, x, experts, weights):
+    def _fused_dispatch(self, x, experts, weights, lists=None):
         """Sync-free grouped expert products, summed over the k axis."""
-        contrib = self._fused_contrib(x, experts, weights)
+        contrib = self._fused_contrib(x, experts, weights, lists)
         out = torch.empty_like(x)
         ops._load_hip().moe_sum(out, contrib, experts.shape[1])
         return out
 
-    def _fused_contrib(self, x, experts, weights):
+    def _fused_contrib(self, x, experts, weights, lists=None):
         """The weighted results of each row's experts [T * k, h]: sort the
-        assignments by expert on the device, run the two expert kernels. Every
-        tensor shape here depends only on (T, k, E) — safe under hipGraph
-        capture (reference capability: vLLM fused_moe)."""
+        assignments by expert on the device (`lists`: sorted already, by
+        moe_choose), run the two expert kernels. Every tensor shape here
+        depends only on (T, k, E) — safe under hipGraph capture (reference
+        capability: vLLM fused_moe)."""
         T, k = experts.shape
         TK = T * k
         hip = ops._load_hip()
         if x.data_ptr() % 16:          # the tiles' loads to the LDS
             x = x.clone()
-        flat = experts.reshape(-1).to(torch.int32)
         flat_w = weights.reshape(-1).float()
         act_mode = 1 if self.spec.moe_act == "clamped_swiglu" else 0
         # down bias on tp rank 0 only: the TP all-reduce must sum it once
         db = self.down_b if self.comm.tp_rank == 0 else None
         h = x.shape[1]
         wide_up, wide_down = self._wide_products(TK, h)
-        order, s_tok, counts, offs, tiles, ntiles, *s_w = hip.moe_sort(
-            flat, self.e, k, weights=flat_w if wide_down else None)
+        if lists is None or wide_down:
+            lists = hip.moe_sort(experts.reshape(-1).to(torch.int32), self.e, k,
+                                 weights=flat_w if wide_down else None)
+        order, s_tok, counts, offs, tiles, ntiles, *s_w = lists
         act = x.new_empty(TK, self.i)
         contrib = x.new_empty(TK, h)
         if wide_up:

@@ -695,6 +695,14 @@ def router_plan(T: int, E: int, H: int):
         else (128, 2) if T <= 12000 else (128, 1)
 
 
+def choose_sorts(T: int, E: int) -> bool:
+    """True where the choice of the experts sorts the assignments too (moe_choose): one
+    workgroup's work up to 8 rows, of up to 64 experts 16. us, two launches against one:
+    128 experts 8 rows 7.1 / 5.7, 16 rows 7.0 / 7.0, 256 8 rows 7.4 / 7.1, 16 rows 7.5 /
+    8.6; 64 16 rows 6.4 / 5.7, 24 rows 6.4 / 6.6 (moe_gemm.hip)."""
+    return 0 < T <= (16 if E <= 64 else 8) and E <= 256
+
+
 def moe_wide_wins(rows: int, E: int, N: int, K: int, down: bool) -> bool:
     """Where an expert product of `rows` assignments in tiles of up to 320 rows
     (ops/csrc/moe_wide.hip) measured faster than tiles of 128 (moe_gemm.hip). From

@@ -37,6 +37,7 @@ void gemm_lab_launch(void*, const void*, const void*, int, int, int, int, int*, 
 void moe_tiles_launch(int*, int*, const int*, int, int, hipStream_t);
 void moe_down_scale_launch(void*, const void*, const void*, const int*, const int*, const int*, const float*, const void*, int, int, int, int*, hipStream_t);
 void moe_topk_launch(int*, float*, const float*, int, int, int, int, int, int*, hipStream_t);
+void moe_choose_launch(int*, float*, int*, int*, int*, int*, int*, int*, const float*, int, int, int, int, int, int*, hipStream_t);
 void moe_route_launch(int*, float*, const void*, const void*, int, int, int, int, int, int*, hipStream_t);
 int moe_sort_slices(int);
 void moe_sort_launch(int*, int*, float*, const float*, int*, int*, int*, int*, int*, const int*, int, int, int, int*, hipStream_t);
@@ -634,6 +635,35 @@ std::vector<at::Tensor> moe_sort(at::Tensor experts, long E, long k,
   return {order, s_tok, counts, offs, tiles, n};
 }
 
+// moe_topk and moe_sort (without weights) in one launch: what moe_sort returns
+std::vector<at::Tensor> moe_choose(at::Tensor experts, at::Tensor weights,
+                                   at::Tensor logits, bool renorm) {
+  const int parts = logits.dim() == 3 ? logits.size(0) : 1;
+  const int T = logits.size(-2), E = logits.size(-1), k = experts.size(1);
+  check_i32(experts, (long)T * k, "experts");
+  TORCH_CHECK(logits.is_cuda() && logits.scalar_type() == at::kFloat
+              && logits.is_contiguous(), "logits must be fp32");
+  TORCH_CHECK(weights.is_cuda() && weights.scalar_type() == at::kFloat
+              && weights.is_contiguous()
+              && weights.numel() == (long)T * k
+              && experts.numel() == (long)T * k, "experts / weights [T, k]");
+  const long TK = (long)T * k;
+  auto o = experts.options();
+  at::Tensor order = at::empty({TK}, o), s_tok = at::empty({TK}, o);
+  at::Tensor counts = at::empty({E}, o), offs = at::empty({E}, o);
+  at::Tensor tiles = at::empty({TK / 128 + E, 2}, o), n = at::empty({1}, o);
+  int err = 0;
+  moe_choose_launch(experts.data_ptr<int>(), weights.data_ptr<float>(),
+                    order.data_ptr<int>(), s_tok.data_ptr<int>(),
+                    counts.data_ptr<int>(), offs.data_ptr<int>(),
+                    tiles.data_ptr<int>(), n.data_ptr<int>(),
+                    logits.data_ptr<float>(), T, E, k, renorm ? 1 : 0, parts, &err,
+                    cur_stream(logits));
+  TORCH_CHECK(!err, "moe_choose: unsupported T=", T, " E=", E, " k=", k);
+  HIP_CHECK_LAST();
+  return {order, s_tok, counts, offs, tiles, n};
+}
+
 // moe_tile without bias or another activation, in tiles of up to 320 rows; s_w: the
 // weights that moe_sort sorted
 void moe_wide(bool down, at::Tensor out, at::Tensor src, at::Tensor w,
@@ -998,6 +1028,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rows_gemm", &rows_gemm, "bf16 product of up to 16 rows");
   m.def("moe_route", &moe_route, "router product and choice");
   m.def("moe_topk", &moe_topk, "softmax routing, top k");
+  m.def("moe_choose", &moe_choose,
+        "softmax routing of few rows, assignments by expert and the tile list");
   m.def("moe_sort", &moe_sort, "assignments by expert, and the tile list",
         py::arg("experts"), py::arg("E"), py::arg("k"),
         py::arg("weights") = py::none());

@@ -554,6 +554,59 @@ __global__ __launch_bounds__(1024) void moe_count_kernel(
     hist[(long)blockIdx.x * E + e] = cnt[e];
 }
 
+// From a thread's counts of its experts (ept of them from tid * ept on) to their offsets
+// and the tile list, and to the next free place of each expert's in `cnt`, `before`
+// places in where others come first. By a whole workgroup of 1024; no barrier behind.
+template <int EPT>
+DEVICE_INLINE void moe_offsets(int* cnt, const int (&c)[EPT], const int (&before)[EPT],
+                               int ept, bool lead, int* counts, int* offs, int* tiles,
+                               int* ntiles, int E) {
+  __shared__ int wsum[2][16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  int a = 0, b = 0;
+#pragma unroll
+  for (int j = 0; j < EPT; ++j) {
+    a += c[j];
+    b += (c[j] + MT_M - 1) / MT_M;
+  }
+  const int own_a = a, own_b = b;
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) {   // inclusive sums over the wave
+    const int x = __shfl_up(a, m, 64), y = __shfl_up(b, m, 64);
+    if (lane >= m) {
+      a += x;
+      b += y;
+    }
+  }
+  if (lane == 63) {
+    wsum[0][wave] = a;
+    wsum[1][wave] = b;
+  }
+  __syncthreads();
+  for (int i = 0; i < wave; ++i) {
+    a += wsum[0][i];
+    b += wsum[1][i];
+  }
+  if (lead && tid == 1023) ntiles[0] = b;
+  a -= own_a;
+  b -= own_b;
+#pragma unroll
+  for (int j = 0; j < EPT; ++j) {
+    const int e = tid * ept + j;
+    if (j >= ept || e >= E) continue;
+    cnt[e] = a + before[j];
+    if (lead) {
+      counts[e] = c[j];
+      offs[e] = a;
+      for (int r = 0; r < c[j]; r += MT_M, ++b) {
+        tiles[2 * b] = e;
+        tiles[2 * b + 1] = r;
+      }
+    }
+    a += c[j];
+  }
+}
+
 // gridDim.x slices with their counts in `hist`, or one workgroup without.
 __global__ __launch_bounds__(1024) void moe_sort_kernel(
     int* __restrict__ order, int* __restrict__ s_tok,  // [TK]
@@ -563,9 +616,8 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(
     const int* __restrict__ experts, const int* __restrict__ hist, int TK,
     int E, int k) {
   __shared__ int cnt[MOE_MAX_E];       // counts, then the next free places
-  __shared__ int wsum[2][16];
   constexpr int EPT = MOE_MAX_E / 1024;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x;
   const int from = hist != nullptr ? blockIdx.x * MOE_SLICE : 0;
   const int to = hist != nullptr ? min(TK, from + MOE_SLICE) : TK;
   // thread tid owns experts EPT * tid .. (one each up to 1024 of them)
@@ -600,49 +652,7 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(
       }
     }
   }
-  int a = 0, b = 0;
-#pragma unroll
-  for (int j = 0; j < EPT; ++j) {
-    a += c[j];
-    b += (c[j] + MT_M - 1) / MT_M;
-  }
-  const int own_a = a, own_b = b;
-#pragma unroll
-  for (int m = 1; m < 64; m <<= 1) {   // inclusive sums over the wave
-    const int x = __shfl_up(a, m, 64), y = __shfl_up(b, m, 64);
-    if (lane >= m) {
-      a += x;
-      b += y;
-    }
-  }
-  if (lane == 63) {
-    wsum[0][wave] = a;
-    wsum[1][wave] = b;
-  }
-  __syncthreads();
-  for (int i = 0; i < wave; ++i) {
-    a += wsum[0][i];
-    b += wsum[1][i];
-  }
-  const bool lead = blockIdx.x == 0;
-  if (lead && tid == 1023) ntiles[0] = b;
-  a -= own_a;
-  b -= own_b;
-#pragma unroll
-  for (int j = 0; j < EPT; ++j) {
-    const int e = tid * ept + j;
-    if (j >= ept || e >= E) continue;
-    cnt[e] = a + before[j];
-    if (lead) {
-      counts[e] = c[j];
-      offs[e] = a;
-      for (int r = 0; r < c[j]; r += MT_M, ++b) {
-        tiles[2 * b] = e;
-        tiles[2 * b + 1] = r;
-      }
-    }
-    a += c[j];
-  }
+  moe_offsets(cnt, c, before, ept, blockIdx.x == 0, counts, offs, tiles, ntiles, E);
   __syncthreads();
   moe_walk(experts, from, to, E, [&](int i, int e) {
     const int at = atomicAdd(&cnt[e], 1);
@@ -650,6 +660,45 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(
     s_tok[at] = i / k;
     if (s_w != nullptr) s_w[at] = flat_w[i];
   });
+}
+
+// moe_topk_kernel and moe_sort_kernel in one launch, for up to a row a wave of one
+// workgroup, which counts in the LDS as it chooses and goes on with what it chose. Bound
+// by its chain and, from 8 waves on, by their instructions on one CU: us, two launches /
+// one at 1 / 8 / 16 rows, 8 of 128 experts 6.3 / 5.2, 7.1 / 5.7, 7.0 / 7.0, 6 of 64 5.8 /
+// 4.6, 6.3 / 4.9, 6.4 / 5.7, 8 of 256 6.9 / 6.5, 7.4 / 7.1, 7.5 / 8.6; two rows a wave
+// 7.3 / 10.4 and more.
+constexpr int MOE_CHOOSE = 16;
+
+template <int NV>
+__global__ __launch_bounds__(1024) void moe_choose_kernel(
+    int* __restrict__ experts, float* __restrict__ weights,  // [T, k]
+    int* __restrict__ order, int* __restrict__ s_tok,        // [T * k]
+    int* __restrict__ counts, int* __restrict__ offs,        // [E]
+    int* __restrict__ tiles, int* __restrict__ ntiles,
+    const float* __restrict__ logits,  // [parts, T, E], to be added up
+    int T, int E, int k, int renorm, int parts) {
+  __shared__ int cnt[NV * 64];
+  __shared__ int chosen[MOE_CHOOSE * 64];
+  const int tid = threadIdx.x, lane = tid & 63;
+  if (tid < E) cnt[tid] = 0;
+  __syncthreads();
+  const int t = tid >> 6;
+  if (t < T) {
+    moe_topk_row<NV>(chosen + t * k, weights + (long)t * k, logits + (long)t * E, lane,
+                     E, k, renorm, parts, (long)T * E);
+    if (lane < k) atomicAdd(&cnt[chosen[t * k + lane]], 1);
+  }
+  __syncthreads();
+  const int c[1] = {tid < E ? cnt[tid] : 0}, before[1] = {0};
+  moe_offsets(cnt, c, before, 1, true, counts, offs, tiles, ntiles, E);
+  __syncthreads();
+  for (int i = tid; i < T * k; i += 1024) {
+    const int e = chosen[i], at = atomicAdd(&cnt[e], 1);
+    experts[i] = e;
+    order[at] = i;
+    s_tok[at] = i / k;
+  }
 }
 
 // The tile list alone, from counts that the caller brings.
@@ -710,6 +759,24 @@ void moe_topk_launch(int* experts, float* weights, const float* logits, int T,
   else if (E <= 512) TOPK(8);
   else TOPK(16);
 #undef TOPK
+}
+
+// logits [parts, T, E]; tiles of T * k / 128 + E pairs
+void moe_choose_launch(int* experts, float* weights, int* order, int* s_tok, int* counts,
+                       int* offs, int* tiles, int* ntiles, const float* logits, int T,
+                       int E, int k, int renorm, int parts, int* err_unsupported,
+                       hipStream_t s) {
+  *err_unsupported = E < 1 || E > 256 || k < 1 || k > 64 || k > E || T < 1 ||
+                     T > MOE_CHOOSE;
+  if (*err_unsupported) return;
+#define CHOOSE(NV)                                                                 \
+  hipLaunchKernelGGL((moe_choose_kernel<NV>), dim3(1), dim3(1024), 0, s, experts,  \
+                     weights, order, s_tok, counts, offs, tiles, ntiles, logits, T, \
+                     E, k, renorm, parts)
+  if (E <= 64) CHOOSE(1);
+  else if (E <= 128) CHOOSE(2);
+  else CHOOSE(4);
+#undef CHOOSE
 }
 
 void moe_route_launch(int* experts, float* weights, const void* x,
