@@ -1115,31 +1115,35 @@ class MoEMLP(nn.Module):
         order, s_tok, counts, offs, tiles, ntiles, *s_w = lists
         act = x.new_empty(TK, self.i)
         contrib = x.new_empty(TK, h)
+        bank = self._bank("gate_up")
         if wide_up:
-            hip.moe_wide(False, act, x, self._bank("gate_up"), s_tok, offs,
-                         counts)
+            hip.moe_wide(False, act, x, bank, s_tok, offs, counts)
+        elif self.gate_up_b is None and act_mode == 0 \
+                and bank.data_ptr() % 16 == 0 \
+                and ops.moe_few_wins(TK, self.e, h, False):
+            hip.moe_few(False, act, x, bank, s_tok, tiles, ntiles, offs, counts)
         else:
-            hip.moe_tile(False, act, x, self._bank("gate_up"), s_tok, tiles,
-                         ntiles, offs, counts, bias=self.gate_up_b,
-                         act_mode=act_mode)
+            hip.moe_tile(False, act, x, bank, s_tok, tiles, ntiles, offs,
+                         counts, bias=self.gate_up_b, act_mode=act_mode)
+        bank = self._bank("down")
         if wide_down:
-            hip.moe_wide(True, contrib, act, self._bank("down"), order, offs,
-                         counts, s_w[0])
+            hip.moe_wide(True, contrib, act, bank, order, offs, counts, s_w[0])
             return contrib
-        # Up to one workgroup a CU of long rows: twice as many of 64 columns,
-        # which read the weights again for every 16 rows of an expert. us,
-        # 64 columns against tiles, by assignments: 8 experts of 4096 x 14336
-        # 2: 90 / 192, 16: 179 / 230, 64: 195 / 231, 96: 276 / 231, 128:
-        # 315 / 231; 16 of 4096 x 6400 8: 99 / 103, 12: 129 / 110, 64:
-        # 146 / 134; 8 of 6144 x 16384 4: 114 / 225, 8: 228 / 240, 24:
-        # 320 / 290; 8 of 4096 x 3584 32: 47 / 58; but 64 of 2048 x 2816
-        # 8: 36 / 29, 16: 55 / 49
+        # Up to one tile a CU of long rows 16 rows at a time, whatever bias:
+        # us, tiles / these, by assignments: 8 experts of 4096 x 14336
+        # 2: 115 / 42, 16: 181 / 137, 64: 204 / 173, 96: 208 / 235; 16 of
+        # 4096 x 6400 2: 52 / 20, 8: 66 / 57
         if TK <= 8 * self.e and self.i > 3072 \
                 and min(TK, self.e) * (x.shape[1] // 128) <= 256:
-            hip.moe_down_scale(contrib, act, self._bank("down"), offs, counts,
-                               order, flat_w, bias=db)
+            hip.moe_down_scale(contrib, act, bank, offs, counts,
+                               order, flat_w, bias=db, tiles=tiles,
+                               ntiles=ntiles)
+        elif db is None and bank.data_ptr() % 16 == 0 \
+                and ops.moe_few_wins(TK, self.e, self.i, True):
+            hip.moe_few(True, contrib, act, bank, order, tiles, ntiles, offs,
+                        counts, flat_w)
         else:
-            hip.moe_tile(True, contrib, act, self._bank("down"), order, tiles,
+            hip.moe_tile(True, contrib, act, bank, order, tiles,
                          ntiles, offs, counts, flat_w, bias=db)
         return contrib
 

@@ -703,6 +703,27 @@ def choose_sorts(T: int, E: int) -> bool:
     return 0 < T <= (16 if E <= 64 else 8) and E <= 256
 
 
+def moe_few_wins(rows: int, E: int, K: int, down: bool) -> bool:
+    """Whether an expert product of `rows` assignments takes 16 rows at a time straight
+    from memory (moe_few) in the place of tiles of 128 x 128 (moe_tile): the first product
+    up to 4 rows an expert, the second too of up to 768 k, to one of rows beyond 3072, else
+    to 3/4. More than 16 rows of an expert read its weights again, so the lines
+    allow for uneven routing. us, tiles / this, E experts of N x K, even routing: first, 128
+    of 768 x 2048 8 assignments 22.1 / 13.5, 64 71 / 56, 256 128 / 116, 512 142 / 133, 768
+    145 / 137, 64 of 1024 x 2048 128 101 / 79, 32 of 2048 x 1024 128 42.7 / 40.1, 256 43.5
+    / 44.6, 8 of 14336 x 4096 16 303 / 263, 32 350 / 314; second, 128 of 2048 x 768 8 9.8 /
+    7.4, 256 64 / 59, 512 72 / 70, 64 of 2048 x 1408 48 42 / 33, 384 64 / 66, 64 of 1024 x
+    896 32 11.3 / 11.2, 64 15.4 / 16.0, 512 20.1 / 22.2, 16 of 4096 x 6400 16 106 / 90, 64
+    140 / 142. Uneven, half of 64 rows to one of the experts and 114 of 128 with any, 768 x
+    2048 512 134 / 127 and 2048 x 768 65.8 / 66.0; 96 rows of them, 68 to one,
+    140 / 142 and 70.7 / 75.6."""
+    if rows <= 0:
+        return False
+    if not down or K <= 768:
+        return rows <= 4 * E
+    return rows <= E if K > 3072 else 4 * rows <= 3 * E
+
+
 def moe_wide_wins(rows: int, E: int, N: int, K: int, down: bool) -> bool:
     """Where an expert product of `rows` assignments in tiles of up to 320 rows
     (ops/csrc/moe_wide.hip) measured faster than tiles of 128 (moe_gemm.hip). From

@@ -35,7 +35,7 @@ void gemm8_launch(void*, const void*, const void*, int, int, int, int, int*, hip
 void skinny_gemm_v2_launch(void*, const void*, const void*, void*, int, int, int, int, hipStream_t);
 void gemm_lab_launch(void*, const void*, const void*, int, int, int, int, int*, hipStream_t);
 void moe_tiles_launch(int*, int*, const int*, int, int, hipStream_t);
-void moe_down_scale_launch(void*, const void*, const void*, const int*, const int*, const int*, const float*, const void*, int, int, int, int*, hipStream_t);
+void moe_down_scale_launch(void*, const void*, const void*, const int*, const int*, const int*, const float*, const void*, const int*, const int*, long, int, int, int, int*, hipStream_t);
 void moe_topk_launch(int*, float*, const float*, int, int, int, int, int, int*, hipStream_t);
 void moe_choose_launch(int*, float*, int*, int*, int*, int*, int*, int*, const float*, int, int, int, int, int, int*, hipStream_t);
 void moe_route_launch(int*, float*, const void*, const void*, int, int, int, int, int, int*, hipStream_t);
@@ -45,6 +45,7 @@ bool moe_wide_takes(int, long, long, int, int, int);
 void moe_wide_launch(int, void*, const void*, const void*, const int*, const float*, const int*, const int*, long, long, int, int, int, hipStream_t);
 void moe_sum_launch(void*, const void*, long, int, int, hipStream_t);
 void moe_tile_launch(int, void*, const void*, const void*, const int*, const int*, const int*, const int*, const int*, const float*, const void*, int, long, int, int, int, int*, hipStream_t);
+void moe_few_launch(int, void*, const void*, const void*, const int*, const int*, const int*, const int*, const int*, const float*, long, long, int, int, int, int*, hipStream_t);
 void rows_tile_launch(void*, void*, const void*, const void*, int, int, int, long, int, int, int, int*, hipStream_t);
 void rows_gemm_launch(void*, const void*, const void*, int, int, int, long, int*, hipStream_t);
 bool w4_has(int, int);
@@ -77,6 +78,11 @@ void check_bf16(const at::Tensor& t, const char* name) {
   TORCH_CHECK(t.is_cuda(), name, " must be on GPU");
   TORCH_CHECK(t.scalar_type() == at::kBFloat16, name, " must be bf16");
   TORCH_CHECK(t.is_contiguous(), name, " must be contiguous");
+}
+
+void check_i32(const at::Tensor& t, long n, const char* name) {
+  TORCH_CHECK(t.is_cuda() && t.scalar_type() == at::kInt && t.is_contiguous()
+              && t.numel() >= n, name, " must be a GPU int32 list of ", n);
 }
 
 bool is_fp8_cache(const at::Tensor& t) {
@@ -534,7 +540,9 @@ void skinny_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
 
 void moe_down_scale(at::Tensor contrib, at::Tensor act, at::Tensor w,
                     at::Tensor offs, at::Tensor counts, at::Tensor order,
-                    at::Tensor flat_w, c10::optional<at::Tensor> bias) {
+                    at::Tensor flat_w, c10::optional<at::Tensor> bias,
+                    c10::optional<at::Tensor> tiles,
+                    c10::optional<at::Tensor> ntiles) {
   check_bf16(contrib, "contrib"); check_bf16(act, "act"); check_bf16(w, "w");
   for (auto* t : {&offs, &counts, &order}) {
     TORCH_CHECK(t->scalar_type() == at::kInt && t->is_contiguous());
@@ -549,18 +557,20 @@ void moe_down_scale(at::Tensor contrib, at::Tensor act, at::Tensor w,
     TORCH_CHECK(bias->numel() == (long)E * H, "down bias must be [E, H]");
     bias_ptr = bias->data_ptr();
   }
+  const int *list = nullptr, *n = nullptr;
+  if (tiles.has_value() && ntiles.has_value()) {
+    check_i32(*tiles, 2 * (contrib.size(0) / 128 + E), "tiles");
+    check_i32(*ntiles, 1, "ntiles");
+    list = tiles->data_ptr<int>();
+    n = ntiles->data_ptr<int>();
+  }
   int err = 0;
   moe_down_scale_launch(contrib.data_ptr(), act.data_ptr(), w.data_ptr(),
                         offs.data_ptr<int>(), counts.data_ptr<int>(),
                         order.data_ptr<int>(), flat_w.data_ptr<float>(),
-                        bias_ptr, E, H, I, &err, cur_stream(act));
+                        bias_ptr, list, n, contrib.size(0), E, H, I, &err, cur_stream(act));
   TORCH_CHECK(!err, "moe_down_scale: unsupported dims H=", H, " I=", I);
   HIP_CHECK_LAST();
-}
-
-void check_i32(const at::Tensor& t, long n, const char* name) {
-  TORCH_CHECK(t.is_cuda() && t.scalar_type() == at::kInt && t.is_contiguous()
-              && t.numel() >= n, name, " must be a GPU int32 list of ", n);
 }
 
 void moe_topk(at::Tensor experts, at::Tensor weights, at::Tensor logits,
@@ -748,6 +758,42 @@ void moe_tile(bool down, at::Tensor out, at::Tensor src, at::Tensor w,
                   (int)(out.size(0) / 128 + E), (int)N, K, &err,
                   cur_stream(src));
   TORCH_CHECK(!err, "moe_tile: unsupported dims N=", N, " K=", K);
+  HIP_CHECK_LAST();
+}
+
+// moe_tile without bias or another activation, for few rows an expert
+void moe_few(bool down, at::Tensor out, at::Tensor src, at::Tensor w,
+             at::Tensor rows, at::Tensor tiles, at::Tensor ntiles,
+             at::Tensor offs, at::Tensor counts,
+             c10::optional<at::Tensor> flat_w) {
+  check_bf16(out, "out"); check_bf16(src, "src"); check_bf16(w, "w");
+  TORCH_CHECK(w.dim() == 3 && src.dim() == 2 && out.dim() == 2, "moe_few shapes");
+  const long E = w.size(0), K = w.size(2), TK = out.size(0);
+  const long N = down ? w.size(1) : w.size(1) / 2;
+  check_i32(rows, TK, "rows");
+  check_i32(ntiles, 1, "ntiles");
+  check_i32(offs, E, "offs");
+  check_i32(counts, E, "counts");
+  check_i32(tiles, 2 * (TK / 128 + E), "tiles");
+  TORCH_CHECK(src.size(1) == K && out.size(1) == N &&
+              w.size(1) == (down ? N : 2 * N) && (!down || src.size(0) == TK),
+              "moe_few shapes");
+  TORCH_CHECK((uintptr_t)src.data_ptr() % 16 == 0 &&
+              (uintptr_t)w.data_ptr() % 16 == 0, "moe_few addresses");
+  const float* fw = nullptr;
+  if (down) {
+    TORCH_CHECK(flat_w.has_value() && flat_w->is_cuda() &&
+                flat_w->scalar_type() == at::kFloat && flat_w->is_contiguous() &&
+                flat_w->numel() == TK, "flat_w [TK] fp32");
+    fw = flat_w->data_ptr<float>();
+  }
+  int err = 0;
+  moe_few_launch(down ? 1 : 0, out.data_ptr(), src.data_ptr(), w.data_ptr(),
+                 rows.data_ptr<int>(), tiles.data_ptr<int>(),
+                 ntiles.data_ptr<int>(), offs.data_ptr<int>(),
+                 counts.data_ptr<int>(), fw, src.size(0), TK, (int)E, (int)N,
+                 (int)K, &err, cur_stream(src));
+  TORCH_CHECK(!err, "moe_few: unsupported dims N=", N, " K=", K);
   HIP_CHECK_LAST();
 }
 
@@ -1038,6 +1084,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("rows"), py::arg("offs"), py::arg("counts"),
         py::arg("s_w") = py::none());
   m.def("moe_sum", &moe_sum, "sum of a row's expert contributions");
+  m.def("moe_few", &moe_few, "expert products of few rows an expert",
+        py::arg("down"), py::arg("out"), py::arg("src"), py::arg("w"),
+        py::arg("rows"), py::arg("tiles"), py::arg("ntiles"), py::arg("offs"),
+        py::arg("counts"), py::arg("flat_w") = py::none());
   m.def("moe_tile", &moe_tile, "expert products in 128x128 tiles",
         py::arg("down"), py::arg("out"), py::arg("src"), py::arg("w"),
         py::arg("rows"), py::arg("tiles"), py::arg("ntiles"), py::arg("offs"),
@@ -1058,6 +1108,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("contrib"), py::arg("act"), py::arg("w"), py::arg("offs"),
         py::arg("counts"), py::arg("order"), py::arg("flat_w"),
         py::arg("bias") = py::none(),
+        py::arg("tiles") = py::none(), py::arg("ntiles") = py::none(),
         "grouped MoE down GEMM + routing-weight scale/scatter");
   m.def("w4_gemm", &w4_gemm,
         "W4A16 GEMM: packed-int4 weights dequantized in-register");

@@ -16,117 +16,18 @@
 // exit. Both products run in 128 x 128 tiles (below), from a few rows per
 // expert, where they are bound by the weight stream (128 experts x 1536 x 2048
 // at 64 rows: 147 us, 5.5 TB/s), to whole prompts. The down product has a
-// second form for few workgroups of long rows (moe_down_scale, 64 columns):
-// 16-row MFMA 16x16x32 tiles, A staged through LDS in 512-element K chunks, B
-// streamed from HBM, once per 16 rows.
+// Few rows an expert take both products straight from memory, 16 rows at a time
+// (moe_few_kernel), which is what moe_down_scale is, if need be without a tile list.
 #include "common.h"
 
 #include <type_traits>
 
 namespace {
 
-constexpr int MOE_BN = 64;        // columns of a moe_down_scale workgroup
-constexpr int MOE_KC = 512;       // K chunk staged in LDS
+constexpr int MOE_BN = 64;        // columns that moe_down_scale takes a multiple of
 constexpr int MOE_THREADS = 256;  // 4 waves
 
 typedef __attribute__((ext_vector_type(8))) short m_s16x8;
-
-DEVICE_INLINE f32x4 moe_mfma(u16x8 a, u16x8 b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-      __builtin_bit_cast(m_s16x8, a), __builtin_bit_cast(m_s16x8, b), c, 0, 0, 0);
-}
-
-// stage rows [16][kc] into LDS (row padded to KC+8 elements to break the bank
-// cycle on the A-frag reads)
-DEVICE_INLINE void stage_rows(unsigned short* lds, const unsigned short* src,
-                              long src_stride, int base_row, int nrows, int k0,
-                              int kc, int tid) {
-  const int units = 16 * (kc / 8);         // u16x8 units
-  for (int u = tid; u < units; u += MOE_THREADS) {
-    const int row = u / (kc / 8);
-    const int kk = (u % (kc / 8)) * 8;
-    u16x8 val = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (row < nrows) {
-      val = *reinterpret_cast<const u16x8*>(
-          src + (long)(base_row + row) * src_stride + k0 + kk);
-    }
-    *reinterpret_cast<u16x8*>(lds + row * (MOE_KC + 8) + kk) = val;
-  }
-}
-
-template <bool EXTM = false>
-__global__ __launch_bounds__(MOE_THREADS) void moe_down_scale_kernel(
-    unsigned short* __restrict__ contrib,   // [TK, H] bf16 (original order)
-    const unsigned short* __restrict__ act, // [TK, I] bf16 (sorted rows)
-    const unsigned short* __restrict__ w,   // [E, H, I] bf16
-    const int* __restrict__ offs,           // [E]
-    const int* __restrict__ counts,         // [E]
-    const int* __restrict__ order,          // [TK] sorted -> original index
-    const float* __restrict__ flat_w,       // [TK] routing weight (original)
-    const unsigned short* __restrict__ bias,  // [E, H] bf16 or null
-    int H, int I) {
-  const int nnt = H / MOE_BN;
-  const int e = blockIdx.x / nnt;
-  const int nt = blockIdx.x % nnt;
-  const int cnt = counts[e];
-  if (cnt == 0) return;
-  const int base = offs[e];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & (WAVE_SIZE - 1);
-  const int wave = tid / WAVE_SIZE;
-  const int lc = lane & 15;
-  const int lg = lane >> 4;
-
-  __shared__ unsigned short Al[16 * (MOE_KC + 8)];
-
-  const unsigned short* wd_panel =
-      w + ((long)e * H + nt * MOE_BN + wave * 16) * I;
-  const int first = base;  // act rows are consecutive in sorted space
-
-  const long wrow = (long)lc * I;
-  for (int m0 = 0; m0 < cnt; m0 += 16) {
-    const int nrows = min(16, cnt - m0);
-    f32x4 acc{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < I; k0 += MOE_KC) {
-      const int kc = min(MOE_KC, I - k0);
-      __syncthreads();
-      stage_rows(Al, act, I, first + m0, nrows, k0, kc, tid);
-      __syncthreads();
-      auto body = [&](int kk) {
-        const u16x8 a = *reinterpret_cast<const u16x8*>(
-            Al + lc * (MOE_KC + 8) + kk + lg * 8);
-        const u16x8 b = *reinterpret_cast<const u16x8*>(
-            wd_panel + wrow + k0 + kk + lg * 8);
-        acc = moe_mfma(a, b, acc);
-      };
-      if (kc == MOE_KC) {
-#pragma unroll
-        for (int kk = 0; kk < MOE_KC; kk += 32) body(kk);
-      } else {
-        for (int kk = 0; kk < kc; kk += 32) body(kk);
-      }
-    }
-    float bd = 0.f;
-    if constexpr (EXTM) {
-      bd = (bias != nullptr)
-          ? bf2f(bias[(long)e * H + nt * MOE_BN + wave * 16 + lc]) : 0.f;
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = lg * 4 + r;
-      if (row >= nrows) continue;
-      const int oj = order[base + m0 + row];
-      if constexpr (EXTM) {
-        contrib[(long)oj * H + nt * MOE_BN + wave * 16 + lc] =
-            f2bf((acc[r] + bd) * flat_w[oj]);
-      } else {
-        contrib[(long)oj * H + nt * MOE_BN + wave * 16 + lc] =
-            f2bf(acc[r] * flat_w[oj]);
-      }
-    }
-  }
-}
 
 // ---------------------------------------------------------------------------
 // Tile form. A tile is 128 rows of one expert x 128 weight rows (of gate and
@@ -380,6 +281,119 @@ __global__ __launch_bounds__(MOE_THREADS, 2) void moe_tile_kernel(
     const long to = DOWN ? (long)orow[i] : (long)(first + row);
     *reinterpret_cast<u32x4*>(out + to * N + nt * OW + c * 8) =
         u32x4{a[0], a[1], b[0], b[1]};
+  }
+}
+
+// Few rows an expert: 16 of them, 16 columns of gate and of up or 32 of the down product,
+// straight from memory, k cut over the WAVES of a workgroup 64 by 64, DEPTH blocks of a
+// wave in flight, sums through the LDS. More rows of an expert read its weights again.
+// Bound by the weights: 128 experts of 768 x 2048 gate and up, 52 of them with rows, 56 us
+// for tiles' 71, 126 133 for 142 (6 TB/s; at one row 8 experts, 96 tiles, 13.5 for 22).
+// Three blocks in flight: four are more than 128 registers, and 175 us. Workgroups stay in
+// the order of the experts over the XCDs: an expert's on one XCD, as the tiles are, gains
+// 2 % where routing is even (130 us), but with half the rows at one expert takes 163 for
+// 127. Waves and blocks by k so that few loads are past a wave's end: 8 waves of 1024 k,
+// two blocks for three, 66 us for 4 waves' 48.
+template <bool DOWN, int WAVES, int DEPTH>
+__global__ __launch_bounds__(WAVES * WAVE_SIZE, 4) void moe_few_kernel(
+    unsigned short* __restrict__ out,        // act [TK, I] | contrib [TK, H]
+    const unsigned short* __restrict__ src,  // x [T, H] | act [TK, I]
+    const unsigned short* __restrict__ w,    // [E, 2I, H] | [E, H, I]
+    const int* __restrict__ rows,            // s_tok | order, [TK]
+    const int* __restrict__ tiles,           // null: workgroups for every expert
+    const int* __restrict__ ntiles,
+    const int* __restrict__ offs, const int* __restrict__ counts,
+    const float* __restrict__ flat_w,        // DOWN: [TK] routing weights
+    const unsigned short* __restrict__ bias, // DOWN: [E, H] or null
+    int N, int K) {                          // N = I | H
+  constexpr int OW = DOWN ? 32 : 16;         // columns of the result
+  constexpr int ST = 36;                     // floats of a row of sums
+  __shared__ __attribute__((aligned(16))) float red[WAVES * 16 * ST];
+  const int nnt = N / OW;
+  const int wg = blockIdx.x, tile = wg / nnt;
+  if (tiles != nullptr && tile >= ntiles[0]) return;
+  const int e = tiles != nullptr ? tiles[2 * tile] : tile;
+  const int r0 = tiles != nullptr ? tiles[2 * tile + 1] : 0;
+  const int n0 = wg % nnt * OW;
+  const int tid = threadIdx.x, lane = tid & (WAVE_SIZE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE_SIZE);
+  const int lc = lane & 15, lg = lane >> 4;
+  const int nb = K / 64, n = wave < nb ? (nb - wave + WAVES - 1) / WAVES : 0;
+  // rows lie a power of two apart: workgroups begin at places of their own
+  const int rot = wg % nb;
+  auto block = [&](int j) {
+    const int i = min(wave + j * WAVES, nb - 1) + rot;
+    return i < nb ? i : i - nb;
+  };
+  const char* wb[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+    wb[t] = (const char*)(w + (DOWN ? (long)e * N + n0 + t * 16
+                                    : (long)e * 2 * N + t * N + n0) * K);
+  const unsigned woff = ((unsigned)lc * K + lg * 8) * 2;
+  const int first = offs[e];
+  const int end = tiles != nullptr ? min(counts[e], r0 + MT_M) : counts[e];
+
+  for (int m0 = r0; m0 < end; m0 += 16) {
+    const int nrows = min(16, end - m0);
+    const int at = min(lc, nrows - 1);
+    const char* xb = (const char*)(DOWN ? src + (long)(first + m0) * K : src);
+    const unsigned xoff =
+        ((unsigned)(DOWN ? at : rows[first + m0 + at]) * K + lg * 8) * 2;
+    u32x4 wr[DEPTH][2][2], xr[DEPTH][2];
+    auto load = [&](int j, int in) {
+      const long b = (long)block(j) * 128;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+          wr[in][t][c] = *reinterpret_cast<const u32x4*>(wb[t] + b + c * 64 + woff);
+        xr[in][c] =
+            *reinterpret_cast<const u32x4*>(xb + b + c * 64 + xoff);
+      }
+    };
+    f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int j = 0; j < DEPTH; ++j) load(j, j);
+    for (int q = 0; q < n; q += DEPTH) {
+#pragma unroll
+      for (int j = 0; j < DEPTH; ++j) {
+        if (q + j < n) {
+#pragma unroll
+          for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+              acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  __builtin_bit_cast(m_s16x8, wr[j][t][c]),
+                  __builtin_bit_cast(m_s16x8, xr[j][c]), acc[t], 0, 0, 0);
+          if (q + j + DEPTH < n) load(q + j + DEPTH, j);
+        }
+      }
+    }
+    // column lg * 4 + r of row lc
+    if (m0 > r0) __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+      *reinterpret_cast<f32x4*>(red + (wave * 16 + lc) * ST + t * 16 + lg * 4) = acc[t];
+    __syncthreads();
+    for (int u = tid; u < 16 * OW; u += WAVES * WAVE_SIZE) {
+      const int row = u / OW, c = u % OW;
+      if (row >= nrows) continue;
+      float v[2] = {0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < WAVES; ++i)
+#pragma unroll
+        for (int t = 0; t < (DOWN ? 1 : 2); ++t)
+          v[t] += red[(i * 16 + row) * ST + t * 16 + c];
+      if constexpr (DOWN) {
+        const long to = rows[first + m0 + row];
+        if (bias != nullptr) v[0] += bf2f(bias[(long)e * N + n0 + c]);
+        out[to * N + n0 + c] = f2bf(v[0] * flat_w[to]);
+      } else {
+        out[(long)(first + m0 + row) * N + n0 + c] =
+            f2bf(v[0] / (1.f + __expf(-v[0])) * v[1]);
+      }
+    }
   }
 }
 
@@ -858,24 +872,55 @@ void moe_tile_launch(int down, void* out, const void* src, const void* w,
 #undef TILE
 }
 
+// Without tiles every expert has workgroups, of which those without rows exit.
+static void moe_few(int down, void* out, const void* src, const void* w,
+                    const int* rows, const int* tiles, const int* ntiles,
+                    const int* offs, const int* counts, const float* flat_w,
+                    const void* bias, long groups, int N, int K, hipStream_t s) {
+#define FEW(D, W, B)                                                            \
+  hipLaunchKernelGGL((moe_few_kernel<D, W, B>),                                 \
+                     dim3((unsigned)groups * (N / (D ? 32 : 16))),              \
+                     dim3(W * WAVE_SIZE), 0, s, (unsigned short*)out,           \
+                     (const unsigned short*)src, (const unsigned short*)w,      \
+                     rows, tiles, ntiles, offs, counts, flat_w,                 \
+                     (const unsigned short*)bias, N, K)
+#define FEW_K(D)                           \
+  do {                                     \
+    if (K >= 1536) FEW(D, 8, 3);           \
+    else if (K > 512) FEW(D, 4, 3);        \
+    else FEW(D, 4, 2);                     \
+  } while (0)
+  if (down) FEW_K(true);
+  else FEW_K(false);
+#undef FEW_K
+#undef FEW
+}
+
+// tiles of moe_sort's list: one an expert of those that have rows, and one for 128 rows
+void moe_few_launch(int down, void* out, const void* src, const void* w,
+                    const int* rows, const int* tiles, const int* ntiles,
+                    const int* offs, const int* counts, const float* flat_w,
+                    long src_rows, long TK, int E, int N, int K,
+                    int* err_unsupported, hipStream_t s) {
+  const int ow = down ? 32 : 16;
+  const long groups = (TK < E ? TK : E) + TK / MT_M;
+  *err_unsupported = N % ow != 0 || K % 64 != 0 || K == 0 ||
+                     groups * (N / ow) >= 1l << 31 ||
+                     (!down && src_rows * K * 2 >= 1l << 32);
+  if (*err_unsupported || groups == 0 || N == 0) return;
+  moe_few(down, out, src, w, rows, tiles, ntiles, offs, counts, flat_w, nullptr,
+          groups, N, K, s);
+}
+
 void moe_down_scale_launch(void* contrib, const void* act, const void* w,
                            const int* offs, const int* counts,
                            const int* order, const float* flat_w,
-                           const void* bias, int E,
+                           const void* bias, const int* tiles, const int* ntiles,
+                           long TK, int E,
                            int H, int I, int* err_unsupported, hipStream_t s) {
-  *err_unsupported = 0;
-  if (H % MOE_BN != 0 || I % 128 != 0) { *err_unsupported = 1; return; }
-  dim3 grid(E * (H / MOE_BN));
-  if (bias != nullptr)
-    hipLaunchKernelGGL((moe_down_scale_kernel<true>), grid,
-                       dim3(MOE_THREADS), 0, s, (unsigned short*)contrib,
-                       (const unsigned short*)act, (const unsigned short*)w,
-                       offs, counts, order, flat_w,
-                       (const unsigned short*)bias, H, I);
-  else
-    hipLaunchKernelGGL((moe_down_scale_kernel<false>), grid,
-                       dim3(MOE_THREADS), 0, s, (unsigned short*)contrib,
-                       (const unsigned short*)act, (const unsigned short*)w,
-                       offs, counts, order, flat_w,
-                       (const unsigned short*)bias, H, I);
+  *err_unsupported = H % MOE_BN != 0 || I % 128 != 0 || I == 0;
+  const long groups = tiles != nullptr ? (TK < E ? TK : E) + TK / MT_M : E;
+  if (*err_unsupported || groups == 0 || H == 0) return;
+  moe_few(1, contrib, act, w, order, tiles, ntiles, offs, counts, flat_w, bias,
+          groups, H, I, s);
 }
