@@ -13,11 +13,11 @@
 // (matches models/llama.py MoEMLP._act_mul / the HF GptOss experts)
 //
 // Launch grids do not depend on the routing outcome: workgroups without a tile
-// exit. Both products run in 128 x 128 tiles (below), from a few rows per
-// expert, where they are bound by the weight stream (128 experts x 1536 x 2048
-// at 64 rows: 147 us, 5.5 TB/s), to whole prompts. The down product has a
-// Few rows an expert take both products straight from memory, 16 rows at a time
-// (moe_few_kernel), which is what moe_down_scale is, if need be without a tile list.
+// exit. Up to a few rows an expert both products come straight from memory, 16
+// rows at a time (moe_few_kernel), bound by the weight stream (128 experts x 1536
+// x 2048 at 64 rows: 133 us, 6 TB/s); moe_down_scale is its second one, if need be
+// without a tile list. With more rows they run in 128 x 128 tiles (below), and
+// whole prompts of many rows an expert in wider ones (moe_wide.hip).
 #include "common.h"
 
 #include <type_traits>
