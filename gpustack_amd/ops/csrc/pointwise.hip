@@ -55,7 +55,7 @@ __global__ void rms_norm_kernel(unsigned short* __restrict__ out,
       float f[8];
       bf8_to_f32(u, f);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) ss += f[i] * f[i];
+      for (int i = 0; i < 8; ++i) ss = __builtin_fmaf(f[i], f[i], ss);
     };
     if (cached) {
 #pragma unroll
@@ -160,6 +160,8 @@ __global__ __launch_bounds__(THREADS) void fused_add_rms_norm_kernel(unsigned sh
     // them and not behind the sum (that, the wave's sum without the LDS and eight parts
     // in flight, us a launch behind the writer of the parts: one row of 4096 in 4 parts
     // 2.9 -> 2.6, in 8 3.7 -> 3.4, 48 rows 4.4 -> 4.1 and 6.3 -> 6.2)
+    // Squares are multiply-adds by name: of a sum that begins with a constant 0 the
+    // compiler may round the second one first, and a row in a few hundred is another.
     float vals[SLOTS][8];
     u16x8 wv[SLOTS];
     float ss = 0.f;
@@ -174,7 +176,7 @@ __global__ __launch_bounds__(THREADS) void fused_add_rms_norm_kernel(unsigned sh
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           vals[slot][i] = bf2f(ux[i]) + bf2f(ur[i]);
-          ss += vals[slot][i] * vals[slot][i];
+          ss = __builtin_fmaf(vals[slot][i], vals[slot][i], ss);
         }
         if (pick == nullptr)
           *reinterpret_cast<u16x8*>(rp + v * 8) = f32_to_bf8(vals[slot]);
@@ -187,7 +189,7 @@ __global__ __launch_bounds__(THREADS) void fused_add_rms_norm_kernel(unsigned sh
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           f[i] = bf2f(ux[i]) + bf2f(ur[i]);
-          ss += f[i] * f[i];
+          ss = __builtin_fmaf(f[i], f[i], ss);
         }
         if (pick == nullptr)
           *reinterpret_cast<u16x8*>(rp + v * 8) = f32_to_bf8(f);

@@ -33,3 +33,28 @@ def test_norm_of_parts(H, T, parts):
     res3 = res.clone()
     ops.fused_add_rms_norm(plain, res3, w, 1e-5)
     assert torch.equal(plain, out) and torch.equal(res3, res2)
+
+
+@pytest.mark.parametrize("H", [8, 2048, 8192])
+@pytest.mark.parametrize("T", [1, 600])
+@pytest.mark.parametrize("parts", [0, 2, 6])
+def test_order_of_squares(T, H, parts):
+    """A thread's squares are one chain of multiply-adds from its first number on. Taken
+    so, the squares of these three are 8 in fp32 (worked out in fractions), with the
+    second one rounded in front of the first 8 + 2^-20. The probe behind them lies
+    halfway between two bf16 numbers where the norm is exactly a power of two."""
+    from gpustack_amd import ops
+
+    h = float.fromhex
+    x, res = torch.zeros(T, H).bfloat16(), torch.zeros(T, H).bfloat16()
+    x[:, 0], res[:, 0] = h("0x1.4ep-9"), h("0x1.46p+0")
+    x[:, 1], res[:, 1] = h("0x1.4ap-9"), h("0x1.8cp+0")
+    x[:, 2], res[:, 2] = h("0x1.8ap-6"), h("0x1.f8p+0")
+    w = torch.ones(H).bfloat16()
+    res[:, 3], w[3] = 3 * 2.0 ** -30, 129 * 2.0 ** -7
+    x, res, w = x.cuda(), res.cuda(), w.cuda()
+    if parts:
+        x = torch.cat([x.float()[None], torch.zeros(parts - 1, T, H, device="cuda")])
+    out = ops.add_rms_norm(x, res, w, 0.0)
+    # to even: 194 for 193.5; below it 193
+    assert bool((out[:, 3].float() == 388 * 2.0 ** -37 * (H / 8) ** 0.5).all())
