@@ -95,6 +95,15 @@ DEVICE_INLINE float high_half(float v) {
                             __builtin_bit_cast(unsigned int, v) & 0xffff0000u);
 }
 
+// The fp32 number below one that is positive; 0 of 0, a NaN of a NaN. The high half of
+// it, taken from the number, leaves more than nothing and no more than 17 bits, and
+// once more of that no more than 8: three parts, none of which is 0 (down to 2^-94),
+// so that an infinite value times them is that infinity and no NaN.
+DEVICE_INLINE float next_below(float v) {
+  return __builtin_bit_cast(
+      float, __builtin_elementwise_sub_sat(__builtin_bit_cast(unsigned int, v), 1u));
+}
+
 // eight fp8 -> eight bf16 (exact)
 DEVICE_INLINE u32x4 fp8x8_bf16(u32x2 w) {
   u32x4 o;
@@ -778,15 +787,17 @@ void paged_attn_decode_kernel(
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[i][r] *= corr;
     }
-    // weights in three bf16 parts, whose sum they are
+    // weights in three bf16 parts, whose sum they are; of bf16 pools none of them 0
     u32x4 w[3];
 #pragma unroll
     for (int t = 0; t < 3; ++t) {
 #pragma unroll
       for (int i = 0; i < NK / 2; ++i) {
-        w[t][i] = pack_hi(x[i * 2], x[i * 2 + 1]);
-        x[i * 2] -= high_half(x[i * 2]);
-        x[i * 2 + 1] -= high_half(x[i * 2 + 1]);
+        const float lo = !FP8 && t < 2 ? next_below(x[i * 2]) : x[i * 2];
+        const float hi = !FP8 && t < 2 ? next_below(x[i * 2 + 1]) : x[i * 2 + 1];
+        w[t][i] = pack_hi(lo, hi);
+        x[i * 2] -= high_half(lo);
+        x[i * 2 + 1] -= high_half(hi);
       }
     }
     // Rows that are not the sequence's (behind its end in its last page, in front

@@ -86,3 +86,37 @@ def test_pools_at_odd_places(lens, fp8):
                           torch.tensor(lens, dtype=torch.int32, device="cuda"),
                           128 ** -0.5)
     _check(out, q, kc, vc, bt, lens, fp8, list(range(len(lens)))[:4])
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("lens", [[1, 40, 200, 1000], [150] * 300])
+@pytest.mark.parametrize("G", [1, 4])
+def test_infinite_values(monkeypatch, lens, D, G):
+    """An infinity in the values comes out, whatever its key's weight (the largest one's
+    is exactly 1), and a NaN only where two of them meet; one head a kv head or four."""
+    from gpustack_amd import ops
+
+    monkeypatch.setenv("GPUSTACK_AMD_OSS_KERNELS", "1")
+    kc, vc, bt, q = _pools(lens, 2, D, False, D + len(lens))
+    q = q[:, :2 * G].contiguous()
+    rows = list(range(min(len(lens), 4)))
+    for i in rows:
+        def at(j):                      # the place of key j
+            return bt[i, j // 16].long(), slice(None), j % 16
+        s = (q[i].view(2, G, D)[:, :, None].float() * torch.stack(
+            [kc[at(j)] for j in range(lens[i])], 1)[:, None].float()).sum(-1)
+        top = s[0, 0].argmax().item()   # the largest weight of the first head
+        vc[at(top)][:, 3] = float("inf")
+        vc[at(lens[i] - 1)][:, 5] = float("-inf")
+        vc[at(0)][:, 7], vc[at(lens[i] // 2)][:, 9] = float("inf"), float("inf")
+        vc[at(lens[i] - 1)][:, 9] = float("-inf")
+    out = torch.full_like(q, float("nan"))
+    ops.paged_attn_decode(out, q, kc, vc, bt,
+                          torch.tensor(lens, dtype=torch.int32, device="cuda"),
+                          D ** -0.5)
+    ref = _reference(q[rows], kc, vc, bt[rows], [lens[i] for i in rows], D ** -0.5)
+    out = out[rows].double()
+    odd = ~ref.isfinite()
+    assert int(odd.sum()) >= 4 * len(rows) * 2 * G
+    assert torch.equal(out[odd].nan_to_num(nan=5.0), ref[odd].nan_to_num(nan=5.0))
+    assert bool((out - ref)[~odd].abs().le(ref[~odd].abs() * 2.0 ** -8 + 1e-4).all())
