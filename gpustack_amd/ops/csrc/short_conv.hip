@@ -101,8 +101,8 @@ __global__ __launch_bounds__(256) void short_conv_step_kernel(
 // The same for bf16 rows whose channel count, first column and row stride
 // are multiples of 8: a lane takes 8 neighbouring channels of RB rows in a
 // row with 16-byte loads, its TAPS x 8 weights in registers. Bound by the rows'
-// bytes and the activation: 7032 rows of 6144, four taps, 52.7 us (with expf and a
-// division, and a branch for every tap, 63; row by row, each waited for its
+// bytes and the activation: 7032 rows of 6144, four taps, 51 us (with expf and a
+// division, and a branch for every tap, 61; row by row, each waited for its
 // sequence's numbers and read its taps' rows again, 87).
 // grid (ceil(T / RB), ceil(C / 8 / 256)).
 constexpr int RB = 8;

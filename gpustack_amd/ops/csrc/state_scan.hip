@@ -35,7 +35,7 @@ template <> DEVICE_INLINE void st<unsigned short>(unsigned short* p, float v) {
 }
 
 // (With expf and a division the chunks of an activated scan, 7032 rows of 16 heads of
-// 128 x 128, took 246 us in both launches, and take 228.)
+// 128 x 128, took 262 us in both launches, and take 251.)
 DEVICE_INLINE float silu_f(float z) { return over_one_plus_exp(z, z); }
 DEVICE_INLINE float sigmoid_f(float z) { return over_one_plus_exp(1.f, z); }
 // softplus without a switch-over: max(x, 0) + log1p(exp(-|x|))
@@ -1170,8 +1170,8 @@ __global__ __launch_bounds__(ROW_THREADS) void gated_group_norm_vec_kernel(
 
 // Parts of more than 256 and up to 512 NV channels, a multiple of 8, of rows at 16-byte
 // addresses: a wave to a part, without the LDS or a barrier. Bound by the rows' bytes:
-// 7032 rows of 8 parts of 512 42 us (a workgroup to a part, half of whose lanes had no
-// channels, 62.8).
+// 7032 rows of 8 parts of 512 47.6 us (a workgroup to a part, half of whose lanes had
+// no channels, with expf and a division 68.6).
 template <int NV>
 __global__ __launch_bounds__(ROW_THREADS) void gated_group_norm_wave_kernel(
     unsigned short* __restrict__ out, const float* __restrict__ y,

@@ -135,3 +135,28 @@ def test_activation_of_all_sizes():
     e = (rows - want[1:]).abs()
     assert bool((e[ok] <= want[1:].abs()[ok] * 2.0 ** -8 + 1e-36).all())
     assert bool(rows[src[1:].isnan()].isnan().all())
+
+
+def test_activation_in_fp32():
+    """Every result that fp32 holds to within three halves of its last place (the power
+    of two has one, the quotient one half), those near the end of the range, where the
+    exponential is largest, too; normal numbers on average nearer than expf and a division
+    bring these (3.95e-8)."""
+    g = torch.Generator().manual_seed(4)
+    z = torch.cat([torch.randn(1 << 18, generator=g),
+                   torch.rand(1 << 17, generator=g) * 176 - 88,
+                   torch.rand(1 << 14, generator=g) * 1.4 - 88.7,
+                   torch.linspace(-17, -16, 1 << 15)]).cuda()
+    C, i32 = z.numel(), lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    src = torch.cat([torch.zeros(1, C, device="cuda"), z[None]])
+    w = torch.zeros(C, 2, device="cuda")
+    w[:, 1] = 1
+    out = torch.zeros(2, C, device="cuda")
+    ops.short_conv(out, src, 0, w, None, torch.zeros(1, 1, C, device="cuda"), i32([0]),
+                   i32([2]), i32([0]), i32([0, 0]), i32([0, 1]), silu=True)
+    want = z.double() / (1 + torch.exp(-z.double()))
+    e = (out[1].double() - want).abs()
+    assert bool((e <= want.abs() * 1.5 * 2.0 ** -23).all()), \
+        float((e / want.abs()).max())
+    n = 1 << 18
+    assert float(e[:n].norm() / want[:n].norm()) <= 3.9e-8
