@@ -981,15 +981,13 @@ __global__ __launch_bounds__(256, 2) void state_chunk_kernel(
 // in place and reduces y over the rows through LDS. More rows of a
 // sequence, should a batch bring them, are walked one after the other.
 // U state rows of a lane are in flight, the first of them beside the token's
-// values: one at a time, each behind the store of the one before, 64 sequences
-// of 16 heads of 128 x 128 took 34.4 us where these take 32.4 (134 MB, 4.1
-// TB/s); of 64 heads of 128 x 64 50.2 and 51.0 (268 MB), which is the memory.
-template <typename TS>
+// values; 0: each behind the store of the one before, as the compiler places it
+// (step_flight).
+template <typename TS, int U>
 __global__ __launch_bounds__(256) void state_step_kernel(
     float* __restrict__ y, const TS* __restrict__ src,
     const TS* __restrict__ dt_src, ScanArgs p) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
-  constexpr int U = 8;            // state rows of a lane in flight
   const int N = p.N, P = p.P, P4 = P / 4, RP = 256 / P4;
   float* vs = sm;                 // [P]      (16-byte reads: P % 4 == 0)
   float* part = vs + P;           // [RP][P]
@@ -1006,7 +1004,7 @@ __global__ __launch_bounds__(256) void state_step_kernel(
   const int g = h / (p.H / p.G);
   float* sp = p.state + ((long)slot * p.H + h) * N * P;
   const float skip = p.skip != nullptr ? p.skip[h] : 0.f;
-  f32x4 S[U];
+  f32x4 S[U > 0 ? U : 1];
   auto bring = [&](int n0, bool fresh) {
 #pragma unroll
     for (int j = 0; j < U; ++j) {
@@ -1016,7 +1014,7 @@ __global__ __launch_bounds__(256) void state_step_kernel(
         S[j] = *reinterpret_cast<const f32x4*>(sp + (long)nn * P + cg * 4);
     }
   };
-  bring(r0, hist <= 0);
+  if constexpr (U > 0) bring(r0, hist <= 0);
   for (int r = 0; r < n; ++r) {
     const TS* rp = src + (long)(first + r) * p.ld_src;
     __syncthreads();
@@ -1047,19 +1045,28 @@ __global__ __launch_bounds__(256) void state_step_kernel(
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     if (r0 < RP) {
       const f32x4 v4 = *reinterpret_cast<const f32x4*>(vs + cg * 4);
-      for (int n0 = r0; n0 < N; n0 += U * RP) {
-        if (n0 > r0 || r > 0) bring(n0, fresh);
+      auto put = [&](f32x4 state, int nn) {
+        const float bk = b * ks[nn], qn = qs[nn];
 #pragma unroll
-        for (int j = 0; j < U; ++j) {
-          const int nn = n0 + j * RP;
-          if (nn >= N) break;
-          const float bk = b * ks[nn], qn = qs[nn];
+        for (int k = 0; k < 4; ++k) {
+          state[k] = a * state[k] + bk * v4[k];
+          acc[k] += state[k] * qn;
+        }
+        *reinterpret_cast<f32x4*>(sp + (long)nn * P + cg * 4) = state;
+      };
+      if constexpr (U == 0) {
+        for (int nn = r0; nn < N; nn += RP)
+          put(fresh ? f32x4{0.f, 0.f, 0.f, 0.f}
+                    : *reinterpret_cast<const f32x4*>(sp + (long)nn * P + cg * 4), nn);
+      } else {
+        for (int n0 = r0; n0 < N; n0 += U * RP) {
+          if (n0 > r0 || r > 0) bring(n0, fresh);
 #pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            S[j][k] = a * S[j][k] + bk * v4[k];
-            acc[k] += S[j][k] * qn;
+          for (int j = 0; j < U; ++j) {
+            const int nn = n0 + j * RP;
+            if (nn >= N) break;
+            put(S[j], nn);
           }
-          *reinterpret_cast<f32x4*>(sp + (long)nn * P + cg * 4) = S[j];
         }
       }
       *reinterpret_cast<f32x4*>(part + r0 * P + cg * 4) = acc;
@@ -1071,6 +1078,25 @@ __global__ __launch_bounds__(256) void state_step_kernel(
       y[(long)(first + r) * p.H * P + h * P + i] = o;
     }
   }
+}
+
+// State rows of a lane in flight, by the rows that it has and the workgroups. Few
+// workgroups wait for their own rows, with many each memory channel has work anyway, and
+// a state's few rows then only come to it in another order. us, one by one / four /
+// eight (less than 3 % is within the runs):
+//   2 rows:  256 workgroups 5.0 / 4.9 / 5.1, 1024 7.2 / 6.8 / 7.0, 2048 12.7 / 10.8 / 11.9,
+//            4096 20.0 / 20.9 / 22.8, 8192 33.5 / 34.3 / 38.5
+//   4:       512 7.0 / 6.5 / 6.6, 1024 12.7 / 9.8 / 10.0, 2048 18.6 / 19.7 / 19.8, 4096
+//            31.0 / 32.3 / 33.5, 8192 56.5 / 58.2 / 59.6
+//   8:       256 7.6 / 7.0 / 6.8, 512 13.4 / 10.2 / 10.0, 1024 18.6 / 19.2 / 18.5, 2048
+//            30.8 / 30.5 / 32.5, 4096 58.9 / 55.1 / 56.9, 8192 105.8 / 106.2 / 108.1
+//   16:      256 16.5 / 12.8 / 9.7, 1024 37.3 / 37.4 / 36.0, 2048 65.6 / 60.3 / 60.6,
+//            4096 121.6 / 113.1 / 112.5, 8192 217.6 / 217.5 / 218.1
+int step_flight(int N, int P, long workgroups) {
+  const int rows = (N + 1024 / P - 1) / (1024 / P);
+  if (rows > 8) return 8;
+  if (rows > 4) return workgroups <= 1024 ? 8 : 4;
+  return workgroups <= 1024 ? 4 : 0;
 }
 
 constexpr int ROW_THREADS = 256;
@@ -1406,12 +1432,17 @@ int state_scan_launch(float* y, const void* src, long ld_src, int col_x,
   if (step_rows(single, N, P)) {
     const int P4 = P / 4;
     const size_t smem = (size_t)(2 * N + P + (256 / P4) * P) * sizeof(float);
-    if (src_bf)
-      state_step_kernel<unsigned short><<<dim3(nseq, H), 256, smem, s>>>(
-          y, (const unsigned short*)src, (const unsigned short*)dt_src, p);
-    else
-      state_step_kernel<float><<<dim3(nseq, H), 256, smem, s>>>(
-          y, (const float*)src, (const float*)dt_src, p);
+#define STEP(T_, U)                                                          \
+  state_step_kernel<T_, U><<<dim3(nseq, H), 256, smem, s>>>(                  \
+      y, (const T_*)src, (const T_*)dt_src, p)
+    const int flight = step_flight(N, P, (long)nseq * H);
+    if (src_bf && flight == 8) STEP(unsigned short, 8);
+    else if (src_bf && flight == 4) STEP(unsigned short, 4);
+    else if (src_bf) STEP(unsigned short, 0);
+    else if (flight == 8) STEP(float, 8);
+    else if (flight == 4) STEP(float, 4);
+    else STEP(float, 0);
+#undef STEP
     return 1;
   }
   if (src_bf)
