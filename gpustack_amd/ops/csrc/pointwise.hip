@@ -471,11 +471,12 @@ __global__ __launch_bounds__(256) void qkv_store_kernel(
 
 // ---------------------------------------------------------------------------
 // Greedy sampling: argmax over vocab per row (ties -> lowest index).
-// One block per row: 16 waves with eight 16-byte loads in flight each, the
+// One block per row: 16 waves with four 16-byte loads in flight each, the
 // maximum of eight values first and its place only where it counts. Bound by
 // how fast one CU takes a row in and compares it (256 KB of a 128256-word
-// vocabulary): one row 7.0 us, 16 7.4 (with four loads at a time, and what four
-// do not divide one by one, 7.1 and 7.6).
+// vocabulary): one row 8.1 us, 16 8.6, 64 8.8, 300 17. With eight loads in flight,
+// the last ones once more behind the end, these take 7.6, 8.0, 8.2 and 17.1, but
+// 64 rows of 4096 words 3.9 for 3.1, of 151936 10.1 for 9.5, 300 of 32001 10.4 for 8.6.
 // The words are also left in `host` (pinned memory, or null), which saves a copy
 // behind the kernel.
 // ---------------------------------------------------------------------------
@@ -484,7 +485,6 @@ constexpr int GS_THREADS = 1024;
 __global__ __launch_bounds__(GS_THREADS) void greedy_sample_kernel(
     long* __restrict__ out, long* __restrict__ host,
     const unsigned short* __restrict__ logits, int N, int V) {
-  constexpr int U = 8;
   const int row = blockIdx.x;
   if (row >= N) return;
   const unsigned short* rp = logits + (long)row * V;
@@ -504,14 +504,17 @@ __global__ __launch_bounds__(GS_THREADS) void greedy_sample_kernel(
       besti = v * 8 + i;
     }
   };
-  for (int v0 = threadIdx.x; v0 < nvec; v0 += U * GS_THREADS) {
-    u16x8 u[U];                        // the last ones once more behind the end
+  int v = threadIdx.x;
+  for (; v + 3 * GS_THREADS < nvec; v += 4 * GS_THREADS) {
+    u16x8 u[4];
 #pragma unroll
-    for (int j = 0; j < U; ++j)
-      u[j] = *reinterpret_cast<const u16x8*>(rp + min(v0 + j * GS_THREADS, nvec - 1) * 8);
+    for (int j = 0; j < 4; ++j)
+      u[j] = *reinterpret_cast<const u16x8*>(rp + (v + j * GS_THREADS) * 8);
 #pragma unroll
-    for (int j = 0; j < U; ++j) take(u[j], min(v0 + j * GS_THREADS, nvec - 1));
+    for (int j = 0; j < 4; ++j) take(u[j], v + j * GS_THREADS);
   }
+  for (; v < nvec; v += GS_THREADS)
+    take(*reinterpret_cast<const u16x8*>(rp + v * 8), v);
   for (int gi = nvec * 8 + threadIdx.x; gi < V; gi += GS_THREADS) {
     const float f = bf2f(rp[gi]);
     if (f > best) { best = f; besti = gi; }

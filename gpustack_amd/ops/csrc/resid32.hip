@@ -9,6 +9,8 @@
 // the row stay in L1/L2.
 #include "common.h"
 
+#include <type_traits>
+
 namespace {
 
 template <typename T> DEVICE_INLINE float ld(const T* p);
@@ -464,41 +466,52 @@ __global__ __launch_bounds__(ROW_THREADS) void moe_combine_vec_kernel(
   }
 }
 
-// 16 waves a row with eight 16-byte loads in flight each: bound by the round trip and
-// the joins (64 rows of 32000 4.7 us; four loads of 4 bytes, ten round trips, 5.2). 4
-// waves up to 4096 words, where waves without any are what is left (512 rows of 1000,
-// us: 4.6 -> 3.3). The words are also left in `host` (pinned memory, or null).
-typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
-
-template <int AM_THREADS>
+// 16 waves a row, 4 up to 4096 words, where waves without any are what is left (512 rows
+// of 1000, us: 4.6 -> 3.3). WIDE: four 16-byte loads of a lane in flight, then two and
+// one, else four of a word. Bound by the round trips where CUs have a row, else by the
+// comparisons: us, words / wide, 64 rows of 32000 7.7 / 6.0, of 128256 25 / 15, of 1000
+// 2.96 / 2.77, 600 of 128256 68 / 58; but where some CUs have two rows and most one, and
+// rows are long, the wide form's registers keep a CU at one: 300 rows of 151936 36.9 / 40.9,
+// of 128256 30.8 / 33.4, of 32000 12.1 / 11.9, 500 of 151936 53.6 / 54.1. The words are also
+// left in `host` (pinned memory, or null).
+template <int AM_THREADS, bool WIDE>
 __global__ __launch_bounds__(AM_THREADS) void argmax_f32_kernel(
     long* __restrict__ out, long* __restrict__ host,
     const float* __restrict__ logits, int V) {
-  constexpr int U = 8;
   __shared__ float bv[AM_THREADS / 64];
   __shared__ int bi[AM_THREADS / 64];
   const long t = blockIdx.x;
   const float* z = logits + t * V;
   float v = -INFINITY;
   int idx = 0x7fffffff;
-  const int nvec = V / 4;
-  for (int i0 = threadIdx.x; i0 < nvec; i0 += U * AM_THREADS) {
-    f32x4_any f[U];                    // the last ones once more behind the end
+  int i = threadIdx.x;
+  auto take = [&](auto count, auto each, int n) {   // U pieces of E words at a time
+    constexpr int U = decltype(count)::value, E = decltype(each)::value;
+    typedef float piece_t __attribute__((ext_vector_type(E), aligned(4)));
+    for (; i + (U - 1) * AM_THREADS < n; i += U * AM_THREADS) {
+      piece_t f[U];
 #pragma unroll
-    for (int j = 0; j < U; ++j)
-      f[j] = *reinterpret_cast<const f32x4_any*>(
-          z + min(i0 + j * AM_THREADS, nvec - 1) * 4);
+      for (int j = 0; j < U; ++j)
+        f[j] = *reinterpret_cast<const piece_t*>(z + (long)(i + j * AM_THREADS) * E);
 #pragma unroll
-    for (int j = 0; j < U; ++j)
+      for (int j = 0; j < U; ++j)
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if (f[j][k] > v) {
-          v = f[j][k];
-          idx = min(i0 + j * AM_THREADS, nvec - 1) * 4 + k;
-        }
+        for (int k = 0; k < E; ++k)
+          if (f[j][k] > v) { v = f[j][k]; idx = (i + j * AM_THREADS) * E + k; }
+    }
+  };
+  std::integral_constant<int, 1> one;
+  std::integral_constant<int, 2> two;
+  std::integral_constant<int, 4> four;
+  if constexpr (WIDE) {
+    take(four, four, V / 4);
+    take(two, four, V / 4);
+    take(one, four, V / 4);
+    i = V / 4 * 4 + threadIdx.x;
+  } else {
+    take(four, one, V);
   }
-  for (int i = nvec * 4 + threadIdx.x; i < V; i += AM_THREADS)
-    if (z[i] > v) { v = z[i]; idx = i; }
+  take(one, one, V);
   wave_argmax(v, idx);
   if ((threadIdx.x & 63) == 0) { bv[threadIdx.x >> 6] = v; bi[threadIdx.x >> 6] = idx; }
   __syncthreads();
@@ -663,6 +676,9 @@ void moe_combine_launch(void* out, const void* y, const int* inv,
 void argmax_f32_launch(long* out, long* host, const float* logits, int N, int V,
                        hipStream_t s) {
   if (N == 0) return;
-  if (V <= 4096) argmax_f32_kernel<256><<<N, 256, 0, s>>>(out, host, logits, V);
-  else argmax_f32_kernel<1024><<<N, 1024, 0, s>>>(out, host, logits, V);
+  // rows between one and less than two to a CU, long ones
+  const bool uneven = N > 256 && N <= 448 && V > 40000;
+  if (V <= 4096) argmax_f32_kernel<256, true><<<N, 256, 0, s>>>(out, host, logits, V);
+  else if (uneven) argmax_f32_kernel<1024, false><<<N, 1024, 0, s>>>(out, host, logits, V);
+  else argmax_f32_kernel<1024, true><<<N, 1024, 0, s>>>(out, host, logits, V);
 }

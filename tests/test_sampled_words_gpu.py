@@ -35,6 +35,19 @@ def test_first_of_the_largest(V, dtype):
             assert host.tolist() == want + [-5, -5]
 
 
+@pytest.mark.parametrize("V", [40000, 40005, 69637])
+def test_more_rows_than_the_chip_has(V):
+    """257 rows: fp32 words one at a time above 40000, else four."""
+    x = torch.zeros(257, V, device="cuda")
+    at = [(i * 7919) % V for i in range(257)]
+    for i, j in enumerate(at):
+        x[i, j:] = 1.0
+    x[5, V - 1] = 2.0
+    out = torch.full((257,), -3, dtype=torch.long, device="cuda")
+    ops.greedy_sample_into(out, x)
+    assert out.tolist() == at[:5] + [V - 1] + at[6:]
+
+
 def test_words_in_ordinary_memory_are_refused():
     out = torch.zeros(2, dtype=torch.long, device="cuda")
     for dtype in (torch.bfloat16, torch.float32):
