@@ -1480,8 +1480,13 @@ void gated_group_norm_launch(void* out, const float* y, const float* ysc,
 #undef GGN
     return;
   }
+  // A wave to a part from 6144 of them on; of fewer a part's own chain is what is left,
+  // which a workgroup shares. us, workgroup / wave, gate first and behind, parts of 512:
+  // 512 2.9 / 4.1 and 2.8 / 3.5, 2048 4.1 / 5.3 and 4.0 / 4.3, 4096 6.7 / 7.3 and 6.6 / 6.3,
+  // 6144 8.7 / 8.9 and 8.4 / 7.5, 24576 27 / 24 and 27 / 19; of 1024 2048 5.9 / 7.2 and 5.8 /
+  // 6.4, 6144 11.9 / 12.2 and 11.8 / 11.5; of 264 4096 5.5 / 6.2 and 5.5 / 5.2.
   if (gate_bf && out_bf && gs % 8 == 0 && C == groups * gs && ld_gate % 8 == 0 &&
-      gs <= 1024 && groups > 1 &&
+      gs <= 1024 && groups > 1 && (long)T * groups >= 6144 &&
       (((uintptr_t)gate | (uintptr_t)y | (uintptr_t)w | (uintptr_t)out) % 16) == 0) {
     const long units = (long)T * groups;
     const dim3 wgrid((unsigned)((units + 3) / 4));

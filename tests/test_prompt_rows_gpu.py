@@ -24,6 +24,19 @@ def _rnd(seed):
 @pytest.mark.parametrize("first", [True, False])
 @pytest.mark.parametrize("T", [1, 7])
 def test_parts_of_a_wave(gs, groups, first, T):
+    _parts(gs, groups, first, T)
+
+
+@pytest.mark.parametrize("gs,groups", [(264, 3), (512, 8), (520, 2), (1024, 2)])
+@pytest.mark.parametrize("first", [True, False])
+@pytest.mark.parametrize("more", [-1, 0, 1])
+def test_many_parts(gs, groups, first, more):
+    """Around 6144 of them, from where on a wave has a part; the last workgroup full and
+    not."""
+    _parts(gs, groups, first, 6144 // groups + more)
+
+
+def _parts(gs, groups, first, T):
     rnd, C = _rnd(gs + groups), gs * groups
     y, gate, w = rnd(T, C) * 3, rnd(T, C + 16).bfloat16()[:, 8:8 + C], rnd(C)
     o = torch.zeros(T, C, dtype=torch.bfloat16, device="cuda")
