@@ -502,17 +502,16 @@ __global__ __launch_bounds__(THREADS) void paged_attn_mfma_kernel(
 // so that nothing waits at a barrier and a wave's next keys and these values (16 KB)
 // are under way all the time. S^T = K Q^T in an order of the key rows (key_at) in which
 // a lane's 8 weights of 32 keys are neighbours, as the value pages hold them: the
-// weights stay in its registers. VT tiles of 16 channels, all of them loaded: behind a
-// branch for each that VW may leave out, the wait for the keys took in the values asked
-// for behind them, and a step cost two latencies. Bound by memory, us, with the branches
-// / now: 64 rows of 16 heads on 4 behind 200 to 3000 keys 54.5 / 51.4 (210 MB, cold), in
+// weights stay in its registers. VT tiles of 16 channels, all of them loaded (ALL): behind
+// a branch for each that VW may leave out, the wait for the keys takes in the values asked
+// for behind them, and a step costs two latencies. Bound by memory, us, with the branches
+// / without: 64 rows of 16 heads on 4 behind 200 to 3000 keys 54.5 / 51.4 (210 MB, cold), in
 // a window of 1024 29.1 / 27.7 (118 MB; a workgroup to a tile of 64 keys, its scores and
 // weights through the LDS with three barriers, took 34), 33 rows behind 1000 to 8000 in
 // the window 26.1 / 23.6, 16 behind 300 to 1200 15.8 / 14.8, one behind 7000 20.8 /
-// 19.2; where every CU has four workgroups they ask for more than it takes: 256 rows
-// behind 100 to 1500 90.4 / 91.0, in the window 82 / 85.5. Eight waves for four, of half
-// the keys each, are no faster (27.7, 11.6 for 12.0 behind 7000 in the window, 102 for 94).
-template <typename TO, int VT>
+// 19.2 (launch_mfma has where the branches stay). Eight waves for four, of half the keys
+// each, are no faster (27.7, 11.6 for 12.0 behind 7000 in the window, 102 for 94).
+template <typename TO, int VT, bool ALL>
 __global__ __launch_bounds__(THREADS, 2) void paged_attn_waves_kernel(
     TO* __restrict__ out, const unsigned short* __restrict__ q,
     const unsigned short* __restrict__ k_cache,
@@ -607,8 +606,10 @@ __global__ __launch_bounds__(THREADS, 2) void paged_attn_waves_kernel(
       const unsigned short* pt =
           v_cache + (blk * p.G + g) * (long)VW * BS + (lg & 1) * 8 + lc * BS;
 #pragma unroll
-      for (int c = 0; c < VT; ++c)           // the last ones once more behind VW
-        vreg[c] = *reinterpret_cast<const u16x8*>(pt + min(c * 16, VW - 16) * BS);
+      for (int c = 0; c < VT; ++c)           // ALL: the last ones once more behind VW
+        if (ALL || c * 16 < VW)
+          vreg[c] = *reinterpret_cast<const u16x8*>(
+              pt + (ALL ? min(c * 16, VW - 16) : c * 16) * BS);
     }
     f32x4 s[2];
 #pragma unroll
@@ -659,7 +660,8 @@ __global__ __launch_bounds__(THREADS, 2) void paged_attn_waves_kernel(
         for (int r = 0; r < 4; ++r) acc[c][r] *= alpha;
     }
 #pragma unroll
-    for (int c = 0; c < VT; ++c) acc[c] = ra_mfma(vreg[c], w, acc[c]);
+    for (int c = 0; c < VT; ++c)
+      if (ALL || c * 16 < VW) acc[c] = ra_mfma(vreg[c], w, acc[c]);
   }
   l_run += __shfl_xor(l_run, 16, WAVE_SIZE);
   l_run += __shfl_xor(l_run, 32, WAVE_SIZE);
@@ -1080,14 +1082,20 @@ void launch_mfma(void* out, const void* q, const void* kc, const void* vc,
   bool alone = false;
   if constexpr (NT == 2) {
     alone = p.D == 128;
-    if (alone && p.VW > 96)
-      paged_attn_waves_kernel<TO, 8><<<dim3(ntiles, nsplit), THREADS, 0, s>>>(
-          (TO*)out, (const unsigned short*)q, (const unsigned short*)kc,
-          (const unsigned short*)vc, p, ws_acc, ws_ml);
-    else if (alone)
-      paged_attn_waves_kernel<TO, 6><<<dim3(ntiles, nsplit), THREADS, 0, s>>>(
-          (TO*)out, (const unsigned short*)q, (const unsigned short*)kc,
-          (const unsigned short*)vc, p, ws_acc, ws_ml);
+    // About four tiles a CU of uneven lengths end with the longest, which the others'
+    // values, all asked for at once, keep waiting; us, a branch for each / all: rows behind
+    // 100 to 1500 keys in a window of 1024, 16 heads on 4, 800 tiles 65.8 / 64.3, 864 67.2
+    // / 72.8, 1024 81.5 / 84.6, 1088 85.4 / 87.6, 1152 91.3 / 92.5, 1200 95.7 / 95.3 (but
+    // 1024 behind 600 to 1200 95.4 / 91.6).
+    const bool branch = ntiles > 816 && ntiles <= 1184;
+#define WAVES(VT, ALL)                                                        \
+  paged_attn_waves_kernel<TO, VT, ALL><<<dim3(ntiles, nsplit), THREADS, 0, s>>>( \
+      (TO*)out, (const unsigned short*)q, (const unsigned short*)kc,          \
+      (const unsigned short*)vc, p, ws_acc, ws_ml)
+    if (alone && branch) WAVES(8, false);
+    else if (alone && p.VW > 96) WAVES(8, true);
+    else if (alone) WAVES(6, true);
+#undef WAVES
   }
   if (!alone)
     paged_attn_mfma_kernel<NT, TO><<<dim3(ntiles, nsplit), THREADS, smem, s>>>(

@@ -82,6 +82,17 @@ class TestOptions:
         _run(hists, news, H, 4, 128, nsplit, **kw)
 
 
+@pytest.mark.parametrize("S", [408, 409, 592, 593])
+@pytest.mark.parametrize("VW", [128, 80])
+class TestManyTiles:
+    pytestmark = gpu
+
+    def test_as_the_fp32_path(self, S, VW):
+        """Two kv heads: 816, 818, 1184 and 1186 tiles, the edges between which each
+        tile of channels is behind a branch."""
+        _run([(i * 37) % 300 for i in range(S)], [1] * S, 8, 2, VW, 1, window=128)
+
+
 @pytest.mark.parametrize("nsplit", [1, 2, 5])
 @pytest.mark.parametrize("last", [32, 64, 96, 192])
 class TestNotANumber:
