@@ -24,6 +24,7 @@ HEADERS = ["common.h", "wide_tiles.h", "pinned_words.h"]
 # the fp32-residual op family lives in its own small library: a checkout
 # that serves only such a model compiles these few files and nothing else
 LATENT_SO_PATH = PKG_DIR / "_hip_latent.so"
+SMALL_HEADERS = ["common.h", "short_conv_binding.h", "pinned_words.h"]
 LATENT_SOURCES = ["resid32.hip", "latent_attn.hip", "grouped_ff.hip",
                   "latent_bindings.cpp"]
 
@@ -188,8 +189,7 @@ def _build_small(ext_name: str, sources: list[str], so_path: Path,
     flags = _common_flags(abi, ext_name)
     build_dir = CSRC / f".build{ext_name}"
     build_dir.mkdir(exist_ok=True)
-    newest = max((CSRC / s).stat().st_mtime
-                 for s in sources + ["common.h", "short_conv_binding.h"])
+    newest = max((CSRC / s).stat().st_mtime for s in sources + SMALL_HEADERS)
     if (so_path.exists() and not force
             and so_path.stat().st_mtime >= newest):
         return so_path
