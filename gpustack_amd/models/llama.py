@@ -349,16 +349,16 @@ class Attention(nn.Module):
         qkv = qlinear(x, self.qkv_w, self.qkv_pack, self.qkv_b,
                       parts=store and meta.lora is None and ops.qkv_store_ok(
                           x, self.d, self.rot_dim, self.spec.rope_mode))
+        norms = (self.q_norm, self.k_norm) if head_norm else (None, None)
         if store and meta.own_rows and meta.lora is None \
                 and not (self.sinks is not None or self.window or self.softcap) \
                 and ops.qkv_store_ok(x, self.d, self.rot_dim, self.spec.rope_mode) \
                 and ops.paged_attn_decode_rows_ok(x, self.hq, self.hkv, self.d,
                                                   k_cache, v_cache,
-                                                  meta.block_tables):
+                                                  meta.block_tables, *norms):
             out = torch.empty(T, self.hq, self.d, dtype=x.dtype, device=x.device)
             ops.paged_attn_decode_rows(
-                out, qkv, self.hq, self.hkv, self.q_norm if head_norm else None,
-                self.k_norm if head_norm else None, cos_sin, meta.positions,
+                out, qkv, self.hq, self.hkv, *norms, cos_sin, meta.positions,
                 meta.slot_mapping, k_cache, v_cache, meta.block_tables,
                 meta.seq_lens, self.spec.rms_norm_eps, self.scale)
             return self.comm.all_reduce(

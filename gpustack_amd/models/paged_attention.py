@@ -151,7 +151,7 @@ class PagedRotaryAttention(nn.Module):
         else:
             qkv = ops.linear_auto(
                 h, self.qkv_w, m.head_norm and not self.rope_rows
-                and ops.head_norm_parts_ok(T, m.qk_dim, self.nv))
+                and ops.head_norm_parts_ok(T, m.qk_dim, self.nv, k_cache))
             if qkv.dim() == 3:
                 parts = qkv
                 qkv = torch.empty(T, parts.shape[2], dtype=h.dtype,

@@ -286,10 +286,10 @@ def paged_attn_decode(out, q, k_cache, v_cache, block_tables, seq_lens,
 
 
 def paged_attn_decode_rows_ok(rows, q_heads: int, kv_heads: int, head_dim: int,
-                              k_cache, v_cache, block_tables) -> bool:
+                              k_cache, v_cache, block_tables, *norms) -> bool:
     """Whether paged_attn_decode_rows takes a step: heads of 128 channels, two to
-    eight of them (not three) a kv head, without sinks, window or score cap; and
-    where it is the faster one. It saves 1.2 to 2.7 us up to four workgroups a CU
+    eight of them (not three) a kv head, without sinks, window or score cap, pools and
+    head norms (`norms`, or None) at 16-byte addresses; and where it is the faster one. It saves 1.2 to 2.7 us up to four workgroups a CU
     whatever the lengths (128 rows of 8 kv heads 14.5 -> 13.4 at 40 keys, 41.9 ->
     39.2 at 256 to 383). Behind them it loses contexts under 80 keys (256 rows of 40
     to 58 21.9 -> 22.8, 512 36.8 -> 40.7) and gains longer ones (80 to 109 54.5 ->
@@ -302,7 +302,8 @@ def paged_attn_decode_rows_ok(rows, q_heads: int, kv_heads: int, head_dim: int,
             and group in (2, 4, 5, 6, 7, 8)
             and (groups <= 512 if k_cache.element_size() == 1
                  else groups <= 1024 or pages >= 8)
-            and k_cache.data_ptr() % 16 == 0 and v_cache.data_ptr() % 16 == 0)
+            and not any(t.data_ptr() % 16 for t in (k_cache, v_cache, *norms)
+                        if t is not None))
 
 
 def paged_attn_decode_rows(out, rows, q_heads: int, kv_heads: int, q_norm, k_norm,
@@ -1616,11 +1617,12 @@ def add_layer_norm_rows(x, a, w, b, eps: float, rows, dtype):
     return h
 
 
-def head_norm_parts_ok(T: int, head_dim: int, nv: int) -> bool:
+def head_norm_parts_ok(T: int, head_dim: int, nv: int, k_cache) -> bool:
     """Whether head_norm_store adds a projection's parts up: whole lanes of 8
-    channels, rows whose weights bound the product (64 rows of 3072 x 2048 12.0 us
-    in the library, 6.5 cut over k)."""
-    return T <= 128 and head_dim in (64, 128, 256) and nv % 8 == 0
+    channels, a key pool at a 16-byte address, rows whose weights bound the product
+    (64 rows of 3072 x 2048 12.0 us in the library, 6.5 cut over k)."""
+    return T <= 128 and head_dim in (64, 128, 256) and nv % 8 == 0 \
+        and k_cache.data_ptr() % 16 == 0
 
 
 def head_norm_store(q_out, qkv, nq: int, nk: int, q_w, k_w, head_dim: int,

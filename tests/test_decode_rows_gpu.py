@@ -96,6 +96,43 @@ def test_where_it_is_taken():
     assert not ok(1, 4, Hq=24) and not ok(1, 4, Hq=8) and not ok(1, 4, Hq=72)
 
 
+@pytest.mark.parametrize("skew", [0, 1, 4])
+def test_head_norms_elsewhere(skew):
+    """An attention layer whose head norms lie at any address takes a step of rows of
+    their own, as it takes the same without saying that they are."""
+    from types import SimpleNamespace
+
+    from gpustack_amd.models.llama import Attention, ForwardMeta
+
+    Hq, Hkv, N, H = 8, 2, 3, 256
+    g = torch.Generator(device="cuda").manual_seed(skew)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    a = Attention.__new__(Attention)
+    torch.nn.Module.__init__(a)
+    a.spec = SimpleNamespace(qk_norm=True, qk_norm_full=False, qk_norm_after_rope=False,
+                             rope_mode="neox", rms_norm_eps=1e-5, attn_temp_scale=0)
+    a.comm = SimpleNamespace(all_reduce=lambda x: x)
+    a.hq, a.hkv, a.d, a.rot_dim, a.scale = Hq, Hkv, D, D, D ** -0.5
+    a.use_rope, a.sinks, a.window, a.softcap = True, None, 0, None
+    a.qkv_w, a.o_w = rnd((Hq + 2 * Hkv) * D, H) / 16, rnd(H, Hq * D) / 32
+    a.qkv_b = a.o_b = a.qkv_pack = a.o_pack = None
+    a.q_norm, a.k_norm = (rnd(D + 8)[skew:skew + D] for _ in range(2))
+    x, cs = rnd(N, H), torch.randn(64, D, generator=g, device="cuda")
+    pools = [rnd(4, Hkv, 16, D) for _ in range(2)]
+    pos = torch.tensor([5, 15, 0], device="cuda")
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    res = []
+    for own in (False, True):
+        kc, vc = (t.clone() for t in pools)
+        meta = ForwardMeta(is_prefill=False, positions=pos,
+                           slot_mapping=pos + torch.arange(N, device="cuda") * 16,
+                           logits_indices=None, block_tables=i32([[0], [1], [2]]),
+                           seq_lens=(pos + 1).int(), own_rows=own)
+        res.append((a(x, meta, cs, kc, vc), kc, vc))
+    for u, v in zip(*res):
+        assert torch.equal(u, v)
+
+
 def test_other_heads_are_refused():
     z = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device="cuda")
     for Hq, Hkv, d in ((4, 4, 128), (6, 2, 128), (8, 2, 64)):

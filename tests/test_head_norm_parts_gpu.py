@@ -55,4 +55,21 @@ def test_heads_of_other_sizes_are_refused():
         ops.head_norm_store(z(T, D), z(T, 3 * D), D, D, w, w, D, 0.0, 0, i.int(),
                             None, None, z(1, 1, 16, D), z(1, 1, D, 16), i, 1e-5,
                             parts=torch.zeros(2, T, 3 * D, device="cuda"))
-    assert not ops.head_norm_parts_ok(T, D, D)
+    assert not ops.head_norm_parts_ok(T, D, D, z(16))
+
+
+def test_pools_elsewhere():
+    """Parts only where the key pool is at a 16-byte address; else rows, as before."""
+    T, D, rnd = 5, 64, torch.randn(5, 192, device="cuda").bfloat16()
+    pool = torch.zeros(16 * D + 8, dtype=torch.bfloat16, device="cuda")
+    kc, res = pool[3:3 + 16 * D].view(1, 1, 16, D), []
+    assert ops.head_norm_parts_ok(T, D, D, pool)
+    assert not ops.head_norm_parts_ok(T, D, D, kc)
+    w, i = torch.ones(D, device="cuda"), torch.arange(T, device="cuda")
+    for k in (kc, torch.zeros(1, 1, 16, D, dtype=torch.bfloat16, device="cuda")):
+        q, vc = torch.zeros(T, D, device="cuda").bfloat16(), kc.new_zeros(1, 1, D, 16)
+        ops.head_norm_store(q, rnd.clone(), D, D, w, w, D, 0.0, 0, i.int(), None, None,
+                            k, vc, i, 1e-5)
+        res.append((q, k, vc))
+    for a, b in zip(*res):            # the sum of the squares in another order
+        assert bool(((a - b).abs().float() <= b.abs().float() * 2.0 ** -7).all())
