@@ -18,7 +18,7 @@
 //    keys instead of four per key.
 //  - probabilities stay fp32. paged_attn_decode_kernel multiplies them with the values
 //    on the matrix cores, in three parts; paged_attn_heads_kernel, for one query head a
-//    kv head, with fp32 FMA.
+//    kv head and some of two of 64 channels, with fp32 FMA.
 //  - fp8 keys become bf16 exactly (e4m3 has 3 mantissa bits) in registers.
 //
 // Bound by the K/V stream where the chip is full (5.3 to 5.5 TB/s), else by the longest
@@ -29,8 +29,9 @@
 
 #include <type_traits>
 
-// parts of a sequence, a part's keys, and whether a kv head's query heads go together
-struct DecodeParts { int n, least, grouped; };
+// parts of a sequence, a part's keys, and the query heads of a workgroup: one or two
+// (paged_attn_heads_kernel), or 0, all of a kv head (paged_attn_decode_kernel)
+struct DecodeParts { int n, least, heads; };
 
 // The step's rows as they leave the projection, where the kernel norms, rotates and
 // stores them itself: q | k | v in bf16, or (rows null) as fp32 parts of it.
@@ -155,10 +156,13 @@ DEVICE_INLINE int window_start(int len, int window) {
 // heads of 128 63 / 69, 72 x 39 14.9 / 16.6, 31 x 37 in fp8 6.6 / 8.3; 64 channels
 // in fp8, 476 x 1150 in a window of 128 63 / 79. (Of 36 batches of 128 channels the
 // products would be the faster ones by 5 % on average, 9 of them slower, to 1.27.)
+// Two heads of 64 channels (GQ = 2), us, this / those: 16 on 8 in fp8, 8 x 20 to 64 keys
+// behind a wide table 4.8 / 5.7, 384 11.0 / 14.8, 8 x 200 to 400 6.0 / 7.1, 128 x 500 to
+// 1200 30.9 / 28.1; 8 x 20 to 64 behind a table of 64 3.4 / 4.0, in bf16 too.
 //  - probabilities go through LDS to a layout of 16 lanes a value row (D/16 channels
 //    each) x 4 keys, where the weighted sum is fp32 FMA on values loaded 16 bytes
 //    (bf16) or 8 bytes (fp8) a lane.
-template <int D, bool FP8, bool EXT>
+template <int D, int GQ, bool FP8, bool EXT>
 __global__ __launch_bounds__(THREADS, D == 64 ? 5 : D == 256 ? (FP8 ? 3 : 2) : 4)
 void paged_attn_heads_kernel(
     unsigned short* __restrict__ out,        // [N, Hq, D]
@@ -167,13 +171,12 @@ void paged_attn_heads_kernel(
     const char* __restrict__ vc,             // [B, Hkv, BS, D]
     const int* __restrict__ block_tables,    // [N, max_blocks]
     const int* __restrict__ seq_lens,        // [N]
-    float* __restrict__ part,                // [N, Hq, nsplit, D + 2]
+    float* __restrict__ part,                // [N, Hq / GQ, nsplit, GQ, D + 2]
     int least,                               // keys of a part (part_tokens)
     int Hkv, int rep, int max_blocks, float scale, long q_stride,
     const float* __restrict__ sinks,         // [Hq] or null (GPT-OSS)
     int window,                              // 0 = full attention
     float softcap) {                         // 0 = off (Gemma-2 tanh cap)
-  constexpr int GQ = 1;
   constexpr int DV = D / 16;        // value channels per lane
   constexpr int ES = FP8 ? 1 : 2;   // bytes per cached number
   constexpr int QK = D / 32;        // products per 16 keys
@@ -182,10 +185,10 @@ void paged_attn_heads_kernel(
   static_assert(D == 64 || D == 128 || D == 256, "D in {64, 128, 256}");
 
   const int seq = blockIdx.x;
-  const int h = blockIdx.y;         // query head; rep of them share a kv head
+  const int h = blockIdx.y;         // GQ query heads; rep of these share a kv head
   const int hk = rep == 1 ? h : h / rep;
   const int nsplit = gridDim.z;
-  const int Hq = gridDim.y;
+  const int Hq = gridDim.y * GQ;
   const int len = seq_lens[seq];
   // sliding window (EXT): the query sits at position len - 1 and attends
   // [max(0, len - window), len); the parts cut only that
@@ -407,7 +410,7 @@ void paged_attn_heads_kernel(
       out[((long)seq * Hq + (long)h * GQ + gq) * D + d] =
           f2bf(den > 0.f ? num / den : 0.f);
     } else {
-      float* pp = part + ((((long)seq * Hq + h) * nsplit + blockIdx.z) * GQ +
+      float* pp = part + ((((long)seq * gridDim.y + h) * nsplit + blockIdx.z) * GQ +
                           gq) * (D + 2);
       pp[d] = num;
       if (d == 0) {
@@ -458,7 +461,8 @@ constexpr int ring_bytes(int D, bool fp8, int pages) {
 // 37.3 / 35.5. Where a CU works through many workgroups of one step each, the row's
 // chain stands in front of every one: 512 x 40 to 58 36.8 / 40.7, in fp8 34 / 42.
 template <int D, bool FP8, bool EXT, int PGS, bool NEW>
-__global__ __launch_bounds__(THREADS, D == 256 || ring_bytes(D, FP8, PGS) > 8192 ? 2 : 3)
+__global__ __launch_bounds__(THREADS, D == 256 || ring_bytes(D, FP8, PGS) > 8192 ? 2
+                                    : D == 64 && PGS == 1                      ? 5 : 3)
 void paged_attn_decode_kernel(
     unsigned short* __restrict__ out,        // [N, Hq, D]
     const unsigned short* __restrict__ q,    // [N, Hq, D]
@@ -1011,37 +1015,49 @@ __global__ __launch_bounds__(D) void paged_attn_join_kernel(
 // but not into more than 8 parts.
 // A context of less than one part pays for the join's launch behind a wide
 // block table (one sequence of 100 keys, 8 heads on 8: 5.8 against 4.4).
-// grouped: the pools take 16-byte direct loads.
+// Up to 64 groups (128 of 64-byte rows) parts of 128 keys, one step, where the table has
+// more than 256 and the join is there anyway, one part up to there. us, parts of 256 / of
+// 128, 16 heads on 8: 3 x 200 to 400 7.8 / 6.5, 8 7.9 / 7.0, 3 x 500 to 1200 8.3 / 7.4, 8
+// 10.7 / 10.7, 6 9.1 / 9.5; of 256 channels 3 x 200 to 400 .78 of the time, in fp8 .81; but
+// behind a table of 200 3 x 128 to 200 in one part 5.0, in two 6.2.
+// Two heads a kv head of 64 channels go through paged_attn_heads_kernel as a pair in fp8,
+// and in bf16 behind tables of up to 64 keys up to 512 groups (256 groups .87 of the time,
+// 768 1.06).
+// aligned: the pools take 16-byte direct loads.
 DecodeParts decode_parts(int N, int Hq, int Hkv, int max_blocks, int D, int fp8,
                          int window, int aligned) {
-  const int grouped = Hq > Hkv && aligned && max_blocks > 0;
+  const bool grouped = Hq > Hkv && aligned && max_blocks > 0;
+  const bool pairs =
+      grouped && Hq == 2 * Hkv && D == 64 &&
+      (fp8 || (max_blocks <= 4 && (long)N * Hkv <= 512));
+  const int heads = pairs ? 2 : grouped ? 0 : 1;
   const long base = (long)N * (grouped ? Hkv : Hq);
-  if (base < 1) return {1, 4 * STEP, grouped};
+  if (base < 1) return {1, 4 * STEP, heads};
+  long keys = (long)max_blocks * BS;
+  if (window > 0 && window < keys) keys = window;
   const bool narrow = D * (fp8 ? 1 : 2) <= 128;
   long n, cap = 16;
   int least;
-  if (grouped) {
+  if (heads == 0) {
     const int row = D * (fp8 ? 1 : 2);
     n = row <= 64     ? (base >= 512 ? 1 : 1024 / base)
         : row <= 128  ? (base >= 256 ? 1 : 512 / base)
         : base <= 256 ? 256 / base
         : base < 400  ? (1024 + base - 1) / base
                       : 1;
-    least = base <= 64 ? 256 : 512;
+    least = base > (row <= 64 ? 128 : 64) ? 512 : keys > 256 ? 128 : 256;
   } else {
-    n = narrow        ? 1024 / base
+    n = narrow        ? (pairs && base >= 512 ? 1 : 1024 / base)
         : base >= 512 ? 1
         : D > 128     ? (1024 + base - 1) / base
                       : (512 + base - 1) / base;
     least = base >= 256 ? 512 : base >= 128 ? 256 : 128;
     if (D > 128) cap = 8;
   }
-  long keys = (long)max_blocks * BS;
-  if (window > 0 && window < keys) keys = window;
   const long most =
-      base >= 128 && !grouped ? keys / least : (keys + least - 1) / least;
+      base >= 128 && heads > 0 ? keys / least : (keys + least - 1) / least;
   if (n > most) n = most;
-  return {(int)(n < 1 ? 1 : n > cap ? cap : n), least, grouped};
+  return {(int)(n < 1 ? 1 : n > cap ? cap : n), least, heads};
 }
 
 namespace {
@@ -1065,38 +1081,45 @@ struct DecodeArgs {
 template <int D, bool FP8, bool EXT>
 void decode_launch(const DecodeArgs& a) {
   const int GQ = a.Hq / a.Hkv;
-  auto run = [&](auto kernel, int heads, auto... extra) {
-    hipLaunchKernelGGL(kernel, dim3(a.N, heads, a.parts.n), dim3(THREADS), 0, a.s,
+  auto run = [&](auto kernel, int units, int per, auto... extra) {
+    hipLaunchKernelGGL(kernel, dim3(a.N, units, a.parts.n), dim3(THREADS), 0, a.s,
                        a.out, a.q, a.kc, a.vc, a.block_tables, a.seq_lens, a.part,
-                       a.parts.least, a.Hkv, GQ, a.max_blocks, a.scale, a.q_stride,
+                       a.parts.least, a.Hkv, per, a.max_blocks, a.scale, a.q_stride,
                        a.sinks, a.window, a.softcap, extra...);
   };
-  if (!a.parts.grouped) {
-    run(paged_attn_heads_kernel<D, FP8, EXT>, a.Hq);
+  if (a.parts.heads == 1) {
+    run(paged_attn_heads_kernel<D, 1, FP8, EXT>, a.Hq, GQ);
     return;
   }
-  // Pages a step: two of fp8 rows and of 64 channels, one of 256 channels in bf16; of
-  // 128 in bf16 two up to one workgroup a CU, which then has more under way (us, one
-  // page / two: 32 sequences of 1000 to 6000 keys, 32 heads on 8 99 / 93, 24 of 300 to
-  // 1200 21.4 / 19.0, but of 40 to 60 4.4 / 4.8), one where they are more and share it
-  // (40 x 300 to 1200 32.1 / 34.4, 64 x 500 29.5 / 33.0, 512 x 40 to 60 26.1 / 33.9, but
-  // 384 x 200 to 400 93 / 88).
-  constexpr bool ONE = !FP8 && D >= 128, TWO = FP8 || D <= 128;
+  if constexpr (D == 64) {
+    if (a.parts.heads == 2) {
+      run(paged_attn_heads_kernel<D, 2, FP8, EXT>, a.Hkv, 1);
+      return;
+    }
+  }
+  // Pages a step: two of fp8 rows, one of 256 channels in bf16; of fewer in bf16 two up to
+  // one workgroup a CU, which then has more under way (us, one page / two: 32 sequences of
+  // 1000 to 6000 keys, 32 heads on 8 of 128 99 / 93, 24 of 300 to 1200 21.4 / 19.0, but of
+  // 40 to 60 4.4 / 4.8), one where they are more and share it (40 x 300 to 1200 32.1 /
+  // 34.4, 64 x 500 29.5 / 33.0, 512 x 40 to 60 26.1 / 33.9, but 384 x 200 to 400 93 / 88; of
+  // 64 channels, 16 heads on 8, five of whose workgroups then share it, 384 x 20 to 64
+  // 10.0 / 12.9, 128 x 200 to 400 .94 to 1.02, 500 to 1200 .96 to .99 of the time).
+  constexpr bool ONE = !FP8, TWO = FP8 || D <= 128;
   constexpr bool FUSED = D == 128 && !EXT;
   if constexpr (ONE) {
     if (!TWO || (long)a.N * a.Hkv > 256) {
       if (FUSED && a.rows.slots != nullptr)
-        run(paged_attn_decode_kernel<D, FP8, EXT, 1, FUSED>, a.Hkv, a.rows);
+        run(paged_attn_decode_kernel<D, FP8, EXT, 1, FUSED>, a.Hkv, GQ, a.rows);
       else
-        run(paged_attn_decode_kernel<D, FP8, EXT, 1, false>, a.Hkv, a.rows);
+        run(paged_attn_decode_kernel<D, FP8, EXT, 1, false>, a.Hkv, GQ, a.rows);
       return;
     }
   }
   if constexpr (TWO) {
     if (FUSED && a.rows.slots != nullptr)
-      run(paged_attn_decode_kernel<D, FP8, EXT, 2, FUSED>, a.Hkv, a.rows);
+      run(paged_attn_decode_kernel<D, FP8, EXT, 2, FUSED>, a.Hkv, GQ, a.rows);
     else
-      run(paged_attn_decode_kernel<D, FP8, EXT, 2, false>, a.Hkv, a.rows);
+      run(paged_attn_decode_kernel<D, FP8, EXT, 2, false>, a.Hkv, GQ, a.rows);
   }
 }
 }  // namespace
@@ -1115,7 +1138,7 @@ void paged_attn_decode_launch(void* out, const void* q, const void* kc,
   const bool ext = (sinks != nullptr) || window > 0 || softcap > 0.f;
   *err_unsupported = (D != 128 && D != 64 && D != 256) || GQ < 1 || GQ > 8 ||
                      GQ == 3 || (D == 256 && GQ > 4) ||
-                     (rows != nullptr && (D != 128 || ext || !parts.grouped));
+                     (rows != nullptr && (D != 128 || ext || parts.heads != 0));
   if (*err_unsupported || N == 0) return;
   const DecodeArgs a{(unsigned short*)out, (const unsigned short*)q,
                      (const char*)kc, (const char*)vc, block_tables, seq_lens,
@@ -1129,7 +1152,7 @@ void paged_attn_decode_launch(void* out, const void* q, const void* kc,
 #define JOIN(DD)                                                              \
   hipLaunchKernelGGL((paged_attn_join_kernel<DD>), dim3(N, Hq), dim3(DD), 0,  \
                      s, (unsigned short*)out, part, seq_lens,                 \
-                     parts.grouped ? GQ : 1, nsplit,                          \
+                     parts.heads == 0 ? GQ : parts.heads, nsplit,             \
                      parts.least, sinks, window)
   if (D == 128) JOIN(128);
   else if (D == 64) JOIN(64);

@@ -15,7 +15,7 @@ void reshape_and_cache_launch(const void*, const void*, void*, void*, const long
 void greedy_sample_launch(long*, long*, const void*, int, int, hipStream_t);
 void mla_decode_launch(float*, const void*, const void*, const int*, const int*, int, int, int, int, int, int, float, int*, hipStream_t);
 void qkv_store_launch(void*, const float*, int, const void*, const void*, const float*, const long*, const long*, void*, void*, long, int, int, int, int, float, int, int*, hipStream_t);
-struct DecodeParts { int n, least, grouped; };
+struct DecodeParts { int n, least, heads; };
 struct NewRows {
   const unsigned short* rows;
   const float* parts;

@@ -120,3 +120,35 @@ def test_infinite_values(monkeypatch, lens, D, G):
     assert int(odd.sum()) >= 4 * len(rows) * 2 * G
     assert torch.equal(out[odd].nan_to_num(nan=5.0), ref[odd].nan_to_num(nan=5.0))
     assert bool((out - ref)[~odd].abs().le(ref[~odd].abs() * 2.0 ** -8 + 1e-4).all())
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("pages", [4, 5, 16, 17])
+@pytest.mark.parametrize("copies", [1, 64, 65])
+@pytest.mark.parametrize("extra", [False, True])
+def test_two_heads(monkeypatch, fp8, D, pages, copies, extra):
+    """Two query heads a kv head, behind tables up to and above 64 keys (pairs of 64
+    channels) and 256 (parts of 128 keys); 8, 512 and 520 groups; with a window and sinks."""
+    from gpustack_amd import ops
+    from gpustack_amd.ops import torch_ref
+
+    monkeypatch.setenv("GPUSTACK_AMD_OSS_KERNELS", "1")
+    lens = [1, 33, 16 * pages - 15, 16 * pages]
+    kc, vc, bt, q = _pools(lens, 2, D, fp8, D + pages)
+    q = q[:, :4].repeat(copies, 1, 1)
+    bt = bt[:, :pages].repeat(copies, 1)
+    lens = lens * copies
+    sl = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    more = {"window": 40, "sinks": torch.tensor([.5, -1., 3., 0.], device="cuda")} \
+        if extra else {}
+    out = torch.full_like(q, float("nan"))
+    ops.paged_attn_decode(out, q, kc, vc, bt, sl, D ** -0.5, **more)
+    if not extra:
+        _check(out, q, kc, vc, bt, lens, fp8, [0, 1, 2, 3])
+    ref = torch.empty_like(q[:4])
+    clean = [t.float().nan_to_num().bfloat16() for t in (kc, vc)]
+    torch_ref.paged_attn_decode(ref, q[:4], *clean, bt[:4], sl[:4], D ** -0.5, **more)
+    assert bool(((out[:4] - ref).abs().float()         # both rounded to bf16
+                 <= ref.abs().float() * 2.0 ** -7 + 1e-4).all())
+    assert bool((out.view(copies, 4, -1) == out[:4].view(4, -1)).all())
