@@ -289,8 +289,8 @@ def paged_attn_decode_rows_ok(rows, q_heads: int, kv_heads: int, head_dim: int,
                               k_cache, v_cache, block_tables, *norms) -> bool:
     """Whether paged_attn_decode_rows takes a step: heads of 128 channels, two to
     eight of them (not three) a kv head, without sinks, window or score cap, pools and
-    head norms (`norms`, or None) at 16-byte addresses; and where it is the faster one. It saves 1.2 to 2.7 us up to four workgroups a CU
-    whatever the lengths (128 rows of 8 kv heads 14.5 -> 13.4 at 40 keys, 41.9 ->
+    head norms (`norms`, or None) at 16-byte addresses; and where it is the faster one.
+    It saves 1.2 to 2.7 us up to four workgroups a CU whatever the lengths (128 rows of 8 kv heads 14.5 -> 13.4 at 40 keys, 41.9 ->
     39.2 at 256 to 383). Behind them it loses contexts under 80 keys (256 rows of 40
     to 58 21.9 -> 22.8, 512 36.8 -> 40.7) and gains longer ones (80 to 109 54.5 ->
     54.7, 100 to 149 67.6 -> 64.5): it is taken where the block table has room for
@@ -787,12 +787,19 @@ def _few_rows_plan(M: int, N: int, K: int, plan, rows: bool):
     k, given what _rows_tile_plan and _rows_gemm_wins say: the form of the least time
     (_few_time), where it is 8 % less than that of theirs; in the library's place one of
     the two, but beyond 16 rows only where it is no more than the library takes at its
-    best (8 us and 5.4 TB/s), and neither up to 8192 columns of 4096 k. Of 2233 such sizes
-    these take 1.024 of the time of the best form, where the two rules alone took 1.114:
-    728 take less by more than 4 %, 41 more, most of them of 2560 k beside the library, 8
-    by more than 8 %, to 1.13. us: 16 rows of 151936 x 2048 130 -> 117, 8 of 10304 x 2048
-    14.7 -> 12.5, 16 of 8192 x 2048 11.0 -> 8.3, 16 of 102400 x 1536 71 -> 63, 32 of 14336
-    x 1024 21.4 -> 7.7."""
+    best (8 us, below 3072 columns 6, and 5.4 TB/s), and neither up to 8192 columns of 4096
+    k. Of 2233 sizes up to 64 rows (8 us everywhere) these take 1.024 of the time of the
+    best form, the two rules alone 1.114; 41 more than with the two rules by over 4 %. us: 16 rows of 151936 x 2048 130 -> 117, 8 of 10304 x 2048 14.7 -> 12.5, 16 of 8192 x
+    2048 11.0 -> 8.3, 16 of 102400 x 1536 71 -> 63, 32 of 14336 x 1024 21.4 -> 7.7.
+    Of 620 sizes of 17 to 64 rows of 1024 to 3968 k that the two rules leave to the library
+    439 are taken, .867 of the time on average, 20 more by over 3 %, to 1.09 (64 rows of
+    27648 x 2560). Below 3072 columns up to 96 of the 256 CUs have a tile, and the library
+    cuts k: with 8 us there 41 took more, to 1.26 (32 of 1536 x 2816 7.4 / 9.3).
+    Of 4096 k the library has numbers that it has not of 4032 (library / tiles of 32 at 1, 8,
+    16, 32, 64 rows: 8192 columns of 4096 17.1 / 17.8, 17.2 / 17.7, 17.1 / 17.4, 17.6 / 17.1,
+    20.1 / 21.0; of 4032 20.3 / 14.1, 20.5 / 14.0, 20.5 / 14.2, 23.0 / 15.3, 29.1 / 21.9), and
+    the tiles' rows lie a power of two apart; of 6144 columns the tiles would take 13.4 to
+    14.2 for 14.3 to 15.3 up to 32 rows, 19.0 for 17.9 at 64; beyond, 9216, 23.5 for 26.0."""
     if not (0 < M <= 64 and 1024 <= K <= 4096 and N >= 1024) or K % 64 or N % 8 \
             or plan and plan[1] > 1:
         return plan, rows
@@ -803,7 +810,7 @@ def _few_rows_plan(M: int, N: int, K: int, plan, rows: bool):
     now = plan[0] if plan else 0 if rows else None
     if now is None:
         if N <= 8192 and K == 4096 \
-                or M > 16 and time[best] > 8 + 2e-6 * N * K / 5.4:
+                or M > 16 and time[best] > (8 if N >= 3072 else 6) + 2e-6 * N * K / 5.4:
             return plan, rows
     elif time[best] >= .92 * time[now]:
         return plan, rows

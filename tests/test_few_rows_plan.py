@@ -24,6 +24,10 @@ def test_forms():
     assert f(32, 14336, 1024)[0] is not None
     assert f(1, 4096, 2048) == (None, True)             # as before
     assert f(64, 8192, 4096) == (None, False)           # the library
+    # few workgroups beyond 16 rows, where the library cuts k
+    for M, N, K in ((32, 1536, 2816), (32, 2560, 3072), (17, 2560, 2304), (48, 1536, 1536)):
+        assert f(M, N, K) == (None, False)
+    assert f(32, 3072, 3072)[0] is not None
     for N in range(1024, 40000, 1000):
         for K in range(1024, 4097, 64):
             plan, rows = f(8, N - N % 8, K)
