@@ -707,8 +707,8 @@ def choose_sorts(T: int, E: int) -> bool:
 def moe_few_wins(rows: int, E: int, K: int, down: bool) -> bool:
     """Whether an expert product of `rows` assignments takes 16 rows at a time straight
     from memory (moe_few) in the place of tiles of 128 x 128 (moe_tile): the first product
-    up to 4 rows an expert, the second too of up to 768 k, to one of rows beyond 3072, else
-    to 3/4. More than 16 rows of an expert read its weights again, so the lines
+    up to 4 rows an expert, the second up to 768 k to 4 where its blocks of 64 k are the same
+    for the four waves, else to 2, to one of rows beyond 3072, else to 3/4. More than 16 rows of an expert read its weights again, so the lines
     allow for uneven routing. us, tiles / this, E experts of N x K, even routing: first, 128
     of 768 x 2048 8 assignments 22.1 / 13.5, 64 71 / 56, 256 128 / 116, 512 142 / 133, 768
     145 / 137, 64 of 1024 x 2048 128 101 / 79, 32 of 2048 x 1024 128 42.7 / 40.1, 256 43.5
@@ -717,11 +717,18 @@ def moe_few_wins(rows: int, E: int, K: int, down: bool) -> bool:
     896 32 11.3 / 11.2, 64 15.4 / 16.0, 512 20.1 / 22.2, 16 of 4096 x 6400 16 106 / 90, 64
     140 / 142. Uneven, half of 64 rows to one of the experts and 114 of 128 with any, 768 x
     2048 512 134 / 127 and 2048 x 768 65.8 / 66.0; 96 rows of them, 68 to one,
-    140 / 142 and 70.7 / 75.6."""
+    140 / 142 and 70.7 / 75.6. The second at 2 / 3 / 4 rows an expert by k, of the tiles' time:
+    128 of 2048 columns 512 .83 / .90 / .93, 640 .88 / .98 / 1.03, 704 .85 / .93 / .97, 768 .85 /
+    .92 / .95, 832 .93 / .96 / .99, 896 .89 / .96 / .98, 1024 .98 / 1.0 / 1.02; 64 of 1024 512
+    .92 / 1.05 / 1.07, 640 1.02 / 1.05 / 1.10, 704 1.02 / 1.03 / 1.07, 768 .95 / .97 / .98, 832
+    1.03 / 1.06 / 1.05, 1024 1.02 / 1.09 / 1.10; beyond 768 k what is left at 1 row is .73 to .95,
+    at 3/4 .67 to 1.02."""
     if rows <= 0:
         return False
-    if not down or K <= 768:
+    if not down:
         return rows <= 4 * E
+    if K <= 768:
+        return rows <= (4 if K % 256 == 0 else 2) * E
     return rows <= E if K > 3072 else 4 * rows <= 3 * E
 
 

@@ -88,6 +88,8 @@ def test_replays():
 @pytest.mark.parametrize("rows,E,K,down,wins", [
     (512, 128, 2048, False, True), (513, 128, 2048, False, False),
     (512, 128, 768, True, True), (513, 128, 768, True, False),
+    (512, 128, 512, True, True), (256, 128, 640, True, True), (257, 128, 640, True, False),
+    (257, 128, 704, True, False), (513, 128, 704, False, False),
     (96, 128, 832, True, True), (97, 128, 3072, True, False),
     (16, 16, 3136, True, True), (17, 16, 6400, True, False),
     (0, 8, 14336, False, False)])
