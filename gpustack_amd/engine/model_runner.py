@@ -858,8 +858,9 @@ class ModelRunner:
     def execute_async(self, batch: ScheduledBatch, reuse_tokens: bool):
         """Submit a greedy decode step without reading results back.
 
-        Samples on-device into the persistent buffer and starts an async
-        D2H copy; read_sampled() collects it one step later. With
+        Samples on-device into the persistent buffer; the sampling kernel
+        leaves the words in pinned memory too, where read_sampled() collects
+        them one step later. With
         reuse_tokens, the previous step's sampled ids feed this step's
         token input device-side (no host round-trip at all)."""
         bs = len(batch.seqs)

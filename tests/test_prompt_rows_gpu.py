@@ -53,13 +53,14 @@ def _parts(gs, groups, first, T):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("G,VW,skew", [(4, 128, 0), (3, 24, 0), (5, 13, 0), (9, 128, 0),
-                                       (4, 128, 2)])
+                                       (4, 128, 1), (3, 24, 2), (9, 128, 4)])
 def test_value_pages(dtype, G, VW, skew):
-    """By 16 bytes and (odd widths, rows that begin elsewhere) value by value; whole
+    """By 16 bytes and (odd widths, rows at other addresses) value by value; whole
     pages, a page's part, rows without a slot."""
     D, nq, nb, T = 64, 64, 9, 40
     nk, nv, rnd = G * D, G * VW, _rnd(G + VW)
-    qkv = rnd(T, nq + nk + nv + skew).to(dtype)[:, skew:]
+    rows = rnd(T, nq + nk + nv).to(dtype)
+    flat = torch.empty(rows.numel() + 8, dtype=dtype, device="cuda")
     slots = torch.full((T,), -1, dtype=torch.long, device="cuda")
     slots[:16] = torch.arange(48, 64, device="cuda")
     slots[16:32] = torch.arange(96, 112, device="cuda")
@@ -73,13 +74,10 @@ def test_value_pages(dtype, G, VW, skew):
         q = torch.zeros(T, nq, dtype=dtype, device="cuda")
         kc = torch.zeros(nb, G, 16, D, dtype=dtype, device="cuda")
         vc = torch.zeros(nb, G, VW, 16, dtype=dtype, device="cuda")
-        rows = qkv if skew else qkv.clone()
-        if skew and impl is ops:
-            rows = torch.empty(T, nq + nk + nv + skew, dtype=dtype,
-                               device="cuda")[:, skew:]
-            rows.copy_(qkv)
-        args = (q, rows.contiguous(), nq, nk, w, w, D, 0.0, 0, pos, None, None, kc, vc,
-                slots, 1e-5)
+        qkv = flat[skew:skew + rows.numel()].view_as(rows)
+        qkv.copy_(rows)
+        assert qkv.data_ptr() % 16 == skew * qkv.element_size() % 16
+        args = (q, qkv, nq, nk, w, w, D, 0.0, 0, pos, None, None, kc, vc, slots, 1e-5)
         if impl is ops:
             ops.head_norm_store(*args, page_groups=groups)
         else:
@@ -97,11 +95,16 @@ def test_embedding(W):
     assert torch.equal(x, table.float()[ids.clamp(0, 10)] * torch.tensor(1.7).cuda())
 
 
-@pytest.mark.parametrize("taps", [2, 3, 4])
-@pytest.mark.parametrize("news", [[8, 8], [1, 40, 2, 3, 21, 8, 16], [300]])
+@pytest.mark.parametrize("taps", [2, 3, 4, 5])
+@pytest.mark.parametrize("news,C", [
+    ([8, 8], 264), ([1, 40, 2, 3, 21, 8, 16], 264), ([300], 264),
+    # from 2^20 numbers on eight rows a lane: groups that begin 0 to 7 rows into a
+    # sequence, lie across two or more of them, and end behind the last row
+    ([300], 4096), ([16, 17, 18, 19, 20, 21, 22, 23, 24, 25, 26, 27], 4104),
+    ([1, 40, 2, 3, 21, 8, 16, 1, 1, 1, 5, 60, 64, 40], 4096), ([1] * 37, 30000)])
 @pytest.mark.parametrize("silu", [True, False])
-def test_convolution(taps, news, silu):
-    C, rnd = 264, _rnd(sum(news) + taps)
+def test_convolution(taps, news, C, silu):
+    rnd = _rnd(sum(news) + taps)
     T, S = sum(news), len(news)
     i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
     first = [sum(news[:i]) for i in range(S)]
