@@ -446,9 +446,10 @@ constexpr int ring_bytes(int D, bool fp8, int pages) {
 // 64 x 200 to 2000 of 32 heads on 4 44 -> 33, 16 x 300 to 1200 20.4 -> 16.3, 4 x 2000
 // to 6000 27 -> 20.7; 512 x 256 to 383 128 -> 125. Of 196 batches of 12 to 512
 // sequences of 40 to 6000 keys none is slower by more than 3 %, .80 of the time on
-// average; of 700 drawn with all options 25 are, most of two heads a kv head and up to
-// 64 keys (16 heads on 8, three x 64 keys 5.5 -> 6.1): a workgroup of one step is its
-// latencies, of which the LDS adds one.
+// average; of 1536 of 1 to 384 sequences of 20 to 1200 keys 94 are, .82 on average, most
+// of two heads a kv head and up to 64 keys (16 heads on 8 of 128, three x 20 to 64 3.9 ->
+// 4.2, 128 in fp8 6.8 -> 7.5): a workgroup of one step is its latencies, of which the LDS
+// adds one.
 // EXT: sinks / sliding window / softcap (GPT-OSS and Gemma variants).
 // NEW: q is not there yet, nor the step's own key and value in the pools. Each workgroup
 // makes its query heads from the projection's row, and the one whose part ends with the
@@ -456,9 +457,9 @@ constexpr int ring_bytes(int D, bool fp8, int pages) {
 // are under way, puts them over the row that these bring into the LDS. All of it, in the
 // order and to the bit of the row kernel (qkv_store), while the first pages come, so that
 // a launch and a round trip are saved. us, in two launches / in one, 32 heads on 8: one
-// row of 1000 keys 11.9 / 10.2, 16 of 300 to 1200 20.5 / 18.3, 512 of 256 to 383 142 /
-// 137, 48 of 3500 to 7900 in fp8 127.6 / 125.4; 64 x 200 to 2000 of 32 on 4 with norms
-// 37.3 / 35.5. Where a CU works through many workgroups of one step each, the row's
+// row of 1000 keys 9.5 / 8.0, 16 of 300 to 1200 19.1 / 16.5, 512 of 256 to 383 139.9 /
+// 131.9, 48 of 3500 to 7900 in fp8 125.4 / 124.2; 64 x 200 to 2000 of 32 on 4 with norms
+// 38.0 / 36.2. Where a CU works through many workgroups of one step each, the row's
 // chain stands in front of every one: 512 x 40 to 58 36.8 / 40.7, in fp8 34 / 42.
 template <int D, bool FP8, bool EXT, int PGS, bool NEW>
 __global__ __launch_bounds__(THREADS, D == 256 || ring_bytes(D, FP8, PGS) > 8192 ? 2
